@@ -123,8 +123,8 @@ template <typename KV, int D> __device__ __forceinline__ LaneRole lane_role(int 
     LaneRole r;
     r.row = lane / S::LPR;
     r.lir = lane - r.row * S::LPR;
-    r.head_local = r.row % p.hpw;
-    r.tok_local = r.row / p.hpw;
+    r.head_local = r.row & (p.hpw - 1);  // (a power of two)
+    r.tok_local = r.row >> __builtin_ctz(p.hpw);
     r.d0 = r.lir * S::EPL;
     return r;
 }
@@ -341,19 +341,19 @@ template <typename KV, typename QT, int D, int NREP, int U> struct Attender {
 };
 
 // Merge the kWaves*TPW row-group partials of every (kv head of the group,
-// query head r) through LDS and hand (qh, d, num[4], M, den) of the merged
-// partial - four consecutive d at a time - to `emit`; out = num/den, M is the
-// base-2 running maximum.
+// query head r) and hand (qh, d, num[4], M, den) of the merged partial - four
+// consecutive d at a time - to `emit`; out = num/den, M is the base-2 running
+// maximum.
 //
-// The waves' lanes hold ROWS = kWaves*RPW partial rows per query head; rows
-// with the same row % hpw belong to the same kv head and are merged.  HR query
-// heads go through LDS per round (as many as the LDS budget allows): every
-// lane writes its accumulators, then one thread per (head, row) computes the
-// row's weight exp2(m_row - M) (and, for the first row of each kv head, M and
-// the merged denominator), then one thread per (head, kv head, d) sums
-// weight * accumulator over the rows.  The row loops are unrolled by 4 (the
-// row count per kv head is kWaves*tpw, a multiple of 4) so that their LDS
-// reads overlap.
+// This is a chain of waits that every piece of a sequence pays for, beside
+// which a short sequence's own keys are little.  A wave's token rows are merged
+// in registers, lane against lane; the waves' rows of HR query heads (as many
+// as the LDS budget allows) go through LDS per round: every lane of the first
+// token row writes its accumulators, then one thread per (head, row) computes
+// the row's weight exp2(m_row - M), M and the merged denominator, then one
+// thread per (head, kv head, d) sums weight * accumulator over the waves.
+// One sequence of 16 keys, 14 / 2 heads of 64 (four token rows per wave): 13.4
+// us for the whole step, 17.7 with every row through LDS two heads at a time.
 template <typename KV, int D, int NREP> struct MergeShape {
     static constexpr int ROWS = kWaves * RowShape<KV, D>::RPW;
     static constexpr int ROWF = D + 2;  // floats of a partial row: D accumulators, m, l
@@ -371,49 +371,84 @@ template <typename KV, int D, int NREP> struct MergeShape {
                   "decode_plan.h and MergeShape disagree");
 };
 
-template <typename KV, int D, int NREP, typename Emit>
-__device__ __forceinline__ void merge_rows(RowState<NREP, RowShape<KV, D>::EPL> &st, float *s_part,
-                                           const PoolArgs &p, const LaneRole &role, int wave, int tid, int hg,
-                                           int rep0, Emit emit) {
+// The values of this lane and of the one whose index differs in the bit MASK (0: in `mask`), in the same order for both.
+template <int MASK> __device__ __forceinline__ float2 lane_pair(float x, int mask) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    if constexpr (MASK == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return float2{__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+    } else if constexpr (MASK == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return float2{__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+    } else {
+        return float2{x, __shfl_xor(x, mask, PA_WAVE)};
+    }
+}
+template <int MASK, int NREP, int EPL> __device__ __forceinline__ void merge_lane_pairs(RowState<NREP, EPL> &st, int mask) {
+#pragma unroll
+    for (int r = 0; r < NREP; ++r) {
+        const float2 m = lane_pair<MASK>(st.m[r], mask);
+        const float M = fmaxf(m.x, m.y), f = __builtin_amdgcn_exp2f(st.m[r] - M);
+        st.m[r] = M;
+        const float2 l = lane_pair<MASK>(st.l[r] * f, mask);
+        st.l[r] = l.x + l.y;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+            const float2 x = lane_pair<MASK>(st.acc[r][e] * f, mask);
+            st.acc[r][e] = x.x + x.y;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (all of them at once take registers that the kernel does not have)
+    }
+}
+// The rows of a wave whose lanes differ in the bits of the lane index from `low` up, merged in all of them.
+template <int NREP, int EPL> __device__ __forceinline__ void merge_lanes(RowState<NREP, EPL> &st, int low) {
+    for (int mask = low; mask < 16; mask *= 2) merge_lane_pairs<0>(st, mask);
+    if (low <= 16) merge_lane_pairs<16>(st, 16);
+    if (low <= 32) merge_lane_pairs<32>(st, 32);
+}
+
+template <typename KV, int D, int NREP, int HR, typename Emit>
+__device__ __forceinline__ void merge_rounds(RowState<NREP, RowShape<KV, D>::EPL> &st, float *s_part, const PoolArgs &p,
+                                             const LaneRole &role, int prow, int tid, int hg, int rep0, Emit emit) {
     using S = RowShape<KV, D>;
-    using MS = MergeShape<KV, D, NREP>;
-    constexpr int ROWS = MS::ROWS, ROWF = MS::ROWF, HR = MS::HR;
-    st.fold_zero_keys();
-    const int prow = wave * S::RPW + role.row;  // = wave*RPW + tok_local*hpw + head_local
-    float *s_wgt = s_part + MS::AUX, *s_M = s_wgt + HR * ROWS, *s_den = s_M + HR * ROWS;
+    constexpr int ROWF = D + 2;
     const int hpw = p.hpw;  // a power of two dividing RPW
     const int lg_hpw = __builtin_ctz(hpw);
+    const int rows = kWaves * hpw;  // (HR * rows never exceeds MergeShape's HR * ROWS)
+    float *s_wgt = s_part + HR * rows * ROWF, *s_M = s_wgt + HR * rows, *s_den = s_M + HR * rows;
 #pragma unroll
     for (int round = 0; round < NREP / HR; ++round) {
         if (rep0 + round * HR >= p.n_rep) break;  // uniform over the workgroup
         __syncthreads();  // the readers of the previous round (or of the previous call) are done
+        if (role.tok_local == 0) {
 #pragma unroll
-        for (int h = 0; h < HR; ++h) {
-            float *row = s_part + (h * ROWS + prow) * ROWF;
+            for (int h = 0; h < HR; ++h) {
+                float *row = s_part + (h * rows + prow) * ROWF;
 #pragma unroll
-            for (int e = 0; e < S::EPL; ++e) row[role.d0 + e] = st.acc[round * HR + h][e];
-            if (role.lir == 0) {
-                row[D] = st.m[round * HR + h];
-                row[D + 1] = st.l[round * HR + h];
+                for (int e = 0; e < S::EPL; ++e) row[role.d0 + e] = st.acc[round * HR + h][e];
+                if (role.lir == 0) {
+                    row[D] = st.m[round * HR + h];
+                    row[D + 1] = st.l[round * HR + h];
+                }
             }
         }
         __syncthreads();
-        for (int idx = tid; idx < HR * ROWS; idx += kThreads) {
-            const int h = idx / ROWS, row = idx - h * ROWS;
-            const int hl = row & (hpw - 1);
-            const float *base = s_part + h * ROWS * ROWF;
-            float M = kNegBig;
-#pragma unroll 4
-            for (int r2 = hl; r2 < ROWS; r2 += hpw) M = fmaxf(M, base[r2 * ROWF + D]);
-            s_wgt[idx] = __builtin_amdgcn_exp2f(base[row * ROWF + D] - M);
-            if (row < hpw) {  // first row of its kv head: the merged maximum and denominator
-                float den = 0.f;
-#pragma unroll 4
-                for (int r2 = hl; r2 < ROWS; r2 += hpw)
-                    den = fmaf(__builtin_amdgcn_exp2f(base[r2 * ROWF + D] - M), base[r2 * ROWF + D + 1], den);
-                s_M[idx] = M;
-                s_den[idx] = den;
+        for (int idx = tid; idx < HR * rows; idx += kThreads) {
+            const int hl = idx & (hpw - 1), h = idx >> (lg_hpw + 2);  // (rows = 4 hpw)
+            const float *base = s_part + (h * rows + hl) * ROWF + D;
+            float m[kWaves], l[kWaves], M = kNegBig, den = 0.f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                m[w] = base[w * hpw * ROWF];
+                l[w] = base[w * hpw * ROWF + 1];
             }
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) M = fmaxf(M, m[w]);
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) den = fmaf(__builtin_amdgcn_exp2f(m[w] - M), l[w], den);
+            s_wgt[idx] = __builtin_amdgcn_exp2f(s_part[idx * ROWF + D] - M);
+            s_M[idx] = M;
+            s_den[idx] = den;
         }
         __syncthreads();
         // four consecutive d per thread: the results leave as one 16-byte store (a part's partial is 8 KB and
@@ -423,26 +458,47 @@ __device__ __forceinline__ void merge_rows(RowState<NREP, RowShape<KV, D>::EPL> 
             const int hl = hd & (hpw - 1), h = hd >> lg_hpw;
             const int r = round * HR + h;
             if (rep0 + r >= p.n_rep) continue;
-            const float *base = s_part + h * ROWS * ROWF + d;
-            const float *wgt = s_wgt + h * ROWS;
+            const float *base = s_part + (h * rows + hl) * ROWF + d;
+            const float *wgt = s_wgt + h * rows + hl;
             float num[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-            for (int r2 = hl; r2 < ROWS; r2 += hpw) {
-                const float w = wgt[r2];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) num[j] = fmaf(w, base[r2 * ROWF + j], num[j]);
+            for (int w = 0; w < kWaves; ++w) {
+                const float f = wgt[w * hpw];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) num[j] = fmaf(f, base[w * hpw * ROWF + j], num[j]);
             }
-            emit((hg * hpw + hl) * p.n_rep + rep0 + r, d, num, s_M[h * ROWS + hl], s_den[h * ROWS + hl]);
+            emit((hg * hpw + hl) * p.n_rep + rep0 + r, d, num, s_M[h * rows + hl], s_den[h * rows + hl]);
         }
     }
     __syncthreads();
 }
 
+template <typename KV, int D, int NREP, typename Emit>
+__device__ __forceinline__ void merge_rows(RowState<NREP, RowShape<KV, D>::EPL> &st, float *s_part,
+                                           const PoolArgs &p, int wave, int tid, int hg,
+                                           int rep0, Emit emit) {
+    using S = RowShape<KV, D>;
+    using MS = MergeShape<KV, D, NREP>;
+    // (from an index that the compiler knows nothing of: places in LDS that it works out ahead of the key loop take registers
+    // that the loop does not have)
+    asm volatile("" : "+v"(tid));
+    const LaneRole role = lane_role<KV, D>(tid & (PA_WAVE - 1), p);
+    st.fold_zero_keys();
+    // The token rows of a wave first, lane against lane; the rows that are left go through LDS, as many more query heads at
+    // once as there are fewer of them.
+    if (p.tpw >= 2) merge_lanes(st, p.hpw * S::LPR);
+    const int prow = wave * p.hpw + role.head_local;
+    if (MS::HR < NREP && p.tpw >= 4)
+        merge_rounds<KV, D, NREP, (MS::HR * 4 < NREP ? MS::HR * 4 : NREP)>(st, s_part, p, role, prow, tid, hg, rep0, emit);
+    else if (MS::HR < NREP && p.tpw == 2)
+        merge_rounds<KV, D, NREP, (MS::HR * 2 < NREP ? MS::HR * 2 : NREP)>(st, s_part, p, role, prow, tid, hg, rep0, emit);
+    else
+        merge_rounds<KV, D, NREP, MS::HR>(st, s_part, p, role, prow, tid, hg, rep0, emit);
+}
+
 // The partition arithmetic (which workgroup owns which blocks, where its partial goes) is in decode_plan.h.
 __device__ __forceinline__ int64_t unit_begin(int64_t w, int64_t total, int64_t grid) { return plan_unit_begin(w, total, grid); }
 __device__ __forceinline__ int owner_of(int64_t u, int64_t total, int64_t grid) { return plan_owner_of(u, total, grid); }
-__device__ __forceinline__ int effective_grid(int64_t total, int grid) { return plan_effective_grid(total, grid); }
-
 // Finish one (sequence, query head): fold `ez` extra all-zero keys into the
 // merged (num, M, den) and normalise.
 __device__ __forceinline__ float finish_row(float num, float M, float den, int ez) {
@@ -635,7 +691,7 @@ __device__ __forceinline__ int wave_inclusive_scan(int x, int lane) {
 // partial in slot (workgroup index + plane*batch + sequence), unique because
 // both terms only grow along the flattened order.
 template <typename KV, typename QT, int D, int NREP, int U>
-__global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs a) {
+__global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void decode_split_kernel(const DecodeArgs a) {
     using S = RowShape<KV, D>;
     extern __shared__ int s_prefix[];  // batch + 1 entries: blocks before each sequence
     __shared__ int s_scan[kThreads];
@@ -648,7 +704,9 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
     const int wave = __builtin_amdgcn_readfirstlane(tid / PA_WAVE);
     const int B = a.batch;
 
-    // ---- block prefix sum over the batch --------------------------------
+    const int planes = p.n_hgroups * p.n_rgroups;
+    int run = 1;  // blocks of a unit
+    // ---- prefix sum of units over the batch -----------------------------
     // blocks of sequence b that hold visible keys: [first_key(b) / bs, ceil(L / bs))
     auto blocks_of = [&](int b) { return plan_blocks_of(a.seq_lens[b], p.bs, p.window); };
     if (B <= kWaveScanBatch) {
@@ -662,14 +720,21 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
             const int b = c * PA_WAVE + lane;
             n[c] = c * PA_WAVE < B && b < B ? blocks_of(b) : 0;
         }
-        int carry = 0;
+        auto scan = [&](int u, bool keep) {
+            int carry = 0;
 #pragma unroll
-        for (int c = 0; c < kWaveScanBatch / PA_WAVE; ++c) {
-            if (c * PA_WAVE >= B) break;  // uniform
-            const int x = wave_inclusive_scan(n[c], lane);
-            if (c * PA_WAVE + lane < B) s_prefix[c * PA_WAVE + lane] = carry + x - n[c];
-            carry += __builtin_amdgcn_readlane(x, PA_WAVE - 1);
-        }
+            for (int c = 0; c < kWaveScanBatch / PA_WAVE; ++c) {
+                if (c * PA_WAVE >= B) break;  // uniform
+                const int r = plan_runs_of(n[c], u), x = wave_inclusive_scan(r, lane);
+                if (keep && c * PA_WAVE + lane < B) s_prefix[c * PA_WAVE + lane] = carry + x - r;
+                carry += __builtin_amdgcn_readlane(x, PA_WAVE - 1);
+            }
+            return carry;
+        };
+        int carry = scan(1, true);
+        run = plan_run_blocks((int64_t)carry * planes, (int64_t)planes * B, (int)gridDim.x,
+                              [&](int u) { return (int64_t)scan(u, false) * planes; });
+        if (run > 1) carry = scan(run, true);
         if (lane == 0) s_prefix[B] = carry;
         if (blockIdx.x == 0 && wave == 0)
             for (int b = lane; b <= B; b += PA_WAVE) a.block_prefix[b] = s_prefix[b];
@@ -686,10 +751,10 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
             s_scan[tid] += add;
             __syncthreads();
         }
-        int run = s_scan[tid] - sum;  // exclusive
+        int before = s_scan[tid] - sum;  // exclusive
         for (int b = lo; b < hi; ++b) {
-            s_prefix[b] = run;
-            run += blocks_of(b);
+            s_prefix[b] = before;
+            before += blocks_of(b);
         }
         if (tid == kThreads - 1) s_prefix[B] = s_scan[tid];
         __syncthreads();
@@ -697,7 +762,6 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
             for (int b = tid; b <= B; b += kThreads) a.block_prefix[b] = s_prefix[b];
     }
     const int64_t per_plane = s_prefix[B];
-    const int planes = p.n_hgroups * p.n_rgroups;
     const int64_t total = per_plane * planes;
     const LaneRole role = lane_role<KV, D>(lane, p);
     if (a.merge_in_split) {
@@ -709,12 +773,12 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
         }
     }
     if (total == 0) return;
-    const int grid = effective_grid(total, (int)gridDim.x);
+    const int grid = plan_run_grid(total, (int)gridDim.x);
     if ((int)blockIdx.x >= grid) return;  // uniform
 
     int64_t cur = unit_begin(blockIdx.x, total, grid);
     const int64_t end = unit_begin((int64_t)blockIdx.x + 1, total, grid);
-    const bool by_chunk = total <= (int64_t)kChunkDealUnits * grid;  // short launches: see attend_blocks_pk
+    const bool by_chunk = total * run <= (int64_t)kChunkDealUnits * grid;  // short launches: see attend_blocks_pk
     while (cur < end) {
         const int plane = (int)(cur / per_plane);
         const int off = (int)(cur - plane * per_plane);
@@ -724,9 +788,9 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
             if (s_prefix[mid] <= off) lo = mid; else hi = mid;
         }
         const int b = lo;
-        const int nblk = s_prefix[b + 1] - s_prefix[b];
-        const int blk0 = off - s_prefix[b];
-        const int blk1 = (int)min((int64_t)nblk, blk0 + (end - cur));
+        const int n_units = s_prefix[b + 1] - s_prefix[b];
+        const int unit0 = off - s_prefix[b];
+        const int unit1 = (int)min((int64_t)n_units, unit0 + (end - cur));
         const int hg = plane % p.n_hgroups;
         const int rg = plane / p.n_hgroups;
         const int kvh = hg * p.hpw + role.head_local;
@@ -734,15 +798,16 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
         const int L = a.seq_lens[b];
         const int k_lo = window_first_key(p, L);  // the query sits at position L-1
         const int fb = k_lo / p.bs;               // first block with a visible key
+        const int blk0 = unit0 * run, blk1 = min(unit1 * run, plan_blocks_of(L, p.bs, p.window));
 
         RowState<NREP, S::EPL> st = Attender<KV, QT, D, NREP, U>::run(
             p, reinterpret_cast<const QT *>(a.q) + (int64_t)b * p.hq * p.d, p.bt + (int64_t)b * p.bt_stride, k_lo, L,
             fb + blk0, fb + blk1, wave, kWaves, by_chunk, role, lane, kvh, rep0);
-        if (blk0 == 0 && blk1 == nblk) {
+        if (unit0 == 0 && unit1 == n_units) {
             // the whole sequence is ours: write the output row
             const int ez = a.extra_zero ? max(0, a.extra_zero[b]) : 0;
             QT *orow = reinterpret_cast<QT *>(a.out) + (int64_t)b * p.hq * p.d;
-            merge_rows<KV, D, NREP>(st, s_part, p, role, wave, tid, hg, rep0,
+            merge_rows<KV, D, NREP>(st, s_part, p, wave, tid, hg, rep0,
                                     [&](int qh, int d, const float (&num)[4], float M, float den) {
                                         if (d >= p.d) return;
 #pragma unroll
@@ -755,7 +820,7 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
             if (slot < a.slot_cap) {  // never write outside the workspace
                 float *acc = a.part_acc + slot * (p.hpw * NREP * D);
                 float *ml = a.part_ml + slot * (p.hpw * NREP * 2);
-                merge_rows<KV, D, NREP>(st, s_part, p, role, wave, tid, hg, rep0,
+                merge_rows<KV, D, NREP>(st, s_part, p, wave, tid, hg, rep0,
                                         [&](int qh, int d, const float (&num)[4], float M, float den) {
                                             const int kv = qh / p.n_rep;
                                             const int idx = (kv - hg * p.hpw) * NREP + (qh - kv * p.n_rep - rep0);
@@ -781,11 +846,11 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(const DecodeArgs
                 // the 256-sequence launch).
                 const int64_t u0 = plane * per_plane + s_prefix[b];
                 const PieceRef piece = {plane, b, hg, rep0, owner_of(u0, total, grid),
-                                        owner_of(u0 + nblk - 1, total, grid)};
+                                        owner_of(u0 + n_units - 1, total, grid)};
                 deliver_piece<QT, D, NREP>(a, piece, &s_last, tid);
             }
         }
-        cur += blk1 - blk0;
+        cur += unit1 - unit0;
     }
 }
 
@@ -822,12 +887,12 @@ __global__ __launch_bounds__(kThreads) void decode_reduce_kernel(const DecodeArg
         return;
     }
     const int64_t u0 = plane * per_plane + a.block_prefix[b];
-    const int grid = effective_grid(total, a.split_grid);
+    const int grid = plan_run_grid(total, a.split_grid);
     const int w0 = owner_of(u0, total, grid), w1 = owner_of(u0 + nblk - 1, total, grid);
     if (w0 == w1) return;  // finished by the split pass
     const int64_t key = (int64_t)plane * a.batch + b;
     const int stride_acc = p.hpw * NREP * D, stride_ml = p.hpw * NREP * 2;
-    // every taking-part workgroup has units (effective_grid never exceeds the number of units), so every index
+    // every taking-part workgroup has units (there are never more workgroups than units), so every index
     // in [w0, w1] left a partial unless its slot fell outside the workspace
     const int v = tid % V4, pl = tid / V4;
     float M = kNegBig, den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
@@ -915,7 +980,7 @@ __global__ __launch_bounds__(kThreads) void decode_reduce_wave_kernel(const Deco
         return;
     }
     const int64_t u0 = plane * per_plane + a.block_prefix[b];
-    const int grid = effective_grid(total, a.split_grid);
+    const int grid = plan_run_grid(total, a.split_grid);
     const int w0 = owner_of(u0, total, grid), w1 = owner_of(u0 + nblk - 1, total, grid);
     if (w0 == w1) return;  // finished by the split pass
     const int64_t key = (int64_t)plane * a.batch + b;
@@ -991,7 +1056,7 @@ __global__ __launch_bounds__(kThreads) void prefill_rowwise_kernel(const Rowwise
         p, reinterpret_cast<const QT *>(a.q) + qrow * p.hq * p.d, p.bt + (int64_t)b * p.bt_stride, k_lo, L,
         k_lo / p.bs, nblk, wave, kWaves, false, role, lane, kvh, rep0);
     QT *orow = reinterpret_cast<QT *>(a.out) + qrow * p.hq * p.d;
-    merge_rows<KV, D, NREP>(st, s_part, p, role, wave, tid, hg, rep0,
+    merge_rows<KV, D, NREP>(st, s_part, p, wave, tid, hg, rep0,
                             [&](int qh, int d, const float (&num)[4], float M, float den) {
                                 if (d >= p.d) return;
 #pragma unroll

@@ -93,6 +93,26 @@ PA_PLAN_FN int plan_effective_grid(int64_t total, int grid) {
     return g < 1 ? 1 : (g < grid ? (int)g : grid);
 }
 
+// Short launches are flattened in runs of u blocks of one (plane, sequence) instead of single blocks, with a workgroup per
+// run: what a workgroup spends is a chain of waits per sequence that it touches (5 to 10 us), hardly more for one block of
+// it than for eight, so a range that crosses from one sequence into the next takes twice as long.  Returns u: the smallest of
+// 1, 2, 4 with which the runs fit the grid, 4 where (plane, sequence) pairs have many blocks (hundreds of one-block partials
+// of a pair would take longer to merge than they save); else 1, and the ranges of plan_unit_begin.  units(u): the runs of u
+// blocks of the launch.  Ranges of at least four blocks took 20.7 us for 4 sequences of 100 keys at 32 / 8 heads of 128, runs
+// take 13.9; 31 -> 14 us for 256 sequences of 16 keys; at 14 / 2 heads of 64, 4 sequences of 16 keys 52.6 -> 13.7, 16 of 1000
+// keys 31 -> 17, 4 of 6000 keys 33 -> 20.  (Single blocks for one sequence of 6000 keys: 20 us at 8 / 2 heads of 128, runs of
+// four 15; hence the line at 48 blocks per pair.)
+constexpr int kPlanRunMost = 4, kPlanShortBlocks = 48;
+template <typename F> PA_PLAN_FN int plan_run_blocks(int64_t total, int64_t keys, int grid, F units) {
+    if (total > (int64_t)kPlanRunMost * grid) return 1;
+    for (int u = total > keys * kPlanShortBlocks ? kPlanRunMost : 1; u <= kPlanRunMost; u *= 2)
+        if (units(u) <= grid) return u;
+    return 1;
+}
+PA_PLAN_FN int plan_runs_of(int blocks, int u) { return (blocks + u - 1) / u; }
+// Workgroups that take part in a launch of `total` runs.
+PA_PLAN_FN int plan_run_grid(int64_t total, int grid) { return total < grid ? (int)total : grid; }
+
 // Partial slot of the piece of (plane, sequence) that workgroup w computed: unique, because along the flattened
 // order both w and plane*batch + sequence only grow.
 PA_PLAN_FN int64_t plan_slot(int w, int plane, int batch, int b) { return (int64_t)w + (int64_t)plane * batch + b; }

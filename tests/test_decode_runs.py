@@ -1,0 +1,76 @@
+"""Short launches of the split pass: runs of blocks, one workgroup each (``plan_run_blocks`` of ``decode_plan.h``, compiled with
+g++).  Every (plane, sequence, block) lies in one run of one workgroup, and where the runs fit the grid no workgroup has two."""
+
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = """
+#include <vector>
+#include "decode_plan.h"
+using namespace pa_decode_detail;
+extern "C" int replay(const int *lens, int batch, int planes, int bs, int window, int grid) {
+    auto runs = [&](int u) { int64_t n = 0; for (int b = 0; b < batch; ++b) n += plan_runs_of(plan_blocks_of(lens[b], bs, window), u); return n * planes; };
+    const int64_t blocks = runs(1);
+    const int u = plan_run_blocks(blocks, (int64_t)planes * batch, grid, runs);
+    const int64_t total = runs(u), per_plane = total / planes;
+    if (total == 0) return u;
+    const int taking = plan_run_grid(total, grid);
+    std::vector<std::vector<int>> seen((size_t)planes * batch);
+    for (int i = 0; i < planes * batch; ++i) seen[i].resize(plan_blocks_of(lens[i % batch], bs, window));
+    for (int w = 0; w < taking; ++w) {
+        const int64_t lo = plan_unit_begin(w, total, taking), hi = plan_unit_begin(w + 1, total, taking);
+        if (hi <= lo || (u > 1 && hi != lo + 1)) return -1;
+        for (int64_t x = lo; x < hi; ++x) {
+            if (plan_owner_of(x, total, taking) != w) return -2;
+            int64_t off = x % per_plane;
+            int b = 0;
+            for (int n; off >= (n = plan_runs_of(plan_blocks_of(lens[b], bs, window), u)); ++b) off -= n;
+            std::vector<int> &s = seen[x / per_plane * batch + b];
+            for (int64_t k = off * u; k < (off + 1) * u && k < (int64_t)s.size(); ++k) ++s[k];
+        }
+    }
+    for (auto &s : seen) for (int n : s) if (n != 1) return -3;
+    return u;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def replay(tmp_path_factory):
+    at = tmp_path_factory.mktemp("runs")
+    (at / "r.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "research_amd", "csrc"), "-o", str(at / "r.so"),
+                    str(at / "r.cpp")], check=True)
+    fn = ctypes.CDLL(str(at / "r.so")).replay
+    fn.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 5
+
+    def run(lens, planes, bs=16, window=0, grid=512):
+        lens = np.ascontiguousarray(lens, np.int32)
+        return fn(lens.ctypes.data, len(lens), planes, bs, window, grid)
+    return run
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_every_block_lies_in_one_run(replay, seed):
+    rng = np.random.default_rng(seed)
+    taken = set()
+    for _ in range(300):
+        batch = int(rng.integers(1, 65))
+        lens = np.exp(rng.uniform(0, np.log(rng.choice([40, 600, 8000])), batch)).astype(int) - 1  # (some are empty)
+        u = replay(lens, int(rng.choice([1, 2, 4])), int(rng.choice([1, 16, 32])), int(rng.choice([0, 0, 100, -64])), int(rng.choice([2, 64, 512])))
+        assert u in (1, 2, 4)
+        taken.add(u)
+    assert taken == {1, 2, 4}
+
+
+def test_lines_of_the_rule(replay):
+    assert replay([16] * 512, 1) == 1 and replay([32] * 256, 1) == 1    # a run per block fills the grid
+    assert replay([32] * 512, 1) == 2 and replay([64] * 512, 1) == 4    # two, four blocks each
+    assert replay([80] * 512, 1) == 1                                   # more than the grid takes in runs of four
+    assert replay([768], 1) == 1 and replay([784], 1) == 4              # 48 and 49 blocks of a sequence
+    assert replay([0, 0], 2) == 1
