@@ -512,7 +512,7 @@ int pa_qkv_conv_append(const void *u, int64_t u_stride, int64_t n_rows, const fl
  *   dim <= 256, any vdim
  * pa_lightning_recurrent walks a portion token by token (decode steps; 32-bit prompts).  pa_lightning_chunked
  * (PA_BF16) multiplies 64 rows at a time on the matrix cores, with the 32-bit factors split into two bf16 terms; given
- * a workspace it cuts long portions of small batches into segments that run at the same time.  max_q_len: at least
+ * a workspace it cuts long portions of small or unequal batches into segments that run at the same time.  max_q_len: at least
  * the longest portion.
  */
 size_t pa_lightning_state_floats(int dim, int vdim);
@@ -553,7 +553,7 @@ int pa_short_conv(const void *u, int64_t u_stride, int64_t n_rows, const float *
  *   out           : [n_rows][heads * vdim] of dtype;  dim <= 256, any vdim
  * Single rows (q_lens NULL), PA_F32 and rows that are not whole 8-byte vectors run token by token; PA_BF16 portions in
  * chunks of 64 rows on the matrix cores, with the 32-bit factors split into two bf16 terms, and, given a workspace, in
- * segments that run at the same time when there are few sequences.  max_q_len: at least the longest portion.
+ * segments that run at the same time when there are few sequences or unequal ones.  max_q_len: at least the longest portion.
  */
 size_t pa_gated_linear_state_floats(int kind, int dim, int vdim);
 size_t pa_gated_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len);

@@ -200,7 +200,9 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     ClPortion p;
     if (!cl_portion(a, b, p)) return;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
-    if (r_beg >= p.n) return;
+    // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
+    const bool last = r_end == p.n;
+    if (r_beg >= p.n || (STATES && last)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int v0 = vsl * L::cols, vw = wave * 16;  // first column of the workgroup, of the wave inside it
     const int l16 = lane & 15, g = lane >> 4;
@@ -427,7 +429,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
             for (int blk = 0; blk < L::blocks; ++blk) decayed *= whole[blk * KD + tid];
         __syncthreads();  // the next rows' operands may be written now
     }
-    float *to = STATES ? seg_state : (a.segments > 1 ? nullptr : pool);
+    float *to = STATES ? seg_state : last ? pool : nullptr;
     if (!to) return;
     const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc((void *)to, 0, state_bytes, 0x00020000);
 #pragma unroll
@@ -440,7 +442,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     if (STATES && vsl == 0 && tid < KD && tid < a.dp) to[state_elems + tid] = decayed;  // (every value slice has the same)
 }
 
-// Segment contributions -> start states, in place; the state after the last segment goes back to the pool.
+// Segment contributions -> start states, in place.
 __global__ __launch_bounds__(256) void channel_scan_kernel(const ClArgs a) {
     const int h = blockIdx.y, b = blockIdx.z;
     ClPortion p;
@@ -448,18 +450,19 @@ __global__ __launch_bounds__(256) void channel_scan_kernel(const ClArgs a) {
     const int64_t n4 = (int64_t)a.dp * a.vp / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
     const int d = (int)(i * 4 / a.vp);
-    float *pool = p.slot >= 0 ? a.state + (p.slot * a.heads + h) * 4 * n4 : nullptr;
+    const float *pool = p.slot >= 0 && p.pos0 > 0 ? a.state + (p.slot * a.heads + h) * 4 * n4 : nullptr;
     const int64_t stride = 4 * n4 + a.dp + 16;
     float *seg = a.ws + ((int64_t)b * a.heads + h) * a.segments * stride;
-    float4 cur = pool && p.pos0 > 0 ? reinterpret_cast<const float4 *>(pool)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int j = 0; (int64_t)j * a.seg_rows < p.n; ++j, seg += stride) {
-        const float keep = seg[4 * n4 + d];
-        float4 *at = reinterpret_cast<float4 *>(seg) + i;
-        const float4 add = *at;
-        *at = cur;
+    const int segments = (p.n + a.seg_rows - 1) / a.seg_rows;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 next = segments > 1 ? reinterpret_cast<const float4 *>(seg)[i] : zero, cur = pool ? reinterpret_cast<const float4 *>(pool)[i] : zero;
+    for (int j = 0; j < segments; ++j, seg += stride) {
+        const float4 add = next;
+        if (j + 2 < segments) next = reinterpret_cast<const float4 *>(seg + stride)[i];
+        const float keep = j + 1 < segments ? seg[4 * n4 + d] : 1.f;
+        reinterpret_cast<float4 *>(seg)[i] = cur;
         cur = make_float4(fmaf(keep, cur.x, add.x), fmaf(keep, cur.y, add.y), fmaf(keep, cur.z, add.z), fmaf(keep, cur.w, add.w));
     }
-    if (pool) reinterpret_cast<float4 *>(pool)[i] = cur;
 }
 
 template <int KD, int NW> int launch_chunks(const ClArgs &a, int batch, hipStream_t s) {
@@ -487,10 +490,7 @@ template <typename T> void launch_recurrent(const ClArgs &a, int batch, hipStrea
     else channel_recurrent_kernel<T, 16><<<grid, block, 0, s>>>(a);
 }
 
-int cl_plan(int64_t batch, int heads, int vdim, int max_q_len) {
-    const int cols = la_value_cols(vdim);
-    return la_segments(batch * heads * ((vdim + cols - 1) / cols), la_cus(), max_q_len);
-}
+size_t cl_segment_bytes(int64_t batch, int heads, int dim, int vdim) { return gl_workspace_bytes(batch, heads, dim, vdim, 2) / 2; }
 
 }  // namespace
 
@@ -500,7 +500,7 @@ extern "C" size_t pa_channel_linear_workspace_bytes(int batch, int num_heads, in
         pa_fail(PA_ERR_INVALID_ARG, "pa_channel_linear_workspace_bytes: sizes out of range");
         return 0;
     }
-    return gl_workspace_bytes(batch, num_heads, dim, vdim, cl_plan(batch, num_heads, vdim, max_q_len));
+    return gl_workspace_bytes(batch, num_heads, dim, vdim, la_most_segments(cl_segment_bytes(batch, num_heads, dim, vdim), max_q_len));
 }
 
 extern "C" int pa_channel_linear(const void *q, int64_t q_stride, int q_act, const void *forget, int64_t f_stride, const float *f_bias,
@@ -539,12 +539,13 @@ extern "C" int pa_channel_linear(const void *q, int64_t q_stride, int q_act, con
         PA_CHECK_LAUNCH("pa_channel_linear");
         return PA_OK;
     }
-    a.segments = cl_plan(batch, num_heads, vdim, max_q_len);
-    while (a.segments > 1 && (!workspace || gl_workspace_bytes(batch, num_heads, dim, vdim, a.segments) > workspace_bytes))
-        --a.segments;
+    const int cols = la_value_cols(vdim);
+    a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(), 0.0, max_q_len, n_rows,
+                                    cl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
+                                    pa_aligned16(workspace));
+    PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
     a.seg_rows = la_segment_rows(max_q_len, a.segments);
     a.ws = (float *)workspace;
-    PA_REQUIRE(a.segments == 1 || pa_aligned16(workspace), "the workspace must be 16-byte aligned");
     const bool wide = la_value_cols(vdim) == 128;
     if (dim <= 64) return wide ? launch_chunks<64, 8>(a, batch, s) : launch_chunks<64, 4>(a, batch, s);
     if (dim <= 128) return wide ? launch_chunks<128, 8>(a, batch, s) : launch_chunks<128, 4>(a, batch, s);

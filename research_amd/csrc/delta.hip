@@ -151,9 +151,6 @@ template <typename T, int R> __global__ __launch_bounds__(256, 4) void delta_rec
 
 // ------------------------------------------------------------------ chunks: T and C
 constexpr int kDcPitch = 72;  // bf16 per row of T and C in LDS
-// Operands that meet a result as their partner have the inner order 4 g + 0 .. 3, 16 + 4 g + 0 .. 3 within 32: stored in that
-// order, a lane's eight elements are one 16-byte chunk.  Position of element c:
-__host__ __device__ constexpr int delta_paired(int c) { return (c & ~31) | (c & 12) << 1 | (c & 16) >> 2 | (c & 3); }
 struct DeltaChunk {           // what the first pass leaves per chunk and head (columns of T and C paired)
     uint16_t t_hi[64][64], t_lo[64][64], c_hi[64][64], c_lo[64][64];
     float k_in[64];   // e^F times k's unit factor (on K S)
@@ -202,8 +199,8 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
             const int blk = tid + 256 * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
             const LaBlock x = la_load_block(tq, la_block_off(a.ldq, r, c, a.dim), (uint32_t)a.ldq * 2u);
             const LaBlock y = la_load_block(tk, la_block_off(a.ldk, r, c, a.dim), (uint32_t)a.ldk * 2u);
-            la_put_block<false>(x, r, c, q_s, kLd, nullptr);
-            la_put_block<false>(y, r, c, k_s, kLd, nullptr);
+            la_put_block<false>(x, r, c, q_s, kLd);
+            la_put_block<false>(y, r, c, k_s, kLd);
         }
     }
     if (wave == 0) {
@@ -276,8 +273,8 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
         uint2 hi, lo;
         la_split2(c[0], c[1], hi.x, lo.x);
         la_split2(c[2], c[3], hi.y, lo.y);
-        *reinterpret_cast<uint2 *>(&out->c_hi[t][delta_paired(16 * st + 4 * g)]) = hi;
-        *reinterpret_cast<uint2 *>(&out->c_lo[t][delta_paired(16 * st + 4 * g)]) = lo;
+        *reinterpret_cast<uint2 *>(&out->c_hi[t][la_paired(16 * st + 4 * g)]) = hi;
+        *reinterpret_cast<uint2 *>(&out->c_lo[t][la_paired(16 * st + 4 * g)]) = lo;
     }
     // (the wave's own 16 rows of mat: its accesses are in order, the compiler must keep them so)
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -324,33 +321,14 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
         uint2 hi, lo;
         la_split2(x[0], x[1], hi.x, lo.x);
         la_split2(x[2], x[3], hi.y, lo.y);
-        *reinterpret_cast<uint2 *>(&out->t_hi[r][delta_paired(c)]) = hi;
-        *reinterpret_cast<uint2 *>(&out->t_lo[r][delta_paired(c)]) = lo;
+        *reinterpret_cast<uint2 *>(&out->t_hi[r][la_paired(c)]) = hi;
+        *reinterpret_cast<uint2 *>(&out->t_lo[r][la_paired(c)]) = lo;
     }
 }
 
 // ------------------------------------------------------------------ chunks: the walk
-// Tiles of Q and K: paired columns, chunk c of row r at position c ^ delta_hash(r).  Operand reads (16 rows, one chunk) and
-// transposing reads (four rows, four chunks) both spread over the banks.
-template <int KD> __device__ __forceinline__ int delta_hash(int r) { return (KD == 64 ? (r & 2) << 1 : (r & 3) << 2) | (r >> 2 & 3); }
-template <int KD> __device__ __forceinline__ void delta_put(const LaBlock &b, int r, int c, __bf16 *tile) {
-    const int e = delta_paired(c);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(tile + (r + i) * KD + (((e >> 3) ^ delta_hash<KD>(r + i)) << 3) + (e & 4)) = b.r[i];
-}
-
 template <int KD, int COLS> constexpr size_t delta_walk_lds() {
     return (size_t)(2 * 64 * KD + 64 * (COLS + 8) + 4 * 64 * kDcPitch) * 2 + 3 * 64 * 4 + 64;
-}
-
-// Two bf16 terms of eight values of a result tile pair, as an operand whose inner index runs 4 g + 0 .. 3, then 16 more
-__device__ __forceinline__ LaSplit delta_split(const f4 &x, const f4 &y) {
-    LaSplit s;
-    la_split2(x[0], x[1], s.hi[0], s.lo[0]);
-    la_split2(x[2], x[3], s.hi[1], s.lo[1]);
-    la_split2(y[0], y[1], s.hi[2], s.lo[2]);
-    la_split2(y[2], y[3], s.hi[3], s.lo[3]);
-    return s;
 }
 
 // KD: dim padded to 64, 128 or 256.  A workgroup of NW waves owns 16 NW value columns of a head and all chunks of a portion.
@@ -423,13 +401,13 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
         for (int i = 0; i < kKB; ++i) {
             const int blk = tid + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
             if (!k_live) continue;
-            delta_put<KD>(qb[i], r, c, q_s);
-            delta_put<KD>(kb[i], r, c, k_s);
+            la_put_paired<false, KD>(qb[i], r, c, q_s);
+            la_put_paired<false, KD>(kb[i], r, c, k_s);
         }
 #pragma unroll
         for (int i = 0; i < kVB; ++i) {
             const int blk = tid + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
-            la_put_block<false>(vb[i], r, c, v_s, kLv, nullptr);
+            la_put_block<false>(vb[i], r, c, v_s, kLv);
         }
 #pragma unroll
         for (int i = 0; i < kMB; ++i) {
@@ -450,12 +428,11 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
         for (int tt = 0; tt < 4; ++tt) u[tt] = o[tt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int dd = 0; dd < KD / 32; ++dd) {
-            const LaSplit sp = delta_split(s[2 * dd], s[2 * dd + 1]);
+            const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) {
-                const int at = (16 * tt + l16) * KD + ((4 * dd + g) ^ delta_hash<KD>(l16)) * 8;
-                const bf8 xk = la_read8(k_s + at), xq = la_read8(q_s + at);
+                const bf8 xk = la_read_paired<KD>(k_s, 16 * tt + l16, l16, dd, g), xq = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
                 u[tt] = la_mfma(xk, hi, u[tt]);
                 u[tt] = la_mfma(xk, lo, u[tt]);
                 o[tt] = la_mfma(hi, xq, o[tt]);
@@ -479,7 +456,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
         for (int tt = 0; tt < 4; ++tt) w[tt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const LaSplit sp = delta_split(u[2 * kk], u[2 * kk + 1]);
+            const LaSplit sp = la_split_pair(u[2 * kk], u[2 * kk + 1]);
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
             for (int tt = 2 * kk; tt < 4; ++tt) {
@@ -498,7 +475,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             {
-                const LaSplit sp = delta_split(w[2 * kk], w[2 * kk + 1]);
+                const LaSplit sp = la_split_pair(w[2 * kk], w[2 * kk + 1]);
                 const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
                 for (int tt = 2 * kk; tt < 4; ++tt) {
@@ -515,13 +492,11 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
 #pragma unroll
                 for (int i = 0; i < 4; ++i) w[2 * kk + half][i] *= ko[i];
             }
-            const LaSplit sp = delta_split(w[2 * kk], w[2 * kk + 1]);
+            const LaSplit sp = la_split_pair(w[2 * kk], w[2 * kk + 1]);
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
             for (int dt = 0; dt < KD / 16; ++dt) {
-                const int row = 4 * g + l16 / 4;
-                const __bf16 *at = k_s + (32 * kk + row) * KD + ((dt / 2 * 4 + l16 % 4) ^ delta_hash<KD>(row)) * 8 + dt % 2 * 4;
-                const bf8 xk = la_join(la_read_tr(at), la_read_tr(at + 16 * KD));
+                const bf8 xk = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
                 s[dt] = la_mfma(xk, hi, s[dt]);
                 s[dt] = la_mfma(xk, lo, s[dt]);
             }

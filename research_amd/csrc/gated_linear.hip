@@ -12,7 +12,8 @@
 // M the running maximum of i - F (kSsd: i = 0 and M = 0; b stays a factor), both from one wave's prefix scans,
 //     O = diag(e^(F_t or m0 - M_t)) Q S + ((Q K^T) * e^(F_t - F_s or i_s - F_s - M_t) b_s, s <= t) V
 // and the state moves on by the same weights at the chunk's last row.  All logarithms are to base 2.
-// n is followed by the vector units; its product with q and the sums of the weighted scores give the denominators.
+// n follows by the same products, with the weights as three bf16 terms (all 24 bits); its product with q, by the vector units,
+// and the sums of the weighted scores give the denominators.
 #include "linear_tiles.h"
 
 namespace {
@@ -190,13 +191,11 @@ struct GlRows {
     float whole, pad[15];             // factor on the old state
 };
 
-// Elements of the tiles: Q and K row-major, the two terms of the weighted scores, the transposed K and V.
-template <int KD> constexpr int gl_r_elems() { return 64 * (KD + 8); }
-constexpr int kGlAElems = 2 * 64 * kLaPitchA;
-template <int KD, int NW> constexpr int gl_t_elems() { return (KD + 16 * NW) * 64; }
+// Elements of the tiles: K and Q (paired), V (row-major), the two terms of the weighted scores.
+template <int KD, int NW> constexpr int gl_kv_elems() { return 64 * KD + 64 * (16 * NW + 8); }
 template <int KD, int NW, int KIND, bool STATES> constexpr size_t gl_lds_bytes() {
-    const size_t elems = STATES ? 2 * gl_t_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
-                                : 2 * gl_r_elems<KD>() + kGlAElems + gl_t_elems<KD, NW>();
+    const size_t elems = STATES ? 2 * gl_kv_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
+                                : gl_kv_elems<KD, NW>() + 64 * KD + 2 * 64 * kLaPitchA;
     return elems * 2 + (STATES ? 2 : 1) * sizeof(GlRows) + (KIND == kMlstm && !STATES ? (3 * 64 + KD) * 4 : 0);
 }
 
@@ -227,25 +226,29 @@ __device__ __forceinline__ float gl_scan_max(float x, int lane) {
 // KD: dim padded to 64, 128 or 256.  NW: waves; each owns 16 value columns.  All products are taken transposed (value
 // columns, or keys, as the rows of the result), so that a lane holds four consecutive elements of one row t.
 // STATES: only the segment's own contribution to the state, to the workspace (first pass over a portion in segments).
+// The tiles and the two passes as in lightning attention's kernel.  One prompt of 15999 rows, 4 heads of 256 x 512 (mLSTM):
+// 181 -> 172 us for the second pass, 68 -> 71 for the first; 128 prompts of 16 .. 130 rows (SSD, 64 heads of 128 x 64) 178 -> 172.
 template <int KD, int NW, int KIND, bool STATES>
 __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_chunk_kernel(const GlArgs a) {
-    constexpr int kCols = 16 * NW, kLdR = KD + 8, kThr = 64 * NW;
+    constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
+    constexpr int kNd = (KD / 32 + NW - 1) / NW;  // kMlstm: 32-row pieces of n per wave
     extern __shared__ __align__(16) char lds[];
     GlRows *rows = reinterpret_cast<GlRows *>(lds);
     float *nq_s = reinterpret_cast<float *>(rows + (STATES ? 2 : 1));  // kMlstm: n . q per row, two parts of the score sums, n
     float *sum_s = nq_s + 64, *n_s = sum_s + 128;
     __bf16 *tiles = reinterpret_cast<__bf16 *>(KIND == kMlstm && !STATES ? n_s + KD : nq_s);
-    __bf16 *kt_s = tiles, *vt_s = kt_s + KD * 64;
-    __bf16 *q_s = tiles + gl_t_elems<KD, NW>(), *k_s = q_s + gl_r_elems<KD>(), *a_hi = k_s + gl_r_elems<KD>();
-    __bf16 *a_lo = a_hi + 64 * kLaPitchA;
+    __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
+    __bf16 *q_s = tiles + gl_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
     const int h = blockIdx.x, seg = blockIdx.y % a.segments, vsl = blockIdx.y / a.segments, b = blockIdx.z;
     GlPortion p;
     if (!gl_portion(a, b, p)) return;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
-    if (r_beg >= p.n) return;
+    // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
+    const bool last = r_end == p.n;
+    if (r_beg >= p.n || (STATES && last)) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int v0 = vsl * kCols, vw = wave * 16;  // first column of the workgroup, of the wave inside it
     const int l16 = tid & 15, g = (tid & 63) >> 4;
@@ -270,16 +273,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             for (int i = 0; i < 4; ++i)
                 s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + (16 * dt + i) * a.vp * 4, 0, 0));
     }
-    // n and m of the workgroup: thread d follows n[d], the first wave m
+    // n and m of the workgroup: a wave follows its 32-row pieces of n (n[j][e][i]: row 32 (kNd wave + j) + 16 e + 4 g + i, the
+    // same in all columns), the first wave m
     const int rep0 = v0 / kRecCols;
-    float n_own = 0.f, m_prev = STATES ? kGlNone : 0.f, decayed = 0.f;
-    if constexpr (KIND == kMlstm && !STATES) {
+    f4 n[KIND == kMlstm ? kNd : 1][2];
+    float m_prev = STATES ? kGlNone : 0.f, decayed = 0.f;
+    auto n_row = [&](int j, int e) { return 32 * (kNd * wave + j) + 16 * e + 4 * g; };
+    if constexpr (KIND == kMlstm) {
         const float *np = from ? from + state_elems + (a.segments > 1 ? 0 : rep0 * (a.dp + 16)) : nullptr;
-        if (np) {
-            if (tid < a.dp && tid < KD) n_own = np[tid];
-            m_prev = a.segments > 1 ? np[a.dp + 2] : np[a.dp];
-        }
-        if (tid < KD) n_s[tid] = n_own;
+#pragma unroll
+        for (int j = 0; j < kNd; ++j)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                n[j][e] = f4{0.f, 0.f, 0.f, 0.f};
+                if (np && n_row(j, e) < a.dp) n[j][e] = *reinterpret_cast<const f4 *>(np + n_row(j, e));
+                if (!STATES && l16 == 0 && n_row(j, e) < KD) *reinterpret_cast<f4 *>(n_s + la_paired(n_row(j, e))) = n[j][e];
+            }
+        if (np) m_prev = a.segments > 1 ? np[a.dp + 2] : np[a.dp];
     }
 
     const int grp = h / a.per_group;
@@ -319,14 +329,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     fetch(r_beg);
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
+        const int lt = la_again(tid);
 #pragma unroll
         for (int i = 0; i < kKPass; ++i) {
-            const int blk = tid + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
+            const int blk = lt + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
             if (kKBlocks % kThr != 0 && blk >= kKBlocks) continue;
-            la_put_block<false>(kb[i], sr, c, STATES ? nullptr : k_s, kLdR, kt_s);
-            if (!STATES) la_put_block<false>(qb[i], sr, c, q_s, kLdR, nullptr);
+            la_put_paired<false, KD>(kb[i], sr, c, k_s);
+            if (!STATES) la_put_paired<false, KD>(qb[i], sr, c, q_s);
         }
-        la_put_block<false>(vb, tid / (kCols / 4) * 4, tid % (kCols / 4) * 4, nullptr, 0, vt_s);
+        la_put_block<false>(vb, lt / (kCols / 4) * 4, lt % (kCols / 4) * 4, v_s, kLdV);
         if (wave == 0) {  // the chunk's gates, one row per lane
             float decay, in;
             gl_gate<KIND>(a, hd, raw_a, raw_b, decay, in);
@@ -356,6 +367,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
         if (r0 + kLaChunk < r_end) fetch(r0 + kLaChunk);
         __syncthreads();
 
+        const int lr = KD == 256 ? la_again(tid) : tid, l16 = lr & 15, g = (lr & 63) >> 4;
         f4 o[4];  // O^T: v = 4 g + i of the wave's columns, t = 16 tt + l16
         if constexpr (!STATES) {
             // score tiles (st, rt): keys 16 st + 4 g + i, rows 16 rt + l16
@@ -365,11 +377,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             for (int m = 0; m < kST; ++m) sc[m] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kk = 0; kk < KD / 32; ++kk) {
-                const bf8 bq = la_read8(q_s + (16 * rt + l16) * kLdR + 32 * kk + 8 * g);
+                const bf8 bq = la_read_paired<KD>(q_s, 16 * rt + l16, l16, kk, g);
 #pragma unroll
                 for (int m = 0; m < kST; ++m) {
                     const int st = NW == 8 ? 2 * m + (wave & 1) : m;
-                    if (st <= rt) sc[m] = la_mfma(la_read8(k_s + (16 * st + l16) * kLdR + 32 * kk + 8 * g), bq, sc[m]);
+                    if (st <= rt) sc[m] = la_mfma(la_read_paired<KD>(k_s, 16 * st + l16, l16, kk, g), bq, sc[m]);
                 }
             }
             // the rows' part from before the chunk: Q S, then its factors
@@ -377,15 +389,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             for (int tt = 0; tt < 4; ++tt) o[tt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int dd = 0; dd < KD / 32; ++dd) {
-                LaSplit sp;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    la_split2(s[2 * dd + j / 2][2 * j % 4], s[2 * dd + j / 2][2 * j % 4 + 1], sp.hi[j], sp.lo[j]);
+                const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
                 const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
                 for (int tt = 0; tt < 4; ++tt) {
-                    const __bf16 *qr = q_s + (16 * tt + l16) * kLdR + 32 * dd + 4 * g;
-                    const bf8 bq = la_read44(qr, qr + 16);
+                    const bf8 bq = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
                     o[tt] = la_mfma(hi, bq, o[tt]);
                     o[tt] = la_mfma(lo, bq, o[tt]);
                 }
@@ -398,15 +406,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             }
             if constexpr (KIND == kMlstm) {  // n . q: NW lanes per row
                 const int t = tid / NW;
-                constexpr int kPer = KD / NW;
-                const __bf16 *qr = q_s + t * kLdR + tid % NW * kPer;
-                const float *nr = n_s + tid % NW * kPer;
+                constexpr int kPer = KD / NW / 8;  // 16-byte chunks of Q, whose order n_s has as well
                 float acc = 0.f;
 #pragma unroll
-                for (int d = 0; d < kPer; d += 8) {
-                    const bf8 x = la_read8(qr + d);
+                for (int d = tid % NW * kPer; d < tid % NW * kPer + kPer; ++d) {
+                    const bf8 x = la_read8(q_s + t * KD + (d ^ la_hash<KD>(t)) * 8);
+                    const float *nr = n_s + 8 * d;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) acc = fmaf((float)x[j], nr[d + j], acc);
+                    for (int j = 0; j < 8; ++j) acc = fmaf((float)x[j], nr[j], acc);
                 }
                 acc = pa_group_sum<NW>(acc);
                 if (tid % NW == 0) nq_s[t] = acc;
@@ -434,8 +441,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
                 uint2 hi, lo;
                 la_split2(x[0], x[1], hi.x, lo.x);
                 la_split2(x[2], x[3], hi.y, lo.y);
-                *reinterpret_cast<uint2 *>(a_hi + t * kLaPitchA + c) = hi;
-                *reinterpret_cast<uint2 *>(a_lo + t * kLaPitchA + c) = lo;
+                *reinterpret_cast<uint2 *>(a_hi + t * kLaPitchA + la_paired(c)) = hi;
+                *reinterpret_cast<uint2 *>(a_lo + t * kLaPitchA + la_paired(c)) = lo;
             }
             if constexpr (KIND == kMlstm) {
                 sum += __shfl_xor(sum, 16, 64);
@@ -446,7 +453,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             __syncthreads();
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                const bf8 av = la_read8(vt_s + la_tr(vw + l16, 32 * kk + 8 * g));
+                const bf8 av = la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g);
 #pragma unroll
                 for (int tt = 2 * kk; tt < 4; ++tt) {
                     o[tt] = la_mfma(av, la_read8(a_hi + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
@@ -475,46 +482,57 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
         for (int dt = 0; dt < KD / 16; ++dt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
+        if constexpr (KIND == kMlstm) {
+#pragma unroll
+            for (int j = 0; j < kNd; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    n[j][0][i] *= whole;
+                    n[j][1][i] *= whole;
+                }
+        }
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            LaSplit sp;
-            const la_u4 bv = *reinterpret_cast<const la_u4 *>(vt_s + la_tr(vw + l16, 32 * kk + 8 * g));
-            const f4 w0 = *reinterpret_cast<const f4 *>(rows->add + 32 * kk + 8 * g);
-            const f4 w1 = *reinterpret_cast<const f4 *>(rows->add + 32 * kk + 8 * g + 4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t pair = bv[j];
-                la_split2(__builtin_bit_cast(float, pair << 16) * (j < 2 ? w0 : w1)[2 * j % 4],
-                          __builtin_bit_cast(float, pair & 0xffff0000u) * (j < 2 ? w0 : w1)[2 * j % 4 + 1], sp.hi[j], sp.lo[j]);
-            }
+            const f4 w0 = *reinterpret_cast<const f4 *>(rows->add + 32 * kk + 4 * g), w1 = *reinterpret_cast<const f4 *>(rows->add + 32 * kk + 16 + 4 * g);
+            const LaSplit sp = la_split_weighted(la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g), w0, w1);
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
             for (int dt = 0; dt < KD / 16; ++dt) {
-                const bf8 ak = la_read8(kt_s + la_tr(16 * dt + l16, 32 * kk + 8 * g));
+                const bf8 ak = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
                 s[dt] = la_mfma(ak, hi, s[dt]);
                 s[dt] = la_mfma(ak, lo, s[dt]);
             }
-        }
-        if (KIND == kMlstm && tid < KD) {  // n likewise, with k alone
-            float acc = whole * n_own;
+            if constexpr (KIND == kMlstm) {  // n likewise, with k alone: the weights in every column
+                const LaSplit3 ones = la_split3(w0, w1);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const bf8 x = la_read8(kt_s + la_tr(tid, 8 * c));
+                for (int j = 0; j < kNd; ++j) {
+                    const int piece = kNd * wave + j;
+                    if (piece >= KD / 32) break;  // (uniform)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc = fmaf(rows->add[8 * c + j], (float)x[j], acc);
+                    for (int e = 0; e < 2; ++e) {
+                        const bf8 ak = la_read_paired_tr<KD>(k_s, 32 * kk, 2 * piece + e, l16, g);
+#pragma unroll
+                        for (int x = 0; x < 3; ++x) n[j][e] = la_mfma(ak, ones.term[x], n[j][e]);
+                    }
+                }
             }
-            n_own = acc;
-            if (!STATES) n_s[tid] = acc;  // (read again after the next chunk's first barrier)
+        }
+        if constexpr (KIND == kMlstm && !STATES) {
+#pragma unroll
+            for (int j = 0; j < kNd; ++j)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)  // (read again after the next chunk's first barrier)
+                    if (l16 == 0 && n_row(j, e) < KD) *reinterpret_cast<f4 *>(n_s + la_paired(n_row(j, e))) = n[j][e];
         }
         if constexpr (!STATES) {
             __syncthreads();  // the next chunk's tiles and gates may be written now
         } else {              // the other half of the tiles and gates
-            kt_s = kt_s == tiles ? tiles + gl_t_elems<KD, NW>() : tiles;
-            vt_s = kt_s + KD * 64;
+            k_s = k_s == tiles ? tiles + gl_kv_elems<KD, NW>() : tiles;
+            v_s = k_s + 64 * KD;
             rows = rows == reinterpret_cast<GlRows *>(lds) ? rows + 1 : reinterpret_cast<GlRows *>(lds);
         }
     }
-    float *to = STATES ? seg_state : (a.segments > 1 ? nullptr : pool);
+    float *to = STATES ? seg_state : last ? pool : nullptr;
     if (!to) return;
     const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc((void *)to, 0, state_bytes, 0x00020000);
     uint32_t base = soff;
@@ -526,9 +544,18 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             const float f = s[dt][i];
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), dst, base + (16 * dt + i) * a.vp * 4, 0, 0);
         }
+    auto put_n = [&](float *np) {
+        if constexpr (KIND == kMlstm) {
+#pragma unroll
+            for (int j = 0; j < kNd; ++j)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    if (l16 == 0 && n_row(j, e) < a.dp) *reinterpret_cast<f4 *>(np + n_row(j, e)) = n[j][e];
+        }
+    };
     if constexpr (STATES) {  // (every value slice has the same n, m and decay)
         if (vsl != 0) return;
-        if (KIND == kMlstm && tid < a.dp && tid < KD) to[state_elems + tid] = n_own;
+        put_n(to + state_elems);
         if (tid == 0) {
             to[state_elems + a.dp] = m_prev;
             to[state_elems + a.dp + 1] = decayed;
@@ -537,56 +564,47 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
         const int reps = (a.vdim + kRecCols - 1) / kRecCols;
         for (int r = rep0; r < reps && r < rep0 + (kCols + kRecCols - 1) / kRecCols; ++r) {
             float *np = to + state_elems + r * (a.dp + 16);
-            if (tid < a.dp && tid < KD) np[tid] = n_own;
+            put_n(np);
             if (tid == 0) np[a.dp] = m_prev;
         }
     }
 }
 
-// Segment contributions -> start states, in place; the state after the last segment goes back to the pool.  One thread per
-// four elements of S, then of n; the first of n's threads also writes m.
+// Segment contributions -> start states, in place.  One thread per four elements of S, then of n; the first of n's threads
+// also writes m.
 template <int KIND> __global__ __launch_bounds__(256) void gated_scan_kernel(const GlArgs a) {
     const int h = blockIdx.y, b = blockIdx.z;
     GlPortion p;
     if (!gl_portion(a, b, p)) return;
     const int64_t n4 = (int64_t)a.dp * a.vp / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool of_n = i >= n4;
     if (i >= n4 + (KIND == kMlstm ? a.dp / 4 : 0)) return;
-    float *pool = p.slot >= 0 ? a.state + (p.slot * a.heads + h) * a.head_floats : nullptr;
+    const float *pool = p.slot >= 0 && p.pos0 > 0 ? a.state + (p.slot * a.heads + h) * a.head_floats : nullptr;
     const int64_t stride = 4 * n4 + a.dp + 16;
     float *seg = a.ws + ((int64_t)b * a.heads + h) * a.segments * stride;
-    const bool resume = pool && p.pos0 > 0;
-    float4 cur = resume ? reinterpret_cast<const float4 *>(pool)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    float m = KIND == kMlstm && resume ? pool[4 * n4 + a.dp] : 0.f;
-    for (int j = 0; (int64_t)j * a.seg_rows < p.n; ++j, seg += stride) {
-        const float decay = seg[4 * n4 + a.dp + 1];
-        float keep, take = 1.f, next = 0.f;
-        if (KIND == kMlstm) {
-            const float m_seg = seg[4 * n4 + a.dp];
-            next = fmaxf(decay + m, m_seg);
-            keep = exp2f(decay + m - next);
-            take = exp2f(m_seg - next);
-        } else {
-            keep = exp2f(decay);
+    const int segments = (p.n + a.seg_rows - 1) / a.seg_rows;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 next = segments > 1 ? reinterpret_cast<const float4 *>(seg)[i] : zero, cur = pool ? reinterpret_cast<const float4 *>(pool)[i] : zero;
+    float m = KIND == kMlstm && pool ? pool[4 * n4 + a.dp] : 0.f;
+    for (int j = 0; j < segments; ++j, seg += stride) {
+        const float4 add = next;
+        if (j + 2 < segments) next = reinterpret_cast<const float4 *>(seg + stride)[i];
+        float keep = 1.f, take = 1.f, m_next = 0.f;
+        if (j + 1 < segments) {
+            const float decay = seg[4 * n4 + a.dp + 1];
+            if (KIND == kMlstm) {
+                const float m_seg = seg[4 * n4 + a.dp];
+                m_next = fmaxf(decay + m, m_seg);
+                keep = exp2f(decay + m - m_next);
+                take = exp2f(m_seg - m_next);
+            } else {
+                keep = exp2f(decay);
+            }
         }
-        float4 *at = reinterpret_cast<float4 *>(seg) + i;
-        const float4 add = *at;
-        *at = cur;
+        reinterpret_cast<float4 *>(seg)[i] = cur;
         if (KIND == kMlstm && i == n4) seg[4 * n4 + a.dp + 2] = m;
         cur = make_float4(fmaf(keep, cur.x, take * add.x), fmaf(keep, cur.y, take * add.y), fmaf(keep, cur.z, take * add.z),
                           fmaf(keep, cur.w, take * add.w));
-        m = next;
-    }
-    if (!pool) return;
-    if (!of_n) {
-        reinterpret_cast<float4 *>(pool)[i] = cur;
-        return;
-    }
-    const int reps = (a.vdim + kRecCols - 1) / kRecCols;
-    for (int r = 0; r < reps; ++r) {
-        float *np = pool + 4 * n4 + (int64_t)r * (a.dp + 16);
-        reinterpret_cast<float4 *>(np)[i - n4] = cur;
-        if (i == n4) np[a.dp] = m;
+        m = m_next;
     }
 }
 
@@ -622,11 +640,7 @@ template <typename T, int KIND> void launch_recurrent(const GlArgs &a, int batch
     else gated_recurrent_kernel<T, 16, KIND><<<grid, block, 0, s>>>(a);
 }
 
-int gl_plan(int64_t batch, int heads, int dim, int vdim, int max_q_len) {
-    const int cols = la_value_cols(vdim);
-    const int at_once = cols == 64 && dim <= 128 ? 2 * la_cus() : la_cus();  // workgroups: two of four waves fit a compute unit
-    return la_segments(batch * heads * ((vdim + cols - 1) / cols), at_once, max_q_len);
-}
+size_t gl_segment_bytes(int64_t batch, int heads, int dim, int vdim) { return gl_workspace_bytes(batch, heads, dim, vdim, 2) / 2; }
 
 }  // namespace
 
@@ -640,7 +654,7 @@ extern "C" size_t pa_gated_linear_workspace_bytes(int batch, int num_heads, int 
         pa_fail(PA_ERR_INVALID_ARG, "pa_gated_linear_workspace_bytes: sizes out of range");
         return 0;
     }
-    return gl_workspace_bytes(batch, num_heads, dim, vdim, gl_plan(batch, num_heads, dim, vdim, max_q_len));
+    return gl_workspace_bytes(batch, num_heads, dim, vdim, la_most_segments(gl_segment_bytes(batch, num_heads, dim, vdim), max_q_len));
 }
 
 extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const void *k, int64_t k_stride, const void *v,
@@ -695,11 +709,13 @@ extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const 
         PA_CHECK_LAUNCH("pa_gated_linear");
         return PA_OK;
     }
-    a.segments = gl_plan(batch, num_heads, dim, vdim, max_q_len);
-    while (a.segments > 1 && (!workspace || gl_workspace_bytes(batch, num_heads, dim, vdim, a.segments) > workspace_bytes))
-        --a.segments;
+    const int cols = la_value_cols(vdim);  // (two workgroups of four waves share a compute unit)
+    a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(),
+                                    cols == 64 && dim <= 128 ? 1.25 : 0.0, max_q_len, n_rows,
+                                    gl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
+                                    pa_aligned16(workspace));
+    PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
     a.seg_rows = la_segment_rows(max_q_len, a.segments);
     a.ws = (float *)workspace;
-    PA_REQUIRE(a.segments == 1 || pa_aligned16(workspace), "the workspace must be 16-byte aligned");
     return kind == kSsd ? launch_chunks_kind<kSsd>(a, batch, s) : launch_chunks_kind<kMlstm>(a, batch, s);
 }

@@ -118,23 +118,27 @@ template <typename T, int R> __global__ __launch_bounds__(256) void lightning_re
 }
 
 // ------------------------------------------------------------------ chunks on the matrix cores
-// Elements of the tiles: Q and K row-major, the two terms of the decayed scores, the transposed K and V, the output.
-template <int KD> constexpr int la_r_elems() { return 64 * (KD + 8); }
-constexpr int kLaAElems = 2 * 64 * kLaPitchA;
-template <int KD, int NW> constexpr int la_t_elems() { return (KD + 16 * NW) * 64; }
-template <int NW> constexpr int la_o_elems() { return 64 * (16 * NW + 8); }
+// Elements of the tiles: K and Q (paired), V (row-major), the two terms of the decayed scores.
+template <int KD, int NW> constexpr int la_kv_elems() { return 64 * KD + 64 * (16 * NW + 8); }
 template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
-    const size_t elems = STATES ? 2 * la_t_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
-                                : 2 * la_r_elems<KD>() + kLaAElems + la_t_elems<KD, NW>() + la_o_elems<NW>();
+    const size_t elems = STATES ? 2 * la_kv_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
+                                : la_kv_elems<KD, NW>() + 64 * KD + 2 * 64 * kLaPitchA;
     return elems * 2 + (64 + 64 + 64 + 80) * 4;
 }
 
 // KD: dim padded to 64, 128 or 256.  NW: waves; each owns 16 value columns.  All products are taken transposed (value
 // columns, or keys, as the rows of the result), so that a lane holds four consecutive elements of one row t.
 // STATES: only the segment's own contribution to the state, to the workspace (first pass over a portion in segments).
+// Bound by the vector instructions that turn 32-bit factors into two bf16 terms and by the waits between the stages of a chunk
+// (the matrix cores are busy a sixth of the time).  So a tile lies in LDS in the one layout that both of its products read (K by
+// rows and, with transposing reads, by columns), results leave the registers straight for the output, and the first pass leaves out
+// each portion's last segment, whose state the second pass itself writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128:
+// first pass 55 -> 48 us, second 127 -> 101, with five segments of unequal sequences instead of two.
+// (At dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
+// chunk, let two share one, which was 10 % faster where there were two and 3 to 8 % slower where not.)
 template <int KD, int NW, bool STATES>
 __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArgs a) {
-    constexpr int kCols = 16 * NW, kLdR = KD + 8, kLdO = kCols + 8, kThr = 64 * NW;
+    constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     extern __shared__ __align__(16) char lds[];
@@ -142,15 +146,16 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
     float *rev_tail = rev + 64;                   // ... and of a portion's last chunk
     float *pw = rev + 192;                        // powers 0 .. 64, behind 64 zeros for the keys after a row
     __bf16 *tiles = reinterpret_cast<__bf16 *>(rev + 272);
-    __bf16 *kt_s = tiles, *vt_s = kt_s + KD * 64;
-    __bf16 *q_s = tiles + la_t_elems<KD, NW>(), *k_s = q_s + la_r_elems<KD>(), *a_hi = k_s + la_r_elems<KD>();
-    __bf16 *a_lo = a_hi + 64 * kLaPitchA, *o_s = a_hi + kLaAElems;
+    __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
+    __bf16 *q_s = tiles + la_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
     const int h = blockIdx.x, seg = blockIdx.y % a.segments, vsl = blockIdx.y / a.segments, b = blockIdx.z;
     Portion p;
     if (!la_portion(a, b, p)) return;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
-    if (r_beg >= p.n) return;
+    // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
+    const bool last = r_end == p.n;
+    if (r_beg >= p.n || (STATES && last)) return;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int v0 = vsl * kCols, vw = wave * 16;  // first column of the workgroup, of the wave inside it
     const float *powers = a.decay + h * (kLaChunk + 1);
@@ -190,37 +195,36 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
     const int vcols = a.vdim - v0 < kCols ? a.vdim - v0 : kCols;
     const uint32_t row_bytes = (uint32_t)a.ldu * 2u;
     LaBlock kb[kKPass], qb[STATES ? 1 : kKPass], vb;
-    uint32_t koff[kKPass];
-#pragma unroll
-    for (int i = 0; i < kKPass; ++i) {
-        const int blk = tid + kThr * i;
-        koff[i] = blk < kKBlocks ? la_block_off(a.ldu, blk / kDB * 4, blk % kDB * 4, a.dim) : kLaOutside;
-    }
-    const uint32_t voff = la_block_off(a.ldu, tid / (kCols / 4) * 4, tid % (kCols / 4) * 4, vcols);
     auto fetch = [&](int r0) {
         const int rows = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
         const int64_t at = (int64_t)r0 * a.ldu;
+        const int ft = la_again(tid);
+        auto koff = [&](int i) {
+            const int blk = ft + kThr * i;
+            return blk < kKBlocks ? la_block_off(a.ldu, blk / kDB * 4, blk % kDB * 4, a.dim) : kLaOutside;
+        };
         const __amdgpu_buffer_rsrc_t tk = la_tile(uk + at, a.ldu, rows, a.dim), tv = la_tile(uv + at, a.ldu, rows, vcols);
         if (!STATES) {
             const __amdgpu_buffer_rsrc_t tq = la_tile(uq + at, a.ldu, rows, a.dim);
 #pragma unroll
-            for (int i = 0; i < kKPass; ++i) qb[i] = la_load_block(tq, koff[i], row_bytes);
+            for (int i = 0; i < kKPass; ++i) qb[i] = la_load_block(tq, koff(i), row_bytes);
         }
 #pragma unroll
-        for (int i = 0; i < kKPass; ++i) kb[i] = la_load_block(tk, koff[i], row_bytes);
-        vb = la_load_block(tv, voff, row_bytes);
+        for (int i = 0; i < kKPass; ++i) kb[i] = la_load_block(tk, koff(i), row_bytes);
+        vb = la_load_block(tv, la_block_off(a.ldu, ft / (kCols / 4) * 4, ft % (kCols / 4) * 4, vcols), row_bytes);
     };
     fetch(r_beg);
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
+        const int lt = la_again(tid);
 #pragma unroll
         for (int i = 0; i < kKPass; ++i) {
-            const int blk = tid + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
+            const int blk = lt + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
             if (kKBlocks % kThr != 0 && blk >= kKBlocks) continue;
-            la_put_block<true>(kb[i], sr, c, STATES ? nullptr : k_s, kLdR, kt_s);
-            if (!STATES) la_put_block<true>(qb[i], sr, c, q_s, kLdR, nullptr);
+            la_put_paired<true, KD>(kb[i], sr, c, k_s);
+            if (!STATES) la_put_paired<true, KD>(qb[i], sr, c, q_s);
         }
-        la_put_block<true>(vb, tid / (kCols / 4) * 4, tid % (kCols / 4) * 4, nullptr, 0, vt_s);
+        la_put_block<true>(vb, lt / (kCols / 4) * 4, lt % (kCols / 4) * 4, v_s, kLdV);
         if (nv < kLaChunk && tid < 64) rev_tail[tid] = tid < nv ? powers[nv - 1 - tid] : 0.f;
         if (r0 + kLaChunk < r_end) fetch(r0 + kLaChunk);
         __syncthreads();
@@ -234,11 +238,11 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
             for (int m = 0; m < kST; ++m) sc[m] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kk = 0; kk < KD / 32; ++kk) {
-                const bf8 bq = la_read8(q_s + (16 * rt + l16) * kLdR + 32 * kk + 8 * g);
+                const bf8 bq = la_read_paired<KD>(q_s, 16 * rt + l16, l16, kk, g);
 #pragma unroll
                 for (int m = 0; m < kST; ++m) {
                     const int st = NW == 8 ? 2 * m + (wave & 1) : m;
-                    if (st <= rt) sc[m] = la_mfma(la_read8(k_s + (16 * st + l16) * kLdR + 32 * kk + 8 * g), bq, sc[m]);
+                    if (st <= rt) sc[m] = la_mfma(la_read_paired<KD>(k_s, 16 * st + l16, l16, kk, g), bq, sc[m]);
                 }
             }
             // the rows' part from before the chunk: Q S, then the decay of the way from the chunk's start
@@ -246,15 +250,11 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
             for (int tt = 0; tt < 4; ++tt) o[tt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int dd = 0; dd < KD / 32; ++dd) {
-                LaSplit sp;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    la_split2(s[2 * dd + j / 2][2 * j % 4], s[2 * dd + j / 2][2 * j % 4 + 1], sp.hi[j], sp.lo[j]);
+                const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
                 const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
                 for (int tt = 0; tt < 4; ++tt) {
-                    const __bf16 *qr = q_s + (16 * tt + l16) * kLdR + 32 * dd + 4 * g;
-                    const bf8 bq = la_read44(qr, qr + 16);
+                    const bf8 bq = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
                     o[tt] = la_mfma(hi, bq, o[tt]);
                     o[tt] = la_mfma(lo, bq, o[tt]);
                 }
@@ -272,23 +272,27 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
                 uint2 hi, lo;
                 la_split2(sc[m][0] * f[0], sc[m][1] * f[-1], hi.x, lo.x);
                 la_split2(sc[m][2] * f[-2], sc[m][3] * f[-3], hi.y, lo.y);
-                *reinterpret_cast<uint2 *>(a_hi + t * kLaPitchA + c) = hi;
-                *reinterpret_cast<uint2 *>(a_lo + t * kLaPitchA + c) = lo;
+                *reinterpret_cast<uint2 *>(a_hi + t * kLaPitchA + la_paired(c)) = hi;
+                *reinterpret_cast<uint2 *>(a_lo + t * kLaPitchA + la_paired(c)) = lo;
             }
             __syncthreads();
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                const bf8 av = la_read8(vt_s + la_tr(vw + l16, 32 * kk + 8 * g));
+                const bf8 av = la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g);
 #pragma unroll
                 for (int tt = 2 * kk; tt < 4; ++tt) {
                     o[tt] = la_mfma(av, la_read8(a_hi + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
                     o[tt] = la_mfma(av, la_read8(a_lo + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
                 }
             }
+            const int ldo = a.heads * a.vdim, c = vw + 4 * g;
+            const uint16_t *first = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0) * (int64_t)ldo + h * a.vdim + v0;
+            const __amdgpu_buffer_rsrc_t dst = la_tile(first, ldo, nv, vcols);
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)  // to LDS, so that rows are stored 16 bytes per lane
-                *reinterpret_cast<uint2 *>(o_s + (16 * tt + l16) * kLdO + vw + 4 * g) =
-                    make_uint2(row_pack_bf16(o[tt][0], o[tt][1]), row_pack_bf16(o[tt][2], o[tt][3]));
+            for (int tt = 0; tt < 4; ++tt) {
+                const la_u2 x = {row_pack_bf16(o[tt][0], o[tt][1]), row_pack_bf16(o[tt][2], o[tt][3])};
+                __builtin_amdgcn_raw_buffer_store_b64(x, dst, c < vcols ? (uint32_t)((16 * tt + l16) * ldo + c) * 2u : kLaOutside, 0, 0);
+            }
         }
         // S <- decay^nv S + K^T (decay^(nv-1-s) V)
         const float whole = pw[nv];
@@ -299,43 +303,24 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
             for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            LaSplit sp;
-            const la_u4 bv = *reinterpret_cast<const la_u4 *>(vt_s + la_tr(vw + l16, 32 * kk + 8 * g));
-            const f4 w0 = *reinterpret_cast<const f4 *>(wt + 32 * kk + 8 * g);
-            const f4 w1 = *reinterpret_cast<const f4 *>(wt + 32 * kk + 8 * g + 4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t pair = bv[j];
-                la_split2(__builtin_bit_cast(float, pair << 16) * (j < 2 ? w0 : w1)[2 * j % 4],
-                          __builtin_bit_cast(float, pair & 0xffff0000u) * (j < 2 ? w0 : w1)[2 * j % 4 + 1], sp.hi[j], sp.lo[j]);
-            }
+            const LaSplit sp = la_split_weighted(la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g), *reinterpret_cast<const f4 *>(wt + 32 * kk + 4 * g),
+                                                 *reinterpret_cast<const f4 *>(wt + 32 * kk + 16 + 4 * g));
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
             for (int dt = 0; dt < KD / 16; ++dt) {
-                const bf8 ak = la_read8(kt_s + la_tr(16 * dt + l16, 32 * kk + 8 * g));
+                const bf8 ak = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
                 s[dt] = la_mfma(ak, hi, s[dt]);
                 s[dt] = la_mfma(ak, lo, s[dt]);
             }
         }
         if constexpr (!STATES) {
-            __syncthreads();
-            const int ldo = a.heads * a.vdim;
-            const uint16_t *first = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0) * (int64_t)ldo + h * a.vdim + v0;
-            const __amdgpu_buffer_rsrc_t dst = la_tile(first, ldo, nv, vcols);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {  // (64 rows of kCols columns are two 16-byte vectors per thread)
-                const int vec = tid + kThr * i, t = vec / (kCols / 8), c = vec % (kCols / 8) * 8;
-                const la_u4 x = *reinterpret_cast<const la_u4 *>(o_s + t * kLdO + c);
-                __builtin_amdgcn_raw_buffer_store_b128(x, dst, c < vcols ? (uint32_t)(t * ldo + c) * 2u : kLaOutside, 0, 0);
-            }
-            // (the next chunk's tiles may be written now: their readers are past the barrier above, and its scores and
-            // output come behind barriers of its own)
-        } else {  // the other half of the tiles
-            kt_s = kt_s == tiles ? tiles + la_t_elems<KD, NW>() : tiles;
-            vt_s = kt_s + KD * 64;
+            __syncthreads();  // the next chunk's tiles may be written now
+        } else {              // the other half of the tiles
+            k_s = k_s == tiles ? tiles + la_kv_elems<KD, NW>() : tiles;
+            v_s = k_s + 64 * KD;
         }
     }
-    float *to = STATES ? seg_state : (a.segments > 1 ? nullptr : pool);
+    float *to = STATES ? seg_state : last ? pool : nullptr;
     if (!to) return;
     const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc((void *)to, 0, state_bytes, 0x00020000);
     uint32_t base = soff;
@@ -349,31 +334,26 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
         }
 }
 
-// Segment contributions -> start states, in place; the state after the last segment goes back to the pool.
+// Segment contributions -> start states, in place.  A chain of one load per segment, so the next one is in flight.
 __global__ __launch_bounds__(256) void lightning_scan_kernel(const LaArgs a) {
     const int h = blockIdx.y, b = blockIdx.z;
     Portion p;
     if (!la_portion(a, b, p)) return;
     const int64_t n4 = (int64_t)a.dp * a.vp / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
-    float4 *pool = p.slot >= 0 ? reinterpret_cast<float4 *>(a.state) + (p.slot * a.heads + h) * n4 + i : nullptr;
+    const float4 *pool = p.slot >= 0 && p.pos0 > 0 ? reinterpret_cast<const float4 *>(a.state) + (p.slot * a.heads + h) * n4 + i : nullptr;
     float4 *seg = reinterpret_cast<float4 *>(a.ws) + ((int64_t)b * a.heads + h) * a.segments * n4 + i;
-    float4 cur = pool && p.pos0 > 0 ? *pool : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float *pw = a.decay + h * (kLaChunk + 1);
-    float whole = 1.f;  // decay^seg_rows, seg_rows a multiple of the chunk
-    for (int c = 0; c < a.seg_rows / kLaChunk; ++c) whole *= pw[kLaChunk];
-    for (int j = 0; j * a.seg_rows < p.n; ++j) {
-        float f = whole;
-        const int left = p.n - j * a.seg_rows;
-        if (left < a.seg_rows) {
-            f = pw[left % kLaChunk];
-            for (int c = 0; c < left / kLaChunk; ++c) f *= pw[kLaChunk];
-        }
-        const float4 add = seg[j * n4];
+    const int segments = (p.n + a.seg_rows - 1) / a.seg_rows;
+    float4 next = segments > 1 ? *seg : make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 cur = pool ? *pool : make_float4(0.f, 0.f, 0.f, 0.f);
+    float f = 1.f;  // decay^seg_rows, seg_rows a multiple of the chunk
+    for (int c = 0; c < a.seg_rows / kLaChunk; ++c) f *= a.decay[h * (kLaChunk + 1) + kLaChunk];
+    for (int j = 0; j < segments; ++j) {
+        const float4 add = next;
+        if (j + 2 < segments) next = seg[(j + 1) * n4];
         seg[j * n4] = cur;
         cur = make_float4(fmaf(f, cur.x, add.x), fmaf(f, cur.y, add.y), fmaf(f, cur.z, add.z), fmaf(f, cur.w, add.w));
     }
-    if (pool) *pool = cur;
 }
 
 template <int KD, int NW> int launch_chunks(const LaArgs &a, int batch, hipStream_t s) {
@@ -423,11 +403,7 @@ int la_fill(const char *what, LaArgs &a, const void *u, int64_t u_stride, int64_
     return PA_OK;
 }
 
-int la_plan(int64_t batch, int heads, int dim, int vdim, int max_q_len) {
-    (void)dim;
-    const int cols = la_value_cols(vdim);
-    return la_segments(batch * heads * ((vdim + cols - 1) / cols), la_cus(), max_q_len);
-}
+size_t la_segment_bytes(int64_t batch, int heads, int dim, int vdim) { return la_workspace_bytes(batch, heads, dim, vdim, 2) / 2; }
 
 }  // namespace
 
@@ -458,7 +434,7 @@ extern "C" size_t pa_lightning_workspace_bytes(int batch, int num_heads, int dim
         pa_fail(PA_ERR_INVALID_ARG, "pa_lightning_workspace_bytes: sizes out of range");
         return 0;
     }
-    return la_workspace_bytes(batch, num_heads, dim, vdim, la_plan(batch, num_heads, dim, vdim, max_q_len));
+    return la_workspace_bytes(batch, num_heads, dim, vdim, la_most_segments(la_segment_bytes(batch, num_heads, dim, vdim), max_q_len));
 }
 
 extern "C" int pa_lightning_chunked(const void *u, int64_t u_stride, int64_t n_rows, float *state, int64_t state_rows,
@@ -477,12 +453,14 @@ extern "C" int pa_lightning_chunked(const void *u, int64_t u_stride, int64_t n_r
         return rc;
     if (n_rows == 0 || batch == 0 || max_q_len == 0) return PA_OK;
     PA_REQUIRE(q_lens, "NULL q_lens / q_starts");
-    a.segments = la_plan(batch, num_heads, dim, vdim, max_q_len);
-    while (a.segments > 1 && (!workspace || la_workspace_bytes(batch, num_heads, dim, vdim, a.segments) > workspace_bytes))
-        --a.segments;
+    const int cols = la_value_cols(vdim);
+    a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(),
+                                    cols == 64 && dim <= 128 ? 1.25 : dim <= 64 ? 1.6 : 0.0, max_q_len, n_rows,
+                                    la_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
+                                    pa_aligned16(workspace));
+    PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
     a.seg_rows = la_segment_rows(max_q_len, a.segments);
     a.ws = (float *)workspace;
-    PA_REQUIRE(a.segments == 1 || pa_aligned16(workspace), "the workspace must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     // rows that are not whole 16-byte vectors, or too far apart for a tile's 32-bit offsets: token by token
     if (dim % 8 != 0 || vdim % 8 != 0 || u_stride % 8 != 0 || !pa_aligned16(u) || !pa_aligned16(out) ||

@@ -26,6 +26,52 @@ static inline int la_segments(int64_t workgroups, int cus, int max_len) {
     return want < 1 ? 1 : (int)want;
 }
 
+// The same for a batch whose rows are known: `per_seq` workgroups for each sequence, n_rows rows in all; together: by how much
+// a workgroup is slower when two share a compute unit (0: they cannot).  In units of a chunk of the second pass: without
+// segments the launch lasts as long as its longest sequence or, with more workgroups than compute units, its share of the
+// rows; with segments of c chunks it lasts c where a compute unit has one of them at most, else its share and half a
+// segment, and 45 % more for the first pass, half a unit per segment for the scan between the two, and two units for the
+// launches.  Measured, 16 heads of 128 x 128 (lightning; HGRN2; mLSTM with 4 of 256 x 512), us, as many segments as
+// compute units / workgroups -> by this rule: 8 sequences of 400 .. 4000 rows 187 -> 128, 305 -> 216, 311 -> 249; 12 of them 239 ->
+// 161, 389 -> 284, 423 -> 341; 12 equal ones stay unsegmented (172, 276, 312; in segments 201, 354, 398).
+static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, int most) {
+    if (batch <= 0 || per_seq <= 0 || max_len <= 0) return 1;
+    if (n_rows > batch * max_len) n_rows = batch * max_len;
+    const int chunks = (max_len + kLaChunk - 1) / kLaChunk;
+    const double rows = (double)n_rows / kLaChunk, share = rows * per_seq / cus * (together > 0 ? together / 2 : 1.0);
+    double best = share > chunks ? share : chunks;
+    int segments = 1;
+    for (int s = 2; s <= most; ++s) {
+        const double c = (chunks + s - 1) / s;
+        const double spread = rows / c + 0.5 * batch, live = per_seq * (spread < (double)batch * s ? spread : (double)batch * s);
+        double part = c;
+        if (live > cus) part = live <= 2.0 * cus && together > 0 ? c * together : share + 0.5 * c;
+        if (part < c) part = c;
+        const double t = 1.45 * part + 0.5 * s + 2.0;
+        if (t < best) {
+            best = t;
+            segments = s;
+        }
+    }
+    return segments;
+}
+// Most segments: none shorter than kLaMinSegChunks chunks, and states of seg_bytes for each (of all sequences) that fit `room`.
+constexpr size_t kLaMostSegBytes = (size_t)256 << 20;
+static inline int la_most_segments(size_t seg_bytes, int max_len, size_t room = kLaMostSegBytes) {
+    const int most = la_segments(1, kLaMaxSegments, max_len);
+    if (room > kLaMostSegBytes) room = kLaMostSegBytes;
+    const int64_t fit = seg_bytes ? (int64_t)(room / seg_bytes) : most;
+    return fit < 1 ? 1 : fit < most ? (int)fit : most;
+}
+// Segments of a launch with a workspace of `room` bytes (0: none).  0: they would need the workspace, which is not aligned; a
+// batch that fills the device without segments takes such a workspace for none.
+static inline int la_launch_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows,
+                                     size_t seg_bytes, size_t room, bool aligned) {
+    const int most = la_most_segments(seg_bytes, max_len, room);
+    if (!aligned) return most > 1 && la_segments(batch * per_seq, cus, max_len) > 1 ? 0 : 1;
+    return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
+}
+
 // Rows per segment: whole chunks.
 static inline int la_segment_rows(int max_len, int segments) {
     const int chunks = (max_len + kLaChunk - 1) / kLaChunk;

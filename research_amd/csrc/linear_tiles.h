@@ -1,5 +1,5 @@
 // What the chunked linear-recurrence kernels share: 64-row tiles of bf16 rows loaded in 4 x 4 blocks and laid out in LDS
-// row-major and transposed, 32-bit factors as a sum of two bf16 terms, states as buffers.
+// so that operands are whole reads in either direction, 32-bit factors as a sum of two bf16 terms, states as buffers.
 #pragma once
 #include "lightning_plan.h"
 #include "row_common.h"
@@ -12,14 +12,20 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t la_u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t la_u4 __attribute__((ext_vector_type(4)));
 
-// LDS layouts.  Row-major [64][KD + 8] for Q and K (the pad moves a row by 16 bytes over the banks).  Transposed
-// [rows][64 s] for K^T and V^T: eight 16-byte chunks per row, chunk c of row r at position c ^ la_hash(r), so that
-// both the transposing 8-byte writes (rows 4 apart) and the 16-byte operand reads (consecutive rows) spread over the
-// banks without a pad.
-// (Of the row bits that change over the lanes of an access - 0 to 3 in reads, 2 to 6 in writes - bit 0 picks half of the
-// banks, and three more have to reach all eight chunks.)
-__device__ __forceinline__ int la_hash(int r) { return ((r >> 1) & 7) ^ ((r >> 4) & 1); }
-__device__ __forceinline__ int la_tr(int r, int s) { return r * 64 + ((((s >> 3) ^ la_hash(r)) << 3) | (s & 7)); }
+// x, as a value that the compiler knows nothing of: places in LDS that follow from it are worked out again in every chunk
+// instead of kept in registers over the loop.
+__device__ __forceinline__ int la_again(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// LDS tiles of Q and K: [64][KD], columns paired, 16-byte chunk c of row r at position c ^ la_hash(r).  Operands that meet a
+// result as their partner have the inner order 4 g + 0 .. 3, 16 + 4 g + 0 .. 3 within 32: stored in that order, a lane's
+// eight elements are one chunk, and four rows of a result's columns are one transposing read, so that no tile is stored
+// transposed as well (which took the conflicting 8-byte writes of a 64-row tile and its space in LDS).  Operand reads (16 rows,
+// one chunk) and transposing reads (four rows, four chunks) both spread over the banks.
+__host__ __device__ constexpr int la_paired(int c) { return (c & ~31) | (c & 12) << 1 | (c & 16) >> 2 | (c & 3); }
+template <int KD> __device__ __forceinline__ int la_hash(int r) { return (KD == 64 ? (r & 2) << 1 : (r & 3) << 2) | (r >> 2 & 3); }
 
 __device__ __forceinline__ f4 la_mfma(bf8 x, bf8 y, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0); }
 
@@ -48,11 +54,11 @@ struct LaBlock {  // four rows of four consecutive columns, raw bf16
     uint2 r[4];
 };
 
-// A tile of `rows` rows of `cols` columns at row stride `ld` as a buffer: loads past its end give zeros, stores past it
-// are dropped.  (Columns past `cols` inside a row are the caller's: it gives such lanes the offset kLaOutside.)
+// A tile of `rows` rows (none: 0 or less) of `cols` columns at row stride `ld` as a buffer: loads past its end give zeros,
+// stores past it are dropped.  (Columns past `cols` inside a row are the caller's: it gives such lanes the offset kLaOutside.)
 constexpr uint32_t kLaOutside = 0x40000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t la_tile(const uint16_t *base, int64_t ld, int rows, int cols) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)(((rows - 1) * ld + cols) * 2), 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, rows > 0 ? (int)(((rows - 1) * ld + cols) * 2) : 0, 0x00020000);
 }
 // Byte offset of the 4 x 4 block at (row s, column c)
 __device__ __forceinline__ uint32_t la_block_off(int64_t ld, int s, int c, int cols) {
@@ -74,24 +80,74 @@ __device__ __forceinline__ uint32_t la_silu2(uint32_t w) {
                          row_silu<pa_bf16>(__builtin_bit_cast(float, w & 0xffff0000u)));
 }
 
-// The block, or with ACT its silu, to a row-major tile (when `rm` is given) and, transposed, to a [column][64] tile
-template <bool ACT> __device__ __forceinline__ void la_put_block(LaBlock b, int s, int c, __bf16 *rm, int ld_rm, __bf16 *tr) {
+template <bool ACT> __device__ __forceinline__ void la_act_block(LaBlock &b) {
     if constexpr (ACT) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) b.r[i] = make_uint2(la_silu2(b.r[i].x), la_silu2(b.r[i].y));
     }
-    if (rm) {
+}
+// The block, or with ACT its silu, to a row-major tile, and to a paired one
+template <bool ACT> __device__ __forceinline__ void la_put_block(LaBlock b, int s, int c, __bf16 *rm, int ld_rm) {
+    la_act_block<ACT>(b);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(rm + (s + i) * ld_rm + c) = b.r[i];
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(rm + (s + i) * ld_rm + c) = b.r[i];
+}
+template <bool ACT, int KD> __device__ __forceinline__ void la_put_paired(LaBlock b, int r, int c, __bf16 *tile) {
+    la_act_block<ACT>(b);
+    const int e = la_paired(c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(tile + (r + i) * KD + (((e >> 3) ^ la_hash<KD>(r + i)) << 3) + (e & 4)) = b.r[i];
+}
+// Row `row` (row % 16 = l16) of a paired tile, elements of the 32 columns from 32 dd on
+template <int KD> __device__ __forceinline__ bf8 la_read_paired(const __bf16 *tile, int row, int l16, int dd, int g) {
+    return la_read8(tile + row * KD + ((4 * dd + g) ^ la_hash<KD>(l16)) * 8);
+}
+// Column 16 dt + l16 of rows first + 4 g + 0 .. 3 and first + 16 + 4 g + 0 .. 3: of a paired tile, and of a row-major one
+template <int KD> __device__ __forceinline__ bf8 la_read_paired_tr(const __bf16 *tile, int first, int dt, int l16, int g) {
+    const int row = 4 * g + l16 / 4;
+    const __bf16 *at = tile + (first + row) * KD + ((dt / 2 * 4 + l16 % 4) ^ la_hash<KD>(row)) * 8 + dt % 2 * 4;
+    return la_join(la_read_tr(at), la_read_tr(at + 16 * KD));
+}
+__device__ __forceinline__ bf8 la_read_rows_tr(const __bf16 *tile, int ld, int first, int col, int l16, int g) {
+    const __bf16 *at = tile + (first + 4 * g + l16 / 4) * ld + col + l16 % 4 * 4;
+    return la_join(la_read_tr(at), la_read_tr(at + 16 * ld));
+}
+// Two bf16 terms of eight values of a result tile pair, as an operand in the paired order
+__device__ __forceinline__ LaSplit la_split_pair(const f4 &x, const f4 &y) {
+    LaSplit s;
+    la_split2(x[0], x[1], s.hi[0], s.lo[0]);
+    la_split2(x[2], x[3], s.hi[1], s.lo[1]);
+    la_split2(y[0], y[1], s.hi[2], s.lo[2]);
+    la_split2(y[2], y[3], s.hi[3], s.lo[3]);
+    return s;
+}
+// All 24 bits of eight values, as three terms
+struct LaSplit3 {
+    bf8 term[3];
+};
+__device__ __forceinline__ LaSplit3 la_split3(const f4 &x, const f4 &y) {
+    la_u4 t[3];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float a = (j < 2 ? x : y)[2 * j % 4], b = (j < 2 ? x : y)[2 * j % 4 + 1];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            t[n][j] = row_pack_bf16(a, b);
+            a -= __builtin_bit_cast(float, t[n][j] << 16);
+            b -= __builtin_bit_cast(float, t[n][j] & 0xffff0000u);
+        }
     }
-    if (!tr) return;
-    // columns 0/1 and 2/3 of rows 0..3 as pairs over rows (v_perm picks the low or the high halves)
-    auto low = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_perm(y, x, 0x05040100u); };
-    auto high = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_perm(y, x, 0x07060302u); };
-    *reinterpret_cast<uint2 *>(tr + la_tr(c, s)) = make_uint2(low(b.r[0].x, b.r[1].x), low(b.r[2].x, b.r[3].x));
-    *reinterpret_cast<uint2 *>(tr + la_tr(c + 1, s)) = make_uint2(high(b.r[0].x, b.r[1].x), high(b.r[2].x, b.r[3].x));
-    *reinterpret_cast<uint2 *>(tr + la_tr(c + 2, s)) = make_uint2(low(b.r[0].y, b.r[1].y), low(b.r[2].y, b.r[3].y));
-    *reinterpret_cast<uint2 *>(tr + la_tr(c + 3, s)) = make_uint2(high(b.r[0].y, b.r[1].y), high(b.r[2].y, b.r[3].y));
+    return LaSplit3{{__builtin_bit_cast(bf8, t[0]), __builtin_bit_cast(bf8, t[1]), __builtin_bit_cast(bf8, t[2])}};
+}
+// Two terms of eight raw values times weights (x: rows 4 g + 0 .. 3, y: 16 further on)
+__device__ __forceinline__ LaSplit la_split_weighted(bf8 raw, const f4 &x, const f4 &y) {
+    const la_u4 v = __builtin_bit_cast(la_u4, raw);
+    LaSplit s;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        la_split2(__builtin_bit_cast(float, v[j] << 16) * (j < 2 ? x : y)[2 * j % 4],
+                  __builtin_bit_cast(float, v[j] & 0xffff0000u) * (j < 2 ? x : y)[2 * j % 4 + 1], s.hi[j], s.lo[j]);
+    return s;
 }
 
 constexpr int kLaPitchA = 72;  // bf16 per row of the decayed scores

@@ -1,0 +1,73 @@
+"""Segments of prompts of unequal lengths: the rule that chooses them, in a plain C++ build, and one launch that it cuts
+although the batch alone fills the device, against the oracle's token-by-token recurrence."""
+
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_segments_follow_the_rows_of_a_batch(tmp_path):
+    src = tmp_path / "plan.cpp"
+    src.write_text('''
+#include "lightning_plan.h"
+#include <cstdio>
+#include <initializer_list>
+int main() {
+    for (double together : {0.0, 1.25, 1.6})
+        for (long long batch : {1LL, 2LL, 7LL, 40LL, 3000LL})
+            for (int per : {1, 5, 16, 64})
+                for (int len = 1; len < 40000; len = len * 3 / 2 + 1)
+                    for (double part : {0.0, 0.3, 1.0}) {
+                        const size_t one = la_workspace_bytes(batch, per, 128, 128, 2) / 2;
+                        const int most = la_most_segments(one, len);
+                        if (most < 1 || most > kLaMaxSegments || (most > 1 && most * one > kLaMostSegBytes)) return 1;
+                        const long long rows = (long long)(batch * len * part) + 1;
+                        const int s = la_launch_segments(batch, per, 256, together, len, rows, one, most * one, true);
+                        if (s < 1 || s > most || (long long)s * la_segment_rows(len, s) < len) return 2;
+                        for (size_t room : {(size_t)0, one, 3 * one + 5}) {  // a workspace too small for all of them
+                            const int t = la_launch_segments(batch, per, 256, together, len, rows, one, room, true);
+                            if (t < 1 || (t > 1 && t * one > room)) return 3;
+                        }
+                        // unaligned: refused where few sequences need it, ignored where the batch fills the device
+                        const int u = la_launch_segments(batch, per, 256, together, len, rows, one, most * one, false);
+                        if (u != (most > 1 && la_segments(batch * per, 256, len) > 1 ? 0 : 1)) return 4;
+                        if (la_launch_segments(batch, per, 256, together, len, rows, one, 0, false) != 1) return 5;
+                    }
+    const size_t big = (size_t)1 << 20;
+    if (la_balanced_segments(16, 16, 256, 0.0, 4096, 16 * 4096, 64) != 1) return 6;  // equal and full: no segments
+    if (la_balanced_segments(16, 16, 256, 0.0, 4096, 5 * 4096, 64) < 2) return 7;    // a few long ones: segments
+    if (la_balanced_segments(1, 16, 256, 0.0, 4096, 4096, la_most_segments(big, 4096)) < 4) return 8;
+    if (la_balanced_segments(0, 16, 256, 0.0, 4096, 0, 64) != 1 || la_balanced_segments(4, 16, 256, 0.0, 0, 0, 64) != 1) return 9;
+    if (la_most_segments(big * 300, 40000) != 1 || la_most_segments(0, 40000) != 64) return 10;
+    std::puts("ok");
+}
+''')
+    exe = tmp_path / "plan"
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "research_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], stdout=subprocess.PIPE).returncode == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,dim,vdim", [(32, 64, 64), (32, 64, 128), (16, 128, 128)])
+def test_a_batch_of_unequal_prompts_in_segments(heads, dim, vdim):
+    import torch
+
+    from tests.gpu_helpers import announce
+    from tests.test_gpu_lightning import Case
+
+    announce(f"ragged segments {heads}x{dim}x{vdim}")
+    decay = [1.0 - 0.5 ** (1 + i * 12 / heads) for i in range(heads)]
+    # one sequence of many segments, some that end inside the first, on and beside a segment's edge
+    lens = [2500, 1, 64, 511, 512, 513, 1025, 700, 30, 2000]
+    case = Case(lens, heads, dim, vdim, decay, torch.bfloat16, seed=5)
+    slots = [(3 * b + 1) % len(lens) for b in range(len(lens))]
+    head = [(b, 0, (n + 1) // 2) for b, n in enumerate(lens)]
+    tail = [(b, (n + 1) // 2, n // 2) for b, n in enumerate(lens) if n > 1]
+    for picks in (head, tail):  # (the second starts from the states that the first left)
+        for (b, lo, _), got in zip(picks, case.run(picks, slots)):
+            case.check(b, lo, got)
+    for b, n in enumerate(lens):
+        case.check_state(b, slots[b])
