@@ -57,10 +57,12 @@ __device__ __forceinline__ int scored_block_id(const ScoredArgs &a, const int32_
 __device__ __forceinline__ int scored_slot_of(const ScoredArgs &a, int id, int key, int end) {
     return key < end && key / a.bs < a.bt_stride && (uint32_t)id < (uint64_t)a.num_blocks ? id * a.bs + key % a.bs : -1;
 }
-// 16 bytes of a row, zeros where there is none: always one load, so that nothing waits for it before it is used.
+// 16 bytes of a row, zeros where there is none: always one load, so that nothing waits for it before it is used.  (Of global
+// memory, and said so: a choice of two pointers leaves the compiler a flat load, which every wait for LDS waits for too.)
 static __device__ const uint32_t kScoredZeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 __device__ __forceinline__ scored_u4 scored_load16(const uint16_t *p, bool there) {
-    return *reinterpret_cast<const scored_u4 *>(there ? p : reinterpret_cast<const uint16_t *>(kScoredZeros));
+    typedef const __attribute__((address_space(1))) scored_u4 *global_u4;
+    return *reinterpret_cast<global_u4>(there ? reinterpret_cast<uintptr_t>(p) : reinterpret_cast<uintptr_t>(kScoredZeros));
 }
 
 constexpr float kScoredLog2e = 1.4426950408889634f;
