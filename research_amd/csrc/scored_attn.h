@@ -85,4 +85,4 @@ inline int scored_splits(int64_t workgroups, int cus, int64_t span, bool full) {
 
 // false: no matrix-core kernel for these sizes
 bool pa_scored_decode_launch(const ScoredArgs &a, int dtype, hipStream_t s, int &rc);
-bool pa_scored_prefill_launch(const ScoredArgs &a, int dtype, hipStream_t s, int &rc);
+bool pa_scored_prefill_launch(const ScoredArgs &a, int dtype, int cus, hipStream_t s, int &rc);

@@ -141,7 +141,7 @@ extern "C" int pa_scored_attention(const void *q1, int64_t q1_row, int64_t q1_he
         PA_REQUIRE(a.splits == 1 || pa_aligned16(workspace), "the workspace must be 16-byte aligned");
     }
     int rc = PA_OK;
-    if (pa_scored_decode_launch(a, dtype, s, rc) || pa_scored_prefill_launch(a, dtype, s, rc)) return rc;
+    if (pa_scored_decode_launch(a, dtype, s, rc) || pa_scored_prefill_launch(a, dtype, scored_cus(), s, rc)) return rc;
     if (dtype == PA_F32) launch_vector<float>(a, s);
     else launch_vector<pa_bf16>(a, s);
     PA_CHECK_LAUNCH("pa_scored_attention");
