@@ -327,12 +327,16 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
 }
 
 // ------------------------------------------------------------------ chunks: the walk
+// Bound by the chain of one wave per SIMD: the products of a chunk take a quarter of it, 72 KB through the compute unit's 64 bytes
+// a cycle another seventh.  So operands are read a step ahead of their products and the next tile's loads are spread over the
+// chunk; a chunk of four waves at 128 x 64 took 10.5 thousand cycles and takes 7.6 (8 prompts of 700 .. 4000 rows, 16 heads of
+// 128 x 128: 273 -> 196 us; eight waves a workgroup, whose SIMDs have two: 32 prompts of about 900 rows 324 -> 309).
 template <int KD, int COLS> constexpr size_t delta_walk_lds() {
     return (size_t)(2 * 64 * KD + 64 * (COLS + 8) + 4 * 64 * kDcPitch) * 2 + 3 * 64 * 4 + 64;
 }
 
 // KD: dim padded to 64, 128 or 256.  A workgroup of NW waves owns 16 NW value columns of a head and all chunks of a portion.
-template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_walk_kernel(const DeltaArgs a) {
+template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW == 4 ? 2 : 1) void delta_walk_kernel(const DeltaArgs a) {
     constexpr int kCols = 16 * NW, kThr = 64 * NW, kLv = kCols + 8;
     constexpr int kBlocks = 16 * (KD / 4), kKB = (kBlocks + kThr - 1) / kThr;  // 4 x 4 blocks of K, of V; 16-byte pieces of T and C
     constexpr int kVB = 16 * (kCols / 4) / kThr, kMB = 4 * 64 * 8 / kThr;
@@ -371,102 +375,166 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
     LaBlock qb[kKB], kb[kKB], vb[kVB];
     la_u4 mb[kMB];
     float keep_next = 0.f, row_g0 = 0.f, row_g1 = 0.f, row_g2 = 0.f;
-    auto fetch = [&](int r0) {
+    // The next chunk's tiles, a part at a time: all loads at once would hold up a wave for longer than it computes.
+    auto again = [](int x) { return NW == 8 ? la_again(x) : x; };  // (eight waves: too few registers to keep every place)
+    auto fetch = [&](int part, int r0) {
+        if (r0 >= p.n) return;
+        const int ft = again(tid);
         const int nr = p.n - r0 < 64 ? p.n - r0 : 64;
-        const __amdgpu_buffer_rsrc_t tq = la_tile(uq + r0 * a.ldq, a.ldq, nr, a.dim), tk = la_tile(uk + r0 * a.ldk, a.ldk, nr, a.dim);
-        const __amdgpu_buffer_rsrc_t tv = la_tile(uv + r0 * a.ldv, a.ldv, nr, vcols);
-#pragma unroll
-        for (int i = 0; i < kKB; ++i) {
-            const int blk = tid + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
-            qb[i] = la_load_block(tq, k_live ? la_block_off(a.ldq, r, c, a.dim) : kLaOutside, (uint32_t)a.ldq * 2u);
-            kb[i] = la_load_block(tk, k_live ? la_block_off(a.ldk, r, c, a.dim) : kLaOutside, (uint32_t)a.ldk * 2u);
-        }
-#pragma unroll
-        for (int i = 0; i < kVB; ++i) {
-            const int blk = tid + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
-            vb[i] = la_load_block(tv, la_block_off(a.ldv, r, c, vcols), (uint32_t)a.ldv * 2u);
-        }
         const DeltaChunk *m = mats + (int64_t)(r0 / 64) * a.heads;
+        if (part == 0) {
 #pragma unroll
-        for (int i = 0; i < kMB; ++i) mb[i] = reinterpret_cast<const la_u4 *>(m)[tid + kThr * i];
-        row_g0 = m->k_in[tid & 63];
-        row_g1 = m->q_in[tid & 63];
-        row_g2 = m->k_out[tid & 63];
-        keep_next = m->keep;
+            for (int i = 0; i < kMB; ++i) mb[i] = reinterpret_cast<const la_u4 *>(m)[ft + kThr * i];
+        } else if (part == 1) {
+            const __amdgpu_buffer_rsrc_t tk = la_tile(uk + r0 * a.ldk, a.ldk, nr, a.dim);
+#pragma unroll
+            for (int i = 0; i < kKB; ++i) {
+                const int blk = ft + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
+                kb[i] = la_load_block(tk, k_live ? la_block_off(a.ldk, r, c, a.dim) : kLaOutside, (uint32_t)a.ldk * 2u);
+            }
+        } else if (part == 2) {
+            const __amdgpu_buffer_rsrc_t tq = la_tile(uq + r0 * a.ldq, a.ldq, nr, a.dim);
+#pragma unroll
+            for (int i = 0; i < kKB; ++i) {
+                const int blk = ft + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
+                qb[i] = la_load_block(tq, k_live ? la_block_off(a.ldq, r, c, a.dim) : kLaOutside, (uint32_t)a.ldq * 2u);
+            }
+        } else {
+            const __amdgpu_buffer_rsrc_t tv = la_tile(uv + r0 * a.ldv, a.ldv, nr, vcols);
+#pragma unroll
+            for (int i = 0; i < kVB; ++i) {
+                const int blk = ft + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
+                vb[i] = la_load_block(tv, la_block_off(a.ldv, r, c, vcols), (uint32_t)a.ldv * 2u);
+            }
+            row_g0 = m->k_in[ft & 63];
+            row_g1 = m->q_in[ft & 63];
+            row_g2 = m->k_out[ft & 63];
+            keep_next = m->keep;
+        }
     };
-    fetch(0);
+#pragma unroll
+    for (int part = 0; part < 4; ++part) fetch(part, 0);
     for (int r0 = 0; r0 < p.n; r0 += 64) {
+        const int lt = again(tid);
         const int nv = p.n - r0 < 64 ? p.n - r0 : 64;
 #pragma unroll
         for (int i = 0; i < kKB; ++i) {
-            const int blk = tid + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
+            const int blk = lt + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
             if (!k_live) continue;
             la_put_paired<false, KD>(qb[i], r, c, q_s);
             la_put_paired<false, KD>(kb[i], r, c, k_s);
         }
 #pragma unroll
         for (int i = 0; i < kVB; ++i) {
-            const int blk = tid + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
+            const int blk = lt + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
             la_put_block<false>(vb[i], r, c, v_s, kLv);
         }
 #pragma unroll
         for (int i = 0; i < kMB; ++i) {
-            const int at = tid + kThr * i;  // 16-byte piece: row at / 8 over the four matrices
+            const int at = lt + kThr * i;  // 16-byte piece: row at / 8 over the four matrices
             *reinterpret_cast<la_u4 *>(m_s + at / 8 * kDcPitch + at % 8 * 8) = mb[i];
         }
-        if (tid < 64) {
-            rows[tid] = row_g0;
-            rows[64 + tid] = row_g1;
-            rows[128 + tid] = row_g2;
+        if (lt < 64) {
+            rows[lt] = row_g0;
+            rows[64 + lt] = row_g1;
+            rows[128 + lt] = row_g2;
         }
         const float keep = keep_next;
-        if (r0 + 64 < p.n) fetch(r0 + 64);
         __syncthreads();
-        // K S (rows t = 16 tt + 4 g + i, columns v) and, transposed, Q S (v = 4 g + i of the wave's columns, t = 16 tt + l16)
+        const int lr = again(tid) & 63, l16 = lr & 15, g = lr >> 4;
+        // K S (rows t = 16 tt + 4 g + i, columns v) and, transposed, Q S (v = 4 g + i of the wave's columns, t = 16 tt + l16).
+        // Operands are read a step ahead of their products: nothing else covers the wait, a SIMD has this one wave.
         f4 u[4], o[4];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) u[tt] = o[tt] = f4{0.f, 0.f, 0.f, 0.f};
+        bf8 xk[2][4], xq[2][4], th[4], tl[4], th2[2], tl2[2];
+        f4 ki[4];
+        la_bf4 vv[4];
+        float qi[4];
+        auto ahead = [] {
+            if constexpr (NW < 8) __builtin_amdgcn_sched_barrier(0);
+        };
+        auto read_rows = [&](int dd) {
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) {
+                xk[dd & 1][tt] = la_read_paired<KD>(k_s, 16 * tt + l16, l16, dd, g);
+                xq[dd & 1][tt] = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
+            }
+        };
+        auto mat = [&](const __bf16 *m, int tt, int kk) { return la_read8(m + (16 * tt + l16) * kDcPitch + 32 * kk + 8 * g); };
+        read_rows(0);
 #pragma unroll
         for (int dd = 0; dd < KD / 32; ++dd) {
+            if (dd + 1 < KD / 32) {
+                read_rows(dd + 1);
+            } else {
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) {
+                    ki[tt] = *reinterpret_cast<const f4 *>(rows + 16 * tt + 4 * g);
+                    vv[tt] = la_read_tr(v_s + (16 * tt + 4 * g + l16 / 4) * kLv + vw + l16 % 4 * 4);
+                    qi[tt] = rows[64 + 16 * tt + l16];
+                }
+            }
+            if (dd < 2) fetch(dd, r0 + 64);
+            ahead();
             const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) {
-                const bf8 xk = la_read_paired<KD>(k_s, 16 * tt + l16, l16, dd, g), xq = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
-                u[tt] = la_mfma(xk, hi, u[tt]);
-                u[tt] = la_mfma(xk, lo, u[tt]);
-                o[tt] = la_mfma(hi, xq, o[tt]);
-                o[tt] = la_mfma(lo, xq, o[tt]);
+                u[tt] = la_mfma(xk[dd & 1][tt], hi, u[tt]);
+                o[tt] = la_mfma(hi, xq[dd & 1][tt], o[tt]);
+            }
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) {
+                u[tt] = la_mfma(xk[dd & 1][tt], lo, u[tt]);
+                o[tt] = la_mfma(lo, xq[dd & 1][tt], o[tt]);
             }
         }
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
-            const f4 ki = *reinterpret_cast<const f4 *>(rows + 16 * tt + 4 * g);
-            const la_bf4 vv = la_read_tr(v_s + (16 * tt + 4 * g + l16 / 4) * kLv + vw + l16 % 4 * 4);
-            const float qi = rows[64 + 16 * tt + l16];
+            th[tt] = mat(t_hi, tt, 0);
+            tl[tt] = mat(t_lo, tt, 0);
+        }
+        fetch(2, r0 + 64);
+        ahead();
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                u[tt][i] = (float)vv[i] - ki[i] * u[tt][i];
-                o[tt][i] *= qi;
+                u[tt][i] = (float)vv[tt][i] - ki[tt][i] * u[tt][i];
+                o[tt][i] *= qi[tt];
             }
-        }
         // U = T R
         f4 w[4];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) w[tt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const LaSplit sp = la_split_pair(u[2 * kk], u[2 * kk + 1]);
-            const bf8 hi = sp.high(), lo = sp.low();
-#pragma unroll
-            for (int tt = 2 * kk; tt < 4; ++tt) {
-                const int at = (16 * tt + l16) * kDcPitch + 32 * kk + 8 * g;
-                const bf8 th = la_read8(t_hi + at), tl = la_read8(t_lo + at);
-                w[tt] = la_mfma(th, hi, w[tt]);
-                w[tt] = la_mfma(th, lo, w[tt]);
-                w[tt] = la_mfma(tl, hi, w[tt]);
-            }
+        for (int tt = 0; tt < 2; ++tt) {
+            th2[tt] = mat(t_hi, 2 + tt, 1);
+            tl2[tt] = mat(t_lo, 2 + tt, 1);
         }
+        f4 ko[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) ko[tt] = *reinterpret_cast<const f4 *>(rows + 128 + 16 * tt + 4 * g);
+        fetch(3, r0 + 64);
+        ahead();
+        auto times_t = [&](bf8 x, bf8 y, bf8 hi, bf8 lo, f4 &to) {
+            to = la_mfma(x, hi, to);
+            to = la_mfma(x, lo, to);
+            to = la_mfma(y, hi, to);
+        };
+        const LaSplit r_lo = la_split_pair(u[0], u[1]), r_hi = la_split_pair(u[2], u[3]);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) times_t(th[tt], tl[tt], r_lo.high(), r_lo.low(), w[tt]);
+        bf8 ch[4], cl[4], kt[KD / 16];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            ch[tt] = mat(c_hi, tt, 0);
+            cl[tt] = mat(c_lo, tt, 0);
+        }
+        ahead();
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) times_t(th2[tt], tl2[tt], r_hi.high(), r_hi.low(), w[2 + tt]);
         // O += C U (transposed), S <- keep S + K^T (k_out U)
 #pragma unroll
         for (int dt = 0; dt < KD / 16; ++dt)
@@ -474,32 +542,36 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, 1) void delta_wa
             for (int i = 0; i < 4; ++i) s[dt][i] *= keep;
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt) kt[dt] = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
+            ahead();
             {
                 const LaSplit sp = la_split_pair(w[2 * kk], w[2 * kk + 1]);
                 const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
                 for (int tt = 2 * kk; tt < 4; ++tt) {
-                    const int at = (16 * tt + l16) * kDcPitch + 32 * kk + 8 * g;
-                    const bf8 ch = la_read8(c_hi + at), cl = la_read8(c_lo + at);
-                    o[tt] = la_mfma(hi, ch, o[tt]);
-                    o[tt] = la_mfma(lo, ch, o[tt]);
-                    o[tt] = la_mfma(hi, cl, o[tt]);
+                    o[tt] = la_mfma(hi, ch[tt], o[tt]);
+                    o[tt] = la_mfma(lo, ch[tt], o[tt]);
+                    o[tt] = la_mfma(hi, cl[tt], o[tt]);
                 }
             }
 #pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                const f4 ko = *reinterpret_cast<const f4 *>(rows + 128 + 32 * kk + 16 * half + 4 * g);
+            for (int half = 0; half < 2; ++half)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w[2 * kk + half][i] *= ko[i];
-            }
+                for (int i = 0; i < 4; ++i) w[2 * kk + half][i] *= ko[2 * kk + half][i];
             const LaSplit sp = la_split_pair(w[2 * kk], w[2 * kk + 1]);
             const bf8 hi = sp.high(), lo = sp.low();
+            if (kk == 0) {
 #pragma unroll
-            for (int dt = 0; dt < KD / 16; ++dt) {
-                const bf8 xk = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
-                s[dt] = la_mfma(xk, hi, s[dt]);
-                s[dt] = la_mfma(xk, lo, s[dt]);
+                for (int tt = 2; tt < 4; ++tt) {
+                    ch[tt] = mat(c_hi, tt, 1);
+                    cl[tt] = mat(c_lo, tt, 1);
+                }
             }
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt) s[dt] = la_mfma(kt[dt], hi, s[dt]);
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt) s[dt] = la_mfma(kt[dt], lo, s[dt]);
         }
         const int ldo = a.heads * a.vdim, c = vw + 4 * g;
         const uint16_t *first = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0) * (int64_t)ldo + h * a.vdim + v0;

@@ -4,7 +4,7 @@
 // 64 keys and values in LDS; the next tile is on its way in registers.  As in prefill_mfma.h everything is transposed:
 // S^T = K Q^T leaves a lane 16 keys of one row, which in register order are the operand of O^T += V^T P^T.  The distance
 // biases of a wave's head lie in LDS, newest key last, with margins on both sides, so that a lane reads the biases of
-// consecutive keys side by side and nothing is clamped; blocks of keys past the last distance share one number.
+// consecutive keys side by side; keys past the last distance read its margin.
 //
 // Bound by a wave's own chain: staging a tile (8 KB of a wave's loads and writes, 1500 of 6000 cycles), scores and weights (four
 // transcendentals for two elements with a cap), and no more than two waves of 220 registers on a SIMD to cover it; products of one
