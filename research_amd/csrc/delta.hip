@@ -327,10 +327,11 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
 }
 
 // ------------------------------------------------------------------ chunks: the walk
-// Bound by the chain of one wave per SIMD: the products of a chunk take a quarter of it, 72 KB through the compute unit's 64 bytes
-// a cycle another seventh.  So operands are read a step ahead of their products and the next tile's loads are spread over the
-// chunk; a chunk of four waves at 128 x 64 took 10.5 thousand cycles and takes 7.6 (8 prompts of 700 .. 4000 rows, 16 heads of
-// 128 x 128: 273 -> 196 us; eight waves a workgroup, whose SIMDs have two: 32 prompts of about 900 rows 324 -> 309).
+// Bound by the chain of one wave per SIMD: the products of a chunk take a quarter of it, 64 KB through the compute unit's 64 bytes
+// a cycle another seventh.  So operands are read a step ahead of their products, and the next tile's loads are spread over the
+// chunk, in the order in which they are written to LDS.  A second set of tiles, written while the first is read, gave nothing (the
+// walk then lacks registers).  8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128: 273 -> 187 us; eight waves a workgroup, whose
+// SIMDs have two each: 32 prompts of about 900 rows, with the first pass, 324 -> 311.
 template <int KD, int COLS> constexpr size_t delta_walk_lds() {
     return (size_t)(2 * 64 * KD + 64 * (COLS + 8) + 4 * 64 * kDcPitch) * 2 + 3 * 64 * 4 + 64;
 }
@@ -339,7 +340,9 @@ template <int KD, int COLS> constexpr size_t delta_walk_lds() {
 template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW == 4 ? 2 : 1) void delta_walk_kernel(const DeltaArgs a) {
     constexpr int kCols = 16 * NW, kThr = 64 * NW, kLv = kCols + 8;
     constexpr int kBlocks = 16 * (KD / 4), kKB = (kBlocks + kThr - 1) / kThr;  // 4 x 4 blocks of K, of V; 16-byte pieces of T and C
-    constexpr int kVB = 16 * (kCols / 4) / kThr, kMB = 4 * 64 * 8 / kThr;
+    constexpr bool kFew = NW < 8;  // a SIMD has one wave: all its registers
+    constexpr int kVB = 16 * (kCols / 4) / kThr, kMB = 4 * (kFew ? 48 : 64) * 8 / kThr;
+    constexpr int kSteps = kFew && KD > 64 ? 1 : 2;  // parts of the next chunk's loads beside a product of 32 columns
     static_assert(16 * (kCols / 4) % kThr == 0 && (kBlocks % kThr == 0 || kKB == 1), "whole passes");
     const bool k_live = kBlocks >= kThr || (int)threadIdx.x < kBlocks;
     extern __shared__ __align__(16) char lds[];
@@ -375,37 +378,46 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
     LaBlock qb[kKB], kb[kKB], vb[kVB];
     la_u4 mb[kMB];
     float keep_next = 0.f, row_g0 = 0.f, row_g1 = 0.f, row_g2 = 0.f;
-    // The next chunk's tiles, a part at a time: all loads at once would hold up a wave for longer than it computes.
-    auto again = [](int x) { return NW == 8 ? la_again(x) : x; };  // (eight waves: too few registers to keep every place)
+    auto again = [](int x) { return kFew ? x : la_again(x); };  // (with too few registers places in memory are worked out again)
+    // 16-byte piece `at` of T's and C's terms: its row of the four, its column.  A wave with registers for its places leaves out the
+    // quarter above the diagonal blocks of 32.
+    auto piece = [](int at, int &row, int &col) {
+        const int r = at % 384;
+        row = !kFew ? at / 8 : at / 384 * 64 + (r < 128 ? r / 4 : 16 + r / 8);
+        col = !kFew ? at % 8 : r < 128 ? r % 4 : r % 8;
+    };
+    // Tiles in eight parts: loads all at once would hold up a wave for longer than it computes.
     auto fetch = [&](int part, int r0) {
         if (r0 >= p.n) return;
         const int ft = again(tid);
         const int nr = p.n - r0 < 64 ? p.n - r0 : 64;
         const DeltaChunk *m = mats + (int64_t)(r0 / 64) * a.heads;
-        if (part == 0) {
+        if (part < 2) {
 #pragma unroll
-            for (int i = 0; i < kMB; ++i) mb[i] = reinterpret_cast<const la_u4 *>(m)[ft + kThr * i];
-        } else if (part == 1) {
-            const __amdgpu_buffer_rsrc_t tk = la_tile(uk + r0 * a.ldk, a.ldk, nr, a.dim);
+            for (int i = 0; i < kMB; ++i) {
+                if (i * 2 / kMB != part) continue;
+                int row, col;
+                piece(ft + kThr * i, row, col);
+                mb[i] = reinterpret_cast<const la_u4 *>(m)[row * 8 + col];
+            }
+        } else if (part < 6) {
+            const bool keys = part < 4;
+            const int64_t ld = keys ? a.ldk : a.ldq;
+            const __amdgpu_buffer_rsrc_t tile = keys ? la_tile(uk + r0 * ld, ld, nr, a.dim) : la_tile(uq + r0 * ld, ld, nr, a.dim);
 #pragma unroll
             for (int i = 0; i < kKB; ++i) {
+                if (i * 2 / kKB != part % 2) continue;
                 const int blk = ft + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
-                kb[i] = la_load_block(tk, k_live ? la_block_off(a.ldk, r, c, a.dim) : kLaOutside, (uint32_t)a.ldk * 2u);
+                (keys ? kb : qb)[i] = la_load_block(tile, k_live ? la_block_off(ld, r, c, a.dim) : kLaOutside, (uint32_t)ld * 2u);
             }
-        } else if (part == 2) {
-            const __amdgpu_buffer_rsrc_t tq = la_tile(uq + r0 * a.ldq, a.ldq, nr, a.dim);
-#pragma unroll
-            for (int i = 0; i < kKB; ++i) {
-                const int blk = ft + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
-                qb[i] = la_load_block(tq, k_live ? la_block_off(a.ldq, r, c, a.dim) : kLaOutside, (uint32_t)a.ldq * 2u);
-            }
-        } else {
+        } else if (part == 6) {
             const __amdgpu_buffer_rsrc_t tv = la_tile(uv + r0 * a.ldv, a.ldv, nr, vcols);
 #pragma unroll
             for (int i = 0; i < kVB; ++i) {
                 const int blk = ft + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
                 vb[i] = la_load_block(tv, la_block_off(a.ldv, r, c, vcols), (uint32_t)a.ldv * 2u);
             }
+        } else {
             row_g0 = m->k_in[ft & 63];
             row_g1 = m->q_in[ft & 63];
             row_g2 = m->k_out[ft & 63];
@@ -413,26 +425,27 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         }
     };
 #pragma unroll
-    for (int part = 0; part < 4; ++part) fetch(part, 0);
+    for (int part = 0; part < 8; ++part) fetch(part, 0);
     for (int r0 = 0; r0 < p.n; r0 += 64) {
-        const int lt = again(tid);
+        const int lt = again(tid);  // (written in the order of loading)
         const int nv = p.n - r0 < 64 ? p.n - r0 : 64;
+#pragma unroll
+        for (int i = 0; i < kMB; ++i) {
+            int row, col;
+            piece(lt + kThr * i, row, col);
+            *reinterpret_cast<la_u4 *>(m_s + row * kDcPitch + col * 8) = mb[i];
+        }
 #pragma unroll
         for (int i = 0; i < kKB; ++i) {
             const int blk = lt + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
             if (!k_live) continue;
-            la_put_paired<false, KD>(qb[i], r, c, q_s);
             la_put_paired<false, KD>(kb[i], r, c, k_s);
+            la_put_paired<false, KD>(qb[i], r, c, q_s);
         }
 #pragma unroll
         for (int i = 0; i < kVB; ++i) {
             const int blk = lt + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
             la_put_block<false>(vb[i], r, c, v_s, kLv);
-        }
-#pragma unroll
-        for (int i = 0; i < kMB; ++i) {
-            const int at = lt + kThr * i;  // 16-byte piece: row at / 8 over the four matrices
-            *reinterpret_cast<la_u4 *>(m_s + at / 8 * kDcPitch + at % 8 * 8) = mb[i];
         }
         if (lt < 64) {
             rows[lt] = row_g0;
@@ -452,7 +465,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         la_bf4 vv[4];
         float qi[4];
         auto ahead = [] {
-            if constexpr (NW < 8) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (kFew) __builtin_amdgcn_sched_barrier(0);
         };
         auto read_rows = [&](int dd) {
 #pragma unroll
@@ -475,7 +488,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
                     qi[tt] = rows[64 + 16 * tt + l16];
                 }
             }
-            if (dd < 2) fetch(dd, r0 + 64);
+#pragma unroll
+            for (int part = kSteps * dd; part < kSteps * (dd + 1) && part < 4; ++part) fetch(part, r0 + 64);
             ahead();
             const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
             const bf8 hi = sp.high(), lo = sp.low();
@@ -495,7 +509,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
             th[tt] = mat(t_hi, tt, 0);
             tl[tt] = mat(t_lo, tt, 0);
         }
-        fetch(2, r0 + 64);
+        fetch(4, r0 + 64);
+        if constexpr (!kFew) fetch(5, r0 + 64);
         ahead();
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt)
@@ -516,7 +531,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         f4 ko[4];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) ko[tt] = *reinterpret_cast<const f4 *>(rows + 128 + 16 * tt + 4 * g);
-        fetch(3, r0 + 64);
+        if constexpr (!kFew) fetch(6, r0 + 64);
+        fetch(kFew ? 5 : 7, r0 + 64);
         ahead();
         auto times_t = [&](bf8 x, bf8 y, bf8 hi, bf8 lo, f4 &to) {
             to = la_mfma(x, hi, to);
@@ -544,6 +560,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
             for (int dt = 0; dt < KD / 16; ++dt) kt[dt] = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
+            if constexpr (kFew) fetch(6 + kk, r0 + 64);
             ahead();
             {
                 const LaSplit sp = la_split_pair(w[2 * kk], w[2 * kk + 1]);
