@@ -10,6 +10,8 @@
 // 32-bit operands have a plain kernel.  The weights' rows are zero-padded to whole 64-element steps; token rows are not
 // read past their end.  All products are taken transposed (weight rows as the rows of the result), so that a lane holds
 // four consecutive outputs of one item.
+#include <type_traits>
+
 #include "moe_plan.h"
 #include "row_common.h"
 
@@ -498,7 +500,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
     constexpr int kBM = 16 * TM * WM, kBN = 16 * TN * WN, kWaves = WM * WN;
     constexpr int kLoadsA = kBM / 8 / kWaves, kLoadsB = kBN / 8 / kWaves;  // wave-wide loads of eight 128-byte rows
     constexpr int kOut = GLU ? kBN / 2 : kBN;  // outputs per tile
-    constexpr int kRing = 4, kAhead = 2, kGroups = 2 * TN;  // groups of TM products: 32 elements of one weight tile
+    constexpr int kRing = 8, kAhead = 5, kGroups = 2 * TN;  // groups of TM products: 32 elements of one weight tile
     constexpr int kStores = TM * (GLU ? TN / 4 : TN / 2);
     static_assert(kBM % (8 * kWaves) == 0 && kBN % (32 * kWaves) == 0 && kBM == 64 * (kWaves / 2) && TN % 4 == 0, "whole loads per wave");
     extern __shared__ __align__(16) char lds[];
@@ -625,7 +627,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
     for (int t = 0; t < kAhead; ++t) wb[t] = b_tile(0, t);
     // One step from buffer `buf`.  Behind its last reads: the other buffer's tiles have come (`stores`: the last tile's results,
     // which are younger, need not have been written), every wave is through with this one, and step `far` is sent for.
-    auto run = [&](int buf, int far, bool stores) {
+    // `live`: the wave has items in this tile.  Without, it leaves the matrix cores to the other wave of its SIMD, which has the
+    // items 128 places before its own, and only keeps the pipeline going.
+    auto run = [&](auto live, int buf, int far, bool stores) {
+        constexpr bool kLive = decltype(live)::value;
 #pragma unroll
         for (int q = 0; q < kGroups; ++q) {
             if (q == kGroups - kAhead) {
@@ -637,8 +642,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
                 fetch(src, far, buf);
             }
             const int to = q + kAhead;
-            wb[to % kRing] = to < kGroups ? b_tile(buf, to) : b_tile(buf ^ 1, to - kGroups);
-            if (q == TN / 2) {  // the second half's items
+            if (kLive || to >= kGroups) wb[to % kRing] = to < kGroups ? b_tile(buf, to) : b_tile(buf ^ 1, to - kGroups);
+            if (kLive && q == TN / 2) {  // the second half's items
 #pragma unroll
                 for (int m = 0; m < TM; ++m) xa[1][m] = a_tile(buf, 1, m);
             }
@@ -646,8 +651,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
 #pragma unroll
                 for (int m = 0; m < TM; ++m) xa[0][m] = a_tile(buf ^ 1, 0, m);
             }
+            if constexpr (kLive) {
 #pragma unroll
-            for (int m = 0; m < TM; ++m) acc[q % TN][m] = moe_mfma(wb[q % kRing], xa[q / TN][m], acc[q % TN][m]);
+                for (int m = 0; m < TM; ++m) acc[q % TN][m] = moe_mfma(wb[q % kRing], xa[q / TN][m], acc[q % TN][m]);
+            }
         }
     };
     const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(a.out, 0, (int)(uint32_t)(a.items * a.n * 2), 0x00020000);
@@ -660,16 +667,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
             for (int m = 0; m < TM; ++m) acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
         const int tile_next = tile + stride;
         const bool more = tile_next < end;
-        for (int step = 0; step < steps; ++step) {
-            // (the next tile's items came before the wait of step 1, in every wave before its barrier)
-            if (step == steps - 2 && more) src = sources(next, half ^ 1);
-            run(buf, step + 2 < steps ? step + 2 : step + 2 - steps, step == 0 && !first);
-            buf ^= 1;
-            if (step == 0 && more) {  // (every wave is past its use of the other half of item_s)
-                next = look_up(tile_next);
-                fetch_items(next, half ^ 1);
+        auto walk = [&](auto live) {
+            for (int step = 0; step < steps; ++step) {
+                // (the next tile's items came before the wait of step 1, in every wave before its barrier)
+                if (step == steps - 2 && more) src = sources(next, half ^ 1);
+                run(live, buf, step + 2 < steps ? step + 2 : step + 2 - steps, step == 0 && !first);
+                buf ^= 1;
+                if (step == 0 && more) {  // (every wave is past its use of the other half of item_s)
+                    next = look_up(tile_next);
+                    fetch_items(next, half ^ 1);
+                }
             }
-        }
+        };
+        if (now.m0 + 16 * TM * wm < now.count) walk(std::true_type{});
+        else walk(std::false_type{});
 #pragma unroll
         for (int m = 0; m < TM; ++m) {  // (as many stores in every wave; those of missing items or outputs go past the end)
             const int r = 16 * (wm * TM + m) + l16;
@@ -877,7 +888,8 @@ template <bool GLU> int launch_bf16(const MoeArgs &a, hipStream_t s) {
     const int64_t most = 0xffffff00ll, x_rows = a.items / a.per_row;
     const bool stay = a.kp >= kStayLeastSteps * kStayStep && a.n % 8 == 0 && a.experts <= 1024 && x_rows * a.ldx * 2 <= most &&
                       a.w_rows * a.kp * 2 <= most && a.items * a.n * 2 <= most;
-    return shape == kMoeTile256 && stay ? launch_stay<GLU>(a, s) : launch_tiles<2, 4, 2, 2, GLU>(a, s);
+    const bool full = moe_stays(a.items, a.experts, (a.n + (GLU ? 127 : 255)) / (GLU ? 128 : 256), moe_cus());
+    return shape == kMoeTile256 && stay && full ? launch_stay<GLU>(a, s) : launch_tiles<2, 4, 2, 2, GLU>(a, s);
 }
 
 }  // namespace
