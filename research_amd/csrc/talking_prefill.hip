@@ -35,7 +35,7 @@ template <int DK> __global__ __launch_bounds__(256, 2) void talk_sums_kernel(con
     __shared__ __align__(16) uint16_t ks[kTsKeys * kPitch];
     __shared__ float biases[4][2][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, col = lane & 31;
-    const int kvh = blockIdx.y, b = talk_sequence(blockIdx.x, blockIdx.z, a.batch);
+    const int kvh = blockIdx.y, b = talk_sequence(a, blockIdx.x, blockIdx.z);
     ScoredPortion p;
     if (!scored_portion(a, b, p)) return;
     const int n_tasks = (p.n + 31) / 32 * a.n_rep;
@@ -163,7 +163,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     char *w_s = tm_lds + L::pBytes;
     __bf16 *v_all = reinterpret_cast<__bf16 *>(w_s + L::wBytes), *k_s = v_all + L::vBytes / 2;
     float *biases = reinterpret_cast<float *>(w_s + L::wBytes + L::vBytes + L::kBytes) + wave * L::biasFloats;
-    const int b = talk_sequence(blockIdx.x, blockIdx.y, a.batch);
+    const int b = talk_sequence(a, blockIdx.x, blockIdx.y);
     ScoredPortion p;
     if (!scored_portion(a, b, p)) return;
     const int row0 = (int)(gridDim.y - 1 - blockIdx.y) * kTmRows;  // (the rows with the most keys first)
