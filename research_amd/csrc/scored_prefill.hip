@@ -39,8 +39,8 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
     const int table_n = bias_n + kSpLow + kSpHigh;
     float *bias = reinterpret_cast<float *>(sp_lds + L::tiles) + wave * table_n;
     // Workgroups start in the order of their ids, and every eighth shares a die.  The rows with the most keys of all sequences come
-    // first, and sequences take turns on the dies; the second workgroup of each compute unit comes the other way round, so that
-    // the longest shares its unit with a short one.
+    // first, and sequences take turns on the dies (an odd number of them does by itself: 9 of 700 .. 4000 rows in turn 435 us, else
+    // 320); the second workgroup of each compute unit comes the other way round, so that the longest shares its unit with a short one.
     int kvh = blockIdx.x, turn = blockIdx.z, y = blockIdx.y;
     const uint64_t per = (uint64_t)gridDim.x * gridDim.y, place = per * turn + gridDim.x * (uint64_t)y + kvh;
     const uint32_t both = (uint32_t)min(2 * (uint64_t)cus, per * gridDim.z);
@@ -50,7 +50,7 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
         kvh = back % one % gridDim.x;
         y = back % one / gridDim.x;
     }
-    const int b = (y + turn) % (int)gridDim.y;
+    const int b = gridDim.y % 2 == 0 ? (y + turn) % (int)gridDim.y : y;
     ScoredPortion p;
     if (!scored_portion(a, b, p)) return;
     const int n_tasks = (p.n + 31) / 32 * a.n_rep;
