@@ -8,6 +8,7 @@ Python and nothing is routed to torch kernels.
 
 from __future__ import annotations
 
+import functools
 from typing import NamedTuple, Optional, Tuple
 
 import torch
@@ -26,13 +27,16 @@ def _ptr(t: Optional[Tensor]) -> Optional[int]:
 
 
 def _stream(t: Tensor) -> Optional[int]:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise RuntimeError(f"libpaged_attn computes only on a HIP device; got a tensor on {t.device}")
-    return torch.cuda.current_stream(t.device).cuda_stream or None
+    # (the number alone: torch.cuda.current_stream makes an object around it, 1.9 us of a call's 12)
+    return torch._C._cuda_getCurrentRawStream(t.get_device()) or None
 
 
 def _run(name: str, *args) -> None:
-    _lib.check(name, getattr(_lib.load(), name)(*args))
+    status = getattr(_lib.load(), name)(*args)
+    if status:
+        _lib.check(name, status)
 
 
 def kv_scatter(k_cache: Tensor, v_cache: Tensor, k_src: Tensor, v_src: Tensor, slots: Tensor) -> None:
@@ -334,9 +338,11 @@ def dequantize_blocks_e4m3(cache: Tensor, scale: Tensor, block_ids: Tensor, bloc
 
 def _row_stride(t: Tensor) -> int:
     """Elements between the rows of a 2-D tensor whose rows are contiguous (a column slice of a wider one)."""
-    if t.dim() != 2 or (t.shape[1] > 1 and t.stride(1) != 1):
-        raise ValueError("expected a 2-D tensor with contiguous rows")
-    return t.stride(0) if t.shape[0] > 1 else max(t.stride(0), t.shape[1])
+    if t.dim() == 2:
+        (rows, cols), (row, col) = t.shape, t.stride()
+        if cols <= 1 or col == 1:
+            return row if rows > 1 else max(row, cols)
+    raise ValueError("expected a 2-D tensor with contiguous rows")
 
 
 def _dense(*tensors: Optional[Tensor]) -> None:
@@ -595,6 +601,7 @@ def short_conv(u: Tensor, portions: Portions, weight: Tensor, bias: Optional[Ten
     return out
 
 
+@functools.lru_cache(maxsize=256)
 def gated_linear_state_floats(kind: str, dim: int, vdim: int) -> int:
     """Floats per head of a gated recurrence's state."""
     return int(_lib.load().pa_gated_linear_state_floats(_GATED[kind], dim, vdim))
@@ -622,12 +629,13 @@ def gated_linear(kind: str, q: Tensor, k: Tensor, v: Tensor, gates: Tuple[Tensor
         raise ValueError("q / k / v / out do not fit each other")
     if any(c is not None and c.numel() != heads for c in constants) or tuple(ga.shape) != (rows, heads):
         raise ValueError("gates / constants do not fit the heads")
-    if gb is not None and (tuple(gb.shape) != (rows, heads) or _row_stride(gb) != _row_stride(ga)):
+    gate_stride = _row_stride(ga)
+    if gb is not None and (tuple(gb.shape) != (rows, heads) or _row_stride(gb) != gate_stride):
         raise ValueError("the two gates differ in their rows")
     if tuple(state.shape[1:]) != (heads, gated_linear_state_floats(kind, dim, vdim)):
         raise ValueError("state of another size")
     _run("pa_gated_linear", _GATED[kind], _ptr(q), _row_stride(q), _ptr(k), _row_stride(k), _ptr(v), _row_stride(v),
-         heads_per_group, _ptr(ga), _ptr(gb), _row_stride(ga), *(_ptr(c) for c in constants), float(cap), float(q_scale),
+         heads_per_group, _ptr(ga), _ptr(gb), gate_stride, *map(_ptr, constants), float(cap), float(q_scale),
          float(den_eps), rows, _ptr(state), state.shape[0], _ptr(portions.ctx_lens), _ptr(portions.q_lens),
          _ptr(portions.q_starts), _ptr(portions.state_slots), batch, portions.max_q_len, _ptr(out), heads, dim, vdim,
          PA_DTYPE[v.dtype], _ptr(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0,
