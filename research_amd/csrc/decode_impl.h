@@ -384,27 +384,34 @@ template <int MASK> __device__ __forceinline__ float2 lane_pair(float x, int mas
         return float2{x, __shfl_xor(x, mask, PA_WAVE)};
     }
 }
-template <int MASK, int NREP, int EPL> __device__ __forceinline__ void merge_lane_pairs(RowState<NREP, EPL> &st, int mask) {
+// EXACT (32-bit pools): one rounding for a sum, as where rows are summed one after the other.  (One of the two rows has the larger
+// maximum and so a weight of one.)
+template <int MASK, bool EXACT, int NREP, int EPL> __device__ __forceinline__ void merge_lane_pairs(RowState<NREP, EPL> &st, int mask) {
 #pragma unroll
     for (int r = 0; r < NREP; ++r) {
         const float2 m = lane_pair<MASK>(st.m[r], mask);
-        const float M = fmaxf(m.x, m.y), f = __builtin_amdgcn_exp2f(st.m[r] - M);
+        const float M = fmaxf(m.x, m.y), f = __builtin_amdgcn_exp2f(EXACT ? fminf(m.x, m.y) - M : st.m[r] - M);
         st.m[r] = M;
-        const float2 l = lane_pair<MASK>(st.l[r] * f, mask);
-        st.l[r] = l.x + l.y;
+        auto sum = [&](float x) {
+            if constexpr (EXACT) {
+                const float2 p = lane_pair<MASK>(x, mask);
+                return m.x < m.y ? fmaf(p.x, f, p.y) : fmaf(p.y, f, p.x);
+            } else {
+                const float2 p = lane_pair<MASK>(x * f, mask);
+                return p.x + p.y;
+            }
+        };
+        st.l[r] = sum(st.l[r]);
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-            const float2 x = lane_pair<MASK>(st.acc[r][e] * f, mask);
-            st.acc[r][e] = x.x + x.y;
-        }
+        for (int e = 0; e < EPL; ++e) st.acc[r][e] = sum(st.acc[r][e]);
         __builtin_amdgcn_sched_barrier(0);  // (all of them at once take registers that the kernel does not have)
     }
 }
 // The rows of a wave whose lanes differ in the bits of the lane index from `low` up, merged in all of them.
-template <int NREP, int EPL> __device__ __forceinline__ void merge_lanes(RowState<NREP, EPL> &st, int low) {
-    for (int mask = low; mask < 16; mask *= 2) merge_lane_pairs<0>(st, mask);
-    if (low <= 16) merge_lane_pairs<16>(st, 16);
-    if (low <= 32) merge_lane_pairs<32>(st, 32);
+template <bool EXACT, int NREP, int EPL> __device__ __forceinline__ void merge_lanes(RowState<NREP, EPL> &st, int low) {
+    for (int mask = low; mask < 16; mask *= 2) merge_lane_pairs<0, EXACT>(st, mask);
+    if (low <= 16) merge_lane_pairs<16, EXACT>(st, 16);
+    if (low <= 32) merge_lane_pairs<32, EXACT>(st, 32);
 }
 
 template <typename KV, int D, int NREP, int HR, typename Emit>
@@ -486,7 +493,7 @@ __device__ __forceinline__ void merge_rows(RowState<NREP, RowShape<KV, D>::EPL> 
     st.fold_zero_keys();
     // The token rows of a wave first, lane against lane; the rows that are left go through LDS, as many more query heads at
     // once as there are fewer of them.
-    if (p.tpw >= 2) merge_lanes(st, p.hpw * S::LPR);
+    if (p.tpw >= 2) merge_lanes<sizeof(KV) == 4>(st, p.hpw * S::LPR);
     const int prow = wave * p.hpw + role.head_local;
     if (MS::HR < NREP && p.tpw >= 4)
         merge_rounds<KV, D, NREP, (MS::HR * 4 < NREP ? MS::HR * 4 : NREP)>(st, s_part, p, role, prow, tid, hg, rep0, emit);
