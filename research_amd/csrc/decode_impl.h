@@ -487,8 +487,8 @@ __device__ __forceinline__ void merge_rows(RowState<NREP, RowShape<KV, D>::EPL> 
     using S = RowShape<KV, D>;
     using MS = MergeShape<KV, D, NREP>;
     // (from an index that the compiler knows nothing of: places in LDS that it works out ahead of the key loop take registers
-    // that the loop does not have)
-    asm volatile("" : "+v"(tid));
+    // that the loop does not have.  A wave of one row has few places, and they are better known: 32-bit pools of 256, 61 us so, 67.)
+    if constexpr (S::RPW > 1) asm volatile("" : "+v"(tid));
     const LaneRole role = lane_role<KV, D>(tid & (PA_WAVE - 1), p);
     st.fold_zero_keys();
     // The token rows of a wave first, lane against lane; the rows that are left go through LDS, as many more query heads at
