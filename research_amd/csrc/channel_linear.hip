@@ -196,7 +196,8 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     uint4 *scores = reinterpret_cast<uint4 *>(whole + L::blocks * KD);               // per block and lane: four scores, two terms
     int *unsafe = reinterpret_cast<int *>(STATES ? scores : scores + L::blocks * 64);
 
-    const int h = blockIdx.x, seg = blockIdx.y % a.segments, vsl = blockIdx.y / a.segments, b = blockIdx.z;
+    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW));
+    const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     ClPortion p;
     if (!cl_portion(a, b, p)) return;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
@@ -469,7 +470,7 @@ template <int KD, int NW> int launch_chunks(const ClArgs &a, int batch, hipStrea
     constexpr size_t lds = ClTile<KD, NW, false>::bytes, lds_states = ClTile<KD, NW, true>::bytes;
     static_assert(lds <= 160 * 1024 && lds_states <= 160 * 1024, "LDS of one compute unit");
     const int slices = (a.vdim + 16 * NW - 1) / (16 * NW);
-    const dim3 grid((unsigned)a.heads, (unsigned)(slices * a.segments), (unsigned)batch), block(64 * NW);
+    const dim3 grid = la_grid(a.heads, slices, batch, a.segments), block(64 * NW);
     if (a.segments > 1) {
         if (int rc = la_big_lds(channel_chunk_kernel<KD, NW, true>, lds_states, "pa_channel_linear")) return rc;
         channel_chunk_kernel<KD, NW, true><<<grid, block, lds_states, s>>>(a);

@@ -149,7 +149,8 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
     __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
     __bf16 *q_s = tiles + la_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
-    const int h = blockIdx.x, seg = blockIdx.y % a.segments, vsl = blockIdx.y / a.segments, b = blockIdx.z;
+    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW));
+    const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     Portion p;
     if (!la_portion(a, b, p)) return;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
@@ -360,7 +361,7 @@ template <int KD, int NW> int launch_chunks(const LaArgs &a, int batch, hipStrea
     constexpr size_t lds = la_lds_bytes<KD, NW, false>(), lds_states = la_lds_bytes<KD, NW, true>();
     static_assert(lds <= 160 * 1024 && lds_states <= 160 * 1024, "LDS of one compute unit");
     const int slices = (a.vdim + 16 * NW - 1) / (16 * NW);
-    const dim3 grid((unsigned)a.heads, (unsigned)(slices * a.segments), (unsigned)batch), block(64 * NW);
+    const dim3 grid = la_grid(a.heads, slices, batch, a.segments), block(64 * NW);
     if (a.segments > 1) {
         if (int rc = la_big_lds(lightning_chunk_kernel<KD, NW, true>, lds_states, "pa_lightning_chunked")) return rc;
         lightning_chunk_kernel<KD, NW, true><<<grid, block, lds_states, s>>>(a);

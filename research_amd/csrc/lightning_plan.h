@@ -29,8 +29,8 @@ static inline int la_segments(int64_t workgroups, int cus, int max_len) {
 // The same for a batch whose rows are known: `per_seq` workgroups for each sequence, n_rows rows in all; together: by how much
 // a workgroup is slower when two share a compute unit (0: they cannot).  In units of a chunk of the second pass: without
 // segments the launch lasts as long as its longest sequence or, with more workgroups than compute units, its share of the
-// rows; with segments of c chunks it lasts c where a compute unit has one of them at most, else its share and half a
-// segment, and 45 % more for the first pass, half a unit per segment for the scan between the two, and two units for the
+// rows; with segments of c chunks it lasts c where a compute unit has one of them at most (with some to spare where
+// their number is a guess), 1.6 c where some have two, else its share and half a segment, and 45 % more for the first pass, half a unit per segment for the scan between the two, and two units for the
 // launches.  Measured, 16 heads of 128 x 128 (lightning; HGRN2; mLSTM with 4 of 256 x 512), us, as many segments as
 // compute units / workgroups -> by this rule: 8 sequences of 400 .. 4000 rows 187 -> 128, 305 -> 216, 311 -> 249; 12 of them 239 ->
 // 161, 389 -> 284, 423 -> 341; 12 equal ones stay unsegmented (172, 276, 312; in segments 201, 354, 398).
@@ -43,9 +43,13 @@ static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, 
     int segments = 1;
     for (int s = 2; s <= most; ++s) {
         const double c = (chunks + s - 1) / s;
-        const double spread = rows / c + 0.5 * batch, live = per_seq * (spread < (double)batch * s ? spread : (double)batch * s);
+        const double spread = rows / c + 0.5 * batch, all = (double)batch * s, live = per_seq * (spread < all ? spread : all);
         double part = c;
-        if (live > cus) part = live <= 2.0 * cus && together > 0 ? c * together : share + 0.5 * c;
+        if (live > (spread < all ? 0.85 : 1.0) * cus) {
+            part = share + 0.5 * c;
+            if (live <= 2.0 * cus && together > 0) part = c * together;
+            else if (live <= 1.3 * cus && part < 1.6 * c) part = 1.6 * c;
+        }
         if (part < c) part = c;
         const double t = 1.45 * part + 0.5 * s + 2.0;
         if (t < best) {
