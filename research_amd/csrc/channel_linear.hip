@@ -25,7 +25,7 @@ struct ClArgs {
     void *out;  // [rows][heads * vdim]
     float *ws;  // segment states: S [dp][vp], the segment's factors [dp], padding
     int heads, dim, vdim, dp, vp;
-    int segments, seg_rows;
+    int batch, segments, seg_rows;
 };
 
 struct ClPortion {
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     uint4 *scores = reinterpret_cast<uint4 *>(whole + L::blocks * KD);               // per block and lane: four scores, two terms
     int *unsafe = reinterpret_cast<int *>(STATES ? scores : scores + L::blocks * 64);
 
-    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW));
+    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW), a.batch);
     const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     ClPortion p;
     if (!cl_portion(a, b, p)) return;
@@ -545,6 +545,7 @@ extern "C" int pa_channel_linear(const void *q, int64_t q_stride, int q_act, con
                                     cl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
                                     pa_aligned16(workspace));
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
+    a.batch = batch;
     a.seg_rows = la_segment_rows(max_q_len, a.segments);
     a.ws = (float *)workspace;
     const bool wide = la_value_cols(vdim) == 128;

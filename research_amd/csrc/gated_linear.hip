@@ -37,7 +37,7 @@ struct GlArgs {
     void *out;  // [rows][heads * vdim]
     float *ws;  // segment states: S [dp][vp], n [dp], m, log decay, starting m
     int heads, per_group, dim, vdim, dp, vp;
-    int segments, seg_rows;
+    int batch, segments, seg_rows;
 };
 
 struct GlPortion {
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
     __bf16 *q_s = tiles + gl_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
-    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW));
+    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW), a.batch);
     const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     GlPortion p;
     if (!gl_portion(a, b, p)) return;
@@ -716,6 +716,7 @@ extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const 
                                     gl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
                                     pa_aligned16(workspace));
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
+    a.batch = batch;
     a.seg_rows = la_segment_rows(max_q_len, a.segments);
     a.ws = (float *)workspace;
     return kind == kSsd ? launch_chunks_kind<kSsd>(a, batch, s) : launch_chunks_kind<kMlstm>(a, batch, s);

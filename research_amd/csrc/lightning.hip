@@ -26,7 +26,7 @@ struct LaArgs {
     void *out;  // [rows][heads * vdim]
     float *ws;  // segment states
     int heads, dim, vdim, dp, vp;
-    int segments, seg_rows;
+    int batch, segments, seg_rows;
 };
 
 // The portion of sequence b: rows [row0, row0 + n), the first at position pos0.  False: nothing to do.
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
     __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
     __bf16 *q_s = tiles + la_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
-    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW));
+    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW), a.batch);
     const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     Portion p;
     if (!la_portion(a, b, p)) return;
@@ -460,6 +460,7 @@ extern "C" int pa_lightning_chunked(const void *u, int64_t u_stride, int64_t n_r
                                     la_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
                                     pa_aligned16(workspace));
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
+    a.batch = batch;
     a.seg_rows = la_segment_rows(max_q_len, a.segments);
     a.ws = (float *)workspace;
     hipStream_t s = (hipStream_t)stream;

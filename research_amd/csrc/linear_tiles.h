@@ -151,21 +151,23 @@ __device__ __forceinline__ LaSplit la_split_weighted(bf8 raw, const f4 &x, const
 }
 
 // Which piece a workgroup of a chunked kernel takes.  Workgroups go to the dies, and there to groups of compute units, in the order
-// of their ids, and wait for the one whose turn it is: so the heads and value slices of a segment lie side by side, then sequences,
-// and the last segments, of which only long portions have any, behind all others.  (With a portion's segments side by side half of
-// the units were idle: 5 portions of 1100 .. 2400 rows in 4 segments, 4 heads of 256 x 512, mLSTM 274 us, so 153.)  A single
-// sequence's slices of one segment, which read the same keys, share a die (15999 rows: 236 us, else 245).
+// of their ids, and wait for the one whose turn it is.  With 16 heads or 32 a segment fills its turn by itself, and a portion's
+// segments follow each other (8 portions of 400 .. 4000 rows, lightning, 16 heads of 128 x 128: 151 us, with sequences side by side
+// 211).  With fewer the places of the last segments, which only long portions have, would come to the same units each time (5
+// portions of 1100 .. 2400 rows in 4 segments, 4 heads of 256 x 512, mLSTM 274 us, with sequences side by side 153): so heads and
+// value slices lie side by side, then sequences, and the last segments behind all others.  A single sequence's slices of one
+// segment, which read the same keys, share a die (15999 rows: 236 us, else 245).
 struct LaPlace {
     int h, vsl, b, seg;
 };
-__device__ __forceinline__ LaPlace la_place(int segments, int slices) {
+__host__ __device__ __forceinline__ bool la_by_portion(int heads, int batch, int segments) { return segments == 1 || batch == 1 || heads % 16 == 0; }
+__device__ __forceinline__ LaPlace la_place(int segments, int slices, int batch) {
     const int h = blockIdx.x, y = blockIdx.y, z = blockIdx.z;
-    if (segments == 1) return LaPlace{h, y, z, 0};
-    return gridDim.z == 1 ? LaPlace{h, y / segments, 0, y % segments} : LaPlace{h, y % slices, y / slices, z};
+    return la_by_portion(gridDim.x, batch, segments) ? LaPlace{h, y / segments, z, y % segments} : LaPlace{h, y % slices, y / slices, z};
 }
 inline dim3 la_grid(int heads, int slices, int batch, int segments) {  // (segments > 1: batch and vdim are bounded by their workspace)
-    if (segments == 1) return dim3((unsigned)heads, (unsigned)slices, (unsigned)batch);
-    return batch == 1 ? dim3((unsigned)heads, (unsigned)(slices * segments), 1) : dim3((unsigned)heads, (unsigned)(slices * batch), (unsigned)segments);
+    return la_by_portion(heads, batch, segments) ? dim3((unsigned)heads, (unsigned)(slices * segments), (unsigned)batch)
+                                                 : dim3((unsigned)heads, (unsigned)(slices * batch), (unsigned)segments);
 }
 
 constexpr int kLaPitchA = 72;  // bf16 per row of the decayed scores
