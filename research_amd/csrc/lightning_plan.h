@@ -29,11 +29,12 @@ static inline int la_segments(int64_t workgroups, int cus, int max_len) {
 // The same for a batch whose rows are known: `per_seq` workgroups for each sequence, n_rows rows in all; together: by how much
 // a workgroup is slower when two share a compute unit (0: they cannot).  In units of a chunk of the second pass: without
 // segments the launch lasts as long as its longest sequence or, with more workgroups than compute units, its share of the
-// rows; with segments of c chunks it lasts c where a compute unit has one of them at most (with some to spare where
-// their number is a guess), 1.6 c where some have two, else its share and half a segment, and 45 % more for the first pass, half a unit per segment for the scan between the two, and two units for the
-// launches.  Measured, 16 heads of 128 x 128 (lightning; HGRN2; mLSTM with 4 of 256 x 512), us, as many segments as
-// compute units / workgroups -> by this rule: 8 sequences of 400 .. 4000 rows 187 -> 128, 305 -> 216, 311 -> 249; 12 of them 239 ->
-// 161, 389 -> 284, 423 -> 341; 12 equal ones stay unsegmented (172, 276, 312; in segments 201, 354, 398).
+// rows; with segments of c chunks it lasts c where a compute unit has one of them at most (with some to spare where their number
+// is a guess), 1.6 c where some have two, else its share and half a segment, and 45 % more for the first pass, half a unit per
+// segment for the scan between the two, and two units for the
+// launches.  Measured, 16 heads of 128 x 128 (lightning; HGRN2; SSD), us, as many segments as compute units / workgroups (of portions,
+// not of rows) -> by this rule: 6 sequences of 400 .. 4000 rows 156 -> 90, 270 -> 122, 139 -> 77; 8 of them 230 -> 151, 398 -> 258,
+// 201 -> 133; 12 of them 320 -> 177, 545 -> 296, 273 -> 153; 12 equal ones stay unsegmented (164, 275, 144).
 static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, int most) {
     if (batch <= 0 || per_seq <= 0 || max_len <= 0) return 1;
     if (n_rows > batch * max_len) n_rows = batch * max_len;
