@@ -132,10 +132,10 @@ template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
 // Bound by the vector instructions that turn 32-bit factors into two bf16 terms and by the waits between the stages of a chunk
 // (the matrix cores are busy a sixth of the time).  So a tile lies in LDS in the one layout that both of its products read (K by
 // rows and, with transposing reads, by columns), results leave the registers straight for the output, and the first pass leaves out
-// each portion's last segment, whose state the second pass itself writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128:
-// first pass 55 -> 48 us, second 127 -> 101, with five segments of unequal sequences instead of two.
+// each portion's last segment, whose state the second pass itself writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128,
+// in five segments: first pass 55 -> 47 us, second 127 -> 116.
 // (At dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
-// chunk, let two share one, which was 10 % faster where there were two and 3 to 8 % slower where not.)
+// chunk, let two share one, which was 13 % faster where there were two, 101 us here, and 3 to 8 % slower where not.)
 template <int KD, int NW, bool STATES>
 __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArgs a) {
     constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
