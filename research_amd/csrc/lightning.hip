@@ -134,10 +134,11 @@ template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
 // rows and, with transposing reads, by columns), results leave the registers straight for the output, and the first pass leaves out
 // each portion's last segment, whose state the second pass itself writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128,
 // in five segments: first pass 55 -> 47 us, second 127 -> 116.
-// (At dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
-// chunk, let two share one, which was 13 % faster where there were two, 101 us here, and 3 to 8 % slower where not.)
-template <int KD, int NW, bool STATES>
-__global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArgs a) {
+// PAIR: at dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
+// chunk, let two share one: 13 % faster where there are two (101 us here; 12 prompts of 400 .. 4000 rows, all passes, 180 -> 163), and
+// 3 to 8 % slower where not.
+template <int KD, int NW, bool STATES, bool PAIR>
+__global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(const LaArgs a) {
     constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
@@ -230,6 +231,7 @@ __global__ __launch_bounds__(64 * NW, 2) void lightning_chunk_kernel(const LaArg
         if (r0 + kLaChunk < r_end) fetch(r0 + kLaChunk);
         __syncthreads();
 
+        const int lr = PAIR ? la_again(tid) : tid, l16 = lr & 15, g = (lr & 63) >> 4;
         f4 o[4];  // O^T: v = 4 g + i of the wave's columns, t = 16 tt + l16
         if constexpr (!STATES) {
             // score tiles (st, rt): keys 16 st + 4 g + i, rows 16 rt + l16
@@ -357,21 +359,32 @@ __global__ __launch_bounds__(256) void lightning_scan_kernel(const LaArgs a) {
     }
 }
 
-template <int KD, int NW> int launch_chunks(const LaArgs &a, int batch, hipStream_t s) {
+template <int KD, int NW, bool PAIR> int launch_passes(const LaArgs &a, const dim3 &grid, int batch, hipStream_t s) {
     constexpr size_t lds = la_lds_bytes<KD, NW, false>(), lds_states = la_lds_bytes<KD, NW, true>();
     static_assert(lds <= 160 * 1024 && lds_states <= 160 * 1024, "LDS of one compute unit");
-    const int slices = (a.vdim + 16 * NW - 1) / (16 * NW);
-    const dim3 grid = la_grid(a.heads, slices, batch, a.segments), block(64 * NW);
+    const dim3 block(64 * NW);
     if (a.segments > 1) {
-        if (int rc = la_big_lds(lightning_chunk_kernel<KD, NW, true>, lds_states, "pa_lightning_chunked")) return rc;
-        lightning_chunk_kernel<KD, NW, true><<<grid, block, lds_states, s>>>(a);
+        if (int rc = la_big_lds(lightning_chunk_kernel<KD, NW, true, false>, lds_states, "pa_lightning_chunked")) return rc;
+        lightning_chunk_kernel<KD, NW, true, false><<<grid, block, lds_states, s>>>(a);
         const unsigned gx = (unsigned)(((int64_t)a.dp * a.vp / 4 + 255) / 256);
         lightning_scan_kernel<<<dim3(gx, (unsigned)a.heads, (unsigned)batch), dim3(256), 0, s>>>(a);
     }
-    if (int rc = la_big_lds(lightning_chunk_kernel<KD, NW, false>, lds, "pa_lightning_chunked")) return rc;
-    lightning_chunk_kernel<KD, NW, false><<<grid, block, lds, s>>>(a);
+    if (int rc = la_big_lds(lightning_chunk_kernel<KD, NW, false, PAIR>, lds, "pa_lightning_chunked")) return rc;
+    lightning_chunk_kernel<KD, NW, false, PAIR><<<grid, block, lds, s>>>(a);
     PA_CHECK_LAUNCH("pa_lightning_chunked");
     return PA_OK;
+}
+
+template <int KD, int NW> int launch_chunks(const LaArgs &a, int batch, hipStream_t s) {
+    const int slices = (a.vdim + 16 * NW - 1) / (16 * NW);
+    const dim3 grid = la_grid(a.heads, slices, batch, a.segments);
+    // unequal portions in more segments than compute units (a segment for each of its lengths, and half a one per portion)
+    const double parts = (double)a.n_rows / a.seg_rows + 0.5 * batch;
+    const bool pair = KD == 128 && NW == 8 && a.segments > 1 && parts < (double)batch * a.segments && parts * a.heads * slices > 1.1 * la_cus();
+    if constexpr (KD == 128 && NW == 8) {
+        if (pair) return launch_passes<KD, NW, true>(a, grid, batch, s);
+    }
+    return launch_passes<KD, NW, false>(a, grid, batch, s);
 }
 
 template <typename T> void launch_recurrent(const LaArgs &a, int batch, hipStream_t s) {

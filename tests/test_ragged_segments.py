@@ -51,17 +51,18 @@ int main() {
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("heads,dim,vdim", [(32, 64, 64), (32, 64, 128), (16, 128, 128)])
-def test_a_batch_of_unequal_prompts_in_segments(heads, dim, vdim):
+@pytest.mark.parametrize("heads,dim,vdim,longest", [(32, 64, 64, 2500), (32, 64, 128, 2500), (16, 128, 128, 2500), (16, 128, 128, 8000)])
+def test_a_batch_of_unequal_prompts_in_segments(heads, dim, vdim, longest):
     import torch
 
     from tests.gpu_helpers import announce
     from tests.test_gpu_lightning import Case
 
-    announce(f"ragged segments {heads}x{dim}x{vdim}")
+    announce(f"ragged segments {heads}x{dim}x{vdim} {longest}")
     decay = [1.0 - 0.5 ** (1 + i * 12 / heads) for i in range(heads)]
     # one sequence of many segments, some that end inside the first, on and beside a segment's edge
-    lens = [2500, 1, 64, 511, 512, 513, 1025, 700, 30, 2000]
+    # (8000: more of them than compute units, two of which then share one)
+    lens = [longest, 1, 64, 511, 512, 513, longest // 3, 700, 30, longest * 3 // 5]
     case = Case(lens, heads, dim, vdim, decay, torch.bfloat16, seed=5)
     slots = [(3 * b + 1) % len(lens) for b in range(len(lens))]
     head = [(b, 0, (n + 1) // 2) for b, n in enumerate(lens)]
