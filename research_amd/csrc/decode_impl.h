@@ -719,8 +719,8 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
     if (B <= kWaveScanBatch) {
         // Every wave computes the whole prefix sum by itself: lane l of round c holds sequence 64 c + l, the lengths
         // of all rounds are requested at once, a round is scanned with data-parallel moves and the rounds are
-        // chained through a scalar.  All four waves store the same values to the same LDS words and each reads
-        // back what it has itself written, so no barrier stands between the lengths and the first table entry.
+        // chained through a scalar.  All four waves store the same values to the same LDS words, each word once, and
+        // each reads back what it has itself written, so no barrier stands between the lengths and the first table entry.
         int n[kWaveScanBatch / PA_WAVE];
 #pragma unroll
         for (int c = 0; c < kWaveScanBatch / PA_WAVE; ++c) {
@@ -738,10 +738,7 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
             }
             return carry;
         };
-        int carry = scan(1, true);
-        run = plan_run_blocks((int64_t)carry * planes, (int64_t)planes * B, (int)gridDim.x,
-                              [&](int u) { return (int64_t)scan(u, false) * planes; });
-        if (run > 1) carry = scan(run, true);
+        const int carry = plan_wave_prefix(planes, B, (int)gridDim.x, run, scan);
         if (lane == 0) s_prefix[B] = carry;
         if (blockIdx.x == 0 && wave == 0)
             for (int b = lane; b <= B; b += PA_WAVE) a.block_prefix[b] = s_prefix[b];

@@ -106,10 +106,17 @@ constexpr int kPlanRunMost = 4, kPlanShortBlocks = 48;
 template <typename F> PA_PLAN_FN int plan_run_blocks(int64_t total, int64_t keys, int grid, F units) {
     if (total > (int64_t)kPlanRunMost * grid) return 1;
     for (int u = total > keys * kPlanShortBlocks ? kPlanRunMost : 1; u <= kPlanRunMost; u *= 2)
-        if (units(u) <= grid) return u;
+        if ((u == 1 ? total : units(u)) <= grid) return u;
     return 1;
 }
 PA_PLAN_FN int plan_runs_of(int blocks, int u) { return (blocks + u - 1) / u; }
+// The same where every wave fills the prefix table by itself, without a barrier: scan(u, keep) returns the runs of u blocks of all
+// sequences and, with `keep`, stores the table.  Only the final table is ever stored: waves that lag behind store what the others read.
+template <typename F> PA_PLAN_FN int plan_wave_prefix(int planes, int batch, int grid, int &run, F scan) {
+    run = plan_run_blocks((int64_t)scan(1, false) * planes, (int64_t)planes * batch, grid,
+                          [&](int u) { return (int64_t)scan(u, false) * planes; });
+    return scan(run, true);
+}
 // Workgroups that take part in a launch of `total` runs.
 PA_PLAN_FN int plan_run_grid(int64_t total, int grid) { return total < grid ? (int)total : grid; }
 

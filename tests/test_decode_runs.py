@@ -1,5 +1,7 @@
 """Short launches of the split pass: runs of blocks, one workgroup each (``plan_run_blocks`` of ``decode_plan.h``, compiled with
-g++).  Every (plane, sequence, block) lies in one run of one workgroup, and where the runs fit the grid no workgroup has two."""
+g++).  Every (plane, sequence, block) lies in one run of one workgroup, and where the runs fit the grid no workgroup has two.
+The waves of a workgroup fill the prefix table of runs without a barrier, so no word of it is ever stored with two values
+(``plan_wave_prefix``).  On the device: launches of runs of two and four blocks, merged in either way."""
 
 import ctypes
 import os
@@ -7,6 +9,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
@@ -37,6 +40,28 @@ extern "C" int replay(const int *lens, int batch, int planes, int bs, int window
     for (auto &s : seen) for (int n : s) if (n != 1) return -3;
     return u;
 }
+// Every store that a wave makes to the prefix table, in order.  A wave reads the table behind its own stores, while another one may
+// still have all of its own before it: each of them has to store what is already there.
+extern "C" int stores(const int *lens, int batch, int planes, int bs, int window, int grid) {
+    std::vector<std::vector<int>> stored(batch);
+    int run = 0;
+    auto scan = [&](int u, bool keep) {
+        int carry = 0;
+        for (int b = 0; b < batch; ++b) {
+            if (keep) stored[b].push_back(carry);
+            carry += plan_runs_of(plan_blocks_of(lens[b], bs, window), u);
+        }
+        return carry;
+    };
+    const int total = plan_wave_prefix(planes, batch, grid, run, scan);
+    for (int b = 0, before = 0; b <= batch; ++b) {
+        if (b == batch) return total == before ? run : -1;
+        if (stored[b].empty()) return -2;
+        for (int x : stored[b]) if (x != before) return -3;
+        before += plan_runs_of(plan_blocks_of(lens[b], bs, window), run);
+    }
+    return -4;
+}
 """
 
 
@@ -46,12 +71,15 @@ def replay(tmp_path_factory):
     (at / "r.cpp").write_text(SOURCE)
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "research_amd", "csrc"), "-o", str(at / "r.so"),
                     str(at / "r.cpp")], check=True)
-    fn = ctypes.CDLL(str(at / "r.so")).replay
-    fn.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 5
+    lib = ctypes.CDLL(str(at / "r.so"))
+    for fn in (lib.replay, lib.stores):
+        fn.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 5
 
     def run(lens, planes, bs=16, window=0, grid=512):
         lens = np.ascontiguousarray(lens, np.int32)
-        return fn(lens.ctypes.data, len(lens), planes, bs, window, grid)
+        u = lib.replay(lens.ctypes.data, len(lens), planes, bs, window, grid)
+        assert lib.stores(lens.ctypes.data, len(lens), planes, bs, window, grid) == u
+        return u
     return run
 
 
@@ -74,3 +102,31 @@ def test_lines_of_the_rule(replay):
     assert replay([80] * 512, 1) == 1                                   # more than the grid takes in runs of four
     assert replay([768], 1) == 1 and replay([784], 1) == 4              # 48 and 49 blocks of a sequence
     assert replay([0, 0], 2) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("run,lens,hq,hkv,d,kv", [
+    (2, [100] * 64, 32, 8, 128, "bf16"),                 # two launches
+    (4, [4096], 32, 8, 128, "bf16"),
+    (4, [2000, 0, 1999, 2000, 1], 32, 8, 128, "f16"),
+    (4, [1000] * 16, 14, 2, 64, "bf16"),
+    (2, [700] * 16, 8, 2, 64, "f32"),
+    (2, [50, 49, 64, 33] * 32, 32, 8, 128, "bf16"),      # the pieces merged in the one launch
+    (4, [128, 113, 97, 128] * 32, 32, 8, 128, "bf16"),
+])
+def test_launches_of_runs_on_the_device(replay, run, lens, hq, hkv, d, kv):
+    from oracle import paged_oracle as po
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.test_gpu_decode_merge import Batch
+
+    planes = {(32, 8, 128): 2, (14, 2, 64): 1, (8, 2, 64): 1}[hq, hkv, d]
+    assert replay(lens, planes, grid=2 * torch.cuda.get_device_properties(0).multi_processor_count) == run
+    announce(f"decode runs of {run}: {len(lens)} x {lens[0]} {hq}/{hkv}x{d} {kv}")
+    b = Batch(lens, hq, hkv, d, kv, seed=run)
+    (k, v, _, _), _ = b.device_pools()
+    q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
+    ws, tables = ops.decode_workspace(q, k), tables_to_device(b.tables)
+    got = ops.decode(q, k, v, tables, n, b.bs, b.scale, ws)
+    assert_close(got, po.paged_decode(b.q, b.k, b.v, b.tables, b.lens, b.bs, b.scale), b.tol, "runs of blocks")
+    assert torch.equal(ops.decode(q, k, v, tables, n, b.bs, b.scale, ws), got)
