@@ -13,6 +13,7 @@
 // window 1024 and cap 176 -> 147, no window 277 -> 192, one prompt of 4000 rows 188 -> 145.
 #include "prefill_mfma.h"
 #include "scored_attn.h"
+#include "sequence_turns.h"
 
 namespace {
 
@@ -38,9 +39,11 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, col = lane & 31;
     const int table_n = bias_n + kSpLow + kSpHigh;
     float *bias = reinterpret_cast<float *>(sp_lds + L::tiles) + wave * table_n;
-    // Workgroups start in the order of their ids, and every eighth shares a die.  The rows with the most keys of all sequences come
-    // first, and sequences take turns on the dies (an odd number of them does by itself: 9 of 700 .. 4000 rows in turn 435 us, else
-    // 320); the second workgroup of each compute unit comes the other way round, so that the longest shares its unit with a short one.
+    // The rows with the most keys of all sequences come first, and sequences take turns on the dies and inside them (an odd number of
+    // them does by itself: 9 of 700 .. 4000 rows in turn 435 us, else 320); the second workgroup of each compute unit comes the other
+    // way round, so that the longest shares its unit with a short one.  8 sequences of 400 .. 4000 rows, 16 heads of 128, in turn, on the
+    // dies alone, with fixed places: over one head of keys 185 / 406 / 659 us, two 172 / 239 / 627, four 172 / 184 / 625, eight 184 / 185 /
+    // 366, sixteen 176 / 176 / 228 (unordered about 240); 4 of them over four 200 / 326 / 277; 8 equal ones 93 / 95 / 91.
     int kvh = blockIdx.x, turn = blockIdx.z, y = blockIdx.y;
     const uint64_t per = (uint64_t)gridDim.x * gridDim.y, place = per * turn + gridDim.x * (uint64_t)y + kvh;
     const uint32_t both = (uint32_t)min(2 * (uint64_t)cus, per * gridDim.z);
@@ -50,7 +53,7 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
         kvh = back % one % gridDim.x;
         y = back % one / gridDim.x;
     }
-    const int b = gridDim.y % 2 == 0 ? (y + turn) % (int)gridDim.y : y;
+    const int b = gridDim.y % 2 == 0 ? sequence_in_turn(y, turn, (int)gridDim.y) : y;
     ScoredPortion p;
     if (!scored_portion(a, b, p)) return;
     const int n_tasks = (p.n + 31) / 32 * a.n_rep;

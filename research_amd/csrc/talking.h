@@ -5,6 +5,7 @@
 // lse = log2 of the sum of 2^(s log2 e) per row and head.
 #pragma once
 #include "scored_attn.h"
+#include "sequence_turns.h"
 
 struct TalkArgs : ScoredArgs {  // (q1, n1: the queries; cap, bias, sink, window unused)
     const float *size, *rate;   // [heads], or NULL: no distance bias
@@ -42,7 +43,7 @@ __device__ __forceinline__ float talk_masked_bias(float size, float rate, int di
 // ones with 32 heads of 96 x 64: 91 us, in turn 100; 16 of 500 tokens 77, in turn 80).
 __device__ __forceinline__ int talk_sequence(const TalkArgs &a, int x, int y) {
     const bool turn = a.batch % 2 == 0 && a.n_rows != (int64_t)a.batch * a.max_q_len;
-    return turn ? (int)((uint32_t)(x + y + (y >> 3)) % (uint32_t)a.batch) : x;
+    return turn ? sequence_in_turn(x, y, a.batch) : x;
 }
 
 constexpr int kTalkMaxHeads = 128;
