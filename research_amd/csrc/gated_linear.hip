@@ -234,6 +234,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     constexpr int kNd = (KD / 32 + NW - 1) / NW;  // kMlstm: 32-row pieces of n per wave
+    // Places in LDS are worked out again in every chunk only where registers run out, or where two workgroups share a compute unit and
+    // gain by it.  16 prompts of 900 .. 1000 rows, 16 heads, us, again -> kept: mLSTM 128 x 128 113 -> 108, 256 x 64 177 -> 166, but
+    // 256 x 128 171 -> 317 (spills); SSD 128 x 128 87 -> 81, 256 x 128 143 -> 134, 128 x 64 with 32 heads 105 -> 107.
+    constexpr bool kAgain = KIND == kMlstm ? KD == 256 && NW == 8 : KD >= 128 && NW == 4;
     extern __shared__ __align__(16) char lds[];
     GlRows *rows = reinterpret_cast<GlRows *>(lds);
     float *nq_s = reinterpret_cast<float *>(rows + (STATES ? 2 : 1));  // kMlstm: n . q per row, two parts of the score sums, n
@@ -330,7 +334,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     fetch(r_beg);
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
-        const int lt = la_again(tid);
+        const int lt = kAgain ? la_again(tid) : tid;
 #pragma unroll
         for (int i = 0; i < kKPass; ++i) {
             const int blk = lt + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
         if (r0 + kLaChunk < r_end) fetch(r0 + kLaChunk);
         __syncthreads();
 
-        const int lr = KD == 256 ? la_again(tid) : tid, l16 = lr & 15, g = (lr & 63) >> 4;
+        const int lr = kAgain && KD == 256 ? la_again(tid) : tid, l16 = lr & 15, g = (lr & 63) >> 4;
         f4 o[4];  // O^T: v = 4 g + i of the wave's columns, t = 16 tt + l16
         if constexpr (!STATES) {
             // score tiles (st, rt): keys 16 st + 4 g + i, rows 16 rt + l16
