@@ -142,6 +142,10 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
+    // Places in memory and in LDS are worked out again where registers run out (16 prompts of 900 .. 1000 rows, 16 heads of 256 x 64:
+    // 141 us, else 236), those in LDS also where 64 x 64 gains a little by it (4 heads, 8 prompts of 400 .. 4000 rows, 46.3, else 48.1);
+    // elsewhere they are kept (one prompt of 2000 rows, 16 heads of 128 x 128, 67.9, else 71.3; 32 of 128 x 64, 121, else 125).
+    constexpr bool kFar = PAIR || (KD == 256 && NW == 4), kAgain = kFar || (KD == 64 && NW == 4);
     extern __shared__ __align__(16) char lds[];
     float *rev = reinterpret_cast<float *>(lds);  // decay from row s to the last row of a whole chunk ...
     float *rev_tail = rev + 64;                   // ... and of a portion's last chunk
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     auto fetch = [&](int r0) {
         const int rows = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
         const int64_t at = (int64_t)r0 * a.ldu;
-        const int ft = la_again(tid);
+        const int ft = kFar ? la_again(tid) : tid;
         auto koff = [&](int i) {
             const int blk = ft + kThr * i;
             return blk < kKBlocks ? la_block_off(a.ldu, blk / kDB * 4, blk % kDB * 4, a.dim) : kLaOutside;
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     fetch(r_beg);
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
-        const int lt = la_again(tid);
+        const int lt = kAgain ? la_again(tid) : tid;
 #pragma unroll
         for (int i = 0; i < kKPass; ++i) {
             const int blk = lt + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
