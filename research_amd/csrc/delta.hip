@@ -378,7 +378,9 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
     LaBlock qb[kKB], kb[kKB], vb[kVB];
     la_u4 mb[kMB];
     float keep_next = 0.f, row_g0 = 0.f, row_g1 = 0.f, row_g2 = 0.f;
-    auto again = [](int x) { return kFew ? x : la_again(x); };  // (with too few registers places in memory are worked out again)
+    // (with too few registers places in memory are worked out again: 48 heads of 128 x 128, 8 prompts of 900 .. 1000 rows, 257 us, else
+    // 328; of 64 x 128, which has them, 216, else 225)
+    auto again = [](int x) { return kFew || KD == 64 ? x : la_again(x); };
     // 16-byte piece `at` of T's and C's terms: its row of the four, its column.  A wave with registers for its places leaves out the
     // quarter above the diagonal blocks of 32.
     auto piece = [](int at, int &row, int &col) {
