@@ -143,9 +143,10 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     // Places in memory and in LDS are worked out again where registers run out (16 prompts of 900 .. 1000 rows, 16 heads of 256 x 64:
-    // 141 us, else 236), those in LDS also where 64 x 64 gains a little by it (4 heads, 8 prompts of 400 .. 4000 rows, 46.3, else 48.1);
-    // elsewhere they are kept (one prompt of 2000 rows, 16 heads of 128 x 128, 67.9, else 71.3; 32 of 128 x 64, 121, else 125).
-    constexpr bool kFar = PAIR || (KD == 256 && NW == 4), kAgain = kFar || (KD == 64 && NW == 4);
+    // 141 us, else 236), those in LDS also at dim 64, where two workgroups of eight waves share a compute unit only so (16 heads of
+    // 64 x 128, 9 prompts of 700 .. 4000 rows: 129 us, else 147); elsewhere they are kept (one prompt of 2000 rows, 16 heads of 128 x 128,
+    // 67.9, else 71.3; 32 of 128 x 64, 121, else 125).
+    constexpr bool kFar = PAIR || (KD == 256 && NW == 4), kAgain = kFar || KD == 64;
     extern __shared__ __align__(16) char lds[];
     float *rev = reinterpret_cast<float *>(lds);  // decay from row s to the last row of a whole chunk ...
     float *rev_tail = rev + 64;                   // ... and of a portion's last chunk
