@@ -234,10 +234,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     constexpr int kNd = (KD / 32 + NW - 1) / NW;  // kMlstm: 32-row pieces of n per wave
-    // Places in LDS are worked out again in every chunk only where registers run out, or where two workgroups share a compute unit and
-    // gain by it.  16 prompts of 900 .. 1000 rows, 16 heads, us, again -> kept: mLSTM 128 x 128 113 -> 108, 256 x 64 177 -> 166, but
-    // 256 x 128 171 -> 317 (spills); SSD 128 x 128 87 -> 81, 256 x 128 143 -> 134, 128 x 64 with 32 heads 105 -> 107.
-    constexpr bool kAgain = KIND == kMlstm ? KD == 256 && NW == 8 : KD >= 128 && NW == 4;
+    // Places in LDS are worked out again in every chunk only where registers run out, or where that lets a second workgroup into a compute
+    // unit.  16 prompts of 900 .. 1000 rows, 16 heads, us, again -> kept: mLSTM 128 x 128 113 -> 108, 256 x 64 177 -> 166, but
+    // 256 x 128 171 -> 317 (spills); SSD 128 x 128 87 -> 81, 256 x 128 143 -> 134, 128 x 64 with 32 heads 105 -> 107; first pass of mLSTM
+    // 128 x 256, 8 heads, 6 prompts of 400 .. 4000 rows, 41 -> 54 (123 registers -> 133).
+    constexpr bool kAgain = STATES || (KIND == kMlstm ? KD == 256 && NW == 8 : KD >= 128 && NW == 4);
     extern __shared__ __align__(16) char lds[];
     GlRows *rows = reinterpret_cast<GlRows *>(lds);
     float *nq_s = reinterpret_cast<float *>(rows + (STATES ? 2 : 1));  // kMlstm: n . q per row, two parts of the score sums, n
