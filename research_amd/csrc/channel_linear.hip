@@ -196,10 +196,10 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     uint4 *scores = reinterpret_cast<uint4 *>(whole + L::blocks * KD);               // per block and lane: four scores, two terms
     int *unsafe = reinterpret_cast<int *>(STATES ? scores : scores + L::blocks * 64);
 
-    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW), a.batch);
-    const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
+    LaPlace place;
     ClPortion p;
-    if (!cl_portion(a, b, p)) return;
+    if (!la_place(a, (a.vdim + 16 * NW - 1) / (16 * NW), place, p)) return;
+    const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
     // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
     const bool last = r_end == p.n;

@@ -155,10 +155,10 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
     __bf16 *q_s = tiles + la_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
-    const LaPlace place = la_place(a.segments, (a.vdim + 16 * NW - 1) / (16 * NW), a.batch);
-    const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
+    LaPlace place;
     Portion p;
-    if (!la_portion(a, b, p)) return;
+    if (!la_place(a, (a.vdim + 16 * NW - 1) / (16 * NW), place, p)) return;
+    const int h = place.h, seg = place.seg, vsl = place.vsl, b = place.b;
     const int r_beg = seg * a.seg_rows, r_end = r_beg + a.seg_rows < p.n ? r_beg + a.seg_rows : p.n;
     // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
     const bool last = r_end == p.n;

@@ -4,6 +4,12 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#if defined(__HIPCC__)
+#define PA_LA_FN __host__ __device__ inline __attribute__((always_inline))
+#else
+#define PA_LA_FN static inline
+#endif
+
 constexpr int kLaChunk = 64;      // rows multiplied at once
 constexpr int kLaMinSegChunks = 8;  // a segment is at least this many chunks long
 constexpr int kLaMaxSegments = 64;
@@ -29,28 +35,24 @@ static inline int la_segments(int64_t workgroups, int cus, int max_len) {
 // The same for a batch whose rows are known: `per_seq` workgroups for each sequence, n_rows rows in all; together: by how much
 // a workgroup is slower when two share a compute unit (0: they cannot).  In units of a chunk of the second pass: without
 // segments the launch lasts as long as its longest sequence or, with more workgroups than compute units, its share of the
-// rows; with segments of c chunks it lasts c where a compute unit has one of them at most (with some to spare where their number
-// is a guess), 1.6 c where some have two, else its share and half a segment, and 45 % more for the first pass, half a unit per
-// segment for the scan between the two, and two units for the
-// launches.  Measured, 16 heads of 128 x 128 (lightning; HGRN2; SSD), us, as many segments as compute units / workgroups (of portions,
-// not of rows) -> by this rule: 6 sequences of 400 .. 4000 rows 156 -> 90, 270 -> 122, 139 -> 77; 8 of them 230 -> 151, 398 -> 258,
-// 201 -> 133; 12 of them 320 -> 177, 545 -> 296, 273 -> 153; 12 equal ones stay unsegmented (164, 275, 144).
+// rows; with segments of c chunks it lasts c where a compute unit has one of them at most (of unequal portions' last segments, which
+// are short and start last, half may follow another, up to an eighth of the units), c `together` where some have two, else its share
+// and a third of a segment, and 45 % more for the first pass, half a unit per segment for the scan between the two, and two units for the
+// launches.  Over 182 batches (1 to 30 prompts of 100 .. 12000 rows, 2 to 64 heads, all four recurrences) this is 3.1 % off the best number
+// on average; with 0.85 segments a unit for a guess, half a segment and 1.6 c up to 1.3 of them a unit, 4.3 %.
 static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, int most) {
     if (batch <= 0 || per_seq <= 0 || max_len <= 0) return 1;
     if (n_rows > batch * max_len) n_rows = batch * max_len;
     const int chunks = (max_len + kLaChunk - 1) / kLaChunk;
     const double rows = (double)n_rows / kLaChunk, share = rows * per_seq / cus * (together > 0 ? together / 2 : 1.0);
+    const double most_spare = 0.12 * cus, spare = 0.25 * batch * per_seq < most_spare ? 0.25 * batch * per_seq : most_spare;
     double best = share > chunks ? share : chunks;
     int segments = 1;
     for (int s = 2; s <= most; ++s) {
         const double c = (chunks + s - 1) / s;
         const double spread = rows / c + 0.5 * batch, all = (double)batch * s, live = per_seq * (spread < all ? spread : all);
         double part = c;
-        if (live > (spread < all ? 0.85 : 1.0) * cus) {
-            part = share + 0.5 * c;
-            if (live <= 2.0 * cus && together > 0) part = c * together;
-            else if (live <= 1.3 * cus && part < 1.6 * c) part = 1.6 * c;
-        }
+        if (live > cus + (spread < all ? spare : 0.0)) part = live <= 2.0 * cus && together > 0 ? c * together : share + 0.35 * c;
         if (part < c) part = c;
         const double t = 1.45 * part + 0.5 * s + 2.0;
         if (t < best) {
@@ -75,6 +77,12 @@ static inline int la_launch_segments(int64_t batch, int64_t per_seq, int cus, do
     const int most = la_most_segments(seg_bytes, max_len, room);
     if (!aligned) return most > 1 && la_segments(batch * per_seq, cus, max_len) > 1 ? 0 : 1;
     return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
+}
+
+// Segments of seg_rows rows before a portion's last one.  (Rows past the longest length that a launch was told have no segment.)
+PA_LA_FN int la_full_segments(int rows, int segments, int seg_rows) {
+    const int full = rows > 0 ? (rows - 1) / seg_rows : 0;
+    return full < segments ? full : segments - 1;
 }
 
 // Rows per segment: whole chunks.

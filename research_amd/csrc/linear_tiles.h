@@ -150,24 +150,75 @@ __device__ __forceinline__ LaSplit la_split_weighted(bf8 raw, const f4 &x, const
     return s;
 }
 
-// Which piece a workgroup of a chunked kernel takes.  Workgroups go to the dies, and there to groups of compute units, in the order
-// of their ids, and wait for the one whose turn it is.  With 16 heads or 32 a segment fills its turn by itself, and a portion's
-// segments follow each other (8 portions of 400 .. 4000 rows, lightning, 16 heads of 128 x 128: 151 us, with sequences side by side
-// 211).  With fewer the places of the last segments, which only long portions have, would come to the same units each time (5
-// portions of 1100 .. 2400 rows in 4 segments, 4 heads of 256 x 512, mLSTM 274 us, with sequences side by side 153): so heads and
-// value slices lie side by side, then sequences, and the last segments behind all others.  A single sequence's slices of one
-// segment, which read the same keys, share a die (15999 rows: 236 us, else 245).
+// Which piece a workgroup of a chunked kernel takes.  Workgroups go to the dies, and there to groups of compute units, in the order of
+// their ids, and wait for the one whose turn it is: pieces that short portions do not have would leave some units idle and others with
+// two.  So the pieces that there are get the first ids, found from the lengths (by each wave, a scan, under 1 us): first the segments
+// before the portions' last ones, which have as many rows each, then the last ones, the longest first.  Heads and value slices, which
+// read the same rows, lie side by side; a single portion's slices have their segments in a row instead, so that those of one segment share
+// a die (15999 rows: 236 us, else 245).  us, with ids for all possible pieces by portion / by segment / this, as many segments: 8 prompts
+// of 400 .. 4000 rows, mLSTM, 4 heads of 256 x 512, 230 / 175 / 144, 8 heads 432 / 283 / 271; lightning, 16 heads of 128 x 128, 115 / 115 / 83,
+// of 64 x 64, 63 / 73 / 51; 12 prompts, 8 heads, 106 / 177 / 97, 16 heads 157 / 178 / 157.
 struct LaPlace {
     int h, vsl, b, seg;
 };
-__host__ __device__ __forceinline__ bool la_by_portion(int heads, int batch, int segments) { return segments == 1 || batch == 1 || heads % 16 == 0; }
-__device__ __forceinline__ LaPlace la_place(int segments, int slices, int batch) {
-    const int h = blockIdx.x, y = blockIdx.y, z = blockIdx.z;
-    return la_by_portion(gridDim.x, batch, segments) ? LaPlace{h, y / segments, z, y % segments} : LaPlace{h, y % slices, y / slices, z};
+__device__ __forceinline__ int la_scan(int x, int lane) {  // inclusive sums over the wave
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    const int r0 = __builtin_amdgcn_readlane(x, 15), r1 = r0 + __builtin_amdgcn_readlane(x, 31), r2 = r1 + __builtin_amdgcn_readlane(x, 47);
+    return x + (lane < 16 ? 0 : lane < 32 ? r0 : lane < 48 ? r1 : r2);
 }
-inline dim3 la_grid(int heads, int slices, int batch, int segments) {  // (segments > 1: batch and vdim are bounded by their workspace)
-    return la_by_portion(heads, batch, segments) ? dim3((unsigned)heads, (unsigned)(slices * segments), (unsigned)batch)
-                                                 : dim3((unsigned)heads, (unsigned)(slices * batch), (unsigned)segments);
+// Also the portion `p` (of the caller's type; all that is known of up to 64 sequences is loaded at once, as a second round of loads would
+// keep every workgroup waiting).  False: nothing to do.
+template <typename Args, typename Portion> __device__ __forceinline__ bool la_place(const Args &a, int slices, LaPlace &at, Portion &p) {
+    int n, start, ctx, slot;
+    if (a.segments == 1 || a.batch == 1) {
+        const int y = a.segments == 1 ? 0 : blockIdx.x / a.heads;
+        at = a.segments == 1 ? LaPlace{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, 0} : LaPlace{(int)blockIdx.x % a.heads, y / a.segments, 0, y % a.segments};
+        n = a.q_lens[at.b], start = a.q_starts[at.b], ctx = a.ctx_lens[at.b], slot = a.state_slots[at.b];
+    } else {
+        const int lane = threadIdx.x & 63, y = blockIdx.x / a.heads;
+        at.h = blockIdx.x % a.heads, at.vsl = y % slices;
+        int u = y / slices, first = 0, from = -1;
+        auto load = [&] {
+            const int b = first + lane;
+            n = start = ctx = slot = 0;
+            if (b < a.batch) n = a.q_lens[b], start = a.q_starts[b], ctx = a.ctx_lens[b], slot = a.state_slots[b];
+            return la_full_segments(n, a.segments, a.seg_rows);
+        };
+        for (; from < 0 && first < a.batch; first += 64) {
+            const int full = load(), upto = la_scan(full, lane), all = __builtin_amdgcn_readlane(upto, 63);
+            if (u < all) {  // (uniform)
+                from = __builtin_ctzll(__ballot(upto > u));
+                at.b = first + from, at.seg = u - __builtin_amdgcn_readlane(upto - full, from);
+                break;
+            }
+            u -= all;
+        }
+        if (from < 0) {  // a last one: of up to 64 sequences the longest first
+            if (u >= a.batch) return false;
+            first = a.batch <= 64 ? 0 : u & ~63, from = u & 63;
+            const int full = load(), rest = n - full * a.seg_rows;
+            if (a.batch <= 64) {
+                int longer = 0;
+                for (int i = 0; i < a.batch; ++i) {
+                    const int x = __builtin_amdgcn_readlane(rest, i);
+                    longer += x > rest || (x == rest && i < lane);
+                }
+                from = __builtin_ctzll(__ballot(lane < a.batch && longer == u));
+            }
+            at.b = first + from, at.seg = __builtin_amdgcn_readlane(full, from);
+        }
+        n = __builtin_amdgcn_readlane(n, from), start = __builtin_amdgcn_readlane(start, from);
+        ctx = __builtin_amdgcn_readlane(ctx, from), slot = __builtin_amdgcn_readlane(slot, from);
+    }
+    p.n = n, p.row0 = start, p.pos0 = ctx - n, p.slot = slot < a.state_rows ? slot : -1;
+    return p.n > 0 && p.pos0 >= 0 && p.row0 >= 0 && p.row0 + p.n <= a.n_rows;
+}
+// (segments > 1: the number of workgroups is bounded by the workspace of 256 MB)
+inline dim3 la_grid(int heads, int slices, int batch, int segments) {
+    return segments == 1 ? dim3((unsigned)heads, (unsigned)slices, (unsigned)batch) : dim3((unsigned)heads * slices * batch * segments);
 }
 
 constexpr int kLaPitchA = 72;  // bf16 per row of the decayed scores

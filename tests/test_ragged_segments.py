@@ -1,5 +1,6 @@
-"""Segments of prompts of unequal lengths: the rule that chooses them, in a plain C++ build, and one launch that it cuts
-although the batch alone fills the device, against the oracle's token-by-token recurrence."""
+"""Segments of prompts of unequal lengths: the rule that chooses them, in a plain C++ build, and launches that it cuts, of every
+recurrence, head counts below and above the dies' number, value slices and more sequences than a wave has lanes, against the oracle's
+token-by-token recurrence."""
 
 import os
 import subprocess
@@ -42,6 +43,14 @@ int main() {
     if (la_balanced_segments(1, 16, 256, 0.0, 4096, 4096, la_most_segments(big, 4096)) < 4) return 8;
     if (la_balanced_segments(0, 16, 256, 0.0, 4096, 0, 64) != 1 || la_balanced_segments(4, 16, 256, 0.0, 0, 0, 64) != 1) return 9;
     if (la_most_segments(big * 300, 40000) != 1 || la_most_segments(0, 40000) != 64) return 10;
+    if (la_balanced_segments(2, 24, 256, 0.0, 2570, 5123, 5) != 5) return 11;   // as many as fit whatever the lengths
+    if (la_balanced_segments(5, 16, 256, 0.0, 2066, 8293, 4) != 4) return 12;   // some last ones more than compute units
+    if (la_balanced_segments(1, 16, 256, 0.0, 12000, 12000, 23) != 16) return 13;  // equal segments: one each
+    for (int segments = 1; segments < 9; ++segments)  // before a portion's last one
+        for (int rows : {-3, 0, 1, 511, 512, 513, 1024, 1025, 2560, 9999}) {
+            const int full = la_full_segments(rows, segments, 512);
+            if (full < 0 || full >= segments || (rows > 0 && full * 512 >= rows) || (full < segments - 1 && (full + 1) * 512 < rows)) return 14;
+        }
     std::puts("ok");
 }
 ''')
@@ -72,3 +81,55 @@ def test_a_batch_of_unequal_prompts_in_segments(heads, dim, vdim, longest):
             case.check(b, lo, got)
     for b, n in enumerate(lens):
         case.check_state(b, slots[b])
+
+
+RAGGED = [("mlstm", 16, 64, 192), ("mlstm", 24, 64, 40), ("ssd", 16, 128, 128), ("ssd", 24, 64, 64), ("channel", 16, 64, 64), ("channel", 8, 64, 200), ("channel", 4, 128, 128),
+          ("lightning", 24, 64, 64), ("lightning", 3, 128, 256)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,heads,dim,vdim", RAGGED)
+def test_every_recurrence_over_unequal_prompts(kind, heads, dim, vdim):
+    import torch
+
+    from tests.gpu_helpers import announce
+    from tests.test_gpu_lightning import Case as Lightning
+    from tests.test_gpu_loluzen_ops import Channels
+    from tests.test_gpu_tevirax_ops import Case as Gated
+
+    announce(f"ragged segments {kind} {heads}x{dim}x{vdim}")
+    lens, bf = [2500, 40, 513, 1024, 1, 1025, 700, 100], torch.bfloat16
+    slots = [(3 * b + 1) % len(lens) for b in range(len(lens))]
+    whole = [(b, 0, n) for b, n in enumerate(lens)]
+    cuts = [(b, 0, (n + 1) // 2) for b, n in enumerate(lens)], [(b, (n + 1) // 2, n // 2) for b, n in enumerate(lens) if n > 1]
+    if kind == "channel":  # (its rows are checked where they are run)
+        case = Channels(lens, heads, dim, vdim, bf, seed=6)
+        for picks in (whole, *cuts):
+            case.run(picks, slots)
+        case.check_states(slots)
+        return
+    case = Lightning(lens, heads, dim, vdim, [1.0 - 0.5 ** (1 + i * 12 / heads) for i in range(heads)], bf, seed=6) if kind == "lightning" else \
+        Gated(kind, lens, heads, dim, vdim, bf, 8 if kind == "ssd" else None, seed=6, remember=4.5)
+    for picks in (whole, *cuts):
+        for (b, lo, _), got in zip(picks, case.run(picks, slots)):
+            case.check(b, lo, got)
+    for b in range(len(lens)):
+        case.check_state(b, slots[b])
+
+
+@pytest.mark.gpu
+def test_more_unequal_prompts_than_a_wave_has_lanes():
+    import torch
+
+    from tests.gpu_helpers import announce
+    from tests.test_gpu_lightning import Case
+
+    announce("ragged segments of 150 sequences")
+    lens = [1 + 37 * b % 90 for b in range(150)]
+    lens[3], lens[70], lens[149] = 1100, 1600, 1300
+    case = Case(lens, 2, 32, 32, [0.99, 0.9], torch.bfloat16, seed=7)
+    slots = list(range(150))
+    for (b, lo, _), got in zip(((b, 0, n) for b, n in enumerate(lens)), case.run([(b, 0, n) for b, n in enumerate(lens)], slots)):
+        case.check(b, lo, got)
+    for b in (0, 3, 64, 70, 148, 149):
+        case.check_state(b, b)
