@@ -719,7 +719,7 @@ extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const 
     a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(),
                                     cols == 64 && dim <= 128 ? 1.25 : 0.0, max_q_len, n_rows,
                                     gl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
-                                    pa_aligned16(workspace));
+                                    pa_aligned16(workspace), cols == 64 && dim <= 128 ? 2 : 1);
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
     a.batch = batch;
     a.seg_rows = la_segment_rows(max_q_len, a.segments);

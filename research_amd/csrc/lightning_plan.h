@@ -71,11 +71,11 @@ static inline int la_most_segments(size_t seg_bytes, int max_len, size_t room = 
     return fit < 1 ? 1 : fit < most ? (int)fit : most;
 }
 // Segments of a launch with a workspace of `room` bytes (0: none).  0: they would need the workspace, which is not aligned; a
-// batch that fills the device without segments takes such a workspace for none.
+// batch that fills the device without segments takes such a workspace for none.  shared: workgroups that a compute unit has at once.
 static inline int la_launch_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows,
-                                     size_t seg_bytes, size_t room, bool aligned) {
+                                     size_t seg_bytes, size_t room, bool aligned, int shared = 1) {
     const int most = la_most_segments(seg_bytes, max_len, room);
-    if (!aligned) return most > 1 && la_segments(batch * per_seq, cus, max_len) > 1 ? 0 : 1;
+    if (!aligned) return most > 1 && la_segments(batch * per_seq, shared * cus, max_len) > 1 ? 0 : 1;
     return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
 }
 

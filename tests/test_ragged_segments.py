@@ -46,6 +46,8 @@ int main() {
     if (la_balanced_segments(2, 24, 256, 0.0, 2570, 5123, 5) != 5) return 11;   // as many as fit whatever the lengths
     if (la_balanced_segments(5, 16, 256, 0.0, 2066, 8293, 4) != 4) return 12;   // some last ones more than compute units
     if (la_balanced_segments(1, 16, 256, 0.0, 12000, 12000, 23) != 16) return 13;  // equal segments: one each
+    if (la_launch_segments(3, 64, 256, 1.25, 4096, 3 * 4096, big, 64 * big, false, 2) != 0) return 15;  // refused: two workgroups a unit
+    if (la_launch_segments(3, 64, 256, 1.25, 4096, 3 * 4096, big, 64 * big, false) != 1) return 16;     // ... one: taken for none
     for (int segments = 1; segments < 9; ++segments)  // before a portion's last one
         for (int rows : {-3, 0, 1, 511, 512, 513, 1024, 1025, 2560, 9999}) {
             const int full = la_full_segments(rows, segments, 512);
