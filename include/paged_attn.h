@@ -513,7 +513,9 @@ int pa_qkv_conv_append(const void *u, int64_t u_stride, int64_t n_rows, const fl
  * pa_lightning_recurrent walks a portion token by token (decode steps; 32-bit prompts).  pa_lightning_chunked
  * (PA_BF16) multiplies 64 rows at a time on the matrix cores, with the 32-bit factors split into two bf16 terms; given
  * a workspace it cuts long portions of small or unequal batches into segments that run at the same time.  max_q_len: at least
- * the longest portion.
+ * the longest portion.  pa_lightning_workspace_bytes: what the most segments of any launch of these sizes take, 256 MB at most;
+ * pa_lightning_workspace_bytes_of: what a launch of n_rows rows takes, 0 where the batch fills the device in one piece.  With less, or
+ * none, there are fewer segments.
  */
 size_t pa_lightning_state_floats(int dim, int vdim);
 int pa_lightning_recurrent(const void *u, int64_t u_stride, int64_t n_rows, float *state, int64_t state_rows,
@@ -521,6 +523,7 @@ int pa_lightning_recurrent(const void *u, int64_t u_stride, int64_t n_rows, floa
                            const int32_t *q_starts, const int32_t *state_slots, int batch, void *out,
                            int num_heads, int dim, int vdim, int dtype, void *stream);
 size_t pa_lightning_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len);
+size_t pa_lightning_workspace_bytes_of(int batch, int num_heads, int dim, int vdim, int max_q_len, int64_t n_rows);
 int pa_lightning_chunked(const void *u, int64_t u_stride, int64_t n_rows, float *state, int64_t state_rows,
                          const float *decay_powers, const int32_t *ctx_lens, const int32_t *q_lens,
                          const int32_t *q_starts, const int32_t *state_slots, int batch, int max_q_len,
@@ -553,10 +556,12 @@ int pa_short_conv(const void *u, int64_t u_stride, int64_t n_rows, const float *
  *   out           : [n_rows][heads * vdim] of dtype;  dim <= 256, any vdim
  * Single rows (q_lens NULL), PA_F32 and rows that are not whole 8-byte vectors run token by token; PA_BF16 portions in
  * chunks of 64 rows on the matrix cores, with the 32-bit factors split into two bf16 terms, and, given a workspace, in
- * segments that run at the same time when there are few sequences or unequal ones.  max_q_len: at least the longest portion.
+ * segments that run at the same time when there are few sequences or unequal ones (workspace sizes as for lightning attention).
+ * max_q_len: at least the longest portion.
  */
 size_t pa_gated_linear_state_floats(int kind, int dim, int vdim);
 size_t pa_gated_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len);
+size_t pa_gated_linear_workspace_bytes_of(int batch, int num_heads, int dim, int vdim, int max_q_len, int64_t n_rows);
 int pa_gated_linear(int kind, const void *q, int64_t q_stride, const void *k, int64_t k_stride, const void *v,
                     int64_t v_stride, int heads_per_group, const void *gate_a, const void *gate_b, int64_t gate_stride,
                     const float *head_a, const float *head_b, const float *head_c, float cap, float q_scale,
@@ -662,6 +667,7 @@ int pa_talking_attention(const void *q, int64_t q_row, int64_t q_head, int dim, 
  *   out          : [n_rows][heads * vdim] of dtype;  dim <= 256, any vdim
  */
 size_t pa_channel_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len);
+size_t pa_channel_linear_workspace_bytes_of(int batch, int num_heads, int dim, int vdim, int max_q_len, int64_t n_rows);
 int pa_channel_linear(const void *q, int64_t q_stride, int q_act, const void *forget, int64_t f_stride, const float *f_bias,
                       const float *lower, const void *v, int64_t v_stride, int64_t n_rows, float *state, int64_t state_rows,
                       const int32_t *ctx_lens, const int32_t *q_lens, const int32_t *q_starts, const int32_t *state_slots,

@@ -105,10 +105,12 @@ SIGNATURES.update({
     "pa_lightning_state_floats": (c_size_t, [_i, _i]),
     "pa_lightning_recurrent": (_i, [_p, _l, _l, _p, _l, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _i, _p]),
     "pa_lightning_workspace_bytes": (c_size_t, [_i, _i, _i, _i, _i]),
+    "pa_lightning_workspace_bytes_of": (c_size_t, [_i, _i, _i, _i, _i, _l]),
     "pa_lightning_chunked": (_i, [_p, _l, _l, _p, _l, _p, _p, _p, _p, _p, _i, _i, _p, _i, _i, _i, _i, _p, c_size_t, _p]),
     "pa_short_conv": (_i, [_p, _l, _l, _p, _p, _i, _i, _p, _l, _p, _p, _p, _p, _p, _i, _i, _p, _i, _i, _p]),
     "pa_gated_linear_state_floats": (c_size_t, [_i, _i, _i]),
     "pa_gated_linear_workspace_bytes": (c_size_t, [_i, _i, _i, _i, _i]),
+    "pa_gated_linear_workspace_bytes_of": (c_size_t, [_i, _i, _i, _i, _i, _l]),
     "pa_gated_linear": (_i, [_i, _p, _l, _p, _l, _p, _l, _i, _p, _p, _l, _p, _p, _p, _f, _f, _f, _l, _p, _l, _p, _p, _p, _p,
                              _i, _i, _p, _i, _i, _i, _i, _p, c_size_t, _p]),
     "pa_narrow_linear": (_i, [_p, _l, _p, _p, _l, _i, _i, _i, _p]),
@@ -124,6 +126,7 @@ SIGNATURES.update({
     "pa_scored_attention": (_i, [_p, _l, _l, _i, _p, _l, _l, _i, _p, _i, _p, _i, _i, _p, _l, _i, _l, _p, _p, _p, _l, _i, _i, _i, _i,
                                  _f, _i, _f, _p, _i, _p, _p, _i, _p, c_size_t, _p]),
     "pa_channel_linear_workspace_bytes": (c_size_t, [_i, _i, _i, _i, _i]),
+    "pa_channel_linear_workspace_bytes_of": (c_size_t, [_i, _i, _i, _i, _i, _l]),
     "pa_channel_linear": (_i, [_p, _l, _i, _p, _l, _p, _p, _p, _l, _l, _p, _l, _p, _p, _p, _p, _i, _i, _p, _i, _i, _i, _i, _p, c_size_t, _p]),
     "pa_talking_workspace_bytes": (c_size_t, [_l, _i, _i, _i, _i, _l, _i]),
     "pa_talking_attention": (_i, [_p, _l, _l, _i, _p, _i, _p, _i, _i, _p, _l, _i, _l, _p, _p, _p, _l, _i, _i, _i, _i, _f, _p, _p, _p, _p, _i,

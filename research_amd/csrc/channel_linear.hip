@@ -495,13 +495,19 @@ size_t cl_segment_bytes(int64_t batch, int heads, int dim, int vdim) { return gl
 
 }  // namespace
 
-extern "C" size_t pa_channel_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len) {
+extern "C" size_t pa_channel_linear_workspace_bytes_of(int batch, int num_heads, int dim, int vdim, int max_q_len, int64_t n_rows) {
     pa_clear_error();
     if (batch < 0 || num_heads <= 0 || dim <= 0 || vdim <= 0 || max_q_len < 0) {
         pa_fail(PA_ERR_INVALID_ARG, "pa_channel_linear_workspace_bytes: sizes out of range");
         return 0;
     }
-    return gl_workspace_bytes(batch, num_heads, dim, vdim, la_most_segments(cl_segment_bytes(batch, num_heads, dim, vdim), max_q_len));
+    return gl_workspace_bytes(batch, num_heads, dim, vdim,
+                              la_asked_segments(batch, la_per_sequence(num_heads, vdim), la_cus(), 0.0, max_q_len, n_rows,
+                                                cl_segment_bytes(batch, num_heads, dim, vdim)));
+}
+
+extern "C" size_t pa_channel_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len) {
+    return pa_channel_linear_workspace_bytes_of(batch, num_heads, dim, vdim, max_q_len, -1);
 }
 
 extern "C" int pa_channel_linear(const void *q, int64_t q_stride, int q_act, const void *forget, int64_t f_stride, const float *f_bias,
@@ -540,8 +546,7 @@ extern "C" int pa_channel_linear(const void *q, int64_t q_stride, int q_act, con
         PA_CHECK_LAUNCH("pa_channel_linear");
         return PA_OK;
     }
-    const int cols = la_value_cols(vdim);
-    a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(), 0.0, max_q_len, n_rows,
+    a.segments = la_launch_segments(batch, la_per_sequence(num_heads, vdim), la_cus(), 0.0, max_q_len, n_rows,
                                     cl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
                                     pa_aligned16(workspace));
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");

@@ -646,6 +646,8 @@ template <typename T, int KIND> void launch_recurrent(const GlArgs &a, int batch
     else gated_recurrent_kernel<T, 16, KIND><<<grid, block, 0, s>>>(a);
 }
 
+// (two workgroups of four waves share a compute unit)
+double gl_together(int dim, int vdim) { return la_value_cols(vdim) == 64 && dim <= 128 ? 1.25 : 0.0; }
 size_t gl_segment_bytes(int64_t batch, int heads, int dim, int vdim) { return gl_workspace_bytes(batch, heads, dim, vdim, 2) / 2; }
 
 }  // namespace
@@ -654,13 +656,19 @@ extern "C" size_t pa_gated_linear_state_floats(int kind, int dim, int vdim) {
     return (kind == kSsd || kind == kMlstm) && dim > 0 && vdim > 0 ? gl_state_floats(kind == kMlstm, dim, vdim) : 0;
 }
 
-extern "C" size_t pa_gated_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len) {
+extern "C" size_t pa_gated_linear_workspace_bytes_of(int batch, int num_heads, int dim, int vdim, int max_q_len, int64_t n_rows) {
     pa_clear_error();
     if (batch < 0 || num_heads <= 0 || dim <= 0 || vdim <= 0 || max_q_len < 0) {
         pa_fail(PA_ERR_INVALID_ARG, "pa_gated_linear_workspace_bytes: sizes out of range");
         return 0;
     }
-    return gl_workspace_bytes(batch, num_heads, dim, vdim, la_most_segments(gl_segment_bytes(batch, num_heads, dim, vdim), max_q_len));
+    return gl_workspace_bytes(batch, num_heads, dim, vdim,
+                              la_asked_segments(batch, la_per_sequence(num_heads, vdim), la_cus(), gl_together(dim, vdim), max_q_len, n_rows,
+                                                gl_segment_bytes(batch, num_heads, dim, vdim)));
+}
+
+extern "C" size_t pa_gated_linear_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len) {
+    return pa_gated_linear_workspace_bytes_of(batch, num_heads, dim, vdim, max_q_len, -1);
 }
 
 extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const void *k, int64_t k_stride, const void *v,
@@ -715,11 +723,9 @@ extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const 
         PA_CHECK_LAUNCH("pa_gated_linear");
         return PA_OK;
     }
-    const int cols = la_value_cols(vdim);  // (two workgroups of four waves share a compute unit)
-    a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(),
-                                    cols == 64 && dim <= 128 ? 1.25 : 0.0, max_q_len, n_rows,
+    a.segments = la_launch_segments(batch, la_per_sequence(num_heads, vdim), la_cus(), gl_together(dim, vdim), max_q_len, n_rows,
                                     gl_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
-                                    pa_aligned16(workspace), cols == 64 && dim <= 128 ? 2 : 1);
+                                    pa_aligned16(workspace), gl_together(dim, vdim) > 0 ? 2 : 1);
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");
     a.batch = batch;
     a.seg_rows = la_segment_rows(max_q_len, a.segments);

@@ -422,6 +422,8 @@ int la_fill(const char *what, LaArgs &a, const void *u, int64_t u_stride, int64_
     return PA_OK;
 }
 
+// (two workgroups of four waves share a compute unit, or two of eight at dim 64)
+double la_together(int dim, int vdim) { return la_value_cols(vdim) == 64 && dim <= 128 ? 1.25 : dim <= 64 ? 1.6 : 0.0; }
 size_t la_segment_bytes(int64_t batch, int heads, int dim, int vdim) { return la_workspace_bytes(batch, heads, dim, vdim, 2) / 2; }
 
 }  // namespace
@@ -447,13 +449,19 @@ extern "C" int pa_lightning_recurrent(const void *u, int64_t u_stride, int64_t n
     return PA_OK;
 }
 
-extern "C" size_t pa_lightning_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len) {
+extern "C" size_t pa_lightning_workspace_bytes_of(int batch, int num_heads, int dim, int vdim, int max_q_len, int64_t n_rows) {
     pa_clear_error();
     if (batch < 0 || num_heads <= 0 || dim <= 0 || vdim <= 0 || max_q_len < 0) {
         pa_fail(PA_ERR_INVALID_ARG, "pa_lightning_workspace_bytes: sizes out of range");
         return 0;
     }
-    return la_workspace_bytes(batch, num_heads, dim, vdim, la_most_segments(la_segment_bytes(batch, num_heads, dim, vdim), max_q_len));
+    return la_workspace_bytes(batch, num_heads, dim, vdim,
+                              la_asked_segments(batch, la_per_sequence(num_heads, vdim), la_cus(), la_together(dim, vdim), max_q_len, n_rows,
+                                                la_segment_bytes(batch, num_heads, dim, vdim)));
+}
+
+extern "C" size_t pa_lightning_workspace_bytes(int batch, int num_heads, int dim, int vdim, int max_q_len) {
+    return pa_lightning_workspace_bytes_of(batch, num_heads, dim, vdim, max_q_len, -1);
 }
 
 extern "C" int pa_lightning_chunked(const void *u, int64_t u_stride, int64_t n_rows, float *state, int64_t state_rows,
@@ -472,9 +480,7 @@ extern "C" int pa_lightning_chunked(const void *u, int64_t u_stride, int64_t n_r
         return rc;
     if (n_rows == 0 || batch == 0 || max_q_len == 0) return PA_OK;
     PA_REQUIRE(q_lens, "NULL q_lens / q_starts");
-    const int cols = la_value_cols(vdim);
-    a.segments = la_launch_segments(batch, num_heads * (int64_t)((vdim + cols - 1) / cols), la_cus(),
-                                    cols == 64 && dim <= 128 ? 1.25 : dim <= 64 ? 1.6 : 0.0, max_q_len, n_rows,
+    a.segments = la_launch_segments(batch, la_per_sequence(num_heads, vdim), la_cus(), la_together(dim, vdim), max_q_len, n_rows,
                                     la_segment_bytes(batch, num_heads, dim, vdim), workspace ? workspace_bytes : 0,
                                     pa_aligned16(workspace));
     PA_REQUIRE(a.segments, "the workspace must be 16-byte aligned");

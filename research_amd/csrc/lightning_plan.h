@@ -18,6 +18,8 @@ static inline int la_pad16(int n) { return (n + 15) / 16 * 16; }
 
 // Columns of the value dimension that one workgroup of the chunked kernel owns: 16 for each of its four or eight waves.
 static inline int la_value_cols(int vdim) { return vdim <= 64 ? 64 : 128; }
+// Workgroups of a sequence (of each of its segments): one per head and slice of the value columns.
+static inline int64_t la_per_sequence(int heads, int vdim) { return heads * (int64_t)((vdim + la_value_cols(vdim) - 1) / la_value_cols(vdim)); }
 
 // Segments of a portion of up to max_len rows: as many as (sequences x heads x value slices) leave compute units for,
 // one workgroup each, but no shorter than kLaMinSegChunks chunks (a segment's start state costs a second reading of
@@ -69,6 +71,18 @@ static inline int la_most_segments(size_t seg_bytes, int max_len, size_t room = 
     if (room > kLaMostSegBytes) room = kLaMostSegBytes;
     const int64_t fit = seg_bytes ? (int64_t)(room / seg_bytes) : most;
     return fit < 1 ? 1 : fit < most ? (int)fit : most;
+}
+// Segments whose states a launch of n_rows rows has a use for (< 0: the rows are not known yet; the most of any): 1 where the batch stays
+// in one piece, such as equal portions that fill the device.
+static inline int la_asked_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, size_t seg_bytes) {
+    const int most = la_most_segments(seg_bytes, max_len);
+    if (n_rows >= 0) return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
+    int asked = 1;
+    for (int i = 0; i <= 32; ++i) {  // from one long portion to equal ones
+        const int s = la_balanced_segments(batch, per_seq, cus, together, max_len, max_len + (batch - 1) * max_len * i / 32, most);
+        if (s > asked) asked = s;
+    }
+    return asked;
 }
 // Segments of a launch with a workspace of `room` bytes (0: none).  0: they would need the workspace, which is not aligned; a
 // batch that fills the device without segments takes such a workspace for none.  shared: workgroups that a compute unit has at once.

@@ -607,7 +607,7 @@ class LightningMixer(Mixer):
             ops.lightning(u[:nd], packed.decodes, state, self.decay_powers, s.heads, s.dim, s.vdim, o[:nd])
         if packed.chunks is not None:
             c = packed.chunks
-            need = ops.lightning_workspace_bytes(c.ctx_lens.numel(), s.heads, s.dim, s.vdim, c.max_q_len)
+            need = ops.lightning_workspace_bytes(c.ctx_lens.numel(), s.heads, s.dim, s.vdim, c.max_q_len, u.shape[0])
             ops.lightning(u, c, state, self.decay_powers, s.heads, s.dim, s.vdim, o,
                           workspace=self.backend._scratch_for(need) if need else None)
         g = 2 * s.heads * s.dim + inner
@@ -625,7 +625,7 @@ def _gated_rows(kind: str, q: Tensor, k: Tensor, v: Tensor, gates, constants, st
                          vdim, cut(out), **kw)
     if packed.chunks is not None:
         c = packed.chunks
-        need = ops.gated_linear_workspace_bytes(c.ctx_lens.numel(), heads, dim, vdim, c.max_q_len)
+        need = ops.gated_linear_workspace_bytes(c.ctx_lens.numel(), heads, dim, vdim, c.max_q_len, v.shape[0])
         ops.gated_linear(kind, q, k, v, gates, constants, c, state, heads, dim, vdim, out,
                          workspace=backend._scratch_for(need) if need else None, **kw)
     return out
@@ -945,7 +945,7 @@ class Hgrn2Mixer(Mixer):
             ops.channel_linear(q[:n], f[:n], v[:n], self.f_bias, self.lower, packed.decodes, *tail, o[:n], q_act="silu")
         if packed.chunks is not None:
             c = packed.chunks
-            need = ops.channel_linear_workspace_bytes(c.ctx_lens.numel(), s.heads, s.dim, s.vdim, c.max_q_len)
+            need = ops.channel_linear_workspace_bytes(c.ctx_lens.numel(), s.heads, s.dim, s.vdim, c.max_q_len, u.shape[0])
             ops.channel_linear(q, f, v, self.f_bias, self.lower, c, *tail, o, q_act="silu",
                                workspace=self.backend._scratch_for(need) if need else None)
         return ops.rms_gate(o, None, self.norm, self.eps, groups=s.heads, order=None, out=out)

@@ -540,8 +540,9 @@ def lightning_state(num_slots: int, heads: int, dim: int, vdim: int, device) -> 
     return torch.zeros((num_slots, heads, pad(dim), pad(vdim)), dtype=torch.float32, device=device)
 
 
-def lightning_workspace_bytes(batch: int, heads: int, dim: int, vdim: int, max_q_len: int) -> int:
-    return int(_lib.load().pa_lightning_workspace_bytes(batch, heads, dim, vdim, max_q_len))
+def lightning_workspace_bytes(batch: int, heads: int, dim: int, vdim: int, max_q_len: int, rows: Optional[int] = None) -> int:
+    """Bytes that a launch of portions of up to ``max_q_len`` rows takes, ``rows`` in all (None: the most of any)."""
+    return int(_lib.load().pa_lightning_workspace_bytes_of(batch, heads, dim, vdim, max_q_len, -1 if rows is None else rows))
 
 
 def lightning(u: Tensor, portions: Portions, state: Tensor, decay_powers: Tensor, heads: int, dim: int, vdim: int,
@@ -607,8 +608,8 @@ def gated_linear_state_floats(kind: str, dim: int, vdim: int) -> int:
     return int(_lib.load().pa_gated_linear_state_floats(_GATED[kind], dim, vdim))
 
 
-def gated_linear_workspace_bytes(batch: int, heads: int, dim: int, vdim: int, max_q_len: int) -> int:
-    return int(_lib.load().pa_gated_linear_workspace_bytes(batch, heads, dim, vdim, max_q_len))
+def gated_linear_workspace_bytes(batch: int, heads: int, dim: int, vdim: int, max_q_len: int, rows: Optional[int] = None) -> int:
+    return int(_lib.load().pa_gated_linear_workspace_bytes_of(batch, heads, dim, vdim, max_q_len, -1 if rows is None else rows))
 
 
 def gated_linear(kind: str, q: Tensor, k: Tensor, v: Tensor, gates: Tuple[Tensor, Optional[Tensor]],
@@ -864,8 +865,8 @@ def talking_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, vdim: int, po
     return out
 
 
-def channel_linear_workspace_bytes(batch: int, heads: int, dim: int, vdim: int, max_q_len: int) -> int:
-    return int(_lib.load().pa_channel_linear_workspace_bytes(batch, heads, dim, vdim, max_q_len))
+def channel_linear_workspace_bytes(batch: int, heads: int, dim: int, vdim: int, max_q_len: int, rows: Optional[int] = None) -> int:
+    return int(_lib.load().pa_channel_linear_workspace_bytes_of(batch, heads, dim, vdim, max_q_len, -1 if rows is None else rows))
 
 
 def channel_linear(q: Tensor, forget: Tensor, v: Tensor, f_bias: Optional[Tensor], lower: Tensor, portions: Portions, state: Tensor,

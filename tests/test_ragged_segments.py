@@ -61,6 +61,20 @@ int main() {
     assert subprocess.run([str(exe)], stdout=subprocess.PIPE).returncode == 0
 
 
+@pytest.mark.parametrize("kind", ["lightning", "gated_linear", "channel_linear"])
+def test_a_batch_in_one_piece_asks_for_no_workspace(kind):
+    from research_amd import ops
+
+    need = getattr(ops, kind + "_workspace_bytes")
+    assert need(32, 16, 128, 128, 4096, rows=32 * 4096) == 0              # equal portions that fill the device
+    ragged, most = need(32, 16, 128, 128, 4096, rows=9 * 4096), need(32, 16, 128, 128, 4096)
+    assert 0 < ragged <= most <= 256 << 20                                # a few long ones among them
+    assert need(1, 16, 128, 128, 4096) == need(1, 16, 128, 128, 4096, rows=4096) >= 4 * 16 * 128 * 128 * 4
+    for rows in range(2000, 16000, 700):                                  # (no launch takes more than what any may)
+        assert need(8, 16, 128, 128, 2000, rows=rows) <= need(8, 16, 128, 128, 2000)
+    assert need(64, 16, 128, 128, 900) == 0                               # too short to be cut
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,dim,vdim,longest", [(32, 64, 64, 2500), (32, 64, 128, 2500), (16, 128, 128, 2500), (16, 128, 128, 8000)])
 def test_a_batch_of_unequal_prompts_in_segments(heads, dim, vdim, longest):
