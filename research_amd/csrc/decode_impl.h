@@ -363,7 +363,6 @@ template <typename KV, int D, int NREP> struct MergeShape {
                               : NREP >= 4 && 4 * per_head <= kBudget ? 4
                               : NREP >= 2 && 2 * per_head <= kBudget ? 2
                                                                      : 1;
-    static constexpr int AUX = HR * ROWS * ROWF;   // float offset of the weights
     static constexpr int FLOATS = HR * ROWS * (ROWF + 3);
     // the host-visible statement of the same arithmetic (the launch checks the workgroup's LDS against it)
     static_assert(ROWS == plan_merge_rows(D, (int)sizeof(KV)) && HR == plan_merge_heads_per_round(D, (int)sizeof(KV), NREP) &&
@@ -548,23 +547,6 @@ __device__ __forceinline__ bool arrive_is_last(unsigned long long *ticket, int e
     return last;
 }
 
-// How the pieces w0..w1 of one (plane, sequence) are merged inside the split pass.  Up to kInlinePieces pieces: the
-// workgroup that delivers the last of them merges them all.  More (one sequence that dominates its batch is cut
-// into hundreds): the pieces form groups of `group` consecutive workgroups, the last arrival of a group merges the
-// group into the slot of the group's first piece, and the last group to finish merges the groups - two levels of
-// at most 32 partials each instead of one workgroup reading hundreds.
-constexpr int kInlinePieces = 8;
-struct PieceTree {
-    int pieces, group, n_groups;
-};
-__device__ __forceinline__ PieceTree piece_tree(int pieces) {
-    PieceTree t;
-    t.pieces = pieces;
-    t.group = pieces <= kInlinePieces ? pieces : pieces <= 64 ? 8 : pieces <= 256 ? 16 : 32;
-    t.n_groups = (pieces + t.group - 1) / t.group;
-    return t;
-}
-
 // Merge `count` partials of (plane, sequence b) - the slots of workgroups w_first, w_first + stride, ... - one
 // thread per (query head, four consecutive d), the loads of PIPE partials in flight at a time.  FINAL: normalise and
 // write the plane's output rows; otherwise leave the merged partial in the slot of workgroup w_first (every thread
@@ -640,15 +622,13 @@ struct PieceRef {
 // Count the piece and do whatever merging falls to this workgroup.  s_flag: one LDS word.
 template <typename QT, int D, int NREP>
 __device__ __forceinline__ void deliver_piece(const DecodeArgs &a, const PieceRef &pp, int *s_flag, int tid) {
-    const PieceTree t = piece_tree(pp.w1 - pp.w0 + 1);
+    const PieceTree t = plan_piece_tree(pp.w1 - pp.w0 + 1);
     const int me = (int)blockIdx.x - pp.w0;  // index of this workgroup's piece
     const int g = me / t.group;
     const int g_first = pp.w0 + g * t.group;                      // workgroup of the group's first piece
     const int g_count = min(t.group, t.pieces - g * t.group);     // pieces of this group
     unsigned long long *seq_ticket = a.tickets + ((int64_t)pp.plane * a.batch + pp.b);
-    // a group's ticket is found by the workgroup of its first piece; a workgroup can be that for the sequence that
-    // runs on into it (a later group of it) and for the sequence that starts in it (group 0 of it)
-    unsigned long long *grp_ticket = a.group_tickets + (2 * (int64_t)g_first + (g == 0 ? 1 : 0));
+    unsigned long long *grp_ticket = a.group_tickets + plan_group_ticket(g_first, g);
     wait_all_memory();  // this thread's stores have reached the memory side
     __syncthreads();
     if (tid == 0) *s_flag = arrive_is_last(t.n_groups == 1 ? seq_ticket : grp_ticket, g_count);
@@ -674,7 +654,7 @@ constexpr int kChunkDealUnits = 64;
 
 // Batches up to this size get their block prefix sum from every wave on its own (no barrier); larger ones from the
 // workgroup's scan through LDS.
-constexpr int kWaveScanBatch = 512;
+constexpr int kWaveScanBatch = kPlanWaveScanBatch;
 
 // Inclusive prefix sum of x over the 64 lanes of a wave: four shifted adds inside each row of 16 lanes (a lane
 // with no source in its row adds 0), then the totals of the rows before a lane's own, read through scalars.

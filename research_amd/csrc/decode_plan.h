@@ -16,7 +16,6 @@ namespace pa_decode_detail {
 
 constexpr int kPlanMaxBatch = 8192;      // sequences per call (their block prefix sum lives in LDS)
 constexpr int kPlanMaxSplitGrid = 4096;  // upper bound of the split pass's grid, fixes the caller's workspace size
-constexpr int kPlanMinUnitsPerWorkgroup = 4;
 // Arrival tickets of the merge inside the split pass: 64-bit counters in a region of fixed size at the start of
 // every workspace, so that calls of any shape use the same bytes for the same purpose and nothing else is ever
 // written there: kPlanTicketSlots counters per (plane, sequence), then 2 per workgroup of the largest grid for the
@@ -86,13 +85,6 @@ PA_PLAN_FN int plan_blocks_of(int len, int block_size, int window) {
 PA_PLAN_FN int64_t plan_unit_begin(int64_t w, int64_t total, int64_t grid) { return w * total / grid; }
 PA_PLAN_FN int plan_owner_of(int64_t u, int64_t total, int64_t grid) { return (int)(((u + 1) * grid - 1) / total); }
 
-// Workgroups that take part: with little work a workgroup per pool block would leave hundreds of one-block
-// partials, so a workgroup gets at least kPlanMinUnitsPerWorkgroup units and the rest of the grid leaves at once.
-PA_PLAN_FN int plan_effective_grid(int64_t total, int grid) {
-    const int64_t g = total / kPlanMinUnitsPerWorkgroup;
-    return g < 1 ? 1 : (g < grid ? (int)g : grid);
-}
-
 // Short launches are flattened in runs of u blocks of one (plane, sequence) instead of single blocks, with a workgroup per
 // run: what a workgroup spends is a chain of waits per sequence that it touches (5 to 10 us), hardly more for one block of
 // it than for eight, so a range that crosses from one sequence into the next takes twice as long.  Returns u: the smallest of
@@ -101,7 +93,10 @@ PA_PLAN_FN int plan_effective_grid(int64_t total, int grid) {
 // blocks of the launch.  Ranges of at least four blocks took 20.7 us for 4 sequences of 100 keys at 32 / 8 heads of 128, runs
 // take 13.9; 31 -> 14 us for 256 sequences of 16 keys; at 14 / 2 heads of 64, 4 sequences of 16 keys 52.6 -> 13.7, 16 of 1000
 // keys 31 -> 17, 4 of 6000 keys 33 -> 20.  (Single blocks for one sequence of 6000 keys: 20 us at 8 / 2 heads of 128, runs of
-// four 15; hence the line at 48 blocks per pair.)
+// four 15; hence the line at 48 blocks per pair.)  Above kPlanWaveScanBatch sequences, where the table of units comes from one scan,
+// single blocks and the whole grid: 600 sequences of up to 16 keys 39 -> 31 us at 32 / 8 heads of 128, 54 -> 24 at 14 / 2 of 64; 900 of up to
+// 24 keys 55 -> 54 at 32 / 8.
+constexpr int kPlanWaveScanBatch = 512;
 constexpr int kPlanRunMost = 4, kPlanShortBlocks = 48;
 template <typename F> PA_PLAN_FN int plan_run_blocks(int64_t total, int64_t keys, int grid, F units) {
     if (total > (int64_t)kPlanRunMost * grid) return 1;
@@ -123,6 +118,26 @@ PA_PLAN_FN int plan_run_grid(int64_t total, int grid) { return total < grid ? (i
 // Partial slot of the piece of (plane, sequence) that workgroup w computed: unique, because along the flattened
 // order both w and plane*batch + sequence only grow.
 PA_PLAN_FN int64_t plan_slot(int w, int plane, int batch, int b) { return (int64_t)w + (int64_t)plane * batch + b; }
+
+// How the pieces of one (plane, sequence) are merged inside the split pass.  Up to kPlanInlinePieces pieces: the
+// workgroup that delivers the last of them merges them all.  More (one sequence that dominates its batch is cut
+// into hundreds): the pieces form groups of `group` consecutive workgroups, the last arrival of a group merges the
+// group into the slot of the group's first piece, and the last group to finish merges the groups - two levels of
+// at most 32 partials each instead of one workgroup reading hundreds.
+constexpr int kPlanInlinePieces = 8;
+struct PieceTree {
+    int pieces, group, n_groups;
+};
+PA_PLAN_FN PieceTree plan_piece_tree(int pieces) {
+    PieceTree t;
+    t.pieces = pieces;
+    t.group = pieces <= kPlanInlinePieces ? pieces : pieces <= 64 ? 8 : pieces <= 256 ? 16 : 32;
+    t.n_groups = (pieces + t.group - 1) / t.group;
+    return t;
+}
+// A group's ticket is found by the workgroup of its first piece; a workgroup can be that for the sequence that runs on into
+// it (a later group of it) and for the sequence that starts in it (group 0 of it).
+PA_PLAN_FN int64_t plan_group_ticket(int first, int group) { return 2 * (int64_t)first + (group == 0 ? 1 : 0); }
 
 // workspace = [tickets uint64[kPlanTicketSlots]] [block_prefix int32[batch+1]] [part_ml float[slots][heads][2]]
 //             [part_acc float[slots][heads][D]], heads = hpw*nrep_t query heads of one plane,

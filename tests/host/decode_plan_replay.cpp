@@ -20,7 +20,7 @@ using namespace pa_decode_detail;
     } while (0)
 
 // stats: [0] units, [1] workgroups taking part, [2] partial pieces, [3] rows finished in place, [4] largest slot,
-//        [5] slot capacity, [6] most pieces of one (plane, sequence), [7] workspace bytes
+//        [5] slot capacity, [6] most pieces of one (plane, sequence), [7] workspace bytes, [8] blocks of a unit
 extern "C" int pa_plan_replay(const int32_t *seq_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,
                               int kv_elem_bytes, int block_size, int window, int launch_grid, int grid_cap,
                               int64_t *stats, char *err, int errlen) {
@@ -29,14 +29,27 @@ extern "C" int pa_plan_replay(const int32_t *seq_lens, int batch, int num_q_head
     if (batch < 1 || batch > kPlanMaxBatch) FAIL("batch out of range");
     const WsPlan ws = plan_workspace(batch, h, head_dim, grid_cap);
     const int planes = h.planes();
-    // ---- what every workgroup computes first: blocks before each sequence ----
+    // ---- what every workgroup computes first: units (runs of blocks) before each sequence ----
     std::vector<int64_t> prefix(batch + 1, 0);
-    for (int b = 0; b < batch; ++b) prefix[b + 1] = prefix[b] + plan_blocks_of(seq_lens[b], block_size, window);
-    if (prefix[batch] > 0x7fffffffll) FAIL("block prefix sum leaves 32 bits");
+    auto blocks_of = [&](int b) { return plan_blocks_of(seq_lens[b], block_size, window); };
+    int64_t blocks = 0;
+    for (int b = 0; b < batch; ++b) blocks += blocks_of(b);
+    if (blocks > 0x7fffffffll) FAIL("block prefix sum leaves 32 bits");
+    int run = 1;
+    auto scan = [&](int u, bool keep) {
+        int carry = 0;
+        for (int b = 0; b < batch; ++b) {
+            if (keep) prefix[b] = carry;
+            carry += plan_runs_of(blocks_of(b), u);
+        }
+        return carry;
+    };
+    prefix[batch] = batch <= kPlanWaveScanBatch ? plan_wave_prefix(planes, batch, launch_grid, run, scan) : scan(1, true);
     const int64_t per_plane = prefix[batch];
     const int64_t total = per_plane * planes;
-    for (int i = 0; i < 8; ++i) stats[i] = 0;
+    for (int i = 0; i < 9; ++i) stats[i] = 0;
     stats[0] = total;
+    stats[8] = run;
     stats[5] = ws.slots;
     stats[7] = (int64_t)ws.total;
     if (plan_split_lds_bytes(batch, head_dim, kv_elem_bytes, h.nrep_t) > 65536) FAIL("workgroup LDS above 64 KB");
@@ -48,8 +61,8 @@ extern "C" int pa_plan_replay(const int32_t *seq_lens, int batch, int num_q_head
           ws.ml_off % 256 == 0 && ws.acc_off % 256 == 0))
         FAIL("workspace regions overlap or are misaligned");
     if (total == 0) return 0;
-    const int grid = plan_effective_grid(total, launch_grid);
-    if (grid < 1 || grid > launch_grid) FAIL("effective grid %d outside [1, %d]", grid, launch_grid);
+    const int grid = plan_run_grid(total, launch_grid);
+    if (grid < 1 || grid > launch_grid) FAIL("grid of %d outside [1, %d]", grid, launch_grid);
     stats[1] = grid;
 
     // ---- split pass ----
@@ -70,17 +83,19 @@ extern "C" int pa_plan_replay(const int32_t *seq_lens, int batch, int num_q_head
                 if (prefix[mid] <= off) lo = mid; else hi = mid;
             }
             const int b = lo;
-            const int64_t nblk = prefix[b + 1] - prefix[b];
+            const int64_t nblk = prefix[b + 1] - prefix[b];  // units
             const int64_t blk0 = off - prefix[b];
             const int64_t blk1 = std::min(nblk, blk0 + (end - cur));
             if (nblk < 1 || blk0 < 0 || blk0 >= nblk || blk1 <= blk0)
                 FAIL("workgroup %d: search landed on sequence %d (blocks %lld) with range [%lld, %lld)", w, b,
                      (long long)nblk, (long long)blk0, (long long)blk1);
             if (plane >= planes) FAIL("plane %d of %d", plane, planes);
-            // the blocks it reads: first visible block + [blk0, blk1) must lie inside the sequence
+            // the blocks it reads: first visible block + the runs' blocks must lie inside the sequence, the last unit's up to its end
             const int len = seq_lens[b];
             const int fb = plan_first_key(len, window) / block_size;
-            if ((fb + blk1 - 1) * (int64_t)block_size >= len) FAIL("sequence %d: block %lld past its %d keys", b, (long long)(fb + blk1 - 1), len);
+            const int64_t read0 = blk0 * run, read1 = std::min<int64_t>(blk1 * run, blocks_of(b));
+            if (read0 >= read1 || (fb + read1 - 1) * (int64_t)block_size >= len) FAIL("sequence %d: blocks %lld to %lld of its %d keys", b, (long long)read0, (long long)read1, len);
+            if (blk1 == nblk && read1 != blocks_of(b)) FAIL("sequence %d: %lld of %d blocks read", b, (long long)read1, blocks_of(b));
             for (int64_t u = cur; u < cur + (blk1 - blk0); ++u) {
                 if (owner[(size_t)u] != -1) FAIL("unit %lld attended twice", (long long)u);
                 owner[(size_t)u] = w;
@@ -105,6 +120,24 @@ extern "C" int pa_plan_replay(const int32_t *seq_lens, int batch, int num_q_head
     }
     for (int64_t u = 0; u < total; ++u)
         if (owner[(size_t)u] == -1) FAIL("unit %lld attended by nobody", (long long)u);
+
+    // ---- the merge inside the split pass: groups of pieces, each with a ticket and a slot of its own ----
+    std::set<int64_t> tickets;
+    for (int plane = 0; plane < planes; ++plane)
+        for (int b = 0; b < batch; ++b) {
+            const std::vector<int> &held = pieces[(size_t)plane * batch + b];
+            if (held.empty()) continue;
+            const PieceTree t = plan_piece_tree((int)held.size());
+            if (t.group < 1 || t.group > 32 || (int64_t)t.group * t.n_groups < t.pieces || (int64_t)t.group * (t.n_groups - 1) >= t.pieces)
+                FAIL("%d pieces in %d groups of %d", t.pieces, t.n_groups, t.group);
+            for (int g = 0; g < t.n_groups && t.n_groups > 1; ++g) {
+                const int first = held[0] + g * t.group;
+                const int64_t ticket = plan_group_ticket(first, g);
+                if (ticket >= 2 * (int64_t)launch_grid) FAIL("group ticket %lld of %d workgroups", (long long)ticket, launch_grid);
+                if (!tickets.insert(ticket).second) FAIL("group ticket %lld counts for two groups", (long long)ticket);
+                if (!slots_written.count(plan_slot(first, plane, batch, b))) FAIL("group %d of sequence %d has no slot", g, b);
+            }
+        }
 
     // ---- reduction pass (and the tickets of the merge inside the split pass): per output row ----
     for (int b = 0; b < batch; ++b)

@@ -31,11 +31,11 @@ def replay(tmp_path_factory):
 
     def run(lens, shape, block_size=16, window=0, grid=512, grid_cap=4096):
         lens = np.ascontiguousarray(lens, dtype=np.int32)
-        stats = np.zeros(8, dtype=np.int64)
+        stats = np.zeros(9, dtype=np.int64)
         err = ctypes.create_string_buffer(256)
         rc = fn(lens.ctypes.data, len(lens), *shape, block_size, window, grid, grid_cap, stats.ctypes.data, err, 256)
         assert rc == 0, f"{err.value.decode()} (B={len(lens)}, shape={shape}, bs={block_size}, window={window}, grid={grid})"
-        return dict(zip(("units", "workgroups", "pieces", "in_place", "max_slot", "slot_cap", "max_pieces", "ws_bytes"),
+        return dict(zip(("units", "workgroups", "pieces", "in_place", "max_slot", "slot_cap", "max_pieces", "ws_bytes", "run"),
                         stats.tolist()))
     return run
 
@@ -75,6 +75,19 @@ def test_ragged_batches(replay, seed):
         s = replay(lens, shape, block_size=bs, window=window, grid=grid, grid_cap=max(grid, 4096) if rng.random() < 0.5 else grid)
         assert s["max_slot"] < s["slot_cap"]
         assert s["pieces"] + s["in_place"] >= (1 if s["units"] else 0)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_short_launches_in_runs_of_blocks(replay, shape):
+    """Batches of at most a few blocks a workgroup: units of one, two and four blocks, with slots, pieces and merge groups of their own."""
+    rng, taken = np.random.default_rng(sum(shape)), set()
+    for i in range(150):
+        batch = int(rng.choice([1, 2, 5, 16, 64, 150, 512, 513, 700]))
+        lens = np.exp(rng.uniform(0, np.log(rng.choice([40, 600, 9000]) * 16 // batch + 20), batch)).astype(int) - 1
+        s = replay(lens, shape, block_size=int(rng.choice([16, 16, 8, 32])), window=int(rng.choice([0, 0, 300, -128])), grid=int(rng.choice([512, 512, 64, 304])))
+        assert s["run"] == 1 or batch <= 512
+        taken.add(s["run"])
+    assert taken == {1, 2, 4}
 
 
 def test_extremes(replay):
