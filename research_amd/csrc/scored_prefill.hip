@@ -42,8 +42,9 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
     // The rows with the most keys of all sequences come first, and sequences take turns on the dies and inside them (an odd number of
     // them does by itself: 9 of 700 .. 4000 rows in turn 435 us, else 320); the second workgroup of each compute unit comes the other
     // way round, so that the longest shares its unit with a short one.  8 sequences of 400 .. 4000 rows, 16 heads of 128, in turn, on the
-    // dies alone, with fixed places: over one head of keys 185 / 406 / 659 us, two 172 / 239 / 627, four 172 / 184 / 625, eight 184 / 185 /
-    // 366, sixteen 176 / 176 / 228 (unordered about 240); 4 of them over four 200 / 326 / 277; 8 equal ones 93 / 95 / 91.
+    // dies alone, with fixed places: over one head of keys 171 / 406 / 659 us, two 172 / 239 / 627; on the dies alone, with fixed places:
+    // over four 185 / 625, eight 185 / 366, sixteen 176 / 228 (unordered about 240); 4 of them over four 197 / 329 / 277; 8 equal ones
+    // 93 / 95 / 91.
     int kvh = blockIdx.x, turn = blockIdx.z, y = blockIdx.y;
     const uint64_t per = (uint64_t)gridDim.x * gridDim.y, place = per * turn + gridDim.x * (uint64_t)y + kvh;
     const uint32_t both = (uint32_t)min(2 * (uint64_t)cus, per * gridDim.z);
@@ -53,7 +54,7 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
         kvh = back % one % gridDim.x;
         y = back % one / gridDim.x;
     }
-    const int b = gridDim.y % 2 == 0 ? sequence_in_turn(y, turn, (int)gridDim.y) : y;
+    const int b = gridDim.y % 2 == 0 ? sequence_in_turn(y, turn, (int)gridDim.y, turns_miss_groups(gridDim.x, gridDim.y)) : y;
     ScoredPortion p;
     if (!scored_portion(a, b, p)) return;
     const int n_tasks = (p.n + 31) / 32 * a.n_rep;

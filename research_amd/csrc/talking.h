@@ -39,11 +39,11 @@ __device__ __forceinline__ float talk_masked_bias(float size, float rate, int di
 // Which sequence a workgroup takes whose index in them is x, in the row block (from the longest rows) y.  Workgroups go to the
 // eight XCDs in turn, so that b = x would keep a sequence on one of them where their number is a multiple of 8, on some where it is
 // even, and a batch of ragged lengths would wait for the one with the longest: 8 sequences of 818 to 3868 tokens with 16 heads
-// 1260 us, in turn 519.  An odd number turns by itself, and equal lengths are better off with a sequence's keys on one XCD (7 ragged
+// 1260 us, in turn 508.  An odd number turns by itself, and equal lengths are better off with a sequence's keys on one XCD (7 ragged
 // ones with 32 heads of 96 x 64: 91 us, in turn 100; 16 of 500 tokens 77, in turn 80).
 __device__ __forceinline__ int talk_sequence(const TalkArgs &a, int x, int y) {
     const bool turn = a.batch % 2 == 0 && a.n_rows != (int64_t)a.batch * a.max_q_len;
-    return turn ? sequence_in_turn(x, y, a.batch) : x;
+    return turn ? sequence_in_turn(x, y, a.batch, true) : x;
 }
 
 constexpr int kTalkMaxHeads = 128;

@@ -15,7 +15,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 @pytest.fixture(scope="module")
 def order(tmp_path_factory):
     at = tmp_path_factory.mktemp("turns")
-    (at / "t.cpp").write_text('#include "sequence_turns.h"\nextern "C" int order(int x, int turn, int batch) { return sequence_in_turn(x, turn, batch); }\n')
+    (at / "t.cpp").write_text('#include "sequence_turns.h"\nextern "C" int order(int x, int turn, int batch, int side) { return sequence_in_turn(x, turn, batch, turns_miss_groups(side, batch)); }\n')
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "research_amd", "csrc"), "-o", str(at / "t.so"),
                     str(at / "t.cpp")], check=True)
     return ctypes.CDLL(str(at / "t.so")).order
@@ -27,7 +27,7 @@ def test_no_place_gets_most_of_a_sequence(order, batch, side):
     turns = 256
     seen = np.zeros((batch, 8, 4), dtype=np.int64)
     for turn in range(turns):
-        took = [order(x, turn, batch) for x in range(batch)]
+        took = [order(x, turn, batch, side) for x in range(batch)]
         assert sorted(took) == list(range(batch))
         for x, b in enumerate(took):
             for s in range(side):
