@@ -341,7 +341,7 @@ template <typename KV, typename QT, int D, int NREP, int U> struct Attender {
 };
 
 // Merge the kWaves*TPW row-group partials of every (kv head of the group,
-// query head r) and hand (qh, d, num[4], M, den) of the merged partial - four
+// query head r) and hand (live, qh, d, num[4], M, den) of the merged partial - four
 // consecutive d at a time - to `emit`; out = num/den, M is the base-2 running
 // maximum.
 //
@@ -413,6 +413,9 @@ template <bool EXACT, int NREP, int EPL> __device__ __forceinline__ void merge_l
     if (low <= 32) merge_lane_pairs<32, EXACT>(st, 32);
 }
 
+// `emit` may have one branch by lane at most: where two end at the same place the compiler widens exec once, for both, and under register
+// pressure it puts copies of accumulators that later rounds need in front of that, where only the inner branch's lanes get them (eight
+// query heads per kv head over fp8 pools of 64: two of sixteen values of head 5 were lost in pieces of a sequence).
 template <typename KV, int D, int NREP, int HR, typename Emit>
 __device__ __forceinline__ void merge_rounds(RowState<NREP, RowShape<KV, D>::EPL> &st, float *s_part, const PoolArgs &p,
                                              const LaneRole &role, int prow, int tid, int hg, int rep0, Emit emit) {
@@ -463,7 +466,6 @@ __device__ __forceinline__ void merge_rounds(RowState<NREP, RowShape<KV, D>::EPL
             const int d = (o & (D / 4 - 1)) * 4, hd = o / (D / 4);
             const int hl = hd & (hpw - 1), h = hd >> lg_hpw;
             const int r = round * HR + h;
-            if (rep0 + r >= p.n_rep) continue;
             const float *base = s_part + (h * rows + hl) * ROWF + d;
             const float *wgt = s_wgt + h * rows + hl;
             float num[4] = {0.f, 0.f, 0.f, 0.f};
@@ -473,7 +475,7 @@ __device__ __forceinline__ void merge_rounds(RowState<NREP, RowShape<KV, D>::EPL
 #pragma unroll
                 for (int j = 0; j < 4; ++j) num[j] = fmaf(f, base[w * hpw * ROWF + j], num[j]);
             }
-            emit((hg * hpw + hl) * p.n_rep + rep0 + r, d, num, s_M[h * rows + hl], s_den[h * rows + hl]);
+            emit(rep0 + r < p.n_rep, (hg * hpw + hl) * p.n_rep + rep0 + r, d, num, s_M[h * rows + hl], s_den[h * rows + hl]);
         }
     }
     __syncthreads();
@@ -792,8 +794,8 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
             const int ez = a.extra_zero ? max(0, a.extra_zero[b]) : 0;
             QT *orow = reinterpret_cast<QT *>(a.out) + (int64_t)b * p.hq * p.d;
             merge_rows<KV, D, NREP>(st, s_part, p, wave, tid, hg, rep0,
-                                    [&](int qh, int d, const float (&num)[4], float M, float den) {
-                                        if (d >= p.d) return;
+                                    [&](bool live, int qh, int d, const float (&num)[4], float M, float den) {
+                                        if (!live || d >= p.d) return;
 #pragma unroll
                                         for (int j = 0; j < 4; ++j)
                                             pa_scalar<QT>::store(orow + (int64_t)qh * p.d + d + j,
@@ -805,20 +807,19 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
                 float *acc = a.part_acc + slot * (p.hpw * NREP * D);
                 float *ml = a.part_ml + slot * (p.hpw * NREP * 2);
                 merge_rows<KV, D, NREP>(st, s_part, p, wave, tid, hg, rep0,
-                                        [&](int qh, int d, const float (&num)[4], float M, float den) {
+                                        [&](bool live, int qh, int d, const float (&num)[4], float M, float den) {
+                                            if (!live) return;
                                             const int kv = qh / p.n_rep;
                                             const int idx = (kv - hg * p.hpw) * NREP + (qh - kv * p.n_rep - rep0);
+                                            // (all d of a row store its M and den, the same values: see merge_rounds)
                                             if (a.merge_in_split) {  // uniform: read by another workgroup of this launch
                                                 st_coherent(acc + idx * D + d, num[0], num[1]);
                                                 st_coherent(acc + idx * D + d + 2, num[2], num[3]);
-                                                if (d == 0) st_coherent(ml + idx * 2, M, den);
+                                                st_coherent(ml + idx * 2, M, den);
                                             } else {
                                                 *reinterpret_cast<float4 *>(acc + idx * D + d) =
                                                     float4{num[0], num[1], num[2], num[3]};
-                                                if (d == 0) {
-                                                    ml[idx * 2] = M;
-                                                    ml[idx * 2 + 1] = den;
-                                                }
+                                                *reinterpret_cast<float2 *>(ml + idx * 2) = float2{M, den};
                                             }
                                         });
             }
@@ -1041,8 +1042,8 @@ __global__ __launch_bounds__(kThreads) void prefill_rowwise_kernel(const Rowwise
         k_lo / p.bs, nblk, wave, kWaves, false, role, lane, kvh, rep0);
     QT *orow = reinterpret_cast<QT *>(a.out) + qrow * p.hq * p.d;
     merge_rows<KV, D, NREP>(st, s_part, p, wave, tid, hg, rep0,
-                            [&](int qh, int d, const float (&num)[4], float M, float den) {
-                                if (d >= p.d) return;
+                            [&](bool live, int qh, int d, const float (&num)[4], float M, float den) {
+                                if (!live || d >= p.d) return;
 #pragma unroll
                                 for (int j = 0; j < 4; ++j)
                                     pa_scalar<QT>::store(orow + (int64_t)qh * p.d + d + j, den > 0.f ? num[j] / den : 0.f);

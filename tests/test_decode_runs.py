@@ -130,3 +130,26 @@ def test_launches_of_runs_on_the_device(replay, run, lens, hq, hkv, d, kv):
     got = ops.decode(q, k, v, tables, n, b.bs, b.scale, ws)
     assert_close(got, po.paged_decode(b.q, b.k, b.v, b.tables, b.lens, b.bs, b.scale), b.tol, "runs of blocks")
     assert torch.equal(ops.decode(q, k, v, tables, n, b.bs, b.scale, ws), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("queries", ["bf16", "f16"])
+@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("hq,hkv", [(14, 2), (16, 2), (32, 4), (8, 1), (64, 8)])
+def test_pieces_of_wide_groups_over_fp8_pools(hq, hkv, d, queries):
+    """Up to eight query heads per kv head: kernels that have no registers to spare, sequences in one piece and in several, merged in
+    a second launch and in the one."""
+    from oracle import paged_oracle as po
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.test_gpu_decode_merge import Batch
+
+    announce(f"fp8 pieces {hq}/{hkv}x{d} {queries}")
+    for lens in ([12, 33, 16, 100], [300, 20, 40], [40, 17, 90, 5] * 70):
+        b = Batch(lens, hq, hkv, d, "fp8", seed=d)
+        (k, v, ks, vs), (kr, vr) = b.device_pools()
+        q = b.q.to(torch.float16 if queries == "f16" else torch.bfloat16)
+        got = ops.decode(q.to(DEV), k, v, tables_to_device(b.tables), torch.tensor(b.lens, dtype=torch.int32, device=DEV), b.bs, b.scale,
+                         ops.decode_workspace(q.to(DEV), k), None, ks, vs)
+        # (weights are multiplied by scales and packed to 16 bits: 2^-9 of values of at most 4)
+        assert_close(got, po.paged_decode(q.float(), kr.float(), vr.float(), b.tables, b.lens, b.bs, b.scale), 2e-2, f"{len(lens)} sequences")
