@@ -133,10 +133,11 @@ template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
 // (the matrix cores are busy a sixth of the time).  So a tile lies in LDS in the one layout that both of its products read (K by
 // rows and, with transposing reads, by columns), results leave the registers straight for the output, and the first pass leaves out
 // each portion's last segment, whose state the second pass itself writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128,
-// in five segments: first pass 55 -> 47 us, second 127 -> 116.
+// in five segments: first pass 55 -> 47 us, second 127 -> 116 (41 and 94 since pieces are placed by their lengths).
 // PAIR: at dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
-// chunk, let two share one: 13 % faster where there are two (101 us here; 12 prompts of 400 .. 4000 rows, all passes, 180 -> 163), and
-// 3 to 8 % slower where not.
+// chunk, let two share one.  Where segments outnumber the units: 6 prompts of 2164 .. 8112 rows, 16 heads of 128 x 128, all passes,
+// 294 -> 271 us; 4 of 1271 .. 5972, 40 heads of 96 x 80, 312 -> 281; over 70 batches up to 10 % faster, at most 2.5 % slower.  Elsewhere 3 to
+// 8 % slower.
 template <int KD, int NW, bool STATES, bool PAIR>
 __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(const LaArgs a) {
     constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
