@@ -138,7 +138,7 @@ constexpr float kClSmall = 0x1p-100f;  // a block whose P falls below has its sc
 // KD: dim padded to 64, 128 or 256.  NW: waves; each owns 16 value columns.
 template <int KD, int NW, bool STATES> struct ClTile {
     static constexpr int rows = KD == 256 ? 32 : 64, blocks = rows / kClBlock, cols = 16 * NW, threads = 64 * NW;
-    static constexpr int pitch = KD + 8, vPitch = cols + 8;
+    static constexpr int pitch = KD + 8, vPitch = cols + kLaPadV;
     static constexpr int elems = rows * pitch;                       // one bf16 term of a tile
     static constexpr int units = KD / 2 * rows / 8;                  // (channel pair, 8 rows)
     static constexpr int passes = (units + threads - 1) / threads;

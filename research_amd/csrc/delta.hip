@@ -150,7 +150,6 @@ template <typename T, int R> __global__ __launch_bounds__(256, 4) void delta_rec
 }
 
 // ------------------------------------------------------------------ chunks: T and C
-constexpr int kDcPitch = 72;  // bf16 per row of T and C in LDS
 struct DeltaChunk {           // what the first pass leaves per chunk and head (columns of T and C paired)
     uint16_t t_hi[64][64], t_lo[64][64], c_hi[64][64], c_lo[64][64];
     float k_in[64];   // e^F times k's unit factor (on K S)
@@ -174,9 +173,9 @@ __device__ __forceinline__ float delta_scan(float x, int lane) {
 
 // Workgroup: one chunk of one head.  Wave w: rows 16 w .. of the products.
 template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delta_prepare_kernel(const DeltaArgs a) {
-    constexpr int kLd = KD + 8, kMat = 68, kRowBytes = 2 * 64 * kLd * 2, kMatBytes = 2 * 64 * kMat * 4;
+    constexpr int kMat = 68, kRowBytes = 2 * 64 * KD * 2, kMatBytes = 2 * 64 * kMat * 4;
     __shared__ __align__(16) char room[kRowBytes > kMatBytes ? kRowBytes : kMatBytes];
-    __bf16 *q_s = reinterpret_cast<__bf16 *>(room), *k_s = q_s + 64 * kLd;
+    __bf16 *q_s = reinterpret_cast<__bf16 *>(room), *k_s = q_s + 64 * KD;
     // in their place once the products are made: A below the diagonal, (I + A)^-1
     float(*mat)[kMat] = reinterpret_cast<float(*)[kMat]>(room), (*inv)[kMat] = mat + 64;
     __shared__ float part[4][16][17];
@@ -199,8 +198,8 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
             const int blk = tid + 256 * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
             const LaBlock x = la_load_block(tq, la_block_off(a.ldq, r, c, a.dim), (uint32_t)a.ldq * 2u);
             const LaBlock y = la_load_block(tk, la_block_off(a.ldk, r, c, a.dim), (uint32_t)a.ldk * 2u);
-            la_put_block<false>(x, r, c, q_s, kLd);
-            la_put_block<false>(y, r, c, k_s, kLd);
+            la_put_hashed<KD>(x, r, c, q_s);
+            la_put_hashed<KD>(y, r, c, k_s);
         }
     }
     if (wave == 0) {
@@ -219,7 +218,7 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
         float q2 = 0.f, k2 = 0.f;
 #pragma unroll 4
         for (int d = tid % 4 * 8; d < KD; d += 32) {
-            const bf8 x = la_read8(q_s + r * kLd + d), y = la_read8(k_s + r * kLd + d);
+            const bf8 x = la_read_hashed<KD>(q_s, r, d / 8), y = la_read_hashed<KD>(k_s, r, d / 8);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 q2 = fmaf((float)x[j], (float)x[j], q2);
@@ -248,11 +247,11 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
     for (int st = 0; st < 4; ++st) kk[st] = qk[st] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int d = 0; d < KD / 32; ++d) {
-        const bf8 bk = la_read8(k_s + (16 * wave + l16) * kLd + 32 * d + 8 * g), bq = la_read8(q_s + (16 * wave + l16) * kLd + 32 * d + 8 * g);
+        const bf8 bk = la_read_hashed<KD>(k_s, 16 * wave + l16, 4 * d + g), bq = la_read_hashed<KD>(q_s, 16 * wave + l16, 4 * d + g);
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             if (st > wave) continue;
-            const bf8 x = la_read8(k_s + (16 * st + l16) * kLd + 32 * d + 8 * g);
+            const bf8 x = la_read_hashed<KD>(k_s, 16 * st + l16, 4 * d + g);
             kk[st] = la_mfma(x, bk, kk[st]);
             qk[st] = la_mfma(x, bq, qk[st]);
         }
@@ -333,12 +332,12 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
 // walk then lacks registers).  8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128: 273 -> 187 us; eight waves a workgroup, whose
 // SIMDs have two each: 32 prompts of about 900 rows, with the first pass, 324 -> 311.
 template <int KD, int COLS> constexpr size_t delta_walk_lds() {
-    return (size_t)(2 * 64 * KD + 64 * (COLS + 8) + 4 * 64 * kDcPitch) * 2 + 3 * 64 * 4 + 64;
+    return (size_t)(2 * 64 * KD + 64 * (COLS + kLaPadV) + 4 * 64 * 64) * 2 + 3 * 64 * 4 + 64;
 }
 
 // KD: dim padded to 64, 128 or 256.  A workgroup of NW waves owns 16 NW value columns of a head and all chunks of a portion.
 template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW == 4 ? 2 : 1) void delta_walk_kernel(const DeltaArgs a) {
-    constexpr int kCols = 16 * NW, kThr = 64 * NW, kLv = kCols + 8;
+    constexpr int kCols = 16 * NW, kThr = 64 * NW, kLv = kCols + kLaPadV;
     constexpr int kBlocks = 16 * (KD / 4), kKB = (kBlocks + kThr - 1) / kThr;  // 4 x 4 blocks of K, of V; 16-byte pieces of T and C
     constexpr bool kFew = NW < 8;  // a SIMD has one wave: all its registers
     constexpr int kVB = 16 * (kCols / 4) / kThr, kMB = 4 * (kFew ? 48 : 64) * 8 / kThr;
@@ -348,8 +347,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
     extern __shared__ __align__(16) char lds[];
     __bf16 *q_s = reinterpret_cast<__bf16 *>(lds), *k_s = q_s + 64 * KD, *v_s = k_s + 64 * KD;
     __bf16 *m_s = v_s + 64 * kLv;  // T's two terms, C's two terms
-    float *rows = reinterpret_cast<float *>(m_s + 4 * 64 * kDcPitch);  // k_in, q_in, k_out
-    const __bf16 *t_hi = m_s, *t_lo = m_s + 64 * kDcPitch, *c_hi = m_s + 2 * 64 * kDcPitch, *c_lo = m_s + 3 * 64 * kDcPitch;
+    float *rows = reinterpret_cast<float *>(m_s + 4 * 64 * 64);  // k_in, q_in, k_out
+    const __bf16 *t_hi = m_s, *t_lo = m_s + 64 * 64, *c_hi = m_s + 2 * 64 * 64, *c_lo = m_s + 3 * 64 * 64;
     const int h = blockIdx.x, v0 = blockIdx.y * kCols, b = blockIdx.z;
     DeltaPortion p;
     if (!delta_portion(a, b, p)) return;
@@ -435,7 +434,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         for (int i = 0; i < kMB; ++i) {
             int row, col;
             piece(lt + kThr * i, row, col);
-            *reinterpret_cast<la_u4 *>(m_s + row * kDcPitch + col * 8) = mb[i];
+            *reinterpret_cast<la_u4 *>(m_s + row * 64 + (col ^ la_hash<64>(row)) * 8) = mb[i];
         }
 #pragma unroll
         for (int i = 0; i < kKB; ++i) {
@@ -476,7 +475,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
                 xq[dd & 1][tt] = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
             }
         };
-        auto mat = [&](const __bf16 *m, int tt, int kk) { return la_read8(m + (16 * tt + l16) * kDcPitch + 32 * kk + 8 * g); };
+        auto mat = [&](const __bf16 *m, int tt, int kk) { return la_read_hashed<64>(m, 16 * tt + l16, 4 * kk + g); };
         read_rows(0);
 #pragma unroll
         for (int dd = 0; dd < KD / 32; ++dd) {

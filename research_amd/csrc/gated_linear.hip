@@ -192,7 +192,7 @@ struct GlRows {
 };
 
 // Elements of the tiles: K and Q (paired), V (row-major), the two terms of the weighted scores.
-template <int KD, int NW> constexpr int gl_kv_elems() { return 64 * KD + 64 * (16 * NW + 8); }
+template <int KD, int NW> constexpr int gl_kv_elems() { return 64 * KD + 64 * (16 * NW + kLaPadV); }
 template <int KD, int NW, int KIND, bool STATES> constexpr size_t gl_lds_bytes() {
     const size_t elems = STATES ? 2 * gl_kv_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
                                 : gl_kv_elems<KD, NW>() + 64 * KD + 2 * 64 * kLaPitchA;
@@ -230,7 +230,7 @@ __device__ __forceinline__ float gl_scan_max(float x, int lane) {
 // 181 -> 172 us for the second pass, 68 -> 71 for the first; 128 prompts of 16 .. 130 rows (SSD, 64 heads of 128 x 64) 178 -> 172.
 template <int KD, int NW, int KIND, bool STATES>
 __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_chunk_kernel(const GlArgs a) {
-    constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
+    constexpr int kCols = 16 * NW, kLdV = kCols + kLaPadV, kThr = 64 * NW;
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     constexpr int kNd = (KD / 32 + NW - 1) / NW;  // kMlstm: 32-row pieces of n per wave

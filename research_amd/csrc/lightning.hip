@@ -119,7 +119,7 @@ template <typename T, int R> __global__ __launch_bounds__(256) void lightning_re
 
 // ------------------------------------------------------------------ chunks on the matrix cores
 // Elements of the tiles: K and Q (paired), V (row-major), the two terms of the decayed scores.
-template <int KD, int NW> constexpr int la_kv_elems() { return 64 * KD + 64 * (16 * NW + 8); }
+template <int KD, int NW> constexpr int la_kv_elems() { return 64 * KD + 64 * (16 * NW + kLaPadV); }
 template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
     const size_t elems = STATES ? 2 * la_kv_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
                                 : la_kv_elems<KD, NW>() + 64 * KD + 2 * 64 * kLaPitchA;
@@ -140,7 +140,7 @@ template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
 // 8 % slower.
 template <int KD, int NW, bool STATES, bool PAIR>
 __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(const LaArgs a) {
-    constexpr int kCols = 16 * NW, kLdV = kCols + 8, kThr = 64 * NW;
+    constexpr int kCols = 16 * NW, kLdV = kCols + kLaPadV, kThr = 64 * NW;
     constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     // Places in memory and in LDS are worked out again where registers run out (16 prompts of 900 .. 1000 rows, 16 heads of 256 x 64:

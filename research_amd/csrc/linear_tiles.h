@@ -22,10 +22,15 @@ __device__ __forceinline__ int la_again(int x) {
 // LDS tiles of Q and K: [64][KD], columns paired, 16-byte chunk c of row r at position c ^ la_hash(r).  Operands that meet a
 // result as their partner have the inner order 4 g + 0 .. 3, 16 + 4 g + 0 .. 3 within 32: stored in that order, a lane's
 // eight elements are one chunk, and four rows of a result's columns are one transposing read, so that no tile is stored
-// transposed as well (which took the conflicting 8-byte writes of a 64-row tile and its space in LDS).  Operand reads (16 rows,
-// one chunk) and transposing reads (four rows, four chunks) both spread over the banks.
+// transposed as well (which took the conflicting 8-byte writes of a 64-row tile and its space in LDS).
+// A 16-byte read is served in four groups of lanes, 0 .. 3, 12 .. 15, 20 .. 27 and the rest of 0 .. 31, and the same of 32 .. 63: it takes 4
+// cycles where a group's places spread over 256 bytes, else 8.  For an operand (lane: row lane % 16, chunk lane / 16) that is rows 0 .. 3
+// and 12 .. 15 of a chunk beside rows 4 .. 11 of the next, hence the minus in la_hash; rows at a pitch of 32 modulo 64 bytes spread too.
+// An 8-byte read is served to lanes 0 .. 31 and 32 .. 63: four-row reads of rows 32 modulo 64 bytes apart take 2 cycles, else 4.
+// (8 prompts of 700 .. 4000 rows, us, with both in their way -> without: lightning 142.4 -> 139.9, delta rule 255.4 -> 250.1, HGRN2 466.0 -> 460.5;
+// mLSTM, 15999 rows, 255.8 -> 253.4.)
 __host__ __device__ constexpr int la_paired(int c) { return (c & ~31) | (c & 12) << 1 | (c & 16) >> 2 | (c & 3); }
-template <int KD> __device__ __forceinline__ int la_hash(int r) { return (KD == 64 ? (r & 2) << 1 : (r & 3) << 2) | (r >> 2 & 3); }
+template <int KD> __device__ __forceinline__ int la_hash(int r) { return (KD == 64 ? (r & 2) << 1 : (r & 3) << 2) | (-(r >> 2) & 3); }
 
 __device__ __forceinline__ f4 la_mfma(bf8 x, bf8 y, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0); }
 
@@ -97,6 +102,14 @@ template <bool ACT, int KD> __device__ __forceinline__ void la_put_paired(LaBloc
     const int e = la_paired(c);
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(tile + (r + i) * KD + (((e >> 3) ^ la_hash<KD>(r + i)) << 3) + (e & 4)) = b.r[i];
+}
+// The same without pairs: chunk c of row r at c ^ la_hash(r)
+template <int KD> __device__ __forceinline__ void la_put_hashed(const LaBlock &b, int r, int c, __bf16 *tile) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(tile + (r + i) * KD + (((c >> 3) ^ la_hash<KD>(r + i)) << 3) + (c & 4)) = b.r[i];
+}
+template <int KD> __device__ __forceinline__ bf8 la_read_hashed(const __bf16 *tile, int row, int chunk) {
+    return la_read8(tile + row * KD + (chunk ^ la_hash<KD>(row)) * 8);
 }
 // Row `row` (row % 16 = l16) of a paired tile, elements of the 32 columns from 32 dd on
 template <int KD> __device__ __forceinline__ bf8 la_read_paired(const __bf16 *tile, int row, int l16, int dd, int g) {
@@ -221,7 +234,8 @@ inline dim3 la_grid(int heads, int slices, int batch, int segments) {
     return segments == 1 ? dim3((unsigned)heads, (unsigned)slices, (unsigned)batch) : dim3((unsigned)heads * slices * batch * segments);
 }
 
-constexpr int kLaPitchA = 72;  // bf16 per row of the decayed scores
+constexpr int kLaPitchA = 80;  // bf16 per row of the decayed scores
+constexpr int kLaPadV = 16;    // bf16 behind a row of values
 
 int la_cus() {
     static int cached[64];
