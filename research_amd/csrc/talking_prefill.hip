@@ -140,7 +140,7 @@ constexpr int kTmOut = 2 * kTmWaves;  // out heads of a workgroup, two per wave
 // HW: heads per wave, 2 or 4.  NG: kv heads of the out heads, whose values are staged by the whole workgroup (0: each wave
 // stages its own).  With two heads per wave the keys of up to NG kv heads are staged as well.
 template <int D, int HW, int NG> struct TmTile {
-    static constexpr int heads = kTmWaves * HW, kPitch = D + 8, vPitch = NG ? D + 16 : D + 8;
+    static constexpr int heads = kTmWaves * HW, kPitch = D + 16, vPitch = NG ? D + 16 : D + 8;
     static constexpr bool keys = NG > 0 && HW == 2;
     static constexpr int pair = 4 * heads;  // bytes of a (key, row) pair: both terms of all heads
     static constexpr int pBytes = kTmKeys * kTmRows * pair, wBytes = kTmOut * kTmRows * kTmKeys * 2, kTile = kTmKeys * kPitch, vTile = kTmKeys * vPitch + (NG ? 3 * 64 : 0);
@@ -287,13 +287,15 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     auto near_slot = [&](int id, int k0, int slots) {
         return SAME && !L::keys ? max(talk_slot_of(a, id, min(k0 + (lane & 31), end - 1), end), 0) : slots;
     };
-    // 16-byte pieces of a pair's row and of a (head, row)'s keys at places that spread over the banks; inside a piece the place
-    // of a wave's weights also turns with key / 4, and that of its keys with head / 4
+    // 16-byte pieces of a pair's row and of a (head, row)'s keys at places that spread over the banks (by the groups of lanes that a
+    // read serves together, linear_tiles.h; with the keys' pitch 8 prompts of 818 .. 3868 tokens 508 -> 494 us); inside a piece the place of a
+    // wave's weights also turns with key / 4, and that of its keys with head / 4
+    const int turn16 = -(l16 >> 2) & 3;
     auto pair_at = [&](int key, int piece) {
-        const int at = HP == 32 ? piece ^ ((l16 >> 1) & 7) : piece ^ ((l16 >> 2) & 3);
+        const int at = HP == 32 ? piece ^ ((l16 >> 1) & 7) : piece ^ turn16;
         return tm_lds + (key * kTmRows + l16) * L::pair + 16 * at;
     };
-    auto weights_at = [&](int head, int piece) { return w_s + (head * kTmRows + l16) * (kTmKeys * 2) + 16 * (piece ^ ((l16 >> 2) & 3)); };
+    auto weights_at = [&](int head, int piece) { return w_s + (head * kTmRows + l16) * (kTmKeys * 2) + 16 * (piece ^ turn16); };
 
     int slots = slot_of(id_of(0), 0), id = id_of(kTmKeys), id_near = near_id(kTmKeys);
     fetch_k(slots, near_slot(near_id(0), 0, slots));
