@@ -180,14 +180,17 @@ int decode_launch(int phases, const void *q, const void *k_cache, const void *v_
     a.tickets = (unsigned long long *)(ws + w.ticket_off);
     a.part_ml = (float *)(ws + w.ml_off);
     a.part_acc = (float *)(ws + w.acc_off);
-    // Batches that leave a sequence few pieces are finished by the split pass alone.
+    // Batches that leave a sequence few pieces, or none, are finished by the split pass alone.
     a.group_tickets = (unsigned long long *)(ws + kPlanGroupTicketOff);
-    a.merge_in_split = phases == (kPhaseSplit | kPhaseReduce) && plan_merge_in_split(batch, plan, grid) ? 1 : 0;
+    a.whole = plan_whole_sequences(batch, plan, head_dim, pa_dtype_bytes(kv_dtype), bt_stride, block_size, window) ? 1 : 0;
+    a.merge_in_split = phases == (kPhaseSplit | kPhaseReduce) && (a.whole || plan_merge_in_split(batch, plan, grid)) ? 1 : 0;
 
     hipStream_t s = (hipStream_t)stream;
     a.split_grid = grid;
     if (phases & kPhaseSplit) {
-        ks.split<<<dim3((unsigned)grid), dim3(kThreads), (size_t)(batch + 1) * sizeof(int), s>>>(a);
+        // (whole sequences: a workgroup for each, so that those that end make room)
+        const unsigned wgs = a.whole ? (unsigned)(plan.planes() * batch) : (unsigned)grid;
+        ks.split<<<dim3(wgs), dim3(kThreads), (size_t)(batch + 1) * sizeof(int), s>>>(a);
         PA_CHECK_LAUNCH("pa_decode split pass");
     }
     if ((phases & kPhaseReduce) && !a.merge_in_split) {

@@ -73,6 +73,7 @@ struct DecodeArgs {
     unsigned long long *tickets;        // [planes*batch]: arrivals per (plane, sequence); zero between launches
     unsigned long long *group_tickets;  // [2*split_grid]: arrivals per group of pieces of a many-piece sequence
     int merge_in_split;     // the workgroup that delivers a sequence's last piece merges the pieces (no second pass)
+    int whole;              // a unit is a whole sequence (so that there are no pieces)
 };
 
 struct RowwiseArgs {
@@ -694,7 +695,7 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
     const int B = a.batch;
 
     const int planes = p.n_hgroups * p.n_rgroups;
-    int run = 1;  // blocks of a unit
+    int run = 1;  // blocks of a unit (0: a whole sequence)
     // ---- prefix sum of units over the batch -----------------------------
     // blocks of sequence b that hold visible keys: [first_key(b) / bs, ceil(L / bs))
     auto blocks_of = [&](int b) { return plan_blocks_of(a.seq_lens[b], p.bs, p.window); };
@@ -714,13 +715,13 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
 #pragma unroll
             for (int c = 0; c < kWaveScanBatch / PA_WAVE; ++c) {
                 if (c * PA_WAVE >= B) break;  // uniform
-                const int r = plan_runs_of(n[c], u), x = wave_inclusive_scan(r, lane);
+                const int r = u ? plan_runs_of(n[c], u) : min(n[c], 1), x = wave_inclusive_scan(r, lane);
                 if (keep && c * PA_WAVE + lane < B) s_prefix[c * PA_WAVE + lane] = carry + x - r;
                 carry += __builtin_amdgcn_readlane(x, PA_WAVE - 1);
             }
             return carry;
         };
-        const int carry = plan_wave_prefix(planes, B, (int)gridDim.x, run, scan);
+        const int carry = a.whole ? scan(run = 0, true) : plan_wave_prefix(planes, B, (int)gridDim.x, run, scan);
         if (lane == 0) s_prefix[B] = carry;
         if (blockIdx.x == 0 && wave == 0)
             for (int b = lane; b <= B; b += PA_WAVE) a.block_prefix[b] = s_prefix[b];
@@ -784,7 +785,8 @@ __global__ __launch_bounds__(kThreads, sizeof(KV) == 2 && D >= 64 ? 2 : 1) void 
         const int L = a.seq_lens[b];
         const int k_lo = window_first_key(p, L);  // the query sits at position L-1
         const int fb = k_lo / p.bs;               // first block with a visible key
-        const int blk0 = unit0 * run, blk1 = min(unit1 * run, plan_blocks_of(L, p.bs, p.window));
+        const int blocks = plan_blocks_of(L, p.bs, p.window);
+        const int blk0 = unit0 * run, blk1 = run ? min(unit1 * run, blocks) : blocks;
 
         RowState<NREP, S::EPL> st = Attender<KV, QT, D, NREP, U>::run(
             p, reinterpret_cast<const QT *>(a.q) + (int64_t)b * p.hq * p.d, p.bt + (int64_t)b * p.bt_stride, k_lo, L,

@@ -194,4 +194,22 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
     return (int64_t)grid <= 2 * keys && keys <= kPlanTicketSlots;
 }
 
+// Whether the block tables are so narrow that a workgroup takes a whole (plane, sequence): nothing is left to merge then, and the second
+// launch (4 us, and its gap) goes.  A workgroup reads its keys at 20 to 45 GB/s, so that the line lies where that takes as long as the
+// second launch: 192 KB of keys and values (32-bit pools, whose loop has fewer loads in flight, 128 KB).  Large batches, whose
+// ranges would cross from one sequence into the next, gain up to 384 KB.  us, before -> whole sequences: 14 / 2 heads of 64 (512 bytes a key),
+// 4 sequences of 64 keys 15.4 -> 11.2, 16 of 256 keys 16.3 -> 15.2, of 512 keys 18.7 -> 20.6, 200 of 256 keys 32 -> 18.5; 32 / 8 of 128
+// (2 KB a key), 4 of 64 keys 13.7 -> 10.8, 32 of up to 96 keys 14.4 -> 12.5, of 256 keys 18.8 -> 22.4, 200 of 128 keys 34 -> 24; fp8 16 / 8 of
+// 128, 16 of 64 keys 13.6 -> 11.1, of 128 keys 13.9 -> 14.4, 200 of 256 keys 33.5 -> 30; 32-bit 8 / 2 of 128, 16 of 64 keys 15.6 -> 11.3,
+// 32 of up to 96 keys 15.9 -> 16.3.
+constexpr int kPlanWholeBytes = 192 * 1024;
+PA_PLAN_FN bool plan_whole_sequences(int batch, const HeadPlan &h, int head_dim, int kv_elem_bytes, int64_t table_blocks, int block_size, int window) {
+    if (batch > kPlanWaveScanBatch) return false;
+    const int64_t span = plan_window_span(window), units = (int64_t)h.planes() * batch;
+    if (span > 0 && span / block_size + 2 < table_blocks) table_blocks = span / block_size + 2;
+    const bool many = batch >= 96 && units >= (kv_elem_bytes == 4 ? 512 : 192);
+    const int64_t most = (kv_elem_bytes == 4 ? kPlanWholeBytes * 2 / 3 : kPlanWholeBytes) * (many ? kv_elem_bytes == 4 ? 3 : 2 : 1);
+    return units <= 65535 && table_blocks <= most / ((int64_t)block_size * h.hpw * head_dim * kv_elem_bytes * 2);
+}
+
 }  // namespace pa_decode_detail
