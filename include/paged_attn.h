@@ -239,7 +239,8 @@ int pa_prefill_paged(const void *q, const void *k_cache, const void *v_cache, vo
  * workgroup's keys into up to 8 pieces run by workgroups of their own, which leave (maximum, sum, unnormalised
  * output row) per piece in the workspace, and a second kernel merges them - the arithmetic of pa_decode's
  * reduction pass.  Results equal pa_prefill_paged's to fp32 merge-order rounding.
- *   total_q        : rows of q / out (every q_starts[b] + q_lens[b] <= total_q)
+ *   total_q        : rows of q / out (every q_starts[b] + q_lens[b] <= total_q); also without a workspace, where it
+ *                    says how unequal the prompts are, and with that how the launch is divided (<= 0: not known)
  *   workspace      : pa_prefill_workspace_bytes(...) bytes, 256-byte aligned, contents need not be initialised;
  *                    NULL or too small for any split: the call is pa_prefill_paged.  A smaller workspace is used
  *                    for as many pieces as it holds.

@@ -147,11 +147,13 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
         mfma = pa_prefill_asm_kernel(dtype, d_pad, lower_bounds, !fits);
         if (!lower_bounds && fits) {
             // The plain instance runs several groups of one (sequence, kv head) per workgroup, which share the
-            // set-up of lengths and slot tables: as many (up to 8) as leave a workgroup for every compute unit.
+            // set-up of lengths and slot tables: as many (up to 8) as leave a workgroup for every compute unit, of
+            // unequal prompts fewer.
             const int row_blocks = (max_q_len + kPfRows - 1) / kPfRows;
             const int64_t groups = (row_blocks * (int64_t)a.p.n_rep + kPfTasks - 1) / kPfTasks;
             const int gpw = plan_groups_per_workgroup(num_kv_heads, groups, batch, prefill_cus());
-            a.groups_per_wg = gpw;
+            a.groups_per_wg = plan_ragged_groups(gpw, num_kv_heads, batch, total_q, max_q_len, kPfTasks * kPfRows / a.p.n_rep,
+                                                 bt_stride * (int64_t)block_size, kPfKeys, prefill_cus());
         }
     }
     // head_dim 256: one 32-row task per wave, loads driven by a table of 16-key groups - which must lie inside one

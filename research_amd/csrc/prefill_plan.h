@@ -62,6 +62,26 @@ PA_PLAN_FN int plan_groups_per_workgroup(int num_kv_heads, int64_t groups, int b
     return gpw;
 }
 
+// The same for prompts of unequal length, given the `rows` of q of all of them: of the groups that equal prompts would share a set-up
+// for, the longest prompt's keep one compute unit at work while others have none left.  A launch of U groups, each c tiles of time, takes
+// about (U / cus) (c + s / g) + g c / 2, of which s is a workgroup's set-up and the last term the wait for the workgroups that end
+// last: least at g^2 = 2 s U / (c cus).  s measures 1.1 tiles (equal prompts, 1 against 4 groups: 32 of 256 rows behind 2048 keys 268 and
+// 261 us; 1 against 8: 64 of 512 rows 316 and 284 us).  us, as for equal prompts -> this: 32 / 8 heads of 128, 16 prompts of 64 ..
+// 1024 rows behind 512 keys 172 -> 104, 32 of 97 .. 512 rows 108 -> 81, 64 of 30 .. 250 rows 78 -> 68, of 200 .. 512 rows 214 -> 212;
+// 14 / 2 heads of 64, 64 of 5 .. 100 rows behind 2000 keys 70 -> 42.
+// Prompts whose rows are 7 / 8 of the longest's or more on average, and calls that do not know (rows <= 0), keep `most`; so do pairs, which
+// leave little to spread (16 / 8 heads of 64, 64 prompts of 30 .. 250 rows behind 512 keys: 69 us, one by one 70).
+PA_PLAN_FN int plan_ragged_groups(int most, int num_kv_heads, int batch, int64_t rows, int64_t max_q_len, int64_t rows_per_group,
+                                  int64_t max_keys, int tile_keys, int cus) {
+    if (most <= 2 || rows <= 0 || 8 * rows >= 7 * max_q_len * batch) return most;
+    const int64_t units = num_kv_heads * (rows / (rows_per_group > 0 ? rows_per_group : 1) + (batch + 1) / 2);  // (a last group is half full)
+    const int64_t behind = max_keys > max_q_len ? max_keys - max_q_len : 0;          // keys before a prompt's own rows
+    const int64_t c = (behind + max_q_len / 2) / tile_keys + 3;                      // tiles, and what a group costs beside its loop
+    int g = 1;
+    while (g < most && 5 * (int64_t)(g + 1) * (g + 1) * c * cus <= 11 * units) ++g;
+    return g;
+}
+
 // The i-th group of the workgroup that is chunk `wg_chunk` of `n_chunks`: one of every n_chunks consecutive groups,
 // counted from the front in even rounds and from the back in odd ones, so that under the causal mask (later groups
 // see more keys) the workgroups' totals come out equal.  Strictly increasing in i; a workgroup stops at its first

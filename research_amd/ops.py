@@ -154,11 +154,11 @@ def prefill_paged(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Ten
             _ptr(ctx_lens), _ptr(q_lens), _ptr(q_starts), _ptr(row_first_key) if row_first_key is not None else None,
             block_tables.shape[0], max_q_len, hq, hkv, d, block_size, total_slots // block_size, float(scale),
             int(window), PA_DTYPE[q.dtype], _stream(q))
-    if workspace is not None and not rowwise:
-        # (``pa_prefill_paged_ws``: the launch is cut into pieces over the keys when it has too few rows for the device)
-        _run("pa_prefill_paged_ws", *args, total_q, _ptr(workspace), workspace.numel() * workspace.element_size())
+    if rowwise:
+        _run("pa_prefill_paged_rowwise", *args)
     else:
-        _run("pa_prefill_paged_rowwise" if rowwise else "pa_prefill_paged", *args)
+        # (also without a workspace, which lets a launch of few rows be cut over the keys: the number of rows says how unequal prompts are)
+        _run("pa_prefill_paged_ws", *args, total_q, _ptr(workspace), 0 if workspace is None else workspace.numel() * workspace.element_size())
     return out
 
 
