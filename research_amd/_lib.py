@@ -1,4 +1,5 @@
-"""ctypes binding of ``libpaged_attn.so`` (signatures: ``include/paged_attn.h``).
+"""ctypes binding of ``libpaged_attn.so`` (signatures: ``include/paged_attn.h``); the tensor-level calls of ``ops.py`` go through
+``_host.so`` (``csrc/host_calls.cpp``), which takes tensors themselves.
 
 The library is built in-tree next to this file by ``research_amd/build.py``.
 There is no fallback: if it is missing, loading raises and every attention
@@ -177,6 +178,11 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
         fn = getattr(lib, name)  # AttributeError names the missing symbol
         fn.restype, fn.argtypes = restype, argtypes
     if path is None:
+        try:
+            from . import _host
+        except ImportError as e:
+            raise FileNotFoundError(f"{os.path.dirname(LIB_PATH)}/_host.so does not load ({e}): build it with `python -m research_amd.build`") from e
+        _host.bind(lib._handle)
         _lib = lib
     return lib
 

@@ -22,19 +22,21 @@ PA_DTYPE = {torch.float32: _lib.PA_F32, torch.bfloat16: _lib.PA_BF16, torch.floa
 QKV_TILE_ROWS = _lib.PA_QKV_TILE_ROWS
 
 
-def _ptr(t: Optional[Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
+try:
+    from . import _host
+    from ._host import dense as _dense, nbytes as _nbytes, row_stride as _row_stride, shaped as _shaped, stream as _stream, typed as _typed
+except ImportError:  # not built: loading the library says so
+    def _dense(*_):
+        _lib.load()
 
-
-def _stream(t: Tensor) -> Optional[int]:
-    if not t.is_cuda:
-        raise RuntimeError(f"libpaged_attn computes only on a HIP device; got a tensor on {t.device}")
-    # (the number alone: torch.cuda.current_stream makes an object around it, 1.9 us of a call's 12)
-    return torch._C._cuda_getCurrentRawStream(t.get_device()) or None
+    _nbytes = _row_stride = _shaped = _stream = _typed = _dense
 
 
 def _run(name: str, *args) -> None:
-    status = getattr(_lib.load(), name)(*args)
+    """Call the library's function: tensors and None as its pointers."""
+    if _lib._lib is None:
+        _lib.load()
+    status = getattr(_host, name)(*args)
     if status:
         _lib.check(name, status)
 
@@ -42,7 +44,7 @@ def _run(name: str, *args) -> None:
 def kv_scatter(k_cache: Tensor, v_cache: Tensor, k_src: Tensor, v_src: Tensor, slots: Tensor) -> None:
     """``cache[slots[i]] = src[i]``; caches ``[total_slots, Hkv, D]``, src ``[N, Hkv, D]``, slots int64 ``[N]``."""
     total_slots, hkv, d = k_cache.shape
-    _run("pa_kv_scatter", _ptr(k_cache), _ptr(v_cache), _ptr(k_src), _ptr(v_src), _ptr(slots), slots.numel(),
+    _run("pa_kv_scatter", k_cache, v_cache, k_src, v_src, slots, slots.numel(),
          total_slots, hkv, d, k_cache.element_size(), _stream(k_cache))
 
 
@@ -58,10 +60,10 @@ def kv_gather(k_cache: Tensor, v_cache: Tensor, block_tables: Tensor, seq_lens: 
     else:
         k_out, v_out = out
         for t in (k_out, v_out):
-            if tuple(t.shape) != (batch, max_len, hkv, d) or t.dtype != k_cache.dtype or not t.is_contiguous():
+            if not _shaped(t, batch, max_len, hkv, d) or t.dtype != k_cache.dtype or not t.is_contiguous():
                 raise ValueError("kv_gather: out tensors must be contiguous [B, max_len, Hkv, D] of the pool's type")
-    _run("pa_kv_gather", _ptr(k_cache), _ptr(v_cache), _ptr(k_out), _ptr(v_out), _ptr(block_tables),
-         block_tables.shape[1], _ptr(seq_lens), batch, max_len, total_slots // block_size, block_size, hkv, d,
+    _run("pa_kv_gather", k_cache, v_cache, k_out, v_out, block_tables,
+         block_tables.shape[1], seq_lens, batch, max_len, total_slots // block_size, block_size, hkv, d,
          k_cache.element_size(), _stream(k_cache))
     return k_out, v_out
 
@@ -96,11 +98,10 @@ def decode(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Tensor, se
     total_slots, hkv, _ = k_cache.shape
     if out is None:
         out = torch.empty_like(q)
-    _run(entry, _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(block_tables), block_tables.shape[1],
-         _ptr(seq_lens), _ptr(extra_zero_keys), _ptr(k_scale), _ptr(v_scale), batch, hq, hkv, d, block_size,
+    _run(entry, q, k_cache, v_cache, out, block_tables, block_tables.shape[1],
+         seq_lens, extra_zero_keys, k_scale, v_scale, batch, hq, hkv, d, block_size,
          total_slots // block_size, float(scale), int(window), PA_DTYPE[q.dtype], PA_DTYPE[k_cache.dtype],
-         _ptr(workspace),
-         workspace.numel() * workspace.element_size(), _stream(q))
+         workspace, _nbytes(workspace), _stream(q))
     return out
 
 
@@ -114,8 +115,8 @@ def decode_static(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Ten
     total_slots, hkv, _ = k_cache.shape
     if out is None:
         out = torch.empty_like(q)
-    _run("pa_decode_static", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(block_tables),
-         block_tables.shape[1], _ptr(seq_lens), _ptr(extra_zero_keys), _ptr(k_scale), _ptr(v_scale), batch, hq, hkv,
+    _run("pa_decode_static", q, k_cache, v_cache, out, block_tables,
+         block_tables.shape[1], seq_lens, extra_zero_keys, k_scale, v_scale, batch, hq, hkv,
          d, block_size, total_slots // block_size, float(scale), int(window), PA_DTYPE[q.dtype],
          PA_DTYPE[k_cache.dtype], _stream(q))
     return out
@@ -150,15 +151,15 @@ def prefill_paged(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Ten
     total_slots, hkv, _ = k_cache.shape
     if out is None:
         out = torch.empty_like(q)
-    args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(block_tables), block_tables.shape[1],
-            _ptr(ctx_lens), _ptr(q_lens), _ptr(q_starts), _ptr(row_first_key) if row_first_key is not None else None,
+    args = (q, k_cache, v_cache, out, block_tables, block_tables.shape[1],
+            ctx_lens, q_lens, q_starts, row_first_key,
             block_tables.shape[0], max_q_len, hq, hkv, d, block_size, total_slots // block_size, float(scale),
             int(window), PA_DTYPE[q.dtype], _stream(q))
     if rowwise:
         _run("pa_prefill_paged_rowwise", *args)
     else:
         # (also without a workspace, which lets a launch of few rows be cut over the keys: the number of rows says how unequal prompts are)
-        _run("pa_prefill_paged_ws", *args, total_q, _ptr(workspace), 0 if workspace is None else workspace.numel() * workspace.element_size())
+        _run("pa_prefill_paged_ws", *args, total_q, workspace, _nbytes(workspace))
     return out
 
 
@@ -201,11 +202,11 @@ def attend_masked(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Ten
         raise ValueError("mask_words must be int32 [total_q, heads, words]")
     if out is None:
         out = torch.empty_like(q)
-    _run("pa_attend_masked", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(block_tables),
-         block_tables.shape[1], _ptr(ctx_lens), _ptr(q_lens), _ptr(q_starts), _ptr(mask_words), mask_words.shape[1],
+    _run("pa_attend_masked", q, k_cache, v_cache, out, block_tables,
+         block_tables.shape[1], ctx_lens, q_lens, q_starts, mask_words, mask_words.shape[1],
          mask_words.shape[2], int(n_keys), block_tables.shape[0], max_q_len, hq, hkv, d, block_size,
-         total_slots // block_size, float(scale), PA_DTYPE[q.dtype], PA_DTYPE[k_cache.dtype], _ptr(k_scale),
-         _ptr(v_scale), _stream(q))
+         total_slots // block_size, float(scale), PA_DTYPE[q.dtype], PA_DTYPE[k_cache.dtype], k_scale,
+         v_scale, _stream(q))
     return out
 
 
@@ -215,7 +216,7 @@ def quantize_kv_e4m3(pool: Tensor, block_size: int) -> Tuple[Tensor, Tensor]:
     num_blocks = total_slots // block_size
     dst = torch.empty(pool.shape, dtype=torch.float8_e4m3fn, device=pool.device)
     scale = torch.empty((num_blocks, hkv), dtype=torch.float32, device=pool.device)
-    _run("pa_quantize_kv_e4m3", _ptr(pool), _ptr(dst), _ptr(scale), num_blocks, block_size, hkv, d,
+    _run("pa_quantize_kv_e4m3", pool, dst, scale, num_blocks, block_size, hkv, d,
          PA_DTYPE[pool.dtype], _stream(pool))
     return dst, scale
 
@@ -263,8 +264,8 @@ def kv_append_e4m3(k_cache: Tensor, v_cache: Tensor, k_scale: Tensor, v_scale: T
     total_slots, hkv, d = k_cache.shape
     num_blocks = total_slots // block_size
     blocks, order, start = _touched_args(touched, slots, block_size, num_blocks)
-    _run("pa_kv_append_e4m3", _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale), _ptr(k_src), _ptr(v_src),
-         _ptr(slots), slots.numel(), _ptr(blocks), blocks.numel(), _ptr(order), _ptr(start), num_blocks, block_size,
+    _run("pa_kv_append_e4m3", k_cache, v_cache, k_scale, v_scale, k_src, v_src,
+         slots, slots.numel(), blocks, blocks.numel(), order, start, num_blocks, block_size,
          hkv, d, PA_DTYPE[k_src.dtype], _stream(k_cache))
 
 
@@ -290,8 +291,8 @@ def rope_kv_append(q: Tensor, k_src: Tensor, v_src: Tensor, cos: Tensor, sin: Te
     if cos.shape != sin.shape or cos.dim() != 2 or cos.shape[1] != d:
         raise ValueError("cos / sin must be [rows, head_dim]")
     total_slots = k_cache.shape[0] if k_cache is not None else 0
-    _run("pa_rope_kv_append", _ptr(q), _ptr(q_out), _ptr(k_src), _ptr(v_src), _ptr(k_out), _ptr(k_cache),
-         _ptr(v_cache), _ptr(cos), _ptr(sin), _ptr(positions), cos.shape[0], _ptr(slots), n, total_slots, hq, hkv, d,
+    _run("pa_rope_kv_append", q, q_out, k_src, v_src, k_out, k_cache,
+         v_cache, cos, sin, positions, cos.shape[0], slots, n, total_slots, hq, hkv, d,
          PA_DTYPE[q.dtype], _stream(q))
     return q_out
 
@@ -313,9 +314,9 @@ def rope_kv_append_e4m3(q: Tensor, k_src: Tensor, v_src: Tensor, cos: Tensor, si
     if positions is not None and positions.dtype != torch.int32:
         raise ValueError("positions must be int32")
     blocks, order, start = _touched_args(touched, slots, block_size, num_blocks)
-    _run("pa_rope_kv_append_e4m3", _ptr(q), _ptr(q_out), _ptr(k_src), _ptr(v_src), _ptr(k_cache), _ptr(v_cache),
-         _ptr(k_scale), _ptr(v_scale), _ptr(cos), _ptr(sin), _ptr(positions), cos.shape[0], _ptr(slots), n,
-         _ptr(blocks), blocks.numel(), _ptr(order), _ptr(start), num_blocks, block_size, hq, hkv, d,
+    _run("pa_rope_kv_append_e4m3", q, q_out, k_src, v_src, k_cache, v_cache,
+         k_scale, v_scale, cos, sin, positions, cos.shape[0], slots, n,
+         blocks, blocks.numel(), order, start, num_blocks, block_size, hq, hkv, d,
          PA_DTYPE[q.dtype], _stream(q))
     return q_out
 
@@ -328,33 +329,12 @@ def dequantize_blocks_e4m3(cache: Tensor, scale: Tensor, block_ids: Tensor, bloc
     if block_ids.dtype != torch.int32:
         raise ValueError("block_ids must be int32")
     dst = torch.empty((block_ids.numel() * block_size, hkv, d), dtype=dtype, device=cache.device)
-    _run("pa_dequantize_blocks_e4m3", _ptr(cache), _ptr(scale), _ptr(block_ids), block_ids.numel(), _ptr(dst),
+    _run("pa_dequantize_blocks_e4m3", cache, scale, block_ids, block_ids.numel(), dst,
          total_slots // block_size, block_size, hkv, d, PA_DTYPE[dtype], _stream(cache))
     return dst
 
 
 # ------------------------------------------------------------------ decoder blocks around attention
-
-
-def _row_stride(t: Tensor) -> int:
-    """Elements between the rows of a 2-D tensor whose rows are contiguous (a column slice of a wider one)."""
-    if t.dim() == 2:
-        (rows, cols), (row, col) = t.shape, t.stride()
-        if cols <= 1 or col == 1:
-            return row if rows > 1 else max(row, cols)
-    raise ValueError("expected a 2-D tensor with contiguous rows")
-
-
-def _dense(*tensors: Optional[Tensor]) -> None:
-    for t in tensors:
-        if t is not None and not t.is_contiguous():
-            raise ValueError("expected contiguous tensors")
-
-
-def _typed(dtype: torch.dtype, *tensors: Optional[Tensor]) -> None:
-    for t in tensors:
-        if t is not None and t.dtype != dtype:
-            raise ValueError(f"expected {dtype}, got {t.dtype}")
 
 
 _NORMS = {None: _lib.PA_NORM_NONE, "layer": _lib.PA_NORM_LAYER, "rms": _lib.PA_NORM_RMS}
@@ -389,26 +369,26 @@ def residual_norm(x: Tensor, dtype: torch.dtype, y: Optional[Tensor] = None, y_w
     _typed(dtype, y, table, pos_table, y_extra, other)
     n = rows if row_index is None else row_index.numel()
     m = mix.shape[1] - 1 if mix is not None else 0
-    if (y is not None and tuple(y.shape) != (rows * (m or 1), width)) or (ids is not None and ids.numel() != rows):
+    if (y is not None and not _shaped(y, rows * (m or 1), width)) or (ids is not None and ids.numel() != rows):
         raise ValueError("y / ids do not fit the residual")
-    if (mix is not None and mix.shape[0] != rows) or (y_extra is not None and tuple(y_extra.shape) != (rows, width)):
+    if (mix is not None and mix.shape[0] != rows) or (y_extra is not None and not _shaped(y_extra, rows, width)):
         raise ValueError("mix / y_extra do not fit the residual")
     if positions is not None and positions.numel() != rows:
         raise ValueError("positions do not fit the residual")
     for t in (table, pos_table):
         if t is not None and t.shape[1] != width:
             raise ValueError("table rows are not as wide as the residual")
-    if other is not None and tuple(other.shape) != (rows, width):
+    if other is not None and not _shaped(other, rows, width):
         raise ValueError("y2 does not fit the residual")
     for w in (y_weight, weight, bias, y_bias, own_part, other_part):
         if w is not None and w.numel() != width:
             raise ValueError("norm weights are not as wide as the residual")
     out = torch.empty((n, width), dtype=dtype, device=x.device) if want_out else None
-    _run("pa_residual_norm", _ptr(x), _ptr(y), _ptr(mix), m, _ptr(y_extra), _ptr(y_bias), _ptr(other), _ptr(own_part),
-         _ptr(other_part), _ptr(y_weight), float(y_eps), _ptr(ids), int(ids_add), _ptr(table),
-         table.shape[0] if table is not None else 0, float(table_scale), _ptr(positions), _ptr(pos_table),
-         pos_table.shape[0] if pos_table is not None else 0, _ptr(row_index), rows, _ptr(weight), _ptr(bias), float(eps),
-         _NORMS[norm], _ptr(out), n, width, PA_DTYPE[dtype], _stream(x))
+    _run("pa_residual_norm", x, y, mix, m, y_extra, y_bias, other, own_part,
+         other_part, y_weight, float(y_eps), ids, int(ids_add), table,
+         table.shape[0] if table is not None else 0, float(table_scale), positions, pos_table,
+         pos_table.shape[0] if pos_table is not None else 0, row_index, rows, weight, bias, float(eps),
+         _NORMS[norm], out, n, width, PA_DTYPE[dtype], _stream(x))
     return out
 
 
@@ -421,14 +401,14 @@ def rms_gate(o: Tensor, gate: Optional[Tensor], weight: Tensor, eps: float, grou
     _dense(o, weight)
     _typed(o.dtype, gate)
     _typed(torch.float32, weight)
-    if (gate is None) != (order is None) or (gate is not None and tuple(gate.shape) != (rows, width)) or weight.numel() != width:
+    if (gate is None) != (order is None) or (gate is not None and not _shaped(gate, rows, width)) or weight.numel() != width:
         raise ValueError("gate / weight do not fit o")
     if out is None:
         out = torch.empty_like(o)
     _typed(o.dtype, out)
-    if tuple(out.shape) != (rows, width):
+    if not _shaped(out, rows, width):
         raise ValueError("out does not fit o")
-    _run("pa_rms_gate", _ptr(o), _ptr(gate), _row_stride(gate) if gate is not None else 0, _ptr(weight), float(eps), _ptr(out), _row_stride(out), rows,
+    _run("pa_rms_gate", o, gate, _row_stride(gate) if gate is not None else 0, weight, float(eps), out, _row_stride(out), rows,
          width, groups, _GATES[order], PA_DTYPE[o.dtype], _stream(o))
     return out
 
@@ -442,7 +422,7 @@ def glu(gate: Tensor, up: Tensor, act: str, ids: Optional[Tensor] = None) -> Ten
     if up.shape[1] != width or (up.shape[0] if ids is None else ids.numel()) != rows:
         raise ValueError("up / ids do not fit gate")
     out = torch.empty((rows, width), dtype=gate.dtype, device=gate.device)
-    _run("pa_glu", _ptr(gate), _row_stride(gate), _ptr(up), _row_stride(up), _ptr(ids), up.shape[0], _ptr(out), rows,
+    _run("pa_glu", gate, _row_stride(gate), up, _row_stride(up), ids, up.shape[0], out, rows,
          width, _ACTS[act], PA_DTYPE[gate.dtype], _stream(gate))
     return out
 
@@ -455,7 +435,7 @@ def bias_act(x: Tensor, bias: Optional[Tensor], act: Optional[str]) -> Tensor:
     if bias is not None and bias.numel() != width:
         raise ValueError("bias does not fit x")
     out = torch.empty((rows, width), dtype=x.dtype, device=x.device)
-    _run("pa_bias_act", _ptr(x), _row_stride(x), _ptr(bias), _ptr(out), rows, width, _ACTS[act], PA_DTYPE[x.dtype], _stream(x))
+    _run("pa_bias_act", x, _row_stride(x), bias, out, rows, width, _ACTS[act], PA_DTYPE[x.dtype], _stream(x))
     return out
 
 
@@ -466,14 +446,14 @@ def head_gate(o: Tensor, gate: Optional[Tensor], vdim: int, scale: float = 1.0, 
     _dense(o)
     if gate is not None:
         _typed(o.dtype, gate)
-        if tuple(gate.shape) != (rows, heads):
+        if not _shaped(gate, rows, heads):
             raise ValueError("gate must hold one logit per row and head")
     if out is None:
         out = torch.empty((rows, heads * vdim), dtype=o.dtype, device=o.device)
     _typed(o.dtype, out)
-    if tuple(out.shape) != (rows, heads * vdim):
+    if not _shaped(out, rows, heads * vdim):
         raise ValueError("out does not fit o")
-    _run("pa_head_gate", _ptr(o), _ptr(gate), _row_stride(gate) if gate is not None else 0, float(scale), _ptr(out),
+    _run("pa_head_gate", o, gate, _row_stride(gate) if gate is not None else 0, float(scale), out,
          _row_stride(out), rows, heads, d, vdim, PA_DTYPE[o.dtype], _stream(o))
     return out
 
@@ -516,20 +496,20 @@ def qkv_conv_append(u: Tensor, portions: Portions, slots: Tensor, k_cache: Tenso
     batch = portions.ctx_lens.numel()
     if slots.numel() != rows or v_cache.shape != k_cache.shape or u.shape[1] < channels:
         raise ValueError("slots / v_cache / u do not fit")
-    if conv_weight is not None and (conv_weight.shape[1] != channels or (taps > 1 and tuple(conv_state.shape[1:]) != (taps - 1, channels))):
+    if conv_weight is not None and (conv_weight.shape[1] != channels or (taps > 1 and not _shaped(conv_state, None, taps - 1, channels))):
         raise ValueError("convolution weights or state of another size")
-    if rope is not None and tuple(rope.shape[1:]) != (rot_dims // 2, 2):
+    if rope is not None and not _shaped(rope, None, rot_dims // 2, 2):
         raise ValueError("rope must be [positions, rot_dims / 2, 2]")
-    if v_first is not None and tuple(v_first.shape) != (rows, hkv * vdim):
+    if v_first is not None and not _shaped(v_first, rows, hkv * vdim):
         raise ValueError("v_first must be [rows, Hkv * vdim]")
     if q_out is None:
         q_out = torch.empty((rows, num_q_heads, d), dtype=u.dtype, device=u.device)
     n_tiles = batch if portions.tiles is None else portions.tiles.shape[0]
-    _run("pa_qkv_conv_append", _ptr(u), _row_stride(u), rows, _ptr(bias), _ptr(conv_weight), taps, _ptr(conv_state),
-         conv_state.shape[0] if conv_state is not None else 0, _ptr(rope), rope.shape[0] if rope is not None else 0,
-         rot_dims if rope is not None else 0, _ptr(portions.ctx_lens), _ptr(portions.q_lens), _ptr(portions.q_starts),
-         _ptr(portions.state_slots), _ptr(portions.tiles), n_tiles, batch, _ptr(slots), total_slots, _ptr(q_out),
-         _ptr(k_cache), _ptr(v_cache), _ptr(v_first), _ptr(v_lambda), _V_MODES[v_mode], _ptr(q_norm), _ptr(k_norm),
+    _run("pa_qkv_conv_append", u, _row_stride(u), rows, bias, conv_weight, taps, conv_state,
+         conv_state.shape[0] if conv_state is not None else 0, rope, rope.shape[0] if rope is not None else 0,
+         rot_dims if rope is not None else 0, portions.ctx_lens, portions.q_lens, portions.q_starts,
+         portions.state_slots, portions.tiles, n_tiles, batch, slots, total_slots, q_out,
+         k_cache, v_cache, v_first, v_lambda, _V_MODES[v_mode], q_norm, k_norm,
          num_q_heads, hkv, dim, vdim, d, int(unit_norm), float(eps), float(q_scale), PA_DTYPE[u.dtype], _stream(u))
     return q_out
 
@@ -556,18 +536,17 @@ def lightning(u: Tensor, portions: Portions, state: Tensor, decay_powers: Tensor
     _typed(u.dtype, out)
     rows, batch = u.shape[0], portions.ctx_lens.numel()
     pad = lambda n: -(-n // 16) * 16
-    if tuple(state.shape[1:]) != (heads, pad(dim), pad(vdim)) or tuple(decay_powers.shape) != (heads, 65):
+    if not _shaped(state, None, heads, pad(dim), pad(vdim)) or not _shaped(decay_powers, heads, 65):
         raise ValueError("state or decay table of another size")
-    if tuple(out.shape) != (rows, heads * vdim):
+    if not _shaped(out, rows, heads * vdim):
         raise ValueError("out must be [rows, heads * vdim]")
-    head = (_ptr(u), _row_stride(u), rows, _ptr(state), state.shape[0], _ptr(decay_powers), _ptr(portions.ctx_lens),
-            _ptr(portions.q_lens), _ptr(portions.q_starts), _ptr(portions.state_slots), batch)
-    tail = (_ptr(out), heads, dim, vdim, PA_DTYPE[u.dtype])
+    head = (u, _row_stride(u), rows, state, state.shape[0], decay_powers, portions.ctx_lens,
+            portions.q_lens, portions.q_starts, portions.state_slots, batch)
+    tail = (out, heads, dim, vdim, PA_DTYPE[u.dtype])
     if portions.q_lens is None or u.dtype == torch.float32:
         _run("pa_lightning_recurrent", *head, *tail, _stream(u))
     else:
-        _run("pa_lightning_chunked", *head, portions.max_q_len, *tail, _ptr(workspace),
-             workspace.numel() * workspace.element_size() if workspace is not None else 0, _stream(u))
+        _run("pa_lightning_chunked", *head, portions.max_q_len, *tail, workspace, _nbytes(workspace), _stream(u))
     return out
 
 
@@ -575,7 +554,7 @@ def softcap(x: Tensor, cap: float) -> Tensor:
     """``cap * tanh(x / cap)`` as float32 (``pa_softcap``)."""
     _dense(x)
     out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-    _run("pa_softcap", _ptr(x), _ptr(out), x.numel(), float(cap), PA_DTYPE[x.dtype], _stream(x))
+    _run("pa_softcap", x, out, x.numel(), float(cap), PA_DTYPE[x.dtype], _stream(x))
     return out
 
 
@@ -591,14 +570,14 @@ def short_conv(u: Tensor, portions: Portions, weight: Tensor, bias: Optional[Ten
     _typed(u.dtype, conv_state)
     if weight.shape[1] != channels or (bias is not None and bias.numel() != channels):
         raise ValueError("weight / bias do not fit u")
-    if taps > 1 and (conv_state is None or tuple(conv_state.shape[1:]) != (taps - 1, channels)):
+    if taps > 1 and (conv_state is None or not _shaped(conv_state, None, taps - 1, channels)):
         raise ValueError("carried rows of another size")
     batch = portions.ctx_lens.numel()
     out = torch.empty((rows, channels), dtype=u.dtype, device=u.device)
-    _run("pa_short_conv", _ptr(u), _row_stride(u), rows, _ptr(weight), _ptr(bias), taps, _ACTS[act], _ptr(conv_state),
-         conv_state.shape[0] if conv_state is not None else 0, _ptr(portions.ctx_lens), _ptr(portions.q_lens),
-         _ptr(portions.q_starts), _ptr(portions.state_slots), _ptr(portions.tiles),
-         batch if portions.tiles is None else portions.tiles.shape[0], batch, _ptr(out), channels, PA_DTYPE[u.dtype], _stream(u))
+    _run("pa_short_conv", u, _row_stride(u), rows, weight, bias, taps, _ACTS[act], conv_state,
+         conv_state.shape[0] if conv_state is not None else 0, portions.ctx_lens, portions.q_lens,
+         portions.q_starts, portions.state_slots, portions.tiles,
+         batch if portions.tiles is None else portions.tiles.shape[0], batch, out, channels, PA_DTYPE[u.dtype], _stream(u))
     return out
 
 
@@ -625,22 +604,21 @@ def gated_linear(kind: str, q: Tensor, k: Tensor, v: Tensor, gates: Tuple[Tensor
     _typed(torch.int32, *portions[:4])
     _typed(torch.float32, state, *constants)
     _typed(v.dtype, q, k, ga, gb, out)
-    qk = (rows, heads // heads_per_group * dim)
-    if tuple(q.shape) != qk or tuple(k.shape) != qk or tuple(v.shape) != (rows, heads * vdim) or out.shape != v.shape:
+    wide = heads // heads_per_group * dim
+    if not _shaped(q, rows, wide) or not _shaped(k, rows, wide) or not _shaped(v, rows, heads * vdim) or out.shape != v.shape:
         raise ValueError("q / k / v / out do not fit each other")
-    if any(c is not None and c.numel() != heads for c in constants) or tuple(ga.shape) != (rows, heads):
+    if any(c is not None and c.numel() != heads for c in constants) or not _shaped(ga, rows, heads):
         raise ValueError("gates / constants do not fit the heads")
     gate_stride = _row_stride(ga)
-    if gb is not None and (tuple(gb.shape) != (rows, heads) or _row_stride(gb) != gate_stride):
+    if gb is not None and (not _shaped(gb, rows, heads) or _row_stride(gb) != gate_stride):
         raise ValueError("the two gates differ in their rows")
-    if tuple(state.shape[1:]) != (heads, gated_linear_state_floats(kind, dim, vdim)):
+    if not _shaped(state, None, heads, gated_linear_state_floats(kind, dim, vdim)):
         raise ValueError("state of another size")
-    _run("pa_gated_linear", _GATED[kind], _ptr(q), _row_stride(q), _ptr(k), _row_stride(k), _ptr(v), _row_stride(v),
-         heads_per_group, _ptr(ga), _ptr(gb), gate_stride, *map(_ptr, constants), float(cap), float(q_scale),
-         float(den_eps), rows, _ptr(state), state.shape[0], _ptr(portions.ctx_lens), _ptr(portions.q_lens),
-         _ptr(portions.q_starts), _ptr(portions.state_slots), batch, portions.max_q_len, _ptr(out), heads, dim, vdim,
-         PA_DTYPE[v.dtype], _ptr(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0,
-         _stream(v))
+    _run("pa_gated_linear", _GATED[kind], q, _row_stride(q), k, _row_stride(k), v, _row_stride(v),
+         heads_per_group, ga, gb, gate_stride, *constants, float(cap), float(q_scale),
+         float(den_eps), rows, state, state.shape[0], portions.ctx_lens, portions.q_lens,
+         portions.q_starts, portions.state_slots, batch, portions.max_q_len, out, heads, dim, vdim,
+         PA_DTYPE[v.dtype], workspace, _nbytes(workspace), _stream(v))
     return out
 
 
@@ -651,7 +629,7 @@ def narrow_linear(x: Tensor, w: Tensor) -> Tensor:
     if w.shape[1] != x.shape[1]:
         raise ValueError("w does not fit x")
     out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32, device=x.device)
-    _run("pa_narrow_linear", _ptr(x), _row_stride(x), _ptr(w), _ptr(out), x.shape[0], w.shape[0], w.shape[1],
+    _run("pa_narrow_linear", x, _row_stride(x), w, out, x.shape[0], w.shape[0], w.shape[1],
          PA_DTYPE[x.dtype], _stream(x))
     return out
 
@@ -683,8 +661,8 @@ def moe_choose(logits: Tensor, experts: int, top: int, groups: int, keep: int, s
     counts = torch.empty(every, dtype=torch.int32, device=dev)
     lists = torch.empty((every, rows), dtype=torch.int32, device=dev)
     workspace = torch.empty(int(_lib.load().pa_moe_workspace_bytes(rows, every, top)), dtype=torch.uint8, device=dev)
-    _run("pa_moe_choose", _ptr(logits), logits.shape[1], rows, experts, identity, top, groups, keep, _SHARED[shared], _SCORES[scores],
-         group_top, int(renormalize), _ptr(correction), _ptr(ids), _ptr(weights), _ptr(counts), _ptr(lists), _ptr(workspace),
+    _run("pa_moe_choose", logits, logits.shape[1], rows, experts, identity, top, groups, keep, _SHARED[shared], _SCORES[scores],
+         group_top, int(renormalize), correction, ids, weights, counts, lists, workspace,
          workspace.numel(), _stream(logits))
     return ExpertChoice(ids, weights, counts[:experts], lists[:experts])
 
@@ -700,8 +678,8 @@ def moe_product(x: Tensor, choice: ExpertChoice, w: Tensor, n: int, k: int, glu:
     if w.shape[0] != choice.counts.numel() or w.shape[1] < n * (2 if glu else 1) or w.shape[2] < k:
         raise ValueError("w does not fit the choice")
     out = torch.empty((rows * top, n), dtype=x.dtype, device=x.device)
-    _run("pa_moe_product", _ptr(x), _row_stride(x), rows * top // x.shape[0] if x.shape[0] else 1, _ptr(w), w.shape[1], w.shape[2], k,
-         _ptr(choice.counts), _ptr(choice.lists), rows, top, w.shape[0], int(glu), _ptr(out), n, PA_DTYPE[x.dtype], _stream(x))
+    _run("pa_moe_product", x, _row_stride(x), rows * top // x.shape[0] if x.shape[0] else 1, w, w.shape[1], w.shape[2], k,
+         choice.counts, choice.lists, rows, top, w.shape[0], int(glu), out, n, PA_DTYPE[x.dtype], _stream(x))
     return out
 
 
@@ -720,18 +698,17 @@ def delta_rule(q: Tensor, k: Tensor, v: Tensor, decay_logits: Tensor, beta_logit
     _typed(torch.int32, *portions[:4])
     _typed(torch.float32, state, decay_bias, decay_rate)
     _typed(v.dtype, q, k, decay_logits, beta_logits, out)
-    qk = (rows, heads // heads_per_group * dim)
-    if tuple(q.shape) != qk or tuple(k.shape) != qk or tuple(v.shape) != (rows, heads * vdim) or out.shape != v.shape:
+    wide = heads // heads_per_group * dim
+    if not _shaped(q, rows, wide) or not _shaped(k, rows, wide) or not _shaped(v, rows, heads * vdim) or out.shape != v.shape:
         raise ValueError("q / k / v / out do not fit each other")
-    if any(tuple(g.shape) != (rows, heads) for g in (decay_logits, beta_logits)) or _row_stride(decay_logits) != _row_stride(beta_logits):
+    if any(not _shaped(g, rows, heads) for g in (decay_logits, beta_logits)) or _row_stride(decay_logits) != _row_stride(beta_logits):
         raise ValueError("the two logits do not fit the heads, or differ in their rows")
-    if decay_bias.numel() != heads or decay_rate.numel() != heads or tuple(state.shape[1:]) != (heads, pad(dim), pad(vdim)):
+    if decay_bias.numel() != heads or decay_rate.numel() != heads or not _shaped(state, None, heads, pad(dim), pad(vdim)):
         raise ValueError("constants or state of another size")
-    _run("pa_delta", _ptr(q), _row_stride(q), _ptr(k), _row_stride(k), _ptr(v), _row_stride(v), heads_per_group, _ptr(decay_logits),
-         _ptr(beta_logits), _row_stride(decay_logits), _ptr(decay_bias), _ptr(decay_rate), float(q_scale), rows, _ptr(state),
-         state.shape[0], _ptr(portions.ctx_lens), _ptr(portions.q_lens), _ptr(portions.q_starts), _ptr(portions.state_slots), batch,
-         portions.max_q_len, _ptr(out), heads, dim, vdim, PA_DTYPE[v.dtype], _ptr(workspace),
-         workspace.numel() * workspace.element_size() if workspace is not None else 0, _stream(v))
+    _run("pa_delta", q, _row_stride(q), k, _row_stride(k), v, _row_stride(v), heads_per_group, decay_logits,
+         beta_logits, _row_stride(decay_logits), decay_bias, decay_rate, float(q_scale), rows, state,
+         state.shape[0], portions.ctx_lens, portions.q_lens, portions.q_starts, portions.state_slots, batch,
+         portions.max_q_len, out, heads, dim, vdim, PA_DTYPE[v.dtype], workspace, _nbytes(workspace), _stream(v))
     return out
 
 
@@ -750,22 +727,22 @@ def hyper_norm(x: Tensor, dtype: torch.dtype, y: Optional[Tensor] = None, betwee
     _typed(torch.int64, ids)
     _typed(dtype, y, y_extra, y_self, table)
     m = mix.shape[1] - (1 if y_self is None else 2) if mix is not None else 0
-    if y is not None and tuple(y.shape) != (rows * (m or 1), width):
+    if y is not None and not _shaped(y, rows * (m or 1), width):
         raise ValueError("y does not fit the streams")
-    if (mix is not None and mix.shape[0] != rows) or any(t is not None and tuple(t.shape) != (rows, width) for t in (y_extra, y_self)):
+    if (mix is not None and mix.shape[0] != rows) or any(t is not None and not _shaped(t, rows, width) for t in (y_extra, y_self)):
         raise ValueError("mix / y_extra / y_self do not fit the streams")
     if ids is not None and (ids.numel() != rows or table.shape[1] != width):
         raise ValueError("ids / table do not fit the streams")
-    if (between is not None and tuple(between.shape) != (streams, streams)) or \
+    if (between is not None and not _shaped(between, streams, streams)) or \
             any(t is not None and t.numel() != streams for t in (into, sum_weight)) or (weight is not None and weight.numel() != width):
         raise ValueError("weights do not fit the streams")
     if want == "out":
         out, sum_ = torch.empty((rows, width), dtype=dtype, device=x.device), None
     else:
         out, sum_ = None, torch.empty((rows, width), dtype=torch.float32, device=x.device)
-    _run("pa_hyper_norm", _ptr(x), _ptr(y), _ptr(mix), m, mix.shape[1] if mix is not None else 0, _ptr(y_extra), _ptr(y_self),
-         _ptr(between), _ptr(into), _ptr(ids), _ptr(table), table.shape[0] if table is not None else 0, _ptr(sum_weight), _ptr(weight),
-         float(eps), _ptr(out), _ptr(sum_), rows, streams, width, PA_DTYPE[dtype], _stream(x))
+    _run("pa_hyper_norm", x, y, mix, m, mix.shape[1] if mix is not None else 0, y_extra, y_self,
+         between, into, ids, table, table.shape[0] if table is not None else 0, sum_weight, weight,
+         float(eps), out, sum_, rows, streams, width, PA_DTYPE[dtype], _stream(x))
     return out if sum_ is None else sum_
 
 
@@ -782,13 +759,13 @@ def latent_append(u: Tensor, portions: Portions, slots: Tensor, pool: Tensor, no
     _typed(torch.int64, slots)
     if one != 1 or slots.numel() != rows or norm.numel() != rank or u.shape[1] < heads * (dim + rot_dim) + rank + rot_dim:
         raise ValueError("slots / pool / norm / u do not fit")
-    if rot_dim and tuple(rope.shape[1:]) != (rot_dim // 2, 2):
+    if rot_dim and not _shaped(rope, None, rot_dim // 2, 2):
         raise ValueError("rope must be [positions, rot_dim / 2, 2]")
     q = torch.empty((rows, heads, q_dim), dtype=u.dtype, device=u.device)
     n_tiles = batch if portions.tiles is None else portions.tiles.shape[0]
-    _run("pa_latent_append", _ptr(u), _row_stride(u), rows, _ptr(norm), float(eps), _ptr(rope), rope.shape[0] if rope is not None else 0,
-         _ptr(portions.ctx_lens), _ptr(portions.q_lens), _ptr(portions.q_starts), _ptr(portions.tiles), n_tiles, batch, _ptr(slots),
-         total_slots, _ptr(q), _ptr(pool), heads, dim, rot_dim, rank, q_dim, pool_row, float(q_scale), PA_DTYPE[u.dtype], _stream(u))
+    _run("pa_latent_append", u, _row_stride(u), rows, norm, float(eps), rope, rope.shape[0] if rope is not None else 0,
+         portions.ctx_lens, portions.q_lens, portions.q_starts, portions.tiles, n_tiles, batch, slots,
+         total_slots, q, pool, heads, dim, rot_dim, rank, q_dim, pool_row, float(q_scale), PA_DTYPE[u.dtype], _stream(u))
     return q
 
 
@@ -798,7 +775,7 @@ def latent_gather(pool: Tensor, slots: Tensor) -> Tensor:
     _typed(torch.int64, slots)
     total_slots, _, row = pool.shape
     out = torch.empty((slots.numel(), row), dtype=pool.dtype, device=pool.device)
-    _run("pa_latent_gather", _ptr(pool), _ptr(slots), total_slots, _ptr(out), slots.numel(), row, PA_DTYPE[pool.dtype], _stream(pool))
+    _run("pa_latent_gather", pool, slots, total_slots, out, slots.numel(), row, PA_DTYPE[pool.dtype], _stream(pool))
     return out
 
 
@@ -820,20 +797,19 @@ def scored_attention(q: Tuple[Tensor, ...], k_cache: Tensor, v_cache: Tensor, vd
     _typed(torch.int32, block_tables, *portions[:4])
     _typed(torch.float32, bias, sink)
     _typed(out.dtype, k_cache, v_cache, *q)
-    if any(tuple(t.shape[:2]) != (rows, heads) or t.stride(2) != 1 for t in q) or not 1 <= len(q) <= 2:
+    if any(not _shaped(t, rows, heads, None) or t.stride(2) != 1 for t in q) or not 1 <= len(q) <= 2:
         raise ValueError("q pieces do not fit each other")
-    if tuple(v_cache.shape[:2]) != (total_slots, kv_heads) or tuple(out.shape) != (rows, heads, vdim):
+    if not _shaped(v_cache, total_slots, kv_heads, None) or not _shaped(out, rows, heads, vdim):
         raise ValueError("v_cache / out do not fit")
     if (bias is not None and bias.shape[0] != heads) or (sink is not None and sink.numel() != heads):
         raise ValueError("bias / sink must have a row per head")
-    piece = lambda t: (_ptr(t), t.stride(0), t.stride(1), t.shape[2])
+    piece = lambda t: (t, t.stride(0), t.stride(1), t.shape[2])
     second = piece(q[1]) if len(q) == 2 else (None, 0, 0, 0)
     batch = portions.ctx_lens.numel()
-    _run("pa_scored_attention", *piece(q[0]), *second, _ptr(k_cache), k_dim, _ptr(v_cache), v_cache.shape[2], vdim, _ptr(block_tables),
-         block_tables.shape[1], block_size, total_slots // block_size, _ptr(portions.ctx_lens), _ptr(portions.q_lens),
-         _ptr(portions.q_starts), rows, batch, portions.max_q_len, heads, kv_heads, float(scale), int(window), float(softcap), _ptr(bias),
-         bias.shape[1] if bias is not None else 0, _ptr(sink), _ptr(out), PA_DTYPE[out.dtype], _ptr(workspace),
-         workspace.numel() * workspace.element_size() if workspace is not None else 0, _stream(out))
+    _run("pa_scored_attention", *piece(q[0]), *second, k_cache, k_dim, v_cache, v_cache.shape[2], vdim, block_tables,
+         block_tables.shape[1], block_size, total_slots // block_size, portions.ctx_lens, portions.q_lens,
+         portions.q_starts, rows, batch, portions.max_q_len, heads, kv_heads, float(scale), int(window), float(softcap), bias,
+         bias.shape[1] if bias is not None else 0, sink, out, PA_DTYPE[out.dtype], workspace, _nbytes(workspace), _stream(out))
     return out
 
 
@@ -853,15 +829,14 @@ def talking_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, vdim: int, po
     _typed(torch.int32, block_tables, *portions[:4])
     _typed(torch.float32, talk, bias_size, bias_rate)
     _typed(out.dtype, k_cache, v_cache, q)
-    if q.stride(2) != 1 or tuple(v_cache.shape[:2]) != (total_slots, kv_heads) or tuple(out.shape) != (rows, heads, vdim):
+    if q.stride(2) != 1 or not _shaped(v_cache, total_slots, kv_heads, None) or not _shaped(out, rows, heads, vdim):
         raise ValueError("q / v_cache / out do not fit")
-    if tuple(talk.shape) != (heads, heads) or any(t is not None and t.numel() != heads for t in (bias_size, bias_rate)):
+    if not _shaped(talk, heads, heads) or any(t is not None and t.numel() != heads for t in (bias_size, bias_rate)):
         raise ValueError("talk / bias_size / bias_rate do not fit the heads")
-    _run("pa_talking_attention", _ptr(q), q.stride(0), q.stride(1), dim, _ptr(k_cache), k_dim, _ptr(v_cache), v_cache.shape[2], vdim,
-         _ptr(block_tables), block_tables.shape[1], block_size, total_slots // block_size, _ptr(portions.ctx_lens), _ptr(portions.q_lens),
-         _ptr(portions.q_starts), rows, portions.ctx_lens.numel(), portions.max_q_len, heads, kv_heads, float(scale), _ptr(bias_size),
-         _ptr(bias_rate), _ptr(talk), _ptr(out), PA_DTYPE[out.dtype], _ptr(workspace),
-         workspace.numel() * workspace.element_size() if workspace is not None else 0, _stream(out))
+    _run("pa_talking_attention", q, q.stride(0), q.stride(1), dim, k_cache, k_dim, v_cache, v_cache.shape[2], vdim,
+         block_tables, block_tables.shape[1], block_size, total_slots // block_size, portions.ctx_lens, portions.q_lens,
+         portions.q_starts, rows, portions.ctx_lens.numel(), portions.max_q_len, heads, kv_heads, float(scale), bias_size,
+         bias_rate, talk, out, PA_DTYPE[out.dtype], workspace, _nbytes(workspace), _stream(out))
     return out
 
 
@@ -879,12 +854,11 @@ def channel_linear(q: Tensor, forget: Tensor, v: Tensor, f_bias: Optional[Tensor
     _typed(torch.int32, *portions[:4])
     _typed(torch.float32, state, f_bias, lower)
     _typed(v.dtype, q, forget, out)
-    if any(tuple(t.shape) != (rows, heads * dim) for t in (q, forget)) or tuple(v.shape) != (rows, heads * vdim) or out.shape != v.shape:
+    if any(not _shaped(t, rows, heads * dim) for t in (q, forget)) or not _shaped(v, rows, heads * vdim) or out.shape != v.shape:
         raise ValueError("q / forget / v / out do not fit each other")
-    if any(t is not None and t.numel() != heads * dim for t in (f_bias, lower)) or tuple(state.shape[1:]) != (heads, pad(dim), pad(vdim)):
+    if any(t is not None and t.numel() != heads * dim for t in (f_bias, lower)) or not _shaped(state, None, heads, pad(dim), pad(vdim)):
         raise ValueError("constants or state of another size")
-    _run("pa_channel_linear", _ptr(q), _row_stride(q), _ACTS[q_act], _ptr(forget), _row_stride(forget), _ptr(f_bias), _ptr(lower), _ptr(v),
-         _row_stride(v), rows, _ptr(state), state.shape[0], _ptr(portions.ctx_lens), _ptr(portions.q_lens), _ptr(portions.q_starts),
-         _ptr(portions.state_slots), batch, portions.max_q_len, _ptr(out), heads, dim, vdim, PA_DTYPE[v.dtype], _ptr(workspace),
-         workspace.numel() * workspace.element_size() if workspace is not None else 0, _stream(v))
+    _run("pa_channel_linear", q, _row_stride(q), _ACTS[q_act], forget, _row_stride(forget), f_bias, lower, v,
+         _row_stride(v), rows, state, state.shape[0], portions.ctx_lens, portions.q_lens, portions.q_starts,
+         portions.state_slots, batch, portions.max_q_len, out, heads, dim, vdim, PA_DTYPE[v.dtype], workspace, _nbytes(workspace), _stream(v))
     return out

@@ -1,0 +1,75 @@
+"""The calls from Python (``research_amd/csrc/host_calls.cpp``) on the CPU: the checks against what they stand for, the arguments that the
+library's functions take, and what is refused."""
+
+import re
+
+import pytest
+import torch
+
+from research_amd import _lib, ops
+
+host = pytest.importorskip("research_amd._host")
+_lib.load()
+
+
+def test_checks():
+    a, b = torch.zeros(3, 8), torch.zeros(4, 6, dtype=torch.int32)
+    host.dense(a, None, b, a[1:], torch.nn.Parameter(a))
+    with pytest.raises(ValueError, match="contiguous"):
+        host.dense(None, b, a[:, 1:])
+    host.typed(torch.float32, a, None, a[:, 1:])
+    with pytest.raises(ValueError, match="expected torch.float32, got torch.int32"):
+        host.typed(torch.float32, None, a, b)
+    assert host.nbytes(None) == 0 and host.nbytes(b) == 96 and host.nbytes(a[:, 1:3].to(torch.bfloat16)) == 12
+    assert host.shaped(a, 3, 8) and host.shaped(a, None, 8) and not host.shaped(a, 3, 7) and not host.shaped(a, 3) and not host.shaped(a, 3, 8, 1)
+    assert host.shaped(torch.zeros(()),) and host.shaped(torch.zeros(0, 2), 0, None)
+    for bad in (3, "x", None):
+        with pytest.raises(TypeError):
+            host.shaped(bad, 1)
+        with pytest.raises(TypeError):
+            host.dense(a, bad if bad is not None else 1.0)
+    with pytest.raises(RuntimeError, match="HIP device"):
+        host.stream(a)
+
+
+@pytest.mark.parametrize("t", [torch.zeros(3, 8), torch.zeros(3, 8)[:, 2:5], torch.zeros(1, 8), torch.zeros(1, 8)[:, :3], torch.zeros(5, 1),
+                               torch.zeros(8, 5)[:, :1], torch.zeros(0, 4), torch.zeros(4, 0), torch.zeros(4, 3).t(), torch.zeros(1, 4, 3)[0].t()[:, :1],
+                               torch.zeros(3, 8)[::2], torch.zeros(8)[None].expand(3, 8), torch.zeros(3), torch.zeros(2, 3, 4), torch.zeros(3, 8)[:, ::2]])
+def test_row_stride(t):
+    want = None
+    if t.dim() == 2:
+        (rows, cols), (row, col) = t.shape, t.stride()
+        if cols <= 1 or col == 1:
+            want = row if rows > 1 else max(row, cols)
+    if want is None:
+        with pytest.raises(ValueError, match="contiguous rows"):
+            host.row_stride(t)
+    else:
+        assert host.row_stride(t) == want
+
+
+def test_every_call_takes_what_the_library_declares():
+    source = open(ops.__file__).read()
+    names = set(re.findall(r'_run\("(pa_\w+)"', source)) | {"pa_decode", "pa_decode_split", "pa_decode_reduce", "pa_prefill_paged"}
+    assert len(names) > 30
+    for name in names:
+        with pytest.raises(TypeError, match=f"takes {len(_lib.SIGNATURES[name][1])} arguments, got 0"):
+            getattr(host, name)()
+
+
+def test_arguments():
+    lib = _lib.load()
+    assert host.pa_moe_workspace_bytes(1000, 64, 8) == lib.pa_moe_workspace_bytes(1000, 64, 8) > 0
+    assert host.pa_moe_workspace_bytes(1000, 64 + (1 << 32), True) == lib.pa_moe_workspace_bytes(1000, 64, 1)  # (integers wrap, as in ctypes)
+    for bad in (1.5, None, "8", torch.zeros(1)):
+        with pytest.raises(TypeError):
+            host.pa_moe_workspace_bytes(1000, 64, bad)
+    t = torch.zeros(4)
+    call = lambda x, out, n, cap: host.pa_softcap(x, out, n, cap, 0, None)
+    assert call(t, None, 0, 1.0) == 0 and call(t.data_ptr(), t, 0, 1) == 0  # (nothing to do)
+    assert call(t, t, -1, 1.0) == _lib.PA_ERR_INVALID_ARG and "softcap" in _lib.last_error()
+    for bad in (1.5, "x", [t]):
+        with pytest.raises(TypeError):
+            call(bad, t, 0, 1.0)
+    with pytest.raises(TypeError):
+        call(t, t, 0, "1")
