@@ -23,9 +23,10 @@ constexpr int kSpKeys = 64, kSpLow = 32, kSpHigh = 64, kSpMaxBias = 4096;  // (m
 constexpr float kSpSlack = 8.f;  // log2 of the factor by which a row's reference maximum may lag
 
 // (values: a transposing read takes 64 bytes of four rows, which spread over the banks at a pitch of 64 modulo 256 bytes; at 16 two prompts of
-// 754 .. 2313 rows, 16 heads of 128 over 4, took 62.4 us, now 59.9)
+// 754 .. 2313 rows, 16 heads of 128 over 4, took 62.4 us, now 59.9; keys and values of 64 gain nothing: 8 heads over 2, 6 prompts of
+// 420 .. 671 rows, 22.3 us at 16, 22.6 at 64)
 template <int DK, int DV> struct SpTile {
-    static constexpr int k_pitch = DK + 8, v_pitch = DV + 32;
+    static constexpr int k_pitch = DK + 8, v_pitch = DK == 64 && DV == 64 ? DV + 8 : DV + 32;
     static constexpr size_t tiles = (size_t)kSpKeys * (k_pitch + v_pitch) * 2;
 };
 
