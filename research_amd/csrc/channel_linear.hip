@@ -41,19 +41,23 @@ __device__ __forceinline__ bool cl_portion(const ClArgs &a, int b, ClPortion &p)
     return p.n > 0 && p.pos0 >= 0 && p.row0 >= 0 && p.row0 + p.n <= a.n_rows;
 }
 
-// f and 1 - f, neither by subtraction from one
+// f and 1 - f, neither by subtraction from one, of 16-bit logits; x: -log2(e) times the logit.  (Past 2^115 f is its lower bound in 32 bits
+// either way, and the product with e would not be finite.  NaN stays NaN.)
+constexpr float kClLog2e = 1.4426950408889634f;
+__device__ __forceinline__ void cl_gate16(float x, float lower, float &f, float &k) {
+    const float e = __builtin_amdgcn_exp2f(__builtin_elementwise_minimum(x, 115.f));
+    const float big = __builtin_amdgcn_rcpf(1.f + e), open = 1.f - lower;
+    f = fmaf(open, big, lower);
+    k = open * (e * big);
+}
 template <typename T> __device__ __forceinline__ void cl_gate(float z, float lower, float &f, float &k) {
-    float e, big;
     if constexpr (sizeof(T) == 4) {
-        e = expf(-fabsf(z));
-        big = 1.f / (1.f + e);
+        const float e = expf(-fabsf(z)), big = 1.f / (1.f + e), small = e * big, open = 1.f - lower;
+        f = fmaf(open, z >= 0.f ? big : small, lower);
+        k = open * (z >= 0.f ? small : big);
     } else {
-        e = __builtin_amdgcn_exp2f(-1.4426950408889634f * fabsf(z));
-        big = __builtin_amdgcn_rcpf(1.f + e);
+        cl_gate16(-kClLog2e * z, lower, f, k);
     }
-    const float small = e * big, open = 1.f - lower;
-    f = fmaf(open, z >= 0.f ? big : small, lower);
-    k = open * (z >= 0.f ? small : big);
 }
 
 // ------------------------------------------------------------------ token by token
@@ -181,6 +185,11 @@ template <int KD> __device__ __noinline__ f4 cl_slow_scores(const uint16_t *uq, 
     return out;
 }
 
+// Bound by the vector unit: per row and channel the gate, three products split into two terms each and q's activation, and per block and wave its
+// part of S split again.  So 1 / P is made once per block instead of by row (P R = B), a last chunk's missing rows are masked in that chunk
+// alone, and the blocks of a chunk are unrolled, with the state's update and the outputs of one block as independent chains between them
+// (outputs of the next block ahead of the barrier behind the scores were slower: they wait for the update).  8 prompts of 700 .. 4000 rows,
+// 32 heads of 128 x 128, both passes: 463 -> 409 us.
 // STATES: only the segment's own contribution to the state and its factors, to the workspace (first pass over a portion in
 // segments).
 template <int KD, int NW, bool STATES>
@@ -246,7 +255,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int d = 2 * pair[u] + e, c = h * a.dim + d;
-            bias[u][e] = d < a.dim && a.bias ? a.bias[c] : 0.f;
+            bias[u][e] = d < a.dim && a.bias ? -kClLog2e * a.bias[c] : 0.f;
             lower[u][e] = d < a.dim ? a.lower[c] : 1.f;
         }
     }
@@ -276,71 +285,81 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     fetch(r_beg);
     for (int r0 = r_beg; r0 < r_end; r0 += kRows) {
         const int nv = r_end - r0 < kRows ? r_end - r0 : kRows;
-        if (!STATES && tid < L::blocks) unsafe[tid] = 0;
         // ---- operands ----
-        bool bad[L::passes];
 #pragma unroll
         for (int u = 0; u < L::passes; ++u) {
-            bad[u] = false;
             if (!mine[u]) continue;
             float f[8][2], k[8][2], up[2] = {1.f, 1.f};
 #pragma unroll
             for (int r = 0; r < 8; ++r)
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const float z = __builtin_bit_cast(float, e ? zr[u][r] & 0xffff0000u : zr[u][r] << 16) + bias[u][e];
-                    cl_gate<pa_bf16>(z, lower[u][e], f[r][e], k[r][e]);
-                    if (8 * oct[u] + r >= nv) {
-                        f[r][e] = 1.f;
-                        k[r][e] = 0.f;
-                    }
-                    up[e] *= f[r][e];
-                }
+                for (int e = 0; e < 2; ++e)
+                    cl_gate16(fmaf(__builtin_bit_cast(float, e ? zr[u][r] & 0xffff0000u : zr[u][r] << 16), -kClLog2e, bias[u][e]), lower[u][e], f[r][e], k[r][e]);
+            if (nv < kRows) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        if (8 * oct[u] + r >= nv) {
+                            f[r][e] = 1.f;
+                            k[r][e] = 0.f;
+                        }
+            }
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                up[0] *= f[r][0];
+                up[1] *= f[r][1];
+            }
             // the other half of the block: what lies ahead of this one, and behind it
             const bool second = lane >= 32;
-            float ahead[2], behind[2];
+            float ahead[2], back[2], open[2];
+            bool bad = false;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const float other = __shfl_xor(up[e], 32, 64);
+                const float other = __shfl_xor(up[e], 32, 64), all = up[e] * other;
                 ahead[e] = second ? other : 1.f;
-                behind[e] = second ? 1.f : other;
-                if (second) whole[(oct[u] >> 1) * KD + 2 * pair[u] + e] = up[e] * other;
-                bad[u] = bad[u] || up[e] * other < kClSmall;
+                back[e] = second ? 1.f : other;
+                if (second) whole[(oct[u] >> 1) * KD + 2 * pair[u] + e] = all;
+                bad = bad || all < kClSmall;
+                open[e] = __builtin_amdgcn_rcpf(all);
+            }
+            if constexpr (!STATES) {  // (the wave's channels of one block; kPairs / 32 waves share it)
+                const bool any = __ballot(bad) != 0;
+                if (lane == 0) unsafe[wave + NW * u] = any;
             }
             uint32_t *dst = reinterpret_cast<uint32_t *>(k_hi) + (8 * oct[u] * kPitch) / 2 + pair[u];
             constexpr int kRow = kPitch / 2, kTerm = L::elems / 2;
-            {
-                float back[2] = {behind[0], behind[1]};
 #pragma unroll
-                for (int r = 7; r >= 0; --r) {
-                    uint32_t hi, lo;
-                    la_split2(k[r][0] * back[0], k[r][1] * back[1], hi, lo);
-                    dst[r * kRow] = hi;
-                    dst[kTerm + r * kRow] = lo;
-                    back[0] *= f[r][0];
-                    back[1] *= f[r][1];
+            for (int r = 7; r >= 0; --r) {  // R K, and, as P R = B in every row, K / P = K / B R (in this order nothing small is lost)
+                const float x = k[r][0] * back[0], y = k[r][1] * back[1];
+                uint32_t hi, lo;
+                la_split2(x, y, hi, lo);
+                dst[r * kRow] = hi;
+                dst[kTerm + r * kRow] = lo;
+                if constexpr (!STATES) {
+                    la_split2(k[r][0] * open[0] * back[0], k[r][1] * open[1] * back[1], hi, lo);
+                    dst[4 * kTerm + r * kRow] = hi;
+                    dst[5 * kTerm + r * kRow] = lo;
                 }
+                back[0] *= f[r][0];
+                back[1] *= f[r][1];
             }
             if constexpr (!STATES) {
                 float fwd[2] = {ahead[0], ahead[1]};
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
-                    float q[2], inv[2];
+                    float q[2];
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         fwd[e] *= f[r][e];
                         q[e] = __builtin_bit_cast(float, e ? qr[u][r] & 0xffff0000u : qr[u][r] << 16);
                         if (a.silu) q[e] = row_silu<pa_bf16>(q[e]);
                         q[e] *= fwd[e];
-                        inv[e] = k[r][e] * __builtin_amdgcn_rcpf(fwd[e]);
                     }
                     uint32_t hi, lo;
                     la_split2(q[0], q[1], hi, lo);
                     dst[2 * kTerm + r * kRow] = hi;
                     dst[3 * kTerm + r * kRow] = lo;
-                    la_split2(inv[0], inv[1], hi, lo);
-                    dst[4 * kTerm + r * kRow] = hi;
-                    dst[5 * kTerm + r * kRow] = lo;
                 }
             }
         }
@@ -352,16 +371,14 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
         if (r0 + kRows < r_end) fetch(r0 + kRows);
         __syncthreads();
         if constexpr (!STATES) {
-            // (flags go up behind the barrier that follows their clearing, and are read behind the next)
-#pragma unroll
-            for (int u = 0; u < L::passes; ++u)
-                if (bad[u]) unsafe[oct[u] >> 1] = 1;
-            __syncthreads();
             // ---- scores: keys 4 g + i, row l16 of the wave's block ----
             if (wave < L::blocks) {
                 const int first = wave * kClBlock;
                 f4 sc = f4{0.f, 0.f, 0.f, 0.f};
-                if (unsafe[wave] == 0) {
+                int bad = 0;
+#pragma unroll
+                for (int i = 0; i < kPairs / 32; ++i) bad |= unsafe[wave * (kPairs / 32) + i];
+                if (__builtin_amdgcn_readfirstlane(bad) == 0) {
 #pragma unroll
                     for (int kk = 0; kk < KD / 32; ++kk) {
                         const int at = (first + l16) * kPitch + 32 * kk + 8 * g;
@@ -386,7 +403,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
             __syncthreads();
         }
         // ---- blocks in turn; every wave its own columns ----
-#pragma unroll 1
+#pragma unroll
         for (int blk = 0; blk < L::blocks; ++blk) {
             if (blk * kClBlock >= nv) break;
             const int first = blk * kClBlock;

@@ -339,6 +339,30 @@ def test_channel_gates_that_forget_everything_or_nothing(shift, logit):
             case.check_states(slots[:2] + [1])
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (1, 128, 128), (1, 256, 80), (3, 40, 72)])
+def test_channel_gates_that_write_little_ahead_of_forgetting(heads, dim, vdim):
+    """Blocks of 16 rows whose first half writes 1e-20 of its values and whose second half forgets nearly everything: products of the two are not
+    numbers of 32 bits, the outputs of the first half are."""
+    announce(f"channels little {heads} {dim} {vdim}")
+    n, gen = 72, torch.Generator().manual_seed(dim)
+    u = torch.randn(n, heads * (2 * dim + vdim), generator=gen).to(BF)
+    q, z, v = u.split([heads * dim, heads * dim, heads * vdim], 1)
+    z[:] = torch.where(torch.arange(n)[:, None] % 16 < 8, 45.0, -6.0).to(BF)  # (a block's factors: 2^-69)
+    f, k = torch.sigmoid(z.double()).view(n, heads, dim), torch.sigmoid(-z.double()).view(n, heads, dim)
+    qd, vd = q.double().view(n, heads, dim), v.double().view(n, heads, vdim)
+    qd, s, want = qd * torch.sigmoid(qd), torch.zeros(heads, dim, vdim, dtype=torch.float64), []
+    for t in range(n):
+        s = f[t][:, :, None] * s + k[t][:, :, None] * vd[t][:, None, :]
+        want.append((s * qd[t][:, :, None]).sum(1).reshape(-1))
+    pad = lambda x: -(-x // 16) * 16
+    state = torch.zeros(1, heads, pad(dim), pad(vdim), device=DEV)
+    out = torch.full((n, heads * vdim), float("nan"), dtype=BF, device=DEV)
+    q, z, v = u.to(DEV).split([heads * dim, heads * dim, heads * vdim], 1)
+    ops.channel_linear(q, z, v, None, torch.zeros(heads * dim, device=DEV), _portions([(0, 0, n)], [0], tiles=False), state, heads, dim, vdim, out, q_act="silu")
+    err = (out.cpu().double() - torch.stack(want)).norm(dim=1) / torch.stack(want).norm(dim=1)
+    assert float(err.max()) < 2.0 ** -8, err  # (the outputs' rounding to 16 bits, at most 2^-9 of each)
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (1, 128, 128), (1, 256, 80), (2, 96, 200)])
 def test_long_portions_run_in_segments(heads, dim, vdim):
     announce(f"channels segments {heads} {dim} {vdim}")
