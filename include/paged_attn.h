@@ -109,8 +109,7 @@ size_t pa_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, i
 /*
  * Kernel launches one pa_decode call of these shapes makes on the current device at most: 1 when the batch is large
  * enough that the split pass merges a sequence's pieces itself, else 2 (split pass, reduction pass); negative on
- * error.  (A call whose block tables are narrow - 192 KB of keys and values of a sequence, and of the kv heads that a
- * workgroup takes - is one launch in any case.)  For callers that time or profile the passes.  (No counterpart in the reference.)
+ * error.  (A call whose block tables are narrow takes other kernels, one launch or, for few sequences in several runs each, two.)  For callers that time or profile the passes.  (No counterpart in the reference.)
  */
 int pa_decode_passes(int batch, int num_q_heads, int num_kv_heads, int head_dim, int kv_dtype);
 

@@ -187,6 +187,21 @@ int decode_launch(int phases, const void *q, const void *k_cache, const void *v_
 
     hipStream_t s = (hipStream_t)stream;
     a.split_grid = grid;
+    a.splits = ks.few ? plan_short_splits(batch, plan, w, pa_dtype_bytes(kv_dtype), bt_stride, block_size, window, num_cus()) : 0;
+    if (a.splits > 0) {
+        a.leave = a.splits > 1 || phases != (kPhaseSplit | kPhaseReduce) ? 1 : 0;
+        if (phases & kPhaseSplit) {
+            const int reps = (plan.n_rep + kPlanShortHeads - 1) / kPlanShortHeads;
+            ks.few<<<dim3((unsigned)num_kv_heads, (unsigned)batch, (unsigned)(reps * a.splits)), dim3(kThreads), 0, s>>>(a);
+            PA_CHECK_LAUNCH("pa_decode (short sequences)");
+        }
+        if ((phases & kPhaseReduce) && a.leave) {
+            const int64_t items = (int64_t)batch * num_q_heads * (head_dim / 4);
+            ks.few_merge<<<dim3((unsigned)((items + kThreads - 1) / kThreads)), dim3(kThreads), 0, s>>>(a);
+            PA_CHECK_LAUNCH("pa_decode (short sequences, merge)");
+        }
+        return PA_OK;
+    }
     if (phases & kPhaseSplit) {
         // (whole sequences: a workgroup for each, so that those that end make room)
         const unsigned wgs = a.whole ? (unsigned)(plan.planes() * batch) : (unsigned)grid;

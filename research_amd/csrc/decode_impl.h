@@ -74,6 +74,7 @@ struct DecodeArgs {
     unsigned long long *group_tickets;  // [2*split_grid]: arrivals per group of pieces of a many-piece sequence
     int merge_in_split;     // the workgroup that delivers a sequence's last piece merges the pieces (no second pass)
     int whole;              // a unit is a whole sequence (so that there are no pieces)
+    int splits, leave;      // decode_short.h: equal runs of a sequence's tiles, a workgroup each; whether their results are left for the merge
 };
 
 struct RowwiseArgs {
@@ -1061,6 +1062,7 @@ struct KernelSet {
     reduce_fn reduce = nullptr;
     reduce_fn reduce_wave = nullptr;  // for batches with few pieces per sequence
     rowwise_fn rowwise = nullptr;
+    split_fn few = nullptr, few_merge = nullptr;  // sequences over narrow tables (decode_short.h; NULL: there are none for these types)
 };
 
 template <typename KV, typename QT, int D> KernelSet kernels_for_d(int nrep_t) {

@@ -1,6 +1,6 @@
 // Instantiates the single-query-row attention kernels for a fp8 KV pool with bf16 queries.
-#include "decode_impl.h"
+#include "decode_short.h"
 
 namespace pa_decode_detail {
-KernelSet pa_kernels_fp8_bf16(int d, int nrep_t) { return kernels_for<pa_fp8, pa_bf16>(d, nrep_t); }
+KernelSet pa_kernels_fp8_bf16(int d, int nrep_t) { return with_short<pa_fp8, pa_bf16>(kernels_for<pa_fp8, pa_bf16>(d, nrep_t), d); }
 }  // namespace pa_decode_detail

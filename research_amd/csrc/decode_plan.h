@@ -194,7 +194,44 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
     return (int64_t)grid <= 2 * keys && keys <= kPlanTicketSlots;
 }
 
-// Whether the block tables are so narrow that a workgroup takes a whole (plane, sequence): nothing is left to merge then, and the second
+// How decode_short.h's kernel takes the launch: 0: not at all; else the runs a sequence's tiles are cut into, a workgroup per (kv head, sequence,
+// run).  From shapes alone; the tables' width stands for the longest sequence.
+// Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (3.5 us: 600 keys of 128).
+// us, the split pass (one launch or two) -> this, sequences of n keys each: 32 / 8 heads of 128, 1 of 256 keys 14.1 -> 7.4, 1024 15.5 -> 9.0, 4096
+// 16.2 -> 12.0; 32 of 256 19.6 -> 8.3; 96 of 256 33.9 -> 19.7; 14 / 2 of 64, 1 of 256 15.2 -> 5.8, 4096 16.4 -> 11.0; 32 of 1024 22.1 -> 11.0, 16384
+// 64 -> 51; 192 of 1024 45 -> 21; fp8 32 / 8 of 128, 32 of 256 24.5 -> 6.8; fp8 14 / 2 of 256, 16 of 2048 47 -> 14.5, 256 of 2048 185 -> 91.
+// Where the split pass stays: its ranges are equal whatever the lengths, so that unequal sequences in long runs are faster there once memory
+// counts.  More than four query heads a kv head hold up its vector unit, so the line lies further out, for fp8 furthest (unequal, keys n / 8 .. n,
+// the split pass -> runs of that length: 32 / 4 heads of 128, 32 of 8192 65 -> 76, 96 of 2048 57 -> 61, equal ones 70 -> 66; 14 / 2 of 64, 128 of
+// 4096 48 -> 40).  32 / 8 of 128, unequal: 16 of 2048 22.4 -> 24.2, 48 of 2048 44.8 -> 47.4, 1024 33 -> 27; equal, 256 of 512 90 -> 94.  One or two
+// query heads a kv head: 16 / 8 of 256, 16 of 1024 19.5 -> 24; 8 / 8 of 64, 3 of 8192 18 -> 24.  8 / 2 of 128, 1 of 8192 14.6 -> 15.2, 4096 14 -> 12.
+// (Over 1400 batches of 1 .. 384 sequences and thirteen shapes none was slower by more than the runs of one side differ, 3 %.)
+constexpr int kPlanShortHeads = 16, kPlanShortTile = 16, kPlanShortRuns = 64;
+PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, int kv_elem_bytes, int64_t table_blocks, int block_size, int window, int cus) {
+    if (block_size % kPlanShortTile != 0 || batch > kPlanWaveScanBatch || h.hkv > 65535) return 0;
+    const int64_t span = plan_window_span(window);
+    if (span > 0 && span / block_size + 2 < table_blocks) table_blocks = span / block_size + 2;
+    const int64_t keys = table_blocks * block_size, reps = (h.n_rep + kPlanShortHeads - 1) / kPlanShortHeads, wgs = (int64_t)h.hkv * batch * reps;
+    int64_t runs = 1;
+    const bool brief = keys * h.d_pad <= 600 * 128;
+    if (!brief) {
+        runs = 4 * wgs <= cus ? cus / wgs : 3 * (int64_t)cus / 2 / wgs;  // (few more workgroups than units are as slow as twice as many)
+        if (runs > keys / 128) runs = keys / 128;
+        if (runs > kPlanShortRuns) runs = kPlanShortRuns;
+        const int64_t room = w.slots * h.heads_per_slot() / ((int64_t)batch * h.hq);  // (their results are as long as a slot's)
+        if (runs > room) runs = room;
+        if (runs < 1) runs = 1;
+    }
+    const int64_t row = (int64_t)h.d_pad * kv_elem_bytes, kb = 1024;
+    const int64_t run_most = h.n_rep > 4 ? (kv_elem_bytes == 1 ? 4096 * row : row <= 128 ? 512 * kb : 256 * kb) : h.n_rep > 2 ? 128 * kb : 64 * kb;
+    const int64_t all_most = h.n_rep > 4 ? (int64_t)1 << 62 : (h.n_rep > 2 ? 128 : 64) * kb * kb;
+    const bool few = h.n_rep <= 4 && wgs < 6 && keys > 4096;
+    const bool fits = (brief || keys / runs * row <= run_most) && wgs * keys * row <= all_most && !few;
+    return fits && runs * reps <= 65535 ? (int)runs : 0;
+}
+
+// Of what the split pass still has (32-bit pools, blocks that are no whole tiles, large batches of 16-bit ones): whether the block tables are so
+// narrow that a workgroup takes a whole (plane, sequence): nothing is left to merge then, and the second
 // launch (4 us, and its gap) goes.  A workgroup reads its keys at 20 to 45 GB/s, so that the line lies where that takes as long as the
 // second launch: 192 KB of keys and values (32-bit pools, whose loop has fewer loads in flight, 128 KB).  Large batches, whose
 // ranges would cross from one sequence into the next, gain up to 384 KB.  us, before -> whole sequences: 14 / 2 heads of 64 (512 bytes a key),

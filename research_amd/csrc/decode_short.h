@@ -1,0 +1,356 @@
+// Decode over narrow block tables (16-bit queries over 16-bit or fp8 pools): a workgroup per (kv head, sequence), or several with a merge behind
+// them (plan_short_splits of decode_plan.h: where, how many, and what they measured).
+//
+// Short sequences are bound by waits and by the instructions that a workgroup fetches once, not by bytes: the split pass, whose loop is unrolled
+// for streams, spent 1.3 us on the table of units, 1.6 on finding its sequence, 2.6 to 3.2 on the keys and 2.5 to 4 on the merge for 17
+// to 47 keys.  Here the length, the block table and the query rows are on their way at once, then all keys and values; the group's query heads (up
+// to 16) are the columns of one matrix product, so that a lane holds four logits of one head and every step stays short:
+//     S = K Q^T     keys as rows, 16 at a time; a lane's 16 bytes of a row are an operand as they come from memory
+//     O^T += V^T P^T   S's layout is P's as an operand; V goes through the wave's own part of LDS, read transposed
+// P is a sum of two 16-bit terms: with one, short sequences came out less exact than the split pass, whose every row of lanes has a weight of
+// one (error against 64 bits, 14 / 2 heads of 64, 8 sequences of 94 .. 683 keys: split pass 1.78e-3, one term 2.06e-3, two 1.67e-3).
+// Waves take tiles of 16 keys in turn, two at a time up to 64 elements a row; their sums meet in LDS with two barriers.  One tile at a time at
+// 128 leaves registers for four workgroups a compute unit: 256 sequences of 16 keys, 32 / 8 heads, 16.1 -> 9.0 us.
+#pragma once
+#include "decode_impl.h"
+
+namespace pa_decode_detail {
+
+template <typename T> struct ShortMfma;
+template <> struct ShortMfma<pa_bf16> {
+    typedef __bf16 x8 __attribute__((ext_vector_type(8)));
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ f4 mul(pa_u4 a, pa_u4 b, f4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(x8, a), __builtin_bit_cast(x8, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ uint32_t pack(float x, float y) {
+        typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, v2{(__bf16)x, (__bf16)y});
+    }
+    static __device__ __forceinline__ float2 unpack(uint32_t w) {
+        return make_float2(__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u));
+    }
+};
+template <> struct ShortMfma<pa_f16> {
+    typedef _Float16 x8 __attribute__((ext_vector_type(8)));
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ f4 mul(pa_u4 a, pa_u4 b, f4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(x8, a), __builtin_bit_cast(x8, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ uint32_t pack(float x, float y) {
+        typedef _Float16 v2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, v2{(_Float16)x, (_Float16)y});
+    }
+    static __device__ __forceinline__ float2 unpack(uint32_t w) {
+        typedef _Float16 v2 __attribute__((ext_vector_type(2)));
+        const v2 h = __builtin_bit_cast(v2, w);
+        return make_float2((float)h[0], (float)h[1]);
+    }
+};
+
+constexpr int kShortHeads = kPlanShortHeads, kShortKeys = kPlanShortTile;  // query heads of a workgroup, keys of a tile
+
+// Four consecutive outputs (rows are multiples of 16 bytes long; the first need not lie on one of 8).
+template <typename QT, typename Num> __device__ __forceinline__ void short_store(QT *to, const Num &num, float best, float den, int ez) {
+    using M = ShortMfma<QT>;
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = finish_row(num[i], best, den, ez);
+    if (((uintptr_t)to & 7u) == 0) {
+        *reinterpret_cast<uint2 *>(to) = make_uint2(M::pack(y[0], y[1]), M::pack(y[2], y[3]));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pa_scalar<QT>::store(to + i, y[i]);
+    }
+}
+
+// Blocks are whole tiles (block_size % 16 == 0).
+// A workgroup has one of a.splits equal runs of its sequence's tiles and, with a.leave, leaves the maximum, sum and unnormalised outputs of its
+// keys for the merge.
+template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void decode_short_kernel(const DecodeArgs a) {
+    using M = ShortMfma<QT>;
+    using f4 = typename M::f4;
+    constexpr bool kFp8 = sizeof(KV) == 1;
+    constexpr int EL = 16 / sizeof(KV), KL = D / (4 * EL);  // elements of a 16-byte load; loads of a tile of K, and of V
+    constexpr int NT = D >= 128 ? 1 : 2;                    // tiles at a time (registers for four waves a SIMD, at 256 two)
+    constexpr int kPitch = D + 16;                          // (four rows of a transposing read lie 32 bytes apart modulo 64)
+    constexpr int HR = D == 256 ? 8 : kShortHeads, kPitchO = D + 4;  // heads merged at a time
+    constexpr int kBytesV = kWaves * NT * kShortKeys * kPitch * 2, kBytesO = kWaves * HR * kPitchO * 4;
+    __shared__ __align__(16) char room[kBytesV > kBytesO ? kBytesV : kBytesO];
+    __shared__ float s_m[kWaves][kShortHeads], s_l[kWaves][kShortHeads];
+    const PoolArgs &p = a.p;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
+    const int kvh = blockIdx.x, b = blockIdx.y, rep0 = (blockIdx.z / a.splits) * kShortHeads, nr = min(kShortHeads, p.n_rep - rep0);
+    const int split = blockIdx.z % a.splits;
+    const int32_t *bt_row = p.bt + (int64_t)b * p.bt_stride;
+    const int tiles_per_block = p.bs / kShortKeys;
+    auto table = [&](int first) {  // the block of tile first + lane (-1: there is none)
+        const int blk = (first + lane) / tiles_per_block;
+        const int bid = blk < p.bt_stride ? bt_row[blk] : -1;
+        return bid < p.num_blocks ? bid : -1;
+    };
+    const bool known = p.window == 0 && a.splits == 1;  // the first tile, ahead of the length
+    int bids = known ? table(0) : -1;
+    const int L = a.seq_lens[b];
+    QT *orow = reinterpret_cast<QT *>(a.out) + ((int64_t)b * p.hq + kvh * p.n_rep + rep0) * p.d;
+    // queries: lane l16 has head rep0 + l16, the elements of its loads of K
+    pa_u4 qr[KL][EL / 8];
+    {
+        const QT *qp = reinterpret_cast<const QT *>(a.q) + ((int64_t)b * p.hq + kvh * p.n_rep + rep0 + (l16 < nr ? l16 : 0)) * p.d;
+#pragma unroll
+        for (int j = 0; j < KL; ++j)
+#pragma unroll
+            for (int e = 0; e < EL / 8; ++e) {
+                const int d = EL * (4 * j + g) + 8 * e;
+                qr[j][e] = l16 < nr && d < p.d ? *reinterpret_cast<const pa_u4 *>(qp + d) : pa_u4{0, 0, 0, 0};
+            }
+    }
+    if (L <= 0 && !a.leave) {  // uniform
+        for (int i = tid; i < nr * p.d; i += kThreads) pa_scalar<QT>::store(orow + i, 0.f);
+        return;
+    }
+    const int ez = a.extra_zero ? max(0, a.extra_zero[b]) : 0;
+    const int k_lo = plan_first_key(L, p.window);
+    int t0 = k_lo / kShortKeys, n_tiles = L > 0 ? (L - 1) / kShortKeys + 1 - t0 : 0;
+    if (a.splits > 1) {
+        const int from = (int)((int64_t)n_tiles * split / a.splits);
+        n_tiles = (int)((int64_t)n_tiles * (split + 1) / a.splits) - from;
+        t0 += from;
+    }
+    const int tok = p.hkv * p.d * (int)sizeof(KV), head = kvh * p.d * (int)sizeof(KV);  // bytes between tokens, before the head
+    uint16_t *vs = reinterpret_cast<uint16_t *>(room) + wave * NT * kShortKeys * kPitch;
+
+    float m = kNegBig, l = 0.f;
+    f4 acc[D / 16];  // O^T: d = 16 dt + 4 g + i, head l16
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) acc[dt] = f4{0.f, 0.f, 0.f, 0.f};
+    pa_u4 kr[NT][KL], vr[NT][KL];
+    float kscale = 1.f, vscale = 1.f;  // of tile `lane` of the 64 at hand
+#pragma unroll 1
+    for (int first = 0; first < n_tiles; first += 64) {
+        const int n = min(64, n_tiles - first), tile0 = t0 + first;
+        if (first > 0 || !known) bids = table(tile0);
+        if constexpr (kFp8) {
+            const int64_t at = bids >= 0 ? (int64_t)bids * p.hkv + kvh : 0;
+            kscale = bids >= 0 ? p.k_scale[at] : 1.f;
+            vscale = bids >= 0 ? p.v_scale[at] : 1.f;
+        }
+        auto fetch = [&](int at) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int tile = tile0 + at + t, bid = at + t < n ? __builtin_amdgcn_readlane(bids, at + t) : -1;
+                const int rows = bid >= 0 ? min(kShortKeys, L - tile * kShortKeys) : 0;  // (rows past them read as zeros)
+                const int skip = k_lo - tile * kShortKeys;                               // rows before the window: zeros of V
+                const int64_t slot = ((int64_t)max(bid, 0) * p.bs + tile % tiles_per_block * kShortKeys) * tok;
+                const int bytes = rows > 0 ? (rows - 1) * tok + head + p.d * (int)sizeof(KV) : 0;
+                const __amdgpu_buffer_rsrc_t k = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.k) + slot), 0, bytes, 0x00020000);
+                const __amdgpu_buffer_rsrc_t v = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.v) + slot), 0, bytes, 0x00020000);
+#pragma unroll
+                for (int j = 0; j < KL; ++j) {
+                    const int d = EL * (4 * j + g);
+                    kr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(k, d < p.d ? l16 * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
+                }
+#pragma unroll
+                for (int j = 0; j < KL; ++j) {
+                    const int c = lane + 64 * j, row = c / (D / EL), d = c % (D / EL) * EL;
+                    vr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(v, d < p.d && row >= skip ? row * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
+                }
+            }
+        };
+        if (wave * NT < n) fetch(wave * NT);
+#pragma unroll 1
+        for (int at = wave * NT; at < n; at += kWaves * NT) {
+            float x[NT][4], mx = m;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                f4 s = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < KL; ++j) {
+                    if constexpr (kFp8) {
+                        uint32_t w[8];
+                        PoolWords<KV, QT>::unpack(kr[t][j], w);
+                        s = M::mul(pa_u4{w[0], w[1], w[2], w[3]}, qr[j][0], s);
+                        s = M::mul(pa_u4{w[4], w[5], w[6], w[7]}, qr[j][1], s);
+                    } else {
+                        s = M::mul(kr[t][j], qr[j][0], s);
+                    }
+                }
+                const int lim = at + t < n ? L - (tile0 + at + t) * kShortKeys : 0, lo = k_lo - (tile0 + at + t) * kShortKeys;
+                float f = p.scale_log2;
+                if constexpr (kFp8) f *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, kscale), (at + t) & 63));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    x[t][i] = 4 * g + i < lim && 4 * g + i >= lo ? s[i] * f : -INFINITY;
+                    mx = fmaxf(mx, x[t][i]);
+                }
+                // V, for the transposing reads
+#pragma unroll
+                for (int j = 0; j < KL; ++j) {
+                    const int c = lane + 64 * j, row = t * kShortKeys + c / (D / EL), d = c % (D / EL) * EL;
+                    pa_u4 *to = reinterpret_cast<pa_u4 *>(vs + row * kPitch + d);
+                    if constexpr (kFp8) {
+                        uint32_t w[8];
+                        PoolWords<KV, QT>::unpack(vr[t][j], w);
+                        to[0] = pa_u4{w[0], w[1], w[2], w[3]};
+                        to[1] = pa_u4{w[4], w[5], w[6], w[7]};
+                    } else {
+                        to[0] = vr[t][j];
+                    }
+                }
+            }
+            if (at + kWaves * NT < n) fetch(at + kWaves * NT);
+            {
+                const float2 y = lane_pair<16>(mx, 16);
+                mx = fmaxf(y.x, y.y);
+                const float2 z = lane_pair<32>(mx, 32);
+                mx = fmaxf(z.x, z.y);
+            }
+            const float alpha = __builtin_amdgcn_exp2f(m - mx);
+            m = mx;
+            l *= alpha;
+            uint32_t pw[4] = {0, 0, 0, 0}, pl[4] = {0, 0, 0, 0};  // the weights as a sum of two terms
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                float e[4], f = 1.f;
+                if constexpr (kFp8) f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vscale), (at + t) & 63));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    e[i] = __builtin_amdgcn_exp2f(x[t][i] - m);  // 0 for masked keys
+                    l += e[i];
+                    if constexpr (kFp8) e[i] *= f;
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    pw[2 * t + i] = M::pack(e[2 * i], e[2 * i + 1]);
+                    const float2 high = M::unpack(pw[2 * t + i]);
+                    float2 rest = make_float2(e[2 * i] - high.x, e[2 * i + 1] - high.y);
+                    if constexpr (kFp8 && std::is_same<QT, pa_f16>::value)  // (a scale beyond the type: the first term alone)
+                        rest = make_float2(rest.x == -INFINITY ? 0.f : rest.x, rest.y == -INFINITY ? 0.f : rest.y);
+                    pl[2 * t + i] = M::pack(rest.x, rest.y);
+                }
+            }
+            const pa_u4 pb{pw[0], pw[1], pw[2], pw[3]}, pc{pl[0], pl[1], pl[2], pl[3]};
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) {
+                typedef short s4 __attribute__((ext_vector_type(4)));
+                auto column = [&](int t) {
+                    uint16_t *from = vs + (t * kShortKeys + 4 * g + l16 / 4) * kPitch + 16 * dt + 4 * (l16 % 4);
+                    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *)from));
+                };
+                const uint2 v0 = column(0), v1 = NT == 2 ? column(1) : make_uint2(0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
+                const pa_u4 v{v0.x, v0.y, v1.x, v1.y};
+                acc[dt] = M::mul(v, pb, acc[dt]);
+                acc[dt] = M::mul(v, pc, acc[dt]);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    {
+        const float2 y = lane_pair<16>(l, 16);
+        l = y.x + y.y;
+        const float2 z = lane_pair<32>(l, 32);
+        l = z.x + z.y;
+    }
+    if (g == 0) {
+        s_m[wave][l16] = m;
+        s_l[wave][l16] = l;
+    }
+    __syncthreads();
+    float top = kNegBig;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, s_m[w][l16]);
+    const float mine = __builtin_amdgcn_exp2f(m - top);
+    float *part = reinterpret_cast<float *>(room);  // (every wave is through with V)
+#pragma unroll
+    for (int h0 = 0; h0 < kShortHeads; h0 += HR) {
+        if (h0 >= nr) break;  // uniform
+        if (h0 > 0) __syncthreads();
+        if (l16 >= h0 && l16 < min(h0 + HR, nr)) {
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt)
+                *reinterpret_cast<f4 *>(part + (wave * HR + l16 - h0) * kPitchO + 16 * dt + 4 * g) = f4{acc[dt][0] * mine, acc[dt][1] * mine, acc[dt][2] * mine, acc[dt][3] * mine};
+        }
+        __syncthreads();
+        const int heads = min(HR, nr - h0);
+#pragma unroll 1
+        for (int item = tid; item < heads * (D / 4); item += kThreads) {
+            const int h = item / (D / 4), d = item % (D / 4) * 4;
+            float best = kNegBig, den = 0.f;
+            f4 num = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) best = fmaxf(best, s_m[w][h0 + h]);
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                den = fmaf(__builtin_amdgcn_exp2f(s_m[w][h0 + h] - best), s_l[w][h0 + h], den);
+                num += *reinterpret_cast<const f4 *>(part + (w * HR + h) * kPitchO + d);
+            }
+            if (d >= p.d) continue;
+            if (a.leave) {  // uniform
+                const int64_t at = ((int64_t)b * p.hq + kvh * p.n_rep + rep0 + h0 + h) * a.splits + split;
+                *reinterpret_cast<f4 *>(a.part_acc + at * p.d + d) = num;
+                if (d == 0) *reinterpret_cast<float2 *>(a.part_ml + 2 * at) = make_float2(best, den);
+                continue;
+            }
+            short_store<QT>(orow + (int64_t)(h0 + h) * p.d + d, num, best, den, ez);
+        }
+    }
+}
+
+// One thread per row and four of its elements.
+template <typename QT> __global__ __launch_bounds__(kThreads) void decode_short_merge_kernel(const DecodeArgs a) {
+    constexpr int kPipe = 8;
+    const PoolArgs &p = a.p;
+    const int per = p.d / 4, item = blockIdx.x * kThreads + threadIdx.x, row = item / per, d = (item - row * per) * 4;
+    if (row >= a.batch * p.hq) return;
+    const float *ml = a.part_ml + (int64_t)row * a.splits * 2, *acc = a.part_acc + (int64_t)row * a.splits * p.d + d;
+    const int ez = a.extra_zero && a.seq_lens[row / p.hq] > 0 ? max(0, a.extra_zero[row / p.hq]) : 0;
+    float best = kNegBig, den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = 0; s < a.splits; s += kPipe) {
+        float m[kPipe], l[kPipe], top = best;
+        float4 x[kPipe];
+#pragma unroll
+        for (int j = 0; j < kPipe; ++j) {
+            const int at = min(s + j, a.splits - 1);
+            const float2 y = *reinterpret_cast<const float2 *>(ml + 2 * at);
+            x[j] = *reinterpret_cast<const float4 *>(acc + (int64_t)at * p.d);
+            m[j] = s + j < a.splits ? y.x : kNegBig;
+            l[j] = s + j < a.splits ? y.y : 0.f;
+            top = fmaxf(top, m[j]);
+        }
+        const float old = __builtin_amdgcn_exp2f(best - top);
+        best = top;
+        den *= old;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) num[i] *= old;
+#pragma unroll
+        for (int j = 0; j < kPipe; ++j) {
+            const float f = s + j < a.splits ? __builtin_amdgcn_exp2f(m[j] - top) : 0.f;
+            den = fmaf(f, l[j], den);
+            num[0] = fmaf(f, x[j].x, num[0]);
+            num[1] = fmaf(f, x[j].y, num[1]);
+            num[2] = fmaf(f, x[j].z, num[2]);
+            num[3] = fmaf(f, x[j].w, num[3]);
+        }
+    }
+    short_store<QT>(reinterpret_cast<QT *>(a.out) + (int64_t)row * p.d + d, num, best, den, ez);
+}
+
+template <typename KV, typename QT> KernelSet with_short(KernelSet k, int d) {
+    if (!k.split) return k;
+    k.few_merge = decode_short_merge_kernel<QT>;
+    if (d == 64) k.few = decode_short_kernel<KV, QT, 64>;
+    if (d == 128) k.few = decode_short_kernel<KV, QT, 128>;
+    if (d == 256) k.few = decode_short_kernel<KV, QT, 256>;
+    if constexpr (sizeof(KV) == 2) {
+        if (d == 32) k.few = decode_short_kernel<KV, QT, 32>;
+    }
+    return k;
+}
+
+}  // namespace pa_decode_detail

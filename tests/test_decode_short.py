@@ -1,0 +1,146 @@
+"""Decode over narrow tables (``decode_short.h``): how a launch is divided (``plan_short_splits`` of ``decode_plan.h``) on the CPU; on the device
+lengths around the edges of tiles, waves and runs against the oracle, for every kind of pool, head size and group that the kernel takes, and the
+two passes as separate calls."""
+
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = """
+#include "decode_plan.h"
+using namespace pa_decode_detail;
+extern "C" int runs(int batch, int hq, int hkv, int d, int bytes, long long blocks, int bs, int window, int cap) {
+    const HeadPlan h = plan_heads(hq, hkv, d, bytes);
+    return plan_short_splits(batch, h, plan_workspace(batch, h, plan_pad_dim(d), cap), bytes, blocks, bs, window, 256);
+}
+extern "C" int fits(int batch, int hq, int hkv, int d, int bytes, int runs, int cap) {  // the runs' results into the workspace's partials
+    const HeadPlan h = plan_heads(hq, hkv, d, bytes);
+    const WsPlan w = plan_workspace(batch, h, plan_pad_dim(d), cap);
+    const size_t rows = (size_t)batch * hq * runs;
+    return w.ml_off + rows * 8 <= w.acc_off && w.acc_off + rows * d * 4 <= w.total;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    at = tmp_path_factory.mktemp("short")
+    (at / "s.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "research_amd", "csrc"), "-o", str(at / "s.so"),
+                    str(at / "s.cpp")], check=True)
+    lib = ctypes.CDLL(str(at / "s.so"))
+    lib.runs.argtypes = [ctypes.c_int] * 5 + [ctypes.c_longlong] + [ctypes.c_int] * 3
+    return lib
+
+
+def test_lines_of_the_rule(plan):
+    runs = lambda batch, shape, keys, bs=16, window=0, cap=4096: plan.runs(batch, *shape, keys // bs, bs, window, cap)
+    wide, many, fp8, one = (32, 8, 128, 2), (14, 2, 64, 2), (32, 8, 128, 1), (8, 8, 64, 2)
+    assert runs(1, wide, 592) == 1 and runs(1, wide, 608) == 4 and runs(1, wide, 4096) == 32 and runs(4, wide, 4096) == 8
+    assert runs(16, wide, 1024) == 3 and runs(32, wide, 608) == 0 and runs(32, wide, 592) == 1 and runs(256, wide, 256) == 1 and runs(256, wide, 272) == 0
+    assert runs(4, wide, 4096 + 16) == 0 and runs(1, wide, 1 << 20) == 0                      # long runs: the split pass
+    assert runs(1, many, 16384) == 64 and runs(256, many, 4096) == 1 and runs(256, many, 4112) == 0
+    assert runs(16, fp8, 2048) == 3 and runs(1, one, 1200) == 1 and runs(96, one, 1216) == 0
+    assert runs(1, wide, 1 << 20, window=500) == 1 and runs(1, wide, 1 << 20, window=-1024) == 8
+    assert runs(4, wide, 64, bs=8) == 0 and runs(4, wide, 96, bs=48) == 1 and runs(513, wide, 16) == 0 and runs(4, wide, 0) == 1
+    assert runs(1, (8, 2, 128, 2), 4096) == 32 and runs(1, (8, 2, 128, 2), 4112) == 0
+
+
+def test_results_of_the_runs_fit_the_workspace(plan):
+    rng = np.random.default_rng(0)
+    for _ in range(20000):
+        hkv, rep = int(rng.choice([1, 2, 3, 4, 8, 16, 40])), int(rng.choice([1, 2, 3, 4, 5, 7, 8, 12, 16, 17, 40]))
+        bytes_ = int(rng.choice([1, 2]))
+        d = int(rng.choice([64, 128, 256] if bytes_ == 1 else [8, 32, 64, 72, 96, 128, 192, 256]))
+        batch, cap = int(rng.integers(1, 513)) if rng.random() < 0.5 else int(rng.integers(1, 9)), int(rng.choice([64, 512, 4096]))
+        n = plan.runs(batch, hkv * rep, hkv, d, bytes_, int(2 ** rng.uniform(0, 14)), 16, 0, cap)
+        assert 0 <= n <= 64 and (n == 0 or plan.fits(batch, hkv * rep, hkv, d, bytes_, n, cap)), (batch, hkv, rep, d, bytes_, cap, n)
+
+
+EDGES = [1, 15, 16, 17, 31, 32, 33, 0, 47, 63, 64, 65, 127, 128, 129, 200, 255, 256, 257]
+CASES = [(EDGES, *shape, kv, window, bs) for shape, kv, window, bs in [
+    ((14, 2, 64), "bf16", 0, 16), ((32, 8, 128), "bf16", 0, 16), ((32, 8, 128), "f16", 50, 16), ((8, 2, 72), "f16", 0, 48), ((4, 4, 32), "bf16", -64, 16),
+    ((20, 1, 96), "bf16", 0, 32), ((36, 2, 128), "f16", 0, 16), ((14, 2, 256), "bf16", 33, 16), ((32, 2, 256), "f16", 0, 16), ((6, 2, 192), "bf16", 0, 16),
+    ((16, 8, 128), "fp8", 0, 16), ((14, 2, 256), "fp8", 17, 16), ((16, 16, 64), "fp8", 0, 32), ((34, 2, 64), "fp8", -48, 16), ((3, 1, 8), "f16", 0, 16),
+]] + [
+    ([1300, 2047, 1, 0, 16], 32, 8, 128, "bf16", 0, 16), ([4000, 129, 128], 14, 2, 64, "bf16", 0, 16), ([3000, 17], 16, 2, 128, "fp8", 0, 16),
+    ([1025, 700, 64, 3], 14, 2, 256, "f16", 0, 16), ([5000, 2, 0], 14, 2, 64, "f16", 1500, 16), ([2500, 1200], 18, 1, 128, "bf16", -1300, 16),
+    ([2000, 900, 1] * 30, 14, 2, 64, "fp8", 0, 16),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,hq,hkv,d,kv,window,bs", CASES)
+def test_against_the_oracle(plan, lens, hq, hkv, d, kv, window, bs):
+    from oracle import paged_oracle as po
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.test_gpu_decode_merge import Batch
+
+    announce(f"decode short: {len(lens)} x {max(lens)} {hq}/{hkv}x{d} {kv} window {window} blocks of {bs}")
+    b = Batch(lens, hq, hkv, d, kv, seed=len(lens) + d, bs=bs)
+    (k, v, ks, vs), (kr, vr) = b.device_pools()
+    tables = tables_to_device(b.tables)
+    assert plan.runs(len(lens), hq, hkv, d, 1 if kv == "fp8" else 2, tables.shape[1], bs, window, 4096) > 0
+    holes = [list(t) for t in b.tables]
+    if not window:  # blocks that are not there count as zero keys: a negative id, one past the pool
+        for t in holes[:3]:
+            if len(t) > 1:
+                t[len(t) // 2] = -1
+        holes[-1][:1] = [b.num_blocks] if holes[-1] else []
+    spare = (set(range(b.num_blocks)) - {x for t in b.tables for x in t}).pop()  # (the oracle's zero keys)
+    kr, vr = kr.float().clone(), vr.float().clone()
+    kr[spare * bs: (spare + 1) * bs] = vr[spare * bs: (spare + 1) * bs] = 0
+    q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
+    for t, ez in ((b.tables, None), (holes, None)) + (() if window else ((b.tables, max(lens) - n),)):
+        ws = ops.decode_workspace(q, k)
+        first = [(x - 1) // -window * -window if window < 0 and x else 0 for x in b.lens]
+        if window < 0 and any(f % bs for f in first):
+            continue  # (the oracle's stand-in for chunks, below, wants whole blocks)
+        call = (k, v, tables_to_device(t), n, bs, b.scale, ws, ez, ks, vs)
+        got = ops.decode(q, *call, window=window)
+        want = po.paged_decode(b.q.float(), kr, vr, [[x if 0 <= x < b.num_blocks else spare for x in r[f // bs:]] for r, f in zip(t, first)],
+                               [x - f for x, f in zip(b.lens, first)], bs, b.scale, pad_zero_keys=ez is not None, window=max(window, 0))
+        # (weights carry 16 or more bits, sums are of 32: what is left is the output's rounding, half a unit of 2^-8 or 2^-11, doubled for sums)
+        assert_close(got, want, 2.0 ** (-10 if kv == "f16" else -7), "one call")
+        for i, x in enumerate(b.lens):
+            assert x or not got[i].any()
+        two = torch.full_like(q, float("nan"))
+        for entry in ("pa_decode_split", "pa_decode_reduce"):
+            ops.decode(q, *call, out=two, entry=entry, window=window)
+        assert_close(two, got.double().cpu().numpy(), 2.0 ** (-10 if kv == "f16" else -7), "two calls")
+        assert torch.equal(ops.decode(q, *call, window=window), got)
+    # an output that starts between two 8-byte words
+    room = torch.full((q.numel() + 1,), 7.0, dtype=q.dtype, device=DEV)
+    out = room[1:].view(q.shape)
+    call = (k, v, tables, n, bs, b.scale, ws, None, ks, vs)
+    assert torch.equal(ops.decode(q, *call, out=out, window=window), ops.decode(q, *call, window=window)) and float(room[0]) == 7.0
+
+
+@pytest.mark.gpu
+def test_rows_that_are_not_seen_do_not_matter():
+    """NaN and infinities in a block's rows past a sequence's end and ahead of its window."""
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce
+
+    announce("decode short: rows out of sight")
+    for dtype, window in ((torch.bfloat16, 0), (torch.float16, 37), (torch.bfloat16, -40)):
+        gen = torch.Generator().manual_seed(5)
+        n = [50, 33, 700, 1]
+        k, v = (torch.randn(1024, 2, 64, generator=gen).to(dtype) for _ in range(2))
+        tables = torch.arange(64, dtype=torch.int32).view(1, 64)[:, :48].repeat(4, 1)
+        for i in range(4):  # every sequence its own call: the same pool, other rows out of sight
+            kk, vv = k.clone(), v.clone()
+            first = max(0, n[i] - window) if window > 0 else (n[i] - 1) // 40 * 40 if window < 0 else 0
+            for t in (kk, vv):
+                t[n[i]:] = float("nan")
+                t[:first] = float("inf")
+            q = torch.randn(1, 14, 64, generator=gen).to(dtype).to(DEV)
+            call = lambda a, b: ops.decode(q, a.to(DEV), b.to(DEV), tables[:1].to(DEV), torch.tensor([n[i]], dtype=torch.int32, device=DEV), 16, 0.125,
+                                           ops.decode_workspace(q, a.to(DEV)), window=window)
+            assert torch.equal(call(kk, vv), call(k, v))
