@@ -472,14 +472,24 @@ __global__ __launch_bounds__(256) void channel_scan_kernel(const ClArgs a) {
     const int64_t stride = 4 * n4 + a.dp + 16;
     float *seg = a.ws + ((int64_t)b * a.heads + h) * a.segments * stride;
     const int segments = (p.n + a.seg_rows - 1) / a.seg_rows;
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 next = segments > 1 ? reinterpret_cast<const float4 *>(seg)[i] : zero, cur = pool ? reinterpret_cast<const float4 *>(pool)[i] : zero;
-    for (int j = 0; j < segments; ++j, seg += stride) {
-        const float4 add = next;
-        if (j + 2 < segments) next = reinterpret_cast<const float4 *>(seg + stride)[i];
-        const float keep = j + 1 < segments ? seg[4 * n4 + d] : 1.f;
-        reinterpret_cast<float4 *>(seg)[i] = cur;
-        cur = make_float4(fmaf(keep, cur.x, add.x), fmaf(keep, cur.y, add.y), fmaf(keep, cur.z, add.z), fmaf(keep, cur.w, add.w));
+    float4 cur = pool ? reinterpret_cast<const float4 *>(pool)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 1
+    for (int first = 0; first < segments; first += kLaScanAhead, seg += kLaScanAhead * stride) {
+        float4 add[kLaScanAhead];  // (the last one leaves nothing)
+        float keep[kLaScanAhead];
+#pragma unroll
+        for (int j = 0; j < kLaScanAhead; ++j)
+            if (first + j + 1 < segments) {
+                add[j] = reinterpret_cast<const float4 *>(seg + j * stride)[i];
+                keep[j] = seg[j * stride + 4 * n4 + d];
+            }
+#pragma unroll
+        for (int j = 0; j < kLaScanAhead; ++j) {
+            if (first + j >= segments) break;
+            reinterpret_cast<float4 *>(seg + j * stride)[i] = cur;
+            if (first + j + 1 < segments)
+                cur = make_float4(fmaf(keep[j], cur.x, add[j].x), fmaf(keep[j], cur.y, add[j].y), fmaf(keep[j], cur.z, add[j].z), fmaf(keep[j], cur.w, add[j].w));
+        }
     }
 }
 

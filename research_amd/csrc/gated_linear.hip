@@ -588,29 +588,37 @@ template <int KIND> __global__ __launch_bounds__(256) void gated_scan_kernel(con
     const int64_t stride = 4 * n4 + a.dp + 16;
     float *seg = a.ws + ((int64_t)b * a.heads + h) * a.segments * stride;
     const int segments = (p.n + a.seg_rows - 1) / a.seg_rows;
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 next = segments > 1 ? reinterpret_cast<const float4 *>(seg)[i] : zero, cur = pool ? reinterpret_cast<const float4 *>(pool)[i] : zero;
+    float4 cur = pool ? reinterpret_cast<const float4 *>(pool)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     float m = KIND == kMlstm && pool ? pool[4 * n4 + a.dp] : 0.f;
-    for (int j = 0; j < segments; ++j, seg += stride) {
-        const float4 add = next;
-        if (j + 2 < segments) next = reinterpret_cast<const float4 *>(seg + stride)[i];
-        float keep = 1.f, take = 1.f, m_next = 0.f;
-        if (j + 1 < segments) {
-            const float decay = seg[4 * n4 + a.dp + 1];
-            if (KIND == kMlstm) {
-                const float m_seg = seg[4 * n4 + a.dp];
-                m_next = fmaxf(decay + m, m_seg);
-                keep = exp2f(decay + m - m_next);
-                take = exp2f(m_seg - m_next);
-            } else {
-                keep = exp2f(decay);
+#pragma unroll 1
+    for (int first = 0; first < segments; first += kLaScanAhead, seg += kLaScanAhead * stride) {
+        float4 add[kLaScanAhead];  // (the last one leaves nothing)
+        float decay[kLaScanAhead], top[kLaScanAhead];
+#pragma unroll
+        for (int j = 0; j < kLaScanAhead; ++j)
+            if (first + j + 1 < segments) {
+                add[j] = reinterpret_cast<const float4 *>(seg + j * stride)[i];
+                decay[j] = seg[j * stride + 4 * n4 + a.dp + 1];
+                if (KIND == kMlstm) top[j] = seg[j * stride + 4 * n4 + a.dp];
             }
+#pragma unroll
+        for (int j = 0; j < kLaScanAhead; ++j) {
+            if (first + j >= segments) break;
+            reinterpret_cast<float4 *>(seg + j * stride)[i] = cur;
+            if (KIND == kMlstm && i == n4) seg[j * stride + 4 * n4 + a.dp + 2] = m;
+            if (first + j + 1 >= segments) break;
+            float keep, take = 1.f;
+            if (KIND == kMlstm) {
+                const float m_next = fmaxf(decay[j] + m, top[j]);
+                keep = exp2f(decay[j] + m - m_next);
+                take = exp2f(top[j] - m_next);
+                m = m_next;
+            } else {
+                keep = exp2f(decay[j]);
+            }
+            cur = make_float4(fmaf(keep, cur.x, take * add[j].x), fmaf(keep, cur.y, take * add[j].y), fmaf(keep, cur.z, take * add[j].z),
+                              fmaf(keep, cur.w, take * add[j].w));
         }
-        reinterpret_cast<float4 *>(seg)[i] = cur;
-        if (KIND == kMlstm && i == n4) seg[4 * n4 + a.dp + 2] = m;
-        cur = make_float4(fmaf(keep, cur.x, take * add.x), fmaf(keep, cur.y, take * add.y), fmaf(keep, cur.z, take * add.z),
-                          fmaf(keep, cur.w, take * add.w));
-        m = m_next;
     }
 }
 

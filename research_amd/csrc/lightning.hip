@@ -343,7 +343,7 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
         }
 }
 
-// Segment contributions -> start states, in place.  A chain of one load per segment, so the next one is in flight.
+// Segment contributions -> start states, in place.  The loads of kLaScanAhead segments are in flight at once.
 __global__ __launch_bounds__(256) void lightning_scan_kernel(const LaArgs a) {
     const int h = blockIdx.y, b = blockIdx.z;
     Portion p;
@@ -353,15 +353,22 @@ __global__ __launch_bounds__(256) void lightning_scan_kernel(const LaArgs a) {
     const float4 *pool = p.slot >= 0 && p.pos0 > 0 ? reinterpret_cast<const float4 *>(a.state) + (p.slot * a.heads + h) * n4 + i : nullptr;
     float4 *seg = reinterpret_cast<float4 *>(a.ws) + ((int64_t)b * a.heads + h) * a.segments * n4 + i;
     const int segments = (p.n + a.seg_rows - 1) / a.seg_rows;
-    float4 next = segments > 1 ? *seg : make_float4(0.f, 0.f, 0.f, 0.f);
     float4 cur = pool ? *pool : make_float4(0.f, 0.f, 0.f, 0.f);
     float f = 1.f;  // decay^seg_rows, seg_rows a multiple of the chunk
     for (int c = 0; c < a.seg_rows / kLaChunk; ++c) f *= a.decay[h * (kLaChunk + 1) + kLaChunk];
-    for (int j = 0; j < segments; ++j) {
-        const float4 add = next;
-        if (j + 2 < segments) next = seg[(j + 1) * n4];
-        seg[j * n4] = cur;
-        cur = make_float4(fmaf(f, cur.x, add.x), fmaf(f, cur.y, add.y), fmaf(f, cur.z, add.z), fmaf(f, cur.w, add.w));
+#pragma unroll 1
+    for (int first = 0; first < segments; first += kLaScanAhead) {
+        float4 add[kLaScanAhead];  // (the last one leaves nothing)
+#pragma unroll
+        for (int j = 0; j < kLaScanAhead; ++j)
+            if (first + j + 1 < segments) add[j] = seg[(first + j) * n4];
+#pragma unroll
+        for (int j = 0; j < kLaScanAhead; ++j) {
+            if (first + j >= segments) break;
+            seg[(first + j) * n4] = cur;
+            if (first + j + 1 < segments)
+                cur = make_float4(fmaf(f, cur.x, add[j].x), fmaf(f, cur.y, add[j].y), fmaf(f, cur.z, add[j].z), fmaf(f, cur.w, add[j].w));
+        }
     }
 }
 

@@ -11,8 +11,10 @@
 #endif
 
 constexpr int kLaChunk = 64;      // rows multiplied at once
-constexpr int kLaMinSegChunks = 8;  // a segment is at least this many chunks long
+constexpr int kLaMinSegChunks = 8;    // a segment is at least this many chunks long ...
 constexpr int kLaMaxSegments = 64;
+constexpr int kLaLeastSegChunks = 2;  // ... or, of few sequences, this many
+constexpr int kLaScanAhead = 8;       // segments whose states the scan between the passes loads at once
 
 static inline int la_pad16(int n) { return (n + 15) / 16 * 16; }
 
@@ -24,11 +26,11 @@ static inline int64_t la_per_sequence(int heads, int vdim) { return heads * (int
 // Segments of a portion of up to max_len rows: as many as (sequences x heads x value slices) leave compute units for,
 // one workgroup each, but no shorter than kLaMinSegChunks chunks (a segment's start state costs a second reading of
 // its keys and values and two passes over a state's bytes).
-static inline int la_segments(int64_t workgroups, int cus, int max_len) {
+static inline int la_segments(int64_t workgroups, int cus, int max_len, int least = kLaMinSegChunks) {
     if (workgroups <= 0 || max_len <= 0) return 1;
     const int64_t chunks = (max_len + kLaChunk - 1) / kLaChunk;
     int64_t want = cus / workgroups;
-    const int64_t most = chunks / kLaMinSegChunks;
+    const int64_t most = chunks / least;
     if (want > most) want = most;
     if (want > kLaMaxSegments) want = kLaMaxSegments;
     return want < 1 ? 1 : (int)want;
@@ -39,9 +41,13 @@ static inline int la_segments(int64_t workgroups, int cus, int max_len) {
 // segments the launch lasts as long as its longest sequence or, with more workgroups than compute units, its share of the
 // rows; with segments of c chunks it lasts c where a compute unit has one of them at most (of unequal portions' last segments, which
 // are short and start last, half may follow another, up to an eighth of the units), c `together` where some have two, else its share
-// and a third of a segment, and 45 % more for the first pass, half a unit per segment for the scan between the two, and two units for the
-// launches.  Over 182 batches (1 to 30 prompts of 100 .. 12000 rows, 2 to 64 heads, all four recurrences) this is 3.1 % off the best number
-// on average; with 0.85 segments a unit for a guess, half a segment and 1.6 c up to 1.3 of them a unit, 4.3 %.
+// and a third of a segment (which of one sequence, in equal segments, has to promise 5 % more), and 45 % more for the first pass, a fifth of a unit per segment for the scan between
+// the two, and three units for the launches.  Segments shorter than kLaMinSegChunks only where a compute unit has one at most: what each begins
+// and ends with counts (16 heads of 128 x 128, SSD, 5 prompts of 1611 .. 2178 rows, 96 us in three, 108 in eight).
+// Before, no segment was shorter than eight chunks, and a segment of the scan half a unit: us, that -> this, one sequence: lightning, 8 heads of
+// 128 x 128, 1500 rows 90 -> 35, 12000 98 -> 70; HGRN2, 8 heads of 128 x 128, 2500 rows 117 -> 57; mLSTM, 4 heads of 256 x 512, 700 rows 101 -> 57;
+// SSD, 64 heads of 128 x 64, 1500 rows 85 -> 48.  Over 250 batches (1 to 40 prompts of 200 .. 16000 rows, 1 to 64 heads, four recurrences)
+// 1.06 to 1.27 times as fast on average, none slower by more than 2 %.
 static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, int most) {
     if (batch <= 0 || per_seq <= 0 || max_len <= 0) return 1;
     if (n_rows > batch * max_len) n_rows = batch * max_len;
@@ -54,9 +60,11 @@ static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, 
         const double c = (chunks + s - 1) / s;
         const double spread = rows / c + 0.5 * batch, all = (double)batch * s, live = per_seq * (spread < all ? spread : all);
         double part = c;
-        if (live > cus + (spread < all ? spare : 0.0)) part = live <= 2.0 * cus && together > 0 ? c * together : share + 0.35 * c;
+        const bool more = live > cus + (spread < all ? spare : 0.0);
+        if (more && s > chunks / kLaMinSegChunks) continue;  // (short ones, several a unit: what each begins and ends with counts)
+        if (more) part = live <= 2.0 * cus && together > 0 ? c * together : share + 0.35 * c;
         if (part < c) part = c;
-        const double t = 1.45 * part + 0.5 * s + 2.0;
+        const double t = (1.45 * part + 0.2 * s + 3.0) * (more && batch == 1 ? 1.05 : 1.0);
         if (t < best) {
             best = t;
             segments = s;
@@ -64,10 +72,12 @@ static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, 
     }
     return segments;
 }
-// Most segments: none shorter than kLaMinSegChunks chunks, and states of seg_bytes for each (of all sequences) that fit `room`.
+// Chunks of a segment at least: fewer where the sequences in one piece leave compute units without a workgroup.
+static inline int la_least_chunks(int64_t batch, int64_t per_seq, int cus) { return batch * per_seq < cus ? kLaLeastSegChunks : kLaMinSegChunks; }
+// Most segments: none shorter than `least` chunks, and states of seg_bytes for each (of all sequences) that fit `room`.
 constexpr size_t kLaMostSegBytes = (size_t)256 << 20;
-static inline int la_most_segments(size_t seg_bytes, int max_len, size_t room = kLaMostSegBytes) {
-    const int most = la_segments(1, kLaMaxSegments, max_len);
+static inline int la_most_segments(size_t seg_bytes, int max_len, size_t room = kLaMostSegBytes, int least = kLaMinSegChunks) {
+    const int most = la_segments(1, kLaMaxSegments, max_len, least);
     if (room > kLaMostSegBytes) room = kLaMostSegBytes;
     const int64_t fit = seg_bytes ? (int64_t)(room / seg_bytes) : most;
     return fit < 1 ? 1 : fit < most ? (int)fit : most;
@@ -75,7 +85,7 @@ static inline int la_most_segments(size_t seg_bytes, int max_len, size_t room = 
 // Segments whose states a launch of n_rows rows has a use for (< 0: the rows are not known yet; the most of any): 1 where the batch stays
 // in one piece, such as equal portions that fill the device.
 static inline int la_asked_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, size_t seg_bytes) {
-    const int most = la_most_segments(seg_bytes, max_len);
+    const int most = la_most_segments(seg_bytes, max_len, kLaMostSegBytes, la_least_chunks(batch, per_seq, cus));
     if (n_rows >= 0) return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
     int asked = 1;
     for (int i = 0; i <= 32; ++i) {  // from one long portion to equal ones
@@ -88,8 +98,8 @@ static inline int la_asked_segments(int64_t batch, int64_t per_seq, int cus, dou
 // batch that fills the device without segments takes such a workspace for none.  shared: workgroups that a compute unit has at once.
 static inline int la_launch_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows,
                                      size_t seg_bytes, size_t room, bool aligned, int shared = 1) {
-    const int most = la_most_segments(seg_bytes, max_len, room);
-    if (!aligned) return most > 1 && la_segments(batch * per_seq, shared * cus, max_len) > 1 ? 0 : 1;
+    const int most = la_most_segments(seg_bytes, max_len, room, la_least_chunks(batch, per_seq, cus));
+    if (!aligned) return la_most_segments(seg_bytes, max_len, room) > 1 && la_segments(batch * per_seq, shared * cus, max_len) > 1 ? 0 : 1;
     return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
 }
 

@@ -76,6 +76,62 @@ def test_a_batch_in_one_piece_asks_for_no_workspace(kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,heads,dim,vdim", [("lightning", 8, 128, 128), ("lightning", 4, 64, 64), ("mlstm", 4, 256, 512), ("mlstm", 4, 64, 128),
+                                                 ("ssd", 16, 128, 64), ("ssd", 2, 64, 128), ("channel", 8, 128, 128), ("channel", 3, 96, 80)])
+@pytest.mark.parametrize("lens", [[257], [128, 700, 1, 65], [1500], [6000, 130], [0, 640, 513]])
+def test_few_prompts_in_short_segments(kind, heads, dim, vdim, lens):
+    """A workgroup for each of more segments than a prompt has eights of chunks, the scan over more of them than it loads at once: as in one piece."""
+    import torch
+
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce
+
+    announce(f"short segments {kind} {heads}x{dim}x{vdim} {lens}")
+    gen, batch, before = torch.Generator().manual_seed(dim + len(lens)), len(lens), 70
+    parts = {"lightning": (heads * dim, heads * dim, heads * vdim), "channel": (heads * dim, heads * dim, heads * vdim)}.get(
+        kind, (heads * dim, heads * dim, heads * vdim, 2 * heads))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    pad = lambda x: -(-x // 16) * 16
+    need = {"lightning": ops.lightning_workspace_bytes, "channel": ops.channel_linear_workspace_bytes}.get(kind, ops.gated_linear_workspace_bytes)
+    room = need(batch, heads, dim, vdim, max(lens), rows=sum(lens))
+    if max(lens) >= 1500:
+        assert room >= 8 * heads * pad(dim) * pad(vdim) * 4
+    shape = (batch, heads, ops.gated_linear_state_floats(kind, dim, vdim)) if kind in ("ssd", "mlstm") else (batch, heads, pad(dim), pad(vdim))
+    constant = lambda a, b, m=heads: (a + (b - a) * torch.rand(m, generator=gen)).to(DEV)
+    decay = torch.tensor([1.0 - 0.5 ** (3 + i) for i in range(heads)], dtype=torch.float64)
+    powers = (decay[:, None] ** torch.arange(65, dtype=torch.float64)).float().to(DEV)
+    gates = (constant(-5, -3), constant(1, 16), constant(-1, 1)) if kind == "ssd" else (constant(-1, 1), constant(3, 6), None)
+    f_bias, lower = constant(1, 4, heads * dim), constant(0, 0.9, heads * dim)
+
+    def run(u, behind, new, state, ws):
+        p = ops.Portions(i32([behind + x for x in new]), i32(list(range(batch))), i32(new), i32([sum(new[:i]) for i in range(batch)]), None, max(new))
+        out = torch.full((sum(new), heads * vdim), float("nan"), dtype=torch.bfloat16, device=DEV)
+        q, k, v = u.split(parts, 1)[:3]
+        if kind == "lightning":
+            ops.lightning(u, p, state, powers, heads, dim, vdim, out, workspace=ws)
+        elif kind == "channel":
+            ops.channel_linear(q, k, v, f_bias, lower, p, state, heads, dim, vdim, out, q_act="silu", workspace=ws)
+        else:
+            a, b = u[:, -2 * heads: -heads], u[:, -heads:]
+            ops.gated_linear(kind, q, k, v, (a, None if kind == "ssd" else b), gates, p, state, heads, dim, vdim, out, cap=15.0, q_scale=dim ** -0.5,
+                             den_eps=1e-6, workspace=ws)
+        return out
+
+    rows = lambda m: torch.randn(m, sum(parts), generator=gen).to(torch.bfloat16).to(DEV)
+    first = torch.zeros(shape, device=DEV)
+    run(rows(before * batch), 0, [before] * batch, first, None)
+    u, results = rows(sum(lens)), []
+    for ws in (None, torch.full((max(room, 16),), 0x7f, dtype=torch.uint8, device=DEV)):
+        state = first.clone()
+        results.append((run(u, before, lens, state, ws).double(), state.double()))
+    (out, state), (want, want_state) = results[1], results[0]
+    assert torch.isfinite(out).all() and torch.isfinite(state).all()
+    # (both round an output of 32-bit sums to 16 bits: 2^-9 of it each; states carry two 16-bit terms of every factor, 2^-16, over sums of many)
+    assert float((out - want).norm() / want.norm()) < 2.0 ** -8
+    assert float((state - want_state).norm() / want_state.norm()) < 1e-4
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,dim,vdim,longest", [(32, 64, 64, 2500), (32, 64, 128, 2500), (16, 128, 128, 2500), (16, 128, 128, 8000)])
 def test_a_batch_of_unequal_prompts_in_segments(heads, dim, vdim, longest):
     import torch
