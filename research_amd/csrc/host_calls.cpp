@@ -71,6 +71,11 @@ bool take(PyObject *x, float &to) {
     return true;
 }
 
+struct Unlocked {  // other Python threads run meanwhile (also while an exception leaves the library)
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 template <int I, typename F> struct Call;
 template <int I, typename R, typename... A> struct Call<I, R (*)(A...)> {
     template <size_t... N> static bool take_all(PyObject *const *args, std::tuple<A...> &to, std::index_sequence<N...>) {
@@ -88,10 +93,10 @@ template <int I, typename R, typename... A> struct Call<I, R (*)(A...)> {
         }
         std::tuple<A...> values;
         if (!take_all(args, values, std::index_sequence_for<A...>{})) return nullptr;
-        R result;
-        Py_BEGIN_ALLOW_THREADS
-        result = std::apply(reinterpret_cast<R (*)(A...)>(bound[I]), values);
-        Py_END_ALLOW_THREADS
+        const R result = [&] {
+            Unlocked unlocked;
+            return std::apply(reinterpret_cast<R (*)(A...)>(bound[I]), values);
+        }();
         if constexpr (std::is_signed_v<R>) return PyLong_FromLongLong((long long)result);
         else return PyLong_FromUnsignedLongLong((unsigned long long)result);
         END_HANDLE_TH_ERRORS
