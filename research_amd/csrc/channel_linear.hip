@@ -143,11 +143,12 @@ constexpr float kClSmall = 0x1p-100f;  // a block whose P falls below has its sc
 template <int KD, int NW, bool STATES> struct ClTile {
     static constexpr int rows = KD == 256 ? 32 : 64, blocks = rows / kClBlock, cols = 16 * NW, threads = 64 * NW;
     static constexpr int pitch = KD + 8, vPitch = cols + kLaPadV;
-    static constexpr int elems = rows * pitch;                       // one bf16 term of a tile
+    static constexpr int pitchK = KD + 16;  // (R K is read by transposing reads alone: rows 32 modulo 64 bytes apart)
+    static constexpr int elems = rows * pitch, elemsK = rows * pitchK;  // one bf16 term of a tile
     static constexpr int units = KD / 2 * rows / 8;                  // (channel pair, 8 rows)
     static constexpr int passes = (units + threads - 1) / threads;
     static constexpr int vLoads = rows * cols / 4 / threads;         // four columns each
-    static constexpr size_t bytes = (size_t)elems * (STATES ? 2 : 6) * 2 + (size_t)rows * vPitch * 2 + (size_t)blocks * KD * 4 +
+    static constexpr size_t bytes = (size_t)elemsK * 2 * 2 + (STATES ? 0 : (size_t)elems * 4 * 2) + (size_t)rows * vPitch * 2 + (size_t)blocks * KD * 4 +
                                     (STATES ? 0 : (size_t)blocks * 64 * 16) + 64;
 };
 
@@ -189,7 +190,7 @@ template <int KD> __device__ __noinline__ f4 cl_slow_scores(const uint16_t *uq, 
 // part of S split again.  So 1 / P is made once per block instead of by row (P R = B), a last chunk's missing rows are masked in that chunk
 // alone, and the blocks of a chunk are unrolled, with the state's update and the outputs of one block as independent chains between them
 // (outputs of the next block ahead of the barrier behind the scores were slower: they wait for the update).  8 prompts of 700 .. 4000 rows,
-// 32 heads of 128 x 128, both passes: 463 -> 409 us.
+// 32 heads of 128 x 128, both passes: 463 -> 409 us, and 401 with R K at a pitch that its reads spread over the banks.
 // STATES: only the segment's own contribution to the state and its factors, to the workspace (first pass over a portion in
 // segments).
 template <int KD, int NW, bool STATES>
@@ -197,8 +198,8 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     using L = ClTile<KD, NW, STATES>;
     constexpr int kRows = L::rows, kPitch = L::pitch, kThr = L::threads, kPairs = KD / 2;
     extern __shared__ __align__(16) char lds[];
-    __bf16 *k_hi = reinterpret_cast<__bf16 *>(lds), *k_lo = k_hi + L::elems;         // R K
-    __bf16 *q_hi = k_lo + L::elems, *q_lo = q_hi + L::elems;                         // P Q
+    __bf16 *k_hi = reinterpret_cast<__bf16 *>(lds), *k_lo = k_hi + L::elemsK;        // R K
+    __bf16 *q_hi = k_lo + L::elemsK, *q_lo = q_hi + L::elems;                         // P Q
     __bf16 *i_hi = q_lo + L::elems, *i_lo = i_hi + L::elems;                         // K / P
     __bf16 *v_s = STATES ? q_hi : i_lo + L::elems;
     float *whole = reinterpret_cast<float *>(v_s + kRows * L::vPitch);               // B per block
@@ -327,19 +328,20 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 const bool any = __ballot(bad) != 0;
                 if (lane == 0) unsafe[wave + NW * u] = any;
             }
-            uint32_t *dst = reinterpret_cast<uint32_t *>(k_hi) + (8 * oct[u] * kPitch) / 2 + pair[u];
-            constexpr int kRow = kPitch / 2, kTerm = L::elems / 2;
+            uint32_t *dst_k = reinterpret_cast<uint32_t *>(k_hi) + (8 * oct[u] * L::pitchK) / 2 + pair[u];
+            uint32_t *dst = reinterpret_cast<uint32_t *>(q_hi) + (8 * oct[u] * kPitch) / 2 + pair[u];
+            constexpr int kRow = kPitch / 2, kTerm = L::elems / 2, kRowK = L::pitchK / 2, kTermK = L::elemsK / 2;
 #pragma unroll
             for (int r = 7; r >= 0; --r) {  // R K, and, as P R = B in every row, K / P = K / B R (in this order nothing small is lost)
                 const float x = k[r][0] * back[0], y = k[r][1] * back[1];
                 uint32_t hi, lo;
                 la_split2(x, y, hi, lo);
-                dst[r * kRow] = hi;
-                dst[kTerm + r * kRow] = lo;
+                dst_k[r * kRowK] = hi;
+                dst_k[kTermK + r * kRowK] = lo;
                 if constexpr (!STATES) {
                     la_split2(k[r][0] * open[0] * back[0], k[r][1] * open[1] * back[1], hi, lo);
-                    dst[4 * kTerm + r * kRow] = hi;
-                    dst[5 * kTerm + r * kRow] = lo;
+                    dst[2 * kTerm + r * kRow] = hi;
+                    dst[3 * kTerm + r * kRow] = lo;
                 }
                 back[0] *= f[r][0];
                 back[1] *= f[r][1];
@@ -358,8 +360,8 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                     }
                     uint32_t hi, lo;
                     la_split2(q[0], q[1], hi, lo);
-                    dst[2 * kTerm + r * kRow] = hi;
-                    dst[3 * kTerm + r * kRow] = lo;
+                    dst[r * kRow] = hi;
+                    dst[kTerm + r * kRow] = lo;
                 }
             }
         }
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 __builtin_amdgcn_raw_buffer_store_b64(x, dst, c < vcols ? (uint32_t)(l16 * ldo + c) * 2u : kLaOutside, 0, 0);
             }
             const float *keep = whole + blk * KD + 4 * g;
-            const __bf16 *kh = k_hi + (first + 4 * g + (l16 >> 2)) * kPitch + 4 * (l16 & 3), *kl = kh + L::elems;
+            const __bf16 *kh = k_hi + (first + 4 * g + (l16 >> 2)) * L::pitchK + 4 * (l16 & 3), *kl = kh + L::elemsK;
 #pragma unroll
             for (int dt = 0; dt < KD / 16; ++dt) {
                 const f4 f = *reinterpret_cast<const f4 *>(keep + 16 * dt);
