@@ -14,7 +14,9 @@ constexpr int kLaChunk = 64;      // rows multiplied at once
 constexpr int kLaMinSegChunks = 8;    // a segment is at least this many chunks long ...
 constexpr int kLaMaxSegments = 64;
 constexpr int kLaLeastSegChunks = 2;  // ... or, of few sequences, this many
-constexpr int kLaScanAhead = 8;       // segments whose states the scan between the passes loads at once
+// Segments whose states the scan between the passes loads at once (8 prompts in five segments, 16 heads of 128 x 128, all passes: 2 137.4 us, 4
+// 137.9, 8 139.0; one of 12000 rows in 32, 8 heads: 70.5, 69.5, 69.0).
+constexpr int kLaScanAhead = 4;
 
 static inline int la_pad16(int n) { return (n + 15) / 16 * 16; }
 
@@ -45,8 +47,9 @@ static inline int la_segments(int64_t workgroups, int cus, int max_len, int leas
 // the two, and three units for the launches.  Segments shorter than kLaMinSegChunks only where a compute unit has one at most: what each begins
 // and ends with counts (16 heads of 128 x 128, SSD, 5 prompts of 1611 .. 2178 rows, 96 us in three, 108 in eight).
 // Before, no segment was shorter than eight chunks, and a segment of the scan half a unit: us, that -> this, one sequence: lightning, 8 heads of
-// 128 x 128, 1500 rows 90 -> 35, 12000 98 -> 70; HGRN2, 8 heads of 128 x 128, 2500 rows 117 -> 57; mLSTM, 4 heads of 256 x 512, 700 rows 101 -> 57;
-// SSD, 64 heads of 128 x 64, 1500 rows 85 -> 48.  Over 250 batches (1 to 40 prompts of 200 .. 16000 rows, 1 to 64 heads, four recurrences)
+// 128 x 128, 4000 rows 74 -> 42, 12000 84 -> 70; HGRN2, 8 heads of 128 x 128, 2500 rows 114 -> 50; mLSTM, 4 heads of 256 x 512, 700 rows 101 -> 56;
+// of 64 x 128, 12000 81 -> 61; SSD, 64 heads of 128 x 64, 1500 rows 65 -> 55.  Over 250 batches (1 to 40 prompts of 200 .. 16000 rows, 1 to 64 heads,
+// four recurrences)
 // 1.06 to 1.27 times as fast on average, none slower by more than 2 %.
 static inline int la_balanced_segments(int64_t batch, int64_t per_seq, int cus, double together, int max_len, int64_t n_rows, int most) {
     if (batch <= 0 || per_seq <= 0 || max_len <= 0) return 1;
