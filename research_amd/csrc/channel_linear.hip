@@ -321,7 +321,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 ahead[e] = second ? other : 1.f;
                 back[e] = second ? 1.f : other;
                 if (second) whole[(oct[u] >> 1) * KD + 2 * pair[u] + e] = all;
-                bad = bad || all < kClSmall;
+                bad = bad || !(all >= kClSmall);  // (also NaN, which by way of `open` would reach the K / P of rows before its own)
                 open[e] = __builtin_amdgcn_rcpf(all);
             }
             if constexpr (!STATES) {  // (the wave's channels of one block; kPairs / 32 waves share it)

@@ -363,6 +363,30 @@ def test_channel_gates_that_write_little_ahead_of_forgetting(heads, dim, vdim):
     assert float(err.max()) < 2.0 ** -8, err  # (the outputs' rounding to 16 bits, at most 2^-9 of each)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (2, 128, 128), (2, 256, 80), (3, 40, 72)])
+@pytest.mark.parametrize("at", [5, 15, 37, 64, 71])
+def test_a_channel_gate_that_is_not_a_number_leaves_earlier_rows_alone(heads, dim, vdim, at):
+    """A forget logit of row `at` and one head: rows before it, also of its own block of 16, and other heads are what they are without it."""
+    announce(f"channels nan {heads} {dim} {vdim} {at}")
+    n, gen = 80, torch.Generator().manual_seed(dim)
+    u = torch.randn(n, heads * (2 * dim + vdim), generator=gen).to(BF)
+    pad = lambda x: -(-x // 16) * 16
+
+    def run(u):
+        state = torch.zeros(1, heads, pad(dim), pad(vdim), device=DEV)
+        out = torch.full((n, heads * vdim), 9.0, dtype=BF, device=DEV)
+        q, z, v = u.to(DEV).split([heads * dim, heads * dim, heads * vdim], 1)
+        ops.channel_linear(q, z, v, None, torch.zeros(heads * dim, device=DEV), _portions([(0, 0, n)], [0], tiles=False), state, heads, dim, vdim, out, q_act="silu")
+        return out.cpu().view(n, heads, vdim)
+
+    clean = run(u)
+    u[at, heads * dim + dim // 2] = float("nan")  # a channel of head 0
+    got = run(u)
+    assert torch.equal(got[:, 1:], clean[:, 1:]) and bool(got[at:, 0].isnan().all())
+    assert torch.equal(got[: at // 16 * 16, 0], clean[: at // 16 * 16, 0])
+    assert_close(got[:at, 0], clean[:at, 0], 2.0 ** -7)  # (the block's scores come about in another order: both round to 2^-9)
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 64), (1, 128, 128), (1, 256, 80), (2, 96, 200)])
 def test_long_portions_run_in_segments(heads, dim, vdim):
     announce(f"channels segments {heads} {dim} {vdim}")
