@@ -9,6 +9,8 @@
 //     O^T += V^T P^T   S's layout is P's as an operand; V goes through the wave's own part of LDS, read transposed
 // P is a sum of two 16-bit terms: with one, short sequences came out less exact than the split pass, whose every row of lanes has a weight of
 // one (error against 64 bits, 14 / 2 heads of 64, 8 sequences of 94 .. 683 keys: split pass 1.78e-3, one term 2.06e-3, two 1.67e-3).
+// Over fp8 pools a weight meets its block's scale, and the terms are of bf16 whatever the queries are: fp16 has no room for small scales (fp16
+// queries, those sequences, terms of fp16 -> bf16: 2.071e-4 -> 2.069e-4, with values of 0.001 instead of one 1.0e-2 -> 2.4e-4).
 // Waves take tiles of 16 keys in turn, two at a time up to 64 elements a row; their sums meet in LDS with two barriers.  One tile at a time at
 // 128 leaves registers for four workgroups a compute unit: 256 sequences of 16 keys, 32 / 8 heads, 16.1 -> 9.0 us.
 #pragma once
@@ -69,8 +71,10 @@ template <typename QT, typename Num> __device__ __forceinline__ void short_store
 // keys for the merge.
 template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void decode_short_kernel(const DecodeArgs a) {
     using M = ShortMfma<QT>;
-    using f4 = typename M::f4;
     constexpr bool kFp8 = sizeof(KV) == 1;
+    using VT = std::conditional_t<kFp8, pa_bf16, QT>;  // the second product's type (fp8 values are exact in either)
+    using W = ShortMfma<VT>;
+    using f4 = typename M::f4;
     constexpr int EL = 16 / sizeof(KV), KL = D / (4 * EL);  // elements of a 16-byte load; loads of a tile of K, and of V
     constexpr int NT = D >= 128 ? 1 : 2;                    // tiles at a time (registers for four waves a SIMD, at 256 two)
     constexpr int kPitch = D + 16;                          // (four rows of a transposing read lie 32 bytes apart modulo 64)
@@ -190,7 +194,7 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                     pa_u4 *to = reinterpret_cast<pa_u4 *>(vs + row * kPitch + d);
                     if constexpr (kFp8) {
                         uint32_t w[8];
-                        PoolWords<KV, QT>::unpack(vr[t][j], w);
+                        PoolWords<KV, VT>::unpack(vr[t][j], w);
                         to[0] = pa_u4{w[0], w[1], w[2], w[3]};
                         to[1] = pa_u4{w[4], w[5], w[6], w[7]};
                     } else {
@@ -221,12 +225,9 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    pw[2 * t + i] = M::pack(e[2 * i], e[2 * i + 1]);
-                    const float2 high = M::unpack(pw[2 * t + i]);
-                    float2 rest = make_float2(e[2 * i] - high.x, e[2 * i + 1] - high.y);
-                    if constexpr (kFp8 && std::is_same<QT, pa_f16>::value)  // (a scale beyond the type: the first term alone)
-                        rest = make_float2(rest.x == -INFINITY ? 0.f : rest.x, rest.y == -INFINITY ? 0.f : rest.y);
-                    pl[2 * t + i] = M::pack(rest.x, rest.y);
+                    pw[2 * t + i] = W::pack(e[2 * i], e[2 * i + 1]);
+                    const float2 high = W::unpack(pw[2 * t + i]);
+                    pl[2 * t + i] = W::pack(e[2 * i] - high.x, e[2 * i + 1] - high.y);
                 }
             }
             const pa_u4 pb{pw[0], pw[1], pw[2], pw[3]}, pc{pl[0], pl[1], pl[2], pl[3]};
@@ -243,8 +244,8 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
                 const pa_u4 v{v0.x, v0.y, v1.x, v1.y};
-                acc[dt] = M::mul(v, pb, acc[dt]);
-                acc[dt] = M::mul(v, pc, acc[dt]);
+                acc[dt] = W::mul(v, pb, acc[dt]);
+                acc[dt] = W::mul(v, pc, acc[dt]);
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();

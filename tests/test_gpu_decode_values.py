@@ -1,0 +1,79 @@
+"""Decode on values at the edges of the 16-bit types, on each way that a launch can take: a workgroup per sequence and runs with a merge
+behind them (``decode_short.h``), and the split pass (``decode_impl.h``), which block tables far wider than the sequences lead to."""
+
+import numpy as np
+import pytest
+import torch
+
+from research_amd import ops
+from tests.gpu_helpers import DEV, announce
+
+pytestmark = pytest.mark.gpu
+
+BS = 16
+WIDE = 1 << 16  # blocks of a table: no kernel for short sequences takes it
+
+
+def _tables(lens, width=None):
+    """Consecutive blocks; how many there are."""
+    per = [-(-n // BS) for n in lens]
+    out = np.full((len(lens), width or max(per)), -1, dtype=np.int32)
+    at = 0
+    for row, n in zip(out, per):
+        row[:n] = np.arange(at, at + n)
+        at += n
+    return torch.from_numpy(out).to(DEV), at
+
+
+def _attend(q, k, v, lens, scale):
+    """64-bit outputs and what the weights' sizes let them err by: the sums of |weight * value|."""
+    q, k, v = q.double(), k.double(), v.double()
+    hq, hkv = q.shape[1], k.shape[1]
+    out, size, at = [], [], 0
+    for b, n in enumerate(lens):
+        kk, vv = (t[at * BS: at * BS + n].repeat_interleave(hq // hkv, 1) for t in (k, v))
+        w = torch.softmax(torch.einsum("hd,nhd->hn", q[b], kk) * scale, 1)
+        out.append(torch.einsum("hn,nhd->hd", w, vv))
+        size.append(torch.einsum("hn,nhd->hd", w, vv.abs()))
+        at += -(-n // BS)
+    return torch.stack(out), torch.stack(size)
+
+
+WAYS = [("whole", [300, 33], None), ("runs", [1500, 40], None)]
+SHAPES = [(14, 2, 64), (8, 2, 128), (32, 8, 128), (6, 2, 256), (3, 3, 64)]
+
+
+@pytest.mark.parametrize("what", ["small", "tiny", "large", "mixed", "zeros", "dominant"])
+@pytest.mark.parametrize("hq,hkv,d", SHAPES)
+@pytest.mark.parametrize("way,lens,width", WAYS)
+def test_fp8_pools_whose_values_are_far_from_one(way, lens, width, hq, hkv, d, what):
+    """The weights of an fp8 pool meet its scales, which fp16 has no room for: values of 0.001, of 2000, of both, blocks of zeros (whose
+    scale is one) beside small ones, and a key whose weight is nearly one and whose values are zero."""
+    announce(f"decode values fp8 f16 {way} {hq}/{hkv}x{d} {what}")
+    gen = torch.Generator().manual_seed(d + hq)
+    tables, blocks = _tables(lens, width)
+    k, v = (torch.randn(blocks * BS, hkv, d, generator=gen) for _ in range(2))
+    q = torch.randn(len(lens), 1, d, generator=gen) + 0.1 * torch.randn(len(lens), hq, d, generator=gen)
+    size = {"small": 0.03, "tiny": 1e-3, "large": 2000.0, "mixed": 1.0, "zeros": 1e-3, "dominant": 0.03}[what]
+    v *= size
+    if what == "mixed":
+        v *= 10.0 ** (torch.arange(blocks) % 7 - 3.0).repeat_interleave(BS)[:, None, None]
+    if what == "zeros":
+        v[torch.arange(blocks).repeat_interleave(BS) % 3 == 1] = 0
+    if what == "dominant":
+        at = 0
+        for b, n in enumerate(lens):
+            k[at * BS + n // 2] = 11.0 * d ** 0.5 * q[b].mean(0) / (q[b].mean(0) ** 2).sum()
+            v[at * BS + n // 2] = 0
+            at += -(-n // BS)
+    q = q.to(torch.float16)
+    kb, ks = ops.quantize_kv_e4m3(k.to(torch.float16).to(DEV), BS)
+    vb, vs = ops.quantize_kv_e4m3(v.to(torch.bfloat16).to(DEV), BS)
+    every = lambda x, s: x.cpu().double() * s.cpu().double().repeat_interleave(BS, 0)[:, :, None]
+    want, size = _attend(q, every(kb, ks), every(vb, vs), lens, d ** -0.5)
+    qd = q.to(DEV)
+    got = ops.decode(qd, kb, vb, tables, torch.tensor(lens, dtype=torch.int32, device=DEV), BS, d ** -0.5, ops.decode_workspace(qd, kb), k_scale=ks, v_scale=vs)
+    err = (got.cpu().double() - want).abs()
+    # (outputs are rounded to 11 bits, or to a multiple of 2^-24, weights to 11 bits at least)
+    room = 2.0 ** -11 * want.abs() + 2.0 ** -25 + 2.0 ** -11 * size
+    assert bool((err <= room).all()), (float((err / room).max()), float(err.norm() / want.norm()))
