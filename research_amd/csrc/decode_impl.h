@@ -325,6 +325,7 @@ template <typename KV, typename QT, int D, int NREP, int U> struct Attender {
                 attend_blocks_pk<KV, QT, D, NREP, U, false>(st, qpk, p, bt_row, k_lo, L, blk_first, blk_end, wave,
                                                             n_waves, (p.bs + p.tpw * U - 1) / (p.tpw * U), by_chunk,
                                                             lane, lane_voff, kvh, role.tok_local == 0);
+            if (pk_units<KV, QT>) st.to_ones();
             StaticFor<NREP>::run([&](auto h) {
                 out.m[h.value] = HS::template bcast<h.value>(st.m);
                 out.l[h.value] = HS::template bcast<h.value>(st.l);

@@ -2,7 +2,8 @@
 // pools (head_dim 64, 128, 256) and fp8-e4m3 pools with bf16 / fp16 queries
 // (head_dim 64, 128, 256).  An fp8 pool is widened two elements at a time to
 // the query type (v_cvt_scalef32_pk_*_fp8, exact) and then runs the same
-// 16-bit arithmetic; its per-(block, head) scales multiply the logit and p.
+// 16-bit arithmetic; its per-(block, head) scales multiply the logit and p (in
+// fp16 counted in units, PkState::in_units).
 //
 // The generic loop converts every K/V element to fp32 and spends most of its
 // issue slots on conversions, per-head cross-lane sums and redundant softmax
@@ -220,6 +221,7 @@ template <int NREP, int VPL, int EPL> struct PkState {
     float m[VPL], l[VPL];
     float acc[NREP][EPL];
     int zero_keys;
+    int unit;  // acc counts in 2^unit (other than 0 for fp8 pools with fp16 arithmetic alone)
     __device__ __forceinline__ void init() {
 #pragma unroll
         for (int j = 0; j < VPL; ++j) { m[j] = -1.0e30f; l[j] = 0.f; }
@@ -228,8 +230,38 @@ template <int NREP, int VPL, int EPL> struct PkState {
 #pragma unroll
             for (int e = 0; e < EPL; ++e) acc[r][e] = 0.f;
         zero_keys = 0;
+        unit = 0;
+    }
+    // What a weight is multiplied by for a block whose V scale is v_sc: the scale in units that keep it within a factor of 32 of one, since the
+    // product is rounded to fp16, whose smallest numbers lie at 2^-24.  A block outside of that brings its own unit, and what was summed is
+    // counted in it (uniform: pools of like values do so once).  Scales below 2^-40 give outputs that fp16 does not have.
+    // (fp16 queries, with the scale itself -> this, 16 sequences of 900 .. 9000 keys: error against 64 bits with values of 0.001, 14 / 2 heads of
+    // 64, 4.5e-3 -> 6.7e-4, 32 / 8 of 128 7.3e-3 -> 6.4e-4, half of it the outputs' own rounding; us 87 -> 76, 51.5 -> 50.6, 16 / 16 of 64 33.1 -> 33.9,
+    // 14 / 2 of 256 84.2 -> 86.4, and 64 of 90 .. 3000 keys, 16 / 8 of 128, 47.7 -> 49.4)
+    __device__ __forceinline__ float in_units(float v_sc) {
+        float f = __builtin_amdgcn_ldexpf(v_sc, -unit);
+        const bool far = fabsf(f) > 32.f || (fabsf(f) < 0x1p-5f && v_sc != 0.f);
+        if (__builtin_amdgcn_ballot_w64(far) != 0) {
+            const int to = far ? max(__builtin_amdgcn_frexp_expf(v_sc), -40) : unit;
+#pragma unroll
+            for (int r = 0; r < NREP; ++r)
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) acc[r][e] = __builtin_amdgcn_ldexpf(acc[r][e], unit - to);
+            unit = to;
+            f = __builtin_amdgcn_ldexpf(v_sc, -unit);
+        }
+        return f;
+    }
+    __device__ __forceinline__ void to_ones() {
+#pragma unroll
+        for (int r = 0; r < NREP; ++r)
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[r][e] = __builtin_amdgcn_ldexpf(acc[r][e], unit);
+        unit = 0;
     }
 };
+
+template <typename KV, typename AT> constexpr bool pk_units = sizeof(KV) == 1 && std::is_same<AT, pa_f16>::value;
 
 template <int N> struct StaticFor {
     template <typename F> static __device__ __forceinline__ void run(F &&f) {
@@ -266,7 +298,7 @@ __device__ __forceinline__ void attend_blocks_pk(
     bool count_zero_keys) {
     static_assert(U % 2 == 0, "tokens are consumed in pairs");
     constexpr int LPR = D * (int)sizeof(KV) / 16;
-    constexpr bool kFp8 = sizeof(KV) == 1;
+    constexpr bool kFp8 = sizeof(KV) == 1, kUnits = pk_units<KV, AT>;
     using HS = HeadScatter<NREP, LPR>;
     using PK = Pk16<AT>;
     using PW = PoolWords<KV, AT>;
@@ -391,6 +423,7 @@ __device__ __forceinline__ void attend_blocks_pk(
                 });
             }
             // ---- p.v, two tokens per step ----------------------------------
+            const float v_by = kUnits ? st.in_units(v_sc) : v_sc;  // (here, so that no load above waits for the scale's)
 #pragma unroll
             for (int u = 0; u < U; u += 2) {
                 if (SHORT && u * p.tpw >= rem) continue;  // uniform: both token steps lie past the block
@@ -400,7 +433,7 @@ __device__ __forceinline__ void attend_blocks_pk(
                     const float p0 = __builtin_amdgcn_exp2f(sv[u][j] - st.m[j]);  // 0 for masked tokens
                     const float p1 = __builtin_amdgcn_exp2f(sv[u + 1][j] - st.m[j]);
                     st.l[j] += p0 + p1;
-                    ppk[j] = kFp8 ? PK::pack(p0 * v_sc, p1 * v_sc) : PK::pack(p0, p1);
+                    ppk[j] = kFp8 ? PK::pack(p0 * v_by, p1 * v_by) : PK::pack(p0, p1);
                 }
                 uint32_t lo[NW], hi[NW];  // (v_t0[2i], v_t1[2i]) and (v_t0[2i+1], v_t1[2i+1])
                 PW::interleave(vraw[u], vraw[u + 1], lo, hi);
@@ -430,7 +463,7 @@ __device__ __forceinline__ void attend_blocks_pk_multi(
     static_assert(U % SPB == 0 && SPB % 2 == 0, "whole blocks per iteration, token pairs inside one block");
     constexpr int G = U / SPB;  // blocks per iteration
     constexpr int LPR = D * (int)sizeof(KV) / 16;
-    constexpr bool kFp8 = sizeof(KV) == 1;
+    constexpr bool kFp8 = sizeof(KV) == 1, kUnits = pk_units<KV, AT>;
     using HS = HeadScatter<NREP, LPR>;
     using PK = Pk16<AT>;
     using PW = PoolWords<KV, AT>;
@@ -540,6 +573,7 @@ __device__ __forceinline__ void attend_blocks_pk_multi(
         for (int u = 0; u < U; u += 2) {
             const int g = u / SPB;
             if (partial && (u % SPB) * p.tpw >= ntok[g]) continue;  // uniform: both steps lie past the block's end
+            if (kUnits && u % SPB == 0) v_sc[g] = st.in_units(v_sc[g]);
             uint32_t ppk[VPL];
 #pragma unroll
             for (int j = 0; j < VPL; ++j) {

@@ -39,7 +39,7 @@ def _attend(q, k, v, lens, scale):
     return torch.stack(out), torch.stack(size)
 
 
-WAYS = [("whole", [300, 33], None), ("runs", [1500, 40], None)]
+WAYS = [("whole", [300, 33], None), ("runs", [1500, 40], None), ("split", [300, 33], WIDE), ("split", [1500, 40], WIDE)]
 SHAPES = [(14, 2, 64), (8, 2, 128), (32, 8, 128), (6, 2, 256), (3, 3, 64)]
 
 
