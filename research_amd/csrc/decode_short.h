@@ -124,132 +124,146 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
     const int tok = p.hkv * p.d * (int)sizeof(KV), head = kvh * p.d * (int)sizeof(KV);  // bytes between tokens, before the head
     uint16_t *vs = reinterpret_cast<uint16_t *>(room) + wave * NT * kShortKeys * kPitch;
 
-    float m = kNegBig, l = 0.f;
+    float m, l;
     f4 acc[D / 16];  // O^T: d = 16 dt + 4 g + i, head l16
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) acc[dt] = f4{0.f, 0.f, 0.f, 0.f};
     pa_u4 kr[NT][KL], vr[NT][KL];
     float kscale = 1.f, vscale = 1.f;  // of tile `lane` of the 64 at hand
+    // An infinite value times a weight's second term, which is zero or negative as often as not, makes a sum NaN that is infinite.  So a wave whose
+    // sums are not all finite goes over its keys once more with the first terms alone, as the split pass has them: twice, and halved behind the loop.
+    // (us: 8 sequences of 94 .. 683 keys, 32 / 8 heads of 128, 9.6 -> 9.9, 14 / 2 of 64 7.4 -> 7.4, of 256 11.6 -> 12.0)
+    bool again = false;
 #pragma unroll 1
-    for (int first = 0; first < n_tiles; first += 64) {
-        const int n = min(64, n_tiles - first), tile0 = t0 + first;
-        if (first > 0 || !known) bids = table(tile0);
-        if constexpr (kFp8) {
-            const int64_t at = bids >= 0 ? (int64_t)bids * p.hkv + kvh : 0;
-            kscale = bids >= 0 ? p.k_scale[at] : 1.f;
-            vscale = bids >= 0 ? p.v_scale[at] : 1.f;
-        }
-        auto fetch = [&](int at) {
+    for (;; again = true) {
+        m = kNegBig;
+        l = 0.f;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const int tile = tile0 + at + t, bid = at + t < n ? __builtin_amdgcn_readlane(bids, at + t) : -1;
-                const int rows = bid >= 0 ? min(kShortKeys, L - tile * kShortKeys) : 0;  // (rows past them read as zeros)
-                const int skip = k_lo - tile * kShortKeys;                               // rows before the window: zeros of V
-                const int64_t slot = ((int64_t)max(bid, 0) * p.bs + tile % tiles_per_block * kShortKeys) * tok;
-                const int bytes = rows > 0 ? (rows - 1) * tok + head + p.d * (int)sizeof(KV) : 0;
-                const __amdgpu_buffer_rsrc_t k = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.k) + slot), 0, bytes, 0x00020000);
-                const __amdgpu_buffer_rsrc_t v = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.v) + slot), 0, bytes, 0x00020000);
-#pragma unroll
-                for (int j = 0; j < KL; ++j) {
-                    const int d = EL * (4 * j + g);
-                    kr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(k, d < p.d ? l16 * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
-                }
-#pragma unroll
-                for (int j = 0; j < KL; ++j) {
-                    const int c = lane + 64 * j, row = c / (D / EL), d = c % (D / EL) * EL;
-                    vr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(v, d < p.d && row >= skip ? row * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
-                }
+        for (int dt = 0; dt < D / 16; ++dt) acc[dt] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int first = 0; first < n_tiles; first += 64) {
+            const int n = min(64, n_tiles - first), tile0 = t0 + first;
+            if (first > 0 || !known || again) bids = table(tile0);
+            if constexpr (kFp8) {
+                const int64_t at = bids >= 0 ? (int64_t)bids * p.hkv + kvh : 0;
+                kscale = bids >= 0 ? p.k_scale[at] : 1.f;
+                vscale = bids >= 0 ? p.v_scale[at] : 1.f;
             }
-        };
-        if (wave * NT < n) fetch(wave * NT);
-#pragma unroll 1
-        for (int at = wave * NT; at < n; at += kWaves * NT) {
-            float x[NT][4], mx = m;
+            auto fetch = [&](int at) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                f4 s = f4{0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < NT; ++t) {
+                    const int tile = tile0 + at + t, bid = at + t < n ? __builtin_amdgcn_readlane(bids, at + t) : -1;
+                    const int rows = bid >= 0 ? min(kShortKeys, L - tile * kShortKeys) : 0;  // (rows past them read as zeros)
+                    const int skip = k_lo - tile * kShortKeys;                               // rows before the window: zeros of V
+                    const int64_t slot = ((int64_t)max(bid, 0) * p.bs + tile % tiles_per_block * kShortKeys) * tok;
+                    const int bytes = rows > 0 ? (rows - 1) * tok + head + p.d * (int)sizeof(KV) : 0;
+                    const __amdgpu_buffer_rsrc_t k = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.k) + slot), 0, bytes, 0x00020000);
+                    const __amdgpu_buffer_rsrc_t v = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.v) + slot), 0, bytes, 0x00020000);
 #pragma unroll
-                for (int j = 0; j < KL; ++j) {
-                    if constexpr (kFp8) {
-                        uint32_t w[8];
-                        PoolWords<KV, QT>::unpack(kr[t][j], w);
-                        s = M::mul(pa_u4{w[0], w[1], w[2], w[3]}, qr[j][0], s);
-                        s = M::mul(pa_u4{w[4], w[5], w[6], w[7]}, qr[j][1], s);
-                    } else {
-                        s = M::mul(kr[t][j], qr[j][0], s);
+                    for (int j = 0; j < KL; ++j) {
+                        const int d = EL * (4 * j + g);
+                        kr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(k, d < p.d ? l16 * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
+                    }
+#pragma unroll
+                    for (int j = 0; j < KL; ++j) {
+                        const int c = lane + 64 * j, row = c / (D / EL), d = c % (D / EL) * EL;
+                        vr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(v, d < p.d && row >= skip ? row * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
                     }
                 }
-                const int lim = at + t < n ? L - (tile0 + at + t) * kShortKeys : 0, lo = k_lo - (tile0 + at + t) * kShortKeys;
-                float f = p.scale_log2;
-                if constexpr (kFp8) f *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, kscale), (at + t) & 63));
+            };
+            if (wave * NT < n) fetch(wave * NT);
+#pragma unroll 1
+            for (int at = wave * NT; at < n; at += kWaves * NT) {
+                float x[NT][4], mx = m;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    x[t][i] = 4 * g + i < lim && 4 * g + i >= lo ? s[i] * f : -INFINITY;
-                    mx = fmaxf(mx, x[t][i]);
-                }
-                // V, for the transposing reads
+                for (int t = 0; t < NT; ++t) {
+                    f4 s = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int j = 0; j < KL; ++j) {
-                    const int c = lane + 64 * j, row = t * kShortKeys + c / (D / EL), d = c % (D / EL) * EL;
-                    pa_u4 *to = reinterpret_cast<pa_u4 *>(vs + row * kPitch + d);
-                    if constexpr (kFp8) {
-                        uint32_t w[8];
-                        PoolWords<KV, VT>::unpack(vr[t][j], w);
-                        to[0] = pa_u4{w[0], w[1], w[2], w[3]};
-                        to[1] = pa_u4{w[4], w[5], w[6], w[7]};
-                    } else {
-                        to[0] = vr[t][j];
+                    for (int j = 0; j < KL; ++j) {
+                        if constexpr (kFp8) {
+                            uint32_t w[8];
+                            PoolWords<KV, QT>::unpack(kr[t][j], w);
+                            s = M::mul(pa_u4{w[0], w[1], w[2], w[3]}, qr[j][0], s);
+                            s = M::mul(pa_u4{w[4], w[5], w[6], w[7]}, qr[j][1], s);
+                        } else {
+                            s = M::mul(kr[t][j], qr[j][0], s);
+                        }
+                    }
+                    const int lim = at + t < n ? L - (tile0 + at + t) * kShortKeys : 0, lo = k_lo - (tile0 + at + t) * kShortKeys;
+                    float f = p.scale_log2;
+                    if constexpr (kFp8) f *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, kscale), (at + t) & 63));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        x[t][i] = 4 * g + i < lim && 4 * g + i >= lo ? s[i] * f : -INFINITY;
+                        mx = fmaxf(mx, x[t][i]);
+                    }
+                    // V, for the transposing reads
+#pragma unroll
+                    for (int j = 0; j < KL; ++j) {
+                        const int c = lane + 64 * j, row = t * kShortKeys + c / (D / EL), d = c % (D / EL) * EL;
+                        pa_u4 *to = reinterpret_cast<pa_u4 *>(vs + row * kPitch + d);
+                        if constexpr (kFp8) {
+                            uint32_t w[8];
+                            PoolWords<KV, VT>::unpack(vr[t][j], w);
+                            to[0] = pa_u4{w[0], w[1], w[2], w[3]};
+                            to[1] = pa_u4{w[4], w[5], w[6], w[7]};
+                        } else {
+                            to[0] = vr[t][j];
+                        }
                     }
                 }
-            }
-            if (at + kWaves * NT < n) fetch(at + kWaves * NT);
-            {
-                const float2 y = lane_pair<16>(mx, 16);
-                mx = fmaxf(y.x, y.y);
-                const float2 z = lane_pair<32>(mx, 32);
-                mx = fmaxf(z.x, z.y);
-            }
-            const float alpha = __builtin_amdgcn_exp2f(m - mx);
-            m = mx;
-            l *= alpha;
-            uint32_t pw[4] = {0, 0, 0, 0}, pl[4] = {0, 0, 0, 0};  // the weights as a sum of two terms
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                float e[4], f = 1.f;
-                if constexpr (kFp8) f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vscale), (at + t) & 63));
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    e[i] = __builtin_amdgcn_exp2f(x[t][i] - m);  // 0 for masked keys
-                    l += e[i];
-                    if constexpr (kFp8) e[i] *= f;
+                if (at + kWaves * NT < n) fetch(at + kWaves * NT);
+                {
+                    const float2 y = lane_pair<16>(mx, 16);
+                    mx = fmaxf(y.x, y.y);
+                    const float2 z = lane_pair<32>(mx, 32);
+                    mx = fmaxf(z.x, z.y);
                 }
+                const float alpha = __builtin_amdgcn_exp2f(m - mx);
+                m = mx;
+                l *= alpha;
+                uint32_t pw[4] = {0, 0, 0, 0}, pl[4] = {0, 0, 0, 0};  // the weights as a sum of two terms
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    pw[2 * t + i] = W::pack(e[2 * i], e[2 * i + 1]);
-                    const float2 high = W::unpack(pw[2 * t + i]);
-                    pl[2 * t + i] = W::pack(e[2 * i] - high.x, e[2 * i + 1] - high.y);
+                for (int t = 0; t < NT; ++t) {
+                    float e[4], f = 1.f;
+                    if constexpr (kFp8) f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vscale), (at + t) & 63));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        e[i] = __builtin_amdgcn_exp2f(x[t][i] - m);  // 0 for masked keys
+                        l += e[i];
+                        if constexpr (kFp8) e[i] *= f;
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        pw[2 * t + i] = W::pack(e[2 * i], e[2 * i + 1]);
+                        const float2 high = W::unpack(pw[2 * t + i]);
+                        pl[2 * t + i] = W::pack(e[2 * i] - high.x, e[2 * i + 1] - high.y);
+                    }
                 }
-            }
-            const pa_u4 pb{pw[0], pw[1], pw[2], pw[3]}, pc{pl[0], pl[1], pl[2], pl[3]};
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+                const pa_u4 pb{pw[0], pw[1], pw[2], pw[3]}, pc = again ? pb : pa_u4{pl[0], pl[1], pl[2], pl[3]};
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int dt = 0; dt < D / 16; ++dt) {
-                typedef short s4 __attribute__((ext_vector_type(4)));
-                auto column = [&](int t) {
-                    uint16_t *from = vs + (t * kShortKeys + 4 * g + l16 / 4) * kPitch + 16 * dt + 4 * (l16 % 4);
-                    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *)from));
-                };
-                const uint2 v0 = column(0), v1 = NT == 2 ? column(1) : make_uint2(0, 0);
+                for (int dt = 0; dt < D / 16; ++dt) {
+                    typedef short s4 __attribute__((ext_vector_type(4)));
+                    auto column = [&](int t) {
+                        uint16_t *from = vs + (t * kShortKeys + 4 * g + l16 / 4) * kPitch + 16 * dt + 4 * (l16 % 4);
+                        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *)from));
+                    };
+                    const uint2 v0 = column(0), v1 = NT == 2 ? column(1) : make_uint2(0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
-                const pa_u4 v{v0.x, v0.y, v1.x, v1.y};
-                acc[dt] = W::mul(v, pb, acc[dt]);
-                acc[dt] = W::mul(v, pc, acc[dt]);
+                    for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
+                    const pa_u4 v{v0.x, v0.y, v1.x, v1.y};
+                    acc[dt] = W::mul(v, pb, acc[dt]);
+                    acc[dt] = W::mul(v, pc, acc[dt]);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
         }
+        if constexpr (kFp8) break;  // (that type has no infinities)
+        f4 odd = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) odd += acc[dt] * 0.f;
+        if (again || __builtin_amdgcn_ballot_w64(!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f)) == 0) break;
     }
     {
         const float2 y = lane_pair<16>(l, 16);
@@ -265,7 +279,7 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
     float top = kNegBig;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) top = fmaxf(top, s_m[w][l16]);
-    const float mine = __builtin_amdgcn_exp2f(m - top);
+    const float mine = __builtin_amdgcn_exp2f(m - top) * (again ? 0.5f : 1.f);
     float *part = reinterpret_cast<float *>(room);  // (every wave is through with V)
 #pragma unroll
     for (int h0 = 0; h0 < kShortHeads; h0 += HR) {
@@ -331,7 +345,8 @@ template <typename QT> __global__ __launch_bounds__(kThreads) void decode_short_
         for (int i = 0; i < 4; ++i) num[i] *= old;
 #pragma unroll
         for (int j = 0; j < kPipe; ++j) {
-            const float f = s + j < a.splits ? __builtin_amdgcn_exp2f(m[j] - top) : 0.f;
+            const float f = __builtin_amdgcn_exp2f(m[j] - top);
+            if (s + j >= a.splits) break;  // (uniform; zero times an infinite sum is none)
             den = fmaf(f, l[j], den);
             num[0] = fmaf(f, x[j].x, num[0]);
             num[1] = fmaf(f, x[j].y, num[1]);

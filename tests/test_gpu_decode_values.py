@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from research_amd import ops
-from tests.gpu_helpers import DEV, announce
+from tests.gpu_helpers import DEV, announce, assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +77,32 @@ def test_fp8_pools_whose_values_are_far_from_one(way, lens, width, hq, hkv, d, w
     # (outputs are rounded to 11 bits, or to a multiple of 2^-24, weights to 11 bits at least)
     room = 2.0 ** -11 * want.abs() + 2.0 ** -25 + 2.0 ** -11 * size
     assert bool((err <= room).all()), (float((err / room).max()), float(err.norm() / want.norm()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", SHAPES + [(4, 4, 32)])
+@pytest.mark.parametrize("way,lens,width", WAYS)
+def test_infinities_among_the_values(way, lens, width, hq, hkv, d, dtype):
+    """An infinite value of a key in sight is an infinite output of its column, not NaN; columns without one are what they are without it."""
+    announce(f"decode values inf {way} {hq}/{hkv}x{d} {dtype}")
+    gen = torch.Generator().manual_seed(d)
+    tables, blocks = _tables(lens, width)
+    k, v = (torch.randn(blocks * BS, hkv, d, generator=gen) for _ in range(2))
+    q = (0.5 * torch.randn(len(lens), hq, d, generator=gen)).to(dtype).to(DEV)  # (no weight so small that it is zero in 16 bits)
+    n = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    bad = v.clone()
+    up, down, both, nan = [0, 3], [5], [d - 1], [7]  # columns
+    for at in (2, lens[0] // 2, lens[0] - 1):
+        bad[at, :, up] = float("inf")
+    bad[lens[0] - 2, :, down] = -float("inf")
+    bad[1, :, both], bad[lens[0] - 1, :, both] = float("inf"), -float("inf")
+    bad[4, :, nan] = float("nan")
+    kd = k.to(dtype).to(DEV)
+    call = lambda x: ops.decode(q, kd, x.to(dtype).to(DEV), tables, n, BS, d ** -0.5, ops.decode_workspace(q, kd)).cpu()
+    clean, got = call(v), call(bad)
+    assert torch.equal(got[1], clean[1])
+    assert bool((got[0][:, up] == float("inf")).all()) and bool((got[0][:, down] == -float("inf")).all())
+    assert bool(got[0][:, both + nan].isnan().all())
+    rest = [c for c in range(d) if c not in up + down + both + nan]
+    # (both round to 2^-9 or 2^-12, and the weights of one do)
+    assert_close(got[0][:, rest], clean[0][:, rest], {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype])
