@@ -196,6 +196,8 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 
 // How decode_short.h's kernel takes the launch: 0: not at all; else the runs a sequence's tiles are cut into, a workgroup per (kv head, sequence,
 // run).  From shapes alone; the tables' width stands for the longest sequence.
+// Head sizes up to 32 stay with the generic loop of the split pass, whose weights have 32 bits: 11.1 us for 16 sequences of 16 .. 250 keys, 4 / 4
+// heads of 32, where weights of two bf16 terms took 5.0, but erred by up to 1.1e-6 of the sum of |weight value| where 32 bits err by 0.2e-6.
 // Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (3.5 us: 600 keys of 128).
 // us, the split pass (one launch or two) -> this, sequences of n keys each: 32 / 8 heads of 128, 1 of 256 keys 14.1 -> 7.4, 1024 15.5 -> 9.0, 4096
 // 16.2 -> 12.0; 32 of 256 19.6 -> 8.3; 96 of 256 33.9 -> 19.7; 14 / 2 of 64, 1 of 256 15.2 -> 5.8, 4096 16.4 -> 11.0; 32 of 1024 22.1 -> 11.0, 16384
@@ -208,7 +210,7 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // (Over 1400 batches of 1 .. 384 sequences and thirteen shapes none was slower by more than the runs of one side differ, 3 %.)
 constexpr int kPlanShortHeads = 16, kPlanShortTile = 16, kPlanShortRuns = 64;
 PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, int kv_elem_bytes, int64_t table_blocks, int block_size, int window, int cus) {
-    if (block_size % kPlanShortTile != 0 || batch > kPlanWaveScanBatch || h.hkv > 65535) return 0;
+    if (block_size % kPlanShortTile != 0 || batch > kPlanWaveScanBatch || h.hkv > 65535 || h.d_pad < 64) return 0;
     const int64_t span = plan_window_span(window);
     if (span > 0 && span / block_size + 2 < table_blocks) table_blocks = span / block_size + 2;
     const int64_t keys = table_blocks * block_size, reps = (h.n_rep + kPlanShortHeads - 1) / kPlanShortHeads, wgs = (int64_t)h.hkv * batch * reps;

@@ -1,4 +1,4 @@
-// Decode over narrow block tables (16-bit queries over 16-bit or fp8 pools): a workgroup per (kv head, sequence), or several with a merge behind
+// Decode over narrow block tables (16-bit queries over 16-bit or fp8 pools, heads of more than 32): a workgroup per (kv head, sequence), or several with a merge behind
 // them (plan_short_splits of decode_plan.h: where, how many, and what they measured).
 //
 // Short sequences are bound by waits and by the instructions that a workgroup fetches once, not by bytes: the split pass, whose loop is unrolled
@@ -363,9 +363,6 @@ template <typename KV, typename QT> KernelSet with_short(KernelSet k, int d) {
     if (d == 64) k.few = decode_short_kernel<KV, QT, 64>;
     if (d == 128) k.few = decode_short_kernel<KV, QT, 128>;
     if (d == 256) k.few = decode_short_kernel<KV, QT, 256>;
-    if constexpr (sizeof(KV) == 2) {
-        if (d == 32) k.few = decode_short_kernel<KV, QT, 32>;
-    }
     return k;
 }
 

@@ -48,6 +48,7 @@ def test_lines_of_the_rule(plan):
     assert runs(16, fp8, 2048) == 3 and runs(1, one, 1200) == 1 and runs(96, one, 1216) == 0
     assert runs(1, wide, 1 << 20, window=500) == 1 and runs(1, wide, 1 << 20, window=-1024) == 8
     assert runs(4, wide, 64, bs=8) == 0 and runs(4, wide, 96, bs=48) == 1 and runs(513, wide, 16) == 0 and runs(4, wide, 0) == 1
+    assert runs(4, (8, 2, 32, 2), 64) == runs(4, (3, 1, 8, 2), 64) == 0 and runs(4, (8, 2, 40, 2), 64) == 1  # (weights of 32 bits)
     assert runs(1, (8, 2, 128, 2), 4096) == 32 and runs(1, (8, 2, 128, 2), 4112) == 0
 
 
@@ -64,9 +65,9 @@ def test_results_of_the_runs_fit_the_workspace(plan):
 
 EDGES = [1, 15, 16, 17, 31, 32, 33, 0, 47, 63, 64, 65, 127, 128, 129, 200, 255, 256, 257]
 CASES = [(EDGES, *shape, kv, window, bs) for shape, kv, window, bs in [
-    ((14, 2, 64), "bf16", 0, 16), ((32, 8, 128), "bf16", 0, 16), ((32, 8, 128), "f16", 50, 16), ((8, 2, 72), "f16", 0, 48), ((4, 4, 32), "bf16", -64, 16),
+    ((14, 2, 64), "bf16", 0, 16), ((32, 8, 128), "bf16", 0, 16), ((32, 8, 128), "f16", 50, 16), ((8, 2, 72), "f16", 0, 48), ((4, 4, 40), "bf16", -64, 16),
     ((20, 1, 96), "bf16", 0, 32), ((36, 2, 128), "f16", 0, 16), ((14, 2, 256), "bf16", 33, 16), ((32, 2, 256), "f16", 0, 16), ((6, 2, 192), "bf16", 0, 16),
-    ((16, 8, 128), "fp8", 0, 16), ((14, 2, 256), "fp8", 17, 16), ((16, 16, 64), "fp8", 0, 32), ((34, 2, 64), "fp8", -48, 16), ((3, 1, 8), "f16", 0, 16),
+    ((16, 8, 128), "fp8", 0, 16), ((14, 2, 256), "fp8", 17, 16), ((16, 16, 64), "fp8", 0, 32), ((34, 2, 64), "fp8", -48, 16), ((3, 1, 40), "f16", 0, 16),
 ]] + [
     ([1300, 2047, 1, 0, 16], 32, 8, 128, "bf16", 0, 16), ([4000, 129, 128], 14, 2, 64, "bf16", 0, 16), ([3000, 17], 16, 2, 128, "fp8", 0, 16),
     ([1025, 700, 64, 3], 14, 2, 256, "f16", 0, 16), ([5000, 2, 0], 14, 2, 64, "f16", 1500, 16), ([2500, 1200], 18, 1, 128, "bf16", -1300, 16),

@@ -106,3 +106,26 @@ def test_infinities_among_the_values(way, lens, width, hq, hkv, d, dtype):
     rest = [c for c in range(d) if c not in up + down + both + nan]
     # (both round to 2^-9 or 2^-12, and the weights of one do)
     assert_close(got[0][:, rest], clean[0][:, rest], {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 4, 32), (3, 1, 8), (8, 2, 24)])
+def test_weights_of_head_sizes_up_to_32_have_32_bits(hq, hkv, d, dtype):
+    """Large values whose weighted sum is nearly zero: what is left are the weights' own errors."""
+    announce(f"decode values cancel {hq}/{hkv}x{d} {dtype}")
+    gen, n = torch.Generator().manual_seed(d), 33
+    tables, blocks = _tables([n])
+    k, v = (torch.randn(blocks * BS, hkv, d, generator=gen).to(dtype) for _ in range(2))
+    q = torch.randn(1, hkv, d, generator=gen).to(dtype).repeat_interleave(hq // hkv, 1)  # (the heads of a group are alike: one sum to cancel)
+    w = torch.softmax(torch.einsum("hd,nhd->hn", q[0, :: hq // hkv].double(), k[:n].double()) * d ** -0.5, 1)
+    v *= 1000
+    for at in (n - 1, n - 2):  # two keys take what the others leave, the second the rest of the first's rounding
+        others = torch.einsum("hn,nhd->hd", w, v[:n].double()) - w[:, at, None] * v[at].double()
+        v[at] = (-others / w[:, at, None]).to(dtype)
+    want, size = _attend(q, k, v, [n], d ** -0.5)
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    got = ops.decode(qd, kd, vd, tables, torch.tensor([n], dtype=torch.int32, device=DEV), BS, d ** -0.5, ops.decode_workspace(qd, kd)).cpu().double()
+    err = (got - want).abs()
+    # (the outputs' own rounding, and of the sums what one weight can err by: a logit of up to 8 in base 2 by half a unit of 2^-21, its exponential by 2^-23)
+    room = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype] * want.abs() + 2.0 ** -21 * size
+    assert bool((err <= room).all()), (float((err / room).max()), float((err / size).max()))
