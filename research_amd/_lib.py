@@ -9,6 +9,7 @@ call fails with that error.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from typing import Optional
@@ -178,6 +179,7 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
         fn = getattr(lib, name)  # AttributeError names the missing symbol
         fn.restype, fn.argtypes = restype, argtypes
     if path is None:
+        importlib.invalidate_caches()  # (it may have been built since the package's folder was last looked at)
         try:
             from . import _host
         except ImportError as e:

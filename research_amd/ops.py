@@ -22,20 +22,37 @@ PA_DTYPE = {torch.float32: _lib.PA_F32, torch.bfloat16: _lib.PA_BF16, torch.floa
 QKV_TILE_ROWS = _lib.PA_QKV_TILE_ROWS
 
 
-try:
-    from . import _host
-    from ._host import dense as _dense, nbytes as _nbytes, row_stride as _row_stride, shaped as _shaped, stream as _stream, typed as _typed
-except ImportError:  # not built: loading the library says so
-    def _dense(*_):
-        _lib.load()
+_host = None
 
-    _nbytes = _row_stride = _shaped = _stream = _typed = _dense
+
+def _bind() -> None:
+    global _host, _dense, _nbytes, _row_stride, _shaped, _stream, _typed
+    from . import _host as host
+    _dense, _nbytes, _row_stride, _shaped, _stream, _typed = host.dense, host.nbytes, host.row_stride, host.shaped, host.stream, host.typed
+    _host = host
+
+
+def _late(name: str):
+    def call(*args):
+        _lib.load()  # (says what is missing)
+        _bind()
+        return getattr(_host, name)(*args)
+
+    return call
+
+
+_dense, _nbytes, _row_stride, _shaped, _stream, _typed = map(_late, ("dense", "nbytes", "row_stride", "shaped", "stream", "typed"))
+try:
+    _bind()
+except ImportError:  # not built yet: the first call takes what has been built by then
+    pass
 
 
 def _run(name: str, *args) -> None:
     """Call the library's function: tensors and None as its pointers."""
-    if _lib._lib is None:
+    if _lib._lib is None or _host is None:
         _lib.load()
+        _bind()
     status = getattr(_host, name)(*args)
     if status:
         _lib.check(name, status)

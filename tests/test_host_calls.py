@@ -2,14 +2,49 @@
 library's functions take, and what is refused."""
 
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
 
+from research_amd import _host as host
 from research_amd import _lib, ops
 
-host = pytest.importorskip("research_amd._host")
 _lib.load()
+
+
+def test_a_module_that_is_built_after_the_import():
+    """``ops`` imported while there is no native module: calls say so, and work once there is one."""
+    code = """
+import sys
+class Missing:
+    def find_spec(self, name, path=None, target=None):
+        if name == "research_amd._host":
+            raise ImportError("not built")
+sys.meta_path.insert(0, Missing())
+import torch
+from research_amd import ops
+a = torch.zeros(3, 8)
+for call in (lambda: ops._typed(torch.float32, a), lambda: ops.softcap(a, 1.0)):
+    try:
+        call()
+    except FileNotFoundError as e:
+        assert "research_amd.build" in str(e)
+    else:
+        raise SystemExit("not refused")
+del sys.meta_path[0]
+assert ops._shaped(a, 3, 8) is True and ops._row_stride(a) == 8
+for bad, error in ((lambda: ops._typed(torch.int32, a), ValueError), (lambda: ops._dense(a.t()), ValueError), (lambda: ops.softcap(a, 1.0), RuntimeError)):
+    try:
+        bad()
+    except error:
+        pass
+    else:
+        raise SystemExit("not refused")
+ops._run("pa_softcap", a, None, 0, 1.0, 0, None)
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=ops.__file__.rsplit("/research_amd/", 1)[0])
 
 
 def test_checks():
