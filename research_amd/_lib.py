@@ -1,5 +1,5 @@
 """ctypes binding of ``libpaged_attn.so`` (signatures: ``include/paged_attn.h``); the tensor-level calls of ``ops.py`` go through
-``_host.so`` (``csrc/host_calls.cpp``), which takes tensors themselves.
+the module ``_host`` (``csrc/host_calls.cpp``), which takes tensors themselves.
 
 The library is built in-tree next to this file by ``research_amd/build.py``.
 There is no fallback: if it is missing, loading raises and every attention
@@ -183,7 +183,7 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
         try:
             from . import _host
         except ImportError as e:
-            raise FileNotFoundError(f"{os.path.dirname(LIB_PATH)}/_host.so does not load ({e}): build it with `python -m research_amd.build`") from e
+            raise FileNotFoundError(f"{os.path.dirname(LIB_PATH)}/_host does not load ({e}): build it with `python -m research_amd.build`") from e
         _host.bind(lib._handle)
         _lib = lib
     return lib

@@ -1,5 +1,5 @@
 // The Python side of a call: the library's functions taking torch tensors as their pointers, and the checks that stand before most of them.
-// Built into research_amd/_host.so (plain C++; it finds the functions in the library that _lib.py has loaded).
+// Built into the module research_amd._host (plain C++; it finds the functions in the library that _lib.py has loaded).
 //
 // A call of a small shape is as long as its host side.  us a pass with ctypes and each tensor's pointer, type, shape and strides asked for from
 // Python -> this: mLSTM, 34 rows and two tokens behind them 49.5 -> 30.8; SSD, 235 rows and a token 32.7 -> 21.2; delta rule, 37 rows and three
@@ -250,6 +250,14 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 }  // namespace
 
 PyMODINIT_FUNC PyInit__host() {
+    // What is read here of a tensor lies where the torch that this was built against puts it.
+    PyObject *v = PyImport_ImportModule("torch.version"), *is = v ? PyObject_GetAttrString(v, "__version__") : nullptr;
+    Py_XDECREF(v);
+    if (!is) return nullptr;
+    const bool same = PyUnicode_Check(is) && PyUnicode_CompareWithASCIIString(is, PA_TORCH_VERSION) == 0;
+    if (!same) PyErr_Format(PyExc_ImportError, "built for torch " PA_TORCH_VERSION ", this is torch %S", is);
+    Py_DECREF(is);
+    if (!same) return nullptr;
     PyObject *c = PyImport_ImportModule("torch._C");
     if (!c) return nullptr;
     raw_stream = PyObject_GetAttrString(c, "_cuda_getCurrentRawStream");

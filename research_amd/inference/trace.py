@@ -70,9 +70,9 @@ def replay(engine, lines, out_dir: str, report: TextIO) -> None:
 
 def main(argv: Optional[List[str]] = None) -> int:
     args = parse_args(argv)
-    from .. import _lib, build
+    from .. import build
 
-    if not all(os.path.exists(os.path.join(os.path.dirname(_lib.LIB_PATH), n)) for n in (_lib.LIB_NAME, "_host.so")):
+    if not build.built():
         build.build(jobs=min(16, os.cpu_count() or 1))
     from .engine import InferenceEngine
     from .registry import model_len

@@ -4,6 +4,7 @@ library's functions take, and what is refused."""
 import re
 import subprocess
 import sys
+import sysconfig
 
 import pytest
 import torch
@@ -18,6 +19,7 @@ def test_a_module_that_is_built_after_the_import():
     """``ops`` imported while there is no native module: calls say so, and work once there is one."""
     code = """
 import sys
+import sysconfig
 class Missing:
     def find_spec(self, name, path=None, target=None):
         if name == "research_amd._host":
@@ -108,3 +110,29 @@ def test_arguments():
             call(bad, t, 0, 1.0)
     with pytest.raises(TypeError):
         call(t, t, 0, "1")
+
+
+def test_a_module_of_another_interpreter_or_torch_is_not_taken():
+    root = ops.__file__.rsplit("/research_amd/", 1)[0]
+    assert host.__file__.endswith("_host" + sysconfig.get_config_var("EXT_SUFFIX"))  # (which other interpreters do not look for)
+    code = """
+import torch.version
+torch.version.__version__ = "1.0"
+try:
+    import research_amd._host
+except ImportError as e:
+    assert "torch 1.0" in str(e), e
+else:
+    raise SystemExit("taken")
+from research_amd import _lib
+try:
+    _lib.load()
+except FileNotFoundError as e:
+    assert "research_amd.build" in str(e)
+else:
+    raise SystemExit("taken")
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=root)
+    rules = lambda *args: subprocess.run(["make", "-C", root + "/research_amd/csrc", "-n", f"PYTHON={sys.executable}", *args, "host"], check=True,
+                                         stdout=subprocess.PIPE, text=True).stdout
+    assert "host_calls.cpp" in rules("TORCH_VERSION=1.0")  # (another torch than it was built for: built again)
