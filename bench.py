@@ -17,6 +17,7 @@ behind 200 000 cached keys at head_dim 128 and 256) under ``secondary``.
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -581,9 +582,10 @@ def bench_decode(name, args, dev) -> dict:
     n_pools = 4 if kv_bytes < (1 << 30) else 1
     pools = [(k_pool, v_pool)] + [(k_pool.clone(), v_pool.clone()) for _ in range(n_pools - 1)]
     turn = [0]
-    # one launch (the split pass merges the pieces itself) or two (split pass, reduction pass)
-    passes = int(_lib.load().pa_decode_passes(w.batch, w.num_q_heads, w.num_kv_heads, w.head_dim,
-                                              ops.PA_DTYPE[k_pool.dtype]))
+    # one launch or two (split pass or runs of the kernel for narrow tables, and what merges their results)
+    runs = ctypes.c_int(0)
+    passes = int(_lib.load().pa_decode_launches(w.batch, w.num_q_heads, w.num_kv_heads, w.head_dim, tables.shape[1], w.block_size, 0,
+                                                ops.PA_DTYPE[q.dtype], ops.PA_DTYPE[k_pool.dtype], ctypes.byref(runs)))
 
     def step(entry="pa_decode"):
         kp, vp = pools[turn[0] % n_pools]
@@ -601,7 +603,7 @@ def bench_decode(name, args, dev) -> dict:
     ms_step_mean, ms_step = timed_steps(step, args.steps)
     wall = time.perf_counter() - wall
     n_kernel = max(args.steps, KERNEL_LAUNCHES)
-    # the dominant kernel alone: the split pass (with one launch per step it IS the step)
+    # the dominant kernel alone: the first pass (with one launch per step it IS the step)
     ms_split = timed_ms(lambda: step("pa_decode" if passes == 1 else "pa_decode_split"), n_kernel)
     ms_reduce = None if passes == 1 else timed_ms(lambda: step("pa_decode_reduce"), n_kernel)
 
@@ -695,8 +697,8 @@ def bench_decode(name, args, dev) -> dict:
             "seed": 1000 + int(name[1]), "generate_s": round(t_gen, 1),
         },
         "roofline": {
-            "bound": "hbm", "kernel": "decode_split_kernel", "achieved": achieved, "peak": HBM_PEAK_GBPS,
-            "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS, "traffic": measured_traffic(name),
+            "bound": "hbm", "kernel": "decode_short_kernel" if runs.value else "decode_split_kernel", "achieved": achieved,
+            "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS, "traffic": measured_traffic(name),
             "kernel_ms": ms_split, "kernel_launches": n_kernel, "reduce_kernel_ms": ms_reduce,
         },
     }

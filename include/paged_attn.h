@@ -107,11 +107,23 @@ size_t pa_decode_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, i
                                  int kv_dtype);
 
 /*
- * Kernel launches one pa_decode call of these shapes makes on the current device at most: 1 when the batch is large
- * enough that the split pass merges a sequence's pieces itself, else 2 (split pass, reduction pass); negative on
- * error.  (A call whose block tables are narrow takes other kernels, one launch or, for few sequences in several runs each, two.)  For callers that time or profile the passes.  (No counterpart in the reference.)
+ * Kernel launches one pa_decode call makes on the current device, of these heads and any tables wide enough for the
+ * split pass: 1 when the batch is large enough that it merges a sequence's pieces itself, else 2 (split pass,
+ * reduction pass); negative on error.  Narrow tables can make either one or two of it: pa_decode_launches.  (No
+ * counterpart in the reference.)
  */
 int pa_decode_passes(int batch, int num_q_heads, int num_kv_heads, int head_dim, int kv_dtype);
+
+/*
+ * Kernel launches one pa_decode call of these shapes makes on the current device (0 for an empty batch, else 1 or 2;
+ * of more than 8192 sequences, which are taken in parts: of a part); negative on error.  runs (may be NULL): over
+ * narrow tables, the runs that each sequence is cut into (1: one launch and nothing to merge); 0 where the split
+ * pass takes the call.  Where the answer is 1, pa_decode_split and pa_decode_reduce are no two parts of pa_decode.
+ * (pa_decode_static, whose scratch holds fewer results, may cut a sequence into fewer runs.)  For callers that time
+ * or profile the passes.  (No counterpart in the reference.)
+ */
+int pa_decode_launches(int batch, int num_q_heads, int num_kv_heads, int head_dim, int64_t bt_stride, int block_size,
+                       int window, int q_dtype, int kv_dtype, int *runs);
 
 /*
  * Paged decode attention.  Replaces FlexAttentionBackend._decode_attention
@@ -155,8 +167,8 @@ int pa_decode(const void *q, const void *k_cache, const void *v_cache, void *out
 /*
  * The two passes of pa_decode as separate calls, same arguments:
  * pa_decode_split followed by pa_decode_reduce on the same stream and
- * workspace give pa_decode's result (to rounding: for large batches pa_decode
- * merges inside its one launch, in another order; see pa_decode_passes).  For
+ * workspace give pa_decode's result (to rounding: where pa_decode is one launch,
+ * it merges there, in another order; see pa_decode_launches).  For
  * callers that time or schedule the passes separately.  (The
  * reference has one fused call site, attention/flex_backend.py:227-229; these
  * have no separate counterpart there.)

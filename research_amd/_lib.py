@@ -50,6 +50,7 @@ SIGNATURES = {
     ),
     "pa_decode_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "pa_decode_passes": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "pa_decode_launches": (c_int, [c_int, c_int, c_int, c_int, c_int64, c_int, c_int, c_int, c_int, c_void_p]),
     "pa_decode": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,

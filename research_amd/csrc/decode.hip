@@ -97,6 +97,23 @@ int static_scratch(void **ptr) {
 
 enum { kPhaseSplit = 1, kPhaseReduce = 2 };
 
+// What a call of both passes launches, from shapes alone.
+struct Route {
+    int runs;    // of a sequence, of the kernel for narrow tables; 0: the split pass takes the call
+    bool whole;  // a workgroup of the split pass takes a whole sequence
+    bool merge;  // the split pass leaves nothing to a second launch
+    int launches() const { return runs > 0 ? (runs > 1 ? 2 : 1) : merge ? 1 : 2; }
+};
+Route decode_route(const KernelSet &ks, int batch, const HeadPlan &plan, const WsPlan &w, int head_dim, int kv_dtype, int64_t bt_stride,
+                   int block_size, int window, int grid) {
+    const int bytes = (int)pa_dtype_bytes(kv_dtype);
+    Route r;
+    r.runs = ks.few ? plan_short_splits(batch, plan, w, bytes, bt_stride, block_size, window, num_cus()) : 0;
+    r.whole = plan_whole_sequences(batch, plan, head_dim, bytes, bt_stride, block_size, window);
+    r.merge = r.whole || plan_merge_in_split(batch, plan, grid);
+    return r;
+}
+
 int decode_launch(int phases, const void *q, const void *k_cache, const void *v_cache, void *out,
                   const int32_t *block_tables, int64_t bt_stride, const int32_t *seq_lens,
                   const int32_t *extra_zero_keys, const float *k_scale, const float *v_scale, int batch,
@@ -182,12 +199,13 @@ int decode_launch(int phases, const void *q, const void *k_cache, const void *v_
     a.part_acc = (float *)(ws + w.acc_off);
     // Batches that leave a sequence few pieces, or none, are finished by the split pass alone.
     a.group_tickets = (unsigned long long *)(ws + kPlanGroupTicketOff);
-    a.whole = plan_whole_sequences(batch, plan, head_dim, pa_dtype_bytes(kv_dtype), bt_stride, block_size, window) ? 1 : 0;
-    a.merge_in_split = phases == (kPhaseSplit | kPhaseReduce) && (a.whole || plan_merge_in_split(batch, plan, grid)) ? 1 : 0;
+    const Route route = decode_route(ks, batch, plan, w, head_dim, kv_dtype, bt_stride, block_size, window, grid);
+    a.whole = route.whole ? 1 : 0;
+    a.merge_in_split = phases == (kPhaseSplit | kPhaseReduce) && route.merge ? 1 : 0;
 
     hipStream_t s = (hipStream_t)stream;
     a.split_grid = grid;
-    a.splits = ks.few ? plan_short_splits(batch, plan, w, pa_dtype_bytes(kv_dtype), bt_stride, block_size, window, num_cus()) : 0;
+    a.splits = route.runs;
     if (a.splits > 0) {
         a.leave = a.splits > 1 || phases != (kPhaseSplit | kPhaseReduce) ? 1 : 0;
         if (phases & kPhaseSplit) {
@@ -246,6 +264,20 @@ extern "C" int pa_decode_passes(int batch, int num_q_heads, int num_kv_heads, in
     if (batch < 0 || !plan.nrep_t) return pa_fail(PA_ERR_UNSUPPORTED, "pa_decode_passes: no kernel for these shapes");
     if (batch > kMaxBatch) batch = kMaxBatch;  // launches per group of kMaxBatch sequences
     return plan_merge_in_split(batch, plan, split_grid()) ? 1 : 2;
+}
+
+extern "C" int pa_decode_launches(int batch, int num_q_heads, int num_kv_heads, int head_dim, int64_t bt_stride, int block_size,
+                                  int window, int q_dtype, int kv_dtype, int *runs) {
+    pa_clear_error();
+    PA_REQUIRE(batch >= 0 && bt_stride >= 0 && block_size > 0 && window >= -0x7fffffff, "batch / bt_stride / block_size / window out of range");
+    const HeadPlan plan = plan_heads(num_q_heads, num_kv_heads, head_dim, pa_dtype_bytes(kv_dtype));
+    const KernelSet ks = plan.nrep_t ? pa_pick_kernels(q_dtype, kv_dtype, plan.d_pad, plan.nrep_t) : KernelSet{};
+    if (!ks.split) return pa_fail(PA_ERR_UNSUPPORTED, "pa_decode_launches: no kernel for these shapes");
+    if (batch > kMaxBatch) batch = kMaxBatch;  // launches per group of kMaxBatch sequences
+    const Route r = decode_route(ks, batch, plan, plan_workspace(batch, plan, plan.d_pad, kMaxSplitGrid), head_dim, kv_dtype, bt_stride,
+                                 block_size, window, split_grid());
+    if (runs) *runs = batch > 0 ? r.runs : 0;
+    return batch > 0 ? r.launches() : 0;
 }
 
 #define PA_DECODE_PARAMS                                                                                       \

@@ -142,6 +142,28 @@ def test_decode_workspace_arithmetic():
     assert lib.pa_decode_workspace_bytes(4, 30, 8, 128, _lib.PA_BF16) == 0
 
 
+def test_launches_of_decode_by_the_width_of_its_tables():
+    lib, runs = _lib.load(), ctypes.c_int()
+    bf, f32, fp8 = _lib.PA_BF16, _lib.PA_F32, _lib.PA_FP8_E4M3
+
+    def launches(batch, heads, keys, q=bf, kv=bf, bs=16, window=0):
+        runs.value = -1
+        return lib.pa_decode_launches(batch, *heads, keys // bs, bs, window, q, kv, ctypes.byref(runs)), runs.value
+
+    assert launches(4, (14, 2, 64), 512) == (1, 1) and launches(1, (14, 2, 64), 16384) == (2, 64)
+    # one launch for long tables, two for narrow ones: three runs of each sequence and their merge; and the other way round
+    assert lib.pa_decode_passes(128, 16, 1, 256, bf) == 1 and launches(128, (16, 1, 256), 512) == (2, 3)
+    assert lib.pa_decode_passes(4, 14, 2, 64, bf) == 2
+    for batch, heads, kv in ((256, (32, 8, 128), bf), (16, (32, 8, 128), bf), (8, (32, 8, 128), fp8), (300, (16, 8, 128), fp8)):
+        assert launches(batch, heads, 1 << 20, kv=kv) == (lib.pa_decode_passes(batch, *heads, kv), 0)
+    assert launches(4, (8, 2, 128), 64, f32, f32) == (1, 0) and launches(4, (8, 2, 128), 1024, f32, f32) == (2, 0)  # (whole sequences)
+    assert launches(4, (32, 8, 128), 64, bs=8) == (1, 0) and launches(4, (8, 2, 32), 4096) == (2, 0)
+    assert launches(4, (32, 8, 128), 1 << 20, window=200) == (1, 1) and launches(0, (32, 8, 128), 64) == (0, 0)
+    assert lib.pa_decode_launches(4, 14, 2, 64, 4, 16, 0, bf, bf, None) == 1
+    for bad, word in (((-1, (8, 2, 64), 64), "batch"), ((4, (8, 3, 64), 64), "no kernel"), ((4, (8, 2, 64), 64, f32), "no kernel")):
+        assert launches(*bad)[0] < 0 and word in _lib.last_error()
+
+
 def test_prefill_and_quantize_argument_errors():
     args = [FAKE, FAKE, FAKE, FAKE, FAKE, 4, FAKE, FAKE, FAKE, None, 2, 16, 32, 8, 128, 16, 64, 0.088, 0,
             _lib.PA_FP8_E4M3, None]
