@@ -697,7 +697,7 @@ def bench_decode(name, args, dev) -> dict:
             "seed": 1000 + int(name[1]), "generate_s": round(t_gen, 1),
         },
         "roofline": {
-            "bound": "hbm", "kernel": "decode_short_kernel" if runs.value else "decode_split_kernel", "achieved": achieved,
+            "bound": "hbm", "kernel": "decode_short_kernel" if runs.value > 0 else "decode_split_kernel", "achieved": achieved,
             "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS, "traffic": measured_traffic(name),
             "kernel_ms": ms_split, "kernel_launches": n_kernel, "reduce_kernel_ms": ms_reduce,
         },
