@@ -117,7 +117,7 @@ def test_lines_of_the_rule(replay):
 def test_launches_of_runs_on_the_device(replay, run, lens, hq, hkv, d, kv):
     from oracle import paged_oracle as po
     from research_amd import ops
-    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.gpu_helpers import DEV, WIDE, announce, assert_close, decode_route, tables_to_device
     from tests.test_gpu_decode_merge import Batch
 
     planes = {(32, 8, 128): 2, (14, 2, 64): 1, (8, 2, 64): 1}[hq, hkv, d]
@@ -126,7 +126,8 @@ def test_launches_of_runs_on_the_device(replay, run, lens, hq, hkv, d, kv):
     b = Batch(lens, hq, hkv, d, kv, seed=run)
     (k, v, _, _), _ = b.device_pools()
     q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
-    ws, tables = ops.decode_workspace(q, k), tables_to_device(b.tables)
+    ws, tables = ops.decode_workspace(q, k), tables_to_device(b.tables, WIDE)
+    assert decode_route(len(lens), hq, hkv, d, q.dtype, k.dtype, WIDE, b.bs) == 0
     got = ops.decode(q, k, v, tables, n, b.bs, b.scale, ws)
     assert_close(got, po.paged_decode(b.q, b.k, b.v, b.tables, b.lens, b.bs, b.scale), b.tol, "runs of blocks")
     assert torch.equal(ops.decode(q, k, v, tables, n, b.bs, b.scale, ws), got)
@@ -141,7 +142,7 @@ def test_pieces_of_wide_groups_over_fp8_pools(hq, hkv, d, queries):
     a second launch and in the one."""
     from oracle import paged_oracle as po
     from research_amd import ops
-    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.gpu_helpers import DEV, WIDE, announce, assert_close, decode_route, tables_to_device
     from tests.test_gpu_decode_merge import Batch
 
     announce(f"fp8 pieces {hq}/{hkv}x{d} {queries}")
@@ -149,7 +150,8 @@ def test_pieces_of_wide_groups_over_fp8_pools(hq, hkv, d, queries):
         b = Batch(lens, hq, hkv, d, "fp8", seed=d)
         (k, v, ks, vs), (kr, vr) = b.device_pools()
         q = b.q.to(torch.float16 if queries == "f16" else torch.bfloat16)
-        got = ops.decode(q.to(DEV), k, v, tables_to_device(b.tables), torch.tensor(b.lens, dtype=torch.int32, device=DEV), b.bs, b.scale,
+        assert decode_route(len(lens), hq, hkv, d, q.dtype, k.dtype, WIDE, b.bs) == 0
+        got = ops.decode(q.to(DEV), k, v, tables_to_device(b.tables, WIDE), torch.tensor(b.lens, dtype=torch.int32, device=DEV), b.bs, b.scale,
                          ops.decode_workspace(q.to(DEV), k), None, ks, vs)
         # (weights are multiplied by scales and packed to 16 bits: 2^-9 of values of at most 4)
         assert_close(got, po.paged_decode(q.float(), kr.float(), vr.float(), b.tables, b.lens, b.bs, b.scale), 2e-2, f"{len(lens)} sequences")

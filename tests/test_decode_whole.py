@@ -1,6 +1,7 @@
-"""Decode with narrow block tables: a workgroup takes a whole (plane, sequence), and one launch does (``plan_whole_sequences`` of
-``decode_plan.h``).  The rule's lines on the CPU; on the device the same batch with narrow tables and with tables padded beyond the rule's
-line, which take the split pass and the merge, against the oracle and against each other."""
+"""Decode with narrow block tables that the kernel for them does not take (32-bit pools, blocks that are no whole tiles of 16 keys, large
+batches): a workgroup of the split pass takes a whole (plane, sequence), and one launch does (``plan_whole_sequences`` of ``decode_plan.h``).
+The rule's lines on the CPU; on the device the same batch with narrow tables and with tables padded beyond the rule's line, which take the
+split pass in ranges and the merge, against the oracle and against each other."""
 
 import ctypes
 import os
@@ -44,37 +45,40 @@ def test_lines_of_the_rule(whole):
 
 
 CASES = [
-    ([1, 2, 24, 47], 14, 2, 64, "bf16", 0),              # (and where a workgroup's ranges end in the split pass: 0, 15, 16, 17)
-    ([0, 96, 17, 16, 15, 0, 1, 81], 32, 8, 128, "bf16", 0),
-    ([64, 0, 33, 1], 8, 2, 128, "f32", 0),
-    ([96, 5, 0, 48], 16, 8, 128, "fp8", 0),
-    ([700, 1, 333], 16, 2, 64, "fp8", 0),
-    ([90, 16, 0, 31], 16, 8, 256, "f16", 0),
-    ([200, 3, 0, 129], 8, 2, 72, "f16", 0),
-    ([40, 64, 1, 0], 4, 4, 32, "f32", 0),
-    ([5000, 63, 0, 64, 65, 999], 32, 8, 128, "bf16", 64),  # (long tables, a short window)
-    ([130, 64, 0, 65, 127], 32, 8, 128, "bf16", -64),
-    ([192, 17, 0, 100, 1, 64] * 50, 32, 8, 128, "bf16", 0),  # more workgroups than the split pass has
-    ([64, 50, 49, 33] * 32, 32, 8, 128, "bf16", 0),
-    ([40, 17, 90, 5] * 70, 14, 2, 64, "fp8", 0),
+    ([1, 2, 24, 47], 14, 2, 64, "bf16", 0, 8),              # (and where a workgroup's ranges end in the split pass: 0, 15, 16, 17)
+    ([0, 96, 17, 16, 15, 0, 1, 81], 32, 8, 128, "bf16", 0, 8),
+    ([64, 0, 33, 1], 8, 2, 128, "f32", 0, 16),
+    ([96, 5, 0, 48], 16, 8, 128, "fp8", 0, 8),
+    ([700, 1, 333], 16, 2, 64, "fp8", 0, 4),
+    ([90, 16, 0, 31], 16, 8, 256, "f16", 0, 8),
+    ([200, 3, 0, 129], 8, 2, 72, "f16", 0, 24),
+    ([40, 64, 1, 0], 4, 4, 32, "f32", 0, 16),
+    ([40, 64, 1, 0], 4, 4, 32, "bf16", 0, 16),
+    ([5000, 63, 0, 64, 65, 999], 32, 8, 128, "bf16", 64, 8),  # (long tables, a short window)
+    ([130, 64, 0, 65, 127], 32, 8, 128, "bf16", -64, 8),
+    ([192, 17, 0, 100, 1, 64] * 64, 32, 8, 128, "bf16", 0, 16),  # more workgroups than the split pass has
+    ([192, 17, 0, 100, 1, 64] * 50, 32, 8, 128, "bf16", 0, 8),
+    ([64, 50, 49, 33] * 32, 32, 8, 128, "f16", 0, 8),
+    ([40, 17, 90, 5] * 70, 14, 2, 64, "fp8", 0, 8),
 ]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("lens,hq,hkv,d,kv,window", CASES)
-def test_narrow_and_wide_tables_agree(whole, lens, hq, hkv, d, kv, window):
+@pytest.mark.parametrize("lens,hq,hkv,d,kv,window,bs", CASES)
+def test_narrow_and_wide_tables_agree(whole, lens, hq, hkv, d, kv, window, bs):
     from oracle import paged_oracle as po
     from research_amd import ops
-    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.gpu_helpers import DEV, WIDE, announce, assert_close, decode_route, tables_to_device
     from tests.test_gpu_decode_merge import Batch
 
-    announce(f"decode whole: {len(lens)} x {max(lens)} {hq}/{hkv}x{d} {kv} window {window}")
-    b = Batch(lens, hq, hkv, d, kv, seed=len(lens) + d)
+    announce(f"decode whole: {len(lens)} x {max(lens)} {hq}/{hkv}x{d} {kv} window {window} blocks of {bs}")
+    b = Batch(lens, hq, hkv, d, kv, seed=len(lens) + d, bs=bs)
     (k, v, ks, vs), (kr, vr) = b.device_pools()
     q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
     size = {"f32": 4, "fp8": 1}.get(kv, 2)
     narrow = tables_to_device(b.tables)
-    assert whole(len(lens), (hq, hkv, d, size), narrow.shape[1], window=window)
+    assert whole(len(lens), (hq, hkv, d, size), narrow.shape[1], bs, window)
+    assert decode_route(len(lens), hq, hkv, d, q.dtype, k.dtype, narrow.shape[1], bs, window) == -1
     ws, padding = ops.decode_workspace(q, k), max(lens) - n
     for ez in (None,) if window else (None, padding):
         got = ops.decode(q, k, v, narrow, n, b.bs, b.scale, ws, ez, ks, vs, window=window)
@@ -83,9 +87,8 @@ def test_narrow_and_wide_tables_agree(whole, lens, hq, hkv, d, kv, window):
                                [n - f for n, f in zip(b.lens, first)], b.bs, b.scale, pad_zero_keys=ez is not None, window=max(window, 0))
         assert_close(got, want, b.tol if kv != "fp8" else 2e-2, "narrow tables")
         if not window:
-            padded = torch.full((len(lens), 4096), -1, dtype=torch.int32, device=DEV)
-            padded[:, : narrow.shape[1]] = narrow
-            assert not whole(len(lens), (hq, hkv, d, size), padded.shape[1])
+            padded = tables_to_device(b.tables, WIDE)
+            assert decode_route(len(lens), hq, hkv, d, q.dtype, k.dtype, WIDE, bs) == 0
             other = ops.decode(q, k, v, padded, n, b.bs, b.scale, ws, ez, ks, vs)
             # (both round to the type of q, at most 2^-8 of a value apart, weights to 16 bits on the way: 2^-9 of values of at most 5)
             assert_close(got, other.double().cpu().numpy(), 1e-5 if kv == "f32" else 2e-2, "wide tables")
@@ -95,17 +98,18 @@ def test_narrow_and_wide_tables_agree(whole, lens, hq, hkv, d, kv, window):
 @pytest.mark.gpu
 def test_lengths_beyond_a_narrow_table_count_as_zero_keys():
     from research_amd import ops
-    from tests.gpu_helpers import DEV, announce
+    from tests.gpu_helpers import DEV, WIDE, announce, decode_route
     from tests.test_gpu_decode_merge import Batch
 
     announce("decode whole: lengths beyond the tables")
-    b = Batch([64, 64, 64], 32, 8, 128, "bf16", seed=3)
+    b = Batch([64, 64, 64], 32, 8, 128, "bf16", seed=3, bs=8)
     (k, v, _, _), _ = b.device_pools()
     q = b.q.to(DEV)
     n = torch.tensor([64, 300, 2000], dtype=torch.int32, device=DEV)
     narrow = torch.tensor(b.tables, dtype=torch.int32, device=DEV)
-    padded = torch.full((3, 512), -1, dtype=torch.int32, device=DEV)
-    padded[:, :4] = narrow
+    padded = torch.full((3, WIDE), -1, dtype=torch.int32, device=DEV)
+    padded[:, :8] = narrow
+    assert [decode_route(3, 32, 8, 128, q.dtype, k.dtype, t.shape[1], 8) for t in (narrow, padded)] == [-1, 0]
     ws = ops.decode_workspace(q, k)
     got, want = (ops.decode(q, k, v, t, n, b.bs, b.scale, ws).float() for t in (narrow, padded))
     assert (got - want).abs().max() < 2e-2 and torch.isfinite(got).all()

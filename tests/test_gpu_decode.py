@@ -12,7 +12,7 @@ import torch
 from oracle import paged_oracle as po
 from research_amd import ops
 from research_amd.workloads import make_decode
-from tests.gpu_helpers import DEV, announce, assert_close, run_decode, tables_to_device
+from tests.gpu_helpers import DEV, WIDE, announce, assert_close, decode_by_split_pass, decode_route, run_decode, tables_to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -211,6 +211,8 @@ def test_sliding_window_decode(window):
     got = ops.decode(q, kp, vp, tables, lens, w.block_size, w.scale, ws, window=window)
     want = po.paged_decode(w.q, w.k_pool, w.v_pool, _lists(w), w.seq_lens, w.block_size, w.scale, window=window)
     assert_close(got, want, 2e-2, f"window {window}")
+    got_split = decode_by_split_pass(q, kp, vp, _lists(w), w.seq_lens.tolist(), w.block_size, w.scale, window=window)
+    assert_close(got_split[0], want, 2e-2, f"split pass, window {window}")
     if window >= int(w.seq_lens.max()):
         assert torch.equal(got, ops.decode(q, kp, vp, tables, lens, w.block_size, w.scale, ws))
 
@@ -238,8 +240,10 @@ def test_sliding_window_decode_other_types_and_garbage_before_the_window():
     got = ops.decode(q, k8, v8, tables, lens, w.block_size, w.scale, ws, k_scale=ks, v_scale=vs, window=77)
     kd = po.dequantize_kv_e4m3(k8.cpu().view(torch.uint8), ks.cpu(), w.block_size)
     vd = po.dequantize_kv_e4m3(v8.cpu().view(torch.uint8), vs.cpu(), w.block_size)
-    assert_close(got, po.paged_decode(w.q, kd, vd, _lists(w), w.seq_lens, w.block_size, w.scale, window=77), 6e-2,
-                 "fp8 window")
+    want = po.paged_decode(w.q, kd, vd, _lists(w), w.seq_lens, w.block_size, w.scale, window=77)
+    assert_close(got, want, 6e-2, "fp8 window")
+    got = decode_by_split_pass(q, k8, v8, _lists(w), w.seq_lens.tolist(), w.block_size, w.scale, None, ks, vs, window=77)
+    assert_close(got[0], want, 6e-2, "fp8 window, split pass")
     # blocks wholly before the window may hold anything, including NaN: they are never read; older keys inside
     # the window's first block are real keys of the sequence (finite) and are masked out by selection
     w = make_decode("c2", batch=2, len_range=(300, 400), seed=3)
@@ -259,18 +263,22 @@ def test_sliding_window_decode_other_types_and_garbage_before_the_window():
                      window=window)
     want = po.paged_decode(w.q, w.k_pool, w.v_pool, _lists(w), w.seq_lens, 16, w.scale, window=window)
     assert_close(got, want, 2e-2, "poisoned keys before the window")
+    got = decode_by_split_pass(q, kp.to(DEV), vp.to(DEV), _lists(w), w.seq_lens.tolist(), 16, w.scale, window=window)
+    assert_close(got[0], want, 2e-2, "poisoned keys before the window, split pass")
 
 
-def test_decode_step_in_a_hip_graph():
+@pytest.mark.parametrize("columns", [8, WIDE])  # (a kernel for narrow tables, the split pass)
+def test_decode_step_in_a_hip_graph(columns):
     """The append + decode launches of one step, captured once and replayed: the entry points allocate nothing,
     clear nothing with memsets and read lengths, slots and tables from device memory, so a serving loop can
     update those buffers in place and replay.  Every replay is checked against the checker, with eager work
     and synchronisations between the replays."""
-    announce("decode in a HIP graph")
+    announce(f"decode in a HIP graph, {columns} columns")
     rng = np.random.default_rng(91)
     hq, hkv, d, bs, nb, batch = 8, 2, 128, 16, 64, 3
     lens = np.array([37, 5, 60], dtype=np.int32)
-    tables = np.full((batch, 8), -1, dtype=np.int32)
+    tables = np.full((batch, columns), -1, dtype=np.int32)
+    assert (decode_route(batch, hq, hkv, d, torch.bfloat16, torch.bfloat16, columns, bs) == 0) == (columns == WIDE)
     perm = rng.permutation(nb)
     for b in range(batch):
         tables[b, :6] = perm[b * 6 : b * 6 + 6]  # room for 96 tokens each
@@ -395,3 +403,5 @@ def test_few_kv_heads_with_blocks_of_16(hq, hkv, d, kv):
         got = ops.decode(q.to(DEV), *pools, tables_to_device(tables), torch.tensor(lens, dtype=torch.int32, device=DEV),
                          bs, scale, ws, None, extra.get("k_scale"), extra.get("v_scale"), window=window)
         assert_close(got, checked(window=window), tol, f"window {window}")
+        got = decode_by_split_pass(q.to(DEV), *pools, tables, lens, bs, scale, window=window, **extra)[0]
+        assert_close(got, checked(window=window), tol, f"split pass, window {window}")

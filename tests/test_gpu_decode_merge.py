@@ -17,7 +17,7 @@ import torch
 
 from oracle import paged_oracle as po
 from research_amd import _lib, ops
-from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+from tests.gpu_helpers import DEV, WIDE, announce, assert_close, decode_route, tables_to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -67,7 +67,9 @@ def _three_ways(b, window=0, extra_zero=None, checker_tables=None, what=""):
     (kp, vp, ks, vs), (kref, vref) = b.device_pools()
     q = b.q.to(DEV)
     assert _passes(len(b.lens), b.hq, b.hkv, b.d, kp.dtype) == 1, "this batch was meant to merge inside the split pass"
-    tables = tables_to_device(b.tables)
+    # (tables so wide that no kernel for narrow ones takes the call; a window bounds what the width says, and batches of more than 512 do not ask)
+    tables = tables_to_device(b.tables, None if window or len(b.lens) > 512 else WIDE)
+    assert decode_route(*q.shape[:2], b.hkv, b.d, q.dtype, kp.dtype, tables.shape[1], b.bs, window) == 0
     lens = torch.tensor(b.lens, dtype=torch.int32, device=DEV)
     ez = None if extra_zero is None else torch.tensor(extra_zero, dtype=torch.int32, device=DEV)
     ws = ops.decode_workspace(q, kp)
@@ -137,8 +139,18 @@ def test_window_extra_zero_keys_short_table_and_bad_block_ids(kv):
     b.tables[100] = b.tables[100][:7]
     _three_ways(b, checker_tables=checker_tables, what="short table / bad ids")
     _three_ways(b, extra_zero=[max(b.lens) - n for n in b.lens], checker_tables=checker_tables, what="extra zero keys")
+    b = Batch(_ragged(rng, 520, 1, 300, empties=5), hq, hkv, d, kv, seed=6)
     for window in (1, 16, 37, 150):
-        _three_ways(b, window=window, checker_tables=checker_tables, what=f"window {window}")
+        _three_ways(b, window=window, what=f"window {window}")
+
+
+@pytest.mark.parametrize("kv,batch,hq,hkv", [("bf16", 128, 32, 8), ("fp8", 256, 8, 2)])
+def test_windows_wider_than_narrow_tables(kv, batch, hq, hkv):
+    """Up to 512 sequences, whose table of units every wave makes by itself, with windows that leave them in several pieces."""
+    announce(f"decode merge-in-split wide windows {kv}")
+    b = Batch(_ragged(np.random.default_rng(5), batch, 1, 1500, empties=3), hq, hkv, 128, kv, seed=9)
+    for window in (1200, 1401):
+        _three_ways(b, window=window, what=f"window {window}")
 
 
 def test_one_very_long_sequence_among_255_short_ones():
@@ -230,7 +242,8 @@ def test_append_and_decode_of_256_sequences_replayed_from_a_graph(kv, static):
     lens = start.astype(np.int32).copy()
     lens_dev = torch.from_numpy(lens).to(DEV)
     slots_dev = torch.full((batch,), -1, dtype=torch.int64, device=DEV)  # the warm-up step appends nothing
-    tables_dev = torch.from_numpy(tables).to(DEV)
+    tables_dev = tables_to_device(tables, WIDE)
+    assert decode_route(batch, hq, hkv, d, dtype, kc.dtype, WIDE, bs) == 0  # (the split pass, and its tickets)
     out = torch.empty_like(q)
     ws = ops.decode_workspace(q, kc)
 
@@ -255,7 +268,7 @@ def test_append_and_decode_of_256_sequences_replayed_from_a_graph(kv, static):
         step()
     other = Batch(_ragged(rng, 150, 1, 500), hq, hkv, d, "bf16", seed=77)  # eager calls between the replays
     (okp, ovp, _, _), _ = other.device_pools()
-    oq, otab = other.q.to(DEV), tables_to_device(other.tables)
+    oq, otab = other.q.to(DEV), tables_to_device(other.tables, WIDE)
     olen = torch.tensor(other.lens, dtype=torch.int32, device=DEV)
     owant = po.paged_decode(other.q, other.k, other.v, other.tables, other.lens, bs, other.scale)
     for it in range(5):

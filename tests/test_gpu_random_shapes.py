@@ -8,7 +8,7 @@ import torch
 
 from oracle import paged_oracle as po
 from research_amd import ops
-from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+from tests.gpu_helpers import DEV, announce, assert_close, decode_by_split_pass, tables_to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -76,6 +76,8 @@ def test_random_decode(seed):
                      scale, ws, None, *extra, window=window)
     want = po.paged_decode(q, kref, vref, tables, lens, bs, scale, window=window)
     assert_close(got, want, tol, f"decode window={window}")
+    for copy in decode_by_split_pass(q.to(DEV), *pools, tables, lens, bs, scale, None, *extra, window=window)[[0, -1]]:
+        assert_close(copy, want, tol, f"split pass, window={window}")
 
 
 @pytest.mark.parametrize("seed", range(16))
@@ -113,6 +115,8 @@ def test_random_decode_head_sizes_between(seed):
                      scale, ws, None, *extra, window=window)
     want = po.paged_decode(q, kref, vref, tables, lens, bs, scale, window=window)
     assert_close(got, want, tol, f"decode window={window}")
+    for copy in decode_by_split_pass(q.to(DEV), *pools, tables, lens, bs, scale, None, *extra, window=window)[[0, -1]]:
+        assert_close(copy, want, tol, f"split pass, window={window}")
 
 
 @pytest.mark.parametrize("seed", range(16))
