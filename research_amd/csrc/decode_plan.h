@@ -232,23 +232,33 @@ PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, 
     return fits && runs * reps <= 65535 ? (int)runs : 0;
 }
 
-// Of what the split pass still has (32-bit pools, blocks that are no whole tiles, large batches of 16-bit ones): whether the block tables are so
-// narrow that a workgroup takes a whole (plane, sequence): nothing is left to merge then, and the second
-// launch (4 us, and its gap) goes.  A workgroup reads its keys at 20 to 45 GB/s, so that the line lies where that takes as long as the
-// second launch: 192 KB of keys and values (32-bit pools, whose loop has fewer loads in flight, 128 KB).  Large batches, whose
-// ranges would cross from one sequence into the next, gain up to 384 KB.  us, before -> whole sequences: 14 / 2 heads of 64 (512 bytes a key),
-// 4 sequences of 64 keys 15.4 -> 11.2, 16 of 256 keys 16.3 -> 15.2, of 512 keys 18.7 -> 20.6, 200 of 256 keys 32 -> 18.5; 32 / 8 of 128
-// (2 KB a key), 4 of 64 keys 13.7 -> 10.8, 32 of up to 96 keys 14.4 -> 12.5, of 256 keys 18.8 -> 22.4, 200 of 128 keys 34 -> 24; fp8 16 / 8 of
-// 128, 16 of 64 keys 13.6 -> 11.1, of 128 keys 13.9 -> 14.4, 200 of 256 keys 33.5 -> 30; 32-bit 8 / 2 of 128, 16 of 64 keys 15.6 -> 11.3,
-// 32 of up to 96 keys 15.9 -> 16.3.
+// Of what the split pass still has (32-bit pools, heads of up to 32, blocks that are no whole tiles, large batches of 16-bit ones): whether the
+// block tables are so narrow that a workgroup takes a whole (plane, sequence): nothing is left to merge then, and the second launch (4 us, and its
+// gap) goes.  A workgroup is a chain of waits, 1 to 2 us for each block that a wave takes (for a tile of 16 keys of longer ones), 2 to 4 us where
+// eight query heads a kv head meet fp8 values or the generic loop, so the line lies where the chain takes as long as the second launch and what
+// the ranges, which grow with the batch, take longer: 16 blocks, 32 from 16 workgroups on, half of it for those loops, 12 for the generic loop over 16
+// bits, and 192 KB of keys and values (32-bit pools, whose loop has fewer loads in flight, 128 KB).  Large batches, whose ranges would cross from one
+// sequence into the next, gain up to 64 blocks (the generic loop over 16 bits 32) and 384 KB, beyond 1024 workgroups 192 KB.
+// us, ranges -> whole sequences.  bf16, blocks of 8: 14 / 2 heads of 64, 4 sequences of 64 keys 15.8 -> 12.0, of 384 keys 16.2 -> 19.7, 16 of 256
+// keys 18.6 -> 16.7, 200 of 256 34 -> 19; 32 / 8 of 128, 4 of 96 keys 13.9 -> 12.2, 64 of 96 18.8 -> 12.5, 200 of 192 47 -> 34; blocks of 4, 14 / 2 of 64,
+// 4 of 256 keys 16.1 -> 34, 200 of 64 32 -> 18; blocks of 1, 4 of 64 keys 16.2 -> 32, 200 of 64 40 -> 35, of 256 79 -> 109.  fp8, blocks of 8: 16 / 8 of 128,
+// 4 of 96 keys 13.4 -> 12.5, 200 of 96 29 -> 17; 14 / 2 of 256, 4 of 128 keys 22 -> 24, 64 of 128 45 -> 25.  32-bit: 8 / 2 of 128, 16 of 64 keys
+// 15.6 -> 11.5, 512 of 192 45 -> 42; 14 / 2 of 64, 4 of 128 keys 16.2 -> 14.9, in blocks of 8 16.3 -> 20.3.  bf16, heads of 32: 8 / 2, 4 of 128 keys
+// 16.0 -> 13.7, of 512 16.4 -> 27, 200 of 512 40 -> 32; 4 / 4, 64 of 384 keys 14.9 -> 16.4.  bf16, 500 sequences: 32 / 8 of 128, of 192 keys 89 -> 77;
+// 16 / 8 of 256, of 96 keys 85 -> 94.  (Batches whose equal sequences fit the ranges without a rest lose up to a tenth: 512 of 192 keys, 32 / 8 of 128, 74
+// -> 78; unequal ones, of n / 8 .. n keys, gain more than equal ones throughout: 74 -> 61.)
 constexpr int kPlanWholeBytes = 192 * 1024;
 PA_PLAN_FN bool plan_whole_sequences(int batch, const HeadPlan &h, int head_dim, int kv_elem_bytes, int64_t table_blocks, int block_size, int window) {
     if (batch > kPlanWaveScanBatch) return false;
     const int64_t span = plan_window_span(window), units = (int64_t)h.planes() * batch;
     if (span > 0 && span / block_size + 2 < table_blocks) table_blocks = span / block_size + 2;
-    const bool many = batch >= 96 && units >= (kv_elem_bytes == 4 ? 512 : 192);
-    const int64_t most = (kv_elem_bytes == 4 ? kPlanWholeBytes * 2 / 3 : kPlanWholeBytes) * (many ? kv_elem_bytes == 4 ? 3 : 2 : 1);
-    return units <= 65535 && table_blocks <= most / ((int64_t)block_size * h.hpw * head_dim * kv_elem_bytes * 2);
+    const bool f32 = kv_elem_bytes == 4, many = batch >= 96 && units >= (f32 ? 512 : 192);
+    const bool slow = h.d_pad == 32 && !f32, heavy = h.nrep_t == 8 && (kv_elem_bytes != 2 || slow);
+    int steps = many ? 64 : (units < 16 ? 16 : 32) / (heavy ? 2 : 1);
+    if (slow && steps > (many ? 32 : 12)) steps = many ? 32 : 12;
+    const int64_t most = (f32 ? kPlanWholeBytes * 2 / 3 : kPlanWholeBytes) * (many && units <= 1024 ? f32 ? 3 : 2 : 1);
+    return units <= 65535 && table_blocks <= steps / ((block_size + 15) / 16) &&
+           table_blocks <= most / ((int64_t)block_size * h.hpw * head_dim * kv_elem_bytes * 2);
 }
 
 }  // namespace pa_decode_detail

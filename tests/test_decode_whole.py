@@ -34,14 +34,20 @@ def whole(tmp_path_factory):
 
 def test_lines_of_the_rule(whole):
     small, wide, f32 = (14, 2, 64, 2), (32, 8, 128, 2), (8, 2, 128, 4)  # 512, 2048 and 2048 bytes a key and plane
-    assert whole(4, small, 24) and not whole(4, small, 25)
+    assert whole(4, small, 16) and not whole(4, small, 17) and whole(16, small, 24) and not whole(16, small, 25)
     assert whole(4, wide, 6) and not whole(4, wide, 7)
     assert whole(4, f32, 4) and not whole(4, f32, 5)
     assert whole(96, wide, 12) and not whole(96, wide, 13) and not whole(95, wide, 7)
     assert whole(512, f32, 12) and not whole(511, f32, 5)
     assert whole(512, small, 48) and not whole(513, small, 1)
     assert whole(4, wide, 1 << 40, window=64) and not whole(4, wide, 1 << 40, window=81)  # (six blocks hold any 64 keys)
-    assert whole(4, wide, 1 << 40, window=-64) and whole(4, wide, 96, bs=1) and not whole(4, wide, 97, bs=1)
+    assert whole(4, wide, 1 << 40, window=-64) and whole(4, wide, 16, bs=1) and not whole(4, wide, 17, bs=1)
+    assert whole(8, wide, 32, bs=1) and not whole(8, wide, 33, bs=1) and whole(200, wide, 64, bs=1) and not whole(200, wide, 65, bs=1)
+    assert whole(4, small, 2, bs=100) and not whole(4, small, 3, bs=100)                # (seven tiles of 16 each)
+    fp8, d32 = (16, 2, 64, 1), (8, 2, 32, 2)  # eight query heads a kv head over fp8; the generic loop over 16 bits
+    assert whole(4, fp8, 8) and not whole(4, fp8, 9) and whole(16, fp8, 16) and not whole(16, fp8, 17)
+    assert all(whole(b, d32, 12) and not whole(b, d32, 13) for b in (1, 64)) and whole(200, d32, 32) and not whole(200, d32, 33)
+    assert whole(1024, wide[:3] + (1,), 1) is False and not whole(500, (16, 8, 256, 2), 7) and whole(256, (16, 8, 256, 2), 12)  # (1024 workgroups)
 
 
 CASES = [
@@ -49,9 +55,9 @@ CASES = [
     ([0, 96, 17, 16, 15, 0, 1, 81], 32, 8, 128, "bf16", 0, 8),
     ([64, 0, 33, 1], 8, 2, 128, "f32", 0, 16),
     ([96, 5, 0, 48], 16, 8, 128, "fp8", 0, 8),
-    ([700, 1, 333], 16, 2, 64, "fp8", 0, 4),
+    ([60, 1, 33], 16, 2, 64, "fp8", 0, 8),
     ([90, 16, 0, 31], 16, 8, 256, "f16", 0, 8),
-    ([200, 3, 0, 129], 8, 2, 72, "f16", 0, 24),
+    ([190, 3, 0, 129], 8, 2, 72, "f16", 0, 24),
     ([40, 64, 1, 0], 4, 4, 32, "f32", 0, 16),
     ([40, 64, 1, 0], 4, 4, 32, "bf16", 0, 16),
     ([5000, 63, 0, 64, 65, 999], 32, 8, 128, "bf16", 64, 8),  # (long tables, a short window)
