@@ -204,10 +204,14 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // 64 -> 51; 192 of 1024 45 -> 21; fp8 32 / 8 of 128, 32 of 256 24.5 -> 6.8; fp8 14 / 2 of 256, 16 of 2048 47 -> 14.5, 256 of 2048 185 -> 91.
 // Where the split pass stays: its ranges are equal whatever the lengths, so that unequal sequences in long runs are faster there once memory
 // counts.  More than four query heads a kv head hold up its vector unit, so the line lies further out, for fp8 furthest (unequal, keys n / 8 .. n,
-// the split pass -> runs of that length: 32 / 4 heads of 128, 32 of 8192 65 -> 76, 96 of 2048 57 -> 61, equal ones 70 -> 66; 14 / 2 of 64, 128 of
-// 4096 48 -> 40).  32 / 8 of 128, unequal: 16 of 2048 22.4 -> 24.2, 48 of 2048 44.8 -> 47.4, 1024 33 -> 27; equal, 256 of 512 90 -> 94.  One or two
-// query heads a kv head: 16 / 8 of 256, 16 of 1024 19.5 -> 24; 8 / 8 of 64, 3 of 8192 18 -> 24.  8 / 2 of 128, 1 of 8192 14.6 -> 15.2, 4096 14 -> 12.
-// (Over 1400 batches of 1 .. 384 sequences and thirteen shapes none was slower by more than the runs of one side differ, 3 %.)
+// the split pass -> runs of that length: 32 / 4 heads of 128, 32 of 8192 65 -> 76, 96 of 2048 57 -> 61, equal ones 70 -> 66); the less so the more kv
+// heads of 64 a wave of that pass takes at once (unequal: 14 / 2 of 64, 49 of 10359, runs of 432 KB, 45 -> 49, 141 of 3004, of 376 KB, 45 -> 41; 28 /
+// 4, 25 of 11157, of 465 KB, 45 -> 50; 64 / 8, 34 of 3981, of 498 KB, 54 -> 72).  32 / 8 of 128, unequal: 16 of 2048 22.4 -> 24.2, 48 of 2048
+// 44.8 -> 47.4, 1024 33 -> 27; equal, 256 of 512 90 -> 94.  One or two query heads a kv head: 16 / 8 of 256, 16 of 1024 19.5 -> 24; 8 / 8 of 64, 3 of
+// 8192 18 -> 24; over fp8, where the kernel's conversions count, 8 / 8 of 64, 3 of 8064 in runs of 806 keys 12.7 -> 15.0, 32 / 16, 66 of 917 38 -> 51.
+// 8 / 2 of 128, 1 of 8192 14.6 -> 15.2, 4096 14 -> 12.
+// (Over 1200 shapes of 1 .. 128 sequences that this takes, from 600 keys of 128 on, equal and unequal, 16 of 3600 batches were slower by more than 2 %, of which 4 / 4 heads of 96
+// over fp8 by up to 19, 30 of 1482 keys 15.6 -> 18.6, the others by up to 6; on average they took 0.55 of the split pass's time.)
 constexpr int kPlanShortHeads = 16, kPlanShortTile = 16, kPlanShortRuns = 64;
 PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, int kv_elem_bytes, int64_t table_blocks, int block_size, int window, int cus) {
     if (block_size % kPlanShortTile != 0 || batch > kPlanWaveScanBatch || h.hkv > 65535 || h.d_pad < 64) return 0;
@@ -225,10 +229,12 @@ PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, 
         if (runs < 1) runs = 1;
     }
     const int64_t row = (int64_t)h.d_pad * kv_elem_bytes, kb = 1024;
-    const int64_t run_most = h.n_rep > 4 ? (kv_elem_bytes == 1 ? 4096 * row : row <= 128 ? 512 * kb : 256 * kb) : h.n_rep > 2 ? 128 * kb : 64 * kb;
-    const int64_t all_most = h.n_rep > 4 ? (int64_t)1 << 62 : (h.n_rep > 2 ? 128 : 64) * kb * kb;
+    const int64_t wide_most = row > 128 || h.hpw == 4 ? 256 * kb : h.hpw == 1 ? 512 * kb : h.hpw == 2 ? 384 * kb : 208 * kb;
+    const int64_t run_most = h.n_rep > 4 ? (kv_elem_bytes == 1 ? 4096 * row : wide_most) : h.n_rep > 2 ? 128 * kb : 64 * kb;
+    const int64_t all_most = h.n_rep > 4 ? (int64_t)1 << 62 : (h.n_rep > 2 ? 64 : 32) * kv_elem_bytes * kb * kb;
     const bool few = h.n_rep <= 4 && wgs < 6 && keys > 4096;
-    const bool fits = (brief || keys / runs * row <= run_most) && wgs * keys * row <= all_most && !few;
+    const bool thin = kv_elem_bytes == 1 && h.d_pad == 64 && h.n_rep <= 2 && keys / runs > 768;
+    const bool fits = (brief || keys / runs * row <= run_most) && wgs * keys * row <= all_most && !few && !thin;
     return fits && runs * reps <= 65535 ? (int)runs : 0;
 }
 

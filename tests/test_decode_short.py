@@ -44,7 +44,10 @@ def test_lines_of_the_rule(plan):
     assert runs(1, wide, 592) == 1 and runs(1, wide, 608) == 4 and runs(1, wide, 4096) == 32 and runs(4, wide, 4096) == 8
     assert runs(16, wide, 1024) == 3 and runs(32, wide, 608) == 0 and runs(32, wide, 592) == 1 and runs(256, wide, 256) == 1 and runs(256, wide, 272) == 0
     assert runs(4, wide, 4096 + 16) == 0 and runs(1, wide, 1 << 20) == 0                      # long runs: the split pass
-    assert runs(1, many, 16384) == 64 and runs(256, many, 4096) == 1 and runs(256, many, 4112) == 0
+    assert runs(1, many, 16384) == 64 and runs(256, many, 3072) == 1 and runs(256, many, 3088) == 0
+    four, eight, one8, two8 = (28, 4, 64, 2), (56, 8, 64, 2), (8, 8, 64, 1), (32, 16, 64, 1)  # (kv heads that a wave of the split pass takes at once)
+    assert runs(256, four, 2048) == 1 and runs(256, four, 2064) == 0 and runs(256, eight, 1664) == 1 and runs(256, eight, 1680) == 0
+    assert runs(64, one8, 768) == 1 and runs(64, one8, 784) == 0 and runs(64, two8, 512) == 1 and runs(64, two8, 528) == 0  # (32 MB in all)
     assert runs(16, fp8, 2048) == 3 and runs(1, one, 1200) == 1 and runs(96, one, 1216) == 0
     assert runs(1, wide, 1 << 20, window=500) == 1 and runs(1, wide, 1 << 20, window=-1024) == 8
     assert runs(4, wide, 64, bs=8) == 0 and runs(4, wide, 96, bs=48) == 1 and runs(513, wide, 16) == 0 and runs(4, wide, 0) == 1
