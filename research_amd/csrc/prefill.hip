@@ -152,7 +152,7 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
             const int row_blocks = (max_q_len + kPfRows - 1) / kPfRows;
             const int64_t groups = (row_blocks * (int64_t)a.p.n_rep + kPfTasks - 1) / kPfTasks;
             const int gpw = plan_groups_per_workgroup(num_kv_heads, groups, batch, prefill_cus());
-            a.groups_per_wg = plan_ragged_groups(gpw, num_kv_heads, batch, total_q, max_q_len, kPfTasks * kPfRows / a.p.n_rep,
+            a.groups_per_wg = plan_ragged_groups(gpw, groups, num_kv_heads, batch, total_q, max_q_len, kPfTasks * kPfRows / a.p.n_rep,
                                                  bt_stride * (int64_t)block_size, kPfKeys, prefill_cus());
         }
     }

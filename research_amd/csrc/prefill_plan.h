@@ -71,14 +71,15 @@ PA_PLAN_FN int plan_groups_per_workgroup(int num_kv_heads, int64_t groups, int b
 // 14 / 2 heads of 64, 64 of 5 .. 100 rows behind 2000 keys 70 -> 42.
 // Prompts whose rows are 7 / 8 of the longest's or more on average, and calls that do not know (rows <= 0), keep `most`; so do pairs, which
 // leave little to spread (16 / 8 heads of 64, 64 prompts of 30 .. 250 rows behind 512 keys: 69 us, one by one 70).
-PA_PLAN_FN int plan_ragged_groups(int most, int num_kv_heads, int batch, int64_t rows, int64_t max_q_len, int64_t rows_per_group,
+// Never so few that the longest prompt's `groups` need more than the 65535 workgroups a launch has along y.
+PA_PLAN_FN int plan_ragged_groups(int most, int64_t groups, int num_kv_heads, int batch, int64_t rows, int64_t max_q_len, int64_t rows_per_group,
                                   int64_t max_keys, int tile_keys, int cus) {
     if (most <= 2 || rows <= 0 || 8 * rows >= 7 * max_q_len * batch) return most;
     const int64_t units = num_kv_heads * (rows / (rows_per_group > 0 ? rows_per_group : 1) + (batch + 1) / 2);  // (a last group is half full)
     const int64_t behind = max_keys > max_q_len ? max_keys - max_q_len : 0;          // keys before a prompt's own rows
     const int64_t c = (behind + max_q_len / 2) / tile_keys + 3;                      // tiles, and what a group costs beside its loop
     int g = 1;
-    while (g < most && 5 * (int64_t)(g + 1) * (g + 1) * c * cus <= 11 * units) ++g;
+    while (g < most && (5 * (int64_t)(g + 1) * (g + 1) * c * cus <= 11 * units || (groups + g - 1) / g > 65535)) ++g;
     return g;
 }
 

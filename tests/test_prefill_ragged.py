@@ -14,8 +14,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
 #include "prefill_plan.h"
 using namespace pa_decode_detail;
-extern "C" int ragged(int most, int hkv, int batch, long long rows, long long max_q, long long per, long long keys) {
-    return plan_ragged_groups(most, hkv, batch, rows, max_q, per, keys, 64, 256);
+extern "C" int ragged(int most, int hkv, int batch, long long rows, long long max_q, long long per, long long keys, long long groups) {
+    return plan_ragged_groups(most, groups, hkv, batch, rows, max_q, per, keys, 64, 256);
 }
 """
 
@@ -27,8 +27,8 @@ def ragged(tmp_path_factory):
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "research_amd", "csrc"), "-o", str(at / "r.so"),
                     str(at / "r.cpp")], check=True)
     fn = ctypes.CDLL(str(at / "r.so")).ragged
-    fn.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong] * 4
-    return fn
+    fn.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong] * 5
+    return lambda *args, groups=1: fn(*args, groups)
 
 
 def test_lines_of_the_rule(ragged):
@@ -39,6 +39,9 @@ def test_lines_of_the_rule(ragged):
     assert ragged(1, 8, 64, 64, 512, 64, 512) == 1 and ragged(2, 8, 64, 64, 512, 64, 512) == 2 and ragged(3, 8, 64, 64, 512, 64, 512) == 1
     assert ragged(8, 8, 1024, 1024 * 100, 250, 64, 256) in (4, 5, 6, 7)  # hundreds of groups a unit: set-ups count again
     assert ragged(8, 1 << 20, 65535, 1, 65535, 0, 1 << 40) >= 1     # (no overflow, no division by nothing)
+    # 300 query heads on one kv head, prompts of 65535 and 10 rows: 76800 groups, of which a launch takes no more than 65535 workgroups
+    assert ragged(8, 1, 2, 65545, 65535, 0, 65536, groups=65535) == 1 and ragged(8, 1, 2, 65545, 65535, 0, 65536, groups=76800) == 2
+    assert ragged(8, 1, 2, 65545, 65535, 0, 65536, groups=65535 * 8) == 8
     for rows in range(1, 64 * 512, 997):
         assert 1 <= ragged(5, 8, 64, rows, 512, 36, 4096) <= 5
 
