@@ -93,6 +93,7 @@ struct RowwiseArgs {
     // prefill_asm_kernel without lower bounds: groups of 8 tasks one workgroup runs in turn (grid.y = chunks of that
     // many groups); 1 everywhere else.
     int groups_per_wg;
+    int turned;  // there: chunks take turns over the sequences (plan_turned_chunk; unequal prompts)
 };
 
 __device__ __forceinline__ uint4 ld16(const void *p) { return *reinterpret_cast<const uint4 *>(p); }

@@ -106,7 +106,7 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
     a.q = q; a.out = out; a.ctx_lens = ctx_lens; a.q_lens = q_lens; a.q_starts = q_starts;
     a.row_lo = row_first_key;
     a.batch = batch; a.max_q_len = max_q_len;
-    a.splits = 1; a.part_o = nullptr; a.part_ml = nullptr; a.groups_per_wg = 1;
+    a.splits = 1; a.part_o = nullptr; a.part_ml = nullptr; a.groups_per_wg = 1; a.turned = 0;
     hipStream_t s = (hipStream_t)stream;
     // bf16 / fp16 with head_dim 32, 64, 128 (and 256, below) run on the matrix cores unless the caller asked for the
     // vector kernel
@@ -154,6 +154,7 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
             const int gpw = plan_groups_per_workgroup(num_kv_heads, groups, batch, prefill_cus());
             a.groups_per_wg = plan_ragged_groups(gpw, groups, num_kv_heads, batch, total_q, max_q_len, kPfTasks * kPfRows / a.p.n_rep,
                                                  bt_stride * (int64_t)block_size, kPfKeys, prefill_cus());
+            a.turned = a.groups_per_wg < gpw ? 1 : 0;
         }
     }
     // head_dim 256: one 32-row task per wave, loads driven by a table of 16-key groups - which must lie inside one

@@ -77,7 +77,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
     const int n_chunks = gridDim.y / n_splits, n_seqs = gridDim.z;
     const int lin = chunk_y + n_chunks * blockIdx.z;
     const bool group_major = a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];
-    const int wg_chunk = group_major ? n_chunks - 1 - lin / n_seqs : chunk_y;
+    const int turned = (LO || LONG) || !a.turned ? chunk_y : plan_turned_chunk(chunk_y, (int)blockIdx.z, n_chunks);
+    const int wg_chunk = group_major ? n_chunks - 1 - lin / n_seqs : turned;
     const int b = group_major ? lin % n_seqs : (int)blockIdx.z;
     // (read once and held in scalar registers: a load behind the direct-to-LDS requests would wait for all of them)
     const int q_len = __builtin_amdgcn_readfirstlane(a.q_lens[b]);

@@ -64,11 +64,14 @@ PA_PLAN_FN int plan_groups_per_workgroup(int num_kv_heads, int64_t groups, int b
 
 // The same for prompts of unequal length, given the `rows` of q of all of them: of the groups that equal prompts would share a set-up
 // for, the longest prompt's keep one compute unit at work while others have none left.  A launch of U groups, each c tiles of time, takes
-// about (U / cus) (c + s / g) + g c / 2, of which s is a workgroup's set-up and the last term the wait for the workgroups that end
-// last: least at g^2 = 2 s U / (c cus).  s measures 1.1 tiles (equal prompts, 1 against 4 groups: 32 of 256 rows behind 2048 keys 268 and
-// 261 us; 1 against 8: 64 of 512 rows 316 and 284 us).  us, as for equal prompts -> this: 32 / 8 heads of 128, 16 prompts of 64 ..
-// 1024 rows behind 512 keys 172 -> 104, 32 of 97 .. 512 rows 108 -> 81, 64 of 30 .. 250 rows 78 -> 68, of 200 .. 512 rows 214 -> 212;
-// 14 / 2 heads of 64, 64 of 5 .. 100 rows behind 2000 keys 70 -> 42.
+// about (U / cus) (c + s / g) + g c e, of which s is a workgroup's set-up and the last term the wait for the workgroups that end
+// last, with e the part of the longest prompt's rows that the others lack on average: least at g^2 = s U / (c cus e).  s measures 1.1 tiles (equal
+// prompts, 1 against 4 groups: 32 of 256 rows behind 2048 keys 268 and 261 us; 1 against 8: 64 of 512 rows 316 and 284 us).
+// us, as for equal prompts -> this: 32 / 8 heads of 128, 16 prompts of 64 .. 1024 rows behind 512 keys 196 -> 144 and 200 -> 127 (two batches), 32 of 97
+// .. 512 rows 98 -> 81 and 96 -> 71, 57 of 26 .. 239 behind 1696 278 -> 229, 64 of 30 .. 250 rows 60 -> 59 and 67 -> 68; 14 / 2 heads of 128, 82 of 12 ..
+// 122 rows behind 3824 keys 242 -> 177; 8 / 2, 65 of 64 .. 227 behind 1616 90 -> 88 and 124 -> 88.  Of 8200 batches (1 to 100 prompts of up to 2048 rows, behind
+// nothing or up to 4096 keys), which took 0.95 of the time on average, 80 were slower by more than 2 %, one by more than a sixth (where the
+// former groups happen to fill the device: 16 / 8 heads of 128, 30 of 49 .. 392 rows behind 32 keys 32.6 -> 39.4).
 // Prompts whose rows are 7 / 8 of the longest's or more on average, and calls that do not know (rows <= 0), keep `most`; so do pairs, which
 // leave little to spread (16 / 8 heads of 64, 64 prompts of 30 .. 250 rows behind 512 keys: 69 us, one by one 70).
 // Never so few that the longest prompt's `groups` need more than the 65535 workgroups a launch has along y.
@@ -79,8 +82,18 @@ PA_PLAN_FN int plan_ragged_groups(int most, int64_t groups, int num_kv_heads, in
     const int64_t behind = max_keys > max_q_len ? max_keys - max_q_len : 0;          // keys before a prompt's own rows
     const int64_t c = (behind + max_q_len / 2) / tile_keys + 3;                      // tiles, and what a group costs beside its loop
     int g = 1;
-    while (g < most && (5 * (int64_t)(g + 1) * (g + 1) * c * cus <= 11 * units || (groups + g - 1) / g > 65535)) ++g;
+    const double even = 1.1 * (double)units / ((double)c * cus * (1.0 - (double)rows / ((double)max_q_len * batch)));
+    while (g < most && ((g + 1) * (g + 1) <= even || (groups + g - 1) / g > 65535)) ++g;
     return g;
+}
+
+// Which chunk of sequence `b` workgroup `y` of its n_chunks takes.  Workgroups go to the eight dies, and inside one to its shader engines, in turn, so
+// with the same chunk for the same y and an even number of them the first chunks, which every sequence has, would meet on a few of those while
+// the last ones, which only long sequences have, leave the rest idle.  The sum of b's digits to the base four moves them on.
+// (us, one group a workgroup, 4 chunks: 32 / 8 heads of 64, 49 prompts of 24 .. 213 rows behind 624 keys 109 -> 69; 14 / 2 of 128, 82 of 12 .. 122 behind
+// 3824 272 -> 177; 8 / 2 of 128, 65 of 64 .. 227 behind 1616 133 -> 88)
+PA_PLAN_FN int plan_turned_chunk(int y, int b, int n_chunks) {
+    return n_chunks & 1 ? y : (y + b + (b >> 2) + (b >> 4) + (b >> 6)) % n_chunks;
 }
 
 // The i-th group of the workgroup that is chunk `wg_chunk` of `n_chunks`: one of every n_chunks consecutive groups,

@@ -17,6 +17,7 @@ using namespace pa_decode_detail;
 extern "C" int ragged(int most, int hkv, int batch, long long rows, long long max_q, long long per, long long keys, long long groups) {
     return plan_ragged_groups(most, groups, hkv, batch, rows, max_q, per, keys, 64, 256);
 }
+extern "C" int turned(int y, int b, int n_chunks) { return plan_turned_chunk(y, b, n_chunks); }
 """
 
 
@@ -31,6 +32,12 @@ def ragged(tmp_path_factory):
     return lambda *args, groups=1: fn(*args, groups)
 
 
+@pytest.fixture(scope="module")
+def turned(ragged, tmp_path_factory):
+    fn = ctypes.CDLL(str(tmp_path_factory.getbasetemp() / "ragged0" / "r.so")).turned
+    return fn
+
+
 def test_lines_of_the_rule(ragged):
     assert ragged(8, 8, 64, 64 * 512, 512, 64, 512) == 8            # equal
     assert ragged(4, 8, 32, 32 * 224, 256, 64, 2304) == 4           # seven eighths
@@ -42,8 +49,25 @@ def test_lines_of_the_rule(ragged):
     # 300 query heads on one kv head, prompts of 65535 and 10 rows: 76800 groups, of which a launch takes no more than 65535 workgroups
     assert ragged(8, 1, 2, 65545, 65535, 0, 65536, groups=65535) == 1 and ragged(8, 1, 2, 65545, 65535, 0, 65536, groups=76800) == 2
     assert ragged(8, 1, 2, 65545, 65535, 0, 65536, groups=65535 * 8) == 8
+    # nearly equal ones wait less for the last: three groups of 64 prompts of 153 rows on average, the longest 182; of 100 rows one
+    assert ragged(3, 8, 64, 64 * 153, 182, 64, 192) == 3 and ragged(3, 8, 64, 64 * 100, 182, 64, 192) == 1
     for rows in range(1, 64 * 512, 997):
         assert 1 <= ragged(5, 8, 64, rows, 512, 36, 4096) <= 5
+
+
+@pytest.mark.parametrize("kv_heads,chunks", [(8, 4), (2, 4), (2, 3), (1, 4), (4, 4), (8, 2), (16, 3), (1, 8), (2, 16), (1, 5), (3, 6)])
+def test_first_chunks_spread_over_the_turns(turned, kv_heads, chunks):
+    """Workgroups go to eight dies in turn and, in a die, to four engines: each gets its share of the chunks that every sequence has."""
+    seqs = 128
+    first = np.zeros((8, 4), int)
+    for z in range(seqs):
+        assert sorted(turned(y, z, chunks) for y in range(chunks)) == list(range(chunks))
+        for y in range(chunks):
+            for x in range(kv_heads):
+                at = x + kv_heads * (y + chunks * z)
+                first[at % 8, at // 8 % 4] += turned(y, z, chunks) == 0
+    mean = kv_heads * seqs / 32
+    assert first.max() <= 2 * mean, first  # (up to sixteen times the mean with the same chunk for the same y)
 
 
 @pytest.mark.gpu
