@@ -41,8 +41,9 @@ __device__ __forceinline__ bool cl_portion(const ClArgs &a, int b, ClPortion &p)
     return p.n > 0 && p.pos0 >= 0 && p.row0 >= 0 && p.row0 + p.n <= a.n_rows;
 }
 
-// f and 1 - f, neither by subtraction from one, of 16-bit logits; x: -log2(e) times the logit.  (Past 2^115 f is its lower bound in 32 bits
-// either way, and the product with e would not be finite.  NaN stays NaN.)
+// f and 1 - f, neither by subtraction from one, of 16-bit logits; x: -log2(e) times the logit.  (Past 2^115 the product with e would not be finite at
+// some point: f stays at 2^-115 of the way from its lower bound to one.  With a bound of zero that is what is left of a state that a smaller
+// factor would have to leave nothing of; a block with such a factor takes its scores token by token, as all below kClSmall.  NaN stays NaN.)
 constexpr float kClLog2e = 1.4426950408889634f;
 __device__ __forceinline__ void cl_gate16(float x, float lower, float &f, float &k) {
     const float e = __builtin_amdgcn_exp2f(__builtin_elementwise_minimum(x, 115.f));
