@@ -196,7 +196,7 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 
 // How decode_short.h's kernel takes the launch: 0: not at all; else the runs a sequence's tiles are cut into, a workgroup per (kv head, sequence,
 // run).  From shapes alone; the tables' width stands for the longest sequence.
-// Head sizes up to 32 stay with the generic loop of the split pass, whose weights have 32 bits: 11.1 us for 16 sequences of 16 .. 250 keys, 4 / 4
+// Head sizes up to 32 stay with the generic loop of the split pass, whose weights have 32 bits: 11.8 us for 16 sequences of 16 .. 250 keys, 4 / 4
 // heads of 32, where weights of two bf16 terms took 5.0, but erred by up to 1.1e-6 of the sum of |weight value| where 32 bits err by 0.2e-6.
 // Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (3.5 us: 600 keys of 128).
 // us, the split pass (one launch or two) -> this, sequences of n keys each: 32 / 8 heads of 128, 1 of 256 keys 14.1 -> 7.4, 1024 15.5 -> 9.0, 4096
