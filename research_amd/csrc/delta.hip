@@ -14,6 +14,7 @@
 // diagonal row by row and joining them with 32-bit matrix products).  The second pass walks a portion's chunks with S in
 // accumulator registers; a wave owns value columns, which do not depend on each other.  Unit norms are factors of rows,
 // so q and k enter the products as they are stored; T, C, S, U and V - e^F K S are split into two bf16 terms each.
+#include <type_traits>
 #include "linear_tiles.h"
 
 namespace {
@@ -150,14 +151,24 @@ template <typename T, int R> __global__ __launch_bounds__(256, 4) void delta_rec
 }
 
 // ------------------------------------------------------------------ chunks: T and C
-struct DeltaChunk {           // what the first pass leaves per chunk and head (columns of T and C paired)
-    uint16_t t_hi[64][64], t_lo[64][64], c_hi[64][64], c_lo[64][64];
+// What the first pass leaves per chunk and head.  T and C lie as the walk's operands: piece f (rows 16 tt .., columns 32 kk ..) holds for
+// lane 16 g + l16 the eight elements of row l16 in the paired order, so that a wave reads and writes whole lines; the quarter above the
+// diagonal blocks of 32, all zeros, is left out.
+constexpr int kDeltaPieces = 6;
+__host__ __device__ constexpr int delta_piece(int tt, int kk) { return kk ? 2 + tt : tt; }
+struct DeltaChunk {
+    uint16_t t[2][kDeltaPieces][64][8], c[2][kDeltaPieces][64][8];  // both terms of each
     float k_in[64];   // e^F times k's unit factor (on K S)
     float q_in[64];   // e^F times q's unit factor and scale (on Q S)
     float k_out[64];  // e^(F_last - F) times k's unit factor (on U in the new state)
     float keep;       // e^(F_last)
     float pad[63];
 };
+constexpr int kDeltaMat = 2 * kDeltaPieces * 64 * 8;  // elements of T, of C
+// Operand of a matrix in LDS
+__device__ __forceinline__ bf8 delta_operand(const __bf16 *m, int term, int tt, int kk, int lane) {
+    return la_read8(m + ((term * kDeltaPieces + delta_piece(tt, kk)) * 64 + lane) * 8);
+}
 
 __device__ __forceinline__ f4 delta_mfma32(float x, float y, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
 
@@ -259,21 +270,22 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
     __syncthreads();
     const int t = 16 * wave + l16;
     const float ft = f_s[t], bt = beta_s[t] * kn_s[t], qt = qn_s[t];
+    f4 c[4];
 #pragma unroll
-    for (int st = 0; st < 4; ++st) {
-        float c[4];
+    for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int s = 16 * st + 4 * g + i;
             const float w = s <= t ? __builtin_amdgcn_exp2f(ft - f_s[s]) * kn_s[s] : 0.f;
             mat[t][s] = s < t ? kk[st][i] * w * bt : 0.f;
-            c[i] = qk[st][i] * w * qt;
+            c[st][i] = qk[st][i] * w * qt;
         }
-        uint2 hi, lo;
-        la_split2(c[0], c[1], hi.x, lo.x);
-        la_split2(c[2], c[3], hi.y, lo.y);
-        *reinterpret_cast<uint2 *>(&out->c_hi[t][la_paired(16 * st + 4 * g)]) = hi;
-        *reinterpret_cast<uint2 *>(&out->c_lo[t][la_paired(16 * st + 4 * g)]) = lo;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (half && wave < 2) continue;
+        const LaSplit x = la_split_pair(c[2 * half], c[2 * half + 1]);
+        *reinterpret_cast<bf8 *>(out->c[0][delta_piece(wave, half)][lane]) = x.high();
+        *reinterpret_cast<bf8 *>(out->c[1][delta_piece(wave, half)][lane]) = x.low();
     }
     // (the wave's own 16 rows of mat: its accesses are in order, the compiler must keep them so)
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -312,16 +324,17 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
         }
         __syncthreads();
     }
-    for (int i = tid; i < 64 * 16; i += 256) {
-        const int r = i / 16, c = i % 16 * 4;
-        float x[4];
+    for (int i = tid; i < kDeltaPieces * 64; i += 256) {
+        const int f = i / 64, tt = f < 4 ? f : f - 2, half = f / 4, r = 16 * tt + l16, col = 32 * half + 4 * g;
+        f4 x, y;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = c / 16 <= r / 16 ? inv[r][c + e] * beta_s[c + e] : 0.f;
-        uint2 hi, lo;
-        la_split2(x[0], x[1], hi.x, lo.x);
-        la_split2(x[2], x[3], hi.y, lo.y);
-        *reinterpret_cast<uint2 *>(&out->t_hi[r][la_paired(c)]) = hi;
-        *reinterpret_cast<uint2 *>(&out->t_lo[r][la_paired(c)]) = lo;
+        for (int e = 0; e < 4; ++e) {
+            x[e] = 2 * half <= tt ? inv[r][col + e] * beta_s[col + e] : 0.f;
+            y[e] = 2 * half < tt ? inv[r][col + 16 + e] * beta_s[col + 16 + e] : 0.f;
+        }
+        const LaSplit z = la_split_pair(x, y);
+        *reinterpret_cast<bf8 *>(out->t[0][f][lane]) = z.high();
+        *reinterpret_cast<bf8 *>(out->t[1][f][lane]) = z.low();
     }
 }
 
@@ -332,7 +345,7 @@ template <int KD> __global__ __launch_bounds__(256, KD == 256 ? 2 : 4) void delt
 // walk then lacks registers).  8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128: 273 -> 187 us; eight waves a workgroup, whose
 // SIMDs have two each: 32 prompts of about 900 rows, with the first pass, 324 -> 311.
 template <int KD, int COLS> constexpr size_t delta_walk_lds() {
-    return (size_t)(2 * 64 * KD + 64 * (COLS + kLaPadV) + 4 * 64 * 64) * 2 + 3 * 64 * 4 + 64;
+    return (size_t)(2 * 64 * KD + 64 * (COLS + kLaPadV) + 2 * kDeltaMat) * 2 + 3 * 64 * 4 + 64;
 }
 
 // KD: dim padded to 64, 128 or 256.  A workgroup of NW waves owns 16 NW value columns of a head and all chunks of a portion.
@@ -340,15 +353,15 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
     constexpr int kCols = 16 * NW, kThr = 64 * NW, kLv = kCols + kLaPadV;
     constexpr int kBlocks = 16 * (KD / 4), kKB = (kBlocks + kThr - 1) / kThr;  // 4 x 4 blocks of K, of V; 16-byte pieces of T and C
     constexpr bool kFew = NW < 8;  // a SIMD has one wave: all its registers
-    constexpr int kVB = 16 * (kCols / 4) / kThr, kMB = 4 * (kFew ? 48 : 64) * 8 / kThr;
+    constexpr int kVB = 16 * (kCols / 4) / kThr, kMB = 2 * kDeltaMat / 8 / kThr;
     constexpr int kSteps = kFew && KD > 64 ? 1 : 2;  // parts of the next chunk's loads beside a product of 32 columns
-    static_assert(16 * (kCols / 4) % kThr == 0 && (kBlocks % kThr == 0 || kKB == 1), "whole passes");
+    static_assert(16 * (kCols / 4) % kThr == 0 && (kBlocks % kThr == 0 || kKB == 1) && 2 * kDeltaMat / 8 % kThr == 0, "whole passes");
     const bool k_live = kBlocks >= kThr || (int)threadIdx.x < kBlocks;
     extern __shared__ __align__(16) char lds[];
     __bf16 *q_s = reinterpret_cast<__bf16 *>(lds), *k_s = q_s + 64 * KD, *v_s = k_s + 64 * KD;
-    __bf16 *m_s = v_s + 64 * kLv;  // T's two terms, C's two terms
-    float *rows = reinterpret_cast<float *>(m_s + 4 * 64 * 64);  // k_in, q_in, k_out
-    const __bf16 *t_hi = m_s, *t_lo = m_s + 64 * 64, *c_hi = m_s + 2 * 64 * 64, *c_lo = m_s + 3 * 64 * 64;
+    __bf16 *m_s = v_s + 64 * kLv;  // T, C
+    float *rows = reinterpret_cast<float *>(m_s + 2 * kDeltaMat);  // k_in, q_in, k_out
+    const __bf16 *t_s = m_s, *c_s = m_s + kDeltaMat;
     const int h = blockIdx.x, v0 = blockIdx.y * kCols, b = blockIdx.z;
     DeltaPortion p;
     if (!delta_portion(a, b, p)) return;
@@ -380,13 +393,6 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
     // (with too few registers places in memory are worked out again: 48 heads of 128 x 128, 8 prompts of 900 .. 1000 rows, 257 us, else
     // 328; of 64 x 128, which has them, 216, else 225)
     auto again = [](int x) { return kFew || KD == 64 ? x : la_again(x); };
-    // 16-byte piece `at` of T's and C's terms: its row of the four, its column.  A wave with registers for its places leaves out the
-    // quarter above the diagonal blocks of 32.
-    auto piece = [](int at, int &row, int &col) {
-        const int r = at % 384;
-        row = !kFew ? at / 8 : at / 384 * 64 + (r < 128 ? r / 4 : 16 + r / 8);
-        col = !kFew ? at % 8 : r < 128 ? r % 4 : r % 8;
-    };
     // Tiles in eight parts: loads all at once would hold up a wave for longer than it computes.
     auto fetch = [&](int part, int r0) {
         if (r0 >= p.n) return;
@@ -397,9 +403,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
 #pragma unroll
             for (int i = 0; i < kMB; ++i) {
                 if (i * 2 / kMB != part) continue;
-                int row, col;
-                piece(ft + kThr * i, row, col);
-                mb[i] = reinterpret_cast<const la_u4 *>(m)[row * 8 + col];
+                mb[i] = reinterpret_cast<const la_u4 *>(m)[ft + kThr * i];
             }
         } else if (part < 6) {
             const bool keys = part < 4;
@@ -431,11 +435,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         const int lt = again(tid);  // (written in the order of loading)
         const int nv = p.n - r0 < 64 ? p.n - r0 : 64;
 #pragma unroll
-        for (int i = 0; i < kMB; ++i) {
-            int row, col;
-            piece(lt + kThr * i, row, col);
-            *reinterpret_cast<la_u4 *>(m_s + row * 64 + (col ^ la_hash<64>(row)) * 8) = mb[i];
-        }
+        for (int i = 0; i < kMB; ++i) reinterpret_cast<la_u4 *>(m_s)[lt + kThr * i] = mb[i];
 #pragma unroll
         for (int i = 0; i < kKB; ++i) {
             const int blk = lt + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
@@ -475,7 +475,7 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
                 xq[dd & 1][tt] = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
             }
         };
-        auto mat = [&](const __bf16 *m, int tt, int kk) { return la_read_hashed<64>(m, 16 * tt + l16, 4 * kk + g); };
+        auto mat = [&](const __bf16 *m, int term, int tt, int kk) { return delta_operand(m, term, tt, kk, lr); };
         read_rows(0);
 #pragma unroll
         for (int dd = 0; dd < KD / 32; ++dd) {
@@ -507,8 +507,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         }
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
-            th[tt] = mat(t_hi, tt, 0);
-            tl[tt] = mat(t_lo, tt, 0);
+            th[tt] = mat(t_s, 0, tt, 0);
+            tl[tt] = mat(t_s, 1, tt, 0);
         }
         fetch(4, r0 + 64);
         if constexpr (!kFew) fetch(5, r0 + 64);
@@ -526,8 +526,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         for (int tt = 0; tt < 4; ++tt) w[tt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
-            th2[tt] = mat(t_hi, 2 + tt, 1);
-            tl2[tt] = mat(t_lo, 2 + tt, 1);
+            th2[tt] = mat(t_s, 0, 2 + tt, 1);
+            tl2[tt] = mat(t_s, 1, 2 + tt, 1);
         }
         f4 ko[4];
 #pragma unroll
@@ -546,8 +546,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         bf8 ch[4], cl[4], kt[KD / 16];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
-            ch[tt] = mat(c_hi, tt, 0);
-            cl[tt] = mat(c_lo, tt, 0);
+            ch[tt] = mat(c_s, 0, tt, 0);
+            cl[tt] = mat(c_s, 1, tt, 0);
         }
         ahead();
 #pragma unroll
@@ -582,8 +582,8 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
             if (kk == 0) {
 #pragma unroll
                 for (int tt = 2; tt < 4; ++tt) {
-                    ch[tt] = mat(c_hi, tt, 1);
-                    cl[tt] = mat(c_lo, tt, 1);
+                    ch[tt] = mat(c_s, 0, tt, 1);
+                    cl[tt] = mat(c_s, 1, tt, 1);
                 }
             }
 #pragma unroll
@@ -612,6 +612,326 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         }
 }
 
+// The same walk with its chain and its outputs in different waves.  What a chunk hands to the next one, K S, the system and the new state, is
+// half of its products; as one wave's instructions the other half, Q S, C U, the loads and the stores, lengthen the chain by as much again.
+// So waves 0 .. NW - 1 follow the state, and wave NW + w makes wave w's outputs beside it on the same SIMD: it gets the state's terms and
+// U's through LDS, each lane what the same lane wrote, and the waves of that half bring the tiles.  Two barriers a chunk: until the first
+// one the state's terms, T, V and Q are read (and C written), from there on U's terms and C; K, read in both parts, is there twice.
+// A chunk takes 5600 cycles, about half of them before the first barrier: the waits for LDS and for the other half's products (a SIMD has 2100
+// cycles of them) there, the new state and its split behind.  The loads must be out before the products of their part (behind them: 0.3 us a
+// chunk); operands of T and C straight from memory, or a word of every line touched four chunks ahead, make the requests the limit (239 and
+// 257 us, else 215).
+// 8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128, both passes and two tokens: 245 -> 215 us (one wave a SIMD -> this); 3 prompts of 326 .. 492 rows, 8
+// heads of 96 x 80, 39.7 -> 32.0; 63 of 200 .. 250, 32 heads of 128 x 64, 273 -> 241.
+template <int KD, int NW> constexpr size_t delta_pair_lds() {
+    return (size_t)(3 * 64 * KD + 64 * (16 * NW + kLaPadV) + 2 * kDeltaMat) * 2 + (size_t)NW * (KD / 32 + 2) * 2048;
+}
+
+// KD: dim padded to 64 or 128.  A workgroup of 2 NW waves owns 16 NW value columns of a head and all chunks of a portion.  Rows come in
+// 16-byte pieces (dim, vdim and strides multiples of 8, 16-byte aligned rows).
+template <int KD, int NW> __global__ __launch_bounds__(128 * NW, 1) void delta_pair_kernel(const DeltaArgs a) {
+    constexpr int kCols = 16 * NW, kThr = 64 * NW, kLv = kCols + kLaPadV, kD = KD / 32;
+    constexpr int kKB = 64 * (KD / 8) / kThr, kVB = 64 * (kCols / 8) / kThr, kMB = kDeltaMat / 8 / kThr;  // 16-byte pieces per thread of half the workgroup
+    static_assert(64 * (KD / 8) % kThr == 0 && 64 * (kCols / 8) % kThr == 0 && kDeltaMat / 8 % kThr == 0, "whole passes");
+    constexpr int kTerms = 64 * 8;  // elements of an operand of a wave
+    extern __shared__ __align__(16) char lds[];
+    __bf16 *k2_s = reinterpret_cast<__bf16 *>(lds), *q_s = k2_s + 2 * 64 * KD, *v_s = q_s + 64 * KD;
+    __bf16 *t_s = v_s + 64 * kLv, *c_s = t_s + kDeltaMat, *s_s = c_s + kDeltaMat, *u_s = s_s + NW * kD * 2 * kTerms;
+    const int h = blockIdx.x, v0 = blockIdx.y * kCols, b = blockIdx.z;
+    DeltaPortion p;
+    if (!delta_portion(a, b, p)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = tid & 15, g = lane >> 4;
+    const int pair = wave % NW, vw = pair * 16, chunks = (p.n + 63) / 64;
+    // terms [pair][operand][hi, lo][lane]
+    s_s += pair * kD * 2 * kTerms + lane * 8;
+    u_s += pair * 2 * 2 * kTerms + lane * 8;
+    auto mat = [&](const __bf16 *m, int term, int tt, int kk) { return delta_operand(m, term, tt, kk, lane); };
+    const int vcols = a.vdim - v0 < kCols ? a.vdim - v0 : kCols, grp = h / a.per_group;
+    const DeltaChunk *first = reinterpret_cast<const DeltaChunk *>(a.ws) + (int64_t)b * a.chunks * a.heads + h;
+    auto chunk = [&](int c) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(first + (int64_t)(c < chunks ? c : chunks - 1) * a.heads), 0, sizeof(DeltaChunk), 0x00020000);
+    };
+    if (wave < NW) {
+        __builtin_amdgcn_s_setprio(1);
+        // S: tile dt holds d = 32 (dt / 2) + 8 g + 4 (dt % 2) + i (the rows of K lie in LDS as they are), v = v0 + vw + l16
+        auto s_row = [](int dt, int i) { return 32 * (dt / 2) + 4 * (dt % 2) + i; };
+        f4 s[KD / 16];
+        const int64_t state_elems = (int64_t)a.dp * a.vp;
+        float *pool = p.slot >= 0 ? a.state + (p.slot * a.heads + h) * state_elems : nullptr;
+        const int v = v0 + vw + l16;
+        const uint32_t soff = v < a.vp ? (uint32_t)(8 * g * a.vp + v) * 4u : kLaOutside;
+        {
+            const float *from = p.pos0 > 0 ? pool : nullptr;
+            const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void *)(from ? from : a.state), 0, from ? (int)state_elems * 4 : 0, 0x00020000);
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + s_row(dt, i) * a.vp * 4, 0, 0));
+        }
+        f4 ki[4], ko[4];  // rows' factors, a chunk ahead
+        float keep;
+        auto four = [&](__amdgpu_buffer_rsrc_t x, size_t at, int tt) {
+            return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(x, g * 16, (int)at + 64 * tt, 0));
+        };
+        auto fetch_in = [&](__amdgpu_buffer_rsrc_t x) {
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) ki[tt] = four(x, offsetof(DeltaChunk, k_in), tt);
+            keep = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x, 0, (int)offsetof(DeltaChunk, keep), 0));
+        };
+        auto fetch_out = [&](__amdgpu_buffer_rsrc_t x) {
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) ko[tt] = four(x, offsetof(DeltaChunk, k_out), tt);
+        };
+        fetch_in(chunk(0));
+        fetch_out(chunk(0));
+        LaSplit sp[kD];
+        auto terms = [&](int dd) {
+            sp[dd] = la_split_pair(s[2 * dd], s[2 * dd + 1]);
+            *reinterpret_cast<bf8 *>(s_s + dd * 2 * kTerms) = sp[dd].high();
+            *reinterpret_cast<bf8 *>(s_s + dd * 2 * kTerms + kTerms) = sp[dd].low();
+        };
+        bf8 xk[2][4];
+        auto read_k = [&](const __bf16 *k_s, int dd) {
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) xk[dd & 1][tt] = la_read_hashed<KD>(k_s, 16 * tt + l16, 4 * dd + g);
+        };
+#pragma unroll
+        for (int dd = 0; dd < kD; ++dd) terms(dd);
+        __syncthreads();
+        read_k(k2_s, 0);
+        for (int c = 0; c < chunks; ++c) {  // (no branches inside: loads would be moved behind them, to their use)
+            const __bf16 *k_s = k2_s + (c & 1) * 64 * KD;
+            // K S (rows t = 16 tt + 4 g + i, columns v)
+            bf8 th[4], tl[4], th2[2], tl2[2];
+            la_bf4 vv[4];
+            f4 u[4];
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) u[tt] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int dd = 0; dd < kD; ++dd) {
+                if (dd + 1 < kD) {
+                    read_k(k_s, dd + 1);
+                } else {
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) vv[tt] = la_read_tr(v_s + (16 * tt + 4 * g + l16 / 4) * kLv + vw + l16 % 4 * 4);
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) {
+                        th[tt] = mat(t_s, 0, tt, 0);
+                        tl[tt] = mat(t_s, 1, tt, 0);
+                    }
+#pragma unroll
+                    for (int tt = 0; tt < 2; ++tt) {
+                        th2[tt] = mat(t_s, 0, 2 + tt, 1);
+                        tl2[tt] = mat(t_s, 1, 2 + tt, 1);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) u[tt] = la_mfma(xk[dd & 1][tt], sp[dd].high(), u[tt]);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) u[tt] = la_mfma(xk[dd & 1][tt], sp[dd].low(), u[tt]);
+            }
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[dt][i] *= keep;
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) u[tt][i] = (float)vv[tt][i] - ki[tt][i] * u[tt][i];
+            // U = T R
+            f4 w[4];
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) w[tt] = f4{0.f, 0.f, 0.f, 0.f};
+            auto times_t = [&](bf8 x, bf8 y, const LaSplit &r, f4 &to) {
+                to = la_mfma(x, r.high(), to);
+                to = la_mfma(x, r.low(), to);
+                to = la_mfma(y, r.high(), to);
+            };
+            const LaSplit r_lo = la_split_pair(u[0], u[1]), r_hi = la_split_pair(u[2], u[3]);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_in(chunk(c + 1));
+            bf8 kt[KD / 16];
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt) kt[dt] = la_read_paired_tr<KD>(k_s, 0, dt, l16, g);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) times_t(th[tt], tl[tt], r_lo, w[tt]);
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) times_t(th2[tt], tl2[tt], r_hi, w[2 + tt]);
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) *reinterpret_cast<f4 *>(u_s + tt * kTerms) = w[tt];
+            __syncthreads();
+            // S <- keep S + K^T (k_out U)
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) w[2 * kk + half][i] *= ko[2 * kk + half][i];
+                const LaSplit x = la_split_pair(w[2 * kk], w[2 * kk + 1]);
+                // (a group of tiles ends before the next one starts: its terms are made beside the others' products)
+                constexpr int kGroup = 4;
+#pragma unroll
+                for (int d0 = 0; d0 < KD / 16; d0 += kGroup) {
+#pragma unroll
+                    for (int dt = d0; dt < d0 + kGroup; ++dt) s[dt] = la_mfma(kt[dt], x.high(), s[dt]);
+#pragma unroll
+                    for (int dt = d0; dt < d0 + kGroup; ++dt) s[dt] = la_mfma(kt[dt], x.low(), s[dt]);
+#pragma unroll
+                    for (int dt = d0; dt < d0 + kGroup; ++dt)
+                        if (kk == 0) kt[dt] = la_read_paired_tr<KD>(k_s, 32, dt, l16, g);
+                    if (kk == 1 && d0 == 0) {
+                        read_k(k2_s + ((c + 1) & 1) * 64 * KD, 0);
+                        fetch_out(chunk(c + 1));
+                    }
+                    if (kk == 1)
+#pragma unroll
+                        for (int dd = d0 / 2; dd < (d0 + kGroup) / 2; ++dd) terms(dd);
+                }
+            }
+            __syncthreads();
+        }
+        if (!pool) return;
+        const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc((void *)pool, 0, (int)state_elems * 4, 0x00020000);
+#pragma unroll
+        for (int dt = 0; dt < KD / 16; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float f = s[dt][i];
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), dst, soff + s_row(dt, i) * a.vp * 4, 0, 0);
+            }
+        return;
+    }
+    const int ht = tid - kThr;  // thread of this half
+    const int ldo = a.heads * a.vdim;
+    const uint16_t *uq = reinterpret_cast<const uint16_t *>(a.q) + p.row0 * a.ldq + grp * a.dim;
+    const uint16_t *uk = reinterpret_cast<const uint16_t *>(a.k) + p.row0 * a.ldk + grp * a.dim;
+    const uint16_t *uv = reinterpret_cast<const uint16_t *>(a.v) + p.row0 * a.ldv + h * a.vdim + v0;
+    const uint16_t *uo = reinterpret_cast<const uint16_t *>(a.out) + p.row0 * ldo + h * a.vdim + v0;
+    auto tile = [&](const uint16_t *base, int64_t ld, int c, int cols) {  // a chunk's rows; none past the last
+        const int left = p.n - 64 * c, nr = left < 64 ? left : 64, bytes = ((nr - 1) * (int)ld + cols) * 2;
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(base + 64 * c * ld), 0, left > 0 ? bytes : 0, 0x00020000);
+    };
+    la_u4 kb[kKB], qb[kKB], vb[kVB], tb[kMB], cb[kMB];
+    // 16-byte pieces of rows of N elements
+    auto load_rows = [&](auto n, auto &x, const uint16_t *base, int64_t ld, int c, int cols) {
+        constexpr int N = decltype(n)::value, COUNT = sizeof(x) / sizeof(la_u4);
+        const __amdgpu_buffer_rsrc_t t = tile(base, ld, c, cols);
+        const int row = ht / (N / 8), col = ht % (N / 8) * 8;
+        const uint32_t off = la_block_off(ld, row, col, cols);
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i) x[i] = __builtin_bit_cast(la_u4, __builtin_amdgcn_raw_buffer_load_b128(t, off + i * (kThr / (N / 8)) * (int)ld * 2, 0, 0));
+    };
+    auto put_rows = [&](const la_u4 (&x)[kKB], __bf16 *to) {
+#pragma unroll
+        for (int i = 0; i < kKB; ++i) {
+            const int row = ht / (KD / 8) + i * (kThr / (KD / 8));
+            *reinterpret_cast<la_u4 *>(to + row * KD + ((ht % (KD / 8)) ^ la_hash<KD>(row)) * 8) = x[i];
+        }
+    };
+    auto load_k = [&](int c) { load_rows(std::integral_constant<int, KD>(), kb, uk, a.ldk, c, a.dim); };
+    auto load_q = [&](int c) { load_rows(std::integral_constant<int, KD>(), qb, uq, a.ldq, c, a.dim); };
+    auto load_v = [&](int c) { load_rows(std::integral_constant<int, kCols>(), vb, uv, a.ldv, c, vcols); };
+    auto put_v = [&] {
+#pragma unroll
+        for (int i = 0; i < kVB; ++i)
+            *reinterpret_cast<la_u4 *>(v_s + (ht / (kCols / 8) + i * (kThr / (kCols / 8))) * kLv + ht % (kCols / 8) * 8) = vb[i];
+    };
+    auto load_mat = [&](la_u4 (&x)[kMB], size_t at, int c) {
+        const __amdgpu_buffer_rsrc_t t = chunk(c);
+#pragma unroll
+        for (int i = 0; i < kMB; ++i) x[i] = __builtin_bit_cast(la_u4, __builtin_amdgcn_raw_buffer_load_b128(t, ht * 16, (int)at + i * kThr * 16, 0));
+    };
+    auto put_mat = [&](const la_u4 (&x)[kMB], __bf16 *to) {
+#pragma unroll
+        for (int i = 0; i < kMB; ++i) reinterpret_cast<la_u4 *>(to)[ht + i * kThr] = x[i];
+    };
+    float qi[4], qn[4];
+    auto load_q_in = [&](int c) {
+        const __amdgpu_buffer_rsrc_t x = chunk(c);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+            qn[tt] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x, l16 * 4, (int)offsetof(DeltaChunk, q_in) + 64 * tt, 0));
+    };
+    constexpr size_t kT = offsetof(DeltaChunk, t), kC = offsetof(DeltaChunk, c);
+    load_k(0);
+    load_mat(tb, kT, 0);
+    load_v(0);
+    load_q(0);
+    load_q_in(0);
+    load_mat(cb, kC, 0);
+    put_rows(kb, k2_s);
+    put_mat(tb, t_s);
+    put_v();
+    put_rows(qb, q_s);
+    load_k(1);
+    load_mat(tb, kT, 1);
+    load_v(1);
+    load_q(1);
+    __syncthreads();
+    for (int c = 0; c < chunks; ++c) {  // (past the last chunk: rows that are not there, the last one's matrices)
+        // Q S (transposed: v = 4 g + i of the wave's columns, t = 16 tt + l16)
+        f4 o[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            o[tt] = f4{0.f, 0.f, 0.f, 0.f};
+            qi[tt] = qn[tt];
+        }
+        load_q_in(c + 1);
+#pragma unroll
+        for (int dd = 0; dd < kD; ++dd) {
+            const bf8 hi = la_read8(s_s + dd * 2 * kTerms), lo = la_read8(s_s + dd * 2 * kTerms + kTerms);
+            bf8 x[4];
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) x[tt] = la_read_hashed<KD>(q_s, 16 * tt + l16, 4 * dd + g);
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) o[tt] = la_mfma(hi, x[tt], o[tt]);
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) o[tt] = la_mfma(lo, x[tt], o[tt]);
+        }
+        put_mat(cb, c_s);
+        put_rows(kb, k2_s + ((c + 1) & 1) * 64 * KD);
+        load_mat(cb, kC, c + 1);
+        load_k(c + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[tt][i] *= qi[tt];
+        __syncthreads();
+        put_mat(tb, t_s);
+        put_v();
+        put_rows(qb, q_s);
+        load_mat(tb, kT, c + 2);
+        load_v(c + 2);
+        load_q(c + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        // O += C U, and out
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const LaSplit u = la_split_pair(*reinterpret_cast<const f4 *>(u_s + 2 * kk * kTerms), *reinterpret_cast<const f4 *>(u_s + (2 * kk + 1) * kTerms));
+            const bf8 hi = u.high(), lo = u.low();
+#pragma unroll
+            for (int tt = 2 * kk; tt < 4; ++tt) {
+                const bf8 x = mat(c_s, 0, tt, kk), y = mat(c_s, 1, tt, kk);
+                o[tt] = la_mfma(hi, x, o[tt]);
+                o[tt] = la_mfma(lo, x, o[tt]);
+                o[tt] = la_mfma(hi, y, o[tt]);
+            }
+        }
+        const __amdgpu_buffer_rsrc_t dst = tile(uo, ldo, c, vcols);
+        const int col = vw + 4 * g;
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            const la_u2 x = {row_pack_bf16(o[tt][0], o[tt][1]), row_pack_bf16(o[tt][2], o[tt][3])};
+            __builtin_amdgcn_raw_buffer_store_b64(x, dst, col < vcols ? (uint32_t)((16 * tt + l16) * ldo + col) * 2u : kLaOutside, 0, 0);
+        }
+        __syncthreads();
+    }
+}
+
 template <int KD, int NW> int launch_walk(const DeltaArgs &a, int batch, hipStream_t s) {
     constexpr size_t lds = delta_walk_lds<KD, 16 * NW>();
     static_assert(lds <= 160 * 1024, "LDS of one compute unit");
@@ -619,6 +939,20 @@ template <int KD, int NW> int launch_walk(const DeltaArgs &a, int batch, hipStre
     delta_walk_kernel<KD, NW><<<dim3((unsigned)a.heads, (unsigned)((a.vdim + 16 * NW - 1) / (16 * NW)), (unsigned)batch), dim3(64 * NW), lds, s>>>(a);
     PA_CHECK_LAUNCH("pa_delta (chunks)");
     return PA_OK;
+}
+
+template <int KD, int NW> int launch_pair(const DeltaArgs &a, int batch, hipStream_t s) {
+    constexpr size_t lds = delta_pair_lds<KD, NW>();
+    static_assert(lds <= 160 * 1024, "LDS of one compute unit");
+    if (int rc = la_big_lds(delta_pair_kernel<KD, NW>, lds, "pa_delta")) return rc;
+    delta_pair_kernel<KD, NW><<<dim3((unsigned)a.heads, (unsigned)((a.vdim + 16 * NW - 1) / (16 * NW)), (unsigned)batch), dim3(128 * NW), lds, s>>>(a);
+    PA_CHECK_LAUNCH("pa_delta (chunks)");
+    return PA_OK;
+}
+
+bool delta_pieces_of_16(const DeltaArgs &a) {
+    return a.dim % 8 == 0 && a.vdim % 8 == 0 && a.ldq % 8 == 0 && a.ldk % 8 == 0 && a.ldv % 8 == 0 &&
+           (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15u) == 0;
 }
 
 template <int KD> int launch_delta_chunks(const DeltaArgs &a, int batch, hipStream_t s) {
@@ -631,12 +965,21 @@ template <int KD> int launch_delta_chunks(const DeltaArgs &a, int batch, hipStre
         return launch_walk<KD, 4>(a, batch, s);
     } else {
         if (a.vdim > 64 && heads * ((a.vdim + 127) / 128) >= la_cus()) return launch_walk<KD, 8>(a, batch, s);
-        if (a.vdim > 32 && heads * ((a.vdim + 63) / 64) >= la_cus()) return launch_walk<KD, 4>(a, batch, s);
-        return launch_walk<KD, 2>(a, batch, s);
+        const int64_t slices = heads * ((a.vdim + 63) / 64);
+        const bool four = a.vdim > 32 && slices >= la_cus();
+        // (a compute unit has room for two workgroups of four waves at dim 64, and for one of the paired ones, whose chain is not worth it in
+        // one chunk or two: 32 heads of 64 x 64, us, prompts of 16 .. 30 rows, 9 of them 18.9 against 21.0, 63 54.1 against 58.8; of 60 .. 120
+        // rows, 9 of them 26.1 against 25.0, 63 89.1 against 91.4; of 200 .. 250 rows, 63 220 against 202)
+        const bool brief = KD == 64 && four && (a.chunks == 1 || (a.chunks == 2 && slices >= 2 * la_cus()));
+        if (!brief && delta_pieces_of_16(a)) return four ? launch_pair<KD, 4>(a, batch, s) : launch_pair<KD, 2>(a, batch, s);
+        return four ? launch_walk<KD, 4>(a, batch, s) : launch_walk<KD, 2>(a, batch, s);
     }
 }
 
-size_t delta_ws_bytes(int batch, int heads, int max_q_len) { return (size_t)batch * heads * ((max_q_len + 63) / 64) * sizeof(DeltaChunk); }
+// (what a chunk takes in the interface: two whole matrices of two terms and 1 KB, of which the walk's order leaves a quarter unused)
+constexpr size_t kDeltaChunkBytes = 4 * 64 * 64 * 2 + 1024;
+static_assert(sizeof(DeltaChunk) <= kDeltaChunkBytes && sizeof(DeltaChunk) % 16 == 0, "a chunk's room");
+size_t delta_ws_bytes(int batch, int heads, int max_q_len) { return (size_t)batch * heads * ((max_q_len + 63) / 64) * kDeltaChunkBytes; }
 
 template <typename T> void launch_delta_recurrent(const DeltaArgs &a, int batch, hipStream_t s) {
     const dim3 grid((unsigned)((a.vdim + kDeltaCols - 1) / kDeltaCols), (unsigned)a.heads, (unsigned)batch), block(256);

@@ -47,6 +47,7 @@ __device__ __forceinline__ la_bf4 la_read_tr(const __bf16 *p) {
 // Pairs x = hi + lo, packed bf16
 __device__ __forceinline__ void la_split2(float x0, float x1, uint32_t &hi, uint32_t &lo) {
     hi = row_pack_bf16(x0, x1);
+    asm("" : "+v"(hi));  // (else the compiler converts x0 once more by itself for `hi << 16`: seven instructions a pair instead of six)
     lo = row_pack_bf16(x0 - __builtin_bit_cast(float, hi << 16), x1 - __builtin_bit_cast(float, hi & 0xffff0000u));
 }
 struct LaSplit {  // eight values as two operands

@@ -112,10 +112,12 @@ class DeltaCase:
         pad = lambda x: -(-x // 16) * 16
         self.state = torch.full((len(lens) + 1, heads, pad(dim), pad(vdim)), float("nan"), device=DEV)
 
-    def run(self, picks, slots, decode=False, chunks=True):
+    def run(self, picks, slots, decode=False, chunks=True, pieces=False):
         u = torch.cat([self.rows[b][lo: lo + n] for b, lo, n in picks]).to(DEV)
         sizes = [self.groups * self.dim, self.groups * self.dim, self.heads * self.vdim, self.heads, self.heads]
-        q, k, v, a, b = u.split(sizes, 1)
+        if pieces:  # rows of whole 16-byte pieces
+            u = torch.nn.functional.pad(u, (0, -u.shape[1] % 8), value=float("nan"))
+        q, k, v, a, b = u[:, : sum(sizes)].split(sizes, 1)
         p = _portions(picks, slots, tiles=False)
         if decode:
             p = ops.Portions(p.ctx_lens, p.state_slots)
@@ -163,6 +165,19 @@ def test_delta_rule_in_portions_and_single_tokens(heads, groups, dim, vdim, dtyp
     case.run([(0, 0, 30), (1, 0, 2)], [2, 0])
     case.run([(1, 2, 95), (0, 30, 110)], [2, 0])
     case.check_states([2, 0])
+
+
+@pytest.mark.parametrize("heads,groups,dim,vdim", [(2, 1, 128, 128), (3, 3, 64, 72), (2, 2, 96, 40), (4, 2, 72, 24), (48, 12, 64, 64), (40, 10, 128, 40)])
+def test_delta_rule_rows_of_whole_pieces(heads, groups, dim, vdim):
+    """Chain and outputs in different waves: slices of 32 and (many heads) 64 columns, chunks around 64 rows, states that go on."""
+    announce(f"delta pieces {heads} {groups} {dim} {vdim}")
+    case = DeltaCase([1, 63, 64, 65, 128, 129, 193] if heads < 40 else [130, 64, 1, 65, 70, 3, 193], heads, groups, dim, vdim, BF, seed=7)
+    slots = [3, 0, 6, 1, 5, 2, 7]
+    case.run([(i, 0, n) for i, n in enumerate(case.lens)], slots, pieces=True)
+    case.check_states(slots)
+    for at, n in ((0, 65), (65, 128)):
+        case.run([(6, at, n)], slots, pieces=True)
+    case.check_states(slots)
 
 
 def test_delta_rule_many_heads_take_wide_slices():
