@@ -14,7 +14,6 @@
 // diagonal row by row and joining them with 32-bit matrix products).  The second pass walks a portion's chunks with S in
 // accumulator registers; a wave owns value columns, which do not depend on each other.  Unit norms are factors of rows,
 // so q and k enter the products as they are stored; T, C, S, U and V - e^F K S are split into two bf16 terms each.
-#include <type_traits>
 #include "linear_tiles.h"
 
 namespace {

@@ -38,6 +38,7 @@ struct GlArgs {
     float *ws;  // segment states: S [dp][vp], n [dp], m, log decay, starting m
     int heads, per_group, dim, vdim, dp, vp;
     int batch, segments, seg_rows;
+    bool wide;  // rows of whole, aligned 16-byte pieces
 };
 
 struct GlPortion {
@@ -189,14 +190,17 @@ struct GlRows {
     float inter[64], add[64];         // rows' factor on Q S; weights of the chunk's rows in the new state
     float low[64];                    // exp(-m)
     float whole, pad[15];             // factor on the old state
+    uint16_t one[3][64];              // kMlstm: `add` as three bf16 terms (all 24 bits)
 };
 
-// Elements of the tiles: K and Q (paired), V (row-major), the two terms of the weighted scores.
+// Parts that n . q of a row is summed in: the waves that hold rows of n
+template <int KD, int NW> constexpr int gl_parts() { return KD / 32 < NW ? KD / 32 : NW; }
+// Elements of the tiles: K and Q (hashed), V (row-major), the two terms of the weighted scores.
 template <int KD, int NW> constexpr int gl_kv_elems() { return 64 * KD + 64 * (16 * NW + kLaPadV); }
 template <int KD, int NW, int KIND, bool STATES> constexpr size_t gl_lds_bytes() {
     const size_t elems = STATES ? 2 * gl_kv_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
                                 : gl_kv_elems<KD, NW>() + 64 * KD + 2 * 64 * kLaPitchA;
-    return elems * 2 + (STATES ? 2 : 1) * sizeof(GlRows) + (KIND == kMlstm && !STATES ? (3 * 64 + KD) * 4 : 0);
+    return elems * 2 + 2 * sizeof(GlRows) + (KIND == kMlstm && !STATES ? (gl_parts<KD, NW>() + 2) * 64 * 4 : 0);
 }
 
 // Inclusive scans over the wave: rows of 16 lanes by shifts inside the row, then the rows before.
@@ -226,24 +230,29 @@ __device__ __forceinline__ float gl_scan_max(float x, int lane) {
 // KD: dim padded to 64, 128 or 256.  NW: waves; each owns 16 value columns.  All products are taken transposed (value
 // columns, or keys, as the rows of the result), so that a lane holds four consecutive elements of one row t.
 // STATES: only the segment's own contribution to the state, to the workspace (first pass over a portion in segments).
-// The tiles and the two passes as in lightning attention's kernel.  One prompt of 15999 rows, 4 heads of 256 x 512 (mLSTM):
-// 181 -> 172 us for the second pass, 68 -> 71 for the first; 128 prompts of 16 .. 130 rows (SSD, 64 heads of 128 x 64) 178 -> 172.
+// Rows come in 16-byte pieces and lie in LDS as they are (hashed): the rows of S that an operand's lanes hold are then 8 g .. 8 g + 7 of 32.
+// A SIMD's two waves run in step (a compute unit has room for one workgroup at dim 256), so a chunk takes what its waves wait, and these waits went:
+// operands are read ahead of the products before them, with no branch in between; places that follow from one by an exclusive or are not kept (kept,
+// they were spilled, and each reload waited for the tile's loads); the next tile's loads are spread over the chunk; its gates are made by a wave
+// without score tiles; n . q is a product, and rows' factors are divided once per row and wave.  Cycles of a chunk at 256 x 128 columns, mLSTM: 21400 ->
+// 15000, of which products keep a SIMD busy for 5800 and the vector unit for 5100.
+// One prompt of 15999 rows, 4 heads of 256 x 512 (mLSTM): second pass 168 -> 124 us, first 73 -> 58; 8 prompts of 1226 .. 1840 rows, 16 heads of 128 x 64 (SSD)
+// 92 -> 83; 17 of 480 .. 628, 4 heads of 256 x 512 202 -> 157; single chunks, 23 of 2 .. 25 rows, 8 heads of 128 x 256, 20.4 -> 17.2.
 template <int KD, int NW, int KIND, bool STATES>
-__global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_chunk_kernel(const GlArgs a) {
+__global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : NW == 4 && KD == 64 && KIND == kSsd ? 3 : 2) void gated_chunk_kernel(const GlArgs a) {
     constexpr int kCols = 16 * NW, kLdV = kCols + kLaPadV, kThr = 64 * NW;
-    constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
+    constexpr int kKP = 64 * (KD / 8) / kThr, kKRows = kThr / (KD / 8);  // 16-byte pieces of K per thread, rows between them; of V: two
+    constexpr int kVRows = kThr / (kCols / 8);
+    static_assert(kKP * kThr == 64 * (KD / 8) && 2 * kVRows == 64, "whole passes");
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     constexpr int kNd = (KD / 32 + NW - 1) / NW;  // kMlstm: 32-row pieces of n per wave
-    // Places in LDS are worked out again in every chunk only where registers run out, or where that lets a second workgroup into a compute
-    // unit.  16 prompts of 900 .. 1000 rows, 16 heads, us, again -> kept: mLSTM 128 x 128 113 -> 108, 256 x 64 177 -> 166, but
-    // 256 x 128 171 -> 317 (spills); SSD 128 x 128 87 -> 81, 256 x 128 143 -> 134, 128 x 64 with 32 heads 105 -> 107; first pass of mLSTM
-    // 128 x 256, 8 heads, 6 prompts of 400 .. 4000 rows, 41 -> 54 (123 registers -> 133).
-    constexpr bool kAgain = STATES || (KIND == kMlstm ? KD == 256 && NW == 8 : KD >= 128 && NW == 4);
+    constexpr int kParts = gl_parts<KD, NW>();
+    constexpr int kGates = NW == 8 ? 1 : 0;  // the wave with the fewest score tiles (of eight: none) makes the next chunk's gates meanwhile
     extern __shared__ __align__(16) char lds[];
     GlRows *rows = reinterpret_cast<GlRows *>(lds);
-    float *nq_s = reinterpret_cast<float *>(rows + (STATES ? 2 : 1));  // kMlstm: n . q per row, two parts of the score sums, n
-    float *sum_s = nq_s + 64, *n_s = sum_s + 128;
-    __bf16 *tiles = reinterpret_cast<__bf16 *>(KIND == kMlstm && !STATES ? n_s + KD : nq_s);
+    float *nq_s = reinterpret_cast<float *>(rows + 2);  // kMlstm: n . q per row, kParts parts; two parts of the score sums
+    float *sum_s = nq_s + 64 * kParts;
+    __bf16 *tiles = reinterpret_cast<__bf16 *>(KIND == kMlstm && !STATES ? sum_s + 128 : nq_s);
     __bf16 *k_s = tiles, *v_s = k_s + 64 * KD;
     __bf16 *q_s = tiles + gl_kv_elems<KD, NW>(), *a_hi = q_s + 64 * KD, *a_lo = a_hi + 64 * kLaPitchA;
 
@@ -255,13 +264,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
     const bool last = r_end == p.n;
     if (r_beg >= p.n || (STATES && last)) return;
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int v0 = vsl * kCols, vw = wave * 16;  // first column of the workgroup, of the wave inside it
-    const int l16 = tid & 15, g = (tid & 63) >> 4;
+    const int l16 = tid & 15, g = lane >> 4;
     const GlHead hd = gl_head(a, h);
 
-    // The state slice of this wave: tile dt holds d = 16 dt + 4 g + i, v = v0 + vw + l16
+    // The state slice of this wave: tile dt holds d = 32 (dt / 2) + 8 g + 4 (dt % 2) + i, v = v0 + vw + l16
     f4 s[KD / 16];
+    auto s_row = [](int dt, int i) { return 32 * (dt / 2) + 4 * (dt % 2) + i; };
     const int64_t state_elems = (int64_t)a.dp * a.vp;
     float *pool = p.slot >= 0 ? a.state + (p.slot * a.heads + h) * a.head_floats : nullptr;
     float *seg_state = a.segments > 1 ? a.ws + (((int64_t)b * a.heads + h) * a.segments + seg) * (state_elems + a.dp + 16) : nullptr;
@@ -269,7 +279,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     // (a state as a buffer: rows past dp lie past its end, columns past vp get an offset outside)
     const int state_bytes = (int)state_elems * 4;
     const int v = v0 + vw + l16;
-    const uint32_t soff = v < a.vp ? (uint32_t)(4 * g * a.vp + v) * 4u : kLaOutside;
+    const uint32_t soff = v < a.vp ? (uint32_t)(8 * g * a.vp + v) * 4u : kLaOutside;
     {
         const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(from ? from : a.state), 0, from ? state_bytes : 0, 0x00020000);  // (no state: every load is past the end)
@@ -277,14 +287,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
         for (int dt = 0; dt < KD / 16; ++dt)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + (16 * dt + i) * a.vp * 4, 0, 0));
+                s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + s_row(dt, i) * a.vp * 4, 0, 0));
     }
-    // n and m of the workgroup: a wave follows its 32-row pieces of n (n[j][e][i]: row 32 (kNd wave + j) + 16 e + 4 g + i, the
-    // same in all columns), the first wave m
+    // n and m of the workgroup: a wave follows its 32-row pieces of n (n[j][e][i]: row 32 (kNd wave + j) + 8 g + 4 e + i, the
+    // same in all columns), one wave m
     const int rep0 = v0 / kRecCols;
     f4 n[KIND == kMlstm ? kNd : 1][2];
     float m_prev = STATES ? kGlNone : 0.f, decayed = 0.f;
-    auto n_row = [&](int j, int e) { return 32 * (kNd * wave + j) + 16 * e + 4 * g; };
+    auto n_row = [&](int j, int e) { return 32 * (kNd * wave + j) + 8 * g + 4 * e; };
     if constexpr (KIND == kMlstm) {
         const float *np = from ? from + state_elems + (a.segments > 1 ? 0 : rep0 * (a.dp + 16)) : nullptr;
 #pragma unroll
@@ -293,7 +303,6 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
             for (int e = 0; e < 2; ++e) {
                 n[j][e] = f4{0.f, 0.f, 0.f, 0.f};
                 if (np && n_row(j, e) < a.dp) n[j][e] = *reinterpret_cast<const f4 *>(np + n_row(j, e));
-                if (!STATES && l16 == 0 && n_row(j, e) < KD) *reinterpret_cast<f4 *>(n_s + la_paired(n_row(j, e))) = n[j][e];
             }
         if (np) m_prev = a.segments > 1 ? np[a.dp + 2] : np[a.dp];
     }
@@ -305,103 +314,178 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
     const pa_bf16 *ga = reinterpret_cast<const pa_bf16 *>(a.ga) + p.row0 * a.ldg + h;
     const pa_bf16 *gb = reinterpret_cast<const pa_bf16 *>(a.gb) + p.row0 * a.ldg + h;
     const int vcols = a.vdim - v0 < kCols ? a.vdim - v0 : kCols;
-    LaBlock kb[kKPass], qb[STATES ? 1 : kKPass], vb;
-    const uint32_t voff = la_block_off(a.ldv, tid / (kCols / 4) * 4, tid % (kCols / 4) * 4, vcols);
-    float raw_a = 0.f, raw_b = 0.f;
-    auto fetch = [&](int r0) {
+    la_u4 kb[kKP], qb[STATES ? 1 : kKP], vb[2];
+    const int kr = tid / (KD / 8), kc = tid % (KD / 8), vr = tid / (kCols / 8), vc = tid % (kCols / 8);  // a thread's first row and piece
+    auto fetch_rows = [&](auto &x, const uint16_t *base, int64_t ld, int r0, int row, int piece, int rows_apart, int cols) {
         const int nr = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
-        const __amdgpu_buffer_rsrc_t tk = la_tile(uk + r0 * a.ldk, a.ldk, nr, a.dim), tv = la_tile(uv + r0 * a.ldv, a.ldv, nr, vcols);
-        if (wave == 0 && tid < nr) {
-            raw_a = pa_scalar<pa_bf16>::load(ga + (r0 + tid) * a.ldg);
-            if (KIND == kMlstm) raw_b = pa_scalar<pa_bf16>::load(gb + (r0 + tid) * a.ldg);
-        }
-        if (!STATES) {
-            const __amdgpu_buffer_rsrc_t tq = la_tile(uq + r0 * a.ldq, a.ldq, nr, a.dim);
-#pragma unroll
-            for (int i = 0; i < kKPass; ++i) {
-                const int blk = tid + kThr * i;
-                qb[i] = la_load_block(tq, blk < kKBlocks ? la_block_off(a.ldq, blk / kDB * 4, blk % kDB * 4, a.dim) : kLaOutside,
-                                      (uint32_t)a.ldq * 2u);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kKPass; ++i) {
-            const int blk = tid + kThr * i;
-            kb[i] = la_load_block(tk, blk < kKBlocks ? la_block_off(a.ldk, blk / kDB * 4, blk % kDB * 4, a.dim) : kLaOutside,
-                                  (uint32_t)a.ldk * 2u);
-        }
-        vb = la_load_block(tv, voff, (uint32_t)a.ldv * 2u);
+        const __amdgpu_buffer_rsrc_t t = la_tile(base + r0 * ld, ld, nr, cols);
+        la_load_pieces(x, t, ld, row, piece * 8, rows_apart, cols, a.wide);
     };
-    fetch(r_beg);
+    auto fetch_q = [&](int r0) { fetch_rows(qb, uq, a.ldq, r0, kr, kc, kKRows, a.dim); };
+    auto fetch_k = [&](int r0) { fetch_rows(kb, uk, a.ldk, r0, kr, kc, kKRows, a.dim); };
+    auto fetch_v = [&](int r0) { fetch_rows(vb, uv, a.ldv, r0, vr, vc, kVRows, vcols); };
+    const int row_place = la_place_of<KD>(l16, g), tr_place = la_place_of<KD>(4 * g + l16 / 4, l16 % 4);
+    auto put = [&] {
+        const int at = kr * KD + (kc ^ la_hash<KD>(kr)) * 8;  // (rows 16 apart have the same hash)
+        static_assert(kKRows % 16 == 0 || kKP == 1 || KD == 256, "places of a thread's pieces");
+#pragma unroll
+        for (int i = 0; i < kKP; ++i) {
+            const int to = kKRows % 16 == 0 || kKP == 1 ? at + i * kKRows * KD : (kr + i * kKRows) * KD + (kc ^ la_hash<KD>(kr + i * kKRows)) * 8;
+            *reinterpret_cast<la_u4 *>(k_s + to) = kb[i];
+            if (!STATES) *reinterpret_cast<la_u4 *>(q_s + to) = qb[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *reinterpret_cast<la_u4 *>(v_s + (vr + i * kVRows) * kLdV + vc * 8) = vb[i];
+    };
+    float raw_a = 0.f, raw_b = 0.f;
+    auto fetch_gates = [&](int r0) {
+        if (wave == kGates && lane < r_end - r0) {
+            raw_a = pa_scalar<pa_bf16>::load(ga + (r0 + lane) * a.ldg);
+            if (KIND == kMlstm) raw_b = pa_scalar<pa_bf16>::load(gb + (r0 + lane) * a.ldg);
+        }
+    };
+    auto gates = [&](int r0, GlRows *to) {  // a chunk's gates, one row per lane
+        const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
+        float decay, in;
+        gl_gate<KIND>(a, hd, raw_a, raw_b, decay, in);
+        if (lane >= nv) decay = 0.f;
+        const float f = gl_scan_add(decay, lane), f_last = gl_lane(f, 63);
+        if constexpr (KIND == kSsd) {
+            const float mul = lane < nv ? in : 0.f;
+            to->row[lane] = f;
+            to->col[lane] = -f;
+            to->mul[lane] = mul;
+            to->inter[lane] = exp2f(f);
+            to->add[lane] = exp2f(f_last - f) * mul;
+            if (lane == 0) to->whole = exp2f(f_last);
+        } else {
+            const float col = lane < nv ? in - f : kGlNone;
+            const float top = fmaxf(m_prev, gl_scan_max(col, lane)), top_last = gl_lane(top, 63);
+            to->row[lane] = -top;
+            to->col[lane] = col;
+            to->inter[lane] = exp2f(m_prev - top);
+            float add = exp2f(col - top_last);
+            to->add[lane] = add;
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                const __bf16 x = (__bf16)add;
+                to->one[e][lane] = __builtin_bit_cast(uint16_t, x);
+                add -= (float)x;
+            }
+            to->low[lane] = exp2f(-(f + top));
+            if (lane == 0) to->whole = exp2f(m_prev - top_last);
+            m_prev = f_last + top_last;
+        }
+        decayed += f_last;
+    };
+    if (!STATES) fetch_q(r_beg);
+    fetch_k(r_beg);
+    fetch_v(r_beg);
+    fetch_gates(r_beg);
+    if (wave == kGates) gates(r_beg, rows);
+    fetch_gates(r_beg + kLaChunk);
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
-        const int lt = kAgain ? la_again(tid) : tid;
-#pragma unroll
-        for (int i = 0; i < kKPass; ++i) {
-            const int blk = lt + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
-            if (kKBlocks % kThr != 0 && blk >= kKBlocks) continue;
-            la_put_paired<false, KD>(kb[i], sr, c, k_s);
-            if (!STATES) la_put_paired<false, KD>(qb[i], sr, c, q_s);
-        }
-        la_put_block<false>(vb, lt / (kCols / 4) * 4, lt % (kCols / 4) * 4, v_s, kLdV);
-        if (wave == 0) {  // the chunk's gates, one row per lane
-            float decay, in;
-            gl_gate<KIND>(a, hd, raw_a, raw_b, decay, in);
-            if (tid >= nv) decay = 0.f;
-            const float f = gl_scan_add(decay, tid), f_last = gl_lane(f, 63);
-            if constexpr (KIND == kSsd) {
-                const float mul = tid < nv ? in : 0.f;
-                rows->row[tid] = f;
-                rows->col[tid] = -f;
-                rows->mul[tid] = mul;
-                rows->inter[tid] = exp2f(f);
-                rows->add[tid] = exp2f(f_last - f) * mul;
-                if (tid == 0) rows->whole = exp2f(f_last);
-            } else {
-                const float col = tid < nv ? in - f : kGlNone;
-                const float top = fmaxf(m_prev, gl_scan_max(col, tid)), top_last = gl_lane(top, 63);
-                rows->row[tid] = -top;
-                rows->col[tid] = col;
-                rows->inter[tid] = exp2f(m_prev - top);
-                rows->add[tid] = exp2f(col - top_last);
-                rows->low[tid] = exp2f(-(f + top));
-                if (tid == 0) rows->whole = exp2f(m_prev - top_last);
-                m_prev = f_last + top_last;
-            }
-            decayed += f_last;
-        }
-        if (r0 + kLaChunk < r_end) fetch(r0 + kLaChunk);
+        GlRows *next = rows == reinterpret_cast<GlRows *>(lds) ? rows + 1 : reinterpret_cast<GlRows *>(lds);
+        put();
         __syncthreads();
+        // (the next tile's loads are spread over the chunk: all at once would hold up a wave for 2500 cycles)
+        const bool more = r0 + kLaChunk < r_end;
 
-        const int lr = kAgain && KD == 256 ? la_again(tid) : tid, l16 = lr & 15, g = (lr & 63) >> 4;
+        bf8 av[2];  // V: the wave's columns as rows
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) av[kk] = la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g);
         f4 o[4];  // O^T: v = 4 g + i of the wave's columns, t = 16 tt + l16
-        if constexpr (!STATES) {
-            // score tiles (st, rt): keys 16 st + 4 g + i, rows 16 rt + l16
+        if constexpr (STATES) {
+            if (wave == kGates && more) {
+                gates(r0 + kLaChunk, next);
+                fetch_gates(r0 + 2 * kLaChunk);
+            }
+            if (more) {
+                fetch_k(r0 + kLaChunk);
+                fetch_v(r0 + kLaChunk);
+            }
+        } else {
+            // score tiles (st, rt): keys 16 st + 4 g + i, rows 16 rt + l16.  (No branch inside: each product would wait for its own read.)
             const int rt = NW == 8 ? wave >> 1 : wave;
             f4 sc[kST];
 #pragma unroll
             for (int m = 0; m < kST; ++m) sc[m] = f4{0.f, 0.f, 0.f, 0.f};
+            auto scores = [&](auto count) {
+                constexpr int kN = decltype(count)::value;
+                bf8 bq[2], ak[2][kN];
+                const int at = la_again(row_place), at_q = at + rt * (32 * KD), at_k = at + (NW == 8 ? wave & 1 : 0) * (32 * KD);
+                auto read = [&](int kk) {
+                    bq[kk & 1] = la_read_place<KD>(q_s, at_q, 0, kk);
 #pragma unroll
-            for (int kk = 0; kk < KD / 32; ++kk) {
-                const bf8 bq = la_read_paired<KD>(q_s, 16 * rt + l16, l16, kk, g);
+                    for (int m = 0; m < kN; ++m) ak[kk & 1][m] = la_read_place<KD>(k_s, at_k, 16 * (NW == 8 ? 2 * m : m), kk);
+                };
+                read(0);
 #pragma unroll
-                for (int m = 0; m < kST; ++m) {
-                    const int st = NW == 8 ? 2 * m + (wave & 1) : m;
-                    if (st <= rt) sc[m] = la_mfma(la_read_paired<KD>(k_s, 16 * st + l16, l16, kk, g), bq, sc[m]);
+                for (int kk = 0; kk < KD / 32; ++kk) {
+                    if (kk + 1 < KD / 32) read(kk + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < kN; ++m) sc[m] = la_mfma(ak[kk & 1][m], bq[kk & 1], sc[m]);
                 }
+            };
+            if (wave == kGates && more) {
+                gates(r0 + kLaChunk, next);
+                fetch_gates(r0 + 2 * kLaChunk);
             }
-            // the rows' part from before the chunk: Q S, then its factors
+            if (NW == 4 || wave != kGates) {
+                if (rt >= 2) scores(std::integral_constant<int, kST>());
+                else scores(std::integral_constant<int, kST / 2>());
+            }
+            // the rows' part from before the chunk: Q S, then its factors (a sequence's first chunk has none)
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) o[tt] = f4{0.f, 0.f, 0.f, 0.f};
+            const bool carried = from || r0 > r_beg;
+            if (!carried && more) {
+                fetch_q(r0 + kLaChunk);
+                fetch_k(r0 + kLaChunk);
+            }
+            if (carried) {
+                bf8 bq[2][4];
+                const int at = la_again(row_place);
+                auto read = [&](int dd) {
 #pragma unroll
-            for (int dd = 0; dd < KD / 32; ++dd) {
-                const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
-                const bf8 hi = sp.high(), lo = sp.low();
+                    for (int tt = 0; tt < 4; ++tt) bq[dd & 1][tt] = la_read_place<KD>(q_s, at, 16 * tt, dd);
+                };
+                read(0);
+                if (more) fetch_q(r0 + kLaChunk);
 #pragma unroll
-                for (int tt = 0; tt < 4; ++tt) {
-                    const bf8 bq = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
-                    o[tt] = la_mfma(hi, bq, o[tt]);
-                    o[tt] = la_mfma(lo, bq, o[tt]);
+                for (int dd = 0; dd < KD / 32; ++dd) {
+                    if (dd + 1 < KD / 32) read(dd + 1);
+                    const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
+                    const bf8 hi = sp.high(), lo = sp.low();
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) o[tt] = la_mfma(hi, bq[dd & 1][tt], o[tt]);
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) o[tt] = la_mfma(lo, bq[dd & 1][tt], o[tt]);
+                    if (dd == KD / 64 && more) fetch_k(r0 + kLaChunk);
+                }
+            }
+            if constexpr (KIND == kMlstm) {  // n . q over the wave's rows of n, all 24 bits of them; the same in all rows of the result
+                if (wave < kParts) {
+                    const int at = la_again(row_place);
+                    f4 nq[4];
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) nq[tt] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j < kNd; ++j) {
+                        if (!carried) break;  // (uniform)
+                        const LaSplit3 x = la_split3(n[j][0], n[j][1]);
+                        bf8 bq[4];
+#pragma unroll
+                        for (int tt = 0; tt < 4; ++tt) bq[tt] = la_read_place<KD>(q_s, at, 16 * tt, kNd * wave + j);
+#pragma unroll
+                        for (int e = 0; e < 3; ++e)
+#pragma unroll
+                            for (int tt = 0; tt < 4; ++tt) nq[tt] = la_mfma(x.term[e], bq[tt], nq[tt]);
+                    }
+                    nq_s[lane * kParts + wave] = g == 0 ? nq[0][0] : g == 1 ? nq[1][0] : g == 2 ? nq[2][0] : nq[3][0];
                 }
             }
 #pragma unroll
@@ -410,20 +494,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[tt][i] *= f;
             }
-            if constexpr (KIND == kMlstm) {  // n . q: NW lanes per row
-                const int t = tid / NW;
-                constexpr int kPer = KD / NW / 8;  // 16-byte chunks of Q, whose order n_s has as well
-                float acc = 0.f;
-#pragma unroll
-                for (int d = tid % NW * kPer; d < tid % NW * kPer + kPer; ++d) {
-                    const bf8 x = la_read8(q_s + t * KD + (d ^ la_hash<KD>(t)) * 8);
-                    const float *nr = n_s + 8 * d;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) acc = fmaf((float)x[j], nr[j], acc);
-                }
-                acc = pa_group_sum<NW>(acc);
-                if (tid % NW == 0) nq_s[t] = acc;
-            }
+            if (more) fetch_v(r0 + kLaChunk);
             // the scores' weights
             const int t = 16 * rt + l16;
             const float row_w = rows->row[t];
@@ -457,37 +528,59 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
                 if (NW == 4 && g == 1) sum_s[64 + t] = 0.f;
             }
             __syncthreads();
+            bf8 ah[2][4], al[2][4];  // (all reads ahead of the products)
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                const bf8 av = la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g);
 #pragma unroll
                 for (int tt = 2 * kk; tt < 4; ++tt) {
-                    o[tt] = la_mfma(av, la_read8(a_hi + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
-                    o[tt] = la_mfma(av, la_read8(a_lo + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
+                    ah[kk][tt] = la_read8(a_hi + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g);
+                    al[kk][tt] = la_read8(a_lo + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g);
                 }
+            }
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+                for (int tt = 2 * kk; tt < 4; ++tt) o[tt] = la_mfma(av[kk], ah[kk][tt], o[tt]);
+#pragma unroll
+                for (int tt = 2 * kk; tt < 4; ++tt) o[tt] = la_mfma(av[kk], al[kk][tt], o[tt]);
             }
             const int ldo = a.heads * a.vdim;
             const uint16_t *first = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0) * (int64_t)ldo + h * a.vdim + v0;
             const __amdgpu_buffer_rsrc_t dst = la_tile(first, ldo, nv, vcols);
             const int c = vw + 4 * g;
+            float row_f = a.q_scale;  // of row `lane`
+            if constexpr (KIND == kMlstm) {
+                float nq = 0.f;
+#pragma unroll
+                for (int x = 0; x < kParts; ++x) nq += nq_s[lane * kParts + x];
+                const float den = fmaf(rows->inter[lane], nq, sum_s[lane] + sum_s[64 + lane]);
+                row_f /= fmaxf(fabsf(row_f * den), rows->low[lane]) + a.den_eps;
+            }
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) {
                 const int row = 16 * tt + l16;
-                float f = a.q_scale;
-                if constexpr (KIND == kMlstm) {
-                    const float den = fmaf(rows->inter[row], nq_s[row], sum_s[row] + sum_s[64 + row]);
-                    f /= fmaxf(fabsf(f * den), rows->low[row]) + a.den_eps;
-                }
+                const float f = KIND == kMlstm ? __shfl(row_f, row, 64) : row_f;
                 const la_u2 x = {row_pack_bf16(o[tt][0] * f, o[tt][1] * f), row_pack_bf16(o[tt][2] * f, o[tt][3] * f)};
                 __builtin_amdgcn_raw_buffer_store_b64(x, dst, c < vcols ? (uint32_t)(row * ldo + c) * 2u : kLaOutside, 0, 0);
             }
         }
-        // S <- whole S + K^T (weights V)
+        // S <- whole S + K^T (weights V), operands a group of tiles ahead of their products
+        constexpr int kGroup = 4, kGroups = KD / 16 / kGroup;
+        bf8 ak[2][kGroup];
+        const int at = la_again(tr_place);
+        auto read = [&](int step) {  // (kk, group)
+#pragma unroll
+            for (int j = 0; j < kGroup; ++j) ak[step & 1][j] = la_read_place_tr<KD>(k_s, at, 32 * (step / kGroups), step % kGroups * kGroup + j);
+        };
+        read(0);
         const float whole = rows->whole;
+        auto keep = [&](int first) {
 #pragma unroll
-        for (int dt = 0; dt < KD / 16; ++dt)
+            for (int dt = first; dt < first + kGroup; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
+                for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
+        };
+        keep(0);
         if constexpr (KIND == kMlstm) {
 #pragma unroll
             for (int j = 0; j < kNd; ++j)
@@ -500,42 +593,45 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const f4 w0 = *reinterpret_cast<const f4 *>(rows->add + 32 * kk + 4 * g), w1 = *reinterpret_cast<const f4 *>(rows->add + 32 * kk + 16 + 4 * g);
-            const LaSplit sp = la_split_weighted(la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g), w0, w1);
+            const LaSplit sp = la_split_weighted(av[kk], w0, w1);
             const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
-            for (int dt = 0; dt < KD / 16; ++dt) {
-                const bf8 ak = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
-                s[dt] = la_mfma(ak, hi, s[dt]);
-                s[dt] = la_mfma(ak, lo, s[dt]);
+            for (int x = 0; x < kGroups; ++x) {
+                const int step = kk * kGroups + x;
+                if (step + 1 < 2 * kGroups) read(step + 1);
+                if (step + 1 < kGroups) keep((step + 1) * kGroup);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], hi, s[x * kGroup + j]);
+#pragma unroll
+                for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], lo, s[x * kGroup + j]);
             }
             if constexpr (KIND == kMlstm) {  // n likewise, with k alone: the weights in every column
-                const LaSplit3 ones = la_split3(w0, w1);
+                bf8 ones[3];
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    const __bf16 *x = reinterpret_cast<const __bf16 *>(rows->one[e]) + 32 * kk + 4 * g;
+                    ones[e] = la_read44(x, x + 16);
+                }
 #pragma unroll
                 for (int j = 0; j < kNd; ++j) {
                     const int piece = kNd * wave + j;
                     if (piece >= KD / 32) break;  // (uniform)
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
-                        const bf8 ak = la_read_paired_tr<KD>(k_s, 32 * kk, 2 * piece + e, l16, g);
+                        const bf8 x = la_read_place_tr<KD>(k_s, at, 32 * kk, 2 * piece + e);
 #pragma unroll
-                        for (int x = 0; x < 3; ++x) n[j][e] = la_mfma(ak, ones.term[x], n[j][e]);
+                        for (int y = 0; y < 3; ++y) n[j][e] = la_mfma(x, ones[y], n[j][e]);
                     }
                 }
             }
         }
-        if constexpr (KIND == kMlstm && !STATES) {
-#pragma unroll
-            for (int j = 0; j < kNd; ++j)
-#pragma unroll
-                for (int e = 0; e < 2; ++e)  // (read again after the next chunk's first barrier)
-                    if (l16 == 0 && n_row(j, e) < KD) *reinterpret_cast<f4 *>(n_s + la_paired(n_row(j, e))) = n[j][e];
-        }
+        rows = next;
         if constexpr (!STATES) {
-            __syncthreads();  // the next chunk's tiles and gates may be written now
-        } else {              // the other half of the tiles and gates
+            __syncthreads();  // the next chunk's tiles may be written now
+        } else {              // the other half of the tiles
             k_s = k_s == tiles ? tiles + gl_kv_elems<KD, NW>() : tiles;
             v_s = k_s + 64 * KD;
-            rows = rows == reinterpret_cast<GlRows *>(lds) ? rows + 1 : reinterpret_cast<GlRows *>(lds);
         }
     }
     float *to = STATES ? seg_state : last ? pool : nullptr;
@@ -548,7 +644,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float f = s[dt][i];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), dst, base + (16 * dt + i) * a.vp * 4, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), dst, base + s_row(dt, i) * a.vp * 4, 0, 0);
         }
     auto put_n = [&](float *np) {
         if constexpr (KIND == kMlstm) {
@@ -559,10 +655,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
                     if (l16 == 0 && n_row(j, e) < a.dp) *reinterpret_cast<f4 *>(np + n_row(j, e)) = n[j][e];
         }
     };
+    const bool one = tid == 64 * kGates;  // (of the wave that knows m)
     if constexpr (STATES) {  // (every value slice has the same n, m and decay)
         if (vsl != 0) return;
         put_n(to + state_elems);
-        if (tid == 0) {
+        if (one) {
             to[state_elems + a.dp] = m_prev;
             to[state_elems + a.dp + 1] = decayed;
         }
@@ -571,7 +668,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : 2) void gated_c
         for (int r = rep0; r < reps && r < rep0 + (kCols + kRecCols - 1) / kRecCols; ++r) {
             float *np = to + state_elems + r * (a.dp + 16);
             put_n(np);
-            if (tid == 0) np[a.dp] = m_prev;
+            if (one) np[a.dp] = m_prev;
         }
     }
 }
@@ -714,6 +811,8 @@ extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const 
     a.heads = num_heads; a.dim = dim; a.vdim = vdim; a.dp = la_pad16(dim); a.vp = la_pad16(vdim);
     a.head_floats = (int64_t)gl_state_floats(kind == kMlstm, dim, vdim);
     a.segments = 1;
+    a.wide = dim % 8 == 0 && vdim % 8 == 0 && q_stride % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 &&
+             (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
     hipStream_t s = (hipStream_t)stream;
     // single rows, 32-bit rows, rows that are not whole 8-byte vectors, rows too far apart for 32-bit offsets
     const uintptr_t at = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out;

@@ -1,6 +1,7 @@
 // What the chunked linear-recurrence kernels share: 64-row tiles of bf16 rows loaded in 4 x 4 blocks and laid out in LDS
 // so that operands are whole reads in either direction, 32-bit factors as a sum of two bf16 terms, states as buffers.
 #pragma once
+#include <type_traits>
 #include "lightning_plan.h"
 #include "row_common.h"
 
@@ -80,6 +81,23 @@ __device__ __forceinline__ LaBlock la_load_block(__amdgpu_buffer_rsrc_t tile, ui
     return b;
 }
 
+// 16-byte pieces of rows `apart` rows apart from (row, column c) on.  wide: cols a multiple of 8 and rows 16-byte aligned; else in halves
+// (cols a multiple of 4, 8-byte aligned).
+template <int N> __device__ __forceinline__ void la_load_pieces(la_u4 (&x)[N], __amdgpu_buffer_rsrc_t tile, int64_t ld, int row, int c, int apart, int cols, bool wide) {
+    const uint32_t off = la_block_off(ld, row, c, cols), step = (uint32_t)apart * (uint32_t)ld * 2u;
+    if (wide) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) x[i] = __builtin_bit_cast(la_u4, __builtin_amdgcn_raw_buffer_load_b128(tile, off + i * step, 0, 0));
+    } else {
+        const uint32_t off2 = la_block_off(ld, row, c + 4, cols);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const la_u2 lo = __builtin_amdgcn_raw_buffer_load_b64(tile, off + i * step, 0, 0), hi = __builtin_amdgcn_raw_buffer_load_b64(tile, off2 + i * step, 0, 0);
+            x[i] = la_u4{lo[0], lo[1], hi[0], hi[1]};
+        }
+    }
+}
+
 // silu of a raw pair, packed again
 __device__ __forceinline__ uint32_t la_silu2(uint32_t w) {
     return row_pack_bf16(row_silu<pa_bf16>(__builtin_bit_cast(float, w << 16)),
@@ -111,6 +129,19 @@ template <int KD> __device__ __forceinline__ void la_put_hashed(const LaBlock &b
 }
 template <int KD> __device__ __forceinline__ bf8 la_read_hashed(const __bf16 *tile, int row, int chunk) {
     return la_read8(tile + row * KD + (chunk ^ la_hash<KD>(row)) * 8);
+}
+// The same places as bytes: a lane's place for the first 32 columns (of row `row`, of which a multiple of 16 may be added later; `low`: which
+// of their four chunks), and for the 32 columns number dd.  What follows from one place is one exclusive or, not an address kept for each.
+template <int KD> __device__ __forceinline__ int la_place_of(int row, int low) { return row * (KD * 2) + ((low ^ la_hash<KD>(row)) << 4); }
+template <int KD> __device__ __forceinline__ int la_place_at(int place, int dd) { return (place ^ (dd & 3) << 6) + (dd >> 2 << 8); }
+template <int KD> __device__ __forceinline__ bf8 la_read_place(const __bf16 *tile, int place, int row, int dd) {
+    return *reinterpret_cast<const bf8 *>(reinterpret_cast<const char *>(tile) + la_place_at<KD>(place, dd) + row * (KD * 2));
+}
+// Four rows, then four 16 further on, of column 8 (lane / 4 % 4) + 4 (dt % 2) + lane % 4 of the 32 number dt / 2: an operand whose partner's rows
+// are a lane's two result tiles in a row.  place: la_place_of(4 g + l16 / 4, l16 % 4)
+template <int KD> __device__ __forceinline__ bf8 la_read_place_tr(const __bf16 *tile, int place, int row, int dt) {
+    const __bf16 *at = reinterpret_cast<const __bf16 *>(reinterpret_cast<const char *>(tile) + la_place_at<KD>(place, dt / 2) + row * (KD * 2)) + dt % 2 * 4;
+    return la_join(la_read_tr(at), la_read_tr(at + 16 * KD));
 }
 // Row `row` (row % 16 = l16) of a paired tile, elements of the 32 columns from 32 dd on
 template <int KD> __device__ __forceinline__ bf8 la_read_paired(const __bf16 *tile, int row, int l16, int dd, int g) {

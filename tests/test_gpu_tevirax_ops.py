@@ -384,6 +384,25 @@ def test_long_portions_in_segments(kind, heads, dim, vdim, groups):
                 case.check_state(b, 1 + b)
 
 
+@pytest.mark.parametrize("kind,heads,dim,vdim,groups", [("mlstm", 2, 64, 64, None), ("mlstm", 1, 128, 136, None), ("mlstm", 2, 256, 72, None), ("mlstm", 1, 256, 128, None),
+                                                        ("mlstm", 1, 72, 200, None), ("ssd", 4, 64, 64, 1), ("ssd", 2, 128, 128, 2), ("ssd", 1, 256, 136, 1), ("ssd", 3, 40, 24, 1)])
+def test_rows_of_whole_pieces(kind, heads, dim, vdim, groups):
+    """Rows that are loaded 16 bytes at a time: chunks around 64 rows, in segments (the longest) and not, and states that go on."""
+    announce(f"gated pieces {kind} {heads}x{dim}x{vdim}")
+    lens = [1, 63, 64, 65, 129, 321]
+    case = Case(kind, lens, heads, dim, vdim, BF, groups, seed=8)
+    case.rows = [torch.nn.functional.pad(r, (0, -r.shape[1] % 8), value=float("nan")) for r in case.rows]
+    slots = [3, 0, 5, 1, 6, 2]
+    for use_ws in (True, False):
+        for cuts in ((0,), (0, 70)):  # (the last two sequences once in two portions)
+            for lo, hi in zip(cuts, cuts[1:] + (None,)):
+                picks = [(b, lo, (hi or n) - lo) for b, n in enumerate(lens) if n > 70 or len(cuts) == 1]
+                for (b, at, n), got in zip(picks, case.run(picks, slots, use_ws)):
+                    case.check(b, at, got)
+        for b in range(len(lens)):
+            case.check_state(b, slots[b])
+
+
 @pytest.mark.parametrize("dtype", [BF, F32])
 @pytest.mark.parametrize("kind", ["mlstm", "ssd"])
 def test_a_far_token_is_remembered(kind, dtype):
