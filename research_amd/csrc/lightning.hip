@@ -118,7 +118,7 @@ template <typename T, int R> __global__ __launch_bounds__(256) void lightning_re
 }
 
 // ------------------------------------------------------------------ chunks on the matrix cores
-// Elements of the tiles: K and Q (paired), V (row-major), the two terms of the decayed scores.
+// Elements of the tiles: K and Q (hashed), V (row-major), the two terms of the decayed scores.
 template <int KD, int NW> constexpr int la_kv_elems() { return 64 * KD + 64 * (16 * NW + kLaPadV); }
 template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
     const size_t elems = STATES ? 2 * la_kv_elems<KD, NW>()  // (double-buffered: one barrier per chunk)
@@ -129,25 +129,27 @@ template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
 // KD: dim padded to 64, 128 or 256.  NW: waves; each owns 16 value columns.  All products are taken transposed (value
 // columns, or keys, as the rows of the result), so that a lane holds four consecutive elements of one row t.
 // STATES: only the segment's own contribution to the state, to the workspace (first pass over a portion in segments).
-// Bound by the vector instructions that turn 32-bit factors into two bf16 terms and by the waits between the stages of a chunk
-// (the matrix cores are busy a sixth of the time).  So a tile lies in LDS in the one layout that both of its products read (K by
-// rows and, with transposing reads, by columns), results leave the registers straight for the output, and the first pass leaves out
-// each portion's last segment, whose state the second pass itself writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128,
-// in five segments: first pass 55 -> 47 us, second 127 -> 116 (41 and 94 since pieces are placed by their lengths).
+// Bound by the vector instructions: the silu of Q, K and V (two quarter-rate instructions an element) takes a SIMD 4800 of a chunk's 11600 cycles at
+// 128 x 128, the terms of 32-bit factors and the factors themselves 3500; the matrix cores work for 2700.  So rows come in 16-byte pieces and lie
+// in LDS as they are, in the one layout that both of a tile's products read, with operands ahead of their products and no branch in between; results
+// leave the registers straight for the output, and the first pass leaves out each portion's last segment, whose state the second pass itself
+// writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128, in five segments: first pass 41.3 -> 38.8 us, second 90.7 -> 87.2 (one read, one
+// product at a time, blocks of 4 x 4 -> this); 16 of 900 .. 1000 rows, 16 heads of 256 x 64, 138 -> 121; 10 of 28 .. 81, 32 heads of 128 x 64, 23.0 -> 20.9.
 // PAIR: at dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
-// chunk, let two share one.  Where segments outnumber the units: 6 prompts of 2164 .. 8112 rows, 16 heads of 128 x 128, all passes,
-// 294 -> 271 us; 4 of 1271 .. 5972, 40 heads of 96 x 80, 312 -> 281; over 70 batches up to 10 % faster, at most 2.5 % slower.  Elsewhere 3 to
-// 8 % slower.
+// chunk, let two share one.  Where segments outnumber the units: 6 prompts of 400 .. 2600 rows, 32 heads of 128 x 128, all passes,
+// 155 -> 144 us; 4 of 1271 .. 5972, 40 heads of 96 x 80, 259 -> 232.  Elsewhere up to 4 % slower.
 template <int KD, int NW, bool STATES, bool PAIR>
-__global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(const LaArgs a) {
+__global__ __launch_bounds__(64 * NW, PAIR || (KD == 64 && NW == 8) ? 4 : KD == 256 && NW == 4 ? 1 : 2) void lightning_chunk_kernel(const LaArgs a) {
     constexpr int kCols = 16 * NW, kLdV = kCols + kLaPadV, kThr = 64 * NW;
-    constexpr int kDB = KD / 4, kKBlocks = 16 * kDB, kKPass = (kKBlocks + kThr - 1) / kThr;  // 4x4 blocks of K
+    constexpr int kKP = 64 * (KD / 8) / kThr, kKRows = kThr / (KD / 8);  // 16-byte pieces of K per thread, rows between them; of V: two
+    constexpr int kVRows = kThr / (kCols / 8);
+    static_assert(kKP * kThr == 64 * (KD / 8) && 2 * kVRows == 64, "whole passes");
+    constexpr bool kTight = !STATES && (PAIR || (KD == 64 && NW == 8));  // 128 registers
+    // The next tile's silu beside the products of the state, or as the tile goes to LDS (8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128, us: first pass
+    // 42.8 and 38.8, second 87.2 and 91.6; 13 of 157 .. 258 rows, 32 heads of 64 x 64, both in one 26.3 and 25.1)
+    constexpr bool kBeside = !STATES && !PAIR && KD == 128 && NW == 8;
+    constexpr int kGroup = kTight ? 2 : 4, kGroups = KD / 16 / kGroup;  // state tiles whose products go together
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
-    // Places in memory and in LDS are worked out again where registers run out (16 prompts of 900 .. 1000 rows, 16 heads of 256 x 64:
-    // 141 us, else 236), those in LDS also at dim 64, where two workgroups of eight waves share a compute unit only so (16 heads of
-    // 64 x 128, 9 prompts of 700 .. 4000 rows: 129 us, else 147); elsewhere they are kept (one prompt of 2000 rows, 16 heads of 128 x 128,
-    // 67.9, else 71.3; 32 of 128 x 64, 121, else 125).
-    constexpr bool kFar = PAIR || (KD == 256 && NW == 4), kAgain = kFar || KD == 64;
     extern __shared__ __align__(16) char lds[];
     float *rev = reinterpret_cast<float *>(lds);  // decay from row s to the last row of a whole chunk ...
     float *rev_tail = rev + 64;                   // ... and of a portion's last chunk
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     // (what a portion's last segment adds is for nobody else: the second pass leaves the state behind it)
     const bool last = r_end == p.n;
     if (r_beg >= p.n || (STATES && last)) return;
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int v0 = vsl * kCols, vw = wave * 16;  // first column of the workgroup, of the wave inside it
     const float *powers = a.decay + h * (kLaChunk + 1);
     if (tid <= kLaChunk) pw[tid] = powers[tid];
@@ -172,13 +174,11 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
         rev[tid] = powers[63 - tid];
         pw[tid - 64] = 0.f;
     }
-    const int l16 = tid & 15, g = (tid & 63) >> 4;
-    float pt[4];  // decay from the chunk's start to row 16 tt + l16
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) pt[tt] = powers[16 * tt + l16 + 1];
+    const int l16 = tid & 15, g = lane >> 4;
 
-    // The state slice of this wave: tile dt holds d = 16 dt + 4 g + i, v = v0 + vw + l16
+    // The state slice of this wave: tile dt holds d = 32 (dt / 2) + 8 g + 4 (dt % 2) + i, v = v0 + vw + l16
     f4 s[KD / 16];
+    auto s_row = [](int dt, int i) { return 32 * (dt / 2) + 4 * (dt % 2) + i; };
     const int64_t state_elems = (int64_t)a.dp * a.vp;
     float *pool = p.slot >= 0 ? a.state + (p.slot * a.heads + h) * state_elems : nullptr;
     float *seg_state = a.segments > 1 ? a.ws + (((int64_t)b * a.heads + h) * a.segments + seg) * state_elems : nullptr;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
     // (a state as a buffer: rows past dp lie past its end, columns past vp get an offset outside)
     const int state_bytes = (int)state_elems * 4;
     const int v = v0 + vw + l16;
-    const uint32_t soff = v < a.vp ? (uint32_t)(4 * g * a.vp + v) * 4u : kLaOutside;
+    const uint32_t soff = v < a.vp ? (uint32_t)(8 * g * a.vp + v) * 4u : kLaOutside;
     {
         const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(from ? from : a.state), 0, from ? state_bytes : 0, 0x00020000);  // (no state: every load is past the end)
@@ -194,84 +194,141 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
         for (int dt = 0; dt < KD / 16; ++dt)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + (16 * dt + i) * a.vp * 4, 0, 0));
+                s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + s_row(dt, i) * a.vp * 4, 0, 0));
     }
 
     const uint16_t *u = reinterpret_cast<const uint16_t *>(a.u) + p.row0 * a.ldu;
     const uint16_t *uq = u + h * a.dim, *uk = u + (a.heads + h) * a.dim;
     const uint16_t *uv = u + 2 * a.heads * a.dim + h * a.vdim + v0;
     const int vcols = a.vdim - v0 < kCols ? a.vdim - v0 : kCols;
-    const uint32_t row_bytes = (uint32_t)a.ldu * 2u;
-    LaBlock kb[kKPass], qb[STATES ? 1 : kKPass], vb;
-    auto fetch = [&](int r0) {
-        const int rows = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
-        const int64_t at = (int64_t)r0 * a.ldu;
-        const int ft = kFar ? la_again(tid) : tid;
-        auto koff = [&](int i) {
-            const int blk = ft + kThr * i;
-            return blk < kKBlocks ? la_block_off(a.ldu, blk / kDB * 4, blk % kDB * 4, a.dim) : kLaOutside;
-        };
-        const __amdgpu_buffer_rsrc_t tk = la_tile(uk + at, a.ldu, rows, a.dim), tv = la_tile(uv + at, a.ldu, rows, vcols);
-        if (!STATES) {
-            const __amdgpu_buffer_rsrc_t tq = la_tile(uq + at, a.ldu, rows, a.dim);
+    la_u4 kb[kKP], qb[STATES ? 1 : kKP], vb[2];
+    // PAIR: what follows from a thread's number is made again wherever it is asked for
+    auto thread = [&] { return PAIR ? la_again(tid) : tid; };
+    auto fetch_rows = [&](auto &x, const uint16_t *base, int r0, int per_row, int apart, int cols) {
+        const int rows = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk, t = thread();
+        la_load_pieces(x, la_tile(base + (int64_t)r0 * a.ldu, a.ldu, rows, cols), a.ldu, t / per_row, t % per_row * 8, apart, cols, true);
+    };
+    auto fetch_q = [&](int r0) { fetch_rows(qb, uq, r0, KD / 8, kKRows, a.dim); };
+    auto fetch_k = [&](int r0) { fetch_rows(kb, uk, r0, KD / 8, kKRows, a.dim); };
+    auto fetch_v = [&](int r0) { fetch_rows(vb, uv, r0, kCols / 8, kVRows, vcols); };
+    auto put = [&] {
+        const int t = thread(), kr = t / (KD / 8), kc = t % (KD / 8), vr = t / (kCols / 8), vc = t % (kCols / 8);
 #pragma unroll
-            for (int i = 0; i < kKPass; ++i) qb[i] = la_load_block(tq, koff(i), row_bytes);
+        for (int i = 0; i < kKP; ++i) {  // (rows 16 apart have the same hash)
+            const int row = kr + (kKRows % 16 == 0 ? 0 : i * kKRows), to = row * KD + (kc ^ la_hash<KD>(row)) * 8 + (kKRows % 16 == 0 ? i * kKRows * KD : 0);
+            *reinterpret_cast<la_u4 *>(k_s + to) = kb[i];
+            if (!STATES) *reinterpret_cast<la_u4 *>(q_s + to) = qb[i];
         }
 #pragma unroll
-        for (int i = 0; i < kKPass; ++i) kb[i] = la_load_block(tk, koff(i), row_bytes);
-        vb = la_load_block(tv, la_block_off(a.ldu, ft / (kCols / 4) * 4, ft % (kCols / 4) * 4, vcols), row_bytes);
+        for (int i = 0; i < 2; ++i) *reinterpret_cast<la_u4 *>(v_s + (vr + i * kVRows) * kLdV + vc * 8) = vb[i];
     };
-    fetch(r_beg);
+    const int row_place = PAIR ? 0 : la_place_of<KD>(l16, g), tr_place = PAIR ? 0 : la_place_of<KD>(4 * g + l16 / 4, l16 % 4);
+    auto rows_at = [&] { const int t = thread(); return PAIR ? la_place_of<KD>(t & 15, (t & 63) >> 4) : la_again(row_place); };
+    auto tr_at = [&] { const int t = thread(); return PAIR ? la_place_of<KD>((t & 63) >> 2, t & 3) : la_again(tr_place); };
+    if (!STATES) fetch_q(r_beg);
+    fetch_k(r_beg);
+    fetch_v(r_beg);
+    // The silu of a tile, in its registers and in kActs equal parts
+    constexpr int kActs = 2 * kGroups, kPieces = (STATES ? 1 : 2) * kKP + 2;
+    auto act_part = [&](int part) {
+#pragma unroll
+        for (int i = 0; i < 4 * kPieces; ++i) {
+            if (i * kActs / (4 * kPieces) != part) continue;
+            la_u4 &x = i < 8 ? vb[i / 4] : i < 8 + 4 * kKP ? kb[(i - 8) / 4] : qb[STATES ? 0 : (i - 8 - 4 * kKP) / 4];
+            x[i % 4] = la_silu2(x[i % 4]);
+        }
+    };
+    auto act_all = [&] {
+#pragma unroll
+        for (int part = 0; part < kActs; ++part) act_part(part);
+    };
+    if (kBeside) act_all();
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
-        const int lt = kAgain ? la_again(tid) : tid;
-#pragma unroll
-        for (int i = 0; i < kKPass; ++i) {
-            const int blk = lt + kThr * i, c = blk % kDB * 4, sr = blk / kDB * 4;
-            if (kKBlocks % kThr != 0 && blk >= kKBlocks) continue;
-            la_put_paired<true, KD>(kb[i], sr, c, k_s);
-            if (!STATES) la_put_paired<true, KD>(qb[i], sr, c, q_s);
-        }
-        la_put_block<true>(vb, lt / (kCols / 4) * 4, lt % (kCols / 4) * 4, v_s, kLdV);
+        const bool more = r0 + kLaChunk < r_end;
+        if (!kBeside) act_all();
+        put();
         if (nv < kLaChunk && tid < 64) rev_tail[tid] = tid < nv ? powers[nv - 1 - tid] : 0.f;
-        if (r0 + kLaChunk < r_end) fetch(r0 + kLaChunk);
         __syncthreads();
 
-        const int lr = PAIR ? la_again(tid) : tid, l16 = lr & 15, g = (lr & 63) >> 4;
+        const int lt = thread(), l16 = lt & 15, g = (lt & 63) >> 4;
+        bf8 av[2];  // V: the wave's columns as rows
+        auto read_v = [&] {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) av[kk] = la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g);
+        };
+        if (!kTight) read_v();
         f4 o[4];  // O^T: v = 4 g + i of the wave's columns, t = 16 tt + l16
-        if constexpr (!STATES) {
+        if constexpr (STATES) {
+            if (more) {
+                fetch_k(r0 + kLaChunk);
+                fetch_v(r0 + kLaChunk);
+            }
+        } else {
             // score tiles (st, rt): keys 16 st + 4 g + i, rows 16 rt + l16
             const int rt = NW == 8 ? wave >> 1 : wave;
             f4 sc[kST];
 #pragma unroll
             for (int m = 0; m < kST; ++m) sc[m] = f4{0.f, 0.f, 0.f, 0.f};
+            // (no branch inside: each product would wait for its own read)
+            auto scores = [&](auto count) {
+                constexpr int kN = decltype(count)::value;
+                bf8 bq[2], ak[2][kN];
+                const int at = rows_at(), at_q = at + rt * (32 * KD), at_k = at + (NW == 8 ? wave & 1 : 0) * (32 * KD);
+                auto read = [&](int kk) {
+                    bq[kk & 1] = la_read_place<KD>(q_s, at_q, 0, kk);
 #pragma unroll
-            for (int kk = 0; kk < KD / 32; ++kk) {
-                const bf8 bq = la_read_paired<KD>(q_s, 16 * rt + l16, l16, kk, g);
+                    for (int m = 0; m < kN; ++m) ak[kk & 1][m] = la_read_place<KD>(k_s, at_k, 16 * (NW == 8 ? 2 * m : m), kk);
+                };
+                read(0);
 #pragma unroll
-                for (int m = 0; m < kST; ++m) {
-                    const int st = NW == 8 ? 2 * m + (wave & 1) : m;
-                    if (st <= rt) sc[m] = la_mfma(la_read_paired<KD>(k_s, 16 * st + l16, l16, kk, g), bq, sc[m]);
+                for (int kk = 0; kk < KD / 32; ++kk) {
+                    if (kk + 1 < KD / 32) read(kk + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < kN; ++m) sc[m] = la_mfma(ak[kk & 1][m], bq[kk & 1], sc[m]);
                 }
-            }
-            // the rows' part from before the chunk: Q S, then the decay of the way from the chunk's start
+            };
+            if (rt >= 2) scores(std::integral_constant<int, kST>());
+            else scores(std::integral_constant<int, kST / 2>());
+            // the rows' part from before the chunk: Q S, then the decay of the way from the chunk's start (a sequence's first chunk has none)
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) o[tt] = f4{0.f, 0.f, 0.f, 0.f};
+            if (!from && r0 == r_beg) {
+                if (more) {
+                    fetch_q(r0 + kLaChunk);
+                    fetch_k(r0 + kLaChunk);
+                }
+            } else {
+                bf8 bq[2][4];
+                const int at = rows_at();
+                auto read = [&](int dd) {
 #pragma unroll
-            for (int dd = 0; dd < KD / 32; ++dd) {
-                const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
-                const bf8 hi = sp.high(), lo = sp.low();
+                    for (int tt = 0; tt < 4; ++tt) bq[dd & 1][tt] = la_read_place<KD>(q_s, at, 16 * tt, dd);
+                };
+                read(0);
+                if (more) fetch_q(r0 + kLaChunk);
 #pragma unroll
-                for (int tt = 0; tt < 4; ++tt) {
-                    const bf8 bq = la_read_paired<KD>(q_s, 16 * tt + l16, l16, dd, g);
-                    o[tt] = la_mfma(hi, bq, o[tt]);
-                    o[tt] = la_mfma(lo, bq, o[tt]);
+                for (int dd = 0; dd < KD / 32; ++dd) {
+                    if (!kTight && dd + 1 < KD / 32) read(dd + 1);
+                    if (kTight && dd) read(dd);
+                    const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
+                    const bf8 hi = sp.high(), lo = sp.low();
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) o[tt] = la_mfma(hi, bq[dd & 1][tt], o[tt]);
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt) o[tt] = la_mfma(lo, bq[dd & 1][tt], o[tt]);
+                    if (dd == KD / 64 && more) fetch_k(r0 + kLaChunk);
                 }
             }
+            if (more) fetch_v(r0 + kLaChunk);
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
+            for (int tt = 0; tt < 4; ++tt) {
+                const float f = pw[16 * tt + l16 + 1];  // decay from the chunk's start to the row
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[tt][i] *= pt[tt];
+                for (int i = 0; i < 4; ++i) o[tt][i] *= f;
+            }
 #pragma unroll
             for (int m = 0; m < kST; ++m) {
                 const int st = NW == 8 ? 2 * m + (wave & 1) : m;
@@ -285,14 +342,24 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
                 *reinterpret_cast<uint2 *>(a_lo + t * kLaPitchA + la_paired(c)) = lo;
             }
             __syncthreads();
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const bf8 av = la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g);
+            if (kTight) read_v();
+            bf8 ah[2][4], al[2][4];  // (all reads ahead of the products)
+            auto read = [&](int kk) {
 #pragma unroll
                 for (int tt = 2 * kk; tt < 4; ++tt) {
-                    o[tt] = la_mfma(av, la_read8(a_hi + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
-                    o[tt] = la_mfma(av, la_read8(a_lo + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g), o[tt]);
+                    ah[kk][tt] = la_read8(a_hi + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g);
+                    al[kk][tt] = la_read8(a_lo + (16 * tt + l16) * kLaPitchA + 32 * kk + 8 * g);
                 }
+            };
+            read(0);
+            if (!kTight) read(1);
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                if (kTight && kk) read(1);
+#pragma unroll
+                for (int tt = 2 * kk; tt < 4; ++tt) o[tt] = la_mfma(av[kk], ah[kk][tt], o[tt]);
+#pragma unroll
+                for (int tt = 2 * kk; tt < 4; ++tt) o[tt] = la_mfma(av[kk], al[kk][tt], o[tt]);
             }
             const int ldo = a.heads * a.vdim, c = vw + 4 * g;
             const uint16_t *first = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0) * (int64_t)ldo + h * a.vdim + v0;
@@ -304,24 +371,44 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
             }
         }
         // S <- decay^nv S + K^T (decay^(nv-1-s) V)
+        // (operands a group of tiles ahead of their products)
+        bf8 ak[2][kGroup];
+        const int at = tr_at();
+        auto read = [&](int step) {  // (kk, group)
+#pragma unroll
+            for (int j = 0; j < kGroup; ++j) ak[step & 1][j] = la_read_place_tr<KD>(k_s, at, 32 * (step / kGroups), step % kGroups * kGroup + j);
+        };
+        read(0);
         const float whole = pw[nv];
         const float *wt = nv < kLaChunk ? rev_tail : rev;
+        auto keep = [&](int group) {
 #pragma unroll
-        for (int dt = 0; dt < KD / 16; ++dt)
+            for (int dt = group * kGroup; dt < (group + 1) * kGroup; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
+                for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
+        };
+        keep(0);
+        auto move_on = [&](auto next) {  // (next: the next tile's silu beside the products)
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const LaSplit sp = la_split_weighted(la_read_rows_tr(v_s, kLdV, 32 * kk, vw, l16, g), *reinterpret_cast<const f4 *>(wt + 32 * kk + 4 * g),
-                                                 *reinterpret_cast<const f4 *>(wt + 32 * kk + 16 + 4 * g));
-            const bf8 hi = sp.high(), lo = sp.low();
+            for (int kk = 0; kk < 2; ++kk) {
+                const LaSplit sp = la_split_weighted(av[kk], *reinterpret_cast<const f4 *>(wt + 32 * kk + 4 * g), *reinterpret_cast<const f4 *>(wt + 32 * kk + 16 + 4 * g));
+                const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
-            for (int dt = 0; dt < KD / 16; ++dt) {
-                const bf8 ak = la_read_paired_tr<KD>(k_s, 32 * kk, dt, l16, g);
-                s[dt] = la_mfma(ak, hi, s[dt]);
-                s[dt] = la_mfma(ak, lo, s[dt]);
+                for (int x = 0; x < kGroups; ++x) {
+                    const int step = kk * kGroups + x;
+                    if (step + 1 < 2 * kGroups) read(step + 1);
+                    if (step + 1 < kGroups) keep(step + 1);
+                    if (decltype(next)::value) act_part(step);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], hi, s[x * kGroup + j]);
+#pragma unroll
+                    for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], lo, s[x * kGroup + j]);
+                }
             }
-        }
+        };
+        if (kBeside && more) move_on(std::integral_constant<bool, kBeside>());
+        else move_on(std::false_type());
         if constexpr (!STATES) {
             __syncthreads();  // the next chunk's tiles may be written now
         } else {              // the other half of the tiles
@@ -339,7 +426,7 @@ __global__ __launch_bounds__(64 * NW, PAIR ? 4 : 2) void lightning_chunk_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float f = s[dt][i];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), dst, base + (16 * dt + i) * a.vp * 4, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), dst, base + s_row(dt, i) * a.vp * 4, 0, 0);
         }
 }
 
