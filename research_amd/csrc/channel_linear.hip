@@ -144,7 +144,10 @@ constexpr float kClSmall = 0x1p-100f;  // a block whose P falls below has its sc
 template <int KD, int NW, bool STATES> struct ClTile {
     static constexpr int rows = KD == 256 ? 32 : 64, blocks = rows / kClBlock, cols = 16 * NW, threads = 64 * NW;
     static constexpr int pitch = KD + 8, vPitch = cols + kLaPadV;
-    static constexpr int pitchK = KD + 16;  // (R K is read by transposing reads alone: rows 32 modulo 64 bytes apart)
+    // R K is read by transposing reads alone, whose 32 lanes ask for four pieces of 8 bytes, 16 bytes apart, of each of eight rows: rows lie 64 bytes
+    // apart modulo 256, and in every second four of them the 8-byte halves of 16 change places.  Two octets of rows are written at once: in every
+    // second one the 128-byte halves of 256 change places (dim 64 has none).
+    static constexpr int pitchK = KD + 32, flipK = KD >= 128 ? 64 : 0;
     static constexpr int elems = rows * pitch, elemsK = rows * pitchK;  // one bf16 term of a tile
     static constexpr int units = KD / 2 * rows / 8;                  // (channel pair, 8 rows)
     static constexpr int passes = (units + threads - 1) / threads;
@@ -187,11 +190,15 @@ template <int KD> __device__ __noinline__ f4 cl_slow_scores(const uint16_t *uq, 
     return out;
 }
 
-// Bound by the vector unit: per row and channel the gate, three products split into two terms each and q's activation, and per block and wave its
-// part of S split again.  So 1 / P is made once per block instead of by row (P R = B), a last chunk's missing rows are masked in that chunk
-// alone, and the blocks of a chunk are unrolled, with the state's update and the outputs of one block as independent chains between them
-// (outputs of the next block ahead of the barrier behind the scores were slower: they wait for the update).  8 prompts of 700 .. 4000 rows,
-// 32 heads of 128 x 128, both passes: 463 -> 409 us, and 401 with R K at a pitch that its reads spread over the banks.
+// Bound by the vector unit: per row and channel the gate, three products split into two terms each and q's activation (5600 of a chunk's 17000
+// cycles, no products beside them), and per block and wave its part of S split again.  So 1 / P is made once per block instead of by row (P R = B), a
+// last chunk's missing rows are masked in that chunk alone, and the blocks of a chunk are unrolled, with the state's update and the outputs of one
+// block as independent chains between them.  The scores, which four waves make, are asked for behind the last block, and with that barrier a chunk
+// has two: what follows it reads registers and scores alone.  The next rows' loads are spread over the blocks; no place is kept that would be
+// spilled, as a reload waits for the loads before it.  8 prompts of 700 .. 4000 rows, 32 heads of 128 x 128, second pass: 295 -> 266 us (scores ahead of the
+// blocks, three barriers, one accumulator -> this), 33 of 150 .. 168 rows, 32 heads of 96 x 80, 175 -> 156.
+// Two blocks at a time, whose state is split once, needs P Q of the second from the first one's start as well and is spilled: 449 us for both passes,
+// else 377.
 // STATES: only the segment's own contribution to the state and its factors, to the workspace (first pass over a portion in
 // segments).
 template <int KD, int NW, bool STATES>
@@ -219,15 +226,16 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     const int v0 = vsl * L::cols, vw = wave * 16;  // first column of the workgroup, of the wave inside it
     const int l16 = lane & 15, g = lane >> 4;
 
-    // The state slice of this wave: tile dt holds d = 16 dt + 4 g + i, v = v0 + vw + l16
+    // The state slice of this wave: tile dt holds d = 32 (dt / 2) + 8 g + 4 (dt % 2) + i, v = v0 + vw + l16
     f4 s[KD / 16];
+    auto s_row = [](int dt, int i) { return 32 * (dt / 2) + 4 * (dt % 2) + i; };
     const int64_t state_elems = (int64_t)a.dp * a.vp;
     float *pool = p.slot >= 0 ? a.state + (p.slot * a.heads + h) * state_elems : nullptr;
     float *seg_state = a.segments > 1 ? a.ws + (((int64_t)b * a.heads + h) * a.segments + seg) * (state_elems + a.dp + 16) : nullptr;
     const float *from = STATES ? nullptr : (a.segments > 1 ? seg_state : (p.pos0 > 0 ? pool : nullptr));
     // (a state as a buffer: rows past dp lie past its end, columns past vp get an offset outside)
     const int state_bytes = (int)state_elems * 4, v = v0 + vw + l16;
-    const uint32_t soff = v < a.vp ? (uint32_t)(4 * g * a.vp + v) * 4u : kLaOutside;
+    const uint32_t soff = v < a.vp ? (uint32_t)(8 * g * a.vp + v) * 4u : kLaOutside;
     {
         const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(from ? from : a.state), 0, from ? state_bytes : 0, 0x00020000);  // (no state: every load is past the end)
@@ -235,7 +243,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
         for (int dt = 0; dt < KD / 16; ++dt)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + (16 * dt + i) * a.vp * 4, 0, 0));
+                s[dt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, soff + s_row(dt, i) * a.vp * 4, 0, 0));
     }
     float decayed = 1.f;  // STATES: the segment's factor of channel tid
 
@@ -263,28 +271,35 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     }
     uint32_t zr[L::passes][8], qr[STATES ? 1 : L::passes][8];
     la_u2 vr[L::vLoads];
-    auto fetch = [&](int r0) {
+    auto fetch_pairs = [&](uint32_t (&x)[8], const uint16_t *base, int64_t ld, int r0, int u) {
         const int nr = r_end - r0 < kRows ? r_end - r0 : kRows;
-        const __amdgpu_buffer_rsrc_t tz = la_tile(uz + r0 * a.ldz, a.ldz, nr, a.dim), tv = la_tile(uv + r0 * a.ldv, a.ldv, nr, vcols);
-        const __amdgpu_buffer_rsrc_t tq = la_tile(uq + r0 * a.ldq, a.ldq, nr, a.dim);
+        const __amdgpu_buffer_rsrc_t t = la_tile(base + r0 * ld, ld, nr, a.dim);
+        const uint32_t off = 2 * pair[u] < a.dim ? (uint32_t)(8 * oct[u] * ld + 2 * pair[u]) * 2u : kLaOutside;
 #pragma unroll
-        for (int u = 0; u < L::passes; ++u) {
-            if (!mine[u]) continue;
-            const bool there = 2 * pair[u] < a.dim;
+        for (int r = 0; r < 8; ++r) x[r] = __builtin_amdgcn_raw_buffer_load_b32(t, off + r * (int)ld * 2, 0, 0);
+    };
+    auto fetch_z = [&](int r0) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                zr[u][r] = __builtin_amdgcn_raw_buffer_load_b32(tz, there ? (uint32_t)((8 * oct[u] + r) * a.ldz + 2 * pair[u]) * 2u : kLaOutside, 0, 0);
-                if constexpr (!STATES)
-                    qr[u][r] = __builtin_amdgcn_raw_buffer_load_b32(tq, there ? (uint32_t)((8 * oct[u] + r) * a.ldq + 2 * pair[u]) * 2u : kLaOutside, 0, 0);
-            }
-        }
+        for (int u = 0; u < L::passes; ++u)
+            if (mine[u]) fetch_pairs(zr[u], uz, a.ldz, r0, u);
+    };
+    auto fetch_q = [&](int r0) {
+#pragma unroll
+        for (int u = 0; u < L::passes; ++u)
+            if (!STATES && mine[u]) fetch_pairs(qr[STATES ? 0 : u], uq, a.ldq, r0, u);
+    };
+    auto fetch_v = [&](int r0) {
+        const __amdgpu_buffer_rsrc_t tv = la_tile(uv + r0 * a.ldv, a.ldv, r_end - r0 < kRows ? r_end - r0 : kRows, vcols);
+        const int t = la_again(tid);  // (kept, these places were spilled, and a reload waits for all loads before it)
 #pragma unroll
         for (int n = 0; n < L::vLoads; ++n) {
-            const int c = tid + kThr * n, row = c / (L::cols / 4), col = c % (L::cols / 4) * 4;
+            const int c = t + kThr * n, row = c / (L::cols / 4), col = c % (L::cols / 4) * 4;
             vr[n] = __builtin_amdgcn_raw_buffer_load_b64(tv, la_block_off(a.ldv, row, col, vcols), 0, 0);
         }
     };
-    fetch(r_beg);
+    fetch_z(r_beg);
+    fetch_q(r_beg);
+    fetch_v(r_beg);
     for (int r0 = r_beg; r0 < r_end; r0 += kRows) {
         const int nv = r_end - r0 < kRows ? r_end - r0 : kRows;
         // ---- operands ----
@@ -329,7 +344,9 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 const bool any = __ballot(bad) != 0;
                 if (lane == 0) unsafe[wave + NW * u] = any;
             }
-            uint32_t *dst_k = reinterpret_cast<uint32_t *>(k_hi) + (8 * oct[u] * L::pitchK) / 2 + pair[u];
+            const int pair_k = pair[u] ^ (oct[u] & 1) * (L::flipK / 2);
+            uint32_t *dst_k = reinterpret_cast<uint32_t *>(k_hi) + (8 * oct[u] * L::pitchK) / 2 + pair_k;
+            uint32_t *dst_k2 = reinterpret_cast<uint32_t *>(k_hi) + (8 * oct[u] * L::pitchK) / 2 + (pair_k ^ 2);  // (rows 4 .. 7)
             uint32_t *dst = reinterpret_cast<uint32_t *>(q_hi) + (8 * oct[u] * kPitch) / 2 + pair[u];
             constexpr int kRow = kPitch / 2, kTerm = L::elems / 2, kRowK = L::pitchK / 2, kTermK = L::elemsK / 2;
 #pragma unroll
@@ -337,8 +354,8 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 const float x = k[r][0] * back[0], y = k[r][1] * back[1];
                 uint32_t hi, lo;
                 la_split2(x, y, hi, lo);
-                dst_k[r * kRowK] = hi;
-                dst_k[kTermK + r * kRowK] = lo;
+                (r < 4 ? dst_k : dst_k2)[r * kRowK] = hi;
+                (r < 4 ? dst_k : dst_k2)[kTermK + r * kRowK] = lo;
                 if constexpr (!STATES) {
                     la_split2(k[r][0] * open[0] * back[0], k[r][1] * open[1] * back[1], hi, lo);
                     dst[2 * kTerm + r * kRow] = hi;
@@ -366,12 +383,17 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 }
             }
         }
+        const int vt = la_again(tid);
 #pragma unroll
         for (int n = 0; n < L::vLoads; ++n) {
-            const int c = tid + kThr * n, row = c / (L::cols / 4), col = c % (L::cols / 4) * 4;
+            const int c = vt + kThr * n, row = c / (L::cols / 4), col = c % (L::cols / 4) * 4;
             *reinterpret_cast<la_u2 *>(v_s + row * L::vPitch + col) = vr[n];
         }
-        if (r0 + kRows < r_end) fetch(r0 + kRows);
+        const bool more = r0 + kRows < r_end;
+        if (STATES && more) {
+            fetch_z(r0 + kRows);
+            fetch_v(r0 + kRows);
+        }
         __syncthreads();
         if constexpr (!STATES) {
             // ---- scores: keys 4 g + i, row l16 of the wave's block ----
@@ -381,7 +403,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 int bad = 0;
 #pragma unroll
                 for (int i = 0; i < kPairs / 32; ++i) bad |= unsafe[wave * (kPairs / 32) + i];
-                if (__builtin_amdgcn_readfirstlane(bad) == 0) {
+                if (__builtin_expect(__builtin_amdgcn_readfirstlane(bad) == 0, 1)) {  // (a likely call would put the loop's scalars into vector registers: 387 us, else 377)
 #pragma unroll
                     for (int kk = 0; kk < KD / 32; ++kk) {
                         const int at = (first + l16) * kPitch + 32 * kk + 8 * g;
@@ -403,52 +425,74 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 la_split2(sc[2], sc[3], x.y, x.w);
                 scores[wave * 64 + lane] = x;
             }
-            __syncthreads();
         }
-        // ---- blocks in turn; every wave its own columns ----
+        // ---- blocks in turn; every wave its own columns.  (The scores are asked for behind the last one, so that the waves that make them and the
+        // others do not wait for each other here; the next rows' loads are spread over the blocks.)
+        f4 o[STATES ? 1 : L::blocks];  // v = 4 g + i of the wave's columns, t = l16
+        la_bf4 v4[L::blocks];          // V^T or V: rows 4 g .. 4 g + 3 of the block, column l16 of the wave
 #pragma unroll
         for (int blk = 0; blk < L::blocks; ++blk) {
             if (blk * kClBlock >= nv) break;
             const int first = blk * kClBlock;
-            // V^T or V: rows 4 g .. 4 g + 3 of the block, column l16 of the wave, once for each term beside it
-            const la_bf4 v4 = la_read_tr(v_s + (first + 4 * g + (l16 >> 2)) * L::vPitch + vw + 4 * (l16 & 3));
-            const bf8 v8 = la_join(v4, v4);
+            v4[blk] = la_read_tr(v_s + (first + 4 * g + (l16 >> 2)) * L::vPitch + vw + 4 * (l16 & 3));
+            const bf8 v8 = la_join(v4[blk], v4[blk]);  // (once for each term beside it)
             if constexpr (!STATES) {
-                f4 o = f4{0.f, 0.f, 0.f, 0.f};  // v = 4 g + i of the wave's columns, t = l16
+                o[blk] = f4{0.f, 0.f, 0.f, 0.f};
+                if (blk > 0 || from || r0 > r_beg) {  // (else there is no state yet)
+                    const __bf16 *qh = q_hi + (first + l16) * kPitch + 8 * g, *ql = qh + L::elems;
+                    f4 o1 = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int dd = 0; dd < KD / 32; ++dd) {
-                    LaSplit sp;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        la_split2(s[2 * dd + j / 2][2 * j % 4], s[2 * dd + j / 2][2 * j % 4 + 1], sp.hi[j], sp.lo[j]);
-                    const bf8 hi = sp.high(), lo = sp.low();
-                    const int at = (first + l16) * kPitch + 32 * dd + 4 * g;
-                    const bf8 qh = la_read44(q_hi + at, q_hi + at + 16), ql = la_read44(q_lo + at, q_lo + at + 16);
-                    o = la_mfma(lo, qh, o);
-                    o = la_mfma(hi, ql, o);
-                    o = la_mfma(hi, qh, o);
+                    for (int dd = 0; dd < KD / 32; ++dd) {
+                        const LaSplit sp = la_split_pair(s[2 * dd], s[2 * dd + 1]);
+                        const bf8 hi = sp.high(), lo = sp.low(), xh = la_read8(qh + 32 * dd), xl = la_read8(ql + 32 * dd);
+                        o1 = la_mfma(lo, xh, o1);
+                        o[blk] = la_mfma(hi, xh, o[blk]);
+                        o1 = la_mfma(hi, xl, o1);
+                    }
+                    o[blk] += o1;
                 }
-                o = la_mfma(v8, __builtin_bit_cast(bf8, scores[blk * 64 + lane]), o);
+            }
+            const float *keep = whole + blk * KD + 8 * g;
+            const __bf16 *kh = k_hi + (first + 4 * g + (l16 >> 2)) * L::pitchK + 8 * (l16 & 3);
+            const __bf16 *half[2][2];  // [dt % 2][dt / 4 % 2]
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) half[x][y] = kh + 4 * (x ^ (g & 1)) + (L::flipK ? 64 * (y ^ (g >> 1)) : 64 * y);
+#pragma unroll
+            for (int dt = 0; dt < KD / 16; ++dt) {
+                const int at = 32 * (dt / 2) + 4 * (dt % 2);
+                const f4 f = *reinterpret_cast<const f4 *>(keep + at);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[dt][i] *= f[i];
+                const __bf16 *x = half[dt % 2][dt / 4 % 2] + dt / 8 * 128 + dt / 2 % 2 * 32;
+                s[dt] = la_mfma(la_join(la_read_tr(x), la_read_tr(x + L::elemsK)), v8, s[dt]);
+            }
+            if (!STATES && more) {
+                if (blk == 0) fetch_z(r0 + kRows);
+                if (blk == 1) fetch_q(r0 + kRows);
+                if (blk == L::blocks - 1) fetch_v(r0 + kRows);
+            }
+        }
+        if constexpr (!STATES) {
+            __syncthreads();  // the scores are there; the next rows' operands may be written now
+#pragma unroll
+            for (int blk = 0; blk < L::blocks; ++blk) {
+                if (blk * kClBlock >= nv) break;
+                const int first = blk * kClBlock;
+                o[blk] = la_mfma(la_join(v4[blk], v4[blk]), __builtin_bit_cast(bf8, scores[blk * 64 + lane]), o[blk]);
                 const int ldo = a.heads * a.vdim, c = vw + 4 * g;
                 const uint16_t *out = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0 + first) * (int64_t)ldo + h * a.vdim + v0;
                 const int n = nv - first < kClBlock ? nv - first : kClBlock;
                 const __amdgpu_buffer_rsrc_t dst = la_tile(out, ldo, n, vcols);
-                const la_u2 x = {row_pack_bf16(o[0], o[1]), row_pack_bf16(o[2], o[3])};
+                const la_u2 x = {row_pack_bf16(o[blk][0], o[blk][1]), row_pack_bf16(o[blk][2], o[blk][3])};
                 __builtin_amdgcn_raw_buffer_store_b64(x, dst, c < vcols ? (uint32_t)(l16 * ldo + c) * 2u : kLaOutside, 0, 0);
             }
-            const float *keep = whole + blk * KD + 4 * g;
-            const __bf16 *kh = k_hi + (first + 4 * g + (l16 >> 2)) * L::pitchK + 4 * (l16 & 3), *kl = kh + L::elemsK;
-#pragma unroll
-            for (int dt = 0; dt < KD / 16; ++dt) {
-                const f4 f = *reinterpret_cast<const f4 *>(keep + 16 * dt);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) s[dt][i] *= f[i];
-                s[dt] = la_mfma(la_join(la_read_tr(kh + 16 * dt), la_read_tr(kl + 16 * dt)), v8, s[dt]);
-            }
+        } else {
+            if (tid < KD)
+                for (int blk = 0; blk < L::blocks; ++blk) decayed *= whole[blk * KD + tid];
+            __syncthreads();  // the next rows' operands may be written now
         }
-        if (STATES && tid < KD)
-            for (int blk = 0; blk < L::blocks; ++blk) decayed *= whole[blk * KD + tid];
-        __syncthreads();  // the next rows' operands may be written now
     }
     float *to = STATES ? seg_state : last ? pool : nullptr;
     if (!to) return;
@@ -458,7 +502,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float x = s[dt][i];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), dst, soff + (16 * dt + i) * a.vp * 4, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), dst, soff + s_row(dt, i) * a.vp * 4, 0, 0);
         }
     if (STATES && vsl == 0 && tid < KD && tid < a.dp) to[state_elems + tid] = decayed;  // (every value slice has the same)
 }
