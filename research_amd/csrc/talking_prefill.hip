@@ -137,16 +137,21 @@ template <int DK> __global__ __launch_bounds__(256, 2) void talk_sums_kernel(con
 constexpr int kTmRows = 16, kTmKeys = 32, kTmWaves = 8, kTmThreads = 64 * kTmWaves;
 constexpr int kTmOut = 2 * kTmWaves;  // out heads of a workgroup, two per wave
 
+// Up to 16 heads there is room for the weights of two tiles, and the next tile's are made beside the mixing of this one's: a tile takes 4600 cycles,
+// else 4850, of which the mixing's few reads and products were 500 (8 prompts of 700 .. 4000 rows, 16 heads of 128: 420 -> 404 us).  It begins with two more
+// barriers and a wait for the second tile's keys, so up to eight tiles stay as they were (25 .. 111 rows, 8 heads: 19.8 us, else 20.5).
+constexpr int kTmAhead = 8;
+
 // HW: heads per wave, 2 or 4.  NG: kv heads of the out heads, whose values are staged by the whole workgroup (0: each wave
-// stages its own).  With two heads per wave the keys of up to NG kv heads are staged as well.
+// stages its own).  With two heads per wave the keys of up to NG kv heads are staged as well, and there is room for the weights of two tiles.
 template <int D, int HW, int NG> struct TmTile {
     static constexpr int heads = kTmWaves * HW, kPitch = D + 16, vPitch = NG ? D + 16 : D + 8;
-    static constexpr bool keys = NG > 0 && HW == 2;
+    static constexpr bool ahead = NG > 0 && HW == 2;
     static constexpr int pair = 4 * heads;  // bytes of a (key, row) pair: both terms of all heads
-    static constexpr int pBytes = kTmKeys * kTmRows * pair, wBytes = kTmOut * kTmRows * kTmKeys * 2, kTile = kTmKeys * kPitch, vTile = kTmKeys * vPitch + (NG ? 3 * 64 : 0);
+    static constexpr int pTile = kTmKeys * kTmRows * pair, pBytes = (ahead ? 2 : 1) * pTile, wBytes = kTmOut * kTmRows * kTmKeys * 2, kTile = kTmKeys * kPitch, vTile = kTmKeys * vPitch + (NG ? 3 * 64 : 0);
     // (a transposing read takes four rows of four sets eight apart)
     static constexpr __device__ int vRow(int row) { return row * vPitch + (NG ? row / 8 * 64 : 0); }
-    static constexpr int vBytes = (NG ? NG : kTmWaves) * vTile * 2, kBytes = keys ? NG * kTile * 2 : 0;
+    static constexpr int vBytes = (NG ? NG : kTmWaves) * vTile * 2, kBytes = ahead ? NG * kTile * 2 : 0;
     static constexpr int biasFloats = HW * 48;
     static constexpr size_t bytes = (size_t)pBytes + wBytes + vBytes + kBytes + kTmWaves * biasFloats * 4;
 };
@@ -157,7 +162,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     constexpr bool SAME = NG > 0;
     constexpr int HP = L::heads, KS = D / 32, ET = D / 16;
     constexpr int kPer = D / 8, kTile = kTmKeys * kPer;                     // 16-byte pieces of a row, of a kv head's tile
-    constexpr int NV = SAME ? NG * kTile / kTmThreads : kTile / 64, NK = L::keys ? NV : 2 * KS;
+    constexpr int NV = SAME ? NG * kTile / kTmThreads : kTile / 64, NK = L::ahead ? NV : 2 * KS;
     extern __shared__ __align__(16) char tm_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
     char *w_s = tm_lds + L::pBytes;
@@ -248,7 +253,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     };
     // straight to operands: keys 16 kb + l16 of one kv head (slots: of key lane % 32)
     auto direct_k = [&](int kv, int slots) {
-        if constexpr (!L::keys) {
+        if constexpr (!L::ahead) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
                 const uint16_t *src = reinterpret_cast<const uint16_t *>(a.k) + (uint64_t)(uint32_t)__shfl(slots, 16 * kb + l16, 64) * k_tok + kv * a.k_dim + 8 * g;
@@ -258,7 +263,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
         }
     };
     auto fetch_k = [&](int slots, int near) {  // (near: the slots of keys lane % 32)
-        if constexpr (L::keys) stage_from(a.k, slots, k_tok, a.k_dim, 0, a.n1, kr);
+        if constexpr (L::ahead) stage_from(a.k, slots, k_tok, a.k_dim, 0, a.n1, kr);
         else direct_k(kv_of(head0), near);
     };
     auto own_v = [&](int kv, int slots) {
@@ -283,30 +288,24 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
         }
     };
     // keys by key lane % 32, where they go straight to operands beside values staged by all
-    auto near_id = [&](int k0) { return SAME && !L::keys ? talk_block_id(a, table, min(k0 + (lane & 31), end - 1)) : 0; };
+    auto near_id = [&](int k0) { return SAME && !L::ahead ? talk_block_id(a, table, min(k0 + (lane & 31), end - 1)) : 0; };
     auto near_slot = [&](int id, int k0, int slots) {
-        return SAME && !L::keys ? max(talk_slot_of(a, id, min(k0 + (lane & 31), end - 1), end), 0) : slots;
+        return SAME && !L::ahead ? max(talk_slot_of(a, id, min(k0 + (lane & 31), end - 1), end), 0) : slots;
     };
     // 16-byte pieces of a pair's row and of a (head, row)'s keys at places that spread over the banks (by the groups of lanes that a
     // read serves together, linear_tiles.h; with the keys' pitch 8 prompts of 818 .. 3868 tokens 508 -> 494 us); inside a piece the place of a
     // wave's weights also turns with key / 4, and that of its keys with head / 4
     const int turn16 = -(l16 >> 2) & 3;
+    char *pairs = tm_lds;  // of the tile whose weights are made
     auto pair_at = [&](int key, int piece) {
         const int at = HP == 32 ? piece ^ ((l16 >> 1) & 7) : piece ^ turn16;
-        return tm_lds + (key * kTmRows + l16) * L::pair + 16 * at;
+        return pairs + (key * kTmRows + l16) * L::pair + 16 * at;
     };
     auto weights_at = [&](int head, int piece) { return w_s + (head * kTmRows + l16) * (kTmKeys * 2) + 16 * (piece ^ turn16); };
 
-    int slots = slot_of(id_of(0), 0), id = id_of(kTmKeys), id_near = near_id(kTmKeys);
-    fetch_k(slots, near_slot(near_id(0), 0, slots));
-    fetch_v(slots);
-    if constexpr (L::keys) {
-        stage_to(k_s, L::kTile, my_row * L::kPitch, kr);
-        __syncthreads();
-    }
-    for (int k0 = 0; k0 < end; k0 += kTmKeys) {
-        // ---- scores and weights of keys 16 kb + 4 g + j of row l16 ----
-        // (distances first_pos + r - k of 16 rows and 32 keys, from their smallest; a key behind its row gets no weight)
+    // ---- scores and weights of keys 16 kb + 4 g + j of row l16 ----
+    // (distances first_pos + r - k of 16 rows and 32 keys, from their smallest; a key behind its row gets no weight)
+    auto score_tile = [&](int k0, int slots) {
 #pragma unroll
         for (int i = 0; i < HW; ++i) {
             const float x = talk_masked_bias(size[i], rate[i], first_pos - (k0 + 31) + lane);
@@ -346,7 +345,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
 #pragma unroll
                 for (int k = 0; k < KS; ++k) {
                     bf8 key;
-                    if constexpr (L::keys) key = la_read8(k_s + kv_of(head0) * L::kTile + (16 * kb + l16) * L::kPitch + 32 * k + 8 * g);
+                    if constexpr (L::ahead) key = la_read8(k_s + kv_of(head0) * L::kTile + (16 * kb + l16) * L::kPitch + 32 * k + 8 * g);
                     else key = __builtin_bit_cast(bf8, kr[kb * KS + k]);
 #pragma unroll
                     for (int i = 0; i < HW; ++i) s[i] = la_mfma(key, q[i][k], s[i]);
@@ -373,16 +372,9 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
             put(0, w[0]);
             put(1, w[1]);
         }
-        const int now = slots;
-        // (always, so that waits can be counted: past the last key these are the last key's again)
-        slots = slot_of(id, k0 + kTmKeys);
-        id = id_of(k0 + 2 * kTmKeys);
-        const int near = near_slot(id_near, k0 + kTmKeys, slots);
-        id_near = near_id(k0 + 2 * kTmKeys);
-        fetch_k(slots, near);
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
-        // ---- mixed: keys 4 wave .. 4 wave + 3 of row l16, out heads 4 g + i ----
+    };
+    // ---- mixed: keys 4 wave .. 4 wave + 3 of row l16, out heads 4 g + i ----
+    auto mix_tile = [&]() {
         {
             f4 x[4];
             bf8 one[4];
@@ -405,12 +397,9 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
                 *reinterpret_cast<uint2 *>(weights_at(4 * g + i, wave >> 1) + 8 * ((wave ^ g) & 1)) =
                     make_uint2(row_pack_bf16(x[0][i], x[1][i]), row_pack_bf16(x[2][i], x[3][i]));
         }
-        put_v();
-        if constexpr (L::keys) stage_to(k_s, L::kTile, my_row * L::kPitch, kr);
-        fetch_v(slots);
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
-        // ---- values ----
+    };
+    // ---- values ----
+    auto value_tile = [&](int now, int slots) {
         bf8 x[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) x[i] = la_read8(reinterpret_cast<const __bf16 *>(weights_at(2 * wave + i, g)));
@@ -437,7 +426,70 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
             for (int t = 0; t < ET; ++t) o[1][t] = la_mfma(values(t), x[1], o[1][t]);
             own_v(kv_of(own0), slots);
         }
-        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    int slots = slot_of(id_of(0), 0), id = id_of(kTmKeys), id_near = near_id(kTmKeys);
+    fetch_k(slots, near_slot(near_id(0), 0, slots));
+    fetch_v(slots);
+    auto put_k = [&] {
+        if constexpr (L::ahead) stage_to(k_s, L::kTile, my_row * L::kPitch, kr);
+    };
+    if constexpr (L::ahead) {
+        put_k();
+        __syncthreads();
+    }
+    if (L::ahead && end > kTmAhead * kTmKeys) {
+        // The next tile's weights are made beside the mixing, whose few reads and products alone would only be waited for
+        char *mine = tm_lds;
+        int k_slots = slot_of(id, kTmKeys);
+        id = id_of(2 * kTmKeys);
+        fetch_k(k_slots, 0);
+        score_tile(0, slots);
+        __syncthreads();
+        put_k();
+        slots = k_slots;
+        k_slots = slot_of(id, 2 * kTmKeys);
+        id = id_of(3 * kTmKeys);
+        fetch_k(k_slots, 0);
+        __syncthreads();
+        for (int k0 = 0; k0 < end; k0 += kTmKeys) {
+            pairs = mine;
+            mix_tile();
+            put_v();
+            fetch_v(slots);  // (past the last key these are the last key's again)
+            mine = mine == tm_lds ? tm_lds + L::pTile : tm_lds;
+            pairs = mine;
+            if (k0 + kTmKeys < end) score_tile(k0 + kTmKeys, 0);
+            __syncthreads();
+            put_k();
+            slots = k_slots;
+            k_slots = slot_of(id, k0 + 3 * kTmKeys);
+            id = id_of(k0 + 4 * kTmKeys);
+            fetch_k(k_slots, 0);
+            value_tile(0, 0);
+            __syncthreads();  // the next tile's values and mixed weights may be written now
+        }
+    } else {
+        for (int k0 = 0; k0 < end; k0 += kTmKeys) {
+            score_tile(k0, slots);
+            const int now = slots;
+            // (always, so that waits can be counted: past the last key these are the last key's again)
+            slots = slot_of(id, k0 + kTmKeys);
+            id = id_of(k0 + 2 * kTmKeys);
+            const int near = near_slot(id_near, k0 + kTmKeys, slots);
+            id_near = near_id(k0 + 2 * kTmKeys);
+            fetch_k(slots, near);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            mix_tile();
+            put_v();
+            put_k();
+            fetch_v(slots);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            value_tile(now, slots);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     if (row >= p.n) return;
 #pragma unroll

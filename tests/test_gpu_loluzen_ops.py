@@ -169,6 +169,16 @@ def test_mixed_heads_in_portions_and_single_rows(heads, kv, dim, vdim, dtype):
     case.check([(i, n - 1, 1) for i, n in enumerate(lens)], decode=True, workspace=False)
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(16, 4, 128, 96), (8, 2, 128, 128), (6, 2, 40, 56), (2, 1, 64, 64)])
+def test_prompts_of_many_tiles(heads, kv, dim, vdim):
+    """Rows around the number of keys above which the next tile's weights are made beside the mixing, and behind a context."""
+    announce(f"talking tiles {heads} {kv} {dim} {vdim}")
+    lens = [257, 305, 40, 289]
+    case = Talking(lens, heads, kv, dim, vdim, BF, seed=9, odd_talk=heads == 8).solve()
+    case.check([(i, 0, n) for i, n in enumerate(lens)])
+    case.check([(1, 254, 51), (0, 250, 7), (3, 287, 2)])
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 64), (20, 4, 48, 72)])
 def test_long_decode_steps_run_in_pieces(heads, kv, dim, vdim):
     """One or two sequences of a few thousand tokens: their keys are spread over the device in up to sixteen pieces."""
