@@ -4,7 +4,7 @@
 
 namespace pa_decode_detail {
 prefill_mfma_fn pa_prefill_asm_kernel(int dtype, int head_dim, bool lower_bounds, bool long_table);
-constexpr int kWdTasks = 4, kWdCapGroups = 6144;  // (prefill_d256.h)
+constexpr int kWdTasks = 4, kWdKeys = 32, kWdCapGroups = 6144;  // (prefill_d256.h)
 prefill_mfma_fn pa_prefill_d256_kernel(int dtype, bool lower_bounds, bool long_table);
 }
 
@@ -26,8 +26,14 @@ int prefill_cus() {
 }
 
 // (the split rule, the workspace size and the groups a workgroup runs are host-testable arithmetic: prefill_plan.h)
-int prefill_splits(int64_t workgroups, int cus, int64_t max_keys) {
-    return plan_prefill_splits(workgroups, cus, max_keys, kPfKeys);
+// Pieces of a launch whose groups hold `tasks` tasks.  us, each number of pieces measured (unsplit, 2, 3 .. 8) -> the rule's: 8 / 2 heads of 128,
+// 7 prompts of 248 rows behind 3936 keys 78, 53, 43, 38, 37, 35, 35, 35 -> 35 (53 while pieces had 24 tiles or more and a call's prompts counted as
+// long as its longest); 14 / 2 of 128, 7 of 114 rows behind 3856 52 -> 34; 8 / 2 of 64, 2 of 41 rows behind 3712 41 -> 26; 16 / 8 of 128, 6 of 73
+// rows behind 4096 54 -> 37, 6 of 681 rows behind 1920 52, 47, 42, 40 .. -> 42; 16 / 8 of 256, 4 of 505 rows behind 1392 48 -> 40.  Of 90 drawn batches
+// (1 to 64 prompts behind up to 8192 keys) the rule's pieces took 1.02 of the time of each one's best.
+int prefill_splits(int num_kv_heads, int64_t groups, int batch, int64_t rows, int n_rep, int tasks, int head_dim, int64_t max_keys) {
+    return plan_prefill_splits(plan_prefill_units(num_kv_heads, groups, batch, rows, n_rep, kPfRows, tasks), prefill_cus(), max_keys,
+                               head_dim > 128 ? kWdKeys : kPfKeys, kPlanShortPieceTiles, rows * num_kv_heads * n_rep * (head_dim + 2) * 4);
 }
 size_t prefill_ws_bytes(int64_t total_q, int num_q_heads, int head_dim, int splits) {
     return plan_prefill_ws_bytes(total_q, num_q_heads, head_dim, splits);
@@ -138,9 +144,9 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
         if (workspace) {
             const int row_blocks = (max_q_len + kPfRows - 1) / kPfRows;
             const int64_t groups = (row_blocks * (int64_t)a.p.n_rep + kPfTasks - 1) / kPfTasks;
-            int want = prefill_splits((int64_t)num_kv_heads * groups * batch, prefill_cus(),
+            int want = prefill_splits(num_kv_heads, groups, batch, total_q, a.p.n_rep, kPfTasks, d_pad,
                                       span > 0 ? span + kPfTasks * kPfRows : bt_stride * (int64_t)block_size);
-            while (want > 1 && prefill_ws_bytes(total_q, num_q_heads, d_pad, want) > workspace_bytes) --want;
+            while (want > 1 && (prefill_ws_bytes(total_q, num_q_heads, d_pad, want) > workspace_bytes || groups * want > 65535)) --want;
             split = want;
         }
         const bool lower_bounds = split > 1 || span > 0 || row_first_key != nullptr;
@@ -172,9 +178,9 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
         if (workspace) {  // (as above; a workgroup of this kernel holds kWdTasks tasks)
             const int row_blocks = (max_q_len + kPfRows - 1) / kPfRows;
             const int64_t groups = (row_blocks * (int64_t)a.p.n_rep + kWdTasks - 1) / kWdTasks;
-            int want = prefill_splits((int64_t)num_kv_heads * groups * batch, prefill_cus(),
+            int want = prefill_splits(num_kv_heads, groups, batch, total_q, a.p.n_rep, kWdTasks, d_pad,
                                       span > 0 ? span + kWdTasks * kPfRows : bt_stride * (int64_t)block_size);
-            while (want > 1 && prefill_ws_bytes(total_q, num_q_heads, d_pad, want) > workspace_bytes) --want;
+            while (want > 1 && (prefill_ws_bytes(total_q, num_q_heads, d_pad, want) > workspace_bytes || groups * want > 65535)) --want;
             split = want;
         }
         mfma = pa_prefill_d256_kernel(dtype, split > 1 || span > 0 || row_first_key != nullptr, !fits);
@@ -245,7 +251,7 @@ extern "C" size_t pa_prefill_workspace_bytes(int batch, int max_q_len, int64_t t
     const int tasks = d_pad == 256 ? kWdTasks : kPfTasks;
     const int64_t groups = (row_blocks * (int64_t)n_rep + tasks - 1) / tasks;
     const int64_t span = plan_window_span(window);
-    const int split = prefill_splits((int64_t)num_kv_heads * groups * batch, prefill_cus(),
+    const int split = prefill_splits(num_kv_heads, groups, batch, total_q, n_rep, tasks, d_pad,
                                      span > 0 ? span + tasks * kPfRows : bt_stride * (int64_t)block_size);
     return prefill_ws_bytes(total_q, num_q_heads, d_pad, split);
 }

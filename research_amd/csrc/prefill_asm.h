@@ -73,13 +73,21 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
     const int kvh = blockIdx.x;
     const int n_splits = a.splits;  // pieces a workgroup's tiles are cut into (1: none; more only in the LO instance)
     const int gpw = (LO || LONG) ? 1 : a.groups_per_wg;  // groups per workgroup
-    const int piece = (int)blockIdx.y % n_splits, chunk_y = (int)blockIdx.y / n_splits;
+    int piece = (int)blockIdx.y % n_splits;
+    const int chunk_y = (int)blockIdx.y / n_splits;
     const int n_chunks = gridDim.y / n_splits, n_seqs = gridDim.z;
     const int lin = chunk_y + n_chunks * blockIdx.z;
     const bool group_major = a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];
     const int turned = (LO || LONG) || !a.turned ? chunk_y : plan_turned_chunk(chunk_y, (int)blockIdx.z, n_chunks);
-    const int wg_chunk = group_major ? n_chunks - 1 - lin / n_seqs : turned;
-    const int b = group_major ? lin % n_seqs : (int)blockIdx.z;
+    int wg_chunk = group_major ? n_chunks - 1 - lin / n_seqs : turned;
+    int b = group_major ? lin % n_seqs : (int)blockIdx.z;
+    if constexpr (LO) {
+        if (n_splits > 1) {
+            const int at = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
+            piece = at % n_splits;
+            if (!pf_unit(a.q_lens, n_seqs, p.n_rep, kPfTasks, at / n_splits, b, wg_chunk)) return;  // uniform over the workgroup
+        }
+    }
     // (read once and held in scalar registers: a load behind the direct-to-LDS requests would wait for all of them)
     const int q_len = __builtin_amdgcn_readfirstlane(a.q_lens[b]);
     const int ctx_len = __builtin_amdgcn_readfirstlane(a.ctx_lens[b]);

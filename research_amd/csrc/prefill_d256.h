@@ -71,12 +71,20 @@ __global__ __launch_bounds__(kPfThreads) void prefill_d256_kernel(const RowwiseA
     // workgroup -> (kv head, group of 4 tasks, sequence): the launch order of prefill_mfma_kernel
     const int kvh = blockIdx.x;
     const int n_splits = a.splits;  // pieces a workgroup's tiles are cut into (1: none; more only in the LO instances)
-    const int piece = (int)blockIdx.y % n_splits, group_y = (int)blockIdx.y / n_splits;
+    int piece = (int)blockIdx.y % n_splits;
+    const int group_y = (int)blockIdx.y / n_splits;
     const int n_groups = gridDim.y / n_splits, n_seqs = gridDim.z;
     const int lin = group_y + n_groups * blockIdx.z;
     const bool group_major = a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];
-    const int group = group_major ? n_groups - 1 - lin / n_seqs : group_y;
-    const int b = group_major ? lin % n_seqs : (int)blockIdx.z;
+    int group = group_major ? n_groups - 1 - lin / n_seqs : group_y;
+    int b = group_major ? lin % n_seqs : (int)blockIdx.z;
+    if constexpr (LO) {
+        if (n_splits > 1) {
+            const int at = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
+            piece = at % n_splits;
+            if (!pf_unit(a.q_lens, n_seqs, p.n_rep, kWdTasks, at / n_splits, b, group)) return;  // uniform over the workgroup
+        }
+    }
     const int q_len = a.q_lens[b];
     const int ctx_len = a.ctx_lens[b];
     const int prefix = ctx_len - q_len;

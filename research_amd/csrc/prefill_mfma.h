@@ -103,6 +103,32 @@ __device__ __forceinline__ const char *pf_scalar_ptr(const char *ptr) {
     return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
 }
 
+// Which sequence, and which of its groups (of `tasks` tasks), the unit-th group of all sequences in turn is; false behind the last one.
+// The workgroups of a split launch are numbered by it: with a place for the groups that short prompts lack, as the grid has them, some
+// compute units got two pieces and others none.  Whole waves call this, with the same unit in all lanes.
+__device__ __forceinline__ bool pf_unit(const int32_t *q_lens, int batch, int n_rep, int tasks, int unit, int &b, int &group) {
+    const int lane = threadIdx.x & 63;
+    for (int from = 0; from < batch; from += 64) {
+        const int rows = from + lane < batch ? max(q_lens[from + lane], 0) : 0;
+        const int mine = ((rows + kPfRows - 1) / kPfRows * n_rep + tasks - 1) / tasks;
+        int upto = mine;  // groups of the sequences from .. from + lane
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int below = __shfl_up(upto, d, 64);
+            upto += lane >= d ? below : 0;
+        }
+        const uint64_t behind = __ballot(unit < upto);
+        if (behind) {
+            const int at = (int)__builtin_ctzll(behind);
+            b = from + at;
+            group = unit - __builtin_amdgcn_readlane(upto - mine, at);
+            return true;
+        }
+        unit -= __builtin_amdgcn_readlane(upto, 63);
+    }
+    return false;
+}
+
 // Direct global -> LDS load of 16 bytes per lane: lane i's bytes land at LDS address lds_dst + 16*i.
 // Issued as inline assembly on purpose.  The compiler cannot tell which LDS bytes such a load writes when
 // the destination is computed, and would make every later LDS read wait for all loads in flight - the

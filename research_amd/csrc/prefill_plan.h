@@ -12,7 +12,10 @@ namespace pa_decode_detail {
 
 constexpr int kPlanMaxPrefillSplits = 8;
 constexpr int kPlanMinTilesPerSplit = 24;  // a piece's set-up and write-out cost about six tiles of its loop
+constexpr int kPlanShortPieceTiles = 8;    // the same where the merge is priced as well
 constexpr int kPlanPieceFixedTiles = 6;    // set-up and write-out of a workgroup, in tiles of its loop
+constexpr int kPlanMergeTiles = 9;         // the merge launch, in the same unit (a tile takes about a microsecond)
+constexpr int64_t kPlanMergeBytesPerTile = 4500000;  // and what it and the pieces move meanwhile
 constexpr int kPlanMaxGroupsPerWorkgroup = 8;
 
 // What a launch costs with its workgroups' tiles cut into s pieces, in tile times: the launch takes rounds of
@@ -25,20 +28,34 @@ PA_PLAN_FN int64_t plan_prefill_cost(int64_t workgroups, int cus, int64_t tiles,
 // Pieces to cut every workgroup's tiles into, from shapes alone.  The matrix-core kernels run one workgroup per
 // compute unit, each owning 256 (head_dim 256: 128) row-head pairs and all their keys, so a launch of few rows
 // leaves compute units idle however long the context is.  The split with the lowest cost wins (the smaller on
-// ties), as long as a piece keeps kPlanMinTilesPerSplit tiles of the longest context the block tables can describe.
-PA_PLAN_FN int plan_prefill_splits(int64_t workgroups, int cus, int64_t max_keys, int tile_keys) {
+// ties), as long as a piece keeps min_tiles tiles of the longest context the block tables can describe.  Given the bytes of a piece's
+// partial results the cost has the merge in it, and pieces may be short.
+PA_PLAN_FN int plan_prefill_splits(int64_t workgroups, int cus, int64_t max_keys, int tile_keys, int min_tiles = kPlanMinTilesPerSplit,
+                                   int64_t part_bytes = 0) {
     const int64_t tiles = max_keys / tile_keys;
     int best = 1;
     int64_t best_cost = 0;
     for (int s = 1; s <= kPlanMaxPrefillSplits; ++s) {
-        if (s > 1 && tiles / s < kPlanMinTilesPerSplit) break;
-        const int64_t cost = plan_prefill_cost(workgroups, cus, tiles, s);
+        if (s > 1 && tiles / s < min_tiles) break;
+        const int64_t merge = s > 1 && part_bytes > 0 ? kPlanMergeTiles + 2 * s * part_bytes / kPlanMergeBytesPerTile : 0;
+        const int64_t cost = plan_prefill_cost(workgroups, cus, tiles, s) + merge;
         if (s == 1 || cost < best_cost) {
             best_cost = cost;
             best = s;
         }
     }
     return best;
+}
+
+// Workgroups with rows that a launch of one group (of `tasks` tasks) each has, about: the longest prompt's length would give all `batch`
+// sequences `groups`; `rows` rows fill fewer, and a sequence's last task and last group are half full on average.  A few more than that,
+// as one too many for the device costs a round and one too few only a small part of one.
+PA_PLAN_FN int64_t plan_prefill_units(int num_kv_heads, int64_t groups, int batch, int64_t rows, int n_rep, int rows_per_task, int tasks) {
+    int step = tasks;  // tasks that a sequence's may leave over in its last group: multiples of step
+    while (n_rep % step) step /= 2;
+    int64_t filled = (2 * rows * n_rep / rows_per_task + (int64_t)batch * (n_rep + tasks - step)) / (2 * tasks) + (batch + 15) / 16;
+    filled = filled < batch ? batch : filled;
+    return num_kv_heads * (filled < groups * batch ? filled : groups * batch);
 }
 
 // workspace = [part_o float[row][head][piece][D]] [part_ml float[row][head][piece][2]]

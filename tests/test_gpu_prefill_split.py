@@ -103,6 +103,26 @@ def test_ragged_batch_short_contexts_and_empty_pieces():
         assert not got[b, n:].any()  # rows past the chunk are not written
 
 
+@pytest.mark.parametrize("d,hq,hkv,n", [(128, 7, 1, 70), (64, 4, 1, 129), (256, 2, 1, 64), (128, 12, 2, 3)])
+def test_many_prompts_of_unequal_length_in_pieces(d, hq, hkv, n):
+    """A split launch numbers its workgroups by the groups that have rows: prompts without any, at the ends of the 64 sequences that are
+    looked at together, and of one group more than their neighbours."""
+    announce(f"split prefill: {n} prompts of unequal length, {hq} / {hkv} heads of {d}")
+    rng = np.random.default_rng(n)
+    chunk = rng.choice([0, 1, 31, 32, 33, 40], size=n)
+    chunk[[0, n - 1]] = 0, 40
+    if n > 64:
+        chunk[[63, 64]] = 0, 33
+    prefix = rng.integers(40, 300, size=n)
+    c = Case([int(x) for x in prefix], [int(x) for x in chunk], hq, hkv, d, seed=n, width=1024)
+    base, got, want = c.run(), c.run(2), c.want()
+    for b, rows in enumerate(c.chunk):
+        if rows:
+            assert_close(got[b, :rows], want[b, :rows], 2e-2, f"sequence {b} vs checker")
+            assert_close(got[b, :rows], base[b, :rows], 6e-3, f"sequence {b} vs unsplit")
+        assert not got[b, rows:].any()
+
+
 def test_windows_first_keys_and_absent_blocks_in_pieces():
     announce("split prefill: window, per-row first keys, absent blocks")
     # (under a window a workgroup sees window + 256 keys at most: the library splits only wide windows)

@@ -23,6 +23,9 @@ def plan(tmp_path_factory):
     dll.pa_plan_pieces.argtypes = [ctypes.c_int] * 3 + [ctypes.c_char_p, ctypes.c_int]
     dll.pa_plan_groups.argtypes = [ctypes.c_int] * 3 + [ctypes.POINTER(ctypes.c_int), ctypes.c_char_p, ctypes.c_int]
     dll.pa_plan_splits.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int]
+    dll.pa_plan_splits_merged.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong]
+    dll.pa_plan_units.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong] + [ctypes.c_int] * 3
+    dll.pa_plan_units.restype = ctypes.c_longlong
     dll.pa_plan_cost.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int]
     dll.pa_plan_cost.restype = ctypes.c_longlong
     dll.pa_plan_ws_bytes.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int, ctypes.c_int]
@@ -93,6 +96,37 @@ def test_split_rule_is_the_cheapest_admissible_split(plan, cus):
     assert plan.pa_plan_splits(64, 256, 202048 + 256, 64) == 4      # long-d128: 64 workgroups on 256 compute units
     assert plan.pa_plan_splits(128, 256, 202048 + 256, 64) == 2     # long-d256
     assert plan.pa_plan_splits(512, 256, 2304, 64) == 1             # c3
+
+
+@pytest.mark.parametrize("tasks", [8, 4])
+def test_units_are_about_the_groups_with_rows(plan, tasks):
+    """Between a group for every sequence and what the longest prompt's length would give all, and no further
+    from the groups there are than the last task and group of each sequence, and the reserve of one in sixteen, can make it."""
+    rng = np.random.default_rng(tasks)
+    count = lambda n, n_rep: -(-(-(-n // 32) * n_rep) // tasks)
+    for _ in range(400):
+        n_rep, batch, most, hkv = int(rng.integers(1, 20)), int(rng.integers(1, 300)), int(rng.integers(1, 1500)), int(rng.integers(1, 9))
+        lens = rng.integers(1, most + 1, size=batch)
+        lens[0] = most
+        upper, real = count(most, n_rep) * batch, sum(count(int(n), n_rep) for n in lens)
+        got = plan.pa_plan_units(hkv, count(most, n_rep), batch, int(lens.sum()), n_rep, 32, tasks)
+        assert got % hkv == 0 and hkv * batch <= got <= hkv * upper
+        # (what a sequence's last task and last group lack lies between nothing and twice what is counted for them; floors and ceilings: 2)
+        step = next(x for x in (8, 4, 2, 1) if x <= tasks and n_rep % x == 0)
+        assert abs(got // hkv - real) <= batch * (n_rep + tasks - step) / (2 * tasks) + batch / 16 + 2
+
+
+def test_short_pieces_pay_for_their_merge(plan):
+    cost = lambda w, tiles, s, part: plan.pa_plan_cost(w, 256, tiles, s) + (9 + 2 * s * part // 4500000 if s > 1 else 0)
+    rng = np.random.default_rng(1)
+    for _ in range(400):
+        w, tiles, part = int(rng.integers(1, 1000)), int(rng.integers(1, 200)), int(rng.integers(1, 1 << 25))
+        s = plan.pa_plan_splits_merged(w, 256, tiles * 64, 64, part)
+        admissible = [k for k in range(1, 9) if k == 1 or tiles // k >= 8]
+        assert s in admissible and cost(w, tiles, s, part) == min(cost(w, tiles, k, part) for k in admissible)
+    assert plan.pa_plan_splits_merged(6, 256, 1024, 64, 150 * 8 * 130 * 4) == 1   # 16 tiles: the merge costs what half of them do
+    assert plan.pa_plan_splits_merged(14, 256, 4032, 64, 248 * 8 * 130 * 4) > 4   # few rows behind a long prefix
+    assert plan.pa_plan_splits_merged(2048, 256, 16384, 64, 64 * 256 * 32 * 130 * 4) == 1  # a launch that fills the device
 
 
 def test_workspace_size_is_the_layout_the_kernels_index(plan):
