@@ -40,8 +40,9 @@ size_t prefill_ws_bytes(int64_t total_q, int num_q_heads, int head_dim, int spli
 }
 
 // Merge of the pieces of a split prefill launch: one thread per (row, head, four consecutive d).  The partial rows
-// are d_part floats long (the head size the kernel is compiled for), the output rows d_head elements.
-template <typename T>
+// are d_part floats long (the head size the kernel is compiled for), the output rows d_head elements.  At most M pieces, whose loads are all on their
+// way at once (8 / 2 heads of 256, 18 prompts of 2 .. 18 rows behind 3184 keys in 8 pieces, the whole call: 34.6 -> 30.9 us).
+template <typename T, int M>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part_o, const float *part_ml, T *out,
                                                             const int32_t *q_lens, const int32_t *q_starts, int hq,
                                                             int d_head, int d_part, int splits) {
@@ -52,20 +53,28 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part_o,
     const int h = item / v4, d = (item - h * v4) * 4;
     const int64_t row = (int64_t)q_starts[b] + i;
     const int64_t base = (row * hq + h) * splits;
+    float2 ml[M];
+    float4 o[M];
+#pragma unroll
+    for (int s = 0; s < M; ++s) {
+        const int64_t at = base + min(s, splits - 1);
+        ml[s] = *reinterpret_cast<const float2 *>(part_ml + at * 2);
+        o[s] = *reinterpret_cast<const float4 *>(part_o + at * d_part + d);
+    }
     float m_all = -1.0e30f;
-    for (int s = 0; s < splits; ++s)
-        if (part_ml[(base + s) * 2 + 1] > 0.f) m_all = fmaxf(m_all, part_ml[(base + s) * 2]);
+#pragma unroll
+    for (int s = 0; s < M; ++s)
+        if (ml[s].y > 0.f) m_all = fmaxf(m_all, ml[s].x);
     float den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < splits; ++s) {
-        const float l = part_ml[(base + s) * 2 + 1];
-        if (!(l > 0.f)) continue;  // a piece in which the row saw no key wrote no O row
-        const float w = __builtin_amdgcn_exp2f(part_ml[(base + s) * 2] - m_all);
-        const float4 o = *reinterpret_cast<const float4 *>(part_o + (base + s) * d_part + d);
-        den = fmaf(w, l, den);
-        num[0] = fmaf(w, o.x, num[0]);
-        num[1] = fmaf(w, o.y, num[1]);
-        num[2] = fmaf(w, o.z, num[2]);
-        num[3] = fmaf(w, o.w, num[3]);
+#pragma unroll
+    for (int s = 0; s < M; ++s) {
+        if (s >= splits || !(ml[s].y > 0.f)) continue;  // a piece in which the row saw no key wrote no O row
+        const float w = __builtin_amdgcn_exp2f(ml[s].x - m_all);
+        den = fmaf(w, ml[s].y, den);
+        num[0] = fmaf(w, o[s].x, num[0]);
+        num[1] = fmaf(w, o[s].y, num[1]);
+        num[2] = fmaf(w, o[s].z, num[2]);
+        num[3] = fmaf(w, o[s].w, num[3]);
     }
     const float inv = den > 0.f ? 1.f / den : 0.f;
     T *op = out + (row * hq + h) * d_head + d;
@@ -203,12 +212,11 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
         if (split > 1) {
             const unsigned gx = (unsigned)((num_q_heads * (head_dim / 4) + 255) / 256);
             const dim3 mg(gx, (unsigned)max_q_len, (unsigned)batch);
+            auto merge = [&](auto kernel, auto *to) { kernel<<<mg, dim3(256), 0, s>>>(a.part_o, a.part_ml, to, q_lens, q_starts, num_q_heads, head_dim, d_pad, split); };
             if (dtype == PA_BF16)
-                prefill_merge_kernel<pa_bf16><<<mg, dim3(256), 0, s>>>(a.part_o, a.part_ml, (pa_bf16 *)out, q_lens, q_starts,
-                                                                     num_q_heads, head_dim, d_pad, split);
+                merge(split <= 2 ? prefill_merge_kernel<pa_bf16, 2> : split <= 4 ? prefill_merge_kernel<pa_bf16, 4> : prefill_merge_kernel<pa_bf16, kPlanMaxPrefillSplits>, (pa_bf16 *)out);
             else
-                prefill_merge_kernel<pa_f16><<<mg, dim3(256), 0, s>>>(a.part_o, a.part_ml, (pa_f16 *)out, q_lens, q_starts,
-                                                                    num_q_heads, head_dim, d_pad, split);
+                merge(split <= 2 ? prefill_merge_kernel<pa_f16, 2> : split <= 4 ? prefill_merge_kernel<pa_f16, 4> : prefill_merge_kernel<pa_f16, kPlanMaxPrefillSplits>, (pa_f16 *)out);
             PA_CHECK_LAUNCH("pa_prefill_paged_ws (merge of the pieces)");
         }
         return PA_OK;
