@@ -94,6 +94,7 @@ struct RowwiseArgs {
     // many groups); 1 everywhere else.
     int groups_per_wg;
     int turned;  // there: chunks take turns over the sequences (plan_turned_chunk; unequal prompts)
+    int dense;   // the matrix-core kernels with the assembly loop: workgroups are numbered by the chunks that have rows (plan_prefill_dense)
 };
 
 __device__ __forceinline__ uint4 ld16(const void *p) { return *reinterpret_cast<const uint4 *>(p); }

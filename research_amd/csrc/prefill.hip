@@ -121,7 +121,7 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
     a.q = q; a.out = out; a.ctx_lens = ctx_lens; a.q_lens = q_lens; a.q_starts = q_starts;
     a.row_lo = row_first_key;
     a.batch = batch; a.max_q_len = max_q_len;
-    a.splits = 1; a.part_o = nullptr; a.part_ml = nullptr; a.groups_per_wg = 1; a.turned = 0;
+    a.splits = 1; a.part_o = nullptr; a.part_ml = nullptr; a.groups_per_wg = 1; a.turned = 0; a.dense = 0;
     hipStream_t s = (hipStream_t)stream;
     // bf16 / fp16 with head_dim 32, 64, 128 (and 256, below) run on the matrix cores unless the caller asked for the
     // vector kernel
@@ -201,6 +201,9 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
         int groups = (row_blocks * a.p.n_rep + tasks_per_wg - 1) / tasks_per_wg;
         groups = (groups + a.groups_per_wg - 1) / a.groups_per_wg;  // workgroups along y: chunks of groups
         PA_REQUIRE((int64_t)groups * split <= 65535, "max_q_len=%d is too long for one launch", max_q_len);
+        if (total_q > 0)
+            a.dense = plan_prefill_dense(plan_prefill_units(num_kv_heads, groups, batch, total_q, a.p.n_rep, kPfRows, tasks_per_wg * a.groups_per_wg),
+                                         (int64_t)num_kv_heads * groups * batch, prefill_cus());
         if (split > 1) {
             PA_REQUIRE(((uintptr_t)workspace & 255u) == 0, "workspace must be 256-byte aligned");
             a.splits = split;

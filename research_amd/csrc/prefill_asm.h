@@ -75,18 +75,17 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
     const int gpw = (LO || LONG) ? 1 : a.groups_per_wg;  // groups per workgroup
     int piece = (int)blockIdx.y % n_splits;
     const int chunk_y = (int)blockIdx.y / n_splits;
-    const int n_chunks = gridDim.y / n_splits, n_seqs = gridDim.z;
+    int n_chunks = gridDim.y / n_splits;
+    const int n_seqs = gridDim.z;
     const int lin = chunk_y + n_chunks * blockIdx.z;
     const bool group_major = a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];
     const int turned = (LO || LONG) || !a.turned ? chunk_y : plan_turned_chunk(chunk_y, (int)blockIdx.z, n_chunks);
     int wg_chunk = group_major ? n_chunks - 1 - lin / n_seqs : turned;
     int b = group_major ? lin % n_seqs : (int)blockIdx.z;
-    if constexpr (LO) {
-        if (n_splits > 1) {
-            const int at = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
-            piece = at % n_splits;
-            if (!pf_unit(a.q_lens, n_seqs, p.n_rep, kPfTasks, at / n_splits, b, wg_chunk)) return;  // uniform over the workgroup
-        }
+    if (n_splits > 1 || (a.dense && !group_major)) {
+        const int at = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
+        piece = at % n_splits;
+        if (!pf_unit(a.q_lens, n_seqs, p.n_rep, kPfTasks * gpw, at / n_splits, b, wg_chunk, n_chunks)) return;  // uniform over the workgroup
     }
     // (read once and held in scalar registers: a load behind the direct-to-LDS requests would wait for all of them)
     const int q_len = __builtin_amdgcn_readfirstlane(a.q_lens[b]);

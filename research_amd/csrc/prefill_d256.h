@@ -78,12 +78,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_d256_kernel(const RowwiseA
     const bool group_major = a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];
     int group = group_major ? n_groups - 1 - lin / n_seqs : group_y;
     int b = group_major ? lin % n_seqs : (int)blockIdx.z;
-    if constexpr (LO) {
-        if (n_splits > 1) {
-            const int at = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
-            piece = at % n_splits;
-            if (!pf_unit(a.q_lens, n_seqs, p.n_rep, kWdTasks, at / n_splits, b, group)) return;  // uniform over the workgroup
-        }
+    if (n_splits > 1 || (a.dense && !group_major)) {
+        const int at = (int)blockIdx.y + (int)gridDim.y * (int)blockIdx.z;
+        int of;
+        piece = at % n_splits;
+        if (!pf_unit(a.q_lens, n_seqs, p.n_rep, kWdTasks, at / n_splits, b, group, of)) return;  // uniform over the workgroup
     }
     const int q_len = a.q_lens[b];
     const int ctx_len = a.ctx_lens[b];

@@ -103,25 +103,21 @@ __device__ __forceinline__ const char *pf_scalar_ptr(const char *ptr) {
     return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
 }
 
-// Which sequence, and which of its groups (of `tasks` tasks), the unit-th group of all sequences in turn is; false behind the last one.
-// The workgroups of a split launch are numbered by it: with a place for the groups that short prompts lack, as the grid has them, some
-// compute units got two pieces and others none.  Whole waves call this, with the same unit in all lanes.
-__device__ __forceinline__ bool pf_unit(const int32_t *q_lens, int batch, int n_rep, int tasks, int unit, int &b, int &group) {
+// Which sequence, and which of its groups (of `tasks` tasks; n_groups of them), the unit-th group of all sequences in turn is; false behind the last
+// one.  The workgroups of a split launch are numbered by it, and those of unequal prompts where that is a round less (plan_prefill_dense).  Whole
+// waves call this, with the same unit in all lanes.
+__device__ __forceinline__ bool pf_unit(const int32_t *q_lens, int batch, int n_rep, int tasks, int unit, int &b, int &group, int &n_groups) {
     const int lane = threadIdx.x & 63;
     for (int from = 0; from < batch; from += 64) {
         const int rows = from + lane < batch ? max(q_lens[from + lane], 0) : 0;
         const int mine = ((rows + kPfRows - 1) / kPfRows * n_rep + tasks - 1) / tasks;
-        int upto = mine;  // groups of the sequences from .. from + lane
-#pragma unroll
-        for (int d = 1; d < 64; d *= 2) {
-            const int below = __shfl_up(upto, d, 64);
-            upto += lane >= d ? below : 0;
-        }
+        const int upto = wave_inclusive_scan(mine, lane);  // groups of the sequences from .. from + lane
         const uint64_t behind = __ballot(unit < upto);
         if (behind) {
             const int at = (int)__builtin_ctzll(behind);
             b = from + at;
-            group = unit - __builtin_amdgcn_readlane(upto - mine, at);
+            n_groups = __builtin_amdgcn_readlane(mine, at);
+            group = unit - (__builtin_amdgcn_readlane(upto, at) - n_groups);
             return true;
         }
         unit -= __builtin_amdgcn_readlane(upto, 63);

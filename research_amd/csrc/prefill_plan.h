@@ -58,6 +58,18 @@ PA_PLAN_FN int64_t plan_prefill_units(int num_kv_heads, int64_t groups, int batc
     return num_kv_heads * (filled < groups * batch ? filled : groups * batch);
 }
 
+// Whether a launch's workgroups are numbered by the chunks that have rows (about `units`), not by the places of a grid in which the longest prompt's
+// length gives all sequences as many (`places`).  The grid's places go to compute units in turn, with rows or without, so that some get one workgroup
+// more than others: by number where that is a round less and the last round is well filled (an emptier one finds room among the places
+// without rows).  us, by places -> by number, rounds of 256 places and of chunks: 8 / 2 heads of 128, 29 prompts of 133 .. 319 rows behind
+// 4080 keys (1.1, 0.8) 191 -> 115; 32 / 8 of 128, 13 of 75 .. 158 behind 1504 (1.2, 1.0) 88 -> 57, 48 of 99 .. 145 behind 1008 (4.5, 3.7) 172 -> 150;
+// 14 / 2 of 128, 13 of 385 .. 962 behind 1104 (2.5, 1.8) 118 -> 96, but 47 of 36 .. 218 behind 720 (2.6, 1.4) 58 -> 60; 32 / 8 of 128, 32 of 97 .. 249
+// behind 2048 (4.0, 3.2) 225 -> 234.
+PA_PLAN_FN bool plan_prefill_dense(int64_t units, int64_t places, int cus) {
+    const int64_t rounds = (units + cus - 1) / cus;
+    return rounds < (places + cus - 1) / cus && 8 * (units - (rounds - 1) * cus) >= 5 * cus;
+}
+
 // workspace = [part_o float[row][head][piece][D]] [part_ml float[row][head][piece][2]]
 PA_PLAN_FN size_t plan_prefill_ws_bytes(int64_t total_q, int num_q_heads, int head_dim, int splits) {
     return splits <= 1 ? 0 : (size_t)total_q * num_q_heads * splits * ((size_t)head_dim + 2) * sizeof(float);

@@ -68,6 +68,7 @@ extern "C" int pa_plan_splits_merged(long long workgroups, int cus, long long ma
 extern "C" long long pa_plan_units(int num_kv_heads, long long groups, int batch, long long rows, int n_rep, int rows_per_task, int tasks) {
     return plan_prefill_units(num_kv_heads, groups, batch, rows, n_rep, rows_per_task, tasks);
 }
+extern "C" int pa_plan_dense(long long units, long long places, int cus) { return plan_prefill_dense(units, places, cus); }
 extern "C" long long pa_plan_cost(long long workgroups, int cus, long long tiles, int s) {
     return plan_prefill_cost(workgroups, cus, tiles, s);
 }

@@ -123,6 +123,28 @@ def test_many_prompts_of_unequal_length_in_pieces(d, hq, hkv, n):
         assert not got[b, rows:].any()
 
 
+@pytest.mark.parametrize("d,hq,hkv,n,most,dtype", [(128, 7, 1, 110, 130, torch.bfloat16), (64, 8, 2, 66, 260, torch.float16),
+                                                   (256, 6, 3, 70, 80, torch.bfloat16), (128, 8, 2, 12, 1200, torch.bfloat16)])
+def test_unequal_prompts_numbered_by_rows(d, hq, hkv, n, most, dtype):
+    """Launches whose grid has places for more than a round while the groups with rows fill about one: sequences without rows, more than 64 of
+    them, and workgroups of several groups (the last case's prompts also without the number of rows, which numbers by places)."""
+    announce(f"prefill numbered by rows: {n} prompts, {hq} / {hkv} heads of {d}")
+    rng = np.random.default_rng(n)
+    chunk = rng.integers(0, most // 2 + 1, size=n)
+    chunk[[1, n // 2, n - 1]] = most, 0, most
+    prefix = rng.integers(most, 2 * most, size=n)
+    c = Case([int(x) for x in prefix], [int(x) for x in chunk], hq, hkv, d, dtype=dtype, seed=n, width=1)
+    rows = [int(x) for x in chunk]
+    starts = np.concatenate([[0], np.cumsum(rows)[:-1]])
+    q = torch.cat([c.q[b, :r] for b, r in enumerate(rows)]).to(DEV)
+    got = ops.prefill_paged(q, c.k.to(DEV), c.v.to(DEV), c.dev_tables, _i32(c.ctx), _i32(rows), _i32(starts), most, 16, c.scale).cpu()
+    assert torch.equal(got, torch.cat([x[:r] for x, r in zip(c.run().cpu(), rows)]))  # (run: rows of equal prompts, numbered by places)
+    want = c.want()
+    for b, r in enumerate(rows):
+        if r:
+            assert_close(got[starts[b]: starts[b] + r], want[b, :r], 2e-2, f"sequence {b} vs checker")
+
+
 def test_windows_first_keys_and_absent_blocks_in_pieces():
     announce("split prefill: window, per-row first keys, absent blocks")
     # (under a window a workgroup sees window + 256 keys at most: the library splits only wide windows)

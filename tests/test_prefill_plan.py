@@ -26,6 +26,7 @@ def plan(tmp_path_factory):
     dll.pa_plan_splits_merged.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong]
     dll.pa_plan_units.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong] + [ctypes.c_int] * 3
     dll.pa_plan_units.restype = ctypes.c_longlong
+    dll.pa_plan_dense.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_int]
     dll.pa_plan_cost.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int]
     dll.pa_plan_cost.restype = ctypes.c_longlong
     dll.pa_plan_ws_bytes.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int, ctypes.c_int]
@@ -127,6 +128,13 @@ def test_short_pieces_pay_for_their_merge(plan):
     assert plan.pa_plan_splits_merged(6, 256, 1024, 64, 150 * 8 * 130 * 4) == 1   # 16 tiles: the merge costs what half of them do
     assert plan.pa_plan_splits_merged(14, 256, 4032, 64, 248 * 8 * 130 * 4) > 4   # few rows behind a long prefix
     assert plan.pa_plan_splits_merged(2048, 256, 16384, 64, 64 * 256 * 32 * 130 * 4) == 1  # a launch that fills the device
+
+
+def test_workgroups_are_numbered_by_rows_where_that_is_a_round_less(plan):
+    assert all(not plan.pa_plan_dense(u, u, 256) for u in (1, 160, 255, 256, 257, 512, 700))           # equal prompts: nothing to gain
+    assert [plan.pa_plan_dense(u, 300, 256) for u in (159, 160, 256, 257)] == [0, 1, 1, 0]             # a round instead of two, well filled
+    assert [plan.pa_plan_dense(u, 1152, 256) for u in (800, 927, 928, 1024, 1025)] == [0, 0, 1, 1, 0]  # 4 instead of 5
+    assert [plan.pa_plan_dense(u, 1152, 256) for u in (256 + 159, 256 + 160)] == [0, 1]                # 2 instead of 5
 
 
 def test_workspace_size_is_the_layout_the_kernels_index(plan):
