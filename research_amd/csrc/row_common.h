@@ -28,6 +28,20 @@ template <typename T, int V> __device__ __forceinline__ void row_load(const T *p
     }
 }
 
+// The same for data that is used once: past the caches.
+template <typename T, int V> __device__ __forceinline__ void row_load_once(const T *p, float *f) {
+    typedef uint32_t words __attribute__((ext_vector_type(V * sizeof(T) / 4 > 0 ? V * sizeof(T) / 4 : 1)));
+    if constexpr (V == 1) {
+        f[0] = pa_scalar<T>::load(p);
+    } else {
+        static_assert(V == 4, "four elements");
+        const words r = __builtin_nontemporal_load(reinterpret_cast<const words *>(p));
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            f[i] = __builtin_bit_cast(float, sizeof(T) == 4 ? r[i % (V * sizeof(T) / 4)] : i % 2 ? r[i / 2] & 0xffff0000u : r[i / 2] << 16);
+    }
+}
+
 __device__ __forceinline__ uint32_t row_pack_bf16(float lo, float hi) {
     typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
     const bf2 pair = {(__bf16)lo, (__bf16)hi};

@@ -70,6 +70,25 @@ def test_embeddings_and_weighted_branches(width, dtype):
         ops.residual_norm(x, dtype, y=y[: rows].to(DEV), mix=mix.to(DEV))
 
 
+@pytest.mark.parametrize("parts,with_extra,width,dtype", [(1, False, 37, F32), (1, True, 4096, BF), (3, True, 516, F32), (4, False, 4096, F32), (4, True, 2052, BF),
+                                                          (8, True, 4096, BF), (9, False, 88, BF), (2, True, 8192, BF)])
+def test_weighted_branches_of_many_parts(parts, with_extra, width, dtype):
+    """Numbers of parts around those whose loads travel together; a part's sum is that of its terms in turn."""
+    announce(f"mix of {parts} parts{' and another' if with_extra else ''} {width} {dtype}")
+    rows = 5
+    x0, y, extra, mix = _rand(rows, width, seed=1), _rand(rows * parts, width, dtype=dtype, seed=2), _rand(rows, width, dtype=dtype, seed=3), _rand(rows, parts + 1, seed=4)
+    if not with_extra:
+        mix[:, parts] = float("nan")  # not a part's
+    x = x0.to(DEV)
+    ops.residual_norm(x, dtype, y=y.to(DEV), mix=mix.to(DEV), y_extra=extra.to(DEV) if with_extra else None)
+    terms = y.double().view(rows, parts, width) * mix[:, :parts, None].double()
+    if with_extra:
+        terms = torch.cat([terms, (mix[:, parts:].double() * extra.double())[:, None]], 1)
+    want = x0.double() + terms.sum(1)
+    bound = (terms.shape[1] + 1) * 2.0 ** -24 * (x0.double().abs() + terms.abs().sum(1)) * 1.01  # one rounding a term, one more for x
+    assert bool(((x.cpu().double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("groups,per", [(1, 48), (3, 24), (5, 14), (4, 72), (2, 200), (8, 128), (2, 2048), (3, 33)])
 def test_gated_norms_of_groups(groups, per, dtype):
