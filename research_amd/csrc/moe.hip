@@ -33,7 +33,11 @@ struct NarrowArgs {
     int n, k;
 };
 
-// 16 RT rows x 16 CT columns per workgroup; its NW waves share the inner dimension.  (k: whole 16-byte vectors)
+// 16 RT rows x 16 CT columns per workgroup; its NW waves share the inner dimension.  (k: whole 16-byte vectors)  A step's time is its waves'
+// requests for 16-byte pieces, those of the weights by every workgroup again, so that fewer rows a workgroup only pay while there are compute
+// units without one (the launch's rule).  With few rows there are registers for the next step's weights as well (65 columns behind
+// 4096 elements, 4097 to 8192 rows: 33 -> 28 us; with 64 rows a workgroup, whose steps are longer, it is slower).  A result is the same sum
+// in the same order whatever RT.
 template <int RT, int CT, int NW> __global__ __launch_bounds__(64 * NW) void narrow_mfma_kernel(const NarrowArgs a) {
     __shared__ float red[NW / 2][RT * CT * 4][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -58,38 +62,42 @@ template <int RT, int CT, int NW> __global__ __launch_bounds__(64 * NW) void nar
         for (int c = 0; c < CT; ++c) acc[t][c] = f4{0.f, 0.f, 0.f, 0.f};
     // (the four lanes of a row take 32 consecutive bytes each: whole lines, in the same order for both operands.  The next
     // step's rows are on their way while this one's are multiplied.)
-    bf8 x[2][RT][2];
-    auto fetch = [&](int k0, bf8 (&to)[RT][2]) {
+    constexpr bool kAhead = RT <= 2 && CT >= 4;
+    bf8 x[2][RT][2], w[kAhead ? 2 : 1][CT][2];
+    auto fetch_w = [&](int k0, bf8 (&to)[CT][2]) {
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const int k = k0 + 16 * g + 8 * half;
 #pragma unroll
-            for (int t = 0; t < RT; ++t) to[t][half] = k < a.k ? moe_load(xr[t] + k) : moe_zero();
+            for (int c = 0; c < CT; ++c) to[c][half] = k < a.k ? moe_load(wr[c] + k) : moe_zero();
         }
     };
-    auto multiply = [&](int k0, const bf8 (&x)[RT][2]) {
-        bf8 w[CT][2];
+    auto fetch = [&](int k0, int to) {
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const int k = k0 + 16 * g + 8 * half;
 #pragma unroll
-            for (int c = 0; c < CT; ++c) w[c][half] = k < a.k ? moe_load(wr[c] + k) : moe_zero();
+            for (int t = 0; t < RT; ++t) x[to][t][half] = k < a.k ? moe_load(xr[t] + k) : moe_zero();
         }
+        if constexpr (kAhead) fetch_w(k0, w[to]);
+    };
+    auto multiply = [&](int k0, int of) {
+        if constexpr (!kAhead) fetch_w(k0, w[0]);
 #pragma unroll
         for (int half = 0; half < 2; ++half)
 #pragma unroll
             for (int c = 0; c < CT; ++c)
 #pragma unroll
-                for (int t = 0; t < RT; ++t) acc[t][c] = moe_mfma(w[c][half], x[t][half], acc[t][c]);
+                for (int t = 0; t < RT; ++t) acc[t][c] = moe_mfma(w[kAhead ? of : 0][c][half], x[of][t][half], acc[t][c]);
     };
     constexpr int kStep = 64 * NW;
-    fetch(64 * wave, x[0]);
+    fetch(64 * wave, 0);
     for (int k0 = 64 * wave; k0 < a.k; k0 += 2 * kStep) {
-        fetch(k0 + kStep, x[1]);
-        multiply(k0, x[0]);
+        fetch(k0 + kStep, 1);
+        multiply(k0, 0);
         if (k0 + kStep >= a.k) break;
-        fetch(k0 + 2 * kStep, x[0]);
-        multiply(k0 + kStep, x[1]);
+        fetch(k0 + 2 * kStep, 0);
+        multiply(k0 + kStep, 1);
     }
 #pragma unroll
     for (int step = NW / 2; step >= 1; step /= 2) {
@@ -911,10 +919,15 @@ extern "C" int pa_narrow_linear(const void *x, int64_t x_stride, const void *w, 
     else {
         const int tiles = (n + 15) / 16;
         const bool five = tiles % 4 == 1 && tiles > 1;  // (one row more than whole tiles of 64: the gate of a shared expert)
-        const unsigned gx = (unsigned)((rows + 15) / 16), gx4 = (unsigned)((rows + 63) / 64), gy = (unsigned)((tiles + (five ? 4 : 3)) / (five ? 5 : 4));
-        if (rows <= 1024) narrow_mfma_kernel<1, 1, 8><<<dim3(gx, (unsigned)tiles), dim3(512), 0, s>>>(a);
-        else if (five) narrow_mfma_kernel<4, 5, 4><<<dim3(gx4, gy), dim3(256), 0, s>>>(a);
-        else narrow_mfma_kernel<4, 4, 4><<<dim3(gx4, gy), dim3(256), 0, s>>>(a);
+        const unsigned gy = (unsigned)((tiles + (five ? 4 : 3)) / (five ? 5 : 4));
+        auto blocks = [&](int rt) { return (unsigned)((rows + 16 * rt - 1) / (16 * rt)); };
+        // As few rows a workgroup as leave it a compute unit to itself.  us with 64, 32 and 16 rows (64 columns behind 4096 elements; 256 behind
+        // 7168): 2048 rows 34, 26, 21 and 55, 43, 66; 6001 rows 34, 27, 40 and 109, 119, 192; 12000 rows 35, 49, 59 and 165, 233, 381.
+        const int rt = (int64_t)blocks(1) * gy <= moe_cus() ? 1 : (int64_t)blocks(2) * gy <= moe_cus() ? 2 : 4;
+        auto launch = [&](auto kernel, int rt) { kernel<<<dim3(blocks(rt), gy), dim3(256), 0, s>>>(a); };
+        if (rows <= 1024) narrow_mfma_kernel<1, 1, 8><<<dim3(blocks(1), (unsigned)tiles), dim3(512), 0, s>>>(a);
+        else if (five) launch(rt == 1 ? narrow_mfma_kernel<1, 5, 4> : rt == 2 ? narrow_mfma_kernel<2, 5, 4> : narrow_mfma_kernel<4, 5, 4>, rt);
+        else launch(rt == 1 ? narrow_mfma_kernel<1, 4, 4> : rt == 2 ? narrow_mfma_kernel<2, 4, 4> : narrow_mfma_kernel<4, 4, 4>, rt);
     }
     PA_CHECK_LAUNCH("pa_narrow_linear");
     return PA_OK;

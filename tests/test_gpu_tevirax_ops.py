@@ -469,6 +469,19 @@ def test_narrow_products_are_32_bit(rows, n, k, dtype):
         assert ((got.cpu().double() - want).abs() / (want.abs() + k ** 0.5)).max() < 2e-6
 
 
+@pytest.mark.parametrize("n,k", [(64, 328), (65, 1032), (9, 64)])
+def test_narrow_products_by_rows_of_a_workgroup(n, k):
+    """16, 32 and 64 rows a workgroup, at the ends of their ranges on 256 compute units: the same sums, to the bit."""
+    announce(f"narrow rows of a workgroup {n} {k}")
+    x, w = _rand(16385, k, dtype=BF), _rand(n, k, dtype=BF, seed=1)
+    x_dev, w_dev = x.to(DEV), w.to(DEV)
+    all_rows = ops.narrow_linear(x_dev, w_dev)
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)  # k sums, each off by half a unit in the last place of at most the absolute sum
+    assert bool(((all_rows.cpu().double() - x.double() @ w.double().T).abs() <= bound).all())
+    for rows in (1025, 4096, 4097, 8192, 8193, 16384):
+        assert torch.equal(ops.narrow_linear(x_dev[:rows], w_dev), all_rows[:rows]), rows
+
+
 @pytest.mark.parametrize("rows,experts,top,groups,keep,shared", [(1, 6, 2, 3, 2, True), (37, 8, 3, 2, 1, False), (130, 5, 4, 1, 1, True), (64, 256, 8, 8, 4, True),
                                                                 (9, 100, 20, 100, 40, False), (2000, 16, 4, 4, 2, True), (3, 1, 1, 1, 1, False),
                                                                 (50, 1000, 10, 20, 5, True), (5000, 120, 6, 12, 12, True)])
