@@ -58,6 +58,15 @@ def _run(name: str, *args) -> None:
         _lib.check(name, status)
 
 
+def _whole(name: str, function: str, *args):
+    """A wrapper's native form, which calls the library's ``function``: its result, or None where something does not fit or
+    nothing has been built (the wrapper goes its own way)."""
+    got = getattr(_host, name)(*args) if _host is not None else None
+    if got.__class__ is int and got:
+        _lib.check(function, got)
+    return got
+
+
 def kv_scatter(k_cache: Tensor, v_cache: Tensor, k_src: Tensor, v_src: Tensor, slots: Tensor) -> None:
     """``cache[slots[i]] = src[i]``; caches ``[total_slots, Hkv, D]``, src ``[N, Hkv, D]``, slots int64 ``[N]``."""
     total_slots, hkv, d = k_cache.shape
@@ -547,6 +556,9 @@ def lightning(u: Tensor, portions: Portions, state: Tensor, decay_powers: Tensor
     """Lightning attention over projection rows ``[q | k | v | ...]`` with the state carried in ``state`` (see
     ``lightning_state``): portions of bf16 rows in chunks on the matrix cores (``pa_lightning_chunked``), single rows
     and float32 rows token by token (``pa_lightning_recurrent``).  ``out`` ``[rows, heads * vdim]``."""
+    token = portions.q_lens is None or u.dtype == torch.float32
+    if _whole("lightning", "pa_lightning_recurrent" if token else "pa_lightning_chunked", u, *portions[:4], portions.max_q_len, state, decay_powers, heads, dim, vdim, out, workspace) is not None:
+        return out
     _dense(state, decay_powers, out, *portions[:4])
     _typed(torch.int32, *portions[:4])
     _typed(torch.float32, state, decay_powers)
@@ -560,7 +572,7 @@ def lightning(u: Tensor, portions: Portions, state: Tensor, decay_powers: Tensor
     head = (u, _row_stride(u), rows, state, state.shape[0], decay_powers, portions.ctx_lens,
             portions.q_lens, portions.q_starts, portions.state_slots, batch)
     tail = (out, heads, dim, vdim, PA_DTYPE[u.dtype])
-    if portions.q_lens is None or u.dtype == torch.float32:
+    if token:
         _run("pa_lightning_recurrent", *head, *tail, _stream(u))
     else:
         _run("pa_lightning_chunked", *head, portions.max_q_len, *tail, workspace, _nbytes(workspace), _stream(u))
@@ -615,8 +627,11 @@ def gated_linear(kind: str, q: Tensor, k: Tensor, v: Tensor, gates: Tuple[Tensor
     """A linear recurrence with gates per token and head (``pa_gated_linear``), ``kind`` ``"ssd"`` or ``"mlstm"``.  q, k, v
     and the gates ``[rows, heads]`` may be column slices; ``constants`` float32 ``[heads]`` each: dt bias, decay rate and
     skip, or the biases of the two gates; ``state`` float32 ``[slots, heads, gated_linear_state_floats]``."""
-    rows, batch = v.shape[0], portions.ctx_lens.numel()
     ga, gb = gates
+    if _whole("gated_linear", "pa_gated_linear", _GATED[kind], q, k, v, heads_per_group, ga, gb, *constants, cap, q_scale, den_eps, *portions[:4], portions.max_q_len, state,
+              gated_linear_state_floats(kind, dim, vdim), heads, dim, vdim, out, workspace) is not None:
+        return out
+    rows, batch = v.shape[0], portions.ctx_lens.numel()
     _dense(state, out, *constants, *portions[:4])
     _typed(torch.int32, *portions[:4])
     _typed(torch.float32, state, *constants)
@@ -641,6 +656,9 @@ def gated_linear(kind: str, q: Tensor, k: Tensor, v: Tensor, gates: Tuple[Tensor
 
 def narrow_linear(x: Tensor, w: Tensor) -> Tensor:
     """``x w^T`` summed and returned in float32 (``pa_narrow_linear``), for a few outputs."""
+    out = _whole("narrow_linear", "pa_narrow_linear", x, w)
+    if out is not None:
+        return out
     _dense(w)
     _typed(x.dtype, w)
     if w.shape[1] != x.shape[1]:
@@ -667,6 +685,10 @@ def moe_choose(logits: Tensor, experts: int, top: int, groups: int, keep: int, s
                correction: Optional[Tensor] = None) -> ExpertChoice:
     """``pa_moe_choose`` over float32 ``logits`` ``[rows, experts + identity]``; ``shared`` ``"gated"`` (one column more, its
     gate), ``"plain"`` or None."""
+    got = _whole("moe_choose", "pa_moe_choose", logits, correction, experts, identity, top, groups, keep, _SHARED[shared], int(shared == "gated"), _SCORES[scores], group_top,
+                 int(renormalize))
+    if got is not None:
+        return ExpertChoice(*got)
     rows, every = logits.shape[0], experts + identity
     _dense(logits, correction)
     _typed(torch.float32, logits, correction)
@@ -687,6 +709,9 @@ def moe_choose(logits: Tensor, experts: int, top: int, groups: int, keep: int, s
 def moe_product(x: Tensor, choice: ExpertChoice, w: Tensor, n: int, k: int, glu: bool) -> Tensor:
     """Every item's product with its expert's weights (``pa_moe_product``): ``x`` ``[rows, k]`` or one row per item,
     ``w`` ``[experts, n (glu: 2n), stride]`` zero past k -> ``[rows * top, n]``."""
+    out = _whole("moe_product", "pa_moe_product", x, *choice, w, n, k, int(glu))
+    if out is not None:
+        return out
     rows, top = choice.ids.shape
     _dense(w, *choice)
     _typed(x.dtype, w)
@@ -709,6 +734,9 @@ def delta_rule(q: Tensor, k: Tensor, v: Tensor, decay_logits: Tensor, beta_logit
                heads_per_group: int = 1, workspace: Optional[Tensor] = None) -> Tensor:
     """The gated delta rule (``pa_delta``).  q, k, v and the logits ``[rows, heads]`` may be column slices; ``state`` float32
     ``[slots, heads, pad16(dim), pad16(vdim)]``."""
+    if _whole("delta_rule", "pa_delta", q, k, v, heads_per_group, decay_logits, beta_logits, decay_bias, decay_rate, q_scale, *portions[:4], portions.max_q_len, state, heads,
+              dim, vdim, out, workspace) is not None:
+        return out
     rows, batch = v.shape[0], portions.ctx_lens.numel()
     pad = lambda n: -(-n // 16) * 16
     _dense(state, out, decay_bias, decay_rate, *portions[:4])
@@ -865,6 +893,8 @@ def channel_linear(q: Tensor, forget: Tensor, v: Tensor, f_bias: Optional[Tensor
                    heads: int, dim: int, vdim: int, out: Tensor, q_act: Optional[str] = None, workspace: Optional[Tensor] = None) -> Tensor:
     """Linear attention with a forget gate per channel (``pa_channel_linear``).  q, the gate's logits and v may be column slices;
     ``f_bias`` and ``lower`` float32 ``[heads * dim]``, ``state`` float32 ``[slots, heads, pad16(dim), pad16(vdim)]``."""
+    if _whole("channel_linear", "pa_channel_linear", q, _ACTS[q_act], forget, f_bias, lower, v, *portions[:4], portions.max_q_len, state, heads, dim, vdim, out, workspace) is not None:
+        return out
     rows, batch = v.shape[0], portions.ctx_lens.numel()
     pad = lambda n: -(-n // 16) * 16
     _dense(state, out, f_bias, lower, *portions[:4])

@@ -482,6 +482,38 @@ def test_narrow_products_by_rows_of_a_workgroup(n, k):
         assert torch.equal(ops.narrow_linear(x_dev[:rows], w_dev), all_rows[:rows]), rows
 
 
+@pytest.mark.parametrize("rows,identity,shared", [(1, 0, "gated"), (70, 5, None), (300, 0, "plain")])
+def test_whole_calls_are_the_wrappers(monkeypatch, rows, identity, shared):
+    """Choice, products and narrow products by the native forms of their wrappers, and by the wrappers' own way: types, shapes, views and results."""
+    announce(f"whole calls {rows} {identity} {shared}")
+    h, router = _rand(rows, 136, dtype=BF).to(DEV)[:, :128], _rand(16 + identity + (shared == "gated"), 128, dtype=BF, seed=1).to(DEV)
+    w = torch.zeros(16, 96, 128, dtype=BF)
+    w[:] = _rand(16 * 96, 128, dtype=BF, seed=2).view(16, 96, 128)
+    w = w.to(DEV)
+
+    def run():
+        logits = ops.narrow_linear(h, router)
+        choice = ops.moe_choose(logits, 16, 3, 1, 1, shared, identity)
+        return [logits, *choice[:3], ops.moe_product(h, choice, w, 48, 128, True), ops.moe_product(h, choice, w, 96, 128, False)], choice
+
+    with monkeypatch.context() as m:
+        taken = []
+        whole = ops._whole
+        m.setattr(ops, "_whole", lambda *a: taken.append(whole(*a)) or taken[-1])
+        got, choice = run()
+        assert len(taken) == 4 and all(t is not None for t in taken)
+    monkeypatch.setattr(ops, "_whole", lambda *a: None)
+    want, other = run()
+    assert choice._fields == other._fields and choice.lists.shape == other.lists.shape
+    for e, n in enumerate(other.counts.tolist()):
+        assert sorted(choice.lists[e, :n].tolist()) == sorted(other.lists[e, :n].tolist())
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype and a.device == b.device and a.shape == b.shape and a.stride() == b.stride()
+    live = [0, 1, 2, 3] + ([4, 5] if identity == 0 else [])  # (items of identity experts have no product)
+    for i in live:
+        assert torch.equal(got[i], want[i]), i
+
+
 @pytest.mark.parametrize("rows,experts,top,groups,keep,shared", [(1, 6, 2, 3, 2, True), (37, 8, 3, 2, 1, False), (130, 5, 4, 1, 1, True), (64, 256, 8, 8, 4, True),
                                                                 (9, 100, 20, 100, 40, False), (2000, 16, 4, 4, 2, True), (3, 1, 1, 1, 1, False),
                                                                 (50, 1000, 10, 20, 5, True), (5000, 120, 6, 12, 12, True)])

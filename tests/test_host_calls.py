@@ -112,6 +112,35 @@ def test_arguments():
         call(t, t, 0, "1")
 
 
+@pytest.mark.parametrize("name,count", [("gated_linear", 25), ("delta_rule", 20), ("channel_linear", 17), ("lightning", 13), ("narrow_linear", 2), ("moe_choose", 12),
+                                        ("moe_product", 9)])
+def test_whole_calls_that_do_not_fit_are_left_to_the_wrapper(name, count):
+    """Another number of arguments, arguments of other kinds and tensors that lie on no device: no answer, and no exception."""
+    call = getattr(host, name)
+    t = torch.zeros(4, 4)
+    for args in ((), (t,) * (count - 1), (t,) * count, (1,) * count, (1.0,) * count, (None,) * count, ("x",) * count, (1 << 70,) * count, (-1,) * count):
+        assert call(*args) is None
+    for i in range(count):
+        assert call(*(t if j == i else 1 for j in range(count))) is None and call(*(1.0 if j == i else t for j in range(count))) is None
+
+
+def test_whole_calls_on_the_cpu_say_what_the_wrapper_says():
+    i32 = lambda *n: torch.zeros(*n, dtype=torch.int32)
+    runs = ops.Portions(i32(2), i32(2))
+    rows = torch.zeros(2, 64)
+    for call in (lambda: ops.narrow_linear(rows, torch.zeros(3, 64)), lambda: ops.moe_choose(rows, 64, 2, 1, 1),
+                 lambda: ops.lightning(torch.zeros(2, 192), runs, torch.zeros(2, 1, 64, 64), torch.zeros(1, 65), 1, 64, 64, rows),
+                 lambda: ops.channel_linear(rows, rows, rows, None, torch.zeros(64), runs, torch.zeros(2, 1, 64, 64), 1, 64, 64, rows.clone())):
+        with pytest.raises(RuntimeError, match="HIP device"):
+            call()
+    for call in (lambda: ops.narrow_linear(rows, torch.zeros(3, 63)), lambda: ops.narrow_linear(rows, torch.zeros(64, 3).t()), lambda: ops.moe_choose(rows, 63, 2, 1, 1),
+                 lambda: ops.moe_choose(rows.bfloat16(), 64, 2, 1, 1),
+                 lambda: ops.lightning(torch.zeros(2, 192), runs, torch.zeros(2, 1, 64, 48), torch.zeros(1, 65), 1, 64, 64, rows),
+                 lambda: ops.channel_linear(rows, rows[:, :32], rows, None, torch.zeros(64), runs, torch.zeros(2, 1, 64, 64), 1, 64, 64, rows.clone())):
+        with pytest.raises(ValueError):
+            call()
+
+
 def test_a_module_of_another_interpreter_or_torch_is_not_taken():
     root = ops.__file__.rsplit("/research_amd/", 1)[0]
     assert host.__file__.endswith("_host" + sysconfig.get_config_var("EXT_SUFFIX"))  # (which other interpreters do not look for)
