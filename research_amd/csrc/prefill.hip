@@ -3,7 +3,7 @@
 #include "prefill_plan.h"
 
 namespace pa_decode_detail {
-prefill_mfma_fn pa_prefill_asm_kernel(int dtype, int head_dim, bool lower_bounds, bool long_table);
+prefill_mfma_fn pa_prefill_asm_kernel(int dtype, int head_dim, bool lower_bounds, bool long_table, bool one);
 constexpr int kWdTasks = 4, kWdKeys = 32, kWdCapGroups = 6144;  // (prefill_d256.h)
 prefill_mfma_fn pa_prefill_d256_kernel(int dtype, bool lower_bounds, bool long_table);
 }
@@ -159,7 +159,6 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
             split = want;
         }
         const bool lower_bounds = split > 1 || span > 0 || row_first_key != nullptr;
-        mfma = pa_prefill_asm_kernel(dtype, d_pad, lower_bounds, !fits);
         if (!lower_bounds && fits) {
             // The plain instance runs several groups of one (sequence, kv head) per workgroup, which share the
             // set-up of lengths and slot tables: as many (up to 8) as leave a workgroup for every compute unit, of
@@ -171,6 +170,7 @@ int prefill_launch(bool force_rowwise, const void *q, const void *k_cache, const
                                                  bt_stride * (int64_t)block_size, kPfKeys, prefill_cus());
             a.turned = a.groups_per_wg < gpw ? 1 : 0;
         }
+        mfma = pa_prefill_asm_kernel(dtype, d_pad, lower_bounds, !fits, a.groups_per_wg == 1);
     }
     // head_dim 256: one 32-row task per wave, loads driven by a table of 16-key groups - which must lie inside one
     // pool block (block sizes that are multiples of 16, or a single block per sequence); the kernel fills its table

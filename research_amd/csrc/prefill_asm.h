@@ -36,7 +36,12 @@ namespace pa_decode_detail {
 // the tile of the first key its first row sees, everything the loop counts in is relative to that tile.
 // LONG: the instance for workgroups that run more tiles than the tables hold (the same code with a loop around the
 // assembly that fills the tables again, which costs registers in the set-up).
-template <typename T, bool LO, int D, bool LONG = false>
+// ONE: a workgroup has one group.  What a workgroup does beside its tiles is one wave's instructions per SIMD, four to five cycles each, so that
+// their number is the time of a short launch.  With a loop over groups the compiler derives every group's constants ahead of it and spills scalar
+// registers around the tile loop; without one a workgroup of a single tile takes 21200 cycles, else 24000: of these, between the requests for Q and
+// the tables' loads 570, else 2950 (us a call: 14 / 2 heads of 128, a prompt of 18 rows 13.5 -> 12.7; 16 / 8 of 96, 10 of 111 .. 223 behind 336
+// keys 26.2 -> 24.7; 32 / 8 of 128, 48 of 99 .. 145 behind 1008 148 -> 144, 32 of 97 .. 249 behind 2048 224.6 -> 220.3).
+template <typename T, bool LO, int D, bool LONG = false, bool ONE = LO || LONG>
 __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseArgs a) {
     using M = Mfma16<T>;
     using X8 = typename M::x8;
@@ -71,14 +76,14 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
     // third of what a group costs beside its loop and counts where the loop is short (prompts of a few hundred
     // tokens).
     const int kvh = blockIdx.x;
-    const int n_splits = a.splits;  // pieces a workgroup's tiles are cut into (1: none; more only in the LO instance)
-    const int gpw = (LO || LONG) ? 1 : a.groups_per_wg;  // groups per workgroup
+    const int n_splits = LO ? a.splits : 1;  // pieces a workgroup's tiles are cut into (1: none; more only in the LO instance)
+    const int gpw = ONE ? 1 : a.groups_per_wg;  // groups per workgroup
     int piece = (int)blockIdx.y % n_splits;
     const int chunk_y = (int)blockIdx.y / n_splits;
     int n_chunks = gridDim.y / n_splits;
     const int n_seqs = gridDim.z;
     const int lin = chunk_y + n_chunks * blockIdx.z;
-    const bool group_major = a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];
+    const bool group_major = n_chunks > 1 && a.ctx_lens[0] - a.q_lens[0] < a.q_lens[0];  // (one: no order, and no look at the lengths first)
     const int turned = (LO || LONG) || !a.turned ? chunk_y : plan_turned_chunk(chunk_y, (int)blockIdx.z, n_chunks);
     int wg_chunk = group_major ? n_chunks - 1 - lin / n_seqs : turned;
     int b = group_major ? lin % n_seqs : (int)blockIdx.z;
@@ -308,9 +313,15 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
             uint32_t w[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[e] = M::pack((float)q8[2 * e] * sc, (float)q8[2 * e + 1] * sc);
-            if (padded && (uint32_t)(2 * ks + half) >= real_chunks) w[0] = w[1] = w[2] = w[3] = 0;  // past the row's end
             qreg[c][ks] = __builtin_bit_cast(X8, uint4{w[0], w[1], w[2], w[3]});
         }
+    if (padded) {  // (uniform) zeros past the row's end
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                if ((uint32_t)(2 * ks + half) >= real_chunks) qreg[c][ks] = __builtin_bit_cast(X8, uint4{0, 0, 0, 0});
+    }
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -641,11 +652,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
     }
     // ---- normalise; rows go through LDS so that every store instruction writes whole 256-byte rows ----
     __syncthreads();  // every wave is done with the ring
-    const int group_next = __builtin_amdgcn_readfirstlane(group_of(gi + 1));
+    const int group_next = ONE ? group_end : __builtin_amdgcn_readfirstlane(group_of(gi + 1));
     tile0_ahead = false;
-    if (group_next < group_end) {  // (uniform) the next group's Q rows and its tile 0 travel during the write-out
+    if (!ONE && group_next < group_end) {  // (uniform) the next group's Q rows and its tile 0 travel during the write-out
         issue_q(group_next);
-        if constexpr (!LO && !LONG) {
+        if constexpr (!ONE) {
             issue(0);
             tile0_ahead = true;
         }
@@ -693,13 +704,13 @@ __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseAr
                                                    out_ofs + i * QRPI * (int)q_row_bytes, 0, 0);
     }
     gi = __builtin_amdgcn_readfirstlane(gi + 1);
-    if (group_next >= group_end) break;
+    if (ONE || group_next >= group_end) break;
     // (no barrier: until the next group's barrier behind its Q^T read, a wave touches only its own staged rows)
     }  // groups of the workgroup
 }
 
 // nullptr unless the element type has this kernel; `lower_bounds`: the instance for sliding windows and per-row
-// first keys; `long_table`: the instance that fills its tables more than once
-prefill_mfma_fn pa_prefill_asm_kernel(int dtype, int head_dim, bool lower_bounds, bool long_table);
+// first keys; `long_table`: the instance that fills its tables more than once; `one`: of the others, the instance for one group a workgroup
+prefill_mfma_fn pa_prefill_asm_kernel(int dtype, int head_dim, bool lower_bounds, bool long_table, bool one);
 
 }  // namespace pa_decode_detail

@@ -145,6 +145,21 @@ def test_unequal_prompts_numbered_by_rows(d, hq, hkv, n, most, dtype):
             assert_close(got[starts[b]: starts[b] + r], want[b, :r], 2e-2, f"sequence {b} vs checker")
 
 
+@pytest.mark.parametrize("d,hq,hkv,n,rows", [(64, 8, 8, 32, 513), (128, 16, 8, 33, 300), (32, 8, 8, 64, 257)])
+def test_one_and_several_groups_of_a_workgroup(d, hq, hkv, n, rows):
+    """Launches with a workgroup for every compute unit run several groups in each (an instance of its own); a few of their sequences
+    alone run one: the same results, to the bit."""
+    announce(f"prefill groups of a workgroup: {n} prompts of {rows} rows, {hq} / {hkv} heads of {d}")
+    c = Case([40] * n, [rows] * n, hq, hkv, d, seed=rows, width=1)
+    every = c.run()
+    for lo, hi in ((0, 1), (n - 2, n)):
+        part = object.__new__(Case)
+        part.__dict__.update(c.__dict__, q=c.q[lo:hi], ctx=c.ctx[lo:hi], chunk=c.chunk[lo:hi], prefix=c.prefix[lo:hi], tables=c.tables[lo:hi], dev_tables=c.dev_tables[lo:hi].contiguous())
+        assert torch.equal(part.run(), every[lo:hi])
+    want = po.paged_prefill_chunk(c.q[:1], c.k, c.v, c.tables[:1], c.prefix[:1], c.chunk[:1], 16, c.scale)
+    assert_close(every[:1], want, 2e-2, "first sequence vs checker")
+
+
 def test_windows_first_keys_and_absent_blocks_in_pieces():
     announce("split prefill: window, per-row first keys, absent blocks")
     # (under a window a workgroup sees window + 256 keys at most: the library splits only wide windows)
