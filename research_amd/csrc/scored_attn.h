@@ -65,6 +65,27 @@ __device__ __forceinline__ scored_u4 scored_load16(const uint16_t *p, bool there
     return *reinterpret_cast<global_u4>(there ? reinterpret_cast<uintptr_t>(p) : reinterpret_cast<uintptr_t>(kScoredZeros));
 }
 
+// The rows of one kv head in a pool of less than 2 GiB, read by 32-bit offsets: a row that is not there (slot -1) and what lies past a row's end
+// (an offset of kScoredAway) fall outside the descriptor and come back as zeros.  A 16-byte piece takes two instructions beside its load, by address
+// and choice of one fourteen, which the vector unit pays for where it has no other to spare (portions, 16 / 4 heads of 128, window 1024, cap: 8 of 700
+// .. 4000 rows 146 -> 139 us; the sums of attention with mixed heads are no faster for it, and keep addresses).
+constexpr uint32_t kScoredAway = 0x80000000u;
+struct ScoredRows {
+    __amdgpu_buffer_rsrc_t rows;
+    int row_bytes;
+    __device__ __forceinline__ scored_u4 load16(int slot, uint32_t off) const {  // (fewer than 2^23 slots: 24-bit products)
+        return __builtin_bit_cast(scored_u4, __builtin_amdgcn_raw_buffer_load_b128(rows, (uint32_t)__mul24(slot, row_bytes) + off, 0, 0));
+    }
+};
+__device__ __forceinline__ bool scored_small(const ScoredArgs &a, int dim) {
+    const int64_t row_bytes = (int64_t)a.hkv * dim * 2;
+    return row_bytes >= 256 && row_bytes < (1 << 23) && a.num_blocks * a.bs * row_bytes <= 0x7f000000;
+}
+__device__ __forceinline__ ScoredRows scored_rows(const ScoredArgs &a, const void *pool, int dim, int kvh) {
+    const int row_bytes = a.hkv * dim * 2, first = kvh * dim * 2;
+    return {__builtin_amdgcn_make_buffer_rsrc((char *)const_cast<void *>(pool) + first, 0, (int)(a.num_blocks * a.bs * row_bytes - first), 0x00020000), row_bytes};
+}
+
 constexpr float kScoredLog2e = 1.4426950408889634f;
 constexpr float kScoredNone = -1.0e30f;  // finite stand-in for minus infinity
 

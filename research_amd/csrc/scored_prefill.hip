@@ -103,18 +103,33 @@ template <int DK, int DV, bool CAP> __global__ __launch_bounds__(256, DV == 256 
     // cost as much as the tile's loads), and the block's id, loaded a tile ahead.
     const int k_start = wg_lo / kSpKeys * kSpKeys, step_blk = kSpKeys / a.bs, step_rem = kSpKeys % a.bs, last_blk = (int)min(a.bt_stride, (int64_t)0x7fffffff) - 1;
     int blk = (k_start + lane) / a.bs, rem = (k_start + lane) % a.bs, id = table[min(blk, last_blk)];
+    const bool small = scored_small(a, a.k_dim) && scored_small(a, a.v_dim);
+    const ScoredRows k_rows = scored_rows(a, a.k, a.k_dim, kvh), v_rows = scored_rows(a, a.v, a.v_dim, kvh);
     scored_u4 kr[NK], vr[NV];
     auto fetch = [&](int k0) {
         const int slots = k0 + lane < wg_hi && blk <= last_blk && (uint32_t)id < (uint32_t)a.num_blocks ? id * a.bs + rem : -1;
+        if (small) {
 #pragma unroll
-        for (int n = 0; n < NK; ++n) {
-            const int c = tid + 256 * n, s = __shfl(slots, c / (DK / 8), 64), e = c % (DK / 8) * 8;
-            kr[n] = scored_load16(kp + s * k_tok + e, s >= 0 && e < kreal);
-        }
+            for (int n = 0; n < NK; ++n) {
+                const int c = tid + 256 * n, e = c % (DK / 8) * 8;
+                kr[n] = k_rows.load16(__shfl(slots, c / (DK / 8), 64), e < kreal ? 2u * e : kScoredAway);
+            }
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            const int c = tid + 256 * n, s = __shfl(slots, c / (DV / 8), 64), e = c % (DV / 8) * 8;
-            vr[n] = scored_load16(vp + s * v_tok + e, s >= 0 && e < vreal);
+            for (int n = 0; n < NV; ++n) {
+                const int c = tid + 256 * n, e = c % (DV / 8) * 8;
+                vr[n] = v_rows.load16(__shfl(slots, c / (DV / 8), 64), e < vreal ? 2u * e : kScoredAway);
+            }
+        } else {
+#pragma unroll
+            for (int n = 0; n < NK; ++n) {
+                const int c = tid + 256 * n, s = __shfl(slots, c / (DK / 8), 64), e = c % (DK / 8) * 8;
+                kr[n] = scored_load16(kp + s * k_tok + e, s >= 0 && e < kreal);
+            }
+#pragma unroll
+            for (int n = 0; n < NV; ++n) {
+                const int c = tid + 256 * n, s = __shfl(slots, c / (DV / 8), 64), e = c % (DV / 8) * 8;
+                vr[n] = scored_load16(vp + s * v_tok + e, s >= 0 && e < vreal);
+            }
         }
         blk += step_blk;
         rem += step_rem;

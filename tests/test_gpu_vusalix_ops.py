@@ -266,6 +266,31 @@ SCORED = [  # heads, kv heads, dim, vdim, window, cap, buckets, bias_max
     (20, 1, 40, 40, None, 8.0, 12, 300), (2, 1, 136, 200, 64, 15.0, 6, 64), (5, 5, 24, 16, 1, 4.0, 2, 3), (9, 3, 33, 21, 50, 12.0, 10, 40)]
 
 
+@pytest.mark.parametrize("dim,vdim,window", [(64, 64, 0), (56, 48, 90), (64, 40, 33)])
+def test_pools_read_by_offsets_and_by_addresses(dim, vdim, window):
+    """Rows of 256 bytes and more are read by 32-bit offsets, shorter ones by addresses: two kv heads at once and one at a time, to the bit; blocks that
+    are not there are zeros, and what lies past a row's end and in blocks of no sequence (NaN) is nobody's."""
+    announce(f"scored by offsets {dim} {vdim} {window}")
+    lens = [1, 33, 250, 97]
+    paged = Paged(lens, 2, 64, 64, BF)
+    used = set(paged.tables[paged.tables >= 0].tolist())
+    for blk in set(range(paged.k.shape[0] // 16)) - used:
+        paged.k[blk * 16: blk * 16 + 16] = paged.v[blk * 16: blk * 16 + 16] = float("nan")
+    paged.k[..., (dim + 7) // 8 * 8:] = float("nan")
+    paged.v[..., (vdim + 7) // 8 * 8:] = float("nan")
+    paged.tables[2, 3] = -1
+    q = _rand(sum(lens), 4, dim, seed=9).to(BF)
+    bias, sink = _rand(4, 60, seed=10), _rand(4, seed=11)
+    picks = [(i, 0, n) for i, n in enumerate(lens)]
+    both = _scored(paged, picks, (q,), vdim, BF, 0.2, window, softcap=9.0, bias=bias, sink=sink)
+    assert bool(torch.isfinite(both.float()).all())
+    k, v = paged.k, paged.v
+    for j in range(2):
+        paged.k, paged.v, h = k[:, j: j + 1].contiguous(), v[:, j: j + 1].contiguous(), slice(2 * j, 2 * j + 2)
+        one = _scored(paged, picks, (q[:, h].contiguous(),), vdim, BF, 0.2, window, softcap=9.0, bias=bias[h].contiguous(), sink=sink[h].contiguous())
+        assert torch.equal(one, both[:, h])
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("heads,kv,dim,vdim,window,cap,buckets,most", SCORED)
 def test_biased_attention_in_portions_and_single_rows(heads, kv, dim, vdim, window, cap, buckets, most, dtype):
