@@ -118,7 +118,7 @@ def test_many_prompts_of_unequal_length_in_pieces(d, hq, hkv, n):
     base, got, want = c.run(), c.run(2), c.want()
     for b, rows in enumerate(c.chunk):
         if rows:
-            assert_close(got[b, :rows], want[b, :rows], 2e-2, f"sequence {b} vs checker")
+            assert_close(got[b, :rows], want[b, :rows], 2e-2, f"sequence {b} vs oracle")
             assert_close(got[b, :rows], base[b, :rows], 6e-3, f"sequence {b} vs unsplit")
         assert not got[b, rows:].any()
 
@@ -142,7 +142,7 @@ def test_unequal_prompts_numbered_by_rows(d, hq, hkv, n, most, dtype):
     want = c.want()
     for b, r in enumerate(rows):
         if r:
-            assert_close(got[starts[b]: starts[b] + r], want[b, :r], 2e-2, f"sequence {b} vs checker")
+            assert_close(got[starts[b]: starts[b] + r], want[b, :r], 2e-2, f"sequence {b} vs oracle")
 
 
 @pytest.mark.parametrize("d,hq,hkv,n,rows", [(64, 8, 8, 32, 513), (128, 16, 8, 33, 300), (32, 8, 8, 64, 257)])
@@ -157,7 +157,7 @@ def test_one_and_several_groups_of_a_workgroup(d, hq, hkv, n, rows):
         part.__dict__.update(c.__dict__, q=c.q[lo:hi], ctx=c.ctx[lo:hi], chunk=c.chunk[lo:hi], prefix=c.prefix[lo:hi], tables=c.tables[lo:hi], dev_tables=c.dev_tables[lo:hi].contiguous())
         assert torch.equal(part.run(), every[lo:hi])
     want = po.paged_prefill_chunk(c.q[:1], c.k, c.v, c.tables[:1], c.prefix[:1], c.chunk[:1], 16, c.scale)
-    assert_close(every[:1], want, 2e-2, "first sequence vs checker")
+    assert_close(every[:1], want, 2e-2, "first sequence vs oracle")
 
 
 def test_windows_first_keys_and_absent_blocks_in_pieces():
