@@ -335,9 +335,12 @@ __global__ __launch_bounds__(64 * NW, PAIR || (KD == 64 && NW == 8) ? 4 : KD == 
                 if (st > rt + 1) continue;  // (tile rt + 1 is read as zeros when the last k-step covers it)
                 const int t = 16 * rt + l16, c = 16 * st + 4 * g;
                 const float *f = pw + t - c;
+                f4 x;  // (a later row's key may be no number: its score is put away ahead of the zero that it meets)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] = (c + i <= t ? sc[m][i] : 0.f) * f[-i];
                 uint2 hi, lo;
-                la_split2(sc[m][0] * f[0], sc[m][1] * f[-1], hi.x, lo.x);
-                la_split2(sc[m][2] * f[-2], sc[m][3] * f[-3], hi.y, lo.y);
+                la_split2(x[0], x[1], hi.x, lo.x);
+                la_split2(x[2], x[3], hi.y, lo.y);
                 *reinterpret_cast<uint2 *>(a_hi + t * kLaPitchA + la_paired(c)) = hi;
                 *reinterpret_cast<uint2 *>(a_lo + t * kLaPitchA + la_paired(c)) = lo;
             }

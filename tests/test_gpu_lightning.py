@@ -143,3 +143,37 @@ def test_long_portions_in_segments(heads, dim, vdim):
             for b in (0, 1):
                 case.check(b, first, got[b])
                 case.check_state(b, 1 + b)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("heads,dim,vdim,lens", [(2, 128, 128, [150, 65]), (2, 64, 128, [150, 65]), (3, 64, 48, [150, 65]), (2, 128, 64, [150, 65]), (1, 256, 80, [150, 65]),
+                                                 (1, 256, 144, [150, 65]), (32, 128, 128, [400, 2600, 900, 1900, 1200, 500])])
+def test_a_key_that_is_no_number_leaves_the_rows_before_it_alone(heads, dim, vdim, lens, bad):
+    """Every group of 16 rows of a chunk, its first, a middle and its last one (finite values; the last shape: in segments, two workgroups a
+    compute unit): the rows before are the same, to the bit."""
+    announce(f"lightning keys {heads}x{dim}x{vdim} {bad}")
+    g = torch.Generator().manual_seed(12)
+    u = torch.randn(sum(lens), heads * (2 * dim + vdim), generator=g).to(BF).to(DEV)
+    powers, starts = _powers(np.linspace(0.9, 0.999, heads).tolist()), np.cumsum([0] + lens[:-1]).tolist()
+    n_ws = ops.lightning_workspace_bytes(len(lens), heads, dim, vdim, max(lens), sum(lens))
+    ws = torch.empty(n_ws, dtype=torch.uint8, device=DEV) if n_ws else None
+    portions = ops.Portions(_i32(lens), _i32(range(len(lens))), _i32(lens), _i32(starts), max_q_len=max(lens))
+
+    def run(rows):
+        out = torch.empty(sum(lens), heads * vdim, dtype=BF, device=DEV)
+        return ops.lightning(rows, portions, ops.lightning_state(len(lens), heads, dim, vdim, DEV), powers, heads, dim, vdim, out, ws)
+
+    want = run(u)
+    assert bool(torch.isfinite(want.float()).all())
+    for row in (0, 1, 8, 15, 16, 20, 31, 32, 40, 47, 48, 52, 63):
+        at = starts[0] + 64 + row, starts[1] + row
+        rows = u.clone()
+        for r in at:
+            rows[r, heads * dim + 3] = bad  # a channel of the first head's key
+        got = run(rows)
+        alone = torch.ones(sum(lens), dtype=torch.bool, device=DEV)
+        for r, lo, n in zip(at, starts, lens):
+            alone[r: lo + n] = False
+        first = slice(0, vdim)
+        assert torch.equal(got[alone], want[alone]) and torch.equal(got[:, vdim:], want[:, vdim:]), row
+        assert not bool(torch.isfinite(got[list(at), first].float()).any()), row
