@@ -205,6 +205,9 @@ template <int KD, int NW, bool STATES>
 __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs a) {
     using L = ClTile<KD, NW, STATES>;
     constexpr int kRows = L::rows, kPitch = L::pitch, kThr = L::threads, kPairs = KD / 2;
+    // Outputs behind a chunk's last block.  At dim 256 a chunk has two blocks and its state half of the registers: outputs and loads kept beside the second
+    // one were spilled (second pass, 8 heads of 256 x 256, 6 prompts of 700 .. 4000 rows, us: 265, else 181; 17 of 300 .. 700, 200 x 104, 230, else 147).
+    constexpr bool kLate = KD < 256;
     extern __shared__ __align__(16) char lds[];
     __bf16 *k_hi = reinterpret_cast<__bf16 *>(lds), *k_lo = k_hi + L::elemsK;        // R K
     __bf16 *q_hi = k_lo + L::elemsK, *q_lo = q_hi + L::elems;                         // P Q
@@ -390,8 +393,9 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
             *reinterpret_cast<la_u2 *>(v_s + row * L::vPitch + col) = vr[n];
         }
         const bool more = r0 + kRows < r_end;
-        if (STATES && more) {
+        if ((STATES || !kLate) && more) {
             fetch_z(r0 + kRows);
+            fetch_q(r0 + kRows);
             fetch_v(r0 + kRows);
         }
         __syncthreads();
@@ -426,10 +430,22 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 scores[wave * 64 + lane] = x;
             }
         }
-        // ---- blocks in turn; every wave its own columns.  (The scores are asked for behind the last one, so that the waves that make them and the
-        // others do not wait for each other here; the next rows' loads are spread over the blocks.)
+        // ---- blocks in turn; every wave its own columns.  (kLate: the scores are asked for behind the last one, so that the waves that make them
+        // and the others do not wait for each other here; the next rows' loads are spread over the blocks.)
         f4 o[STATES ? 1 : L::blocks];  // v = 4 g + i of the wave's columns, t = l16
         la_bf4 v4[L::blocks];          // V^T or V: rows 4 g .. 4 g + 3 of the block, column l16 of the wave
+        auto put_rows = [&](int blk) {
+            const int first = blk * kClBlock;
+            f4 &x = o[STATES ? 0 : blk];
+            x = la_mfma(la_join(v4[blk], v4[blk]), __builtin_bit_cast(bf8, scores[blk * 64 + lane]), x);
+            const int ldo = a.heads * a.vdim, c = vw + 4 * g;
+            const uint16_t *out = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0 + first) * (int64_t)ldo + h * a.vdim + v0;
+            const int n = nv - first < kClBlock ? nv - first : kClBlock;
+            const __amdgpu_buffer_rsrc_t dst = la_tile(out, ldo, n, vcols);
+            const la_u2 y = {row_pack_bf16(x[0], x[1]), row_pack_bf16(x[2], x[3])};
+            __builtin_amdgcn_raw_buffer_store_b64(y, dst, c < vcols ? (uint32_t)(l16 * ldo + c) * 2u : kLaOutside, 0, 0);
+        };
+        if (!STATES && !kLate) __syncthreads();
 #pragma unroll
         for (int blk = 0; blk < L::blocks; ++blk) {
             if (blk * kClBlock >= nv) break;
@@ -451,6 +467,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                     }
                     o[blk] += o1;
                 }
+                if (!kLate) put_rows(blk);
             }
             const float *keep = whole + blk * KD + 8 * g;
             const __bf16 *kh = k_hi + (first + 4 * g + (l16 >> 2)) * L::pitchK + 8 * (l16 & 3);
@@ -468,7 +485,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 const __bf16 *x = half[dt % 2][dt / 4 % 2] + dt / 8 * 128 + dt / 2 % 2 * 32;
                 s[dt] = la_mfma(la_join(la_read_tr(x), la_read_tr(x + L::elemsK)), v8, s[dt]);
             }
-            if (!STATES && more) {
+            if (!STATES && kLate && more) {
                 if (blk == 0) fetch_z(r0 + kRows);
                 if (blk == 1) fetch_q(r0 + kRows);
                 if (blk == L::blocks - 1) fetch_v(r0 + kRows);
@@ -476,18 +493,12 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
         }
         if constexpr (!STATES) {
             __syncthreads();  // the scores are there; the next rows' operands may be written now
+            if constexpr (kLate)
 #pragma unroll
-            for (int blk = 0; blk < L::blocks; ++blk) {
-                if (blk * kClBlock >= nv) break;
-                const int first = blk * kClBlock;
-                o[blk] = la_mfma(la_join(v4[blk], v4[blk]), __builtin_bit_cast(bf8, scores[blk * 64 + lane]), o[blk]);
-                const int ldo = a.heads * a.vdim, c = vw + 4 * g;
-                const uint16_t *out = reinterpret_cast<const uint16_t *>(a.out) + (p.row0 + r0 + first) * (int64_t)ldo + h * a.vdim + v0;
-                const int n = nv - first < kClBlock ? nv - first : kClBlock;
-                const __amdgpu_buffer_rsrc_t dst = la_tile(out, ldo, n, vcols);
-                const la_u2 x = {row_pack_bf16(o[blk][0], o[blk][1]), row_pack_bf16(o[blk][2], o[blk][3])};
-                __builtin_amdgcn_raw_buffer_store_b64(x, dst, c < vcols ? (uint32_t)(l16 * ldo + c) * 2u : kLaOutside, 0, 0);
-            }
+                for (int blk = 0; blk < L::blocks; ++blk) {
+                    if (blk * kClBlock >= nv) break;
+                    put_rows(blk);
+                }
         } else {
             if (tid < KD)
                 for (int blk = 0; blk < L::blocks; ++blk) decayed *= whole[blk * KD + tid];
