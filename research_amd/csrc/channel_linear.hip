@@ -293,7 +293,9 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
     };
     auto fetch_v = [&](int r0) {
         const __amdgpu_buffer_rsrc_t tv = la_tile(uv + r0 * a.ldv, a.ldv, r_end - r0 < kRows ? r_end - r0 : kRows, vcols);
-        const int t = la_again(tid);  // (kept, these places were spilled, and a reload waits for all loads before it)
+        // (kept, these places were spilled, and a reload waits for all loads before it; STATES has registers for them, and is bound by the vector
+        // unit: 8 prompts of 700 .. 4000 rows, 32 heads of 128 x 128, first pass 106 us, worked out again 112)
+        const int t = STATES ? tid : la_again(tid);
 #pragma unroll
         for (int n = 0; n < L::vLoads; ++n) {
             const int c = t + kThr * n, row = c / (L::cols / 4), col = c % (L::cols / 4) * 4;
@@ -386,7 +388,7 @@ __global__ __launch_bounds__(64 * NW, 1) void channel_chunk_kernel(const ClArgs 
                 }
             }
         }
-        const int vt = la_again(tid);
+        const int vt = STATES ? tid : la_again(tid);
 #pragma unroll
         for (int n = 0; n < L::vLoads; ++n) {
             const int c = vt + kThr * n, row = c / (L::cols / 4), col = c % (L::cols / 4) * 4;
