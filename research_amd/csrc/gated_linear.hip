@@ -38,7 +38,6 @@ struct GlArgs {
     float *ws;  // segment states: S [dp][vp], n [dp], m, log decay, starting m
     int heads, per_group, dim, vdim, dp, vp;
     int batch, segments, seg_rows;
-    bool wide;  // rows of whole, aligned 16-byte pieces
 };
 
 struct GlPortion {
@@ -238,8 +237,13 @@ __device__ __forceinline__ float gl_scan_max(float x, int lane) {
 // 15000, of which products keep a SIMD busy for 5800 and the vector unit for 5100.
 // One prompt of 15999 rows, 4 heads of 256 x 512 (mLSTM): second pass 168 -> 124 us, first 73 -> 58; 8 prompts of 1226 .. 1840 rows, 16 heads of 128 x 64 (SSD)
 // 92 -> 83; 17 of 480 .. 628, 4 heads of 256 x 512 202 -> 157; single chunks, 23 of 2 .. 25 rows, 8 heads of 128 x 256, 20.4 -> 17.2.
-template <int KD, int NW, int KIND, bool STATES>
-__global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : NW == 4 && KD == 64 && KIND == kSsd ? 3 : 2) void gated_chunk_kernel(const GlArgs a) {
+// WIDE: rows of whole, aligned 16-byte pieces, else of 8-byte ones.  (In one kernel, with a branch, each load of the one kind waited for those of the other,
+// which had never been asked for: q, k and v of a workgroup's first chunk came one after the other.)  The first chunk's gates are asked for
+// ahead of its tiles and made while those are on their way.  At 64 x 64 three workgroups share a compute unit.  Single chunks, 32 heads of 64 x 64, us: branch and
+// two workgroups, WIDE, gates first, three workgroups: mLSTM, 500 of 10 .. 30 rows 235, 200, 191, 152; 130 of 65 .. 128 96, 92, 86, 80.  SSD, which has three
+// anyway, 500 of 10 .. 30 163, 133, 126.
+template <int KD, int NW, int KIND, bool STATES, bool WIDE>
+__global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : NW == 4 && KD == 64 ? 3 : 2) void gated_chunk_kernel(const GlArgs a) {
     constexpr int kCols = 16 * NW, kLdV = kCols + kLaPadV, kThr = 64 * NW;
     constexpr int kKP = 64 * (KD / 8) / kThr, kKRows = kThr / (KD / 8);  // 16-byte pieces of K per thread, rows between them; of V: two
     constexpr int kVRows = kThr / (kCols / 8);
@@ -311,15 +315,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : NW == 4 && KD =
     const uint16_t *uq = reinterpret_cast<const uint16_t *>(a.q) + p.row0 * a.ldq + grp * a.dim;
     const uint16_t *uk = reinterpret_cast<const uint16_t *>(a.k) + p.row0 * a.ldk + grp * a.dim;
     const uint16_t *uv = reinterpret_cast<const uint16_t *>(a.v) + p.row0 * a.ldv + h * a.vdim + v0;
-    const pa_bf16 *ga = reinterpret_cast<const pa_bf16 *>(a.ga) + p.row0 * a.ldg + h;
-    const pa_bf16 *gb = reinterpret_cast<const pa_bf16 *>(a.gb) + p.row0 * a.ldg + h;
+    const uint16_t *ga = reinterpret_cast<const uint16_t *>(a.ga) + p.row0 * a.ldg + h;
+    const uint16_t *gb = reinterpret_cast<const uint16_t *>(a.gb) + p.row0 * a.ldg + h;
     const int vcols = a.vdim - v0 < kCols ? a.vdim - v0 : kCols;
     la_u4 kb[kKP], qb[STATES ? 1 : kKP], vb[2];
     const int kr = tid / (KD / 8), kc = tid % (KD / 8), vr = tid / (kCols / 8), vc = tid % (kCols / 8);  // a thread's first row and piece
     auto fetch_rows = [&](auto &x, const uint16_t *base, int64_t ld, int r0, int row, int piece, int rows_apart, int cols) {
         const int nr = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
         const __amdgpu_buffer_rsrc_t t = la_tile(base + r0 * ld, ld, nr, cols);
-        la_load_pieces(x, t, ld, row, piece * 8, rows_apart, cols, a.wide);
+        la_load_pieces(x, t, ld, row, piece * 8, rows_apart, cols, WIDE);
     };
     auto fetch_q = [&](int r0) { fetch_rows(qb, uq, a.ldq, r0, kr, kc, kKRows, a.dim); };
     auto fetch_k = [&](int r0) { fetch_rows(kb, uk, a.ldk, r0, kr, kc, kKRows, a.dim); };
@@ -337,17 +341,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : NW == 4 && KD =
 #pragma unroll
         for (int i = 0; i < 2; ++i) *reinterpret_cast<la_u4 *>(v_s + (vr + i * kVRows) * kLdV + vc * 8) = vb[i];
     };
-    float raw_a = 0.f, raw_b = 0.f;
+    uint32_t raw_a = 0, raw_b = 0;  // (as they come: a conversion here would wait for all loads before it)
     auto fetch_gates = [&](int r0) {
         if (wave == kGates && lane < r_end - r0) {
-            raw_a = pa_scalar<pa_bf16>::load(ga + (r0 + lane) * a.ldg);
-            if (KIND == kMlstm) raw_b = pa_scalar<pa_bf16>::load(gb + (r0 + lane) * a.ldg);
+            raw_a = ga[(r0 + lane) * a.ldg];
+            if (KIND == kMlstm) raw_b = gb[(r0 + lane) * a.ldg];
         }
     };
     auto gates = [&](int r0, GlRows *to) {  // a chunk's gates, one row per lane
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
         float decay, in;
-        gl_gate<KIND>(a, hd, raw_a, raw_b, decay, in);
+        gl_gate<KIND>(a, hd, __builtin_bit_cast(float, raw_a << 16), __builtin_bit_cast(float, raw_b << 16), decay, in);
         if (lane >= nv) decay = 0.f;
         const float f = gl_scan_add(decay, lane), f_last = gl_lane(f, 63);
         if constexpr (KIND == kSsd) {
@@ -378,10 +382,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && KD == 256 ? 1 : NW == 4 && KD =
         }
         decayed += f_last;
     };
+    fetch_gates(r_beg);  // (first, and its gates are made while the tiles are on their way)
     if (!STATES) fetch_q(r_beg);
     fetch_k(r_beg);
     fetch_v(r_beg);
-    fetch_gates(r_beg);
     if (wave == kGates) gates(r_beg, rows);
     fetch_gates(r_beg + kLaChunk);
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
@@ -719,28 +723,35 @@ template <int KIND> __global__ __launch_bounds__(256) void gated_scan_kernel(con
     }
 }
 
-template <int KD, int NW, int KIND> int launch_chunks(const GlArgs &a, int batch, hipStream_t s) {
+template <int KD, int NW, int KIND, bool WIDE> int launch_chunks(const GlArgs &a, int batch, hipStream_t s) {
     constexpr size_t lds = gl_lds_bytes<KD, NW, KIND, false>(), lds_states = gl_lds_bytes<KD, NW, KIND, true>();
     static_assert(lds <= 160 * 1024 && lds_states <= 160 * 1024, "LDS of one compute unit");
     const int slices = (a.vdim + 16 * NW - 1) / (16 * NW);
     const dim3 grid = la_grid(a.heads, slices, batch, a.segments), block(64 * NW);
     if (a.segments > 1) {
-        if (int rc = la_big_lds(gated_chunk_kernel<KD, NW, KIND, true>, lds_states, "pa_gated_linear")) return rc;
-        gated_chunk_kernel<KD, NW, KIND, true><<<grid, block, lds_states, s>>>(a);
+        if (int rc = la_big_lds(gated_chunk_kernel<KD, NW, KIND, true, WIDE>, lds_states, "pa_gated_linear")) return rc;
+        gated_chunk_kernel<KD, NW, KIND, true, WIDE><<<grid, block, lds_states, s>>>(a);
         const unsigned gx = (unsigned)(((int64_t)a.dp * a.vp / 4 + a.dp / 4 + 255) / 256);
         gated_scan_kernel<KIND><<<dim3(gx, (unsigned)a.heads, (unsigned)batch), dim3(256), 0, s>>>(a);
     }
-    if (int rc = la_big_lds(gated_chunk_kernel<KD, NW, KIND, false>, lds, "pa_gated_linear")) return rc;
-    gated_chunk_kernel<KD, NW, KIND, false><<<grid, block, lds, s>>>(a);
+    if (int rc = la_big_lds(gated_chunk_kernel<KD, NW, KIND, false, WIDE>, lds, "pa_gated_linear")) return rc;
+    gated_chunk_kernel<KD, NW, KIND, false, WIDE><<<grid, block, lds, s>>>(a);
     PA_CHECK_LAUNCH("pa_gated_linear (chunks)");
     return PA_OK;
 }
 
+template <int KIND, bool WIDE> int launch_chunks_of(const GlArgs &a, int batch, hipStream_t s) {
+    const bool many = la_value_cols(a.vdim) == 128;
+    if (a.dim <= 64) return many ? launch_chunks<64, 8, KIND, WIDE>(a, batch, s) : launch_chunks<64, 4, KIND, WIDE>(a, batch, s);
+    if (a.dim <= 128) return many ? launch_chunks<128, 8, KIND, WIDE>(a, batch, s) : launch_chunks<128, 4, KIND, WIDE>(a, batch, s);
+    return many ? launch_chunks<256, 8, KIND, WIDE>(a, batch, s) : launch_chunks<256, 4, KIND, WIDE>(a, batch, s);
+}
+
 template <int KIND> int launch_chunks_kind(const GlArgs &a, int batch, hipStream_t s) {
-    const bool wide = la_value_cols(a.vdim) == 128;
-    if (a.dim <= 64) return wide ? launch_chunks<64, 8, KIND>(a, batch, s) : launch_chunks<64, 4, KIND>(a, batch, s);
-    if (a.dim <= 128) return wide ? launch_chunks<128, 8, KIND>(a, batch, s) : launch_chunks<128, 4, KIND>(a, batch, s);
-    return wide ? launch_chunks<256, 8, KIND>(a, batch, s) : launch_chunks<256, 4, KIND>(a, batch, s);
+    // rows of whole, aligned 16-byte pieces
+    const bool wide = a.dim % 8 == 0 && a.vdim % 8 == 0 && a.ldq % 8 == 0 && a.ldk % 8 == 0 && a.ldv % 8 == 0 &&
+                      (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15u) == 0;
+    return wide ? launch_chunks_of<KIND, true>(a, batch, s) : launch_chunks_of<KIND, false>(a, batch, s);
 }
 
 template <typename T, int KIND> void launch_recurrent(const GlArgs &a, int batch, hipStream_t s) {
@@ -811,8 +822,6 @@ extern "C" int pa_gated_linear(int kind, const void *q, int64_t q_stride, const 
     a.heads = num_heads; a.dim = dim; a.vdim = vdim; a.dp = la_pad16(dim); a.vp = la_pad16(vdim);
     a.head_floats = (int64_t)gl_state_floats(kind == kMlstm, dim, vdim);
     a.segments = 1;
-    a.wide = dim % 8 == 0 && vdim % 8 == 0 && q_stride % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 &&
-             (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
     hipStream_t s = (hipStream_t)stream;
     // single rows, 32-bit rows, rows that are not whole 8-byte vectors, rows too far apart for 32-bit offsets
     const uintptr_t at = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out;
