@@ -1,6 +1,7 @@
 // Row kernels between the matrix products of a decoder block: the 32-bit residual sum fused with the norm that
 // reads it, gated activations, and the gates behind attention and recurrent layers.  HBM-bound; a row lives in
 // registers, every tensor is read once and written once.
+#include <type_traits>
 #include "row_common.h"
 
 namespace {
@@ -32,6 +33,9 @@ struct ResidualArgs {
     int width, norm;
     float y_eps, eps;
 };
+
+// Bytes that a sum of parts moves, parts, residual and output, from which on the parts are read past the caches (of which the largest has 256 MB)
+constexpr int64_t kMixLarge = 320000000;
 
 template <typename T, int TPR, int V, int NV>
 __global__ __launch_bounds__(256) void residual_norm_kernel(const ResidualArgs a) {
@@ -95,31 +99,44 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(const ResidualArgs a
             const float *w = a.mix_w + row * (a.mix + 1);
 #pragma unroll
             for (int i = 0; i < NV; ++i) row_zero<V>(y[i]);
-            // kAtOnce parts' loads are on their way at once (places past the row's or the parts' end: the last ones, which do not count); rows of
-            // more than 16 elements a thread have no registers for that.  Memory-bound: 6001 rows of 4096 with 9 parts, 690 MB, 165 us part
-            // by part, 138 two at once, 131 four, 119 (5.8 TB/s) read past the caches, which the parts leave at once.
-            constexpr int kAtOnce = NV * V > 16 ? 1 : 4;
+            // kAtOnce parts' loads are on their way at once (places past the row's end: its last ones, which do not count).  Rows of more than 16 elements
+            // a thread have no registers for that, and 32-bit parts are no faster for it.  Memory-bound: 6001 rows of 4096 with 9 parts, 690 MB, 165 us part
+            // by part, 138 two at once, 131 four, 114 (6.0 TB/s) read past the caches.  Below kMixLarge parts that were just written are found in
+            // the caches.  us behind a kernel that writes the parts; part by part, four at once past the caches, four at once: 3000 rows of 2048 with 11 parts
+            // 36.6, 38.9, 33.3; 1500 of 4096 with 9 38.7, 34.8, 30.0; above it 6000 of 2048 with 9 64, 59, 58, of 4096 with 5 117, 80, 100.  32 bits, part
+            // by part, the same past the caches: 1500 of 4096 with 6 37, 46, 3000 112, 70.
+            constexpr bool kLong = NV * V > 16;
+            constexpr int kAtOnce = kLong || sizeof(T) == 4 ? 1 : 4;
             const int parts = a.mix + (a.y_extra ? 1 : 0);
-            for (int m0 = 0; m0 < parts; m0 += kAtOnce) {
-                float t[kAtOnce][NV][V], f[kAtOnce];
+            auto every = [&](auto once) {
+                for (int m0 = 0; m0 < parts; m0 += kAtOnce) {
+                    float t[kAtOnce][NV][V], f[kAtOnce];
 #pragma unroll
-                for (int p = 0; p < kAtOnce; ++p) {
-                    const int m = min(m0 + p, parts - 1);
-                    const T *src = m < a.mix ? reinterpret_cast<const T *>(a.y) + (row * a.mix + m) * a.width
-                                             : reinterpret_cast<const T *>(a.y_extra) + row * a.width;
-                    f[p] = w[m];
+                    for (int p = 0; p < kAtOnce; ++p) {
+                        const int m = m0 + p;
+                        if (p > 0 && m >= parts) break;
+                        const T *src = m < a.mix ? reinterpret_cast<const T *>(a.y) + (row * a.mix + m) * a.width
+                                                 : reinterpret_cast<const T *>(a.y_extra) + row * a.width;
+                        f[p] = w[m];
 #pragma unroll
-                    for (int i = 0; i < NV; ++i) row_load_once<T, V>(src + min((i * TPR + lane) * V, a.width - V), t[p][i]);
+                        for (int i = 0; i < NV; ++i) {
+                            const T *at = src + min((i * TPR + lane) * V, a.width - V);
+                            if constexpr (decltype(once)::value) row_load_once<T, V>(at, t[p][i]);
+                            else row_load<T, V>(at, t[p][i]);
+                        }
+                    }
+#pragma unroll
+                    for (int p = 0; p < kAtOnce; ++p) {
+                        if (p > 0 && m0 + p >= parts) break;
+#pragma unroll
+                        for (int i = 0; i < NV; ++i)
+#pragma unroll
+                            for (int j = 0; j < V; ++j) y[i][j] = (i * TPR + lane) * V < a.width ? fmaf(f[p], t[p][i][j], y[i][j]) : 0.f;
+                    }
                 }
-#pragma unroll
-                for (int p = 0; p < kAtOnce; ++p) {
-                    if (m0 + p >= parts) break;
-#pragma unroll
-                    for (int i = 0; i < NV; ++i)
-#pragma unroll
-                        for (int j = 0; j < V; ++j) y[i][j] = (i * TPR + lane) * V < a.width ? fmaf(f[p], t[p][i][j], y[i][j]) : 0.f;
-                }
-            }
+            };
+            if (kLong || a.rows * a.width * (8 + (int64_t)sizeof(T) * (parts + 1)) >= kMixLarge) every(std::true_type());
+            else every(std::false_type());
         } else {
             const T *src = reinterpret_cast<const T *>(a.y) + row * a.width;
 #pragma unroll

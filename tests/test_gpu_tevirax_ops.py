@@ -89,6 +89,28 @@ def test_weighted_branches_of_many_parts(parts, with_extra, width, dtype):
     assert bool(((x.cpu().double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("rows,parts,with_extra,width,dtype", [(2800, 8, True, 4096, BF), (7200, 5, True, 2048, BF), (14000, 7, False, 1028, BF), (2800, 1, True, 8196, BF),
+                                                               (5700, 4, False, 2048, F32)])
+def test_weighted_branches_read_past_the_caches(rows, parts, with_extra, width, dtype):
+    """Calls that move more than the caches hold read their parts past them: the same sums, to the bit, as a few rows at a time."""
+    announce(f"large mix of {parts} parts {rows} x {width} {dtype}")
+    assert rows * width * (8 + (parts + with_extra + 1) * torch.empty(0, dtype=dtype).element_size()) >= 320_000_000
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=DEV)
+    x0, y, extra, mix = rand(rows, width), rand(rows * parts, width).to(dtype), rand(rows, width).to(dtype), rand(rows, parts + 1)
+
+    def run(lo, hi):
+        x = x0[lo:hi].clone()
+        out = ops.residual_norm(x, dtype, y=y[lo * parts: hi * parts], mix=mix[lo:hi], y_extra=extra[lo:hi] if with_extra else None, norm="rms", weight=torch.ones(width, device=DEV))
+        return x, out
+
+    x, out = run(0, rows)
+    for lo in range(0, rows, 512):
+        hi = min(lo + 512, rows)
+        few, few_out = run(lo, hi)
+        assert torch.equal(x[lo:hi], few) and torch.equal(out[lo:hi], few_out), lo
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("groups,per", [(1, 48), (3, 24), (5, 14), (4, 72), (2, 200), (8, 128), (2, 2048), (3, 33)])
 def test_gated_norms_of_groups(groups, per, dtype):
