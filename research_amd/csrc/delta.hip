@@ -439,13 +439,13 @@ template <int KD, int NW> __global__ __launch_bounds__(64 * NW, KD == 64 && NW =
         for (int i = 0; i < kKB; ++i) {
             const int blk = lt + kThr * i, r = blk / (KD / 4) * 4, c = blk % (KD / 4) * 4;
             if (!k_live) continue;
-            la_put_paired<false, KD>(kb[i], r, c, k_s);
-            la_put_paired<false, KD>(qb[i], r, c, q_s);
+            la_put_paired<KD>(kb[i], r, c, k_s);
+            la_put_paired<KD>(qb[i], r, c, q_s);
         }
 #pragma unroll
         for (int i = 0; i < kVB; ++i) {
             const int blk = lt + kThr * i, r = blk / (kCols / 4) * 4, c = blk % (kCols / 4) * 4;
-            la_put_block<false>(vb[i], r, c, v_s, kLv);
+            la_put_block(vb[i], r, c, v_s, kLv);
         }
         if (lt < 64) {
             rows[lt] = row_g0;

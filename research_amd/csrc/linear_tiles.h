@@ -104,20 +104,12 @@ __device__ __forceinline__ uint32_t la_silu2(uint32_t w) {
                          row_silu<pa_bf16>(__builtin_bit_cast(float, w & 0xffff0000u)));
 }
 
-template <bool ACT> __device__ __forceinline__ void la_act_block(LaBlock &b) {
-    if constexpr (ACT) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) b.r[i] = make_uint2(la_silu2(b.r[i].x), la_silu2(b.r[i].y));
-    }
-}
-// The block, or with ACT its silu, to a row-major tile, and to a paired one
-template <bool ACT> __device__ __forceinline__ void la_put_block(LaBlock b, int s, int c, __bf16 *rm, int ld_rm) {
-    la_act_block<ACT>(b);
+// The block to a row-major tile, and to a paired one
+__device__ __forceinline__ void la_put_block(const LaBlock &b, int s, int c, __bf16 *rm, int ld_rm) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(rm + (s + i) * ld_rm + c) = b.r[i];
 }
-template <bool ACT, int KD> __device__ __forceinline__ void la_put_paired(LaBlock b, int r, int c, __bf16 *tile) {
-    la_act_block<ACT>(b);
+template <int KD> __device__ __forceinline__ void la_put_paired(const LaBlock &b, int r, int c, __bf16 *tile) {
     const int e = la_paired(c);
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(tile + (r + i) * KD + (((e >> 3) ^ la_hash<KD>(r + i)) << 3) + (e & 4)) = b.r[i];
