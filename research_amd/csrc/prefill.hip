@@ -33,7 +33,7 @@ int prefill_cus() {
 // (1 to 64 prompts behind up to 8192 keys) the rule's pieces took 1.02 of the time of each one's best.
 int prefill_splits(int num_kv_heads, int64_t groups, int batch, int64_t rows, int n_rep, int tasks, int head_dim, int64_t max_keys) {
     return plan_prefill_splits(plan_prefill_units(num_kv_heads, groups, batch, rows, n_rep, kPfRows, tasks), prefill_cus(), max_keys,
-                               head_dim > 128 ? kWdKeys : kPfKeys, kPlanShortPieceTiles, rows * num_kv_heads * n_rep * (head_dim + 2) * 4);
+                               head_dim > 128 ? kWdKeys : kPfKeys, rows * num_kv_heads * n_rep * (head_dim + 2) * 4);
 }
 size_t prefill_ws_bytes(int64_t total_q, int num_q_heads, int head_dim, int splits) {
     return plan_prefill_ws_bytes(total_q, num_q_heads, head_dim, splits);

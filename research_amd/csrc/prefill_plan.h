@@ -11,8 +11,7 @@
 namespace pa_decode_detail {
 
 constexpr int kPlanMaxPrefillSplits = 8;
-constexpr int kPlanMinTilesPerSplit = 24;  // a piece's set-up and write-out cost about six tiles of its loop
-constexpr int kPlanShortPieceTiles = 8;    // the same where the merge is priced as well
+constexpr int kPlanMinTilesPerSplit = 8;   // of a piece, whose set-up and write-out cost about six
 constexpr int kPlanPieceFixedTiles = 6;    // set-up and write-out of a workgroup, in tiles of its loop
 constexpr int kPlanMergeTiles = 9;         // the merge launch, in the same unit (a tile takes about a microsecond)
 constexpr int64_t kPlanMergeBytesPerTile = 4500000;  // and what it and the pieces move meanwhile
@@ -28,16 +27,15 @@ PA_PLAN_FN int64_t plan_prefill_cost(int64_t workgroups, int cus, int64_t tiles,
 // Pieces to cut every workgroup's tiles into, from shapes alone.  The matrix-core kernels run one workgroup per
 // compute unit, each owning 256 (head_dim 256: 128) row-head pairs and all their keys, so a launch of few rows
 // leaves compute units idle however long the context is.  The split with the lowest cost wins (the smaller on
-// ties), as long as a piece keeps min_tiles tiles of the longest context the block tables can describe.  Given the bytes of a piece's
-// partial results the cost has the merge in it, and pieces may be short.
-PA_PLAN_FN int plan_prefill_splits(int64_t workgroups, int cus, int64_t max_keys, int tile_keys, int min_tiles = kPlanMinTilesPerSplit,
-                                   int64_t part_bytes = 0) {
+// ties), as long as a piece keeps kPlanMinTilesPerSplit tiles of the longest context the block tables can describe.  The cost has the merge in
+// it, part_bytes of partial results for each piece.
+PA_PLAN_FN int plan_prefill_splits(int64_t workgroups, int cus, int64_t max_keys, int tile_keys, int64_t part_bytes) {
     const int64_t tiles = max_keys / tile_keys;
     int best = 1;
     int64_t best_cost = 0;
     for (int s = 1; s <= kPlanMaxPrefillSplits; ++s) {
-        if (s > 1 && tiles / s < min_tiles) break;
-        const int64_t merge = s > 1 && part_bytes > 0 ? kPlanMergeTiles + 2 * s * part_bytes / kPlanMergeBytesPerTile : 0;
+        if (s > 1 && tiles / s < kPlanMinTilesPerSplit) break;
+        const int64_t merge = s > 1 ? kPlanMergeTiles + 2 * s * part_bytes / kPlanMergeBytesPerTile : 0;
         const int64_t cost = plan_prefill_cost(workgroups, cus, tiles, s) + merge;
         if (s == 1 || cost < best_cost) {
             best_cost = cost;
@@ -64,7 +62,8 @@ PA_PLAN_FN int64_t plan_prefill_units(int num_kv_heads, int64_t groups, int batc
 // without rows).  us, by places -> by number, rounds of 256 places and of chunks: 8 / 2 heads of 128, 29 prompts of 133 .. 319 rows behind
 // 4080 keys (1.1, 0.8) 191 -> 115; 32 / 8 of 128, 13 of 75 .. 158 behind 1504 (1.2, 1.0) 88 -> 57, 48 of 99 .. 145 behind 1008 (4.5, 3.7) 172 -> 150;
 // 14 / 2 of 128, 13 of 385 .. 962 behind 1104 (2.5, 1.8) 118 -> 96, but 47 of 36 .. 218 behind 720 (2.6, 1.4) 58 -> 60; 32 / 8 of 128, 32 of 97 .. 249
-// behind 2048 (4.0, 3.2) 225 -> 234.
+// behind 2048 (4.0, 3.2) 225 -> 234.  Over 311 batches (1 to 64 prompts of up to 8192 rows behind nothing or up to 8192 keys, and one of 200 000; head sizes
+// 64 to 256) the rule takes 0.99 of the time of numbering by places, 0.56 at best, and is never slower by more than 3.5 %.
 PA_PLAN_FN bool plan_prefill_dense(int64_t units, int64_t places, int cus) {
     const int64_t rounds = (units + cus - 1) / cus;
     return rounds < (places + cus - 1) / cus && 8 * (units - (rounds - 1) * cus) >= 5 * cus;

@@ -59,14 +59,15 @@ extern "C" int pa_plan_groups(int group_end, int n_chunks, int limit, int *most,
     return 0;
 }
 
-extern "C" int pa_plan_splits(long long workgroups, int cus, long long max_keys, int tile_keys) {
-    return plan_prefill_splits(workgroups, cus, max_keys, tile_keys);
-}
-extern "C" int pa_plan_splits_merged(long long workgroups, int cus, long long max_keys, int tile_keys, long long part_bytes) {
-    return plan_prefill_splits(workgroups, cus, max_keys, tile_keys, kPlanShortPieceTiles, part_bytes);
+extern "C" int pa_plan_splits(long long workgroups, int cus, long long max_keys, int tile_keys, long long part_bytes) {
+    return plan_prefill_splits(workgroups, cus, max_keys, tile_keys, part_bytes);
 }
 extern "C" long long pa_plan_units(int num_kv_heads, long long groups, int batch, long long rows, int n_rep, int rows_per_task, int tasks) {
     return plan_prefill_units(num_kv_heads, groups, batch, rows, n_rep, rows_per_task, tasks);
+}
+extern "C" int pa_plan_ragged_groups(int most, long long groups, int num_kv_heads, int batch, long long rows, long long max_q_len, long long rows_per_group,
+                                     long long max_keys, int tile_keys, int cus) {
+    return plan_ragged_groups(most, groups, num_kv_heads, batch, rows, max_q_len, rows_per_group, max_keys, tile_keys, cus);
 }
 extern "C" int pa_plan_dense(long long units, long long places, int cus) { return plan_prefill_dense(units, places, cus); }
 extern "C" long long pa_plan_cost(long long workgroups, int cus, long long tiles, int s) {

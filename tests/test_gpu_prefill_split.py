@@ -15,6 +15,7 @@ import torch
 from oracle import paged_oracle as po
 from research_amd import _lib, ops
 from tests.gpu_helpers import DEV, announce, assert_close
+from tests.test_prefill_plan import NUMBERED, unequal_prompts
 
 pytestmark = pytest.mark.gpu
 
@@ -123,23 +124,23 @@ def test_many_prompts_of_unequal_length_in_pieces(d, hq, hkv, n):
         assert not got[b, rows:].any()
 
 
-@pytest.mark.parametrize("d,hq,hkv,n,most,dtype", [(128, 7, 1, 110, 130, torch.bfloat16), (64, 8, 2, 66, 260, torch.float16),
-                                                   (256, 6, 3, 70, 80, torch.bfloat16), (128, 8, 2, 12, 1200, torch.bfloat16)])
-def test_unequal_prompts_numbered_by_rows(d, hq, hkv, n, most, dtype):
-    """Launches whose grid has places for more than a round while the groups with rows fill about one: sequences without rows, more than 64 of
-    them, and workgroups of several groups (the last case's prompts also without the number of rows, which numbers by places)."""
+@pytest.mark.parametrize("d,hq,hkv,n,most,gpw", NUMBERED)
+def test_unequal_prompts_numbered_by_rows(d, hq, hkv, n, most, gpw):
+    """Launches whose grid has places for more than a round while the groups with rows fill about one (test_prefill_plan.py: these are numbered by
+    rows, and a call without the number of rows by places): the same results, to the bit."""
     announce(f"prefill numbered by rows: {n} prompts, {hq} / {hkv} heads of {d}")
-    rng = np.random.default_rng(n)
-    chunk = rng.integers(0, most // 2 + 1, size=n)
-    chunk[[1, n // 2, n - 1]] = most, 0, most
-    prefix = rng.integers(most, 2 * most, size=n)
-    c = Case([int(x) for x in prefix], [int(x) for x in chunk], hq, hkv, d, dtype=dtype, seed=n, width=1)
-    rows = [int(x) for x in chunk]
+    dtype = torch.float16 if d == 64 else torch.bfloat16
+    rows, prefix = unequal_prompts(n, most)
+    c = Case(prefix, rows, hq, hkv, d, dtype=dtype, seed=n, width=1)
     starts = np.concatenate([[0], np.cumsum(rows)[:-1]])
     q = torch.cat([c.q[b, :r] for b, r in enumerate(rows)]).to(DEV)
-    got = ops.prefill_paged(q, c.k.to(DEV), c.v.to(DEV), c.dev_tables, _i32(c.ctx), _i32(rows), _i32(starts), most, 16, c.scale).cpu()
-    assert torch.equal(got, torch.cat([x[:r] for x, r in zip(c.run().cpu(), rows)]))  # (run: rows of equal prompts, numbered by places)
-    want = c.want()
+    k, v, ctx, lens, at = c.k.to(DEV), c.v.to(DEV), _i32(c.ctx), _i32(rows), _i32(starts)
+    got = ops.prefill_paged(q, k, v, c.dev_tables, ctx, lens, at, most, 16, c.scale)
+    places = torch.zeros_like(q)
+    ops._run("pa_prefill_paged", q, k, v, places, c.dev_tables, c.dev_tables.shape[1], ctx, lens, at, None, n, most, hq, hkv, d, 16, k.shape[0] // 16, c.scale, 0,
+             ops.PA_DTYPE[dtype], ops._stream(q))
+    assert torch.equal(got, places)
+    want, got = c.want(), got.cpu()
     for b, r in enumerate(rows):
         if r:
             assert_close(got[starts[b]: starts[b] + r], want[b, :r], 2e-2, f"sequence {b} vs oracle")

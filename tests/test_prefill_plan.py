@@ -22,8 +22,8 @@ def plan(tmp_path_factory):
     dll = ctypes.CDLL(lib)
     dll.pa_plan_pieces.argtypes = [ctypes.c_int] * 3 + [ctypes.c_char_p, ctypes.c_int]
     dll.pa_plan_groups.argtypes = [ctypes.c_int] * 3 + [ctypes.POINTER(ctypes.c_int), ctypes.c_char_p, ctypes.c_int]
-    dll.pa_plan_splits.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int]
-    dll.pa_plan_splits_merged.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong]
+    dll.pa_plan_splits.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong]
+    dll.pa_plan_ragged_groups.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_int] + [ctypes.c_longlong] * 4 + [ctypes.c_int] * 2
     dll.pa_plan_units.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_int, ctypes.c_longlong] + [ctypes.c_int] * 3
     dll.pa_plan_units.restype = ctypes.c_longlong
     dll.pa_plan_dense.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_int]
@@ -75,28 +75,83 @@ def test_zigzag_order_balances_causal_work(plan):
     assert max(straight) - min(straight) == gpw * (n_chunks - 1)
 
 
+class Launch:
+    """What a launch of the kernels with the assembly loop is planned as on 256 compute units (``prefill_launch`` of ``prefill.hip``).
+    ``rows``: of q, all prompts' (0: not known); ``keys``: that the block tables can describe."""
+
+    def __init__(self, plan, hq, hkv, d, batch, most, rows, keys):
+        self.plan, self.hkv, self.batch, self.rows, self.keys, self.n_rep = plan, hkv, batch, rows, keys, hq // hkv
+        self.tasks, self.tile = (4, 32) if d > 128 else (8, 64)
+        self.groups = -(-(-(-most // 32) * self.n_rep) // self.tasks)
+        self.part_bytes = rows * hq * ((256 if d > 128 else 128 if d > 64 else 64 if d > 32 else 32) + 2) * 4
+        self.gpw = 1
+        if d <= 128:
+            equal = plan.pa_plan_groups_per_workgroup(hkv, self.groups, batch, 256)
+            self.gpw = plan.pa_plan_ragged_groups(equal, self.groups, hkv, batch, rows, most, 256 // self.n_rep, keys, 64, 256)
+
+    def units(self, gpw=1):
+        return self.plan.pa_plan_units(self.hkv, -(-self.groups // gpw), self.batch, self.rows, self.n_rep, 32, self.tasks * gpw)
+
+    def splits(self):
+        return self.plan.pa_plan_splits(self.units(), 256, self.keys, self.tile, self.part_bytes)
+
+    def dense(self):
+        return self.rows > 0 and bool(self.plan.pa_plan_dense(self.units(self.gpw), self.hkv * -(-self.groups // self.gpw) * self.batch, 256))
+
+
+def unequal_prompts(n, most):
+    """Rows of ``n`` prompts and the tokens before them: two have ``most`` rows, one has none, the others up to half as many."""
+    rng = np.random.default_rng(n)
+    chunk = rng.integers(0, most // 2 + 1, size=n)
+    chunk[[1, n // 2, n - 1]] = most, 0, most
+    return [int(x) for x in chunk], [int(x) for x in rng.integers(most, 2 * most, size=n)]
+
+
+# (head size, query heads, kv heads, prompts, the longest's rows, groups of a workgroup): launches whose workgroups are numbered by the chunks that have
+# rows (test_gpu_prefill_split.py runs them): more than 64 sequences, and workgroups of one group and of two
+NUMBERED = [(128, 8, 2, 110, 130, 2), (64, 8, 2, 66, 260, 1), (256, 6, 3, 70, 80, 1), (128, 8, 2, 12, 1200, 1), (128, 12, 2, 110, 80, 2), (32, 8, 4, 40, 260, 2)]
+
+
+@pytest.mark.parametrize("d,hq,hkv,n,most,gpw", NUMBERED)
+def test_which_unequal_prompts_are_numbered_by_rows(plan, d, hq, hkv, n, most, gpw):
+    chunk, prefix = unequal_prompts(n, most)
+    keys = -(-max(c + p for c, p in zip(chunk, prefix)) // 16) * 16
+    at = Launch(plan, hq, hkv, d, n, most, sum(chunk), keys)
+    assert at.dense() and at.gpw == gpw
+    assert not Launch(plan, hq, hkv, d, n, most, 0, keys).dense()  # (a call that does not know how many rows)
+
+
 @pytest.mark.parametrize("cus", [256, 304, 64])
 def test_split_rule_is_the_cheapest_admissible_split(plan, cus):
     rng = np.random.default_rng(cus)
-    for _ in range(400):
+    for i in range(800):
         workgroups = int(rng.integers(1, 4 * cus))
-        max_keys = int(rng.integers(64, 400000))
-        s = plan.pa_plan_splits(workgroups, cus, max_keys, 64)
+        max_keys = int(rng.integers(64, 400000 if i % 2 else 12800))
+        part = int(rng.integers(0, 1 << 25))
+        s = plan.pa_plan_splits(workgroups, cus, max_keys, 64, part)
         tiles = max_keys // 64
         assert 1 <= s <= 8
         if s > 1:
-            assert tiles // s >= 24  # a piece keeps enough tiles to pay for its set-up
-        cost = lambda k: plan.pa_plan_cost(workgroups, cus, tiles, k)
-        admissible = [k for k in range(1, 9) if k == 1 or tiles // k >= 24]
+            assert tiles // s >= 8  # a piece keeps enough tiles to pay for its set-up
+        cost = lambda k: plan.pa_plan_cost(workgroups, cus, tiles, k) + (9 + 2 * k * part // 4500000 if k > 1 else 0)  # (and the merge)
+        admissible = [k for k in range(1, 9) if k == 1 or tiles // k >= 8]
         # (the rule stops at the first split that is too fine, so the admissible ones are 1 .. some k)
         assert admissible == list(range(1, len(admissible) + 1))
         assert cost(s) == min(cost(k) for k in admissible)
         assert all(cost(k) > cost(s) for k in admissible if k < s)  # the smaller on ties
-    # launches that fill the device several times over stay whole; the long-context shapes of bench.py split
-    assert plan.pa_plan_splits(64 * cus, cus, 1 << 20, 64) == 1
-    assert plan.pa_plan_splits(64, 256, 202048 + 256, 64) == 4      # long-d128: 64 workgroups on 256 compute units
-    assert plan.pa_plan_splits(128, 256, 202048 + 256, 64) == 2     # long-d256
-    assert plan.pa_plan_splits(512, 256, 2304, 64) == 1             # c3
+    # launches that fill the device several times over stay whole
+    assert plan.pa_plan_splits(64 * cus, cus, 1 << 20, 64, 64 * cus * 133120) == 1
+
+
+def test_launches_and_their_pieces(plan):
+    splits = lambda *a: Launch(plan, *a).splits()
+    # the long-context shapes of bench.py, whose 64 and 128 workgroups leave compute units idle, and its batch of 32, which does not
+    assert splits(8, 2, 128, 1, 2048, 2048, 202048) == 4
+    assert splits(8, 2, 256, 1, 2048, 2048, 202048) == 2
+    assert splits(32, 8, 128, 32, 256, 32 * 256, 2304) == 1 and splits(32, 8, 256, 32, 256, 32 * 256, 2304) == 1
+    assert splits(8, 2, 128, 1, 150, 150, 1024) == 1       # 16 tiles: the merge costs what half of them do
+    assert splits(8, 2, 128, 7, 248, 7 * 248, 4184) == 4   # few rows behind a long prefix: 56 workgroups
+    assert splits(32, 8, 128, 64, 256, 64 * 256, 16384) == 1
 
 
 @pytest.mark.parametrize("tasks", [8, 4])
@@ -115,19 +170,6 @@ def test_units_are_about_the_groups_with_rows(plan, tasks):
         # (what a sequence's last task and last group lack lies between nothing and twice what is counted for them; floors and ceilings: 2)
         step = next(x for x in (8, 4, 2, 1) if x <= tasks and n_rep % x == 0)
         assert abs(got // hkv - real) <= batch * (n_rep + tasks - step) / (2 * tasks) + batch / 16 + 2
-
-
-def test_short_pieces_pay_for_their_merge(plan):
-    cost = lambda w, tiles, s, part: plan.pa_plan_cost(w, 256, tiles, s) + (9 + 2 * s * part // 4500000 if s > 1 else 0)
-    rng = np.random.default_rng(1)
-    for _ in range(400):
-        w, tiles, part = int(rng.integers(1, 1000)), int(rng.integers(1, 200)), int(rng.integers(1, 1 << 25))
-        s = plan.pa_plan_splits_merged(w, 256, tiles * 64, 64, part)
-        admissible = [k for k in range(1, 9) if k == 1 or tiles // k >= 8]
-        assert s in admissible and cost(w, tiles, s, part) == min(cost(w, tiles, k, part) for k in admissible)
-    assert plan.pa_plan_splits_merged(6, 256, 1024, 64, 150 * 8 * 130 * 4) == 1   # 16 tiles: the merge costs what half of them do
-    assert plan.pa_plan_splits_merged(14, 256, 4032, 64, 248 * 8 * 130 * 4) > 4   # few rows behind a long prefix
-    assert plan.pa_plan_splits_merged(2048, 256, 16384, 64, 64 * 256 * 32 * 130 * 4) == 1  # a launch that fills the device
 
 
 def test_workgroups_are_numbered_by_rows_where_that_is_a_round_less(plan):
