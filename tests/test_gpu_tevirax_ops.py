@@ -536,6 +536,75 @@ def test_whole_calls_are_the_wrappers(monkeypatch, rows, identity, shared):
         assert torch.equal(got[i], want[i]), i
 
 
+def _both_ways(monkeypatch, calls, call):
+    """Results of ``call()`` by the native form of its wrapper, ``calls`` times, and by the wrapper's own way."""
+    with monkeypatch.context() as m:
+        taken, whole = [], ops._whole
+        m.setattr(ops, "_whole", lambda *a: taken.append(whole(*a)) or taken[-1])
+        got = call()
+        assert taken == [0] * calls
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_whole", lambda *a: None)
+        return got, call()
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("kind", ["ssd", "mlstm", "delta", "channel", "lightning"])
+def test_whole_recurrences_are_the_wrappers(monkeypatch, kind, dtype):
+    """Prompts, with a workspace and without, and tokens behind them, from column slices of rows that hold something else between: each argument
+    differs from its neighbours of the same type, so that none could stand for another."""
+    announce(f"whole recurrences {kind} {dtype}")
+    heads, per, dim, vdim, lens, slots = 6, 1 if kind in ("mlstm", "channel", "lightning") else 2, 72, 40, [70, 700, 3], [4, 0, 2]
+    rows, most = sum(lens), max(lens)
+    starts = np.cumsum([0] + lens[:-1])
+    i32 = lambda x: torch.tensor([int(i) for i in x], dtype=torch.int32, device=DEV)
+    prompts = ops.Portions(i32(lens), i32(slots), i32(lens), i32(starts), None, most)
+    tokens = ops.Portions(i32(n + 1 for n in lens), i32(slots))
+    wide = heads // per * dim
+    cols = {"q": wide, "k": wide, "v": heads * vdim, "a": heads, "b": heads}
+    if kind == "lightning":  # (its q, k and v lie side by side)
+        parts = {"u": _rand(rows, 2 * wide + heads * vdim + 24, dtype=dtype).to(DEV)[:, : 2 * wide + heads * vdim + 8]}
+    else:
+        parts = {n: _rand(rows, w + 8 * (1 + i // 3), dtype=dtype, seed=i).to(DEV)[:, :w] for i, (n, w) in enumerate(cols.items())}
+        parts["k"] = _rand(rows, wide + 24, dtype=dtype, seed=9).to(DEV)[:, 8: 8 + wide]
+    c = [_rand(heads, seed=20 + i).to(DEV) for i in range(3)]
+    rate = c[1].abs() + 0.5
+    c_wide = [_rand(wide, seed=30).to(DEV), torch.rand(wide, generator=torch.Generator().manual_seed(31)).to(DEV)]
+    powers = (torch.tensor([0.9, 0.5, 0.99, 0.999, 0.7, 0.95], dtype=torch.float64)[:, None] ** torch.arange(65, dtype=torch.float64)).float().to(DEV)
+    of = {"ssd": "gated", "mlstm": "gated", "delta": "delta", "channel": "channel", "lightning": "lightning"}[kind]
+    shape = (6, heads, ops.gated_linear_state_floats(kind, dim, vdim)) if of == "gated" else (6, heads, 80, 48)
+
+    def one(portions, n, state, ws):
+        out = torch.full((n, heads * vdim), float("nan"), dtype=dtype, device=DEV)
+        p = {name: x[:n] for name, x in parts.items()}
+        if kind == "ssd":
+            ops.gated_linear("ssd", p["q"], p["k"], p["v"], (p["a"], None), (c[0], rate, c[2]), portions, state, heads, dim, vdim, out, heads_per_group=per, workspace=ws)
+        elif kind == "mlstm":
+            ops.gated_linear("mlstm", p["q"], p["k"], p["v"], (p["a"], p["b"]), (c[0], c[1], None), portions, state, heads, dim, vdim, out, cap=15.0, q_scale=0.125,
+                             den_eps=1e-6, workspace=ws)
+        elif kind == "delta":
+            ops.delta_rule(p["q"], p["k"], p["v"], p["a"], p["b"], c[0], rate, portions, state, heads, dim, vdim, 0.125, out, heads_per_group=per, workspace=ws)
+        elif kind == "channel":
+            ops.channel_linear(p["q"], p["k"], p["v"], c_wide[0], c_wide[1], portions, state, heads, dim, vdim, out, q_act="silu", workspace=ws)
+        else:
+            ops.lightning(p["u"], portions, state, powers, heads, dim, vdim, out, workspace=ws)
+        return out
+
+    need = {"gated": ops.gated_linear_workspace_bytes, "delta": ops.delta_workspace_bytes, "channel": ops.channel_linear_workspace_bytes,
+            "lightning": ops.lightning_workspace_bytes}[of](3, heads, dim, vdim, most)
+
+    def call():
+        results = []
+        for ws in (torch.zeros(need, dtype=torch.uint8, device=DEV), None):
+            state = torch.full(shape, 3.0, device=DEV)
+            results += [one(prompts, rows, state, ws), one(tokens, 3, state, None), state]
+        return results
+
+    got, want = _both_ways(monkeypatch, 4, call)
+    for a, b in zip(got, want):
+        assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("rows,experts,top,groups,keep,shared", [(1, 6, 2, 3, 2, True), (37, 8, 3, 2, 1, False), (130, 5, 4, 1, 1, True), (64, 256, 8, 8, 4, True),
                                                                 (9, 100, 20, 100, 40, False), (2000, 16, 4, 4, 2, True), (3, 1, 1, 1, 1, False),
                                                                 (50, 1000, 10, 20, 5, True), (5000, 120, 6, 12, 12, True)])
