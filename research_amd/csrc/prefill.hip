@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part_o,
     float den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < M; ++s) {
-        if (s >= splits || !(ml[s].y > 0.f)) continue;  // a piece in which the row saw no key wrote no O row
+        if (s >= splits || ml[s].y == 0.f) continue;  // a piece in which the row saw no key wrote no O row (a sum that is no number stays one)
         const float w = __builtin_amdgcn_exp2f(ml[s].x - m_all);
         den = fmaf(w, ml[s].y, den);
         num[0] = fmaf(w, o[s].x, num[0]);

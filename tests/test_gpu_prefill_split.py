@@ -161,6 +161,28 @@ def test_one_and_several_groups_of_a_workgroup(d, hq, hkv, n, rows):
     assert_close(every[:1], want, 2e-2, "first sequence vs oracle")
 
 
+@pytest.mark.parametrize("what,bad", [("k", float("nan")), ("k", float("inf")), ("v", float("nan")), ("v", float("inf"))])
+@pytest.mark.parametrize("d,hq,hkv", [(128, 8, 2), (64, 4, 1), (256, 4, 2)])
+def test_a_key_or_value_that_is_no_number_in_pieces(d, hq, hkv, what, bad):
+    """Its rows are no numbers where they are none in one piece: not the sum of the other pieces' keys.  Heads that do not read it are not touched."""
+    announce(f"split prefill: {what} = {bad}, {hq} / {hkv} heads of {d}")
+    c = Case([1500], [100], hq, hkv, d, seed=d)
+    clean = c.run(4)
+    for key in (70, 900, 1540):  # of the prefix, and one that only later rows see
+        x = getattr(c, what)
+        slot = c.tables[0][key // 16] * 16 + key % 16
+        kept = x[slot, 0, 5].clone()
+        x[slot, 0, 5] = bad
+        one, got = torch.isfinite(c.run().float()), c.run(4)
+        x[slot, 0, 5] = kept
+        assert torch.equal(torch.isfinite(got.float()), one) and not bool(one.all()), key
+        assert torch.equal(got[:, :, hq // hkv:], clean[:, :, hq // hkv:])
+        unseen, before = got[:, : max(0, key - 1500)], clean[:, : max(0, key - 1500)]
+        finite = torch.isfinite(unseen.float())
+        if key > 1500:
+            assert_close(unseen[finite], before[finite], 6e-3, f"rows before key {key}")
+
+
 def test_windows_first_keys_and_absent_blocks_in_pieces():
     announce("split prefill: window, per-row first keys, absent blocks")
     # (under a window a workgroup sees window + 256 keys at most: the library splits only wide windows)
