@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64) void scored_merge_kernel(const ScoredArgs a, in
         float den = a.sink ? __builtin_amdgcn_exp2f(a.sink[h] * kScoredLog2e - m) : 0.f;
         sd_f4 num = sd_f4{0.f, 0.f, 0.f, 0.f};
         for (int s = 0; s < a.splits; ++s) {
-            if (!(ml[2 * s + 1] > 0.f)) continue;  // (a piece without keys wrote no values)
+            if (ml[2 * s + 1] == 0.f) continue;  // (a piece without keys wrote no values; a sum that is no number stays one)
             const float w = __builtin_amdgcn_exp2f(ml[2 * s] - m);
             const sd_f4 x = *reinterpret_cast<const sd_f4 *>(po + (int64_t)s * vc);
             den = fmaf(w, ml[2 * s + 1], den);

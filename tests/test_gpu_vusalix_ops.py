@@ -380,6 +380,24 @@ def test_decode_over_latents_with_long_contexts(heads, rank, rot, window, splits
         assert_close(got[i], p @ rows[:, :rank], 1e-2, i)
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("kv,dim", [(1, 64), (2, 128)])
+def test_a_key_that_is_no_number_in_pieces(kv, dim, bad):
+    """A row is no number where it is none in one piece, not the sum of the other pieces' keys."""
+    announce(f"scored pieces, a key {bad}")
+    paged = Paged([3000, 900], kv, dim, dim, BF)
+    q = _rand(2, 4, dim, seed=9).to(BF)
+    call = lambda splits: torch.isfinite(_scored(paged, [(0, 2999, 1), (1, 899, 1)], (q,), dim, BF, 0.2, 0, decode=True, splits=splits).float())
+    for key in (0, 1700, 2999):
+        slot, x = int(paged.tables[0, key // 16]) * 16 + key % 16, paged.k
+        kept = x[slot, 0, 3].clone()
+        x[slot, 0, 3] = bad
+        one, got = call(False), call(True)
+        x[slot, 0, 3] = kept
+        assert torch.equal(one, got) and bool(one[1].all()), key
+        assert bad == bad or not bool(one[0, : 4 // kv].any()), key  # (infinite ones: by the sign of the query)
+
+
 def test_decode_pieces_with_sinks_and_padding_rows():
     announce("scored pieces")
     heads, dim, lens = 2, 64, [3000, 5]
