@@ -133,7 +133,7 @@ template <int KD, int NW, bool STATES> constexpr size_t la_lds_bytes() {
 // 128 x 128, the terms of 32-bit factors and the factors themselves 3500; the matrix cores work for 2700.  So rows come in 16-byte pieces and lie
 // in LDS as they are, in the one layout that both of a tile's products read, with operands ahead of their products and no branch in between; results
 // leave the registers straight for the output, and the first pass leaves out each portion's last segment, whose state the second pass itself
-// writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128, in five segments: first pass 41.3 -> 38.8 us, second 90.7 -> 87.2 (one read, one
+// writes to the pool.  8 prompts of 700 .. 4000 rows, 16 x 128 x 128, in three segments: first pass 41.5 -> 41.0 us, second 90.9 -> 86.7 (one read, one
 // product at a time, blocks of 4 x 4 -> this); 16 of 900 .. 1000 rows, 16 heads of 256 x 64, 138 -> 121; 10 of 28 .. 81, 32 heads of 128 x 64, 23.0 -> 20.9.
 // PAIR: at dim 128 a workgroup of eight waves has a compute unit to itself.  128 registers, with places in LDS worked out in every
 // chunk, let two share one.  Where segments outnumber the units: 6 prompts of 400 .. 2600 rows, 32 heads of 128 x 128, all passes,
@@ -145,9 +145,6 @@ __global__ __launch_bounds__(64 * NW, PAIR || (KD == 64 && NW == 8) ? 4 : KD == 
     constexpr int kVRows = kThr / (kCols / 8);
     static_assert(kKP * kThr == 64 * (KD / 8) && 2 * kVRows == 64, "whole passes");
     constexpr bool kTight = !STATES && (PAIR || (KD == 64 && NW == 8));  // 128 registers
-    // The next tile's silu beside the products of the state, or as the tile goes to LDS (8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128, us: first pass
-    // 42.8 and 38.8, second 87.2 and 91.6; 13 of 157 .. 258 rows, 32 heads of 64 x 64, both in one 26.3 and 25.1)
-    constexpr bool kBeside = !STATES && !PAIR && KD == 128 && NW == 8;
     constexpr int kGroup = kTight ? 2 : 4, kGroups = KD / 16 / kGroup;  // state tiles whose products go together
     constexpr int kST = NW == 8 ? 2 : 4;  // score tiles per wave
     extern __shared__ __align__(16) char lds[];
@@ -228,25 +225,20 @@ __global__ __launch_bounds__(64 * NW, PAIR || (KD == 64 && NW == 8) ? 4 : KD == 
     if (!STATES) fetch_q(r_beg);
     fetch_k(r_beg);
     fetch_v(r_beg);
-    // The silu of a tile, in its registers and in kActs equal parts
-    constexpr int kActs = 2 * kGroups, kPieces = (STATES ? 1 : 2) * kKP + 2;
-    auto act_part = [&](int part) {
+    auto silu = [](auto &x) {
 #pragma unroll
-        for (int i = 0; i < 4 * kPieces; ++i) {
-            if (i * kActs / (4 * kPieces) != part) continue;
-            la_u4 &x = i < 8 ? vb[i / 4] : i < 8 + 4 * kKP ? kb[(i - 8) / 4] : qb[STATES ? 0 : (i - 8 - 4 * kKP) / 4];
-            x[i % 4] = la_silu2(x[i % 4]);
-        }
-    };
-    auto act_all = [&] {
+        for (auto &piece : x)
 #pragma unroll
-        for (int part = 0; part < kActs; ++part) act_part(part);
+            for (int e = 0; e < 4; ++e) piece[e] = la_silu2(piece[e]);
     };
-    if (kBeside) act_all();
     for (int r0 = r_beg; r0 < r_end; r0 += kLaChunk) {
         const int nv = r_end - r0 < kLaChunk ? r_end - r0 : kLaChunk;
         const bool more = r0 + kLaChunk < r_end;
-        if (!kBeside) act_all();
+        // (beside the products of the chunk before, this was no faster: 8 prompts of 700 .. 4000 rows, 16 heads of 128 x 128, us: first pass 43.9, second
+        // 89.1, here 41.0 and 86.7)
+        silu(vb);
+        silu(kb);
+        if (!STATES) silu(qb);
         put();
         if (nv < kLaChunk && tid < 64) rev_tail[tid] = tid < nv ? powers[nv - 1 - tid] : 0.f;
         __syncthreads();
@@ -391,27 +383,22 @@ __global__ __launch_bounds__(64 * NW, PAIR || (KD == 64 && NW == 8) ? 4 : KD == 
                 for (int i = 0; i < 4; ++i) s[dt][i] *= whole;
         };
         keep(0);
-        auto move_on = [&](auto next) {  // (next: the next tile's silu beside the products)
 #pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const LaSplit sp = la_split_weighted(av[kk], *reinterpret_cast<const f4 *>(wt + 32 * kk + 4 * g), *reinterpret_cast<const f4 *>(wt + 32 * kk + 16 + 4 * g));
-                const bf8 hi = sp.high(), lo = sp.low();
+        for (int kk = 0; kk < 2; ++kk) {
+            const LaSplit sp = la_split_weighted(av[kk], *reinterpret_cast<const f4 *>(wt + 32 * kk + 4 * g), *reinterpret_cast<const f4 *>(wt + 32 * kk + 16 + 4 * g));
+            const bf8 hi = sp.high(), lo = sp.low();
 #pragma unroll
-                for (int x = 0; x < kGroups; ++x) {
-                    const int step = kk * kGroups + x;
-                    if (step + 1 < 2 * kGroups) read(step + 1);
-                    if (step + 1 < kGroups) keep(step + 1);
-                    if (decltype(next)::value) act_part(step);
-                    __builtin_amdgcn_sched_barrier(0);
+            for (int x = 0; x < kGroups; ++x) {
+                const int step = kk * kGroups + x;
+                if (step + 1 < 2 * kGroups) read(step + 1);
+                if (step + 1 < kGroups) keep(step + 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], hi, s[x * kGroup + j]);
+                for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], hi, s[x * kGroup + j]);
 #pragma unroll
-                    for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], lo, s[x * kGroup + j]);
-                }
+                for (int j = 0; j < kGroup; ++j) s[x * kGroup + j] = la_mfma(ak[step & 1][j], lo, s[x * kGroup + j]);
             }
-        };
-        if (kBeside && more) move_on(std::integral_constant<bool, kBeside>());
-        else move_on(std::false_type());
+        }
         if constexpr (!STATES) {
             __syncthreads();  // the next chunk's tiles may be written now
         } else {              // the other half of the tiles
