@@ -196,7 +196,7 @@ template <int KD> __device__ __noinline__ f4 cl_slow_scores(const uint16_t *uq, 
 // block as independent chains between them.  The scores, which four waves make, are asked for behind the last block, and with that barrier a chunk
 // has two: what follows it reads registers and scores alone.  The next rows' loads are spread over the blocks; no place is kept that would be
 // spilled, as a reload waits for the loads before it.  8 prompts of 700 .. 4000 rows, 32 heads of 128 x 128, second pass: 295 -> 266 us (scores ahead of the
-// blocks, three barriers, one accumulator -> this), 33 of 150 .. 168 rows, 32 heads of 96 x 80, 175 -> 156.
+// blocks, three barriers, one accumulator -> this), 33 of 150 .. 168 rows, 32 heads of 96 x 80, 124 -> 104.
 // Two blocks at a time, whose state is split once, needs P Q of the second from the first one's start as well and is spilled: 449 us for both passes,
 // else 377.
 // STATES: only the segment's own contribution to the state and its factors, to the workspace (first pass over a portion in

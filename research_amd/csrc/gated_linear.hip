@@ -235,8 +235,8 @@ __device__ __forceinline__ float gl_scan_max(float x, int lane) {
 // they were spilled, and each reload waited for the tile's loads); the next tile's loads are spread over the chunk; its gates are made by a wave
 // without score tiles; n . q is a product, and rows' factors are divided once per row and wave.  Cycles of a chunk at 256 x 128 columns, mLSTM: 21400 ->
 // 15000, of which products keep a SIMD busy for 5800 and the vector unit for 5100.
-// One prompt of 15999 rows, 4 heads of 256 x 512 (mLSTM): second pass 168 -> 124 us, first 73 -> 58; 8 prompts of 1226 .. 1840 rows, 16 heads of 128 x 64 (SSD)
-// 92 -> 83; 17 of 480 .. 628, 4 heads of 256 x 512 202 -> 157; single chunks, 23 of 2 .. 25 rows, 8 heads of 128 x 256, 20.4 -> 17.2.
+// One prompt of 15999 rows, 4 heads of 256 x 512 (mLSTM): second pass 171 -> 125 us, first 72 -> 54; 8 prompts of 1226 .. 1840 rows, 16 heads of 128 x 64 (SSD)
+// 87 -> 71; 17 of 480 .. 628, 4 heads of 256 x 512 162 -> 110; single chunks, 23 of 2 .. 25 rows, 8 heads of 128 x 256, 20.1 -> 15.9.
 // WIDE: rows of whole, aligned 16-byte pieces, else of 8-byte ones.  (In one kernel, with a branch, each load of the one kind waited for those of the other,
 // which had never been asked for: q, k and v of a workgroup's first chunk came one after the other.)  The first chunk's gates are asked for
 // ahead of its tiles and made while those are on their way.  At 64 x 64 three workgroups share a compute unit.  Single chunks, 32 heads of 64 x 64, us: branch and

@@ -14,7 +14,7 @@ constexpr int kLaChunk = 64;      // rows multiplied at once
 constexpr int kLaMinSegChunks = 8;    // a segment is at least this many chunks long ...
 constexpr int kLaMaxSegments = 64;
 constexpr int kLaLeastSegChunks = 2;  // ... or, of few sequences, this many
-// Segments whose states the scan between the passes loads at once (8 prompts in five segments, 16 heads of 128 x 128, all passes: 2 137.4 us, 4
+// Segments whose states the scan between the passes loads at once (8 prompts in three segments, 16 heads of 128 x 128, all passes: 2 137.4 us, 4
 // 137.9, 8 139.0; one of 12000 rows in 32, 8 heads: 70.5, 69.5, 69.0).
 constexpr int kLaScanAhead = 4;
 

@@ -26,11 +26,10 @@ int prefill_cus() {
 }
 
 // (the split rule, the workspace size and the groups a workgroup runs are host-testable arithmetic: prefill_plan.h)
-// Pieces of a launch whose groups hold `tasks` tasks.  us, each number of pieces measured (unsplit, 2, 3 .. 8) -> the rule's: 8 / 2 heads of 128,
-// 7 prompts of 248 rows behind 3936 keys 78, 53, 43, 38, 37, 35, 35, 35 -> 35 (53 while pieces had 24 tiles or more and a call's prompts counted as
-// long as its longest); 14 / 2 of 128, 7 of 114 rows behind 3856 52 -> 34; 8 / 2 of 64, 2 of 41 rows behind 3712 41 -> 26; 16 / 8 of 128, 6 of 73
-// rows behind 4096 54 -> 37, 6 of 681 rows behind 1920 52, 47, 42, 40 .. -> 42; 16 / 8 of 256, 4 of 505 rows behind 1392 48 -> 40.  Of 90 drawn batches
-// (1 to 64 prompts behind up to 8192 keys) the rule's pieces took 1.02 of the time of each one's best.
+// Pieces of a launch whose groups hold `tasks` tasks.  us, unsplit, in two pieces, in three .. up to the rule's: 8 / 2 heads of 128, 7 prompts of 248
+// rows behind 3936 keys 76, 55, 46, 44 (two while pieces had 24 tiles or more and a call's prompts counted as long as its longest); 14 / 2 of 128, 7
+// of 114 behind 3856 72, 53, 45, 43; 8 / 2 of 64, 2 of 41 behind 3712 56, 38, 29, 25, 22, 21, 20; 16 / 8 of 128, 6 of 73 behind 4096 77, 53, 43, 41, 40.
+// Of 90 drawn batches (1 to 64 prompts behind up to 8192 keys) the rule's pieces took 1.02 of the time of each one's best.
 int prefill_splits(int num_kv_heads, int64_t groups, int batch, int64_t rows, int n_rep, int tasks, int head_dim, int64_t max_keys) {
     return plan_prefill_splits(plan_prefill_units(num_kv_heads, groups, batch, rows, n_rep, kPfRows, tasks), prefill_cus(), max_keys,
                                head_dim > 128 ? kWdKeys : kPfKeys, rows * num_kv_heads * n_rep * (head_dim + 2) * 4);

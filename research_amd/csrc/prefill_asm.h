@@ -39,8 +39,9 @@ namespace pa_decode_detail {
 // ONE: a workgroup has one group.  What a workgroup does beside its tiles is one wave's instructions per SIMD, four to five cycles each, so that
 // their number is the time of a short launch.  With a loop over groups the compiler derives every group's constants ahead of it and spills scalar
 // registers around the tile loop; without one a workgroup of a single tile takes 21200 cycles, else 24000: of these, between the requests for Q and
-// the tables' loads 570, else 2950 (us a call: 14 / 2 heads of 128, a prompt of 18 rows 13.5 -> 12.7; 16 / 8 of 96, 10 of 111 .. 223 behind 336
-// keys 26.2 -> 24.7; 32 / 8 of 128, 48 of 99 .. 145 behind 1008 148 -> 144, 32 of 97 .. 249 behind 2048 224.6 -> 220.3).
+// the tables' loads 570, else 2950 (us with the append: 14 / 2 heads of 128, a prompt of 18 rows 12.2 -> 11.6; 16 / 8 of 96, 10 of 111 .. 223 behind 336
+// keys 25.3 -> 24.2; 32 / 8 of 128, 48 of 99 .. 145 behind 1008 144 -> 139, 32 of 97 .. 249 behind 2048 219 -> 216; over 315 batches 0.97 of the time,
+// none slower by more than 1.1 %).
 template <typename T, bool LO, int D, bool LONG = false, bool ONE = LO || LONG>
 __global__ __launch_bounds__(kPfThreads) void prefill_asm_kernel(const RowwiseArgs a) {
     using M = Mfma16<T>;

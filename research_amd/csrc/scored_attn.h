@@ -68,7 +68,7 @@ __device__ __forceinline__ scored_u4 scored_load16(const uint16_t *p, bool there
 // The rows of one kv head in a pool of less than 2 GiB, read by 32-bit offsets: a row that is not there (slot -1) and what lies past a row's end
 // (an offset of kScoredAway) fall outside the descriptor and come back as zeros.  A 16-byte piece takes two instructions beside its load, by address
 // and choice of one fourteen, which the vector unit pays for where it has no other to spare (portions, 16 / 4 heads of 128, window 1024, cap: 8 of 700
-// .. 4000 rows 146 -> 139 us; the sums of attention with mixed heads are no faster for it, and keep addresses).
+// .. 4000 rows 131 -> 126 us; the sums of attention with mixed heads are no faster for it, and keep addresses).
 constexpr uint32_t kScoredAway = 0x80000000u;
 struct ScoredRows {
     __amdgpu_buffer_rsrc_t rows;

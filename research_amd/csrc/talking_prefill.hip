@@ -138,7 +138,7 @@ constexpr int kTmRows = 16, kTmKeys = 32, kTmWaves = 8, kTmThreads = 64 * kTmWav
 constexpr int kTmOut = 2 * kTmWaves;  // out heads of a workgroup, two per wave
 
 // Up to 16 heads there is room for the weights of two tiles, and the next tile's are made beside the mixing of this one's: a tile takes 4600 cycles,
-// else 4850, of which the mixing's few reads and products were 500 (8 prompts of 700 .. 4000 rows, 16 heads of 128: 420 -> 404 us).  It begins with two more
+// else 4850, of which the mixing's few reads and products were 500 (8 prompts of 700 .. 4000 rows, 16 heads of 128: 419 -> 407 us).  It begins with two more
 // barriers and a wait for the second tile's keys, so up to eight tiles stay as they were (25 .. 111 rows, 8 heads: 19.8 us, else 20.5).
 constexpr int kTmAhead = 8;
 
