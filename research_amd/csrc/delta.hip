@@ -964,13 +964,10 @@ template <int KD> int launch_delta_chunks(const DeltaArgs &a, int batch, hipStre
         return launch_walk<KD, 4>(a, batch, s);
     } else {
         if (a.vdim > 64 && heads * ((a.vdim + 127) / 128) >= la_cus()) return launch_walk<KD, 8>(a, batch, s);
-        const int64_t slices = heads * ((a.vdim + 63) / 64);
-        const bool four = a.vdim > 32 && slices >= la_cus();
-        // (a compute unit has room for two workgroups of four waves at dim 64, and for one of the paired ones, whose chain is not worth it in
-        // one chunk or two: 32 heads of 64 x 64, us, prompts of 16 .. 30 rows, 9 of them 18.9 against 21.0, 63 54.1 against 58.8; of 60 .. 120
-        // rows, 9 of them 26.1 against 25.0, 63 89.1 against 91.4; of 200 .. 250 rows, 63 220 against 202)
-        const bool brief = KD == 64 && four && (a.chunks == 1 || (a.chunks == 2 && slices >= 2 * la_cus()));
-        if (!brief && delta_pieces_of_16(a)) return four ? launch_pair<KD, 4>(a, batch, s) : launch_pair<KD, 2>(a, batch, s);
+        const bool four = a.vdim > 32 && heads * ((a.vdim + 63) / 64) >= la_cus();
+        const int cols = four ? 64 : 32;
+        if (delta_pieces_of_16(a) && la_delta_pairs(heads * ((a.vdim + cols - 1) / cols), (KD == 64) == four ? 2 : 1, four, batch, a.chunks, a.n_rows, la_cus()))
+            return four ? launch_pair<KD, 4>(a, batch, s) : launch_pair<KD, 2>(a, batch, s);
         return four ? launch_walk<KD, 4>(a, batch, s) : launch_walk<KD, 2>(a, batch, s);
     }
 }

@@ -106,6 +106,25 @@ static inline int la_launch_segments(int64_t batch, int64_t per_seq, int cus, do
     return la_balanced_segments(batch, per_seq, cus, together, max_len, n_rows, most);
 }
 
+// Whether the delta rule's walk over `workgroups` workgroups goes to pairs of waves, of whose workgroups a compute unit has one at dim 128, or to single
+// waves, of which it has `walks` for each of the others (four: of four waves, which then share their SIMDs).  A pair is faster through a chunk.  So it
+// decides where no compute unit gets a second workgroup, where two of either fit or one, and where a long chain is waited for: behind unequal prompts,
+// whose chunks in all keep the device busy for less than the longest one's, and above 16 chunks.  Else two walks at once need less than two pairs one
+// after the other; an odd number of pairs' rounds is half a round more for walks of two waves, which pays up to two chunks.  us, walks / pairs: 4
+// heads of 128 x 32, 100 prompts of 40 .. 64 rows (1.6 rounds) 20.7 / 23.4; 8 of 128 x 64, 18 of 100 .. 128 (1.1) 22.2 / 25.3; 16 of 128 x 64, 9 of
+// 1000 .. 1024 (1.1) 89 / 100; 32 of 64 x 64, 20 of 120 .. 192 (2.5) 48.6 / 53.4; but 8 of 128 x 128, 9 of 30 .. 400 (1.1) 28.4 / 23.8; 16 of 128 x 128, 5
+// of 64 .. 1500 (1.2) 78 / 63; 4 of 128 x 32, 160 of 500 .. 512 (2.5) 168 / 152.  Over 325 batches of one to 63 chunks the rule's choice takes 1.004 of the
+// better one's time, no batch more than with pairs alone, which take 1.024 and 1.17 at most.
+static inline bool la_delta_pairs(int64_t workgroups, int walks, bool four, int64_t batch, int chunks, int64_t n_rows, int cus) {
+    if (walks < 2) return true;
+    if (four && chunks == 1) return false;
+    if (workgroups <= cus || chunks > 16) return true;
+    if (chunks <= 2) return false;
+    int64_t all = n_rows / kLaChunk + batch / 2;  // chunks, about
+    if (all > batch * chunks) all = batch * chunks;
+    return workgroups * all <= batch * cus * chunks || (!four && (workgroups + cus - 1) / cus % 2 != 0);
+}
+
 // Segments of seg_rows rows before a portion's last one.  (Rows past the longest length that a launch was told have no segment.)
 PA_LA_FN int la_full_segments(int rows, int segments, int seg_rows) {
     const int full = rows > 0 ? (rows - 1) / seg_rows : 0;

@@ -180,6 +180,17 @@ def test_delta_rule_rows_of_whole_pieces(heads, groups, dim, vdim):
     case.check_states(slots)
 
 
+@pytest.mark.parametrize("heads,groups,dim,vdim,lens", [(40, 10, 128, 32, [70, 64, 128, 66, 127, 120, 65]), (48, 12, 64, 64, [130, 128, 192, 129, 150, 193, 180]),
+                                                        (32, 8, 72, 96, [64, 30, 1])])
+def test_delta_rule_of_about_equal_prompts(heads, groups, dim, vdim, lens):
+    """More workgroups than compute units, which take two at once: rows of whole pieces walked by single waves."""
+    announce(f"delta equal {heads} {groups} {dim} {vdim}")
+    case = DeltaCase(lens, heads, groups, dim, vdim, BF, seed=11)
+    slots = list(range(len(lens)))[::-1]
+    case.run([(i, 0, n) for i, n in enumerate(lens)], slots, pieces=True)
+    case.check_states(slots)
+
+
 def test_delta_rule_many_heads_take_wide_slices():
     announce("delta wide slices")
     for heads, batch, vdim in ((160, 2, 128), (160, 2, 64), (300, 1, 72)):

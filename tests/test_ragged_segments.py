@@ -10,6 +10,22 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+def test_which_delta_rule_walks_go_to_pairs_of_waves(tmp_path):
+    """(workgroups, walks a compute unit has, of four waves, prompts, chunks of the longest, rows, pairs) on 256 compute units."""
+    batches = [(256, 2, 0, 16, 1, 800, 1), (400, 2, 0, 25, 1, 1300, 0), (288, 2, 0, 18, 2, 2050, 0), (288, 2, 0, 18, 2, 700, 0),
+               (384, 2, 0, 3, 1, 90, 0), (288, 2, 0, 9, 7, 1290, 1), (320, 2, 0, 20, 16, 20200, 0), (320, 2, 0, 20, 17, 20800, 1),
+               (640, 2, 0, 40, 2, 4600, 0), (640, 2, 0, 40, 8, 20200, 1), (400, 1, 0, 25, 1, 1300, 1), (640, 2, 1, 20, 3, 3700, 0), (800, 2, 0, 50, 8, 25300, 0),
+               (256, 2, 1, 8, 1, 400, 0), (257, 2, 1, 8, 4, 2000, 0), (256, 2, 1, 8, 4, 2000, 1), (640, 1, 1, 20, 3, 3700, 1), (640, 1, 1, 20, 1, 900, 1),
+               (400, 2, 0, 25, 3, 1 << 40, 0), (400, 2, 0, 25, 3, 0, 1)]
+    src = tmp_path / "plan.cpp"
+    src.write_text('#include "lightning_plan.h"\nint main() {\n' + "".join(
+        f"    if (la_delta_pairs({w}LL, {walks}, {four}, {batch}, {chunks}, {rows}LL, 256) != {want}) return {i + 1};\n"
+        for i, (w, walks, four, batch, chunks, rows, want) in enumerate(batches)) + "}\n")
+    exe = tmp_path / "plan"
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "research_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
+
+
 def test_segments_follow_the_rows_of_a_batch(tmp_path):
     src = tmp_path / "plan.cpp"
     src.write_text('''
