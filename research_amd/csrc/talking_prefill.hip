@@ -10,7 +10,7 @@
 //   2. T times these, the pairs of four keys per wave, and back to LDS as weights of (out head, row), keys side by side;
 //   3. O^T += V^T W^T per out head, V by transposing reads from the wave's own part of LDS.
 // The next tile's keys and values are on their way in registers.  Distance biases of a head are one logarithm per lane and
-// tile, spread by LDS.
+// tile, spread by LDS.  Up to 16 heads whose fours share a kv head have a kernel whose waves are of two kinds (talk_pipe_kernel).
 #include "linear_tiles.h"
 #include "prefill_mfma.h"
 #include "talking.h"
@@ -512,6 +512,358 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     }
 }
 
+// ------------------------------------------------------------------ mixed weights times values, waves of two kinds
+// Up to 16 heads whose fours share a kv head: half of the waves make the weights of a tile of 32 keys while the others mix those of the tile before it
+// and multiply the mixed ones of the tile before that by the values, so that the vector unit (exponentials, terms) and the matrix cores and LDS
+// (mixing, values) are busy side by side, and a tile has one barrier.  A wave has the heads of one kv head, and half of the keys or of the value
+// columns: keys go straight to its operands, values to its own part of LDS.  Up to 8 heads two workgroups share a compute unit.
+// A tile of 16 heads takes 3500 .. 4400 cycles, of which the vector unit is busy 1750, LDS 1950, the matrix cores 1280 and the first cache 3200 (a
+// load of keys that lie 16 bytes a row takes 64 cycles, of whole 128-byte rows 19): what bounds it is the chain of a wave through LDS, at the 128
+// registers that 16 waves leave it.  Eight waves of twice the registers took as long (444 us), keys by way of LDS longer (452).
+// us a call, the kernel above -> this one: 16 / 4 heads of 128, 8 prompts of 818 .. 3868 rows 480 -> 428, one of 1100 106 -> 91; 8 / 2 of 128, one of 1100
+// 87 -> 59; 8 / 2 of 64, 11 of 534 .. 695 55 -> 47, 10 of 28 .. 145 17.1 -> 15.0.  More than 8 heads behind up to 256 keys stay with the kernel above, which
+// begins sooner (5 of 8 .. 24 rows 16.7, else 18.7; 3 of 81 .. 205 26.9, else 28.1; 6 of 133 .. 279 37.2, here 36.0).
+constexpr int kTpRows = 16, kTpKeys = 32;
+constexpr int kTpShort = 256;  // keys that a table has room for
+template <int DV, int G> struct TpTile {  // G: fours of heads, 2 or 4
+    static constexpr int heads = 4 * G, part = 2 * G, threads = 64 * 2 * part;       // waves of a kind
+    static constexpr int pair = 16 * G, pTile = kTpKeys * kTpRows * pair;            // bytes of a (key, row) pair: both terms of all heads
+    static constexpr int wTile = heads * kTpRows * kTpKeys * 2;
+    static constexpr int cols = DV / 2, vTile = kTpKeys * cols * 2;                  // a wave's value columns
+    static constexpr int biasFloats = 4 * 32;                                        // distances of a wave's heads, twice
+    static constexpr int tBytes = G / 2 * 2 * 1024;                                  // both terms of T as operands, in one or two orders
+    static constexpr int ring = 4 * kTpKeys;                                         // pool rows of the tiles to come
+    static constexpr size_t bytes = 2 * (size_t)pTile + 2 * (size_t)wTile + part * ((size_t)vTile + 2 * biasFloats * 4 + 256) + tBytes + ring * 4;
+    // Value rows of 64 or 128 bytes without padding: the 64-byte halves of 128 change places in every second two rows, so that a transposing read (64
+    // bytes of four rows) spreads over the banks.
+    static constexpr __device__ int vTurn(int row) { return cols == 32 ? 0 : (row >> 1 & 1) * 64; }
+};
+
+// A value that is the same in all lanes, as a scalar
+__device__ __forceinline__ float tp_scalar(float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); }
+
+// Which block of 16 rows of which portion has `rank` in their order from the rows furthest behind to the first ones, and that portion (each wave by
+// itself; what is known of up to 64 portions is loaded once).
+__device__ __forceinline__ bool tp_block(const TalkArgs &a, int rank, int &b, int &block, ScoredPortion &p) {
+    const int lane = threadIdx.x & 63, most = (a.max_q_len + kTpRows - 1) / kTpRows;
+    ScoredPortion mine;
+    auto load = [&](int first) { return first + lane < a.batch && scored_portion(a, first + lane, mine) ? min((mine.n + kTpRows - 1) / kTpRows, most) : 0; };
+    int blocks = load(0);
+    auto behind = [&](int i) {  // blocks whose number in their portion is at least i
+        if (a.batch <= 64) return __builtin_amdgcn_readlane(la_scan(max(blocks - i, 0), lane), 63);
+        int n = 0;
+        for (int first = 0; first < a.batch; first += 64) n += max(load(first) - i, 0);
+        return __builtin_amdgcn_readlane(la_scan(n, lane), 63);
+    };
+    if (rank >= behind(0)) return false;
+    int low = 0, high = most;  // behind(low) > rank >= behind(high)
+    while (high - low > 1) {
+        const int mid = (low + high) / 2;
+        if (behind(mid) > rank) low = mid;
+        else high = mid;
+    }
+    block = low;
+    rank -= behind(high);
+    for (int first = 0; first < a.batch; first += 64) {
+        if (a.batch > 64) blocks = load(first);
+        const uint64_t there = __ballot(blocks > low);
+        const int n = __builtin_popcountll(there);
+        if (rank < n) {
+            const int at = __builtin_ctzll(__ballot((there >> lane & 1) != 0 && __builtin_popcountll(there & ((1ull << lane) - 1)) == rank));
+            b = first + at;
+            p.n = __builtin_amdgcn_readlane(mine.n, at);
+            p.pos0 = __builtin_amdgcn_readlane(mine.pos0, at);
+            p.row0 = __builtin_amdgcn_readlane((int)mine.row0, at);  // (q_starts has 32 bits)
+            return true;
+        }
+        rank -= n;
+    }
+    return false;
+}
+
+template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G, 4) void talk_pipe_kernel(const TalkArgs a) {
+    using L = TpTile<DV, G>;
+    constexpr int KS = DK / 32, NC = L::cols / 32;
+    typedef float f16 __attribute__((ext_vector_type(16)));
+    extern __shared__ __align__(16) char tm_lds[];
+    // Workgroups that are all there at once take any block; else those with the most keys come first.
+    int b = blockIdx.x % a.batch, block = blockIdx.x / a.batch;
+    ScoredPortion p;
+    if (gridDim.x > a.at_once ? !tp_block(a, blockIdx.x, b, block, p) : !scored_portion(a, b, p)) return;
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+    const int all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = all % L::part;
+    char *w_all = tm_lds + 2 * L::pTile, *v_all = w_all + 2 * L::wTile;
+    float *bias_all = reinterpret_cast<float *>(v_all + L::part * L::vTile);
+    f4 *from_all = reinterpret_cast<f4 *>(bias_all + L::part * 2 * L::biasFloats);
+    bf8 *t_all = reinterpret_cast<bf8 *>(from_all + L::part * 16);
+    int *ring = reinterpret_cast<int *>(reinterpret_cast<char *>(t_all) + L::tBytes);
+    const int four = wave % G, head0 = 4 * four, half = wave / G;  // the wave's heads, and which half of keys or columns
+    const int kv = min(head0, a.heads - 4) / a.n_rep;
+    // Places in LDS that spread over the banks: 16-byte pieces of a pair of 16 heads and of a (head, row)'s keys turn with the row, those of a pair
+    // of 8 heads with key / 8; the 8-byte halves of a pair's pieces change places with key / 4, those of a (head, row)'s with head / 4.
+    const int turn16 = -(l16 >> 2) & 3;
+    const int row0 = block * kTpRows;
+    if (row0 >= p.n) return;
+    const int row = row0 + l16, first_pos = p.pos0 + row0, end = p.pos0 + min(row0 + kTpRows, p.n), tiles = (end + kTpKeys - 1) / kTpKeys;
+    // Pool row of a key, from its block; past the last key: the last one's, which nothing weighs.
+    const int32_t *table = a.bt + b * a.bt_stride;
+    const int last_block = (int)min(a.bt_stride, (int64_t)0x7fffffff) - 1, known = (int)a.num_blocks;
+    auto block_of = [&](int key) { return (int)(__umulhi(2u * (uint32_t)min(key, end - 1), a.bs_magic) >> a.bs_magic_shift); };
+    auto id_of = [&](int key) { return table[min(block_of(key), last_block)]; };
+    auto slot_of = [&](int id, int key) {
+        const int blk = block_of(key);
+        const bool there = (blk <= last_block) & ((uint32_t)id < (uint32_t)known);
+        return there ? min(key, end - 1) + (id - blk) * a.bs : 0;
+    };
+    const int first_id = id_of(tid % (4 * kTpKeys));
+
+    if (all < L::part) {
+        // ---- weights of keys 16 half + 4 g + j of row l16 ----
+        float *biases = bias_all + wave * 2 * L::biasFloats;
+        const float plain = tp_scalar(a.scale * kScoredLog2e);
+        bf8 q[4][KS];
+        float from[4];
+        const int64_t mem_row = p.row0 + min(row, p.n - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int h = min(head0 + i, a.heads - 1);
+            const uint16_t *src = reinterpret_cast<const uint16_t *>(a.q1) + mem_row * a.q1_row + h * a.q1_head;
+#pragma unroll
+            for (int k = 0; k < KS; ++k) q[i][k] = __builtin_bit_cast(bf8, scored_load16(src + 32 * k + 8 * g, FULL || 32 * k + 8 * g < a.n1));
+            from[i] = a.lse[mem_row * a.heads + h];
+        }
+        // keys straight to operands: a lane's pieces of key 16 half + l16 (columns past the last: zeros)
+        const uint32_t k_tok = (uint32_t)(a.hkv * a.k_dim) * 2u;
+        const char *kp = reinterpret_cast<const char *>(a.k) + ((int64_t)kv * a.k_dim + 8 * g) * 2;
+        const int my_key = 16 * half + l16;
+        bf8 kr[KS];
+        auto fetch = [&](int slot) {
+            const char *src = kp + (uint64_t)(uint32_t)slot * k_tok;
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+                kr[k] = FULL ? *reinterpret_cast<const bf8 *>(src + 64 * k)
+                             : __builtin_bit_cast(bf8, scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, 32 * k + 8 * g < a.n1));
+        };
+        // (distances first_pos + r - k of 16 rows and 16 keys, from their smallest, of two heads a lane; a key behind its row gets no weight)
+        float size[2], rate[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int h = min(head0 + lane / 32 * 2 + i, a.heads - 1);
+            const float x = (a.size ? a.size : a.talk)[h], y = (a.rate ? a.rate : a.talk)[h];
+            size[i] = a.size ? x : 0.f;
+            rate[i] = a.rate ? y : 0.f;
+        }
+        auto put_biases = [&](int k0, float *to) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) to[lane / 32 * 64 + i * 32 + lane % 32] = talk_masked_bias(size[i], rate[i], first_pos - (k0 + 16 * half + 15) + lane % 32);
+        };
+        if (tid < 3 * kTpKeys) ring[tid] = slot_of(first_id, tid);
+        __syncthreads();
+        fetch(ring[my_key]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) from[i] = -(row < p.n && head0 + i < a.heads ? from[i] : -kScoredNone) / plain;  // (no head, no row: no weight)
+        f4 *const start = from_all + wave * 16 + l16;  // the products start from -lse (in LDS: in registers, operands were spilled)
+        if (g == 0) *start = f4{from[0], from[1], from[2], from[3]};
+        put_biases(0, biases);
+        const int my_pairs = ((16 * half + 4 * g) * kTpRows + l16) * L::pair + 8 * ((four ^ g) & 1) + 16 * ((four >> 1) ^ (G == 4 ? turn16 : g >> 1));
+        for (int t = 0; t < tiles; ++t) {
+            const int pairs = my_pairs + (t & 1) * L::pTile;
+            tp_own_lds();
+            const int slot = ring[((t + 1) * kTpKeys + my_key) & (L::ring - 1)];
+            const float *bp = biases + (t & 1) * L::biasFloats + l16 + 15 - 4 * g;
+            f4 s[4];
+            const f4 first = *start;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] = f4{first[i], first[i], first[i], first[i]};
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[i] = la_mfma(kr[k], q[i][k], s[i]);
+            fetch(slot);  // (past the last key any)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[i][j] = __builtin_amdgcn_exp2f(fmaf(s[i][j], plain, bp[i * 32 - j]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint2 hi, lo;
+                la_split2(s[0][j], s[1][j], hi.x, lo.x);
+                la_split2(s[2][j], s[3][j], hi.y, lo.y);
+                *reinterpret_cast<uint2 *>(tm_lds + pairs + j * kTpRows * L::pair) = hi;
+                *reinterpret_cast<uint2 *>(tm_lds + (pairs ^ 8 * G) + j * kTpRows * L::pair) = lo;
+            }
+            put_biases((t + 1) * kTpKeys, biases + (~t & 1) * L::biasFloats);
+            __syncthreads();  // the pairs are there, those of the tile before have been read
+        }
+        __syncthreads();
+        return;
+    }
+
+    // ---- mixing and values ----
+    // T in the pairs' k order.  16 heads: row l16 of T, k = 8 g + e: both terms of 16 heads; 8 heads: two keys at once, rows 8 (key) + head,
+    // k = 16 (key) + 8 (term) + head.  The second term of T meets the first of the weights only.  (In LDS: eight registers less.)
+    const bf8 *t_s = t_all + (G == 4 ? wave & 1 : 0) * 128 + lane;
+    bool t_rest = false;  // (a matrix stored in 16 bits has no second term)
+    {
+        LaSplit sp;
+        bool exact = true;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float x[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int turned = j ^ 2 * (G == 4 ? wave & 1 : g >> 1);
+                const int out = G == 4 ? l16 : l16 & 7, in = (8 * g + 2 * turned + e) % L::heads;
+                const bool there = (out < a.heads) & (in < a.heads) & (G == 4 || l16 >> 3 == g >> 1);
+                const float y = a.talk[min(out, a.heads - 1) * a.heads + min(in, a.heads - 1)];  // (loaded without a branch: one trip to memory for all)
+                x[e] = there ? y : 0.f;
+            }
+            la_split2(x[0], x[1], sp.hi[j], sp.lo[j]);
+            exact = exact && sp.lo[j] == 0;
+            if (G == 4 ? g >= 2 : g & 1) sp.lo[j] = 0;
+        }
+        if (wave < G / 2) {
+            const_cast<bf8 *>(t_s)[0] = sp.high();
+            const_cast<bf8 *>(t_s)[64] = sp.low();
+        }
+        t_rest = __ballot(!exact) != 0;
+    }
+
+    f16 o[2][NC];  // out heads head0 + 2 i + (l16's half of 32 lanes), columns col0 + 32 c + ..
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[i][c][e] = 0.f;
+    // the wave's values: a whole row of its columns at a time by four or eight lanes, in the order of the lanes (columns past the last: the first ones
+    // again, for nobody)
+    constexpr int kPer = L::cols / 8, kEach = 64 / kPer, NV = kTpKeys / kEach;
+    char *const v_s = v_all + wave * L::vTile;
+    const int col0 = half * L::cols, vreal = (a.vdim + 7) / 8 * 8;
+    const uint32_t v_tok = (uint32_t)(a.hkv * a.v_dim) * 2u;
+    const int my_col = col0 + (lane % kPer * 8 ^ L::vTurn(lane / kPer) / 2), my_key = lane / kPer;
+    const char *vp = reinterpret_cast<const char *>(a.v) + ((int64_t)kv * a.v_dim + (FULL || my_col < vreal ? my_col : 0)) * 2;
+    scored_u4 vr[NV];
+    auto fetch = [&](int k0) {
+        const int *slots = ring + ((k0 + my_key) & (L::ring - 1));
+#pragma unroll
+        for (int n = 0; n < NV; ++n) vr[n] = *reinterpret_cast<const scored_u4 *>(vp + (uint64_t)(uint32_t)slots[n * kEach] * v_tok);
+    };
+    auto put_v = [&]() {
+#pragma unroll
+        for (int n = 0; n < NV; ++n) *reinterpret_cast<scored_u4 *>(v_s + lane * 16 + n * 1024) = vr[n];
+    };
+    // mixed: keys 4 wave + m of row l16, out heads 4 g + i (8 heads: keys 8 wave + 4 (g / 2) + m, out heads 4 (g % 2) + i)
+    const int mix_key = G == 4 ? 4 * wave : 8 * wave + 4 * (g >> 1), mix_head = 4 * (G == 4 ? g : g & 1);
+    const int pair_at = (mix_key * kTpRows + l16) * L::pair + 16 * (G == 4 ? g ^ turn16 : (g & 1) ^ (wave & 1));
+    const int mixed_at = (mix_head * kTpRows + l16) * (kTpKeys * 2) + 16 * ((mix_key >> 3) ^ turn16) + 8 * ((mix_key >> 2 ^ mix_head >> 2) & 1);
+    auto mix = [&](const char *pairs, char *w_s) {
+        // (two keys at a time: of four, the loop's registers were spilled)
+        uint32_t mixed[2][4];
+#pragma unroll
+        for (int m = 0; m < 4; m += 2) {
+            const bf8 one = la_read8(reinterpret_cast<const __bf16 *>(pairs + pair_at + m * kTpRows * L::pair));
+            const bf8 two = la_read8(reinterpret_cast<const __bf16 *>(pairs + pair_at + (m + 1) * kTpRows * L::pair));
+            const bf8 t_hi = t_s[0];
+            f4 x = la_mfma(t_hi, one, f4{0.f, 0.f, 0.f, 0.f}), y = la_mfma(t_hi, two, f4{0.f, 0.f, 0.f, 0.f});
+            if (t_rest) {
+                const bf8 t_lo = t_s[64];
+                x = la_mfma(t_lo, one, x);
+                y = la_mfma(t_lo, two, y);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mixed[m / 2][i] = row_pack_bf16(x[i], y[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<uint2 *>(w_s + mixed_at + i * kTpRows * kTpKeys * 2) = make_uint2(mixed[0][i], mixed[1][i]);
+    };
+    const int side = lane >> 5, mine = lane >> 4 & 1;  // (of a product's 32 columns the second 16 are another head's)
+    const int x_at = ((head0 + mine) * kTpRows + l16) * (kTpKeys * 2) + 16 * (side ^ turn16);
+    const int v_row = 8 * side + (l16 >> 2), v_first = (v_row * L::cols * 2 + mine * 32 + (l16 & 3) * 8) ^ L::vTurn(v_row);  // (rows 4 on: the same turn)
+    const int va0 = v_first + (four & 1 ? 4 * L::cols * 2 : 0), va1 = v_first + (four & 1 ? 0 : 4 * L::cols * 2);  // (which four keys come first)
+    auto values = [&](const char *w_s) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {  // 16 keys
+            bf8 x[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) x[i] = la_read8(reinterpret_cast<const __bf16 *>(w_s + (x_at ^ 32 * k) + 2 * i * kTpRows * kTpKeys * 2));
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const bf8 v = la_join(la_read_tr(reinterpret_cast<const __bf16 *>(v_s + (va0 ^ 64 * c) + k * 16 * L::cols * 2)),
+                                      la_read_tr(reinterpret_cast<const __bf16 *>(v_s + (va1 ^ 64 * c) + k * 16 * L::cols * 2)));
+#pragma unroll
+                for (int i = 0; i < 2; ++i) o[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, x[i], o[i][c], 0, 0, 0);
+            }
+        }
+    };
+    int id = id_of(3 * kTpKeys + (lane & 31));
+    __syncthreads();
+    fetch(0);
+    for (int t = 0; t < tiles; ++t) {
+        __syncthreads();  // this tile's pairs are there, the mixed weights of the one before too
+        if (t > 0) {
+            values(w_all + (~t & 1) * L::wTile);
+            tp_own_lds();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        mix(tm_lds + (t & 1) * L::pTile, w_all + (t & 1) * L::wTile);
+        put_v();
+        fetch((t + 1) * kTpKeys);  // (past the last key any)
+        if (wave == 0) {  // pool rows of three tiles ahead: read behind the next barriers, written over four tiles later
+            const int key = (t + 3) * kTpKeys + (lane & 31);
+            ring[key & (L::ring - 1)] = slot_of(id, key);
+            id = id_of(key + kTpKeys);
+        }
+        tp_own_lds();
+    }
+    __syncthreads();
+    values(w_all + (~tiles & 1) * L::wTile);
+    if (row >= p.n) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int h = head0 + 2 * i + mine;
+        if (h >= a.heads) continue;
+        pa_bf16 *out = reinterpret_cast<pa_bf16 *>(a.out) + ((p.row0 + row) * a.heads + h) * a.vdim;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) {
+                const f16 x = o[i][c];
+                const int d = col0 + 32 * c + 2 * e + 4 * side;
+                if (d >= a.vdim) continue;
+                if (FULL || a.vdim % 4 == 0) {
+                    *reinterpret_cast<uint2 *>(out + d) = make_uint2(row_pack_bf16(x[e], x[e + 1]), row_pack_bf16(x[e + 2], x[e + 3]));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (d + j < a.vdim) pa_scalar<pa_bf16>::store(out + d + j, x[e + j]);
+                }
+            }
+    }
+}
+
+template <int DK, int DV, int G, bool FULL> int launch_pipe(const TalkArgs &a, hipStream_t s) {
+    constexpr size_t lds = TpTile<DV, G>::bytes;
+    static_assert(lds <= 160 * 1024 / (4 / G), "LDS of one compute unit");
+    if (int rc = la_big_lds(talk_pipe_kernel<DK, DV, G, FULL>, lds, "pa_talking_attention")) return rc;
+    const int64_t blocks = (int64_t)a.batch * ((a.max_q_len + kTpRows - 1) / kTpRows), side = (int64_t)la_cus() * (4 / G);
+    PA_REQUIRE(blocks <= 0x7fffffff, "pa_talking_attention: batch=%d, max_q_len=%d are too many rows for one launch", a.batch, a.max_q_len);
+    TalkArgs args = a;
+    args.at_once = (unsigned)side;
+    talk_pipe_kernel<DK, DV, G, FULL><<<dim3((unsigned)blocks), dim3(TpTile<DV, G>::threads), lds, s>>>(args);
+    PA_CHECK_LAUNCH("pa_talking_attention (portions)");
+    return PA_OK;
+}
+template <int DK, int DV> int launch_pipe_size(const TalkArgs &a, hipStream_t s) {
+    const bool full = a.n1 == DK && a.vdim == DV;
+    if (a.heads <= 8) return full ? launch_pipe<DK, DV, 2, true>(a, s) : launch_pipe<DK, DV, 2, false>(a, s);
+    return full ? launch_pipe<DK, DV, 4, true>(a, s) : launch_pipe<DK, DV, 4, false>(a, s);
+}
+
 template <int D, int HW, bool FULL, int NG> int launch_mix(const TalkArgs &a, hipStream_t s) {
     constexpr size_t lds = TmTile<D, HW, NG>::bytes;
     static_assert(lds <= 160 * 1024, "LDS of one compute unit");
@@ -543,6 +895,10 @@ bool pa_talking_prefill_launch(const TalkArgs &a, int dtype, hipStream_t s, int 
         if (a.n1 <= 64) talk_sums_kernel<64><<<grid, dim3(256), 0, s>>>(a);
         else talk_sums_kernel<128><<<grid, dim3(256), 0, s>>>(a);
         PA_CHECK_LAUNCH("pa_talking_attention (sums)");
+        if (a.heads <= 16 && a.n_rep % 4 == 0 && (a.heads <= 8 || a.bt_stride * a.bs > kTpShort) && (int64_t)a.hkv * (a.k_dim > a.v_dim ? a.k_dim : a.v_dim) < (1 << 30)) {
+            if (a.n1 <= 64) return a.vdim <= 64 ? launch_pipe_size<64, 64>(a, s) : launch_pipe_size<64, 128>(a, s);
+            return a.vdim <= 64 ? launch_pipe_size<128, 64>(a, s) : launch_pipe_size<128, 128>(a, s);
+        }
         if (a.heads <= 16) return most <= 64 ? launch_mix_size<64, 2>(a, s) : launch_mix_size<128, 2>(a, s);
         return most <= 64 ? launch_mix_size<64, 4>(a, s) : launch_mix_size<128, 4>(a, s);
     }();

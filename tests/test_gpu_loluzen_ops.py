@@ -179,6 +179,17 @@ def test_prompts_of_many_tiles(heads, kv, dim, vdim):
     case.check([(1, 254, 51), (0, 250, 7), (3, 287, 2)])
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(16, 4, 128, 128), (12, 3, 72, 120), (12, 1, 64, 128), (8, 2, 64, 64), (4, 1, 104, 24), (8, 1, 128, 128)])
+def test_prompts_with_more_blocks_of_rows_than_workgroups_side_by_side(heads, kv, dim, vdim):
+    """Kernels with waves of two kinds: 16 rows each, one to ten tiles of keys, in order of their keys over more than 64 portions."""
+    announce(f"talking blocks {heads} {kv} {dim} {vdim}")
+    lens = [300, 16, 33, 129, 161]
+    case = Talking(lens, heads, kv, dim, vdim, BF, seed=11, odd_talk=True).solve()
+    case.check([(i % 5, 0, lens[i % 5]) for i in range(70)])
+    case.check([(i % 5, lens[i % 5] - 1 - i % 3, 1 + i % 3) for i in range(600)])
+    case.check([(0, 283, 17), (4, 160, 1)])
+
+
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 64), (20, 4, 48, 72)])
 def test_long_decode_steps_run_in_pieces(heads, kv, dim, vdim):
     """One or two sequences of a few thousand tokens: their keys are spread over the device in up to sixteen pieces."""
