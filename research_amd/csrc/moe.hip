@@ -414,7 +414,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_tile_kernel(const MoeArgs
     const int l16 = lane & 15, g = lane >> 4;
     int expert, m0, count;
     if (!moe_tile(a, i / n_tiles, kBM, lane, expert, m0, count)) return;
-    const int n0 = i % n_tiles * kOut;
+    // (an expert's row tiles of the same outputs one after the other, which read the same weights: 16 experts of 2048 x 768 and 1296 items 76.8 us a
+    // layer with its outputs one after the other, 73.4 so)
+    const int rows = (count + kBM - 1) / kBM, local = m0 / kBM * n_tiles + i % n_tiles, n0 = local / rows * kOut;
+    m0 = local % rows * kBM;
     // sources of this lane's chunks
     const int r16 = lane / 4, ch = (lane % 4) ^ ((r16 >> 1) & 3);
     const uint16_t *x = reinterpret_cast<const uint16_t *>(a.x), *w = reinterpret_cast<const uint16_t *>(a.w) + expert * a.w_rows * a.kp;
@@ -542,10 +545,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
     struct Tile {
         int expert, m0, count, n0;
     };
+    // (An expert's row tiles of the same outputs one after the other: a die's units read the same weights at the same time, and an expert's items
+    // come from its cache again.  With the outputs one after the other, 64 experts of 4096 x 1408 and 48008 items: misses of the second level 28 and 13
+    // million lines instead of 32 and 20, products 962 and 576 us instead of 1011 and 603.)
     auto look_up = [&](int tile) {
         Tile t;
         const int rt = tile / n_tiles;
-        t.n0 = (tile - rt * n_tiles) * kOut;
         t.expert = 0;
         for (int e0 = 0; e0 < a.experts; e0 += 64) {
             const int e = e0 + lane, upto = e < a.experts ? upto_s[e] : 0x7fffffff;
@@ -557,7 +562,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_stay_kernel(const MoeArgs
         }
         t.expert = __builtin_amdgcn_readfirstlane(t.expert);
         const int before = t.expert > 0 ? upto_s[t.expert - 1] : 0;
-        t.m0 = __builtin_amdgcn_readfirstlane((rt - before) * kBM);
+        const int local = tile - before * n_tiles, rows = upto_s[t.expert] - before;
+        t.n0 = __builtin_amdgcn_readfirstlane(local / rows * kOut);
+        t.m0 = __builtin_amdgcn_readfirstlane(local % rows * kBM);
         t.count = a.counts[t.expert];
         return t;
     };
