@@ -196,7 +196,7 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 
 // How decode_short.h's kernel takes the launch: 0: not at all; else the runs a sequence's tiles are cut into, a workgroup per (kv head, sequence,
 // run).  From shapes alone; the tables' width stands for the longest sequence.
-// Head sizes up to 32 stay with the generic loop of the split pass, whose weights have 32 bits: 11.8 us for 16 sequences of 16 .. 250 keys, 4 / 4
+// Head sizes up to 32 over 16 bits and fp8 stay with the generic loop of the split pass, whose weights have 32 bits: 11.8 us for 16 sequences of 16 .. 250 keys, 4 / 4
 // heads of 32, where weights of two bf16 terms took 5.0, but erred by up to 1.1e-6 of the sum of |weight value| where 32 bits err by 0.2e-6.
 // Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (3.5 us: 600 keys of 128).
 // us, the split pass (one launch or two) -> this, sequences of n keys each: 32 / 8 heads of 128, 1 of 256 keys 14.1 -> 7.4, 1024 15.5 -> 9.0, 4096
@@ -210,35 +210,54 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // 44.8 -> 47.4, 1024 33 -> 27; equal, 256 of 512 90 -> 94.  One or two query heads a kv head: 16 / 8 of 256, 16 of 1024 19.5 -> 24; 8 / 8 of 64, 3 of
 // 8192 18 -> 24; over fp8, where the kernel's conversions count, 8 / 8 of 64, 3 of 8064 in runs of 806 keys 12.7 -> 15.0, 32 / 16, 66 of 917 38 -> 51.
 // 8 / 2 of 128, 1 of 8192 14.6 -> 15.2, 4096 14 -> 12.
+// 32-bit pools, the split pass -> this: from five query heads a kv head on always (runs of up to 2 MB, as far as measured, but for 16 / 2 of 64 and the like, 1 of 81903 30 -> 33: the split pass spends a vector
+// instruction on every head, key and element; 14 / 2 of 72, 105 of 34 .. 127 keys 26.7 -> 8.1, 16 / 2 of 128, 102 of 236 51 -> 24, 23 of 6812 86 -> 57, 1 of 20000 at 24 /
+// 2 37 -> 26).  Three or four: up to 48 MB of keys (32 / 8 of 64, 4 of 155 14.5 -> 8.2, 8 / 2 of 128, 29 of 819 20 -> 17; beyond, unequal, 32 / 8 of 128,
+// 7 of 33764 160 -> 340), unless more than four rounds of workgroups have few keys each (32 / 8 of 64, 206 of 53 13.4 -> 15.0; at 256 more than one, 8 / 2, 163 of 138 21 -> 26) or the few there are
+// have long runs (8 / 2 of 128, 2 of 4000 15.6 -> 18.1, of 64, 8 of 6831 16.5 -> 18.2; of 256, 2 of 1964 17.6 -> 18.6).  One or two: a run each, up to 32 MB
+// and two rounds (16 / 8 of 128, 1 of 176 12.5 -> 8.6, 60 of 201 31 -> 21; 187 of 21 13.4 -> 18.1, 8 / 8 of 64, 16 of 600 14.5 -> 15.2).  A run is cut where four
+// turns of the waves, at 256 two, take longer than a merging launch: 16 keys of 128 each in 1 us (14 / 2 of 256, 6 of 228 in one run 20.7, of 64 keys 16.4, of
+// 32 11.9; 14 / 2 of 128, 16 of 101 8.2, in three 9.4); where most units have a workgroup anyway into two runs a unit, from five heads on four (unequal:
+// 14 / 2 of 72, 140 of 1600 71 -> 78, with four 50; equal 116 -> 100, 77).
+// (Over 740 drawn batches over 32-bit pools the two took 0.71 of the time that the split pass took alone.)
 // (Over 1200 shapes of 1 .. 128 sequences that this takes, from 600 keys of 128 on, equal and unequal, 16 of 3600 batches were slower by more than 2 %, of which 4 / 4 heads of 96
 // over fp8 by up to 19, 30 of 1482 keys 15.6 -> 18.6, the others by up to 6; on average they took 0.55 of the split pass's time.)
 constexpr int kPlanShortHeads = 16, kPlanShortTile = 16, kPlanShortRuns = 64;
 PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, int kv_elem_bytes, int64_t table_blocks, int block_size, int window, int cus) {
-    if (block_size % kPlanShortTile != 0 || batch > kPlanWaveScanBatch || h.hkv > 65535 || h.d_pad < 64) return 0;
+    if (block_size % kPlanShortTile != 0 || batch > kPlanWaveScanBatch || h.hkv > 65535 || (h.d_pad < 64 && kv_elem_bytes < 4)) return 0;
     const int64_t span = plan_window_span(window);
     if (span > 0 && span / block_size + 2 < table_blocks) table_blocks = span / block_size + 2;
     const int64_t keys = table_blocks * block_size, reps = (h.n_rep + kPlanShortHeads - 1) / kPlanShortHeads, wgs = (int64_t)h.hkv * batch * reps;
     int64_t runs = 1;
-    const bool brief = keys * h.d_pad <= 600 * 128;
+    const bool f32 = kv_elem_bytes == 4;
+    const int64_t d = h.d_pad < 64 ? 64 : h.d_pad, least = f32 ? 64 * 128 / d : 128;  // (least: keys of a run)
+    const bool brief = keys * d <= (f32 ? 256 : 600) * 128;
     if (!brief) {
-        runs = 4 * wgs <= cus ? cus / wgs : 3 * (int64_t)cus / 2 / wgs;  // (few more workgroups than units are as slow as twice as many)
-        if (runs > keys / 128) runs = keys / 128;
+        runs = 4 * wgs <= cus ? cus / wgs : (!f32 ? 3 : h.n_rep > 4 ? 8 : 4) * (int64_t)cus / 2 / wgs;  // (few more workgroups than units are as slow as twice as many)
+        if (runs > keys / least) runs = keys / least;
         if (runs > kPlanShortRuns) runs = kPlanShortRuns;
         const int64_t room = w.slots * h.heads_per_slot() / ((int64_t)batch * h.hq);  // (their results are as long as a slot's)
         if (runs > room) runs = room;
         if (runs < 1) runs = 1;
     }
-    const int64_t row = (int64_t)h.d_pad * kv_elem_bytes, kb = 1024;
+    const int64_t row = d * kv_elem_bytes, kb = 1024;
     const int64_t wide_most = row > 128 || h.hpw == 4 ? 256 * kb : h.hpw == 1 ? 512 * kb : h.hpw == 2 ? 384 * kb : 208 * kb;
     const int64_t run_most = h.n_rep > 4 ? (kv_elem_bytes == 1 ? 4096 * row : wide_most) : h.n_rep > 2 ? 128 * kb : 64 * kb;
     const int64_t all_most = h.n_rep > 4 ? (int64_t)1 << 62 : (h.n_rep > 2 ? 64 : 32) * kv_elem_bytes * kb * kb;
     const bool few = h.n_rep <= 4 && wgs < 6 && keys > 4096;
+    if (f32) {
+        const bool lone = keys > 3072 ? wgs < (d == 64 ? 24 : 6) : d == 256 && !brief && wgs < 8;
+        const bool fits = h.n_rep > 4   ? d > 64 || wgs >= 6 || keys <= 8192
+                          : h.n_rep > 2 ? !lone && wgs <= (d == 256 ? 1 : 4) * (int64_t)cus && wgs * keys * row <= 48 * kb * kb
+                                        : d < 256 && brief && wgs <= 2 * (int64_t)cus && wgs * keys * row <= 32 * kb * kb;
+        return fits && keys / runs * row <= 2048 * kb && runs * reps <= 65535 ? (int)runs : 0;
+    }
     const bool thin = kv_elem_bytes == 1 && h.d_pad == 64 && h.n_rep <= 2 && keys / runs > 768;
     const bool fits = (brief || keys / runs * row <= run_most) && wgs * keys * row <= all_most && !few && !thin;
     return fits && runs * reps <= 65535 ? (int)runs : 0;
 }
 
-// Of what the split pass still has (32-bit pools, heads of up to 32, blocks that are no whole tiles, large batches of 16-bit ones): whether the
+// Of what the split pass still has (the larger calls over 32-bit pools, heads of up to 32, blocks that are no whole tiles, large batches of 16-bit ones): whether the
 // block tables are so narrow that a workgroup takes a whole (plane, sequence): nothing is left to merge then, and the second launch (4 us, and its
 // gap) goes.  A workgroup is a chain of waits, 1 to 2 us for each block that a wave takes (for a tile of 16 keys of longer ones), 2 to 4 us where
 // eight query heads a kv head meet fp8 values or the generic loop, so the line lies where the chain takes as long as the second launch and what

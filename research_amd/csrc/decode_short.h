@@ -1,4 +1,4 @@
-// Decode over narrow block tables (16-bit queries over 16-bit or fp8 pools, heads of more than 32): a workgroup per (kv head, sequence), or several with a merge behind
+// Decode over narrow block tables (pools of 16 or 32 bits, or fp8 under 16-bit queries with heads of more than 32): a workgroup per (kv head, sequence), or several with a merge behind
 // them (plan_short_splits of decode_plan.h: where, how many, and what they measured).
 //
 // Short sequences are bound by waits and by the instructions that a workgroup fetches once, not by bytes: the split pass, whose loop is unrolled
@@ -11,6 +11,13 @@
 // one (error against 64 bits, 14 / 2 heads of 64, 8 sequences of 94 .. 683 keys: split pass 1.78e-3, one term 2.06e-3, two 1.67e-3).
 // Over fp8 pools a weight meets its block's scale, and the terms are of bf16 whatever the queries are: fp16 has no room for small scales (fp16
 // queries, those sequences, terms of fp16 -> bf16: 2.071e-4 -> 2.069e-4, with values of 0.001 instead of one 1.0e-2 -> 2.4e-4).
+// Over 32-bit pools both products are of 32-bit operands (16x16x4), a load's four elements one after the other, and nothing goes through LDS: with
+// the rows 4 g + i of V as the i-th operand, S's layout is again P's, and a lane's 16 bytes of a row of V are operands of four tiles of columns.
+// Each sum is a tree over sums of eight (logits) and of four terms (values): in one chain, as the accumulators offer it, errors against 64
+// bits were 1.9 times the split pass's (14 / 2 heads of 64), in trees they are 0.95 of them (0.81 .. 1.04 over 16 kinds of batches).  What bounds it is the
+// matrix unit's rate for these operands, 1024 cycles for 16 keys of 64 (0.9 us with 128), and the chain of waits: the queries of 256 wait in LDS, as registers
+// for two waves a SIMD let a second workgroup's loads fly meanwhile; at 128 three waves spill.  us, the split pass -> this: 14 / 2 heads of 64, 5
+// sequences of 38 keys 11.8 -> 5.8; 8 / 2 of 128, 19 of 61 11.2 -> 5.9; 14 / 2 of 256, 28 of 195 26.5 -> 13.
 // Waves take tiles of 16 keys in turn, two at a time up to 64 elements a row; their sums meet in LDS with two barriers.  One tile at a time at
 // 128 leaves registers for four workgroups a compute unit: 256 sequences of 16 keys, 32 / 8 heads, 16.1 -> 9.0 us.
 #pragma once
@@ -50,6 +57,13 @@ template <> struct ShortMfma<pa_f16> {
     }
 };
 
+template <> struct ShortMfma<float> {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ f4 mul(uint32_t a, uint32_t b, f4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b), c, 0, 0, 0);
+    }
+};
+
 constexpr int kShortHeads = kPlanShortHeads, kShortKeys = kPlanShortTile;  // query heads of a workgroup, keys of a tile
 
 // Four consecutive outputs (rows are multiples of 16 bytes long; the first need not lie on one of 8).
@@ -58,29 +72,36 @@ template <typename QT, typename Num> __device__ __forceinline__ void short_store
     float y[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) y[i] = finish_row(num[i], best, den, ez);
-    if (((uintptr_t)to & 7u) == 0) {
-        *reinterpret_cast<uint2 *>(to) = make_uint2(M::pack(y[0], y[1]), M::pack(y[2], y[3]));
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pa_scalar<QT>::store(to + i, y[i]);
+    if constexpr (sizeof(QT) == 2) {
+        if (((uintptr_t)to & 7u) == 0) {
+            *reinterpret_cast<uint2 *>(to) = make_uint2(M::pack(y[0], y[1]), M::pack(y[2], y[3]));
+            return;
+        }
+    } else if (((uintptr_t)to & 15u) == 0) {
+        *reinterpret_cast<float4 *>(to) = make_float4(y[0], y[1], y[2], y[3]);
+        return;
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pa_scalar<QT>::store(to + i, y[i]);
 }
 
 // Blocks are whole tiles (block_size % 16 == 0).
 // A workgroup has one of a.splits equal runs of its sequence's tiles and, with a.leave, leaves the maximum, sum and unnormalised outputs of its
 // keys for the merge.
-template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void decode_short_kernel(const DecodeArgs a) {
+template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads, D == 256 || (sizeof(KV) == 4 && D == 128) ? 2 : sizeof(KV) == 4 ? 3 : 4) void decode_short_kernel(const DecodeArgs a) {
     using M = ShortMfma<QT>;
-    constexpr bool kFp8 = sizeof(KV) == 1;
+    constexpr bool kFp8 = sizeof(KV) == 1, k32 = sizeof(KV) == 4;
     using VT = std::conditional_t<kFp8, pa_bf16, QT>;  // the second product's type (fp8 values are exact in either)
     using W = ShortMfma<VT>;
     using f4 = typename M::f4;
-    constexpr int EL = 16 / sizeof(KV), KL = D / (4 * EL);  // elements of a 16-byte load; loads of a tile of K, and of V
-    constexpr int NT = D >= 128 ? 1 : 2;                    // tiles at a time (registers for four waves a SIMD, at 256 two)
+    constexpr int EL = 16 / sizeof(KV), KL = D / (4 * EL), QL = EL == 16 ? 2 : 1;  // elements of a 16-byte load; loads of a tile of K, and of V; of a query for each
+    constexpr int NT = D >= 128 ? 1 : 2;                    // tiles at a time (registers for four waves a SIMD, at 256 two; 32 bits: for three and two)
     constexpr int kPitch = D + 16;                          // (four rows of a transposing read lie 32 bytes apart modulo 64)
     constexpr int HR = D == 256 ? 8 : kShortHeads, kPitchO = D + 4;  // heads merged at a time
-    constexpr int kBytesV = kWaves * NT * kShortKeys * kPitch * 2, kBytesO = kWaves * HR * kPitchO * 4;
+    constexpr int kBytesV = k32 ? 0 : kWaves * NT * kShortKeys * kPitch * 2, kBytesO = kWaves * HR * kPitchO * 4;
     __shared__ __align__(16) char room[kBytesV > kBytesO ? kBytesV : kBytesO];
+    constexpr bool kLdsQ = k32 && D == 256;  // the queries are read from LDS: registers for two waves a SIMD
+    __shared__ pa_u4 s_q[kLdsQ ? KL : 1][64];
     __shared__ float s_m[kWaves][kShortHeads], s_l[kWaves][kShortHeads];
     const PoolArgs &p = a.p;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
@@ -98,20 +119,28 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
     const int L = a.seq_lens[b];
     QT *orow = reinterpret_cast<QT *>(a.out) + ((int64_t)b * p.hq + kvh * p.n_rep + rep0) * p.d;
     // queries: lane l16 has head rep0 + l16, the elements of its loads of K
-    pa_u4 qr[KL][EL / 8];
+    pa_u4 qr[kLdsQ ? KL / kWaves : KL][QL];
     {
         const QT *qp = reinterpret_cast<const QT *>(a.q) + ((int64_t)b * p.hq + kvh * p.n_rep + rep0 + (l16 < nr ? l16 : 0)) * p.d;
 #pragma unroll
-        for (int j = 0; j < KL; ++j)
+        for (int j = 0; j < (kLdsQ ? KL / kWaves : KL); ++j)
 #pragma unroll
-            for (int e = 0; e < EL / 8; ++e) {
-                const int d = EL * (4 * j + g) + 8 * e;
+            for (int e = 0; e < QL; ++e) {
+                const int d = EL * (4 * (kLdsQ ? wave * (KL / kWaves) + j : j) + g) + 8 * e;
                 qr[j][e] = l16 < nr && d < p.d ? *reinterpret_cast<const pa_u4 *>(qp + d) : pa_u4{0, 0, 0, 0};
             }
     }
     if (L <= 0 && !a.leave) {  // uniform
         for (int i = tid; i < nr * p.d; i += kThreads) pa_scalar<QT>::store(orow + i, 0.f);
         return;
+    }
+    if constexpr (kLdsQ) {
+#pragma unroll
+        for (int j = 0; j < KL / kWaves; ++j) s_q[wave * (KL / kWaves) + j][lane] = qr[j][0];
+        __syncthreads();
+    } else if constexpr (k32) {
+#pragma unroll
+        for (int j = 0; j < KL; ++j) asm volatile("" : "+v"(qr[j][0]));  // (waits for them here: in the loop for K alone)
     }
     const int ez = a.extra_zero ? max(0, a.extra_zero[b]) : 0;
     const int k_lo = plan_first_key(L, p.window);
@@ -125,7 +154,7 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
     uint16_t *vs = reinterpret_cast<uint16_t *>(room) + wave * NT * kShortKeys * kPitch;
 
     float m, l;
-    f4 acc[D / 16];  // O^T: d = 16 dt + 4 g + i, head l16
+    f4 acc[D / 16];  // O^T: d = 16 dt + 4 g + i (32 bits: 64 (dt / 4) + 16 g + 4 i + dt % 4), head l16
     pa_u4 kr[NT][KL], vr[NT][KL];
     float kscale = 1.f, vscale = 1.f;  // of tile `lane` of the 64 at hand
     // An infinite value times a weight's second term, which is zero or negative as often as not, makes a sum NaN that is infinite.  So a wave whose
@@ -147,7 +176,9 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                 kscale = bids >= 0 ? p.k_scale[at] : 1.f;
                 vscale = bids >= 0 ? p.v_scale[at] : 1.f;
             }
-            auto fetch = [&](int at) {
+            auto fetch = [&](int at, bool keys, bool values) {  // (constants)
+                int at16 = l16, at4 = g;
+                if constexpr (k32) asm volatile("" : "+v"(at16), "+v"(at4));  // (the offsets of 32 loads are not kept over the loop)
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const int tile = tile0 + at + t, bid = at + t < n ? __builtin_amdgcn_readlane(bids, at + t) : -1;
@@ -158,24 +189,39 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                     const __amdgpu_buffer_rsrc_t k = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.k) + slot), 0, bytes, 0x00020000);
                     const __amdgpu_buffer_rsrc_t v = __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(p.v) + slot), 0, bytes, 0x00020000);
 #pragma unroll
-                    for (int j = 0; j < KL; ++j) {
-                        const int d = EL * (4 * j + g);
-                        kr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(k, d < p.d ? l16 * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
+                    for (int j = 0; j < (keys ? KL : 0); ++j) {
+                        const int d = EL * (4 * j + at4);
+                        kr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(k, d < p.d ? at16 * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
                     }
 #pragma unroll
-                    for (int j = 0; j < KL; ++j) {
-                        const int c = lane + 64 * j, row = c / (D / EL), d = c % (D / EL) * EL;
+                    for (int j = 0; j < (values ? KL : 0); ++j) {
+                        const int c = lane + 64 * j, row = k32 ? 4 * at4 + j / (D / 64) : c / (D / EL), d = k32 ? 64 * (j % (D / 64)) + 4 * at16 : c % (D / EL) * EL;
                         vr[t][j] = __builtin_amdgcn_raw_buffer_load_b128(v, d < p.d && row >= skip ? row * tok + head + d * (int)sizeof(KV) : kDeadLaneOffset, 0, kStreamPolicy);
                     }
                 }
             };
-            if (wave * NT < n) fetch(wave * NT);
+            if (wave * NT < n) fetch(wave * NT, true, true);
 #pragma unroll 1
             for (int at = wave * NT; at < n; at += kWaves * NT) {
+                if constexpr (kLdsQ) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (else they are kept over the loop)
                 float x[NT][4], mx = m;
+                f4 raw[NT];
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    f4 s = f4{0.f, 0.f, 0.f, 0.f};
+                    f4 s = f4{0.f, 0.f, 0.f, 0.f}, odd[6], last[2];
+                    // Adds the j-th of the terms of a logit to the sums of two, of four ... of them: the whole sum behind the last one.
+                    auto tree = [&](int j, f4 y) {
+#pragma unroll
+                        for (int level = 0; level < 6; ++level) {
+                            asm volatile("" : "+v"(y));  // (now)
+                            if (!(j >> level & 1)) {
+                                odd[level] = y;
+                                break;
+                            }
+                            y = odd[level] + y;
+                        }
+                        return y;
+                    };
 #pragma unroll
                     for (int j = 0; j < KL; ++j) {
                         if constexpr (kFp8) {
@@ -183,11 +229,24 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                             PoolWords<KV, QT>::unpack(kr[t][j], w);
                             s = M::mul(pa_u4{w[0], w[1], w[2], w[3]}, qr[j][0], s);
                             s = M::mul(pa_u4{w[4], w[5], w[6], w[7]}, qr[j][1], s);
+                        } else if constexpr (k32) {
+                            pa_u4 qj;
+                            if constexpr (kLdsQ) qj = s_q[j][lane];
+                            else qj = qr[j][0];
+                            const f4 none = f4{0.f, 0.f, 0.f, 0.f};
+                            const f4 u = M::mul(kr[t][j][1], qj[1], M::mul(kr[t][j][0], qj[0], none));
+                            const f4 w = M::mul(kr[t][j][3], qj[3], M::mul(kr[t][j][2], qj[2], none));
+                            if (j > 0) tree(j - 1, last[0] + last[1]);
+                            last[0] = u;
+                            last[1] = w;
+                            if (j == KL - 1) s = tree(j, u + w);
+                            __builtin_amdgcn_sched_barrier(0);  // (products in order need few registers)
                         } else {
                             s = M::mul(kr[t][j], qr[j][0], s);
                         }
                     }
                     const int lim = at + t < n ? L - (tile0 + at + t) * kShortKeys : 0, lo = k_lo - (tile0 + at + t) * kShortKeys;
+                    raw[t] = s;
                     float f = p.scale_log2;
                     if constexpr (kFp8) f *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, kscale), (at + t) & 63));
 #pragma unroll
@@ -197,7 +256,7 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                     }
                     // V, for the transposing reads
 #pragma unroll
-                    for (int j = 0; j < KL; ++j) {
+                    for (int j = 0; j < (k32 ? 0 : KL); ++j) {
                         const int c = lane + 64 * j, row = t * kShortKeys + c / (D / EL), d = c % (D / EL) * EL;
                         pa_u4 *to = reinterpret_cast<pa_u4 *>(vs + row * kPitch + d);
                         if constexpr (kFp8) {
@@ -210,7 +269,8 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                         }
                     }
                 }
-                if (at + kWaves * NT < n) fetch(at + kWaves * NT);
+                // (32 bits: behind the last tiles too, of no bytes: where both are without a condition, K's products wait for K alone)
+                if (k32 || at + kWaves * NT < n) fetch(at + kWaves * NT, true, !k32);
                 {
                     const float2 y = lane_pair<16>(mx, 16);
                     mx = fmaxf(y.x, y.y);
@@ -220,46 +280,76 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                 const float alpha = __builtin_amdgcn_exp2f(m - mx);
                 m = mx;
                 l *= alpha;
-                uint32_t pw[4] = {0, 0, 0, 0}, pl[4] = {0, 0, 0, 0};  // the weights as a sum of two terms
+                if constexpr (k32) {
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    float e[4], f = 1.f;
-                    if constexpr (kFp8) f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vscale), (at + t) & 63));
+                    for (int t = 0; t < NT; ++t)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        e[i] = __builtin_amdgcn_exp2f(x[t][i] - m);  // 0 for masked keys
-                        l += e[i];
-                        if constexpr (kFp8) e[i] *= f;
+                        for (int i = 0; i < 4; ++i)
+                            x[t][i] = x[t][i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(raw[t][i], p.scale_log2, -m));
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) l += (x[t][0] + x[t][1]) + (x[t][2] + x[t][3]);
+                    f4 sum[2][4];  // (of the 16 keys and columns at hand, and of those before)
+#pragma unroll
+                    for (int c = 0; c <= D / 16 * NT; ++c) {
+                        if (c < D / 16 * NT) {
+                            const int t = c % NT, dt = c / NT;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                sum[c & 1][i] = M::mul(vr[t][i * (D / 64) + dt / 4][dt % 4], __builtin_bit_cast(uint32_t, x[t][i]), f4{0.f, 0.f, 0.f, 0.f});
+                        }
+                        if (c > 0) {
+                            const int dt = (c - 1) / NT;
+                            const f4(&u)[4] = sum[~c & 1], y = (u[0] + u[1]) + (u[2] + u[3]);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[dt][i] = (c - 1) % NT == 0 ? fmaf(acc[dt][i], alpha, y[i]) : acc[dt][i] + y[i];
+                            asm volatile("" : "+v"(acc[dt]));
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
+                    fetch(at + kWaves * NT, false, true);
+                    continue;
+                } else {
+                    uint32_t pw[4] = {0, 0, 0, 0}, pl[4] = {0, 0, 0, 0};  // the weights as a sum of two terms
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        pw[2 * t + i] = W::pack(e[2 * i], e[2 * i + 1]);
-                        const float2 high = W::unpack(pw[2 * t + i]);
-                        pl[2 * t + i] = W::pack(e[2 * i] - high.x, e[2 * i + 1] - high.y);
+                    for (int t = 0; t < NT; ++t) {
+                        float e[4], f = 1.f;
+                        if constexpr (kFp8) f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vscale), (at + t) & 63));
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            e[i] = __builtin_amdgcn_exp2f(x[t][i] - m);  // 0 for masked keys
+                            l += e[i];
+                            if constexpr (kFp8) e[i] *= f;
+                        }
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            pw[2 * t + i] = W::pack(e[2 * i], e[2 * i + 1]);
+                            const float2 high = W::unpack(pw[2 * t + i]);
+                            pl[2 * t + i] = W::pack(e[2 * i] - high.x, e[2 * i + 1] - high.y);
+                        }
                     }
-                }
-                const pa_u4 pb{pw[0], pw[1], pw[2], pw[3]}, pc = again ? pb : pa_u4{pl[0], pl[1], pl[2], pl[3]};
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
+                    const pa_u4 pb{pw[0], pw[1], pw[2], pw[3]}, pc = again ? pb : pa_u4{pl[0], pl[1], pl[2], pl[3]};
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int dt = 0; dt < D / 16; ++dt) {
-                    typedef short s4 __attribute__((ext_vector_type(4)));
-                    auto column = [&](int t) {
-                        uint16_t *from = vs + (t * kShortKeys + 4 * g + l16 / 4) * kPitch + 16 * dt + 4 * (l16 % 4);
-                        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *)from));
-                    };
-                    const uint2 v0 = column(0), v1 = NT == 2 ? column(1) : make_uint2(0, 0);
+                    for (int dt = 0; dt < D / 16; ++dt) {
+                        typedef short s4 __attribute__((ext_vector_type(4)));
+                        auto column = [&](int t) {
+                            uint16_t *from = vs + (t * kShortKeys + 4 * g + l16 / 4) * kPitch + 16 * dt + 4 * (l16 % 4);
+                            return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *)from));
+                        };
+                        const uint2 v0 = column(0), v1 = NT == 2 ? column(1) : make_uint2(0, 0);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
-                    const pa_u4 v{v0.x, v0.y, v1.x, v1.y};
-                    acc[dt] = W::mul(v, pb, acc[dt]);
-                    acc[dt] = W::mul(v, pc, acc[dt]);
+                        for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
+                        const pa_u4 v{v0.x, v0.y, v1.x, v1.y};
+                        acc[dt] = W::mul(v, pb, acc[dt]);
+                        acc[dt] = W::mul(v, pc, acc[dt]);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
             }
         }
-        if constexpr (kFp8) break;  // (that type has no infinities)
+        if constexpr (kFp8 || k32) break;  // (that type has no infinities; one weight of 32 bits)
         f4 odd = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) odd += acc[dt] * 0.f;
@@ -287,8 +377,12 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
         if (h0 > 0) __syncthreads();
         if (l16 >= h0 && l16 < min(h0 + HR, nr)) {
 #pragma unroll
-            for (int dt = 0; dt < D / 16; ++dt)
-                *reinterpret_cast<f4 *>(part + (wave * HR + l16 - h0) * kPitchO + 16 * dt + 4 * g) = f4{acc[dt][0] * mine, acc[dt][1] * mine, acc[dt][2] * mine, acc[dt][3] * mine};
+            for (int dt = 0; dt < D / 16; ++dt) {
+                f4 y = acc[dt];
+                if constexpr (k32) y = f4{acc[dt / 4 * 4][dt % 4], acc[dt / 4 * 4 + 1][dt % 4], acc[dt / 4 * 4 + 2][dt % 4], acc[dt / 4 * 4 + 3][dt % 4]};
+                const int d = k32 ? 64 * (dt / 4) + 16 * g + 4 * (dt % 4) : 16 * dt + 4 * g;
+                *reinterpret_cast<f4 *>(part + (wave * HR + l16 - h0) * kPitchO + d) = f4{y[0] * mine, y[1] * mine, y[2] * mine, y[3] * mine};
+            }
         }
         __syncthreads();
         const int heads = min(HR, nr - h0);
@@ -360,7 +454,7 @@ template <typename QT> __global__ __launch_bounds__(kThreads) void decode_short_
 template <typename KV, typename QT> KernelSet with_short(KernelSet k, int d) {
     if (!k.split) return k;
     k.few_merge = decode_short_merge_kernel<QT>;
-    if (d == 64) k.few = decode_short_kernel<KV, QT, 64>;
+    if (d == 64 || (d == 32 && sizeof(KV) == 4)) k.few = decode_short_kernel<KV, QT, 64>;
     if (d == 128) k.few = decode_short_kernel<KV, QT, 128>;
     if (d == 256) k.few = decode_short_kernel<KV, QT, 256>;
     return k;

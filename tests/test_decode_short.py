@@ -148,3 +148,60 @@ def test_rows_that_are_not_seen_do_not_matter():
             call = lambda a, b: ops.decode(q, a.to(DEV), b.to(DEV), tables[:1].to(DEV), torch.tensor([n[i]], dtype=torch.int32, device=DEV), 16, 0.125,
                                            ops.decode_workspace(q, a.to(DEV)), window=window)
             assert torch.equal(call(kk, vv), call(k, v))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,hq,hkv,d,window,bs", [
+    (EDGES, 14, 2, 64, 0, 16), (EDGES, 32, 8, 128, 50, 16), (EDGES, 8, 2, 72, 0, 48), (EDGES, 4, 4, 32, -64, 16), (EDGES, 6, 2, 8, 0, 16),
+    (EDGES, 20, 1, 96, 0, 32), (EDGES, 36, 2, 128, 0, 16), (EDGES, 14, 2, 256, 33, 16), (EDGES, 6, 2, 192, 0, 16), ([1300, 2047, 1, 0, 16], 32, 8, 128, 0, 16),
+    ([4000, 129, 128], 14, 2, 64, 0, 16), ([1025, 700, 64, 3], 14, 2, 256, 0, 16), ([2500, 1200], 18, 1, 128, -1300, 16), ([1500, 40], 8, 2, 40, 0, 16),
+])
+def test_pools_of_32_bits(plan, lens, hq, hkv, d, window, bs):
+    """The same edges over 32-bit pools, with rows out of sight that are NaN or infinite; errors against 64 bits beside the split pass's."""
+    from oracle import paged_oracle as po
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce, assert_close, decode_by_split_pass, tables_to_device
+    from tests.test_gpu_decode_merge import Batch
+
+    announce(f"decode short, 32 bits: {len(lens)} x {max(lens)} {hq}/{hkv}x{d} window {window} blocks of {bs}")
+    b = Batch(lens, hq, hkv, d, "f32", seed=len(lens) + d, bs=bs)
+    (k, v, _, _), (kr, vr) = b.device_pools()
+    tables = tables_to_device(b.tables)
+    assert plan.runs(len(lens), hq, hkv, d, 4, tables.shape[1], bs, window, 4096) > 0
+    q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
+    ws, want = ops.decode_workspace(q, k), np.zeros((len(lens), hq, d))
+    for i, x in enumerate(b.lens):
+        first = max(0, x - window) if window > 0 else (x - 1) // -window * -window if window < 0 and x else 0
+        rows = np.array([b.tables[i][j // bs] * bs + j % bs for j in range(first, x)], dtype=np.int64)
+        for pool in (k, v):  # (blocks are a sequence's own)
+            own = np.array([c * bs + r for c in b.tables[i] for r in range(bs)], dtype=np.int64)
+            pool[torch.from_numpy(np.setdiff1d(own, rows)).to(DEV)] = float("nan") if i % 2 else float("inf")
+        if x:
+            kk, vv = (t.double().cpu().numpy().reshape(-1, hkv, d)[rows].repeat(hq // hkv, axis=1) for t in (kr, vr))
+            s = np.einsum("hd,jhd->hj", b.q[i].double().numpy(), kk) * b.scale
+            w = np.exp(s - s.max(axis=1, keepdims=True))
+            want[i] = np.einsum("hj,jhd->hd", w / w.sum(axis=1, keepdims=True), vv)
+    call = (k, v, tables, n, bs, b.scale, ws)
+    got = ops.decode(q, *call, window=window)
+    other = decode_by_split_pass(q, k, v, b.tables, b.lens, bs, b.scale, window=window)[0]
+    # (logits of 32 bits and of at most about 30, so weights to 2^-19 of themselves; sums of up to 4000 terms, in parts)
+    assert_close(got, want, 1e-5, "against 64 bits")
+    # (0.95 of the split pass's on average; a call's few hundred rows, whose logits share an error, scatter about that by a tenth)
+    err = [np.sqrt(((t.double().cpu().numpy() - want) ** 2).mean()) for t in (got, other)]
+    assert err[0] <= 1.25 * err[1], err
+    two = torch.full_like(q, float("nan"))
+    for entry in ("pa_decode_split", "pa_decode_reduce"):
+        ops.decode(q, *call, out=two, entry=entry, window=window)
+    assert_close(two, got, 1e-6, "two calls")
+    assert torch.equal(ops.decode(q, *call, window=window), got) and not got[[x == 0 for x in b.lens]].any()
+    room = torch.full((q.numel() + 1,), 7.0, device=DEV)  # an output that starts between two 8-byte words
+    assert torch.equal(ops.decode(q, *call, out=room[1:].view(q.shape), window=window), got) and float(room[0]) == 7.0
+    if not window:  # padding positions and blocks that are not there are zero keys
+        clean, ez = (kr.float().to(DEV), vr.float().to(DEV)), max(lens) - n
+        t = [[-1 if j == len(x) // 2 and len(x) > 1 else c for j, c in enumerate(x)] for x in b.tables]
+        spare = (set(range(b.num_blocks)) - {x for y in b.tables for x in y}).pop()
+        kz, vz = kr.float().clone(), vr.float().clone()
+        kz[spare * bs: (spare + 1) * bs] = vz[spare * bs: (spare + 1) * bs] = 0
+        got = ops.decode(q, *clean, tables_to_device(t), n, bs, b.scale, ws, ez)
+        want = po.paged_decode(b.q, kz, vz, [[spare if c < 0 else c for c in x] for x in t], b.lens, bs, b.scale, pad_zero_keys=True)
+        assert_close(got, want, 1e-5, "zero keys")
