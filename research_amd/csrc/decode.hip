@@ -215,7 +215,8 @@ int decode_launch(int phases, const void *q, const void *k_cache, const void *v_
         }
         if ((phases & kPhaseReduce) && a.leave) {
             const int64_t items = (int64_t)batch * num_q_heads * (head_dim / 4);
-            ks.few_merge<<<dim3((unsigned)((items + kThreads - 1) / kThreads)), dim3(kThreads), 0, s>>>(a);
+            const int by = a.splits <= 8 ? 0 : a.splits <= 16 ? 1 : a.splits <= 32 ? 2 : 3;  // (a wave for eight runs of 64 items)
+            ks.few_merge[by]<<<dim3((unsigned)((items + 63) / 64)), dim3(64 << by), 0, s>>>(a);
             PA_CHECK_LAUNCH("pa_decode (short sequences, merge)");
         }
         return PA_OK;

@@ -1065,7 +1065,7 @@ struct KernelSet {
     reduce_fn reduce = nullptr;
     reduce_fn reduce_wave = nullptr;  // for batches with few pieces per sequence
     rowwise_fn rowwise = nullptr;
-    split_fn few = nullptr, few_merge = nullptr;  // sequences over narrow tables (decode_short.h; NULL: there are none for these types)
+    split_fn few = nullptr, few_merge[4] = {nullptr, nullptr, nullptr, nullptr};  // sequences over narrow tables (decode_short.h; NULL: there are none for these types)
 };
 
 template <typename KV, typename QT, int D> KernelSet kernels_for_d(int nrep_t) {

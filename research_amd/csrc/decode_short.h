@@ -410,50 +410,90 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
     }
 }
 
-// One thread per row and four of its elements.
-template <typename QT> __global__ __launch_bounds__(kThreads) void decode_short_merge_kernel(const DecodeArgs a) {
-    constexpr int kPipe = 8;
+// One thread per row, four of its elements and eight runs, a wave for 64 of these; P waves of a workgroup take P eights of runs, so that all loads of a row
+// are on their way at once.  What it takes is waits: one thread for all runs of its elements, whose loads the compiler moved to where each is used,
+// waited for one run after the other.  us a call, that -> this, all dense: 14 / 2 heads of 64, one sequence of 4096 keys (32 runs) 11.3 -> 7.8, of 8192 (64)
+// 15.2 -> 8.4; 32 / 8 of 128, one of 1024 (8) 9.0 -> 8.8, of 4096 (32) 12.5 -> 9.4; fp8 14 / 2 of 256, one of 8192 17.7 -> 10.8.
+template <typename QT, int P> __global__ __launch_bounds__(64 * P) void decode_short_merge_kernel(const DecodeArgs a) {
+    using f4 = typename ShortMfma<QT>::f4;
+    constexpr int kPipe = 8, kItems = 64;
+    __shared__ float part[P > 1 ? P - 1 : 1][6][kItems];
     const PoolArgs &p = a.p;
-    const int per = p.d / 4, item = blockIdx.x * kThreads + threadIdx.x, row = item / per, d = (item - row * per) * 4;
-    if (row >= a.batch * p.hq) return;
+    const int per = p.d / 4, at_item = threadIdx.x % kItems, eight = P > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kItems) : 0, item = blockIdx.x * kItems + at_item;
+    const bool live = item < a.batch * p.hq * per;
+    const int row = live ? item / per : 0, d = (live ? item - row * per : 0) * 4;
     const float *ml = a.part_ml + (int64_t)row * a.splits * 2, *acc = a.part_acc + (int64_t)row * a.splits * p.d + d;
     const int ez = a.extra_zero && a.seq_lens[row / p.hq] > 0 ? max(0, a.extra_zero[row / p.hq]) : 0;
     float best = kNegBig, den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int s = 0; s < a.splits; s += kPipe) {
-        float m[kPipe], l[kPipe], top = best;
-        float4 x[kPipe];
+    auto add = [&](float f, float l, f4 x) {
+        den = fmaf(f, l, den);
 #pragma unroll
-        for (int j = 0; j < kPipe; ++j) {
-            const int at = min(s + j, a.splits - 1);
-            const float2 y = *reinterpret_cast<const float2 *>(ml + 2 * at);
-            x[j] = *reinterpret_cast<const float4 *>(acc + (int64_t)at * p.d);
-            m[j] = s + j < a.splits ? y.x : kNegBig;
-            l[j] = s + j < a.splits ? y.y : 0.f;
-            top = fmaxf(top, m[j]);
-        }
+        for (int i = 0; i < 4; ++i) num[i] = fmaf(f, x[i], num[i]);
+    };
+    auto rise = [&](float top) {
         const float old = __builtin_amdgcn_exp2f(best - top);
         best = top;
         den *= old;
 #pragma unroll
         for (int i = 0; i < 4; ++i) num[i] *= old;
+    };
+#pragma unroll 1
+    for (int s = kPipe * eight; s < a.splits; s += kPipe * P) {
+        float m[kPipe], l[kPipe], top = best;
+        f4 x[kPipe];
 #pragma unroll
         for (int j = 0; j < kPipe; ++j) {
-            const float f = __builtin_amdgcn_exp2f(m[j] - top);
-            if (s + j >= a.splits) break;  // (uniform; zero times an infinite sum is none)
-            den = fmaf(f, l[j], den);
-            num[0] = fmaf(f, x[j].x, num[0]);
-            num[1] = fmaf(f, x[j].y, num[1]);
-            num[2] = fmaf(f, x[j].z, num[2]);
-            num[3] = fmaf(f, x[j].w, num[3]);
+            const int at = min(s + j, a.splits - 1);
+            const float2 y = *reinterpret_cast<const float2 *>(ml + 2 * at);
+            x[j] = *reinterpret_cast<const f4 *>(acc + (int64_t)at * p.d);
+            m[j] = y.x;
+            l[j] = y.y;
+        }
+        static_assert(kPipe == 8);
+        // (all of them are on their way before the first one is waited for)
+        asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]));
+#pragma unroll
+        for (int j = 0; j < kPipe; ++j) {  // (past the last run: nothing)
+            const bool is = s + j < a.splits;
+            m[j] = is ? m[j] : kNegBig;
+            l[j] = is ? l[j] : 0.f;
+            x[j] = is ? x[j] : f4{0.f, 0.f, 0.f, 0.f};
+            top = fmaxf(top, m[j]);
+        }
+        rise(top);
+#pragma unroll
+        for (int j = 0; j < kPipe; ++j) add(__builtin_amdgcn_exp2f(m[j] - top), l[j], x[j]);
+    }
+    if constexpr (P > 1) {
+        if (eight > 0) {
+            float *to = &part[eight - 1][0][at_item];
+            to[0] = best;
+            to[kItems] = den;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) to[(2 + i) * kItems] = num[i];
+        }
+        __syncthreads();
+        if (eight > 0) return;
+        float top = best;
+#pragma unroll
+        for (int j = 0; j < P - 1; ++j) top = fmaxf(top, part[j][0][at_item]);
+        rise(top);
+#pragma unroll
+        for (int j = 0; j < P - 1; ++j) {
+            const float *from = &part[j][0][at_item];
+            add(__builtin_amdgcn_exp2f(from[0] - top), from[kItems], f4{from[2 * kItems], from[3 * kItems], from[4 * kItems], from[5 * kItems]});
         }
     }
+    if (!live) return;
     short_store<QT>(reinterpret_cast<QT *>(a.out) + (int64_t)row * p.d + d, num, best, den, ez);
 }
 
 template <typename KV, typename QT> KernelSet with_short(KernelSet k, int d) {
     if (!k.split) return k;
-    k.few_merge = decode_short_merge_kernel<QT>;
+    k.few_merge[0] = decode_short_merge_kernel<QT, 1>;
+    k.few_merge[1] = decode_short_merge_kernel<QT, 2>;
+    k.few_merge[2] = decode_short_merge_kernel<QT, 4>;
+    k.few_merge[3] = decode_short_merge_kernel<QT, 8>;
     if (d == 64 || (d == 32 && sizeof(KV) == 4)) k.few = decode_short_kernel<KV, QT, 64>;
     if (d == 128) k.few = decode_short_kernel<KV, QT, 128>;
     if (d == 256) k.few = decode_short_kernel<KV, QT, 256>;

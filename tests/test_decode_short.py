@@ -205,3 +205,26 @@ def test_pools_of_32_bits(plan, lens, hq, hkv, d, window, bs):
         got = ops.decode(q, *clean, tables_to_device(t), n, bs, b.scale, ws, ez)
         want = po.paged_decode(b.q, kz, vz, [[spare if c < 0 else c for c in x] for x in t], b.lens, bs, b.scale, pad_zero_keys=True)
         assert_close(got, want, 1e-5, "zero keys")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv", ["bf16", "f32"])
+@pytest.mark.parametrize("runs,batch", [(8, 16), (9, 14), (16, 8), (18, 7), (32, 4), (42, 3), (64, 2)])
+def test_runs_that_several_waves_merge(plan, runs, batch, kv):
+    """Around the eights of runs that a wave of the merge takes, with runs that hold no key and positions that count as zero keys."""
+    from oracle import paged_oracle as po
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.test_gpu_decode_merge import Batch
+
+    announce(f"decode short: {runs} runs, {kv}")
+    b = Batch([8180, 40] + [i % 3 for i in range(batch - 2)], 14, 2, 64, kv, seed=runs)
+    (k, v, _, _), _ = b.device_pools()
+    tables = tables_to_device(b.tables)
+    assert plan.runs(batch, 14, 2, 64, 4 if kv == "f32" else 2, tables.shape[1], 16, 0, 4096) == runs
+    q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
+    for ez in (None, 8180 - n):
+        got = ops.decode(q, k, v, tables, n, 16, b.scale, ops.decode_workspace(q, k), ez)
+        want = po.paged_decode(b.q.float(), b.k.float(), b.v.float(), b.tables, b.lens, 16, b.scale, pad_zero_keys=ez is not None)
+        # (16 bits: the output's rounding, half a unit of 2^-8, doubled for sums)
+        assert_close(got, want, 1e-5 if kv == "f32" else 2.0 ** -7, "merged")
