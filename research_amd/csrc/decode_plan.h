@@ -198,7 +198,7 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // run).  From shapes alone; the tables' width stands for the longest sequence.
 // Head sizes up to 32 over 16 bits and fp8 stay with the generic loop of the split pass, whose weights have 32 bits: 11.8 us for 16 sequences of 16 .. 250 keys, 4 / 4
 // heads of 32, where weights of two bf16 terms took 5.0, but erred by up to 1.1e-6 of the sum of |weight value| where 32 bits err by 0.2e-6.
-// Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (3.5 us: 600 keys of 128).
+// Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (2.5 us, with the lines of 16 bits where 3.5 were measured: 600 keys of 128).
 // us, the split pass (one launch or two) -> this, sequences of n keys each: 32 / 8 heads of 128, 1 of 256 keys 14.1 -> 7.4, 1024 15.5 -> 9.0, 4096
 // 16.2 -> 12.0; 32 of 256 19.6 -> 8.3; 96 of 256 33.9 -> 19.7; 14 / 2 of 64, 1 of 256 15.2 -> 5.8, 4096 16.4 -> 11.0; 32 of 1024 22.1 -> 11.0, 16384
 // 64 -> 51; 192 of 1024 45 -> 21; fp8 32 / 8 of 128, 32 of 256 24.5 -> 6.8; fp8 14 / 2 of 256, 16 of 2048 47 -> 14.5, 256 of 2048 185 -> 91.
@@ -210,12 +210,18 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // 44.8 -> 47.4, 1024 33 -> 27; equal, 256 of 512 90 -> 94.  One or two query heads a kv head: 16 / 8 of 256, 16 of 1024 19.5 -> 24; 8 / 8 of 64, 3 of
 // 8192 18 -> 24; over fp8, where the kernel's conversions count, 8 / 8 of 64, 3 of 8064 in runs of 806 keys 12.7 -> 15.0, 32 / 16, 66 of 917 38 -> 51.
 // 8 / 2 of 128, 1 of 8192 14.6 -> 15.2, 4096 14 -> 12.
+// The lines that depend on the merge, whose loads are all on their way at once, were measured with it: above 64 elements a row, from five query heads a kv head on, runs of
+// 16-bit pools up to 416 KB (16 / 2 of 128, 5 of 6169 keys 50 -> 41, 106 of 1351 38 -> 25; beyond, unequal, 4 of 113400 61 -> 70) and of more than 512
+// keys of 128 cut in two where the units have room for it (fp8 16 / 2 of 128, 17 of 12251 29 -> 20, 5 of 57391 36 -> 26; of 256 not: 38 of 4315 35 -> 38); over
+// fp8 up to four heads more in all, of 256 longer ones too (32 / 8 of 128, 93 of 763 41 -> 25, of 256, 68 of 565 43 -> 21; 16 / 8 of 256, 1 of 8756 25 ->
+// 15; but 32 / 8 of 128, 66 of 2214 65 -> 70).  From three heads of 64 on, runs begin at 800 keys while they are few (32 / 8, 3 of 1040 10.8 -> 7.9).
+// (Over 400 drawn batches of more than 600 keys of 128, with the faster merge, 0.92 of the time before, the slowest 1.04.)
 // 32-bit pools, the split pass -> this: from five query heads a kv head on always (runs of up to 2 MB, as far as measured, but for 16 / 2 of 64 and the like, 1 of 81903 30 -> 33: the split pass spends a vector
 // instruction on every head, key and element; 14 / 2 of 72, 105 of 34 .. 127 keys 26.7 -> 8.1, 16 / 2 of 128, 102 of 236 51 -> 24, 23 of 6812 86 -> 57, 1 of 20000 at 24 /
 // 2 37 -> 26).  Three or four: up to 48 MB of keys (32 / 8 of 64, 4 of 155 14.5 -> 8.2, 8 / 2 of 128, 29 of 819 20 -> 17; beyond, unequal, 32 / 8 of 128,
 // 7 of 33764 160 -> 340), unless more than four rounds of workgroups have few keys each (32 / 8 of 64, 206 of 53 13.4 -> 15.0; at 256 more than one, 8 / 2, 163 of 138 21 -> 26) or the few there are
 // have long runs (8 / 2 of 128, 2 of 4000 15.6 -> 18.1, of 64, 8 of 6831 16.5 -> 18.2; of 256, 2 of 1964 17.6 -> 18.6).  One or two: a run each, up to 32 MB
-// and two rounds (16 / 8 of 128, 1 of 176 12.5 -> 8.6, 60 of 201 31 -> 21; 187 of 21 13.4 -> 18.1, 8 / 8 of 64, 16 of 600 14.5 -> 15.2).  A run is cut where four
+// and two rounds (16 / 8 of 128, 1 of 176 12.5 -> 8.6, 28 of 94 15.0 -> 8.9; 187 of 21 13.4 -> 18.1, 8 / 8 of 64, 16 of 600 14.5 -> 15.2).  A run is cut where four
 // turns of the waves, at 256 two, take longer than a merging launch: 16 keys of 128 each in 1 us (14 / 2 of 256, 6 of 228 in one run 20.7, of 64 keys 16.4, of
 // 32 11.9; 14 / 2 of 128, 16 of 101 8.2, in three 9.4); where most units have a workgroup anyway into two runs a unit, from five heads on four (unequal:
 // 14 / 2 of 72, 140 of 1600 71 -> 78, with four 50; equal 116 -> 100, 77).
@@ -231,9 +237,11 @@ PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, 
     int64_t runs = 1;
     const bool f32 = kv_elem_bytes == 4;
     const int64_t d = h.d_pad < 64 ? 64 : h.d_pad, least = f32 ? 64 * 128 / d : 128;  // (least: keys of a run)
-    const bool brief = keys * d <= (f32 ? 256 : 600) * 128;
+    const bool brief = keys * d <= (f32 ? 256 : h.n_rep > 2 && d == 64 && 4 * wgs <= cus ? 400 : 600) * 128;
     if (!brief) {
         runs = 4 * wgs <= cus ? cus / wgs : (!f32 ? 3 : h.n_rep > 4 ? 8 : 4) * (int64_t)cus / 2 / wgs;  // (few more workgroups than units are as slow as twice as many)
+        const int64_t each = keys / (runs < 1 ? 1 : runs) * d;
+        if (!f32 && h.n_rep > 4 && !(kv_elem_bytes == 1 && d == 256) && wgs <= cus && each > (runs > 1 ? 512 : 1024) * 128) runs = 2 * (runs < 1 ? 1 : runs);
         if (runs > keys / least) runs = keys / least;
         if (runs > kPlanShortRuns) runs = kPlanShortRuns;
         const int64_t room = w.slots * h.heads_per_slot() / ((int64_t)batch * h.hq);  // (their results are as long as a slot's)
@@ -241,10 +249,11 @@ PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, 
         if (runs < 1) runs = 1;
     }
     const int64_t row = d * kv_elem_bytes, kb = 1024;
-    const int64_t wide_most = row > 128 || h.hpw == 4 ? 256 * kb : h.hpw == 1 ? 512 * kb : h.hpw == 2 ? 384 * kb : 208 * kb;
-    const int64_t run_most = h.n_rep > 4 ? (kv_elem_bytes == 1 ? 4096 * row : wide_most) : h.n_rep > 2 ? 128 * kb : 64 * kb;
-    const int64_t all_most = h.n_rep > 4 ? (int64_t)1 << 62 : (h.n_rep > 2 ? 64 : 32) * kv_elem_bytes * kb * kb;
-    const bool few = h.n_rep <= 4 && wgs < 6 && keys > 4096;
+    const int64_t wide_most = row > 128 && kv_elem_bytes == 2 ? 416 * kb : row > 128 || h.hpw == 4 ? 256 * kb : h.hpw == 1 ? 512 * kb : h.hpw == 2 ? 384 * kb : 208 * kb;
+    const bool wide8 = kv_elem_bytes == 1 && d > 64;
+    const int64_t run_most = h.n_rep > 4 ? (kv_elem_bytes == 1 ? 4096 * row : wide_most) : (h.n_rep > 2 ? (wide8 && d > 128 ? 384 : 128) : wide8 ? 128 : 64) * kb;
+    const int64_t all_most = h.n_rep > 4 ? (int64_t)1 << 62 : (h.n_rep > 2 ? (wide8 ? (d > 128 ? 200 : 100) : 64 * kv_elem_bytes) : wide8 ? 48 : 32 * kv_elem_bytes) * kb * kb;
+    const bool few = h.n_rep <= 4 && wgs < 6 && keys > 4096 && !wide8;
     if (f32) {
         const bool lone = keys > 3072 ? wgs < (d == 64 ? 24 : 6) : d == 256 && !brief && wgs < 8;
         const bool fits = h.n_rep > 4   ? d > 64 || wgs >= 6 || keys <= 8192

@@ -55,6 +55,19 @@ def test_lines_of_the_rule(plan):
     assert runs(1, (8, 2, 128, 2), 4096) == 32 and runs(1, (8, 2, 128, 2), 4112) == 0
 
 
+def test_lines_of_wide_groups_and_of_32_bits(plan):
+    runs = lambda batch, shape, keys: plan.runs(batch, *shape, keys // 16, 16, 0, 4096)
+    two, fp8 = (16, 2, 128, 2), (16, 2, 128, 1)  # eight query heads a kv head: long runs are cut in two while a unit has one workgroup or none
+    assert runs(37, two, 6176) == 10 and runs(106, two, 1360) == 2 and runs(129, two, 1360) == 1 and runs(17, fp8, 12256) == 14 and runs(38, (14, 2, 256, 1), 4320) == 5
+    assert runs(200, two, 1664) == 1 and runs(200, two, 1680) == 0                                     # 416 KB
+    assert runs(68, (32, 8, 256, 1), 576) == 1 and runs(93, (32, 8, 128, 1), 768) == 1 and runs(93, (32, 8, 128, 1), 1040) == 0
+    assert runs(3, (32, 8, 64, 2), 800) == 1 and runs(3, (32, 8, 64, 2), 816) == 6
+    f32, wide = (14, 2, 64, 4), (32, 8, 128, 4)
+    assert runs(4, f32, 512) == 1 and runs(4, f32, 528) == 4 and runs(4, wide, 256) == 1 and runs(4, wide, 272) == 4 and runs(140, (14, 2, 72, 4), 1600) == 3
+    assert runs(1, f32, 8192) == 64 and runs(1, f32, 8208) == 0 and runs(4, (8, 2, 32, 4), 64) == 1
+    assert runs(7, wide, 33776) == runs(206, (32, 8, 64, 4), 64) == runs(16, (8, 8, 64, 4), 608) == runs(2, (8, 2, 128, 4), 4000) == 0
+
+
 def test_results_of_the_runs_fit_the_workspace(plan):
     rng = np.random.default_rng(0)
     for _ in range(20000):
