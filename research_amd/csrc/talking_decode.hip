@@ -253,20 +253,37 @@ template <int VC, int HP> __global__ __launch_bounds__(256) void talk_values_ker
     }
 }
 
-// The parts of a sequence's pieces added up: four value columns per thread
-__global__ __launch_bounds__(256) void talk_merge_kernel(const TalkArgs a, int vc) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, bh = i / (vc / 4);
-    if (bh >= (int64_t)a.batch * a.heads) return;
+// The parts of a sequence's pieces added up: a thread has four value columns and eight pieces, whose loads are all on their way at once; P waves take the eights of
+// pieces for 64 fours of columns (more than 8 P pieces in turns).  A thread for all pieces, one load after the other, took 7.5 us for 16 pieces of 8 sequences of
+// 1000 .. 8000 keys, 16 heads of 128, this 3.8.
+template <int P> __global__ __launch_bounds__(64 * P) void talk_merge_kernel(const TalkArgs a, int vc) {
+    constexpr int kPipe = 8;
+    __shared__ f4 part[P > 1 ? P - 1 : 1][64];
+    const int lane = threadIdx.x % 64, eight = P > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : 0;
+    const int64_t i = (int64_t)blockIdx.x * 64 + lane, all = (int64_t)a.batch * a.heads, bh = min(i / (vc / 4), all - 1);
     const int d = (int)(i % (vc / 4)) * 4, keys = a.ctx_lens[bh / a.heads];
-    if (d >= a.vdim || keys <= 0) return;
     const float *src = a.part_o + bh * a.splits * vc + d;
     f4 sum = f4{0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < a.splits; ++s) {
-        if (td_piece(a, keys, s).lo >= keys) break;
-        const f4 x = *reinterpret_cast<const f4 *>(src + (int64_t)s * vc);
+    for (int s = kPipe * eight; s < a.splits; s += kPipe * P) {
+        f4 x[kPipe];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum[e] += x[e];
+        for (int j = 0; j < kPipe; ++j) x[j] = *reinterpret_cast<const f4 *>(src + (int64_t)min(s + j, a.splits - 1) * vc);
+        static_assert(kPipe == 8);
+        asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]));
+#pragma unroll
+        for (int j = 0; j < kPipe; ++j) {
+            const bool is = s + j < a.splits && td_piece(a, keys, s + j).lo < keys;  // (the others wrote nothing)
+            sum += is ? x[j] : f4{0.f, 0.f, 0.f, 0.f};
+        }
     }
+    if constexpr (P > 1) {
+        if (eight > 0) part[eight - 1][lane] = sum;
+        __syncthreads();
+        if (eight > 0) return;
+#pragma unroll
+        for (int j = 0; j < P - 1; ++j) sum += part[j][lane];
+    }
+    if (i >= all * (vc / 4) || d >= a.vdim || keys <= 0) return;
     pa_bf16 *out = reinterpret_cast<pa_bf16 *>(a.out) + bh * a.vdim + d;
     if (a.vdim % 4 == 0) {
         *reinterpret_cast<uint2 *>(out) = make_uint2(row_pack_bf16(sum[0], sum[1]), row_pack_bf16(sum[2], sum[3]));
@@ -334,7 +351,9 @@ bool pa_talking_decode_launch(const TalkArgs &in, int dtype, void *workspace, si
         if (int e = vc == 64 ? launch_values_heads<64>(a, grid, s) : vc == 128 ? launch_values_heads<128>(a, grid, s) : launch_values_heads<256>(a, grid, s)) return e;
         if (a.splits > 1) {
             const int64_t items = (int64_t)a.batch * a.heads * (vc / 4);
-            talk_merge_kernel<<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s>>>(a, vc);
+            const dim3 blocks((unsigned)((items + 63) / 64));
+            if (a.splits <= 8) talk_merge_kernel<1><<<blocks, dim3(64), 0, s>>>(a, vc);
+            else talk_merge_kernel<2><<<blocks, dim3(128), 0, s>>>(a, vc);
             PA_CHECK_LAUNCH("pa_talking_attention (merge)");
         }
         return PA_OK;

@@ -427,6 +427,21 @@ def test_decode_pieces_with_sinks_and_padding_rows():
         assert_close(got, torch.stack(want), 1e-2, splits)
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 62), (4, 1, 128, 128), (3, 3, 256, 250)])
+@pytest.mark.parametrize("keys", [600, 2303, 2304, 4100])
+def test_pieces_around_the_eights_that_a_wave_joins(keys, heads, kv, dim, vdim):
+    """Two, eight, nine and sixteen pieces of the longer sequence, one with keys of the shorter, against one piece."""
+    announce(f"scored joins {keys} {heads} {kv} {dim} {vdim}")
+    paged = Paged([keys, 3], kv, dim, dim, BF, seed=keys)
+    q, sink = _rand(2, heads, dim, seed=9).to(BF), _rand(heads, seed=4)
+    call = lambda splits, **kw: _scored(paged, [(0, keys - 1, 1), (1, 2, 1)], (q,), vdim, BF, 0.2, 0, decode=True, splits=splits, **kw).double().cpu()
+    for kw in (dict(), dict(sink=sink)):
+        one, got = call(False, **kw), call(True, **kw)
+        # (each rounds its weights to 16 bits against references of its own, 2^-9 of the weighted mean of |values|, of two at most, and the output, 2^-9 of it:
+        # together twice (2 + |output|) 2^-9)
+        assert_close(got, one, 2.0 ** -7, kw)
+
+
 # ------------------------------------------------------------------ latent rows
 
 
