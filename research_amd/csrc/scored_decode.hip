@@ -276,10 +276,12 @@ template <int P> __global__ __launch_bounds__(64 * P) void scored_merge_kernel(c
         const int d = d0 + 4 * lane;
         const bool live = d < a.vdim;
         const float *po = a.part_o + rh * a.splits * vc + (live ? d : 0);
-        float m = a.sink && eight == 0 ? a.sink[h] * kScoredLog2e : kScoredNone, den = a.sink && eight == 0 ? 1.f : 0.f;
+        const float sink = a.sink ? a.sink[h] * kScoredLog2e : 0.f;  // (minus infinity from the lowest floats on)
+        float m = -INFINITY, den = 0.f;  // (of the pieces with a sum: eight of them may have none, as their scores may all be minus infinity)
         sd_f4 num = sd_f4{0.f, 0.f, 0.f, 0.f};
+        auto factor = [](float from, float to) { return from == to ? 1.f : __builtin_amdgcn_exp2f(from - to); };
         auto rise = [&](float top) {
-            const float old = __builtin_amdgcn_exp2f(m - top);
+            const float old = factor(m, top);
             m = top;
             den *= old;
             num *= old;
@@ -328,7 +330,7 @@ template <int P> __global__ __launch_bounds__(64 * P) void scored_merge_kernel(c
                 rise(top);
 #pragma unroll
                 for (int j = 0; j < P - 1; ++j) {
-                    const float *from = &part[j][0][lane], w = __builtin_amdgcn_exp2f(from[0] - top);
+                    const float *from = &part[j][0][lane], w = factor(from[0], top);
                     den = fmaf(w, from[64], den);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) num[i] = fmaf(w, from[(2 + i) * 64], num[i]);
@@ -336,6 +338,10 @@ template <int P> __global__ __launch_bounds__(64 * P) void scored_merge_kernel(c
             }
         }
         if (!live || eight > 0 || keys < 1) continue;
+        if (a.sink) {
+            rise(fmaxf(m, sink));
+            den += __builtin_amdgcn_exp2f(sink - m);
+        }
         pa_bf16 *out = reinterpret_cast<pa_bf16 *>(a.out) + rh * a.vdim + d;
         const float f = 1.f / den;
         if (a.vdim % 4 == 0) {

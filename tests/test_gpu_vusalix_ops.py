@@ -428,7 +428,7 @@ def test_decode_pieces_with_sinks_and_padding_rows():
 
 
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 62), (4, 1, 128, 128), (3, 3, 256, 250)])
-@pytest.mark.parametrize("keys", [600, 2303, 2304, 4100])
+@pytest.mark.parametrize("keys", [600, 2250, 2304, 4100])  # (tables have room for 32 to 47 keys more)
 def test_pieces_around_the_eights_that_a_wave_joins(keys, heads, kv, dim, vdim):
     """Two, eight, nine and sixteen pieces of the longer sequence, one with keys of the shorter, against one piece."""
     announce(f"scored joins {keys} {heads} {kv} {dim} {vdim}")
@@ -440,6 +440,28 @@ def test_pieces_around_the_eights_that_a_wave_joins(keys, heads, kv, dim, vdim):
         # (each rounds its weights to 16 bits against references of its own, 2^-9 of the weighted mean of |values|, of two at most, and the output, 2^-9 of it:
         # together twice (2 + |output|) 2^-9)
         assert_close(got, one, 2.0 ** -7, kw)
+
+
+@pytest.mark.parametrize("none", [float("-inf"), float(np.finfo(np.float32).min)])
+@pytest.mark.parametrize("pieces,keys", [(8, 2250), (9, 2304), (16, 4100)])  # (tables have room for 32 to 47 keys more)
+def test_pieces_without_a_sum_beside_a_sink_without_weight(pieces, keys, none):
+    """Far keys by their bias and sinks by their size weigh nothing: minus infinity, and the lowest float, whose product with log2 e is minus infinity too.
+    All pieces but the last one or two have no sum then, the first eight of sixteen among them."""
+    announce(f"scored joins {pieces} {none}")
+    heads, dim, near = 4, 64, 200
+    paged = Paged([keys, 40], 1, dim, dim, BF, seed=pieces)
+    q, sink = _rand(2, heads, dim, seed=9).to(BF), torch.tensor([none, none, 0.5, -2.0])
+    bias = torch.zeros(heads, near + 1)
+    bias[:, near], bias[3] = none, 0.0  # (of the last head nothing is far)
+    got = _scored(paged, [(0, keys - 1, 1), (1, 39, 1)], (q,), dim, BF, 0.2, 0, decode=True, bias=bias, sink=sink).cpu()
+    one = _scored(paged, [(0, keys - 1, 1), (1, 39, 1)], (q,), dim, BF, 0.2, 0, decode=True, splits=False, bias=bias, sink=sink).cpu()
+    for i, n in enumerate((keys, 40)):
+        k, v = (paged.rows(t, i)[:, 0].double() for t in (paged.k, paged.v))
+        e = torch.exp(q[i].double() @ k.T * 0.2)
+        e[:3, : max(0, n - near)] = 0
+        want = e @ v / (e.sum(-1, keepdim=True) + torch.where(sink == none, 0.0, torch.exp(sink.double()))[:, None])
+        assert_close(got[i], want, 1e-2, i)
+        assert_close(one[i], want, 1e-2, i)
 
 
 # ------------------------------------------------------------------ latent rows
