@@ -118,8 +118,7 @@ int pa_decode_passes(int batch, int num_q_heads, int num_kv_heads, int head_dim,
  * Kernel launches one pa_decode call of these shapes makes on the current device (0 for an empty batch, else 1 or 2;
  * of more than 8192 sequences, which are taken in parts: of a part); negative on error.  runs (may be NULL): over
  * narrow tables, the runs that each sequence is cut into (1: one launch and nothing to merge); 0 where the split
- * pass takes the call, -1 where it does with a workgroup for each sequence (over 32-bit pools: 0 where sequences are
- * cut, -1 where each has one workgroup, in either kernel).  Where the answer is 1, pa_decode_split and pa_decode_reduce are no two parts of pa_decode.
+ * pass takes the call, -1 where it does with a workgroup for each sequence.  Where the answer is 1, pa_decode_split and pa_decode_reduce are no two parts of pa_decode.
  * (pa_decode_static, whose scratch holds fewer results, may cut a sequence into fewer runs.)  For callers that time
  * or profile the passes.  (No counterpart in the reference.)
  */

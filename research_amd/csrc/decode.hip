@@ -277,9 +277,7 @@ extern "C" int pa_decode_launches(int batch, int num_q_heads, int num_kv_heads, 
     if (batch > kMaxBatch) batch = kMaxBatch;  // launches per group of kMaxBatch sequences
     const Route r = decode_route(ks, batch, plan, plan_workspace(batch, plan, plan.d_pad, kMaxSplitGrid), head_dim, kv_dtype, bt_stride,
                                  block_size, window, split_grid());
-    // (32-bit pools: by what a call does alone, as that is the same in both kernels and the line between them a matter of time)
-    const bool whole = r.runs == 0 ? r.whole : kv_dtype == PA_F32 && r.runs == 1;
-    if (runs) *runs = batch == 0 ? 0 : whole ? -1 : kv_dtype == PA_F32 ? 0 : r.runs;
+    if (runs) *runs = batch == 0 ? 0 : r.runs > 0 ? r.runs : r.whole ? -1 : 0;
     return batch > 0 ? r.launches() : 0;
 }
 

@@ -156,7 +156,9 @@ def test_launches_of_decode_by_the_width_of_its_tables():
     assert lib.pa_decode_passes(4, 14, 2, 64, bf) == 2
     for batch, heads, kv in ((256, (32, 8, 128), bf), (16, (32, 8, 128), bf), (8, (32, 8, 128), fp8), (300, (16, 8, 128), fp8)):
         assert launches(batch, heads, 1 << 20, kv=kv) == (lib.pa_decode_passes(batch, *heads, kv), 0)
-    assert launches(4, (8, 2, 128), 64, f32, f32) == (1, -1) and launches(4, (8, 2, 128), 1024, f32, f32) == (2, 0)  # (whole sequences)
+    assert launches(4, (8, 2, 128), 64, f32, f32) == (1, 1) and launches(4, (8, 2, 128), 1024, f32, f32) == (2, 16)
+    # the split pass: whole sequences, and ranges and their merge
+    assert launches(4, (8, 2, 128), 64, f32, f32, bs=8) == (1, -1) and launches(4, (8, 2, 128), 1024, f32, f32, bs=8) == (2, 0)
     assert launches(4, (32, 8, 128), 64, bs=8) == (1, -1) and launches(4, (8, 2, 32), 4096) == (2, 0)
     assert launches(4, (32, 8, 128), 1 << 20, window=200) == (1, 1) and launches(0, (32, 8, 128), 64) == (0, 0)
     assert lib.pa_decode_launches(4, 14, 2, 64, 4, 16, 0, bf, bf, None) == 1

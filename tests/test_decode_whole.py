@@ -1,4 +1,4 @@
-"""Decode with narrow block tables that the kernel for them does not take (32-bit pools, blocks that are no whole tiles of 16 keys, large
+"""Decode with narrow block tables that the kernel for them does not take (blocks that are no whole tiles of 16 keys, 16-bit heads of up to 32, large
 batches): a workgroup of the split pass takes a whole (plane, sequence), and one launch does (``plan_whole_sequences`` of ``decode_plan.h``).
 The rule's lines on the CPU; on the device the same batch with narrow tables and with tables padded beyond the rule's line, which take the
 split pass in ranges and the merge, against the oracle and against each other."""
@@ -53,12 +53,13 @@ def test_lines_of_the_rule(whole):
 CASES = [
     ([1, 2, 24, 47], 14, 2, 64, "bf16", 0, 8),              # (and where a workgroup's ranges end in the split pass: 0, 15, 16, 17)
     ([0, 96, 17, 16, 15, 0, 1, 81], 32, 8, 128, "bf16", 0, 8),
-    ([64, 0, 33, 1], 8, 2, 128, "f32", 0, 16),
+    ([64, 0, 33, 1], 8, 2, 128, "f32", 0, 8),
     ([96, 5, 0, 48], 16, 8, 128, "fp8", 0, 8),
     ([60, 1, 33], 16, 2, 64, "fp8", 0, 8),
     ([90, 16, 0, 31], 16, 8, 256, "f16", 0, 8),
     ([190, 3, 0, 129], 8, 2, 72, "f16", 0, 24),
-    ([40, 64, 1, 0], 4, 4, 32, "f32", 0, 16),
+    ([40, 64, 1, 0], 4, 4, 32, "f32", 0, 8),
+    ([48, 7, 0, 25], 14, 2, 64, "f32", 0, 24),
     ([40, 64, 1, 0], 4, 4, 32, "bf16", 0, 16),
     ([5000, 63, 0, 64, 65, 999], 32, 8, 128, "bf16", 64, 8),  # (long tables, a short window)
     ([130, 64, 0, 65, 127], 32, 8, 128, "bf16", -64, 8),
