@@ -19,6 +19,10 @@ namespace {
 
 using namespace pa_decode_detail;
 
+// A key whose block is missing: zeros for a row of up to 128 elements.  (Read as global memory, like kScoredZeros.)
+__device__ const uint32_t kTalkNoKey[64] __attribute__((aligned(16))) = {0};
+typedef const __attribute__((address_space(1))) scored_u4 *talk_global;
+
 constexpr float kTpSlack = 8.f;  // log2 of the factor by which a row's reference maximum may lag
 
 __device__ __forceinline__ void tp_own_lds() {  // a wave's own part of LDS: its writes before its reads
@@ -232,11 +236,11 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     const int v_kv0 = kv_of(out0);
     __bf16 *v_s = v_all + (SAME ? kv_of(own0) - v_kv0 : wave) * L::vTile;
     // Block and pool row of the key that this thread stages (values staged by all: the piece of a tile; else key lane % 32); past
-    // the last key: the last one's, which nothing weighs.
+    // the last key: the last one's, which nothing weighs.  -1: its block is missing, a key and a value of zeros.
     const int my_row = SAME ? tid % kTile / kPer : lane & 31;
     auto key_of = [&](int k0) { return min(k0 + my_row, end - 1); };
     auto id_of = [&](int k0) { return talk_block_id(a, table, key_of(k0)); };
-    auto slot_of = [&](int id, int k0) { return max(talk_slot_of(a, id, key_of(k0), end), 0); };
+    auto slot_of = [&](int id, int k0) { return talk_slot_of(a, id, key_of(k0), end); };
     scored_u4 kr[NK], vr[NV];
     // staged by the workgroup: piece tid + 512 n is of kv head (tid + 512 n) / kTile, the thread's own row
     auto stage_from = [&](const void *pool, int slot, uint32_t tok, int head_dim, int kv_first, int real, scored_u4 *to) {
@@ -244,7 +248,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
             const uint16_t *at = src + min(kv_first + (tid + kTmThreads * n) / kTile, a.hkv - 1) * head_dim;
-            to[n] = FULL ? *reinterpret_cast<const scored_u4 *>(at) : scored_load16(at, tid % kPer * 8 < real);
+            to[n] = scored_load16(at, slot >= 0 && (FULL || tid % kPer * 8 < real));
         }
     };
     auto stage_to = [&](__bf16 *tiles, int tile, int row_at, const scored_u4 *from) {
@@ -256,9 +260,12 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
         if constexpr (!L::ahead) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const uint16_t *src = reinterpret_cast<const uint16_t *>(a.k) + (uint64_t)(uint32_t)__shfl(slots, 16 * kb + l16, 64) * k_tok + kv * a.k_dim + 8 * g;
+                const int slot = __shfl(slots, 16 * kb + l16, 64);
+                const uint16_t *pool = reinterpret_cast<const uint16_t *>(a.k) + (uint64_t)(uint32_t)slot * k_tok + kv * a.k_dim;
+                const uintptr_t src = (slot < 0 ? reinterpret_cast<uintptr_t>(kTalkNoKey) : reinterpret_cast<uintptr_t>(pool)) + 16 * g;
 #pragma unroll
-                for (int k = 0; k < KS; ++k) kr[kb * KS + k] = FULL ? *reinterpret_cast<const scored_u4 *>(src + 32 * k) : scored_load16(src + 32 * k, 32 * k + 8 * g < a.n1);
+                for (int k = 0; k < KS; ++k)
+                    kr[kb * KS + k] = FULL ? *reinterpret_cast<talk_global>(src + 64 * k) : scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, 32 * k + 8 * g < a.n1);
             }
         }
     };
@@ -270,8 +277,9 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
         if constexpr (!SAME) {
 #pragma unroll
             for (int n = 0; n < NV; ++n) {
-                const uint16_t *src = reinterpret_cast<const uint16_t *>(a.v) + (uint64_t)(uint32_t)__shfl(slots, (64 * n + lane) / kPer, 64) * v_tok + kv * a.v_dim + lane % kPer * 8;
-                vr[n] = scored_load16(src, lane % kPer * 8 < vreal);
+                const int slot = __shfl(slots, (64 * n + lane) / kPer, 64);
+                const uint16_t *src = reinterpret_cast<const uint16_t *>(a.v) + (uint64_t)(uint32_t)slot * v_tok + kv * a.v_dim + lane % kPer * 8;
+                vr[n] = scored_load16(src, slot >= 0 && lane % kPer * 8 < vreal);
             }
         }
     };
@@ -290,7 +298,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     // keys by key lane % 32, where they go straight to operands beside values staged by all
     auto near_id = [&](int k0) { return SAME && !L::ahead ? talk_block_id(a, table, min(k0 + (lane & 31), end - 1)) : 0; };
     auto near_slot = [&](int id, int k0, int slots) {
-        return SAME && !L::ahead ? max(talk_slot_of(a, id, min(k0 + (lane & 31), end - 1), end), 0) : slots;
+        return SAME && !L::ahead ? talk_slot_of(a, id, min(k0 + (lane & 31), end - 1), end) : slots;
     };
     // 16-byte pieces of a pair's row and of a (head, row)'s keys at places that spread over the banks (by the groups of lanes that a
     // read serves together, linear_tiles.h; with the keys' pitch 8 prompts of 818 .. 3868 tokens 508 -> 494 us); inside a piece the place of a
@@ -605,7 +613,7 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     const int row0 = block * kTpRows;
     if (row0 >= p.n) return;
     const int row = row0 + l16, first_pos = p.pos0 + row0, end = p.pos0 + min(row0 + kTpRows, p.n), tiles = (end + kTpKeys - 1) / kTpKeys;
-    // Pool row of a key, from its block; past the last key: the last one's, which nothing weighs.
+    // Pool row of a key, from its block; past the last key: the last one's, which nothing weighs; -1: its block is missing, a key and a value of zeros.
     const int32_t *table = a.bt + b * a.bt_stride;
     const int last_block = (int)min(a.bt_stride, (int64_t)0x7fffffff) - 1, known = (int)a.num_blocks;
     auto block_of = [&](int key) { return (int)(__umulhi(2u * (uint32_t)min(key, end - 1), a.bs_magic) >> a.bs_magic_shift); };
@@ -613,7 +621,7 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     auto slot_of = [&](int id, int key) {
         const int blk = block_of(key);
         const bool there = (blk <= last_block) & ((uint32_t)id < (uint32_t)known);
-        return there ? min(key, end - 1) + (id - blk) * a.bs : 0;
+        return there ? min(key, end - 1) + (id - blk) * a.bs : -1;
     };
     const int first_id = id_of(tid % (4 * kTpKeys));
 
@@ -638,11 +646,11 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
         const int my_key = 16 * half + l16;
         bf8 kr[KS];
         auto fetch = [&](int slot) {
-            const char *src = kp + (uint64_t)(uint32_t)slot * k_tok;
+            const uintptr_t src = slot < 0 ? reinterpret_cast<uintptr_t>(kTalkNoKey) + 16 * g : reinterpret_cast<uintptr_t>(kp + (uint64_t)(uint32_t)slot * k_tok);
 #pragma unroll
             for (int k = 0; k < KS; ++k)
-                kr[k] = FULL ? *reinterpret_cast<const bf8 *>(src + 64 * k)
-                             : __builtin_bit_cast(bf8, scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, 32 * k + 8 * g < a.n1));
+                kr[k] = __builtin_bit_cast(bf8, FULL ? *reinterpret_cast<talk_global>(src + 64 * k)
+                                                     : scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, 32 * k + 8 * g < a.n1));
         };
         // (distances first_pos + r - k of 16 rows and 16 keys, from their smallest, of two heads a lane; a key behind its row gets no weight)
         float size[2], rate[2];
@@ -751,7 +759,10 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     auto fetch = [&](int k0) {
         const int *slots = ring + ((k0 + my_key) & (L::ring - 1));
 #pragma unroll
-        for (int n = 0; n < NV; ++n) vr[n] = *reinterpret_cast<const scored_u4 *>(vp + (uint64_t)(uint32_t)slots[n * kEach] * v_tok);
+        for (int n = 0; n < NV; ++n) {
+            const int slot = slots[n * kEach];
+            vr[n] = scored_load16(reinterpret_cast<const uint16_t *>(vp + (uint64_t)(uint32_t)slot * v_tok), slot >= 0);
+        }
     };
     auto put_v = [&]() {
 #pragma unroll

@@ -115,12 +115,17 @@ class Talking:
         self.rate = 0.05 + 0.6 * torch.rand(heads, generator=g) if biased else None
         self.q = [F.pad(_rand(n, heads, dim, seed=seed + 20 + i), (0, self.pad - dim)).to(dtype) for i, n in enumerate(lens)]
 
-    def solve(self):
+    def solve(self, holes=()):
+        """``holes``: (sequence, block, the id that stands in the table instead of a block's)."""
         self.want = []
         for i, q in enumerate(self.q):
             k, v = self.paged.rows(self.paged.k, i).double(), self.paged.rows(self.paged.v, i).double()[..., : self.vdim]
+            for _, block, _ in (x for x in holes if x[0] == i):
+                k[16 * block: 16 * block + 16] = v[16 * block: 16 * block + 16] = 0
             bias = None if self.size is None else lo.distance_bias(self.size.double(), self.rate.double(), len(q))
             self.want.append(lo.causal_attention(q.double()[..., : self.dim], k[..., : self.dim], v, self.scale, bias, self.talk.double()))
+        for i, block, instead in holes:
+            self.paged.tables[i, block] = instead
         return self
 
     def run(self, picks, decode=False, workspace=True):
@@ -188,6 +193,33 @@ def test_prompts_with_more_blocks_of_rows_than_workgroups_side_by_side(heads, kv
     case.check([(i % 5, 0, lens[i % 5]) for i in range(70)])
     case.check([(i % 5, lens[i % 5] - 1 - i % 3, 1 + i % 3) for i in range(600)])
     case.check([(0, 283, 17), (4, 160, 1)])
+
+
+MISSING = [  # kernels with waves of two kinds: 16 heads, 8, sizes with padding; of one kind: 16 heads with keys staged by all and by each wave, up to 32
+    (16, 4, 128, 128), (8, 2, 64, 64), (12, 1, 72, 120), (6, 3, 128, 128), (6, 2, 40, 56), (32, 8, 128, 128), (24, 8, 64, 128)]
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim", MISSING)
+def test_missing_blocks_are_rows_of_zeros(heads, kv, dim, vdim):
+    """The first block, one in the middle and the last one of a sequence, by a negative id and by ids outside the pool: keys and values of zeros."""
+    announce(f"talking missing {heads} {kv} {dim} {vdim}")
+    lens = [330, 70]
+    case = Talking(lens, heads, kv, dim, vdim, BF, seed=13)
+    outside = case.paged.k.shape[0] // 16
+    case.solve([(0, 0, -1), (0, 7, outside), (0, 20, 1 << 30), (1, 2, -5), (1, 4, outside)])
+    case.check([(i, 0, n) for i, n in enumerate(lens)])
+    case.check([(0, 300, 30), (1, 33, 37)])
+    case.check([(i, n - 1, 1) for i, n in enumerate(lens)], decode=True)
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim", MISSING)
+def test_a_pool_without_a_whole_block_is_zeros(heads, kv, dim, vdim):
+    announce(f"talking empty pool {heads} {kv} {dim} {vdim}")
+    case = Talking([290], heads, kv, dim, vdim, BF)
+    case.paged.k, case.paged.v = case.paged.k[:8].contiguous(), case.paged.v[:8].contiguous()
+    case.want = [torch.zeros(290, heads, vdim, dtype=torch.float64)]
+    case.check([(0, 0, 290)])
+    case.check([(0, 289, 1)], decode=True)
 
 
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 64), (20, 4, 48, 72)])
