@@ -595,9 +595,9 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     typedef float f16 __attribute__((ext_vector_type(16)));
     extern __shared__ __align__(16) char tm_lds[];
     // Workgroups that are all there at once take any block; else those with the most keys come first.
-    int b = blockIdx.x % a.batch, block = blockIdx.x / a.batch;
+    int b = blockIdx.x, block = blockIdx.y;
     ScoredPortion p;
-    if (gridDim.x > a.at_once ? !tp_block(a, blockIdx.x, b, block, p) : !scored_portion(a, b, p)) return;
+    if (gridDim.x * gridDim.y > a.at_once ? !tp_block(a, (int)(blockIdx.y * gridDim.x + blockIdx.x), b, block, p) : !scored_portion(a, b, p)) return;
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
     const int all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = all % L::part;
     char *w_all = tm_lds + 2 * L::pTile, *v_all = w_all + 2 * L::wTile;
@@ -861,11 +861,11 @@ template <int DK, int DV, int G, bool FULL> int launch_pipe(const TalkArgs &a, h
     constexpr size_t lds = TpTile<DV, G>::bytes;
     static_assert(lds <= 160 * 1024 / (4 / G), "LDS of one compute unit");
     if (int rc = la_big_lds(talk_pipe_kernel<DK, DV, G, FULL>, lds, "pa_talking_attention")) return rc;
-    const int64_t blocks = (int64_t)a.batch * ((a.max_q_len + kTpRows - 1) / kTpRows), side = (int64_t)la_cus() * (4 / G);
-    PA_REQUIRE(blocks <= 0x7fffffff, "pa_talking_attention: batch=%d, max_q_len=%d are too many rows for one launch", a.batch, a.max_q_len);
+    // (two dimensions: in one, the threads of 1024 portions of up to 65535 rows are more than a launch can have)
+    const dim3 grid((unsigned)a.batch, (unsigned)((a.max_q_len + kTpRows - 1) / kTpRows));
     TalkArgs args = a;
-    args.at_once = (unsigned)side;
-    talk_pipe_kernel<DK, DV, G, FULL><<<dim3((unsigned)blocks), dim3(TpTile<DV, G>::threads), lds, s>>>(args);
+    args.at_once = (unsigned)(la_cus() * (4 / G));
+    talk_pipe_kernel<DK, DV, G, FULL><<<grid, dim3(TpTile<DV, G>::threads), lds, s>>>(args);
     PA_CHECK_LAUNCH("pa_talking_attention (portions)");
     return PA_OK;
 }

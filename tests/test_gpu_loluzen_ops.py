@@ -128,8 +128,9 @@ class Talking:
             self.paged.tables[i, block] = instead
         return self
 
-    def run(self, picks, decode=False, workspace=True):
+    def run(self, picks, decode=False, workspace=True, room=0):
         p = _portions(picks, [0] * len(self.q), tiles=False)
+        p = p._replace(max_q_len=max(room, p.max_q_len))
         if decode:
             p = ops.Portions(p.ctx_lens, p.state_slots)
         q = torch.cat([self.q[b][at: at + n] for b, at, n in picks]).to(DEV)
@@ -193,6 +194,15 @@ def test_prompts_with_more_blocks_of_rows_than_workgroups_side_by_side(heads, kv
     case.check([(i % 5, 0, lens[i % 5]) for i in range(70)])
     case.check([(i % 5, lens[i % 5] - 1 - i % 3, 1 + i % 3) for i in range(600)])
     case.check([(0, 283, 17), (4, 160, 1)])
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim,portions", [(16, 4, 128, 128, 1024), (8, 2, 64, 64, 2049)])
+def test_many_prompts_with_room_for_long_ones(heads, kv, dim, vdim, portions):
+    """Portions of up to 65535 rows, as far as the call is told: more threads in all than one dimension of a launch has."""
+    announce(f"talking room {heads} {kv} {dim} {vdim} {portions}")
+    lens = [300, 7, 40]
+    case = Talking(lens, heads, kv, dim, vdim, BF, seed=12).solve()
+    case.check([(i % 3, lens[i % 3] - 1 - i % 2, 1 + i % 2) for i in range(portions - 1)] + [(0, 0, 300)], room=65535)
 
 
 MISSING = [  # kernels with waves of two kinds: 16 heads, 8, sizes with padding; of one kind: 16 heads with keys staged by all and by each wave, up to 32
