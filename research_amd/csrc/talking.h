@@ -16,7 +16,7 @@ struct TalkArgs : ScoredArgs {  // (q1, n1: the queries; cap, bias, sink, window
     int bs_shift;               // log2 of the block size, -1: it is no power of two
     uint32_t bs_magic;          // key / block size = (2 key * bs_magic >> 32) >> bs_magic_shift (key < 2^31)
     int bs_magic_shift;
-    unsigned at_once;           // workgroups that the device has room for
+    bool in_order;              // portions: workgroups take the blocks of rows in the order of their keys
 };
 
 // scored_block_id and scored_slot_of without a division where the block size allows it (key < 2^31, bt_stride > 0)

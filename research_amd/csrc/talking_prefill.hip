@@ -550,19 +550,13 @@ template <int DV, int G> struct TpTile {  // G: fours of heads, 2 or 4
 // A value that is the same in all lanes, as a scalar
 __device__ __forceinline__ float tp_scalar(float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); }
 
-// Which block of 16 rows of which portion has `rank` in their order from the rows furthest behind to the first ones, and that portion (each wave by
-// itself; what is known of up to 64 portions is loaded once).
+// Which block of 16 rows of which of up to 64 portions has `rank` in their order from the rows furthest behind to the first ones, and that portion (each
+// wave by itself).
 __device__ __forceinline__ bool tp_block(const TalkArgs &a, int rank, int &b, int &block, ScoredPortion &p) {
     const int lane = threadIdx.x & 63, most = (a.max_q_len + kTpRows - 1) / kTpRows;
     ScoredPortion mine;
-    auto load = [&](int first) { return first + lane < a.batch && scored_portion(a, first + lane, mine) ? min((mine.n + kTpRows - 1) / kTpRows, most) : 0; };
-    int blocks = load(0);
-    auto behind = [&](int i) {  // blocks whose number in their portion is at least i
-        if (a.batch <= 64) return __builtin_amdgcn_readlane(la_scan(max(blocks - i, 0), lane), 63);
-        int n = 0;
-        for (int first = 0; first < a.batch; first += 64) n += max(load(first) - i, 0);
-        return __builtin_amdgcn_readlane(la_scan(n, lane), 63);
-    };
+    const int blocks = lane < a.batch && scored_portion(a, lane, mine) ? min((mine.n + kTpRows - 1) / kTpRows, most) : 0;
+    auto behind = [&](int i) { return __builtin_amdgcn_readlane(la_scan(max(blocks - i, 0), lane), 63); };  // blocks whose number in their portion is at least i
     if (rank >= behind(0)) return false;
     int low = 0, high = most;  // behind(low) > rank >= behind(high)
     while (high - low > 1) {
@@ -572,21 +566,12 @@ __device__ __forceinline__ bool tp_block(const TalkArgs &a, int rank, int &b, in
     }
     block = low;
     rank -= behind(high);
-    for (int first = 0; first < a.batch; first += 64) {
-        if (a.batch > 64) blocks = load(first);
-        const uint64_t there = __ballot(blocks > low);
-        const int n = __builtin_popcountll(there);
-        if (rank < n) {
-            const int at = __builtin_ctzll(__ballot((there >> lane & 1) != 0 && __builtin_popcountll(there & ((1ull << lane) - 1)) == rank));
-            b = first + at;
-            p.n = __builtin_amdgcn_readlane(mine.n, at);
-            p.pos0 = __builtin_amdgcn_readlane(mine.pos0, at);
-            p.row0 = __builtin_amdgcn_readlane((int)mine.row0, at);  // (q_starts has 32 bits)
-            return true;
-        }
-        rank -= n;
-    }
-    return false;
+    const uint64_t there = __ballot(blocks > low);
+    b = __builtin_ctzll(__ballot((there >> lane & 1) != 0 && __builtin_popcountll(there & ((1ull << lane) - 1)) == rank));
+    p.n = __builtin_amdgcn_readlane(mine.n, b);
+    p.pos0 = __builtin_amdgcn_readlane(mine.pos0, b);
+    p.row0 = __builtin_amdgcn_readlane((int)mine.row0, b);  // (q_starts has 32 bits)
+    return true;
 }
 
 template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G, 4) void talk_pipe_kernel(const TalkArgs a) {
@@ -594,10 +579,12 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     constexpr int KS = DK / 32, NC = L::cols / 32;
     typedef float f16 __attribute__((ext_vector_type(16)));
     extern __shared__ __align__(16) char tm_lds[];
-    // Workgroups that are all there at once take any block; else those with the most keys come first.
-    int b = blockIdx.x, block = blockIdx.y;
+    // Blocks with the most keys first: in order over all portions where those can be looked over by a wave at once and not all workgroups begin together
+    // anyway, else in every portion.  (Beyond 64 portions a look takes as many loads in a row as there are 64s of them, and a search ten looks: 16 / 4 heads
+    // of 128, 511 of 16 .. 64 rows and one of 300 287 us, without the search 155; 8 / 2 of 64, 200 of 1 .. 1000 514, 384.)
+    int b = talk_sequence(a, blockIdx.x, blockIdx.y), block = (int)(gridDim.y - 1 - blockIdx.y);
     ScoredPortion p;
-    if (gridDim.x * gridDim.y > a.at_once ? !tp_block(a, (int)(blockIdx.y * gridDim.x + blockIdx.x), b, block, p) : !scored_portion(a, b, p)) return;
+    if (a.in_order ? !tp_block(a, (int)(blockIdx.y * gridDim.x + blockIdx.x), b, block, p) : !scored_portion(a, b, p)) return;
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
     const int all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = all % L::part;
     char *w_all = tm_lds + 2 * L::pTile, *v_all = w_all + 2 * L::wTile;
@@ -864,7 +851,7 @@ template <int DK, int DV, int G, bool FULL> int launch_pipe(const TalkArgs &a, h
     // (two dimensions: in one, the threads of 1024 portions of up to 65535 rows are more than a launch can have)
     const dim3 grid((unsigned)a.batch, (unsigned)((a.max_q_len + kTpRows - 1) / kTpRows));
     TalkArgs args = a;
-    args.at_once = (unsigned)(la_cus() * (4 / G));
+    args.in_order = a.batch <= 64 && (int64_t)grid.x * grid.y > (int64_t)la_cus() * (4 / G);
     talk_pipe_kernel<DK, DV, G, FULL><<<grid, dim3(TpTile<DV, G>::threads), lds, s>>>(args);
     PA_CHECK_LAUNCH("pa_talking_attention (portions)");
     return PA_OK;

@@ -148,6 +148,8 @@ class Talking:
     def check(self, picks, **kw):
         # (errors against the size of the rows: mixed weights have both signs and their sums may nearly cancel)
         for (b, at, n), got in zip(picks, self.run(picks, **kw)):
+            if not n:
+                continue
             want = self.want[b][at: at + n]
             err = (got.double() - want).abs() / (1.0 + want.abs())
             assert torch.isfinite(got.double()).all()
@@ -187,13 +189,24 @@ def test_prompts_of_many_tiles(heads, kv, dim, vdim):
 
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(16, 4, 128, 128), (12, 3, 72, 120), (12, 1, 64, 128), (8, 2, 64, 64), (4, 1, 104, 24), (8, 1, 128, 128)])
 def test_prompts_with_more_blocks_of_rows_than_workgroups_side_by_side(heads, kv, dim, vdim):
-    """Kernels with waves of two kinds: 16 rows each, one to ten tiles of keys, in order of their keys over more than 64 portions."""
+    """Kernels with waves of two kinds: 16 rows each, one to ten tiles of keys, over more than 64 portions."""
     announce(f"talking blocks {heads} {kv} {dim} {vdim}")
     lens = [300, 16, 33, 129, 161]
     case = Talking(lens, heads, kv, dim, vdim, BF, seed=11, odd_talk=True).solve()
     case.check([(i % 5, 0, lens[i % 5]) for i in range(70)])
     case.check([(i % 5, lens[i % 5] - 1 - i % 3, 1 + i % 3) for i in range(600)])
     case.check([(0, 283, 17), (4, 160, 1)])
+
+
+@pytest.mark.parametrize("portions", [32, 63, 64, 65])
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(16, 4, 128, 128), (8, 2, 64, 64)])
+def test_blocks_of_rows_in_order_of_their_keys(heads, kv, dim, vdim, portions):
+    """Up to 64 portions whose blocks are more than begin side by side go in order over all portions; more than 64 not.  Some without rows."""
+    announce(f"talking order {heads} {kv} {dim} {vdim} {portions}")
+    lens = [300, 17, 160, 1, 96]
+    case = Talking(lens, heads, kv, dim, vdim, BF, seed=14).solve()
+    case.check([(i % 5, 0, lens[i % 5] if i % 7 else 0) for i in range(portions)])
+    case.check([(0, 300 - 4 * i, 4 * i) for i in range(portions)] + [(0, 0, 300)])
 
 
 @pytest.mark.parametrize("heads,kv,dim,vdim,portions", [(16, 4, 128, 128, 1024), (8, 2, 64, 64, 2049)])
