@@ -632,11 +632,14 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
         const int my_key = 16 * half + l16;
         bf8 kr[KS];
         auto fetch = [&](int slot) {
-            const uintptr_t src = slot < 0 ? reinterpret_cast<uintptr_t>(kTalkNoKey) + 16 * g : reinterpret_cast<uintptr_t>(kp + (uint64_t)(uint32_t)slot * k_tok);
+            const char *src = kp + (uint64_t)(uint32_t)slot * k_tok;
+            auto load = [&](bool there) {
 #pragma unroll
-            for (int k = 0; k < KS; ++k)
-                kr[k] = __builtin_bit_cast(bf8, FULL ? *reinterpret_cast<talk_global>(src + 64 * k)
-                                                     : scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, 32 * k + 8 * g < a.n1));
+                for (int k = 0; k < KS; ++k)
+                    kr[k] = __builtin_bit_cast(bf8, scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, there && (FULL || 32 * k + 8 * g < a.n1)));
+            };
+            if (__ballot(slot < 0) == 0) load(true);  // (a choice of addresses for each load in place of a branch: 1 to 2 % of a call)
+            else load(slot >= 0);
         };
         // (distances first_pos + r - k of 16 rows and 16 keys, from their smallest, of two heads a lane; a key behind its row gets no weight)
         float size[2], rate[2];
@@ -744,11 +747,15 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     scored_u4 vr[NV];
     auto fetch = [&](int k0) {
         const int *slots = ring + ((k0 + my_key) & (L::ring - 1));
+        int slot[NV], least = 0;
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            const int slot = slots[n * kEach];
-            vr[n] = scored_load16(reinterpret_cast<const uint16_t *>(vp + (uint64_t)(uint32_t)slot * v_tok), slot >= 0);
-        }
+        for (int n = 0; n < NV; ++n) least |= slot[n] = slots[n * kEach];
+        auto load = [&](auto there) {
+#pragma unroll
+            for (int n = 0; n < NV; ++n) vr[n] = scored_load16(reinterpret_cast<const uint16_t *>(vp + (uint64_t)(uint32_t)slot[n] * v_tok), there(slot[n]));
+        };
+        if (__ballot(least < 0) == 0) load([](int) { return true; });
+        else load([](int x) { return x >= 0; });
     };
     auto put_v = [&]() {
 #pragma unroll
