@@ -69,14 +69,17 @@ def test_lines_of_wide_groups_and_of_32_bits(plan):
 
 
 def test_results_of_the_runs_fit_the_workspace(plan):
-    rng = np.random.default_rng(0)
+    rng, took = np.random.default_rng(0), {1: 0, 2: 0, 4: 0}
     for _ in range(20000):
         hkv, rep = int(rng.choice([1, 2, 3, 4, 8, 16, 40])), int(rng.choice([1, 2, 3, 4, 5, 7, 8, 12, 16, 17, 40]))
-        bytes_ = int(rng.choice([1, 2]))
-        d = int(rng.choice([64, 128, 256] if bytes_ == 1 else [8, 32, 64, 72, 96, 128, 192, 256]))
+        bytes_ = int(rng.choice([1, 2, 4]))
+        d = int(rng.choice([64, 128, 256] if bytes_ == 1 else [8, 16, 24, 32, 40, 64, 72, 96, 128, 192, 256]))  # (32 bits: of up to 32 as of 64)
+        bs, window = int(rng.choice([16, 32, 48, 256])), int(rng.choice([0, 0, 200, -5000]))
         batch, cap = int(rng.integers(1, 513)) if rng.random() < 0.5 else int(rng.integers(1, 9)), int(rng.choice([64, 512, 4096]))
-        n = plan.runs(batch, hkv * rep, hkv, d, bytes_, int(2 ** rng.uniform(0, 14)), 16, 0, cap)
-        assert 0 <= n <= 64 and (n == 0 or plan.fits(batch, hkv * rep, hkv, d, bytes_, n, cap)), (batch, hkv, rep, d, bytes_, cap, n)
+        n = plan.runs(batch, hkv * rep, hkv, d, bytes_, int(2 ** rng.uniform(0, 14)), bs, window, cap)
+        took[bytes_] += n > 1
+        assert 0 <= n <= 64 and (n == 0 or plan.fits(batch, hkv * rep, hkv, d, bytes_, n, cap)), (batch, hkv, rep, d, bytes_, bs, window, cap, n)
+    assert min(took.values()) > 500, took
 
 
 EDGES = [1, 15, 16, 17, 31, 32, 33, 0, 47, 63, 64, 65, 127, 128, 129, 200, 255, 256, 257]
