@@ -1,6 +1,7 @@
 // Entry points of attention with mixed heads, and its kernels on the vector units: 32-bit rows, and sizes that the matrix-core
 // kernels (talking_decode.hip, talking_prefill.hip) do not have.
 #include "talking.h"
+#include "talking_plan.h"
 
 namespace {
 
@@ -150,8 +151,8 @@ extern "C" int pa_talking_attention(const void *q, int64_t q_row, int64_t q_head
     a.max_q_len = q_lens ? max_q_len : 1; a.heads = num_q_heads; a.hkv = num_kv_heads; a.n_rep = num_q_heads / num_kv_heads;
     a.scale = scale; a.out = out; a.splits = 1;
     a.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
-    while (a.bs_magic_shift < 31 && (1ll << a.bs_magic_shift) < block_size) ++a.bs_magic_shift;
-    a.bs_magic = (uint32_t)(((1ull << (31 + a.bs_magic_shift)) + block_size - 1) / block_size);
+    const TalkDivision by = talk_division(block_size);
+    a.bs_magic = by.mul; a.bs_magic_shift = by.shift;
     a.size = bias_size; a.rate = bias_rate; a.talk = talk; a.lse = (float *)workspace;
     hipStream_t s = (hipStream_t)stream;
     int rc = PA_OK;

@@ -14,6 +14,7 @@
 #include "linear_tiles.h"
 #include "prefill_mfma.h"
 #include "talking.h"
+#include "talking_plan.h"
 
 namespace {
 
@@ -530,8 +531,8 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
 // registers that 16 waves leave it.  Eight waves of twice the registers took as long (444 us), keys by way of LDS longer (452).
 // us a call, the kernel above -> this one: 16 / 4 heads of 128, 8 prompts of 818 .. 3868 rows 480 -> 428, one of 1100 106 -> 91; 8 / 2 of 128, one of 1100
 // 87 -> 59; 8 / 2 of 64, 11 of 534 .. 695 55 -> 47, 10 of 28 .. 145 17.1 -> 15.0.  Of more than 8 heads, calls whose blocks meet few keys stay with the kernel
-// above (tp_takes).
-constexpr int kTpRows = 16, kTpKeys = 32;
+// above (talk_pipe_takes).
+constexpr int kTpRows = kTalkPipeRows, kTpKeys = 32;
 template <int DV, int G> struct TpTile {  // G: fours of heads, 2 or 4
     static constexpr int heads = 4 * G, part = 2 * G, threads = 64 * 2 * part;       // waves of a kind
     static constexpr int pair = 16 * G, pTile = kTpKeys * kTpRows * pair;            // bytes of a (key, row) pair: both terms of all heads
@@ -850,21 +851,6 @@ template <int DK, int DV, int G, bool FULL> __global__ __launch_bounds__(256 * G
     }
 }
 
-// Whether a call of more than 8 heads goes to talk_pipe_kernel.  A workgroup of it has a compute unit to itself, and nothing covers its set-up; two of the
-// kernel above share one, which begin sooner.  So the keys that a block meets on average have to make up for each round of workgroups (as measured, for
-// no more than three); where blocks go in order over portions of unequal length, which ends the last round sooner, for one alone.  From shapes alone: the tables' width stands for the longest context.
-// us, the kernel above -> talk_pipe_kernel, prompts of n rows, 16 / 4 heads of 128: one round, 18 of 224 37.7 -> 38.3, 14 of 288 43.0 -> 42.5, 8 of 512 59 -> 56;
-// two, 18 of 300 50.8 -> 56.1, 12 of 416 54 -> 57, 9 of 512 61 -> 58; three, 22 of 512 111 -> 113, 12 of 896 148 -> 144; eight, 333 of 96 161 -> 176, 62 of 512
-// 292 -> 312, 50 of 640 323 -> 332, 36 of 896 390 -> 381; in order, 40 of 1 .. 400 76 -> 69, 40 of 300 .. 600 171 -> 163; 128 of 64 behind 300 97 -> 95.  Over 202 such
-// batches with 16 and 12 heads of 64 to 128 the choice takes 0.955 of the kernel above's time, 1.02 at worst (16 of 175 .. 355).
-bool tp_takes(const TalkArgs &a) {
-    const int64_t most = (a.max_q_len + kTpRows - 1) / kTpRows, cus = la_cus(), whole = (int64_t)a.batch * a.max_q_len;
-    const int64_t blocks = std::min(a.batch * most, a.n_rows / kTpRows + a.batch / 2), rounds = std::min<int64_t>((blocks + cus - 1) / cus, 3);
-    const bool uneven = a.batch <= 64 && 5 * a.n_rows <= 4 * whole;
-    const int64_t behind = std::max<int64_t>(a.bt_stride * a.bs - a.max_q_len, 0), mean = uneven ? a.max_q_len / 2 : std::min<int64_t>(a.max_q_len / 2, a.n_rows / a.batch);
-    return behind + mean >= 128 * (uneven ? 1 : rounds);
-}
-
 template <int DK, int DV, int G, bool FULL> int launch_pipe(const TalkArgs &a, hipStream_t s) {
     constexpr size_t lds = TpTile<DV, G>::bytes;
     static_assert(lds <= 160 * 1024 / (4 / G), "LDS of one compute unit");
@@ -872,7 +858,7 @@ template <int DK, int DV, int G, bool FULL> int launch_pipe(const TalkArgs &a, h
     // (two dimensions: in one, the threads of 1024 portions of up to 65535 rows are more than a launch can have)
     const dim3 grid((unsigned)a.batch, (unsigned)((a.max_q_len + kTpRows - 1) / kTpRows));
     TalkArgs args = a;
-    args.in_order = a.batch <= 64 && (int64_t)grid.x * grid.y > (int64_t)la_cus() * (4 / G);
+    args.in_order = talk_pipe_in_order(a.heads, a.batch, a.max_q_len, la_cus());
     talk_pipe_kernel<DK, DV, G, FULL><<<grid, dim3(TpTile<DV, G>::threads), lds, s>>>(args);
     PA_CHECK_LAUNCH("pa_talking_attention (portions)");
     return PA_OK;
@@ -914,7 +900,7 @@ bool pa_talking_prefill_launch(const TalkArgs &a, int dtype, hipStream_t s, int 
         if (a.n1 <= 64) talk_sums_kernel<64><<<grid, dim3(256), 0, s>>>(a);
         else talk_sums_kernel<128><<<grid, dim3(256), 0, s>>>(a);
         PA_CHECK_LAUNCH("pa_talking_attention (sums)");
-        if (a.heads <= 16 && a.n_rep % 4 == 0 && (a.heads <= 8 || tp_takes(a)) && (int64_t)a.hkv * (a.k_dim > a.v_dim ? a.k_dim : a.v_dim) < (1 << 30)) {
+        if (talk_pipe_takes(a.heads, a.n_rep, a.batch, a.max_q_len, a.n_rows, a.bt_stride * a.bs, la_cus()) && (int64_t)a.hkv * (a.k_dim > a.v_dim ? a.k_dim : a.v_dim) < (1 << 30)) {
             if (a.n1 <= 64) return a.vdim <= 64 ? launch_pipe_size<64, 64>(a, s) : launch_pipe_size<64, 128>(a, s);
             return a.vdim <= 64 ? launch_pipe_size<128, 64>(a, s) : launch_pipe_size<128, 128>(a, s);
         }

@@ -230,15 +230,15 @@ def test_delta_rule_remembers_a_far_token(dtype):
 
 
 class Paged:
-    """Keys and values of sequences in a pool of 16-token blocks in mixed order, blocks of other contents in between."""
+    """Keys and values of sequences in a pool of blocks in mixed order, blocks of other contents in between."""
 
-    def __init__(self, lens, kv, kd, vd, dtype, one=False, seed=0):
+    def __init__(self, lens, kv, kd, vd, dtype, one=False, seed=0, bs=16):
         g = np.random.default_rng(seed)
-        self.bs, self.lens = 16, lens
-        need = [-(-n // 16) for n in lens]
+        self.bs, self.lens = bs, lens
+        need = [-(-n // bs) for n in lens]
         ids = g.permutation(sum(need) + 5)
-        self.k = _rand((sum(need) + 5) * 16, kv, kd, seed=seed + 1).to(dtype)
-        self.v = self.k if one else _rand((sum(need) + 5) * 16, kv, vd, seed=seed + 2).to(dtype)
+        self.k = _rand((sum(need) + 5) * bs, kv, kd, seed=seed + 1).to(dtype)
+        self.v = self.k if one else _rand((sum(need) + 5) * bs, kv, vd, seed=seed + 2).to(dtype)
         self.tables = np.full((len(lens), max(need) + 2), -1, dtype=np.int32)
         at = 0
         for i, n in enumerate(need):
@@ -247,7 +247,7 @@ class Paged:
 
     def rows(self, pool, i, lo=0):
         p = np.arange(lo, self.lens[i])
-        return pool[torch.from_numpy(self.tables[i, p // 16].astype(np.int64) * 16 + p % 16)]
+        return pool[torch.from_numpy(self.tables[i, p // self.bs].astype(np.int64) * self.bs + p % self.bs)]
 
 
 def _scored(paged, picks, q, vdim, dtype, scale, window, decode=False, splits=True, **terms):
