@@ -5,10 +5,10 @@
 
 namespace {
 
-// The score of a key in units of the base-2 exponential (T float: library functions throughout)
-template <typename T> __device__ __forceinline__ float talk_score(const TalkArgs &a, int h, const T *q, const T *k, int dist) {
+// The score of a key in units of the base-2 exponential (T float: library functions throughout).  there: else its block is missing, a key of zeros.
+template <typename T> __device__ __forceinline__ float talk_score(const TalkArgs &a, int h, const T *q, const T *k, bool there, int dist) {
     float s = 0.f;
-    for (int e = 0; e < a.n1; ++e) s = fmaf(pa_scalar<T>::load(q + e), pa_scalar<T>::load(k + e), s);
+    for (int e = 0; e < (there ? a.n1 : 0); ++e) s = fmaf(pa_scalar<T>::load(q + e), pa_scalar<T>::load(k + e), s);
     s *= a.scale;
     if (a.size) s -= a.size[h] * logf(fmaf(a.rate[h], (float)dist, 1.f));
     return s * kScoredLog2e;
@@ -27,7 +27,7 @@ template <typename T> __global__ __launch_bounds__(256) void talk_lse_vector_ker
     float m = kScoredNone, l = 0.f;
     for (int j = lane; j <= pos; j += 64) {
         const int64_t slot = scored_slot(a, table, j);
-        const float s = slot >= 0 ? talk_score<T>(a, h, q, k + slot * ((int64_t)a.hkv * a.k_dim), pos - j) : kScoredNone;
+        const float s = talk_score<T>(a, h, q, k + (slot < 0 ? 0 : slot) * ((int64_t)a.hkv * a.k_dim), slot >= 0, pos - j);
         const float next = fmaxf(m, s);
         l = l * exp2f(m - next) + exp2f(s - next);
         m = next;
@@ -61,7 +61,7 @@ template <typename T, int VPT> __global__ __launch_bounds__(256) void talk_mix_v
         for (int h = wave; h < a.heads; h += 4) {
             const T *k = reinterpret_cast<const T *>(a.k) + (slot < 0 ? 0 : slot) * ((int64_t)a.hkv * a.k_dim) + (h / a.n_rep) * a.k_dim;
             p_s[h * kTalkKeys + lane] =
-                slot >= 0 ? exp2f(talk_score<T>(a, h, q + h * a.q1_head, k, pos - j) - a.lse[row * a.heads + h]) : 0.f;
+                j <= pos ? exp2f(talk_score<T>(a, h, q + h * a.q1_head, k, slot >= 0, pos - j) - a.lse[row * a.heads + h]) : 0.f;
         }
         __syncthreads();
         for (int n = tid; n < a.heads * kTalkKeys; n += 256) {

@@ -246,15 +246,16 @@ def test_many_prompts_with_room_for_long_ones(heads, kv, dim, vdim, portions):
 
 
 MISSING = [  # kernels with waves of two kinds: 16 heads, 8, sizes with padding; of one kind: 16 heads with keys staged by all and by each wave, up to 32
-    (16, 4, 128, 128), (8, 2, 64, 64), (12, 1, 72, 120), (6, 3, 128, 128), (6, 2, 40, 56), (32, 8, 128, 128), (24, 8, 64, 128)]
+    (16, 4, 128, 128, BF), (8, 2, 64, 64, BF), (12, 1, 72, 120, BF), (6, 3, 128, 128, BF), (6, 2, 40, 56, BF), (32, 8, 128, 128, BF), (24, 8, 64, 128, BF),
+    (20, 4, 72, 64, BF), (16, 16, 64, 64, BF), (5, 5, 136, 200, BF), (16, 4, 128, 128, F32), (6, 2, 40, 56, F32), (34, 2, 24, 72, F32)]  # (and on the vector units)
 
 
-@pytest.mark.parametrize("heads,kv,dim,vdim", MISSING)
-def test_missing_blocks_are_rows_of_zeros(heads, kv, dim, vdim):
+@pytest.mark.parametrize("heads,kv,dim,vdim,dtype", MISSING)
+def test_missing_blocks_are_rows_of_zeros(heads, kv, dim, vdim, dtype):
     """The first block, one in the middle and the last one of a sequence, by a negative id and by ids outside the pool: keys and values of zeros."""
-    announce(f"talking missing {heads} {kv} {dim} {vdim}")
+    announce(f"talking missing {heads} {kv} {dim} {vdim} {dtype}")
     lens = [330, 70]
-    case = Talking(lens, heads, kv, dim, vdim, BF, seed=13)
+    case = Talking(lens, heads, kv, dim, vdim, dtype, seed=13)
     outside = case.paged.k.shape[0] // 16
     case.solve([(0, 0, -1), (0, 7, outside), (0, 20, 1 << 30), (1, 2, -5), (1, 4, outside)])
     case.check([(i, 0, n) for i, n in enumerate(lens)])
@@ -262,10 +263,10 @@ def test_missing_blocks_are_rows_of_zeros(heads, kv, dim, vdim):
     case.check([(i, n - 1, 1) for i, n in enumerate(lens)], decode=True)
 
 
-@pytest.mark.parametrize("heads,kv,dim,vdim", MISSING)
-def test_a_pool_without_a_whole_block_is_zeros(heads, kv, dim, vdim):
-    announce(f"talking empty pool {heads} {kv} {dim} {vdim}")
-    case = Talking([290], heads, kv, dim, vdim, BF)
+@pytest.mark.parametrize("heads,kv,dim,vdim,dtype", MISSING)
+def test_a_pool_without_a_whole_block_is_zeros(heads, kv, dim, vdim, dtype):
+    announce(f"talking empty pool {heads} {kv} {dim} {vdim} {dtype}")
+    case = Talking([290], heads, kv, dim, vdim, dtype)
     case.paged.k, case.paged.v = case.paged.k[:8].contiguous(), case.paged.v[:8].contiguous()
     case.want = [torch.zeros(290, heads, vdim, dtype=torch.float64)]
     case.check([(0, 0, 290)])
