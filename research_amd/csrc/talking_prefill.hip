@@ -237,7 +237,13 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     const int v_kv0 = kv_of(out0);
     __bf16 *v_s = v_all + (SAME ? kv_of(own0) - v_kv0 : wave) * L::vTile;
     // Block and pool row of the key that this thread stages (values staged by all: the piece of a tile; else key lane % 32); past
-    // the last key: the last one's, which nothing weighs.  -1: its block is missing, a key and a value of zeros.
+    // the last key: the last one's, which nothing weighs.  -1: its block is missing, a key and a value of zeros.  LATE: the pool's first row is loaded then, and
+    // zeros take its place where the loads are waited for, in a branch that no other tile takes; else by a choice of addresses for each load, where the
+    // branch costs registers that are spilled or saves nothing.  (us, no zeros -> by choice -> LATE: 8 prompts of 818 .. 3868 rows, 6 / 3 heads of 128
+    // 451 -> 462 -> 458; 18 of 300, 16 / 4 of 128 46.9 -> 48.3 -> 47.2; kernel alone, heads of a wave of two kv heads, 6 / 2 of 40 x 56 351 -> 370 -> 369, 24 / 8
+    // of 64 1040 -> 1083 -> 1104.)
+    constexpr bool LATE = SAME && (HW == 2 || D == 64);
+    uint64_t k_gone = 0, v_gone = 0;  // LATE: the lanes whose keys are missing of the tiles in kr and vr
     const int my_row = SAME ? tid % kTile / kPer : lane & 31;
     auto key_of = [&](int k0) { return min(k0 + my_row, end - 1); };
     auto id_of = [&](int k0) { return talk_block_id(a, table, key_of(k0)); };
@@ -245,11 +251,11 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     scored_u4 kr[NK], vr[NV];
     // staged by the workgroup: piece tid + 512 n is of kv head (tid + 512 n) / kTile, the thread's own row
     auto stage_from = [&](const void *pool, int slot, uint32_t tok, int head_dim, int kv_first, int real, scored_u4 *to) {
-        const uint16_t *src = reinterpret_cast<const uint16_t *>(pool) + (uint64_t)(uint32_t)slot * tok + tid % kPer * 8;
+        const uint16_t *src = reinterpret_cast<const uint16_t *>(pool) + (uint64_t)(uint32_t)(LATE ? max(slot, 0) : slot) * tok + tid % kPer * 8;
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
             const uint16_t *at = src + min(kv_first + (tid + kTmThreads * n) / kTile, a.hkv - 1) * head_dim;
-            to[n] = scored_load16(at, slot >= 0 && (FULL || tid % kPer * 8 < real));
+            to[n] = scored_load16(at, (LATE || slot >= 0) && (FULL || tid % kPer * 8 < real));
         }
     };
     auto stage_to = [&](__bf16 *tiles, int tile, int row_at, const scored_u4 *from) {
@@ -262,8 +268,8 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
                 const int slot = __shfl(slots, 16 * kb + l16, 64);
-                const uint16_t *pool = reinterpret_cast<const uint16_t *>(a.k) + (uint64_t)(uint32_t)slot * k_tok + kv * a.k_dim;
-                const uintptr_t src = (slot < 0 ? reinterpret_cast<uintptr_t>(kTalkNoKey) : reinterpret_cast<uintptr_t>(pool)) + 16 * g;
+                const uint16_t *pool = reinterpret_cast<const uint16_t *>(a.k) + (uint64_t)(uint32_t)(LATE ? max(slot, 0) : slot) * k_tok + kv * a.k_dim;
+                const uintptr_t src = (LATE || slot >= 0 ? reinterpret_cast<uintptr_t>(pool) : reinterpret_cast<uintptr_t>(kTalkNoKey)) + 16 * g;
 #pragma unroll
                 for (int k = 0; k < KS; ++k)
                     kr[kb * KS + k] = FULL ? *reinterpret_cast<talk_global>(src + 64 * k) : scored_load16(reinterpret_cast<const uint16_t *>(src) + 32 * k, 32 * k + 8 * g < a.n1);
@@ -271,6 +277,7 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
         }
     };
     auto fetch_k = [&](int slots, int near) {  // (near: the slots of keys lane % 32)
+        if constexpr (LATE) k_gone = __ballot((L::ahead ? slots : near) < 0);
         if constexpr (L::ahead) stage_from(a.k, slots, k_tok, a.k_dim, 0, a.n1, kr);
         else direct_k(kv_of(head0), near);
     };
@@ -285,10 +292,15 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
         }
     };
     auto fetch_v = [&](int slots) {
+        if constexpr (LATE) v_gone = __ballot(slots < 0);
         if constexpr (SAME) stage_from(a.v, slots, v_tok, a.v_dim, v_kv0, vreal, vr);
         else own_v(kv_of(own0), slots);
     };
     auto put_v = [&]() {
+        if (LATE && (v_gone >> lane & 1)) {
+#pragma unroll
+            for (int n = 0; n < NV; ++n) vr[n] = scored_u4{0, 0, 0, 0};
+        }
         if constexpr (SAME) {
             stage_to(v_all, L::vTile, L::vRow(my_row), vr);
         } else {
@@ -321,6 +333,13 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
             if (lane < 48) biases[i * 48 + lane] = x;
         }
         tp_own_lds();
+        if constexpr (LATE && !L::ahead) {
+            if (k_gone != 0) {
+#pragma unroll
+                for (int i = 0; i < 2 * KS; ++i)
+                    if (k_gone >> (16 * (i / KS) + l16) & 1) kr[i] = scored_u4{0, 0, 0, 0};
+            }
+        }
         auto weights = [&](int i, int kb, f4 s, float *w) {
             const float *bp = biases + i * 48 + l16 + 31 - 16 * kb - 4 * g;
 #pragma unroll
@@ -441,7 +460,13 @@ template <int D, int HW, bool FULL, int NG> __global__ __launch_bounds__(kTmThre
     fetch_k(slots, near_slot(near_id(0), 0, slots));
     fetch_v(slots);
     auto put_k = [&] {
-        if constexpr (L::ahead) stage_to(k_s, L::kTile, my_row * L::kPitch, kr);
+        if constexpr (L::ahead) {
+            if (LATE && (k_gone >> lane & 1)) {
+#pragma unroll
+                for (int n = 0; n < NK; ++n) kr[n] = scored_u4{0, 0, 0, 0};
+            }
+            stage_to(k_s, L::kTile, my_row * L::kPitch, kr);
+        }
     };
     if constexpr (L::ahead) {
         put_k();
@@ -891,7 +916,7 @@ bool pa_talking_prefill_launch(const TalkArgs &a, int dtype, hipStream_t s, int 
     const int most = a.n1 > a.vdim ? a.n1 : a.vdim;
     const uintptr_t at = (uintptr_t)a.q1 | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out;
     if (dtype != PA_BF16 || !a.q_lens || most > 128 || a.heads > 32 || (at & 15u) != 0 || a.n1 % 8 != 0 || a.k_dim % 8 != 0 ||
-        a.v_dim % 8 != 0 || a.q1_row % 8 != 0 || a.q1_head % 8 != 0 || a.num_blocks * a.bs >= 0x7fffffff || a.bt_stride == 0 || !(a.scale > 0.f))
+        a.v_dim % 8 != 0 || a.q1_row % 8 != 0 || a.q1_head % 8 != 0 || a.num_blocks * a.bs >= 0x7fffffff || a.num_blocks == 0 || a.bt_stride == 0 || !(a.scale > 0.f))
         return false;
     rc = [&]() -> int {
         const int groups = ((a.max_q_len + 31) / 32 * a.n_rep + 3) / 4;
