@@ -210,7 +210,7 @@ int decode_launch(int phases, const void *q, const void *k_cache, const void *v_
         a.leave = a.splits > 1 || phases != (kPhaseSplit | kPhaseReduce) ? 1 : 0;
         if (phases & kPhaseSplit) {
             const int reps = (plan.n_rep + kPlanShortHeads - 1) / kPlanShortHeads;
-            ks.few<<<dim3((unsigned)num_kv_heads, (unsigned)batch, (unsigned)(reps * a.splits)), dim3(kThreads), 0, s>>>(a);
+            ks.few<<<dim3((unsigned)num_kv_heads, (unsigned)(reps * a.splits), (unsigned)batch), dim3(kThreads), 0, s>>>(a);
             PA_CHECK_LAUNCH("pa_decode (short sequences)");
         }
         if ((phases & kPhaseReduce) && a.leave) {
