@@ -198,7 +198,8 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // run).  From shapes alone; the tables' width stands for the longest sequence.
 // Head sizes up to 32 over 16 bits and fp8 stay with the generic loop of the split pass, whose weights have 32 bits: 11.8 us for 16 sequences of 16 .. 250 keys, 4 / 4
 // heads of 32, where weights of two bf16 terms took 5.0, but erred by up to 1.1e-6 of the sum of |weight value| where 32 bits err by 0.2e-6.
-// Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch (2.5 us, with the lines of 16 bits where 3.5 were measured: 600 keys of 128).
+// Runs: one for each compute unit, of at least 128 keys, where the longest sequence takes longer than a merging launch: from 600 keys of 128 on over 16 bits and fp8 (measured with a merge
+// of 3.5 us), from 256 on over 32 bits (with the present one, 2.5 us).
 // us, the split pass (one launch or two) -> this, sequences of n keys each: 32 / 8 heads of 128, 1 of 256 keys 14.1 -> 7.4, 1024 15.5 -> 9.0, 4096
 // 16.2 -> 12.0; 32 of 256 19.6 -> 8.3; 96 of 256 33.9 -> 19.7; 14 / 2 of 64, 1 of 256 15.2 -> 5.8, 4096 16.4 -> 11.0; 32 of 1024 22.1 -> 11.0, 16384
 // 64 -> 51; 192 of 1024 45 -> 21; fp8 32 / 8 of 128, 32 of 256 24.5 -> 6.8; fp8 14 / 2 of 256, 16 of 2048 47 -> 14.5, 256 of 2048 185 -> 91.
@@ -215,17 +216,21 @@ PA_PLAN_FN bool plan_merge_in_split(int batch, const HeadPlan &h, int grid) {
 // keys of 128 cut in two where the units have room for it (fp8 16 / 2 of 128, 17 of 12251 29 -> 20, 5 of 57391 36 -> 26; of 256 not: 38 of 4315 35 -> 38); over
 // fp8 up to four heads more in all, of 256 longer ones too (32 / 8 of 128, 93 of 763 41 -> 25, of 256, 68 of 565 43 -> 21; 16 / 8 of 256, 1 of 8756 25 ->
 // 15; but 32 / 8 of 128, 66 of 2214 65 -> 70).  From three heads of 64 on, runs begin at 800 keys while they are few (32 / 8, 3 of 1040 10.8 -> 7.9).
-// (Over 400 drawn batches of more than 600 keys of 128, with the faster merge, 0.92 of the time before, the slowest 1.04.)
-// 32-bit pools, the split pass -> this: from five query heads a kv head on always (runs of up to 2 MB, as far as measured, but for 16 / 2 of 64 and the like, 1 of 81903 30 -> 33: the split pass spends a vector
-// instruction on every head, key and element; 14 / 2 of 72, 105 of 34 .. 127 keys 26.7 -> 8.1, 16 / 2 of 128, 102 of 236 51 -> 24, 23 of 6812 86 -> 57, 1 of 20000 at 24 /
-// 2 37 -> 26).  Three or four: up to 48 MB of keys (32 / 8 of 64, 4 of 155 14.5 -> 8.2, 8 / 2 of 128, 29 of 819 20 -> 17; beyond, unequal, 32 / 8 of 128,
-// 7 of 33764 160 -> 340), unless more than four rounds of workgroups have few keys each (32 / 8 of 64, 206 of 53 13.4 -> 15.0; at 256 more than one, 8 / 2, 163 of 138 21 -> 26) or the few there are
+// (Over 321 batches over 16 bits and 216 over fp8, such lengths, 0.90 and 0.85 of the time before these lines, the slowest 1.04.)
+// 32-bit pools, the split pass -> this: from five query heads a kv head on wherever a run of the longest sequence, which all others may have to wait for, is short enough; the split pass spends a vector
+// instruction on every head, key and element, but divides any batch equally (14 / 2 of 72, 105 of 34 .. 127 keys 26.7 -> 8.1, 16 / 2 of 128, 102 of 236 51 -> 24).  Runs of 192 KB at up to 64
+// elements a row (14 / 2 of 64, 64 of 30000 and 1500 48 -> 179 in runs of 940 KB, 8 of 22400 and 1120 23 -> 34 of 350, equal steps 32 -> 29; 16 of 8000 23 -> 19 of 125), of 384 where sequences
+// are so few that each has 32 runs (1 of 40000 26 -> 20, 81920 35 -> 33, 130000 42 -> 47) or there are two workgroups for every four units without runs (200 of 4000 122 -> 51); above 64 416
+// (5 / 1 of 128, 1 of 60000, runs of 470 KB, 34 -> 37; 40 / 8 of 128, 4 of 5600, 350, 44 -> 30) and 832 (40 / 8 of 128, 100 of 1000 155 -> 80, 14 / 2 of 256, 250 of 1000 274 -> 126).
+// Three or four: up to 48 MB of keys, in runs of 176 KB (32 / 8 of 64, 4 of 155 14.5 -> 8.2, 8 / 2 of 128, 29 of 819 20 -> 17; beyond, runs of 200 KB, 32 / 8 of 256,
+// 3 of 2000 23 -> 27, of 64, 3 of 8000 24 -> 24, one of 8000 among 400 20 -> 23; unequal, of 128, 7 of 33764 160 -> 340), unless more than four rounds of workgroups have few keys each (32 / 8 of 64, 206 of 53 13.4 -> 15.0; at 256 more than one, 8 / 2, 163 of 138 21 -> 26) or the few there are
 // have long runs (8 / 2 of 128, 2 of 4000 15.6 -> 18.1, of 64, 8 of 6831 16.5 -> 18.2; of 256, 2 of 1964 17.6 -> 18.6).  One or two: a run each, up to 32 MB
 // and two rounds (16 / 8 of 128, 1 of 176 12.5 -> 8.6, 28 of 94 15.0 -> 8.9; 187 of 21 13.4 -> 18.1, 8 / 8 of 64, 16 of 600 14.5 -> 15.2).  A run is cut where four
 // turns of the waves, at 256 two, take longer than a merging launch: 16 keys of 128 each in 1 us (14 / 2 of 256, 6 of 228 in one run 20.7, of 64 keys 16.4, of
 // 32 11.9; 14 / 2 of 128, 16 of 101 8.2, in three 9.4); where most units have a workgroup anyway into two runs a unit, from five heads on four (unequal:
 // 14 / 2 of 72, 140 of 1600 71 -> 78, with four 50; equal 116 -> 100, 77).
-// (Over 740 drawn batches over 32-bit pools the two took 0.71 of the time that the split pass took alone.)
+// (Over 3053 batches over 32-bit pools, from five heads on, lengths in equal steps, drawn ones, one long one among others of a twentieth: 0.68, 0.73 and 0.77 of the split pass's time;
+// 76 were slower by more than 2 %, by up to 1.4: 5 / 1 of 128, one of 8000 among 199 of 400 46 -> 64.)
 // (Over 1200 shapes of 1 .. 128 sequences that this takes, from 600 keys of 128 on, equal and unequal, 16 of 3600 batches were slower by more than 2 %, of which 4 / 4 heads of 96
 // over fp8 by up to 19, 30 of 1482 keys 15.6 -> 18.6, the others by up to 6; on average they took 0.55 of the split pass's time.)
 constexpr int kPlanShortHeads = 16, kPlanShortTile = 16, kPlanShortRuns = 64;
@@ -256,10 +261,12 @@ PA_PLAN_FN int plan_short_splits(int batch, const HeadPlan &h, const WsPlan &w, 
     const bool few = h.n_rep <= 4 && wgs < 6 && keys > 4096 && !wide8;
     if (f32) {
         const bool lone = keys > 3072 ? wgs < (d == 64 ? 24 : 6) : d == 256 && !brief && wgs < 8;
-        const bool fits = h.n_rep > 4   ? d > 64 || wgs >= 6 || keys <= 8192
-                          : h.n_rep > 2 ? !lone && wgs <= (d == 256 ? 1 : 4) * (int64_t)cus && wgs * keys * row <= 48 * kb * kb
+        const bool full = 2 * wgs >= cus, spread = 32 * wgs <= cus && h.d_pad >= 64;
+        const int64_t most = (d > 64 ? (full ? 832 : 416) : full || spread ? 384 : 192) * kb;
+        const bool fits = h.n_rep > 4   ? keys / runs * row <= most
+                          : h.n_rep > 2 ? !lone && wgs <= (d == 256 ? 1 : 4) * (int64_t)cus && wgs * keys * row <= 48 * kb * kb && keys / runs * row <= 176 * kb
                                         : d < 256 && brief && wgs <= 2 * (int64_t)cus && wgs * keys * row <= 32 * kb * kb;
-        return fits && keys / runs * row <= 2048 * kb && runs * reps <= 65535 ? (int)runs : 0;
+        return fits && runs * reps <= 65535 ? (int)runs : 0;
     }
     const bool thin = kv_elem_bytes == 1 && h.d_pad == 64 && h.n_rep <= 2 && keys / runs > 768;
     const bool fits = (brief || keys / runs * row <= run_most) && wgs * keys * row <= all_most && !few && !thin;

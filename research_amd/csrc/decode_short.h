@@ -91,7 +91,7 @@ template <typename QT, typename Num> __device__ __forceinline__ void short_store
 // Neighbouring workgroups have the heads and runs of one sequence, the sequences come one after the other (z): with the runs further apart, as many
 // as there are sequences and heads, all runs of a long one came to few compute units, often after every other one had run.  us, one sequence of n keys among
 // others of n / 20, runs furthest apart -> next to each other: 32-bit 14 / 2 heads of 64, 64 of 11200 74 -> 38; 40 / 8 of 128, 16 of 2800 34 -> 26; 16-bit
-// 40 / 8 of 128, 16 of 5600 50 -> 24; fp8 14 / 2 of 256, 64 of 5600 0.65 of the time.  (Over 1458 batches, equal steps of length, drawn ones and such: 0.96, 0.95 and 0.92.)
+// 40 / 8 of 128, 16 of 5600 50 -> 24; fp8 14 / 2 of 256, 64 of 5600 0.65 of the time.  (Over 486 batches each of equal steps of length, drawn ones and such: 0.97, 0.95 and 0.93.)
 template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads, D == 256 || (sizeof(KV) == 4 && D == 128) ? 2 : sizeof(KV) == 4 ? 3 : 4) void decode_short_kernel(const DecodeArgs a) {
     using M = ShortMfma<QT>;
     constexpr bool kFp8 = sizeof(KV) == 1, k32 = sizeof(KV) == 4;

@@ -64,7 +64,13 @@ def test_lines_of_wide_groups_and_of_32_bits(plan):
     assert runs(3, (32, 8, 64, 2), 800) == 1 and runs(3, (32, 8, 64, 2), 816) == 6
     f32, wide = (14, 2, 64, 4), (32, 8, 128, 4)
     assert runs(4, f32, 512) == 1 and runs(4, f32, 528) == 4 and runs(4, wide, 256) == 1 and runs(4, wide, 272) == 4 and runs(140, (14, 2, 72, 4), 1600) == 3
-    assert runs(1, f32, 8192) == 64 and runs(1, f32, 8208) == 0 and runs(4, (8, 2, 32, 4), 64) == 1
+    # the longest run that a batch may wait for: 384 KB of few sequences and where most units have a workgroup, else 192; above 64 elements 832 and 416
+    assert runs(1, f32, 98352) == 64 and runs(1, f32, 98368) == 0 and runs(4, f32, 49168) == 32 and runs(4, f32, 49184) == 0 and runs(4, (8, 2, 32, 4), 64) == 1
+    assert runs(5, f32, 19216) == 25 and runs(5, f32, 19232) == 0 and runs(63, f32, 6144) == 8 and runs(63, f32, 6160) == 0
+    assert runs(64, f32, 12288) == 8 and runs(64, f32, 12304) == 0 and runs(1, (14, 2, 32, 4), 49200) == 64 and runs(1, (14, 2, 32, 4), 49216) == 0
+    assert runs(15, (40, 8, 128, 4), 6656) == 8 and runs(15, (40, 8, 128, 4), 6672) == 0 and runs(16, (40, 8, 128, 4), 13312) == 8 and runs(16, (40, 8, 128, 4), 13328) == 0
+    assert runs(200, (14, 2, 256, 4), 1664) == 2 and runs(200, (14, 2, 256, 4), 1680) == 0
+    assert runs(3, wide, 3520) == 10 and runs(3, wide, 3536) == 0 and runs(3, (32, 8, 64, 4), 7040) == 10 and runs(3, (32, 8, 64, 4), 7056) == 0  # (176 KB)
     assert runs(7, wide, 33776) == runs(206, (32, 8, 64, 4), 64) == runs(16, (8, 8, 64, 4), 608) == runs(2, (8, 2, 128, 4), 4000) == 0
 
 
@@ -234,12 +240,13 @@ def test_runs_that_several_waves_merge(plan, runs, batch, kv):
     from tests.test_gpu_decode_merge import Batch
 
     announce(f"decode short: {runs} runs, {kv}")
-    b = Batch([8180, 40] + [i % 3 for i in range(batch - 2)], 14, 2, 64, kv, seed=runs)
+    most = 8180 if runs > 9 else 6100
+    b = Batch([most, 40] + [i % 3 for i in range(batch - 2)], 14, 2, 64, kv, seed=runs)
     (k, v, _, _), _ = b.device_pools()
     tables = tables_to_device(b.tables)
     assert plan.runs(batch, 14, 2, 64, 4 if kv == "f32" else 2, tables.shape[1], 16, 0, 4096) == runs
     q, n = b.q.to(DEV), torch.tensor(b.lens, dtype=torch.int32, device=DEV)
-    for ez in (None, 8180 - n):
+    for ez in (None, most - n):
         got = ops.decode(q, k, v, tables, n, 16, b.scale, ops.decode_workspace(q, k), ez)
         want = po.paged_decode(b.q.float(), b.k.float(), b.v.float(), b.tables, b.lens, 16, b.scale, pad_zero_keys=ez is not None)
         # (16 bits: the output's rounding, half a unit of 2^-8, doubled for sums)
