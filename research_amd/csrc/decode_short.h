@@ -285,11 +285,22 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                 m = mx;
                 l *= alpha;
                 if constexpr (k32) {
+                    // (a logit's own rounding is in m, but not in the product here: up to a quarter below 2^23, 128 from 2^31 on, where no weight is finite
+                    // or none is left.  Rows that have such logits take the rounded ones.)
+                    float factor = p.scale_log2;
+                    const bool far = !(fabsf(m) < 0x1p23f);
+                    if (__builtin_amdgcn_ballot_w64(far) != 0) {  // uniform
+                        factor = far ? 1.f : factor;
+#pragma unroll
+                        for (int t = 0; t < NT; ++t)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) raw[t][i] = far ? x[t][i] : raw[t][i];
+                    }
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            x[t][i] = x[t][i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(raw[t][i], p.scale_log2, -m));
+                            x[t][i] = x[t][i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(raw[t][i], factor, -m));
 #pragma unroll
                     for (int t = 0; t < NT; ++t) l += (x[t][0] + x[t][1]) + (x[t][2] + x[t][3]);
                     f4 sum[2][4];  // (of the 16 keys and columns at hand, and of those before)

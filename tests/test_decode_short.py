@@ -230,6 +230,37 @@ def test_pools_of_32_bits(plan, lens, hq, hkv, d, window, bs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bits", [12, 20, 24, 31, 40, 60])
+@pytest.mark.parametrize("lens,hq,hkv,d", [([300, 40, 1, 0, 17], 14, 2, 64), ([1100, 40], 8, 2, 128), ([200, 64], 6, 1, 256)])
+def test_far_logits_of_32_bits(plan, lens, hq, hkv, d, bits):
+    """Logits about 2^bits, whose own rounding is much of a power of two or more: the largest key's value is what remains."""
+    from research_amd import ops
+    from tests.gpu_helpers import DEV, announce, assert_close, tables_to_device
+    from tests.test_gpu_decode_merge import Batch
+
+    announce(f"decode short, 32 bits: logits of 2^{bits}, {hq}/{hkv}x{d}")
+    b = Batch(lens, hq, hkv, d, "f32", seed=bits)
+    (k, v, _, _), (kr, vr) = b.device_pools()
+    tables = tables_to_device(b.tables)
+    assert plan.runs(len(lens), hq, hkv, d, 4, tables.shape[1], 16, 0, 4096) > 0
+    q, n = b.q * 2.0 ** bits, torch.tensor(b.lens, dtype=torch.int32, device=DEV)
+    want, tied = np.zeros((len(lens), hq, d)), np.zeros((len(lens), hq, 1), dtype=bool)
+    for i, x in enumerate(b.lens):
+        if x:
+            rows = np.array([b.tables[i][j // 16] * 16 + j % 16 for j in range(x)], dtype=np.int64)
+            kk, vv = (t.double().cpu().numpy().reshape(-1, hkv, d)[rows].repeat(hq // hkv, axis=1) for t in (kr, vr))
+            s = np.einsum("hd,jhd->hj", q[i].double().numpy(), kk) * b.scale
+            w = np.exp(s - s.max(axis=1, keepdims=True))
+            want[i] = np.einsum("hj,jhd->hd", w / w.sum(axis=1, keepdims=True), vv)
+            # (a sum of d products of 32 bits errs by less than d 2^-23 of the largest logit: rows whose two largest keys are closer have no one answer)
+            top = np.sort(np.concatenate([s, s[:, :1] * 0 - np.inf], axis=1), axis=1)[:, -2:]
+            tied[i, :, 0] = top[:, 1] - top[:, 0] < 16 + d * 2.0 ** -22 * np.abs(s).max(axis=1)
+    got = ops.decode(q.to(DEV), k, v, tables, n, 16, b.scale, ops.decode_workspace(q.to(DEV), k)).double().cpu().numpy()
+    assert np.isfinite(got).all() and tied.mean() < 0.25
+    assert_close(np.where(tied, want, got), want, 1e-5, "the largest key's value")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kv", ["bf16", "f32"])
 @pytest.mark.parametrize("runs,batch", [(8, 16), (9, 14), (16, 8), (18, 7), (32, 4), (42, 3), (64, 2)])
 def test_runs_that_several_waves_merge(plan, runs, batch, kv):
