@@ -271,7 +271,7 @@ def test_runs_that_several_waves_merge(plan, runs, batch, kv):
     from tests.test_gpu_decode_merge import Batch
 
     announce(f"decode short: {runs} runs, {kv}")
-    most = 8180 if runs > 9 else 6100
+    most = 8180 if kv == "bf16" or runs > 9 else 6100
     b = Batch([most, 40] + [i % 3 for i in range(batch - 2)], 14, 2, 64, kv, seed=runs)
     (k, v, _, _), _ = b.device_pools()
     tables = tables_to_device(b.tables)

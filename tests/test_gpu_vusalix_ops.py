@@ -428,7 +428,7 @@ def test_decode_pieces_with_sinks_and_padding_rows():
 
 
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 62), (4, 1, 128, 128), (3, 3, 256, 250)])
-@pytest.mark.parametrize("keys", [600, 2250, 2304, 4100])  # (tables have room for 32 to 47 keys more)
+@pytest.mark.parametrize("keys", [600, 2250, 2303, 2304, 4100])  # (tables have room for 32 to 47 keys more)
 def test_pieces_around_the_eights_that_a_wave_joins(keys, heads, kv, dim, vdim):
     """Two, eight, nine and sixteen pieces of the longer sequence, one with keys of the shorter, against one piece."""
     announce(f"scored joins {keys} {heads} {kv} {dim} {vdim}")
