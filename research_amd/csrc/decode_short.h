@@ -286,7 +286,8 @@ template <typename KV, typename QT, int D> __global__ __launch_bounds__(kThreads
                 l *= alpha;
                 if constexpr (k32) {
                     // (a logit's own rounding is in m, but not in the product here: up to a quarter below 2^23, 128 from 2^31 on, where no weight is finite
-                    // or none is left.  Rows that have such logits take the rounded ones.)
+                    // or none is left.  Rows that have such logits take the rounded ones.  us without -> with it: 14 / 2 heads of 64, 4 of 64 keys 6.02 -> 6.06, 200 of
+                    // 1000 47.1 -> 47.4; of 256, 100 of 500 51.4 -> 52.3; 40 / 8 of 128, 100 of 1000 152.8 -> 153.7)
                     float factor = p.scale_log2;
                     const bool far = !(fabsf(m) < 0x1p23f);
                     if (__builtin_amdgcn_ballot_w64(far) != 0) {  // uniform
